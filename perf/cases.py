@@ -90,12 +90,12 @@ MODELS = {
 def listed():
     return [
         # a three-token prompt to a test model, as `axon logits` is first tried: nothing but launches and host work
-        dict(name="tiny, 3 tokens", model="tiny", dtype="bfloat16", page=64, kind="prompt", requests=1, shortest=3, longest=3),
+        dict(name="tiny 3 tokens", model="tiny", dtype="bfloat16", page=64, kind="prompt", requests=1, shortest=3, longest=3),
         # serving the headline model: eight conversations of unequal length, the usual load of one small server
-        dict(name="7b decode, 8 ragged", model="qwen2.5-7b", dtype="bfloat16", page=16, kind="decode", requests=8, shortest=301,
+        dict(name="7b decode 8 ragged", model="qwen2.5-7b", dtype="bfloat16", page=16, kind="decode", requests=8, shortest=301,
              longest=3907),
         # a full server: many conversations, mostly short
-        dict(name="7b decode, 64 short", model="qwen2.5-7b", dtype="bfloat16", page=64, kind="decode", requests=64, shortest=64,
+        dict(name="7b decode 64 short", model="qwen2.5-7b", dtype="bfloat16", page=64, kind="decode", requests=64, shortest=64,
              longest=900),
         # a prompt of the headline benchmark's length in one step
         dict(name="7b prompt 2048", model="qwen2.5-7b", dtype="bfloat16", page=16, kind="prompt", requests=1, shortest=2048,
@@ -109,16 +109,16 @@ def listed():
         # the 32-bit path, which shows what bfloat16 hides: scoring a prompt, and decoding a few conversations
         dict(name="dense fp32 prompt 777", model="dense 2048", dtype="float32", page=64, kind="prompt", requests=1, shortest=777,
              longest=777),
-        dict(name="dense fp32 decode, 5", model="dense 2048", dtype="float32", page=64, kind="decode", requests=5, shortest=100,
+        dict(name="dense fp32 decode 5", model="dense 2048", dtype="float32", page=64, kind="decode", requests=5, shortest=100,
              longest=1500),
         # the other designs, prompts and decoding: several ragged prompts in a step, a single long one, conversations
         dict(name="pikesun prompt 2048", model="pikesun", dtype="bfloat16", page=64, kind="prompt", requests=1, shortest=2048,
              longest=2048),
-        dict(name="pikesun decode, 8", model="pikesun", dtype="bfloat16", page=64, kind="decode", requests=8, shortest=200,
+        dict(name="pikesun decode 8", model="pikesun", dtype="bfloat16", page=64, kind="decode", requests=8, shortest=200,
              longest=2500),
-        dict(name="zugutar prompts, 3 ragged", model="zugutar", dtype="bfloat16", page=64, kind="prompt", requests=3,
+        dict(name="zugutar prompts 3 ragged", model="zugutar", dtype="bfloat16", page=64, kind="prompt", requests=3,
              shortest=311, longest=1203),
-        dict(name="bafavik decode, 16", model="bafavik", dtype="bfloat16", page=64, kind="decode", requests=16, shortest=90,
+        dict(name="bafavik decode 16", model="bafavik", dtype="bfloat16", page=64, kind="decode", requests=16, shortest=90,
              longest=1700),
     ]
 
