@@ -5,194 +5,285 @@
 // (the reference states the rule for its own kernels: src/cuda/decode.cu:352-369,
 // src/cuda/prefill.cu:6-16).  Rows only ride along.
 //
-// gemm_fma: any M, N, K and strides, 32-bit FMA, a chain per output and 32 k, whose sums are added in
-// ascending order (a third of the rounding of one chain over all k): the float32 build's
+// gemm_fma: any M, N, K and strides, 32-bit multiply-adds, a chain per output and 32 k, whose sums are
+// added in ascending order (a third of the rounding of one chain over all k): the float32 build's
 // product (true 32-bit), and the bfloat16 build's fallback for shapes the MFMA kernels refuse.
+// The chains run on the 32-bit matrix cores: a 16x16x4 product of 32-bit operands gives, bit for bit,
+// what four fmaf in ascending k give (measured over random operands, denormals among them), at
+// twice the rate that the vector unit has without its packed instructions.
 #include "api.h"
 #include "common.h"
 #include "instances.h"
 
-#define FMA_BN 64
-#define FMA_BK 16
 #define FMA_PART 32    // k of one chain
-#define FMA_THREADS 256
+typedef __attribute__((ext_vector_type(4))) float f32x4;
 
-// BM rows x 64 columns per block of 256 threads; thread (ty, tx) owns RM = BM / 16 rows and
-// 4 columns.  K is walked in steps of 16 through LDS; inside a step k ascends.
-template <int BM, bool GLU>
-__global__ void __launch_bounds__(FMA_THREADS)
-gemm_fma_kernel(const elem_t* __restrict__ x, int x_stride, const elem_t* __restrict__ w, const void* __restrict__ bias,
-                int bias_is_f32, void* __restrict__ out, int out_stride, int M, int N, int K, int mode, bool vec_x,
-                bool vec_w) {
-  constexpr int RM = BM / 16;
-  __shared__ float xs[FMA_BK][BM + 4];
-  __shared__ float ws[FMA_BK][FMA_BN + 4];
-  __shared__ float us[GLU ? FMA_BK : 1][FMA_BN + 4];  // the up rows of the same columns (GLU: W holds 2 N rows)
-  const int tid = threadIdx.x;
-  const int tx = tid & 15, ty = tid >> 4;
-  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * FMA_BN;
+#define FMA_STEP(acc, a, b, j) acc = __builtin_amdgcn_mfma_f32_16x16x4f32((a)[j], (b)[j], acc, 0, 0, 0)
 
-  float acc[RM][4], acc_up[GLU ? RM : 1][4], sum[RM][4], sum_up[GLU ? RM : 1][4];
+// Four k of a row from `k` on; what lies behind K reads other numbers of the row here (VEC: K is a multiple of four,
+// one 16-byte load; a branch round it would have the compiler wait for every load under way) and is cleared
+// when it is used.  Rows that do not exist read a row that does: their outputs are not stored.
+template <bool VEC>
+__device__ __forceinline__ void fma_load(const elem_t* __restrict__ row, int k, int K, float (&out)[4]) {
+  if (VEC) {
+    load4_guarded(row + min(k, K - 4), 4, true, out);
+  } else {
 #pragma unroll
-  for (int i = 0; i < RM; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      acc[i][j] = sum[i][j] = 0.0f;
-      if (GLU) acc_up[i][j] = sum_up[i][j] = 0.0f;
-    }
-
-  // loader: each thread brings 4 consecutive k of one row, a step ahead of the products
-  const int lrow = tid >> 2, lk = (tid & 3) * 4;
-  float pw[4], pu[4], px[4];
-  auto fetch = [&](int k0) {
-    const int n = n0 + lrow, m = m0 + lrow;
-    const int left = max(0, min(4, K - (k0 + lk)));
-    load4_guarded(w + (size_t)n * K + k0 + lk, n < N ? left : 0, vec_w, pw);
-    if (GLU) load4_guarded(w + (size_t)(N + n) * K + k0 + lk, n < N ? left : 0, vec_w, pu);
-    if (lrow < BM) load4_guarded(x + (size_t)m * x_stride + k0 + lk, m < M ? left : 0, vec_x, px);
-  };
-  fetch(0);
-  for (int k0 = 0; k0 < K; k0 += FMA_BK) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      ws[lk + i][lrow] = pw[i];
-      if (GLU) us[lk + i][lrow] = pu[i];
-      if (lrow < BM) xs[lk + i][lrow] = px[i];
-    }
-    __syncthreads();
-    if (k0 + FMA_BK < K) fetch(k0 + FMA_BK);
-#pragma unroll
-    for (int kk = 0; kk < FMA_BK; ++kk) {
-      float a[RM], b[4];
-#pragma unroll
-      for (int i = 0; i < RM; ++i) a[i] = xs[kk][ty * RM + i];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) b[j] = ws[kk][tx * 4 + j];
-#pragma unroll
-      for (int i = 0; i < RM; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
-      if (GLU) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) b[j] = us[kk][tx * 4 + j];
-#pragma unroll
-        for (int i = 0; i < RM; ++i)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) acc_up[i][j] = fmaf(a[i], b[j], acc_up[i][j]);
-      }
-    }
-    if ((k0 + FMA_BK) % FMA_PART == 0 || k0 + FMA_BK >= K) {
-#pragma unroll
-      for (int i = 0; i < RM; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          sum[i][j] += acc[i][j];
-          acc[i][j] = 0.0f;
-          if (GLU) { sum_up[i][j] += acc_up[i][j]; acc_up[i][j] = 0.0f; }
-        }
-    }
-    __syncthreads();
-  }
-
-#pragma unroll
-  for (int i = 0; i < RM; ++i) {
-    const int m = m0 + ty * RM + i;
-    if (m >= M) continue;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int n = n0 + tx * 4 + j;
-      if (n >= N) continue;
-      float v = sum[i][j];
-      if (bias) v += load_vec(bias, bias_is_f32, n);
-      const size_t at = (size_t)m * out_stride + n;
-      if (GLU) ((elem_t*)out)[at] = from_float(swiglu1(v, sum_up[i][j]));
-      else if (mode_stores_elem(mode)) ((elem_t*)out)[at] = from_float(mode_value(v, mode));
-      else if (mode == MODE_ADD_F32) ((float*)out)[at] += v;
-      else ((float*)out)[at] = v;
-    }
+    for (int e = 0; e < 4; ++e) out[e] = to_float(row[min(k + e, K - 1)]);
   }
 }
-
-// Up to 16 rows (a decoding step): 16 rows x 16 columns a block, one output a thread, K in steps
-// of 256 through LDS, the next step's loads in flight while this one is multiplied.  Such a
-// product only waits for W, so it wants many blocks with much in flight each (the tile above
-// gives N / 64 blocks with 4 KB each).  The chains of an output are the same.
-#define FEW_BK 256
-#define FEW_LD (FEW_BK + 4)   // rows 4 banks apart: the 16 rows a wave reads fall into all 64 banks
-template <bool GLU>
-__global__ void __launch_bounds__(FMA_THREADS)
-gemm_fma_few_rows_kernel(const elem_t* __restrict__ x, int x_stride, const elem_t* __restrict__ w,
-                         const void* __restrict__ bias, int bias_is_f32, void* __restrict__ out, int out_stride, int M,
-                         int N, int K, int mode, bool vec_x, bool vec_w) {
-  __shared__ __align__(16) float xs[16][FEW_LD];
-  __shared__ __align__(16) float ws[16][FEW_LD];
-  __shared__ __align__(16) float us[GLU ? 16 : 1][GLU ? FEW_LD : 4];
-  const int tid = threadIdx.x;
-  const int tx = tid & 15, ty = tid >> 4;
-  const int n0 = blockIdx.x * 16;
-
-  // loader: a tile is 16 rows of 64 groups of four k; a thread brings groups tid + 256 j
-  float px[4][4], pw[4][4], pu[GLU ? 4 : 1][4];
-  auto fetch = [&](int k0) {
+__device__ __forceinline__ void fma_clear(float (&v)[4], int k, int K) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int g = tid + FMA_THREADS * j, row = g >> 6, k = k0 + 4 * (g & 63);
-      const int left = max(0, min(4, K - k)), n = n0 + row;
-      load4_guarded(x + (size_t)row * x_stride + k, row < M ? left : 0, vec_x, px[j]);
-      load4_guarded(w + (size_t)n * K + k, n < N ? left : 0, vec_w, pw[j]);
-      if (GLU) load4_guarded(w + (size_t)(N + n) * K + k, n < N ? left : 0, vec_w, pu[j]);
-    }
-  };
-  auto stage = [&]() {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int g = tid + FMA_THREADS * j, row = g >> 6, kk = 4 * (g & 63);
-      *reinterpret_cast<float4*>(&xs[row][kk]) = make_float4(px[j][0], px[j][1], px[j][2], px[j][3]);
-      *reinterpret_cast<float4*>(&ws[row][kk]) = make_float4(pw[j][0], pw[j][1], pw[j][2], pw[j][3]);
-      if (GLU) *reinterpret_cast<float4*>(&us[row][kk]) = make_float4(pu[j][0], pu[j][1], pu[j][2], pu[j][3]);
-    }
-  };
+  for (int e = 0; e < 4; ++e) v[e] = k + e < K ? v[e] : 0.0f;
+}
 
-  float sum = 0.0f, sum_up = 0.0f;
-  fetch(0);
-  for (int k0 = 0; k0 < K; k0 += FEW_BK) {
-    stage();
-    __syncthreads();
-    if (k0 + FEW_BK < K) fetch(k0 + FEW_BK);
-    const int k_end = min(FEW_BK, K - k0);   // beyond K the stage holds zeros
-    for (int part = 0; part < k_end; part += FMA_PART) {
-      float acc = 0.0f, acc_up = 0.0f;
-#pragma unroll 4
-      for (int i = 0; i < FMA_PART; i += 4) {    // beyond K, too: zeros
-        const float4 a = *reinterpret_cast<const float4*>(&xs[ty][part + i]);
-        const float4 b = *reinterpret_cast<const float4*>(&ws[tx][part + i]);
-        acc = fmaf(a.x, b.x, acc);
-        acc = fmaf(a.y, b.y, acc);
-        acc = fmaf(a.z, b.z, acc);
-        acc = fmaf(a.w, b.w, acc);
-        if (GLU) {
-          const float4 u = *reinterpret_cast<const float4*>(&us[tx][part + i]);
-          acc_up = fmaf(a.x, u.x, acc_up);
-          acc_up = fmaf(a.y, u.y, acc_up);
-          acc_up = fmaf(a.z, u.z, acc_up);
-          acc_up = fmaf(a.w, u.w, acc_up);
-        }
-      }
-      sum += acc;
-      sum_up += acc_up;
-    }
-    __syncthreads();
-  }
-
-  const int m = ty, n = n0 + tx;
-  if (m >= M || n >= N) return;
-  float v = sum;
+__device__ inline void fma_store(float v, float up, bool glu, const void* bias, int bias_is_f32, void* out, size_t at, int n,
+                                 int mode) {
   if (bias) v += load_vec(bias, bias_is_f32, n);
-  const size_t at = (size_t)m * out_stride + n;
-  if (GLU) ((elem_t*)out)[at] = from_float(swiglu1(v, sum_up));
+  if (glu) ((elem_t*)out)[at] = from_float(swiglu1(v, up));
   else if (mode_stores_elem(mode)) ((elem_t*)out)[at] = from_float(mode_value(v, mode));
   else if (mode == MODE_ADD_F32) ((float*)out)[at] += v;
   else ((float*)out)[at] = v;
+}
+
+// Many rows: 64 x 64 outputs a block of 4 waves, each 2 x 2 tiles of 16 x 16 (gated: half of a wave's
+// columns are gate rows of W, half the up rows of the same outputs).  K is walked a chain at a time through
+// two stages of LDS; the stage's operands are read first, then the next stage is written and the one
+// after it asked for, all beside this stage's products.  A lane of a product holds k = 4 i + q of
+// its row (q = lane / 16), so a row's 16 k are staged in the order [q][i]: one 16-byte read is a
+// lane's operand of four products.  Rows of the stage are 144 bytes apart: the 16 rows that a read
+// takes at a time fall into 16 different slots of the 64 banks.
+#define TILE_M 64
+#define TILE_LD (FMA_PART + 4)
+template <bool GLU, bool VEC>
+__global__ void __launch_bounds__(256, 2)
+gemm_fma_kernel(const elem_t* __restrict__ x, int x_stride, const elem_t* __restrict__ w, const void* __restrict__ bias,
+                int bias_is_f32, void* __restrict__ out, int out_stride, int M, int N, int K, int mode) {
+  constexpr int R = 2, BM = TILE_M, ROWS = 2 * BM; // rows of X and then of W in a stage
+  constexpr int BN = GLU ? BM / 2 : BM;            // columns of the output
+  constexpr int LOADS = ROWS * FMA_PART / 4 / 256; // groups of four k a thread brings
+  constexpr int ACROSS = FMA_PART / 4, DOWN = 256 / ACROSS;   // neighbouring threads bring a row's stage
+  __shared__ __align__(16) float stages[2 * ROWS * TILE_LD];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
+  const int r16 = lane & 15, q = lane >> 4;
+  const int wm = (wave >> 1) * 16 * R, wn = (wave & 1) * 16 * R;
+
+  float in[LOADS][4];
+  const elem_t* from[LOADS];
+#pragma unroll
+  for (int j = 0; j < LOADS; ++j) {
+    const int row = tid / ACROSS + DOWN * j;
+    if (DOWN * j < BM) {
+      from[j] = x + (size_t)min(m0 + row, M - 1) * x_stride;
+    } else {
+      // gated: a wave's columns are R / 2 tiles of gate rows, then the up rows of the same outputs
+      const int half = (row - BM) / (16 * R), place = (row - BM) % (16 * R);
+      const bool up = GLU && place >= 8 * R;
+      const int n = GLU ? n0 + half * 8 * R + place - (up ? 8 * R : 0) : n0 + row - BM;
+      from[j] = w + (size_t)(min(n, N - 1) + (up ? N : 0)) * K;
+    }
+  }
+  const int k_mine = 4 * (tid % ACROSS);
+  auto fetch = [&](int k0) {
+#pragma unroll
+    for (int j = 0; j < LOADS; ++j) fma_load<VEC>(from[j], k0 + k_mine, K, in[j]);
+  };
+  auto stage = [&](int which, int k0) {
+    float* base = stages + which * ROWS * TILE_LD;
+#pragma unroll
+    for (int j = 0; j < LOADS; ++j) {
+      float* to = base + (tid / ACROSS + DOWN * j) * TILE_LD + 16 * (tid % ACROSS / 4) + (tid & 3);
+      if (k0 + FMA_PART > K) fma_clear(in[j], k0 + k_mine, K);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) to[4 * e] = in[j][e];
+    }
+  };
+
+  f32x4 sum[R][R];
+#pragma unroll
+  for (int i = 0; i < R; ++i)
+#pragma unroll
+    for (int j = 0; j < R; ++j) sum[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  fetch(0);
+  stage(0, 0);
+  if (FMA_PART < K) fetch(FMA_PART);
+  __syncthreads();
+  for (int k0 = 0, which = 0; k0 < K; k0 += FMA_PART, which ^= 1) {
+    const float* base = stages + which * ROWS * TILE_LD;
+    f32x4 a[2][R], b[2][R];
+#pragma unroll
+    for (int g = 0; g < 2; ++g)
+#pragma unroll
+      for (int i = 0; i < R; ++i) {
+        a[g][i] = *reinterpret_cast<const f32x4*>(&base[(wm + 16 * i + r16) * TILE_LD + 16 * g + 4 * q]);
+        b[g][i] = *reinterpret_cast<const f32x4*>(&base[(BM + wn + 16 * i + r16) * TILE_LD + 16 * g + 4 * q]);
+      }
+    // the next stage's numbers, asked for a step ago, go into LDS beside this stage's products
+    if (k0 + FMA_PART < K) stage(which ^ 1, k0 + FMA_PART);
+    if (k0 + 2 * FMA_PART < K) fetch(k0 + 2 * FMA_PART);
+    f32x4 acc[R][R];
+#pragma unroll
+    for (int g = 0; g < 2; ++g)
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int i = 0; i < R; ++i)
+#pragma unroll
+          for (int j = 0; j < R; ++j) {
+            if (g == 0 && s == 0) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            FMA_STEP(acc[i][j], a[g][i], b[g][j], s);
+          }
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+#pragma unroll
+      for (int j = 0; j < R; ++j) sum[i][j] += acc[i][j];
+    __syncthreads();
+  }
+
+  constexpr int COLS = GLU ? R / 2 : R;
+#pragma unroll
+  for (int i = 0; i < R; ++i)
+#pragma unroll
+    for (int j = 0; j < COLS; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int m = m0 + wm + 16 * i + 4 * q + e;
+        const int n = n0 + (GLU ? wn / 2 : wn) + 16 * j + r16;
+        if (m < M && n < N)
+          fma_store(sum[i][j][e], GLU ? sum[i][j + (GLU ? COLS : 0)][e] : 0.0f, GLU, bias, bias_is_f32, out,
+                    (size_t)m * out_stride + n, n, mode);
+      }
+}
+
+// Four lanes l, l + 16, l + 32, l + 48 hold k = 4 q + j of a row in register j: after this they hold
+// k = 4 j + q, a product's operand for each j.
+__device__ inline f32x4 fma_operand(const float (&v)[4]) {
+  unsigned r[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) r[j] = __builtin_bit_cast(unsigned, v[j]);
+#pragma unroll
+  for (int j = 0; j < 4; j += 2) {
+    const auto s = __builtin_amdgcn_permlane16_swap(r[j], r[j + 1], false, false);
+    r[j] = s[0];
+    r[j + 1] = s[1];
+  }
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const auto s = __builtin_amdgcn_permlane32_swap(r[j], r[j + 2], false, false);
+    r[j] = s[0];
+    r[j + 2] = s[1];
+  }
+  return f32x4{__builtin_bit_cast(float, r[0]), __builtin_bit_cast(float, r[1]), __builtin_bit_cast(float, r[2]),
+               __builtin_bit_cast(float, r[3])};
+}
+
+// Few rows (decoding): such a product only waits for W, so a block takes NR (16 or 8) columns and the
+// chains of an output, which do not need each other, are shared out over its 8 waves: every wave
+// streams its chains' W from memory straight into operands, leaves the chains' sums in LDS, and a thread
+// an output adds them in ascending order.  MT tiles of 16 rows of X ride along with each W (a wave reads
+// them from L2 beside W: with 64 rows of X that is what bounds it).  5 rows: 2,560 x K 2,048 25 -> 16 us,
+// 2,048 x 5,632 63 -> 27, 32,000 x 2,048 (262 MB) 85 -> 61 us, 4.3 TB/s; 64 rows of 2,048 x 5,632 332 -> 63 us.
+#define FEW_WAVES 8
+template <int MT, int NR, bool GLU, bool VEC>
+__global__ void __launch_bounds__(64 * FEW_WAVES, 2)
+gemm_fma_few_rows_kernel(const elem_t* __restrict__ x, int x_stride, const elem_t* __restrict__ w,
+                         const void* __restrict__ bias, int bias_is_f32, void* __restrict__ out, int out_stride, int M,
+                         int N, int K, int mode) {
+  constexpr int NT = GLU ? 2 : 1;
+  constexpr int PW = MT * NT >= 8 ? 1 : MT * NT >= 3 ? 2 : MT * NT == 2 ? 4 : 8;   // chains of a wave in a round
+  constexpr int PARTS = FEW_WAVES * PW, OUTS = MT * 16 * NR;
+  __shared__ __align__(16) float chains[PARTS * NT * OUTS];                        // [chain][gate, up][row][column]
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int r16 = lane & 15, q = lane >> 4;
+  const int n0 = blockIdx.x * NR, m0 = blockIdx.y * MT * 16;
+  const elem_t* w_row = w + (size_t)min(n0 + min(r16, NR - 1), N - 1) * K;
+  const elem_t* x_row[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) x_row[i] = x + (size_t)min(m0 + 16 * i + r16, M - 1) * x_stride;
+  const int n_parts = (K + FMA_PART - 1) / FMA_PART;
+  constexpr int MINE = (OUTS + 64 * FEW_WAVES - 1) / (64 * FEW_WAVES);
+  float sum[MINE], sum_up[MINE];
+#pragma unroll
+  for (int i = 0; i < MINE; ++i) sum[i] = sum_up[i] = 0.0f;
+
+  for (int first = 0; first < n_parts; first += PARTS) {
+    float wv[NT][PW][2][4];
+#pragma unroll
+    for (int p = 0; p < PW; ++p)
+#pragma unroll
+      for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+          fma_load<VEC>(w_row + (size_t)t * N * K, (first + wave * PW + p) * FMA_PART + 16 * g + 4 * q, K, wv[t][p][g]);
+#pragma unroll
+    for (int p = 0; p < PW; ++p) {
+      const int part = wave * PW + p, k0 = (first + part) * FMA_PART;
+      if (k0 >= K) break;                            // the same for the whole wave
+      f32x4 a[NT][2];
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+          if (k0 + FMA_PART > K) fma_clear(wv[t][p][g], k0 + 16 * g + 4 * q, K);
+          a[t][g] = fma_operand(wv[t][p][g]);
+        }
+#pragma unroll
+      for (int i = 0; i < MT; ++i) {
+        f32x4 b[2];
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+          float xv[4];
+          fma_load<VEC>(x_row[i], k0 + 16 * g + 4 * q, K, xv);
+          if (k0 + FMA_PART > K) fma_clear(xv, k0 + 16 * g + 4 * q, K);
+          b[g] = fma_operand(xv);
+        }
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          f32x4 acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+          for (int g = 0; g < 2; ++g)
+#pragma unroll
+            for (int s = 0; s < 4; ++s) FMA_STEP(acc, a[t][g], b[g], s);
+          // columns 4 q .. 4 q + 3 of row 16 i + r16
+          if (4 * q < NR) *reinterpret_cast<f32x4*>(&chains[(part * NT + t) * OUTS + (16 * i + r16) * NR + 4 * q]) = acc;
+        }
+      }
+    }
+    __syncthreads();
+    const int count = min(PARTS, n_parts - first);
+#pragma unroll
+    for (int i = 0; i < MINE; ++i) {
+      const int o = tid + 64 * FEW_WAVES * i;
+      if (o < OUTS) {
+#pragma unroll 8
+        for (int p = 0; p < count; ++p) {
+          sum[i] += chains[p * NT * OUTS + o];
+          if (GLU) sum_up[i] += chains[(p * NT + NT - 1) * OUTS + o];
+        }
+      }
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int i = 0; i < MINE; ++i) {
+    const int o = tid + 64 * FEW_WAVES * i, m = m0 + o / NR, col = n0 + o % NR;
+    if (o < OUTS && m < M && col < N)
+      fma_store(sum[i], sum_up[i], GLU, bias, bias_is_f32, out, (size_t)m * out_stride + col, col, mode);
+  }
+}
+
+template <int MT, bool GLU, bool VEC>
+static void launch_fma_few(const elem_t* x, int x_stride, const elem_t* w, const void* bias, int bias_is_f32, void* out,
+                           int out_stride, int m, int n, int k, int mode, hipStream_t stream) {
+  const int rows = ceil_div(m, 16 * MT);
+  // blocks of 8 columns where blocks of 16 would leave CUs without one
+  if ((long)ceil_div(n, 16) * rows < 256)
+    gemm_fma_few_rows_kernel<MT, 8, GLU, VEC><<<dim3(ceil_div(n, 8), rows), 64 * FEW_WAVES, 0, stream>>>(
+        x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode);
+  else
+    gemm_fma_few_rows_kernel<MT, 16, GLU, VEC><<<dim3(ceil_div(n, 16), rows), 64 * FEW_WAVES, 0, stream>>>(
+        x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode);
 }
 
 static int launch_fma(const elem_t* x, int x_stride, const elem_t* w, const void* bias, int bias_is_f32, void* out,
@@ -200,19 +291,28 @@ static int launch_fma(const elem_t* x, int x_stride, const elem_t* w, const void
   const size_t vbytes = 4 * sizeof(elem_t);
   const bool vec_w = (k % 4 == 0) && ((uintptr_t)w % vbytes == 0);
   const bool vec_x = (k % 4 == 0) && (x_stride % 4 == 0) && ((uintptr_t)x % vbytes == 0);
-#define FMA_LAUNCH(BM, GLU)                                                                                      \
-  AXK_INSTANCE(INST_GEMM_FMA, BM, GLU);                                                                          \
-  if (BM == 16)                                                                                                  \
-    gemm_fma_few_rows_kernel<GLU><<<dim3(ceil_div(n, 16)), FMA_THREADS, 0, stream>>>(                            \
-        x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode, vec_x, vec_w);                        \
-  else                                                                                                           \
-    gemm_fma_kernel<64, GLU><<<dim3(ceil_div(n, FMA_BN), ceil_div(m, 64)), FMA_THREADS, 0, stream>>>(            \
-        x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode, vec_x, vec_w)
-  if (mode == MODE_SWIGLU) {
-    if (m <= 16) { FMA_LAUNCH(16, true); } else { FMA_LAUNCH(64, true); }
-  } else {
-    if (m <= 16) { FMA_LAUNCH(16, false); } else { FMA_LAUNCH(64, false); }
+#define FMA_ARGS x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode, stream
+// Up to 64 rows a product waits for W; from 65 to 128 so it does where the tiles would be fewer than
+// the CUs (2,048 columns of K 5,632 at 128 rows: 143 us with 64 tiles, 67 us with a wave a part of K), while
+// 352 tiles (a gated product of 5,632 columns) take 90 us against 117.
+#define FMA_LAUNCH(GLU, VEC)                                                                  \
+  if (m <= 16) {                                                                              \
+    AXK_INSTANCE(INST_GEMM_FMA, 16, GLU);                                                     \
+    launch_fma_few<1, GLU, VEC>(FMA_ARGS);                                                    \
+  } else {                                                                                    \
+    AXK_INSTANCE(INST_GEMM_FMA, 64, GLU);                                                     \
+    const dim3 tiles(ceil_div(n, GLU ? TILE_M / 2 : TILE_M), ceil_div(m, TILE_M));            \
+    if (m <= 32) launch_fma_few<2, GLU, VEC>(FMA_ARGS);                                       \
+    else if (m <= 64 || (m <= 128 && (long)tiles.x * tiles.y < 256)) launch_fma_few<4, GLU, VEC>(FMA_ARGS); \
+    else gemm_fma_kernel<GLU, VEC><<<tiles, 256, 0, stream>>>(x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode); \
   }
+  const bool glu = mode == MODE_SWIGLU;
+  if (vec_x && vec_w) {
+    if (glu) { FMA_LAUNCH(true, true) } else { FMA_LAUNCH(false, true) }
+  } else {
+    if (glu) { FMA_LAUNCH(true, false) } else { FMA_LAUNCH(false, false) }
+  }
+#undef FMA_ARGS
 #undef FMA_LAUNCH
   AXK_LAUNCH_CHECK("gemm_fma");
   return 0;
