@@ -55,7 +55,7 @@ int axk_attention(const void* q, int q_stride, const void* k_cache, const void* 
                   const int32_t* seq_rows, void* out, int n_tokens, int n_heads, int n_kv_heads,
                   int head_dim, int page_size, int window, float scale, void* stream);
 
-// The matrix-core attention kernels (bfloat16 build; the float32 build refuses them).
+// The attention kernels on the matrix cores.
 // axk_attention_fast_ok: 1 if they take this head size, page size and group of heads.
 // axk_attention_prefill: tiles [n_tiles][4] = (first token, count <= 128) twice: consecutive
 // tokens of one request, and a second such run (count 0: none) that the same block takes after
@@ -73,6 +73,8 @@ int axk_attention(const void* q, int q_stride, const void* k_cache, const void* 
 // each with its own maximum, folded ascending): a position's result is bit for bit the same from
 // either, alone or in any batch.
 int axk_attention_fast_ok(int head_dim, int page_size, int n_heads, int n_kv_heads);
+// The same for this build: in float32 the kernels of attention_f32.hip, with the bits of axk_attention.
+int axk_attention_blocks_ok(int head_dim, int page_size, int n_heads, int n_kv_heads);
 int axk_attention_prefill_tile(void);      // the most tokens of a run (128)
 int axk_attention_prefill(const void* q, int q_stride, const void* k_cache, const void* v_cache,
                           const int32_t* block_table, int table_stride, const int32_t* positions,

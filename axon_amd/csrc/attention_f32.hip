@@ -1,0 +1,449 @@
+// Paged causal attention on the 32-bit matrix cores (float32 build only): a kernel for prompt portions
+// and one for decoding tokens, called as the bfloat16 build's (attention_mfma.hip) are, with the
+// arithmetic of attention_rows (attention.hip), bit for bit:
+//   s_p = (chain over the dims, ascending) scale;  m = max;  e_p = expf(s_p - m), 0 where the token does not see p;
+//   l = the butterfly of attention_rows over the block's 64 places;  o = chain over the positions, ascending;
+//   blocks of 64 positions folded in ascending order; out = O / L.
+// A 16x16x4 product of 32-bit operands rounds as four fmaf in ascending k, and a position that a token
+// does not see adds 0 times a finite value, which changes nothing.  (Values that are not finite are
+// dealt with apart: see `spoiled`.)
+//
+// Both compute S^T = K Q^T and O^T = V^T P^T.  A lane of a product holds k = 4 i + q of its row for
+// step i (q = lane / 16): where the operand comes from memory a lane loads k = 4 q .. 4 q + 3 and four
+// lanes exchange (f32_operand); what S^T leaves in a lane, positions 4 q .. 4 q + 3 of one column, becomes
+// the B operand of O^T by the same exchange.
+#include <math.h>
+
+#include "api.h"
+#include "common.h"
+
+#define ATT_BLOCK 64
+#define DC_CHUNK 256
+#define CMB_MAX_CHUNKS 1024
+
+#if !AXON_BF16
+
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+
+#define F32_STEP(acc, a, b, j) acc = __builtin_amdgcn_mfma_f32_16x16x4f32((a)[j], (b)[j], acc, 0, 0, 0)
+#define F32_ZERO (f32x4{0.0f, 0.0f, 0.0f, 0.0f})
+
+// Lanes l, l + 16, l + 32, l + 48 hold k = 4 q + j in register j; afterwards k = 4 j + q.
+__device__ __forceinline__ f32x4 f32_operand(f32x4 v) {
+  unsigned r[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) r[j] = __float_as_uint(v[j]);
+#pragma unroll
+  for (int j = 0; j < 4; j += 2) {
+    const auto s = __builtin_amdgcn_permlane16_swap(r[j], r[j + 1], false, false);
+    r[j] = s[0];
+    r[j + 1] = s[1];
+  }
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const auto s = __builtin_amdgcn_permlane32_swap(r[j], r[j + 2], false, false);
+    r[j] = s[0];
+    r[j + 2] = s[1];
+  }
+  return f32x4{__builtin_bit_cast(float, r[0]), __builtin_bit_cast(float, r[1]), __builtin_bit_cast(float, r[2]),
+               __builtin_bit_cast(float, r[3])};
+}
+
+// A block's raw scores (tile t, register e: position p0 + 16 t + 4 q + e of the lane's column) to weights;
+// m_b and l_b in every lane of the column.
+__device__ __forceinline__ void f32_weights(f32x4 (&s)[4], int p0, int lo, int pos, float scale, int q, float& m_b, float& l_b) {
+  float m = -INFINITY;
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int p = p0 + 16 * t + 4 * q + e;
+      s[t][e] = p >= lo && p <= pos ? s[t][e] * scale : -INFINITY;
+      m = fmaxf(m, s[t][e]);
+    }
+  m = fmaxf(m, __shfl_xor(m, 32, AXON_WAVE));
+  m = fmaxf(m, __shfl_xor(m, 16, AXON_WAVE));
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int p = p0 + 16 * t + 4 * q + e;
+      s[t][e] = p >= lo && p <= pos ? expf(s[t][e] - m) : 0.0f;
+    }
+  // the butterfly over places 0 .. 63 at distances 32, 16, 8, 4, 2, 1
+  float b[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    b[e] = (s[0][e] + s[2][e]) + (s[1][e] + s[3][e]);
+    b[e] += __shfl_xor(b[e], 32, AXON_WAVE);
+    b[e] += __shfl_xor(b[e], 16, AXON_WAVE);
+  }
+  m_b = m;
+  l_b = (b[0] + b[2]) + (b[1] + b[3]);
+}
+
+__device__ __forceinline__ int page_index(int p, int page_size) { return p >> (31 - __builtin_clz(page_size)); }
+__device__ __forceinline__ int page_offset(int p, int page_size) { return p & (page_size - 1); }
+
+// ============================================================================ prompt portions
+// A block takes 64 tokens (four waves of 16) of a tile and one query head and walks their blocks of
+// positions; a block's K [64][HD] and V^T [HD][64] go through LDS, rows in the order [16 k][q][i] so that
+// a 16-byte read is a lane's operand of four products, rows a multiple of 16 bytes and an odd number
+// of them apart (16 rows fall into 16 slots of the 64 banks).  The next block's numbers are asked for
+// while this one is multiplied.  grid (pairs of tiles, heads, 4): which tile of the pair and which half of it.
+// Bound by the products (2 x 128 of 32 cycles a wave and block at head size 128) of the tokens that see most:
+// 16 heads, 777 tokens 806 -> 95 us (the kernel of a wave a token and head before), 2,048 tokens 4,514 -> 258 us, 67 TFLOP/s.
+template <int HD>
+__global__ void __launch_bounds__(256, 2)
+attention_f32_prefill_kernel(const float* __restrict__ q, int q_stride, const float* __restrict__ k_cache,
+                             const float* __restrict__ v_cache, const int32_t* __restrict__ block_table, int table_stride,
+                             const int32_t* __restrict__ positions, const int32_t* __restrict__ seq_rows,
+                             float* __restrict__ out, const int32_t* __restrict__ tiles, int n_heads, int n_kv_heads,
+                             int page_size, int window, float scale) {
+  constexpr int KG = HD / 16, DT = HD / 16, K_LD = HD + 4, V_LD = ATT_BLOCK + 4, LOADS = ATT_BLOCK * HD / 4 / 256;
+  extern __shared__ __align__(16) float smem[];      // K [64][K_LD], V^T [HD][V_LD]
+  float* ks = smem;
+  float* vs = smem + ATT_BLOCK * K_LD;
+  const int32_t* mine = tiles + 4 * blockIdx.x + 2 * (blockIdx.z >> 1);
+  const int skip = 64 * (blockIdx.z & 1), count = mine[1] - skip, t0 = mine[0] + skip;
+  if (count <= 0) return;                            // the same for the whole block
+  const int head = blockIdx.y, kvh = head / (n_heads / n_kv_heads);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r16 = lane & 15, g4 = lane >> 4;
+  const int n = min(count, 64), first_pos = positions[t0], last_pos = positions[t0 + n - 1];
+  const bool wave_live = 16 * wave < n;
+  const int row = t0 + min(16 * wave + r16, n - 1), pos = positions[row];
+  const int lo = window > 0 ? max(0, pos + 1 - window) : 0;
+  const int from = window > 0 ? max(0, first_pos + 1 - window) : 0, upto = window > 0 ? max(0, last_pos + 1 - window) : 0;
+  const int32_t* table_row = block_table + (size_t)seq_rows[t0] * table_stride;
+  const size_t page_stride = (size_t)n_kv_heads * HD * page_size;
+  const float* k_head = k_cache + (size_t)kvh * HD * page_size;
+  const float* v_head = v_cache + (size_t)kvh * HD * page_size;
+
+  f32x4 qf[KG];
+#pragma unroll
+  for (int g = 0; g < KG; ++g)
+    qf[g] = f32_operand(*reinterpret_cast<const f32x4*>(q + (size_t)row * q_stride + (size_t)head * HD + 16 * g + 4 * g4));
+
+  // thread: K row tid / 4 + .., four dims; V^T row, four positions.  What no token of the block has
+  // written or sees reads a place that one does.
+  f32x4 kin[LOADS], vin[LOADS];
+  auto fetch = [&](int p0) {
+#pragma unroll
+    for (int j = 0; j < LOADS; ++j) {
+      const int i = tid + 256 * j;
+      const int p = min(p0 + i / (HD / 4), last_pos);
+      kin[j] = *reinterpret_cast<const f32x4*>(k_head + (size_t)table_row[page_index(p, page_size)] * page_stride +
+                                               (size_t)page_offset(p, page_size) * HD + 4 * (i % (HD / 4)));
+      const int d = i / 16, pv = min(p0 + 4 * (i % 16), last_pos) & ~3;
+      vin[j] = *reinterpret_cast<const f32x4*>(v_head + (size_t)table_row[page_index(pv, page_size)] * page_stride +
+                                               (size_t)d * page_size + page_offset(pv, page_size));
+    }
+  };
+  float M = -INFINITY, L = 0.0f;
+  f32x4 O[DT];
+#pragma unroll
+  for (int d = 0; d < DT; ++d) O[d] = F32_ZERO;
+
+  const int b_end = last_pos / ATT_BLOCK;
+  fetch(from / ATT_BLOCK * ATT_BLOCK);
+  for (int b = from / ATT_BLOCK; b <= b_end; ++b) {
+    const int p0 = b * ATT_BLOCK;
+    const bool whole = p0 >= upto && p0 + ATT_BLOCK - 1 <= first_pos;      // every token sees every position
+    __syncthreads();
+    bool odd = false;
+#pragma unroll
+    for (int j = 0; j < LOADS; ++j) {
+      const int i = tid + 256 * j, c = i % (HD / 4), d = i / 16, c4 = i % 16;
+      float* kd = ks + (i / (HD / 4)) * K_LD + 16 * (c / 4) + c % 4;
+      float* vd = vs + d * V_LD + 16 * (c4 / 4) + c4 % 4;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        kd[4 * e] = kin[j][e];
+        float v = vin[j][e];
+        if (!whole) {
+          const int p = p0 + 4 * c4 + e;
+          v = p >= from && p <= last_pos ? v : 0.0f;
+          odd |= !__builtin_isfinite(v);
+        }
+        vd[4 * e] = v;
+      }
+    }
+    // a value that is not finite, in a block that some tokens see a part of: no products with 0 there
+    const bool spoiled = whole ? (__syncthreads(), false) : __syncthreads_or(odd);
+    if (b < b_end) fetch(p0 + ATT_BLOCK);
+    const bool seen = p0 <= pos && p0 + ATT_BLOCK - 1 >= lo;               // by this lane's token
+    if (!wave_live || !__any(seen)) continue;
+
+    f32x4 s[4] = {F32_ZERO, F32_ZERO, F32_ZERO, F32_ZERO};
+#pragma unroll
+    for (int g = 0; g < KG; ++g) {
+      f32x4 a[4];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) a[t] = *reinterpret_cast<const f32x4*>(&ks[(16 * t + r16) * K_LD + 16 * g + 4 * g4]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) F32_STEP(s[t], a[t], qf[g], i);
+    }
+    float m_b, l_b;
+    f32_weights(s, p0, lo, pos, scale, g4, m_b, l_b);
+    f32x4 o[DT];
+    if (!spoiled) {
+      f32x4 pf[4];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) pf[t] = f32_operand(s[t]);
+#pragma unroll
+      for (int d = 0; d < DT; ++d) o[d] = F32_ZERO;
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int dh = 0; dh < DT; dh += 4) {
+          f32x4 a[4];
+#pragma unroll
+          for (int d = 0; d < 4; ++d) a[d] = *reinterpret_cast<const f32x4*>(&vs[(16 * (dh + d) + r16) * V_LD + 16 * t + 4 * g4]);
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int d = 0; d < 4; ++d) F32_STEP(o[dh + d], a[d], pf[t], i);
+        }
+    } else {
+#pragma unroll
+      for (int d = 0; d < DT; ++d) o[d] = F32_ZERO;
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        for (int g = 0; g < 4; ++g)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int place = 16 * t + 4 * g + e;
+            const float w = __shfl(s[t][e], r16 + 16 * g, AXON_WAVE);
+            if (p0 + place < lo || p0 + place > pos) continue;
+#pragma unroll
+            for (int d = 0; d < DT; ++d)
+#pragma unroll
+              for (int r = 0; r < 4; ++r) o[d][r] = fmaf(w, vs[(16 * d + 4 * g4 + r) * V_LD + 16 * t + 4 * e + g], o[d][r]);
+          }
+    }
+    const float mn = fmaxf(M, m_b), alpha = expf(M - mn), wgt = expf(m_b - mn);
+    if (seen) {
+      L = fmaf(l_b, wgt, L * alpha);
+      M = mn;
+#pragma unroll
+      for (int d = 0; d < DT; ++d)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) O[d][r] = fmaf(o[d][r], wgt, O[d][r] * alpha);
+    }
+  }
+  if (16 * wave + r16 >= n) return;
+  float* orow = out + ((size_t)row * n_heads + head) * HD;
+#pragma unroll
+  for (int d = 0; d < DT; ++d)
+    *reinterpret_cast<f32x4*>(orow + 16 * d + 4 * g4) = f32x4{O[d][0] / L, O[d][1] / L, O[d][2] / L, O[d][3] / L};
+}
+
+// ============================================================================ decoding tokens
+// A wave takes one block of 64 positions of a (token, kv head), with the query heads of the group (up to
+// 16) as the columns; K and V^T go from the pages straight into registers, all 64 KB asked for at
+// once, and (o_b, m_b, l_b) of every head are left in `partial` for the fold (work list and layout as in
+// attention_mfma.hip).  A wave a block of threads: an even spread of the loads over the CUs.  Bound by the wait
+// for the pages: 8 tokens of 16 heads over 2 at 777 positions 64 -> 19 us with the fold, at 2,048 144 -> 17.
+template <int HD>
+__global__ void __launch_bounds__(64, 1)
+attention_f32_decode_kernel(const float* __restrict__ q, int q_stride, const float* __restrict__ k_cache,
+                            const float* __restrict__ v_cache, const int32_t* __restrict__ block_table, int table_stride,
+                            const int32_t* __restrict__ positions, const int32_t* __restrict__ seq_rows,
+                            const int32_t* __restrict__ token_index, int n_tokens, const int32_t* __restrict__ work,
+                            float* __restrict__ partial, int max_chunks, int n_heads, int n_kv_heads, int page_size,
+                            int window, float scale) {
+  constexpr int KG = HD / 16, DT = HD / 16;
+  const int sub = blockIdx.x & 3, unit = blockIdx.x >> 2, lane = threadIdx.x, r16 = lane & 15, g4 = lane >> 4;
+  const int item = work[unit / n_kv_heads];
+  if (item < 0) return;
+  const int slot = item / CMB_MAX_CHUNKS, chunk = item % CMB_MAX_CHUNKS;
+  if (slot >= n_tokens || chunk >= max_chunks) return;
+  const int t = token_index ? token_index[slot] : slot, kvh = unit % n_kv_heads, group = n_heads / n_kv_heads;
+  const int pos = positions[t], lo = window > 0 ? max(0, pos + 1 - window) : 0;
+  const int p0 = lo / DC_CHUNK * DC_CHUNK + chunk * DC_CHUNK + sub * ATT_BLOCK;
+  if (p0 > pos || p0 + ATT_BLOCK - 1 < lo) return;
+  const int32_t* table_row = block_table + (size_t)seq_rows[t] * table_stride;
+  const size_t page_stride = (size_t)n_kv_heads * HD * page_size;
+  const float* k_head = k_cache + (size_t)kvh * HD * page_size;
+  const float* v_head = v_cache + (size_t)kvh * HD * page_size;
+
+  f32x4 kf[4][KG], vf[4][DT], qf[KG];
+  int k_page[4], v_page[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    k_page[i] = table_row[page_index(min(p0 + 16 * i + r16, pos), page_size)];
+    v_page[i] = table_row[page_index(min(p0 + 16 * i + 4 * g4, pos), page_size)];
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float* kr = k_head + (size_t)k_page[i] * page_stride + (size_t)page_offset(min(p0 + 16 * i + r16, pos), page_size) * HD;
+#pragma unroll
+    for (int g = 0; g < KG; ++g) kf[i][g] = *reinterpret_cast<const f32x4*>(kr + 16 * g + 4 * g4);
+  }
+  const float* qrow = q + (size_t)t * q_stride + (size_t)(kvh * group + min(r16, group - 1)) * HD;
+#pragma unroll
+  for (int g = 0; g < KG; ++g) qf[g] = *reinterpret_cast<const f32x4*>(qrow + 16 * g + 4 * g4);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float* vr = v_head + (size_t)v_page[i] * page_stride + (page_offset(min(p0 + 16 * i + 4 * g4, pos), page_size) & ~3);
+#pragma unroll
+    for (int d = 0; d < DT; ++d) vf[i][d] = *reinterpret_cast<const f32x4*>(vr + (size_t)(16 * d + r16) * page_size);
+  }
+
+  f32x4 s[4] = {F32_ZERO, F32_ZERO, F32_ZERO, F32_ZERO};
+#pragma unroll
+  for (int g = 0; g < KG; ++g) {
+    const f32x4 qo = f32_operand(qf[g]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const f32x4 a = f32_operand(kf[i][g]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) F32_STEP(s[i], a, qo, j);
+    }
+  }
+  float m_b, l_b;
+  f32_weights(s, p0, lo, pos, scale, g4, m_b, l_b);
+  // the weight of a position outside the token's range is 0, and so must be what it is multiplied with
+  if (p0 < lo || p0 + ATT_BLOCK - 1 > pos) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int p = p0 + 16 * i + 4 * g4 + e;
+        const bool live = p >= lo && p <= pos;
+#pragma unroll
+        for (int d = 0; d < DT; ++d) vf[i][d][e] = live ? vf[i][d][e] : 0.0f;
+      }
+  }
+  f32x4 o[DT];
+#pragma unroll
+  for (int d = 0; d < DT; ++d) o[d] = F32_ZERO;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const f32x4 pf = f32_operand(s[i]);
+#pragma unroll
+    for (int d = 0; d < DT; ++d) {
+      const f32x4 a = f32_operand(vf[i][d]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) F32_STEP(o[d], a, pf, j);
+    }
+  }
+  if (r16 >= group) return;
+  float* dst = partial + (((size_t)slot * n_heads + kvh * group + r16) * (max_chunks * (DC_CHUNK / ATT_BLOCK)) +
+                          chunk * (DC_CHUNK / ATT_BLOCK) + sub) * (HD + 2);
+#pragma unroll
+  for (int d = 0; d < DT; ++d) {
+    *reinterpret_cast<float2*>(dst + 16 * d + 4 * g4) = make_float2(o[d][0], o[d][1]);
+    *reinterpret_cast<float2*>(dst + 16 * d + 4 * g4 + 2) = make_float2(o[d][2], o[d][3]);
+  }
+  if (g4 == 0) *reinterpret_cast<float2*>(dst + HD) = make_float2(m_b, l_b);
+}
+
+// The fold of a token's blocks in ascending order, thread d dim d.  The factors depend on the maxima
+// alone, so they are worked out for HD blocks at once and only the multiply-adds remain a chain.
+template <int HD>
+__global__ void __launch_bounds__(HD)
+attention_f32_combine_kernel(const float* __restrict__ partial, const int32_t* __restrict__ positions,
+                             const int32_t* __restrict__ token_index, float* __restrict__ out, int max_chunks, int n_heads,
+                             int window) {
+  __shared__ float m_of[HD], l_of[HD], alpha_of[HD], weight_of[HD];
+  const int t = token_index ? token_index[blockIdx.x] : blockIdx.x, head = blockIdx.y, d = threadIdx.x;
+  const int pos = positions[t], lo = window > 0 ? max(0, pos + 1 - window) : 0, first = lo / DC_CHUNK * DC_CHUNK;
+  const int b0 = (lo - first) / ATT_BLOCK, b1 = (pos - first) / ATT_BLOCK;
+  const float* src = partial + ((size_t)blockIdx.x * n_heads + head) * (max_chunks * (DC_CHUNK / ATT_BLOCK)) * (HD + 2);
+  float M = -INFINITY, L = 0.0f, O = 0.0f;
+  for (int g0 = b0; g0 <= b1; g0 += HD) {
+    const int n = min(HD, b1 - g0 + 1);
+    __syncthreads();
+    if (d < n) {
+      m_of[d] = src[(size_t)(g0 + d) * (HD + 2) + HD];
+      l_of[d] = src[(size_t)(g0 + d) * (HD + 2) + HD + 1];
+    }
+    __syncthreads();
+    float before = M;
+    for (int i = 0; i < n; ++i) {
+      if (i < d) before = fmaxf(before, m_of[i]);
+      M = fmaxf(M, m_of[i]);
+    }
+    if (d < n) {
+      const float mn = fmaxf(before, m_of[d]);
+      alpha_of[d] = expf(before - mn);
+      weight_of[d] = expf(m_of[d] - mn);
+    }
+    __syncthreads();
+    int i = 0;
+    for (; i + 15 < n; i += 16) {
+      float o[16];
+#pragma unroll
+      for (int j = 0; j < 16; ++j) o[j] = src[(size_t)(g0 + i + j) * (HD + 2) + d];
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        L = fmaf(l_of[i + j], weight_of[i + j], L * alpha_of[i + j]);
+        O = fmaf(o[j], weight_of[i + j], O * alpha_of[i + j]);
+      }
+    }
+#pragma unroll 4
+    for (; i < n; ++i) {
+      L = fmaf(l_of[i], weight_of[i], L * alpha_of[i]);
+      O = fmaf(src[(size_t)(g0 + i) * (HD + 2) + d], weight_of[i], O * alpha_of[i]);
+    }
+  }
+  out[((size_t)t * n_heads + head) * HD + d] = O / L;
+}
+
+// What attention_f32 takes: the prompt kernel stages pages in fours of positions; the decoding kernel
+// has the heads of a group side by side in 16 columns.
+int attention_f32_ok(int head_dim, int page_size, int n_heads, int n_kv_heads) {
+  return (head_dim == 64 || head_dim == 128) && page_size >= 4 && (page_size & (page_size - 1)) == 0 && n_kv_heads > 0 &&
+         n_heads % n_kv_heads == 0 && n_heads / n_kv_heads <= 16;
+}
+
+int launch_attention_f32_prefill(const float* q, int q_stride, const float* k_cache, const float* v_cache,
+                                 const int32_t* block_table, int table_stride, const int32_t* positions,
+                                 const int32_t* seq_rows, float* out, const int32_t* tiles, int n_tiles, int n_heads,
+                                 int n_kv_heads, int head_dim, int page_size, int window, float scale, hipStream_t stream) {
+#define LAUNCH(HD)                                                                                                   \
+  {                                                                                                                  \
+    constexpr int lds = (ATT_BLOCK * (HD + 4) + HD * (ATT_BLOCK + 4)) * (int)sizeof(float);                          \
+    static bool configured = lds <= 48 * 1024;                                                                       \
+    if (!configured) {                                                                                               \
+      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attention_f32_prefill_kernel<HD>),           \
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, lds);                           \
+      if (e != hipSuccess) {                                                                                         \
+        axk_set_error("attention_prefill: cannot reserve %d bytes of LDS: %s", lds, hipGetErrorString(e));           \
+        return -2;                                                                                                   \
+      }                                                                                                              \
+      configured = true;                                                                                             \
+    }                                                                                                                \
+    attention_f32_prefill_kernel<HD><<<dim3(n_tiles, n_heads, 4), 256, lds, stream>>>(                               \
+        q, q_stride, k_cache, v_cache, block_table, table_stride, positions, seq_rows, out, tiles, n_heads,          \
+        n_kv_heads, page_size, window, scale);                                                                       \
+  }
+  if (head_dim == 64) LAUNCH(64) else LAUNCH(128)
+#undef LAUNCH
+  AXK_LAUNCH_CHECK("attention_prefill");
+  return 0;
+}
+
+int launch_attention_f32_decode(const float* q, int q_stride, const float* k_cache, const float* v_cache,
+                                const int32_t* block_table, int table_stride, const int32_t* positions,
+                                const int32_t* seq_rows, float* out, const int32_t* token_index, int n_tokens,
+                                const int32_t* work, int n_work, float* partial, int max_chunks, int n_heads,
+                                int n_kv_heads, int head_dim, int page_size, int window, float scale, hipStream_t stream) {
+#define LAUNCH(HD)                                                                                                   \
+  {                                                                                                                  \
+    attention_f32_decode_kernel<HD><<<(unsigned)n_work * n_kv_heads * 4, 64, 0, stream>>>(                           \
+        q, q_stride, k_cache, v_cache, block_table, table_stride, positions, seq_rows, token_index, n_tokens, work,  \
+        partial, max_chunks, n_heads, n_kv_heads, page_size, window, scale);                                         \
+    attention_f32_combine_kernel<HD><<<dim3(n_tokens, n_heads), HD, 0, stream>>>(partial, positions, token_index, out, \
+                                                                                 max_chunks, n_heads, window);       \
+  }
+  if (head_dim == 64) LAUNCH(64) else LAUNCH(128)
+#undef LAUNCH
+  AXK_LAUNCH_CHECK("attention_decode");
+  return 0;
+}
+
+#endif  // !AXON_BF16

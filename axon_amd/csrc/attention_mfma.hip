@@ -856,6 +856,20 @@ attention_combine_kernel(const float* __restrict__ partial, const int32_t* __res
 
 #endif  // AXON_BF16
 
+#if !AXON_BF16
+// the float32 build's kernels behind the same entry points (attention_f32.hip)
+int attention_f32_ok(int head_dim, int page_size, int n_heads, int n_kv_heads);
+int launch_attention_f32_prefill(const float* q, int q_stride, const float* k_cache, const float* v_cache,
+                                 const int32_t* block_table, int table_stride, const int32_t* positions,
+                                 const int32_t* seq_rows, float* out, const int32_t* tiles, int n_tiles, int n_heads,
+                                 int n_kv_heads, int head_dim, int page_size, int window, float scale, hipStream_t stream);
+int launch_attention_f32_decode(const float* q, int q_stride, const float* k_cache, const float* v_cache,
+                                const int32_t* block_table, int table_stride, const int32_t* positions,
+                                const int32_t* seq_rows, float* out, const int32_t* token_index, int n_tokens,
+                                const int32_t* work, int n_work, float* partial, int max_chunks, int n_heads,
+                                int n_kv_heads, int head_dim, int page_size, int window, float scale, hipStream_t stream);
+#endif
+
 // ============================================================================ entry points
 // 1 if the MFMA attention kernels take this head size, page size and group of heads.
 extern "C" int axk_attention_fast_ok(int head_dim, int page_size, int n_heads, int n_kv_heads) {
@@ -868,18 +882,27 @@ extern "C" int axk_attention_fast_ok(int head_dim, int page_size, int n_heads, i
 #endif
 }
 
+// 1 if axk_attention_prefill and axk_attention_decode take these sizes in this build.
+extern "C" int axk_attention_blocks_ok(int head_dim, int page_size, int n_heads, int n_kv_heads) {
+#if AXON_BF16
+  return axk_attention_fast_ok(head_dim, page_size, n_heads, n_kv_heads);
+#else
+  return attention_f32_ok(head_dim, page_size, n_heads, n_kv_heads);
+#endif
+}
+
 extern "C" int axk_attention_prefill(const void* q, int q_stride, const void* k_cache, const void* v_cache,
                                      const int32_t* block_table, int table_stride, const int32_t* positions,
                                      const int32_t* seq_rows, void* out, const int32_t* tiles, int n_tiles, int n_heads,
                                      int n_kv_heads, int head_dim, int page_size, int window, float scale, void* stream) {
-#if AXON_BF16
-  AXK_REQUIRE(axk_attention_fast_ok(head_dim, page_size, n_heads, n_kv_heads),
+  AXK_REQUIRE(axk_attention_blocks_ok(head_dim, page_size, n_heads, n_kv_heads),
               "attention_prefill: head_dim %d, page size %d, %d/%d heads are not taken by this kernel", head_dim,
               page_size, n_heads, n_kv_heads);
   AXK_REQUIRE(n_tiles >= 0 && n_heads <= 65535 && window >= 0 && q_stride % 8 == 0 && ((uintptr_t)q & 15) == 0,
               "attention_prefill: bad arguments (tiles %d, heads %d, window %d, q stride %d)", n_tiles, n_heads, window,
               q_stride);
   if (n_tiles == 0) return 0;
+#if AXON_BF16
   const int group = n_heads / n_kv_heads;
 #define LAUNCH_PAGED(HD, HPB, ONE_PAGE)                                                                             \
   {                                                                                                                 \
@@ -916,8 +939,9 @@ extern "C" int axk_attention_prefill(const void* q, int q_stride, const void* k_
   AXK_LAUNCH_CHECK("attention_prefill");
   return 0;
 #else
-  axk_set_error("attention_prefill: only in the bfloat16 build");
-  return -1;
+  return launch_attention_f32_prefill((const float*)q, q_stride, (const float*)k_cache, (const float*)v_cache, block_table,
+                                      table_stride, positions, seq_rows, (float*)out, tiles, n_tiles, n_heads, n_kv_heads,
+                                      head_dim, page_size, window, scale, (hipStream_t)stream);
 #endif
 }
 
@@ -940,8 +964,7 @@ extern "C" int axk_attention_decode(const void* q, int q_stride, const void* k_c
                                     const int32_t* work, int n_work, float* partial, int max_chunks, int n_heads,
                                     int n_kv_heads, int head_dim, int page_size, int window, float scale,
                                     void* stream) {
-#if AXON_BF16
-  AXK_REQUIRE(axk_attention_fast_ok(head_dim, page_size, n_heads, n_kv_heads),
+  AXK_REQUIRE(axk_attention_blocks_ok(head_dim, page_size, n_heads, n_kv_heads),
               "attention_decode: head_dim %d, page size %d, %d/%d heads are not taken by this kernel", head_dim,
               page_size, n_heads, n_kv_heads);
   AXK_REQUIRE(max_chunks <= CMB_MAX_CHUNKS, "attention_decode: %d chunks of %d positions (at most %d: %d positions)",
@@ -954,6 +977,7 @@ extern "C" int axk_attention_decode(const void* q, int q_stride, const void* k_c
   AXK_REQUIRE(n_work >= 0 && (n_work == 0 || work != nullptr) && (long)n_work * n_kv_heads * 4 < (1l << 31),
               "attention_decode: a work list of %d items", n_work);
   if (n_tokens == 0 || n_work == 0) return 0;
+#if AXON_BF16
   // A wave a block where every wave finds a place on the chip at once (ten a CU): an even spread
   // over the CUs; blocks of four waves where there are more, which are launched faster.
   const bool single = (long)n_work * n_kv_heads * 4 <= 2560;
@@ -985,7 +1009,9 @@ extern "C" int axk_attention_decode(const void* q, int q_stride, const void* k_c
   AXK_LAUNCH_CHECK("attention_decode");
   return 0;
 #else
-  axk_set_error("attention_decode: only in the bfloat16 build");
-  return -1;
+  return launch_attention_f32_decode((const float*)q, q_stride, (const float*)k_cache, (const float*)v_cache, block_table,
+                                     table_stride, positions, seq_rows, (float*)out, token_index, n_tokens, work, n_work,
+                                     partial, max_chunks, n_heads, n_kv_heads, head_dim, page_size, window, scale,
+                                     (hipStream_t)stream);
 #endif
 }

@@ -161,7 +161,7 @@ gemm_fma_kernel(const elem_t* __restrict__ x, int x_stride, const elem_t* __rest
 __device__ inline f32x4 fma_operand(const float (&v)[4]) {
   unsigned r[4];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) r[j] = __builtin_bit_cast(unsigned, v[j]);
+  for (int j = 0; j < 4; ++j) r[j] = __float_as_uint(v[j]);
 #pragma unroll
   for (int j = 0; j < 4; j += 2) {
     const auto s = __builtin_amdgcn_permlane16_swap(r[j], r[j + 1], false, false);

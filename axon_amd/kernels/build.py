@@ -30,7 +30,7 @@ from typing import List
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "csrc")
 ARCH = "gfx950"
 
-KERNEL_SOURCES = ["elementwise.hip", "gemm.hip", "gemm_mfma.hip", "attention.hip", "attention_mfma.hip",
+KERNEL_SOURCES = ["elementwise.hip", "gemm.hip", "gemm_mfma.hip", "attention.hip", "attention_mfma.hip", "attention_f32.hip",
                   "sampling.hip", "grouped_gemm.hip", "recurrent.hip", "state_space.hip", "time_mix.hip", "delta_rule.hip",
                   "linear_attention.hip", "stream.hip", "latent_attention.hip", "masked_attention.hip", "moe.hip", "instances.hip",
                   "support.hip"]

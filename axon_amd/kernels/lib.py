@@ -60,6 +60,7 @@ _SIGNATURES = {
                              c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,
                              c_float, c_void_p],
     "axk_attention_fast_ok": [c_int, c_int, c_int, c_int],
+    "axk_attention_blocks_ok": [c_int, c_int, c_int, c_int],
     "axk_gemm": [c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p,
                  ctypes.c_long, c_void_p],
     "axk_pack_ok": [c_int, c_int, c_int],
@@ -495,6 +496,11 @@ class Kernels:
     def attention_fast_ok(self, head_dim: int, page_size: int, n_heads: int, n_kv_heads: int) -> bool:
         """Whether the matrix-core attention kernels take these sizes (never in float32)."""
         return bool(self.lib.axk_attention_fast_ok(head_dim, page_size, n_heads, n_kv_heads))
+
+    def attention_blocks_ok(self, head_dim: int, page_size: int, n_heads: int, n_kv_heads: int) -> bool:
+        """Whether `attention_prefill` and `attention_decode` take these sizes in this build (float32: on the
+        32-bit matrix cores, with the bits of `attention`)."""
+        return bool(self.lib.axk_attention_blocks_ok(head_dim, page_size, n_heads, n_kv_heads))
 
     def attention_prefill(self, q, q_stride, k_cache, v_cache, block_table, positions, seq_rows, out, tiles, n_heads,
                           n_kv_heads, head_dim, page_size, window, scale) -> torch.Tensor:

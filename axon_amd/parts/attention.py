@@ -188,7 +188,7 @@ class GQAttention(Mixer):
         self.decode_chunk = rt.k.attention_decode_chunk
         self._work_list = rt.k.attention_decode_work
         self._max_context = rt.k.attention_decode_max_context
-        if rt.k.attention_fast_ok(self.hd, 64, self.nh, self.nkv):
+        if rt.k.attention_blocks_ok(self.hd, 64, self.nh, self.nkv):
             self._workspace = rt.k.attention_decode_workspace
         self.w_qkv = rt.k.prepare_weight(store.fused_matrix([self.n[k] + ".weight" for k in ("q", "k", "v")]))
         biases = [store.vector(self.n[k] + ".bias", optional=True) for k in ("q", "k", "v")] if self.qkv_bias else []
@@ -248,7 +248,7 @@ class GQAttention(Mixer):
             k.gemm(h, w, qkv[:, :w.shape[0]], bias, MODE_STORE)
             k.rope_kv_write(qkv, table, ctx.positions, ctx.seq_rows, *cache, rotary, group.page_size, binding.writes)
         att = ctx.ws.take((T, self.q_dim), ctx.rt.dtype)
-        if k.attention_fast_ok(self.hd, group.page_size, self.nh, self.nkv):
+        if k.attention_blocks_ok(self.hd, group.page_size, self.nh, self.nkv):
             plan = attention_plan(ctx, self.window, self.nh, self.hd)
             common = (k_cache, v_cache, group.block_table, ctx.positions, ctx.seq_rows, att)
             sizes = (self.nh, self.nkv, self.hd, group.page_size, self.window, self.scale)

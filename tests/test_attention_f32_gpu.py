@@ -1,0 +1,59 @@
+"""The float32 build's prompt and decoding attention on the matrix cores: the bits of `attention`, whatever the head
+size, group, page size, window and cut; values that are not finite reach only the tokens that see them."""
+import pytest
+import torch
+
+from axon_amd.kernels import kernels
+from gpu_helpers import paged_cache
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(nh, nkv, hd, page, T, window, spoil=None):
+    g = torch.Generator().manual_seed(T + hd)
+    q, keys, vals = (torch.randn(T, n, hd, generator=g) for n in (nh, nkv, nkv))
+    if spoil is not None:
+        vals[spoil, :, 3] = float("inf")
+        vals[spoil, :, 5] = float("nan")
+    kc, vc, table = paged_cache(keys, vals, page, "float32")
+    q, pos, rows = q.cuda().view(T, nh * hd), torch.arange(T, dtype=torch.int32).cuda(), torch.zeros(T, dtype=torch.int32).cuda()
+    want = torch.empty_like(q)
+    k = kernels("float32")
+    sizes = (nh, nkv, hd, page, window, hd ** -0.5)
+    k.attention(q, nh * hd, kc, vc, table, pos, rows, want, *sizes)
+    return k, q, (kc, vc, table, pos, rows), sizes, want
+
+
+def _same(a, b):
+    return torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(7.0), b.nan_to_num(7.0))
+
+
+@pytest.mark.parametrize("nh,nkv,hd,page,T,window", [(2, 2, 64, 4, 1, 0), (4, 1, 64, 8, 65, 0), (7, 1, 128, 16, 130, 0),
+                                                     (16, 1, 64, 64, 63, 40), (8, 4, 128, 128, 300, 70), (6, 2, 128, 64, 257, 64),
+                                                     (2, 1, 64, 32, 400, 0)])
+@pytest.mark.parametrize("spoiled", [False, True])
+def test_prompts_and_decoding_have_the_bits_of_the_rows_kernel(nh, nkv, hd, page, T, window, spoiled):
+    k, q, cache, sizes, want = _case(nh, nkv, hd, page, T, window, T * 2 // 3 if spoiled else None)
+    assert k.attention_blocks_ok(hd, page, nh, nkv)
+    for cut in (128, 77):                                   # runs of up to 128 tokens; two runs a block
+        tiles = [(a, min(cut, T - a)) for a in range(0, T, cut)]
+        pairs = [tiles[i] + (tiles[i + 1] if i + 1 < len(tiles) else (0, 0)) for i in range(0, len(tiles), 2)]
+        out = torch.full_like(q, 5.0)
+        k.attention_prefill(q, nh * hd, *cache, out, torch.tensor(pairs, dtype=torch.int32).cuda(), *sizes)
+        assert _same(out, want), cut
+    chunks = -(-T // k.attention_decode_chunk) + 1
+    partial = torch.full((k.attention_decode_workspace(T, nh, hd, chunks),), float("nan"), device="cuda")
+    out = torch.full_like(q, 5.0)
+    k.attention_decode(q, nh * hd, *cache, out, T, partial, chunks, *sizes)
+    assert _same(out, want)
+    pick = torch.tensor(sorted({T - 1, 0}, reverse=True), dtype=torch.int32).cuda()
+    out2 = torch.full_like(q, 5.0)
+    k.attention_decode(q, nh * hd, *cache, out2, pick, partial, chunks, *sizes)
+    assert _same(out2[T - 1], want[T - 1]) and _same(out2[0], want[0])
+
+
+def test_what_it_takes():
+    k = kernels("float32")
+    assert not k.attention_blocks_ok(80, 16, 4, 2) and not k.attention_blocks_ok(128, 2, 4, 2)
+    assert not k.attention_blocks_ok(128, 24, 4, 2) and not k.attention_blocks_ok(128, 16, 34, 2)
+    assert kernels("bfloat16").attention_blocks_ok(128, 16, 34, 2) == kernels("bfloat16").attention_fast_ok(128, 16, 34, 2)
