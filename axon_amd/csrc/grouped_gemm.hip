@@ -35,6 +35,7 @@ struct GroupedArgs {
   int glu; float glu_limit; float glu_alpha; float glu_shift;
   const int32_t* tiles; const int32_t* n_tiles;
   int M, N, K, G;
+  bool vec_out;                         // four neighbouring outputs are one aligned store
 };
 
 #define GG_ROWS 16
@@ -51,7 +52,7 @@ __device__ inline float clamped_glu(float gate, float up, float limit, float alp
   return (g * (1.0f / (1.0f + expf(-(alpha * g))))) * (u + shift);
 }
 
-__device__ inline void gg_store(const GroupedArgs& a, int g, int orow, int n, float v, float up) {
+__device__ inline float gg_value(const GroupedArgs& a, int g, int orow, int n, float v, float up) {
   if (a.row_scale) {                    // the row of X counts row_scale[orow] times: the product is linear in it
     const float w = a.row_scale[orow];
     v *= w;
@@ -63,9 +64,13 @@ __device__ inline void gg_store(const GroupedArgs& a, int g, int orow, int n, fl
     if (a.glu) up += load_vec(a.bias, a.bias_is_f32, g * per + a.N + n);
   }
   if (a.glu) v = clamped_glu(v, up, a.glu_limit, a.glu_alpha, a.glu_shift);
-  const long col = (long)g * a.out_group_stride + n;
-  if (a.gate) v = v * (1.0f / (1.0f + expf(-a.gate[(long)orow * a.gate_row_stride + (a.gate_per_group ? g : col)])));
-  const long at = (long)orow * a.out_row_stride + col;
+  if (a.gate) v = v * (1.0f / (1.0f + expf(-a.gate[(long)orow * a.gate_row_stride + (a.gate_per_group ? g : (long)g * a.out_group_stride + n)])));
+  return v;
+}
+
+__device__ inline void gg_store(const GroupedArgs& a, int g, int orow, int n, float v, float up) {
+  v = gg_value(a, g, orow, n, v, up);
+  const long at = (long)orow * a.out_row_stride + (long)g * a.out_group_stride + n;
   if (a.out_is_f32) ((float*)a.out)[at] = v;
   else ((elem_t*)a.out)[at] = from_float(v);
 }
@@ -152,19 +157,31 @@ typedef __attribute__((ext_vector_type(4))) float gg_f32x4;
 
 __device__ inline gg_bf16x8 gg_frag(uint4 v) { return __builtin_bit_cast(gg_bf16x8, v); }
 
-__device__ inline uint4 gg_x_frag(const GroupedArgs& a, long at, bool ok) {
-  if (!ok) return make_uint4(0, 0, 0, 0);
-  if (!a.x_is_f32) return *reinterpret_cast<const uint4*>((const bf16_t*)a.x + at);
-  const float4 lo = *reinterpret_cast<const float4*>((const float*)a.x + at);
-  const float4 hi = *reinterpret_cast<const float4*>((const float*)a.x + at + 4);
-  return make_uint4(pack2_bf16(lo.x, lo.y), pack2_bf16(lo.z, lo.w), pack2_bf16(hi.x, hi.y), pack2_bf16(hi.z, hi.w));
+// Columns n .. n + 3 of a row (what a lane holds of a product).
+__device__ inline void gg_store4(const GroupedArgs& a, int g, int orow, int n, const gg_f32x4& v, const gg_f32x4& up) {
+  if (!a.vec_out || n + 4 > a.N) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      if (n + c < a.N) gg_store(a, g, orow, n + c, v[c], up[c]);
+    return;
+  }
+  float r[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) r[c] = gg_value(a, g, orow, n + c, v[c], up[c]);
+  const long at = (long)orow * a.out_row_stride + (long)g * a.out_group_stride + n;
+  if (a.out_is_f32) *reinterpret_cast<float4*>((float*)a.out + at) = make_float4(r[0], r[1], r[2], r[3]);
+  else *reinterpret_cast<uint2*>((bf16_t*)a.out + at) = make_uint2(pack2_bf16(r[0], r[1]), pack2_bf16(r[2], r[3]));
 }
 
 // 16 rows x 64 columns a block of four waves, a wave 16 columns: W rows as the MFMA's first
 // operand, X rows as its second, both straight from memory (lane l holds row l % 16, the eight k
-// from 8 (l / 16)); lane l ends with row l % 16 of the columns 4 (l / 16) .. + 3.  Four steps of
-// 32 k are asked for before the first is multiplied.
-template <bool GLU>
+// from 8 (l / 16)); lane l ends with row l % 16 of the columns 4 (l / 16) .. + 3.  Such a product waits for W
+// alone, and an output is one chain over k, so a wave keeps GG_RING steps of 32 k under way: each is asked
+// for again as soon as it is multiplied.  Rows and columns that do not exist read ones that do.  The 32 pairs
+// of 8 tokens over 32 experts of [1,408, 2,048] and [2,048, 704]: 42 and 19 us, launches included (120 and 45 with four steps
+// asked for at a time and waited for together).
+#define GG_RING 8
+template <bool GLU, bool XF32>
 __global__ void __launch_bounds__(256) grouped_gemm_mfma_kernel(GroupedArgs a) {
   int g, first, count;
   if (!gg_tile(a, g, first, count)) return;
@@ -172,138 +189,213 @@ __global__ void __launch_bounds__(256) grouped_gemm_mfma_kernel(GroupedArgs a) {
   const int n0 = blockIdx.y * GG_COLS + wave * 16;
   if (n0 >= a.N) return;
   const int r = lane & 15, kq = (lane >> 4) * 8;
-  const bool row_ok = r < count;
   const int rr = first + min(r, count - 1);
   const int xr = a.x_rows ? a.x_rows[rr] : rr;
   const int orow = a.out_rows ? a.out_rows[rr] : rr;
   const long x_at = (long)xr * a.x_row_stride + (long)g * a.x_group_stride + kq;
   const int w_rows = GLU ? 2 * a.N : a.N;
-  const bool col_ok = n0 + r < a.N;
   const bf16_t* wrow = a.w + ((long)g * w_rows + min(n0 + r, a.N - 1)) * a.K + kq;
   const bf16_t* urow = wrow + (long)a.N * a.K;
   gg_f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f}, acc_up = {0.0f, 0.0f, 0.0f, 0.0f};
-  const uint4 zero = make_uint4(0, 0, 0, 0);
+  uint4 xf[GG_RING][XF32 ? 2 : 1], wf[GG_RING], uf[GLU ? GG_RING : 1];
+  auto ask = [&](int s, int k) {
+    if (XF32) {
+      xf[s][0] = *reinterpret_cast<const uint4*>((const float*)a.x + x_at + k);
+      xf[s][XF32 ? 1 : 0] = *reinterpret_cast<const uint4*>((const float*)a.x + x_at + k + 4);
+    } else {
+      xf[s][0] = *reinterpret_cast<const uint4*>((const bf16_t*)a.x + x_at + k);
+    }
+    wf[s] = *reinterpret_cast<const uint4*>(wrow + k);
+    if (GLU) uf[GLU ? s : 0] = *reinterpret_cast<const uint4*>(urow + k);
+  };
+  auto multiply = [&](int s) {
+    uint4 x = xf[s][0];
+    if (XF32) {
+      const float4 lo = __builtin_bit_cast(float4, xf[s][0]), hi = __builtin_bit_cast(float4, xf[s][XF32 ? 1 : 0]);
+      x = make_uint4(pack2_bf16(lo.x, lo.y), pack2_bf16(lo.z, lo.w), pack2_bf16(hi.x, hi.y), pack2_bf16(hi.z, hi.w));
+    }
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gg_frag(wf[s]), gg_frag(x), acc, 0, 0, 0);
+    if (GLU) acc_up = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gg_frag(uf[GLU ? s : 0]), gg_frag(x), acc_up, 0, 0, 0);
+  };
+  // (a step behind the last asks for the last again: a branch would have every load under way waited for)
+#pragma unroll
+  for (int s = 0; s < GG_RING; ++s) ask(s, min(32 * s, a.K - 32));
   int k0 = 0;
-  for (; k0 + 128 <= a.K; k0 += 128) {
-    uint4 xf[4], wf[4], uf[4];
+  for (; k0 + 32 * GG_RING <= a.K; k0 += 32 * GG_RING) {
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      xf[s] = gg_x_frag(a, x_at + k0 + 32 * s, row_ok);
-      wf[s] = col_ok ? *reinterpret_cast<const uint4*>(wrow + k0 + 32 * s) : zero;
-      if (GLU) uf[s] = col_ok ? *reinterpret_cast<const uint4*>(urow + k0 + 32 * s) : zero;
-    }
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gg_frag(wf[s]), gg_frag(xf[s]), acc, 0, 0, 0);
-      if (GLU) acc_up = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gg_frag(uf[s]), gg_frag(xf[s]), acc_up, 0, 0, 0);
+    for (int s = 0; s < GG_RING; ++s) {
+      multiply(s);
+      ask(s, min(k0 + 32 * (GG_RING + s), a.K - 32));
     }
   }
-  for (; k0 < a.K; k0 += 32) {
-    const uint4 xf = gg_x_frag(a, x_at + k0, row_ok);
-    const uint4 wf = col_ok ? *reinterpret_cast<const uint4*>(wrow + k0) : zero;
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gg_frag(wf), gg_frag(xf), acc, 0, 0, 0);
-    if (GLU) {
-      const uint4 uf = col_ok ? *reinterpret_cast<const uint4*>(urow + k0) : zero;
-      acc_up = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gg_frag(uf), gg_frag(xf), acc_up, 0, 0, 0);
-    }
-  }
-  if (!row_ok) return;
 #pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    const int n = n0 + (lane >> 4) * 4 + c;
-    if (n < a.N) gg_store(a, g, orow, n, acc[c], acc_up[c]);
-  }
+  for (int s = 0; s < GG_RING; ++s)
+    if (k0 + 32 * s < a.K) multiply(s);
+  if (r >= count) return;
+  gg_store4(a, g, orow, n0 + (lane >> 4) * 4, acc, acc_up);
 }
+
 // Many rows a group (a long prompt's pairs of an expert, the tokens of a prompt through a block of
-// channels): tiles of 64 rows x 128 rows of W through LDS.  Four waves, two by two, each 32 rows x 64
-// rows of W (2 x 4 products a step of 32 k); the next step's operands are asked for while this one is
-// multiplied.  With the gated epilogue a block's 128 rows of W are 64 gate rows and the 64 up rows of
-// the same columns, and a wave holds both of a column.  The chain of an output is the one of the
-// kernel above (16x16x32 products in ascending k), so which of the two runs changes no bit.
+// channels): 64 rows x 256 rows of W a block, through two stages of 64 k of LDS that are filled by direct loads
+// (X in float32: through registers, where it is rounded).  Four waves, each the 64 rows x 64 rows of W
+// (4 x 4 products a step of 32 k); with the gated epilogue a wave's 64 rows of W are 32 gate rows and the 32
+// up rows of the same columns.  The next stage is on its way while this one is multiplied, and the two halves
+// of a stage are read one ahead of the products.  Rows of a stage are 128 bytes, their 16-byte slots permuted by
+// slot ^ (row / 2 % 8): the 16 rows a read takes at a time fall into 16 different slots of the 64 banks.  Bound by the
+// way into LDS and out of it (80 bytes a cycle in, 128 out at the matrix cores' full rate).  The chain of an
+// output is the one of the kernel above (16x16x32 products in ascending k), so which of the two runs changes no
+// bit.  2,048 tokens, 4 of 32 experts of [1,408, 2,048] and [2,048, 704]: 84 and 75 us (163 and 113 with stages of 32 k
+// through registers and 128 rows of W).
 #define GT_ROWS 64
-#define GT_WROWS 128
-template <bool GLU>
-__global__ void __launch_bounds__(256) grouped_gemm_tile_kernel(GroupedArgs a) {
-  __shared__ __align__(16) bf16_t xs[GT_ROWS * 32];
-  __shared__ __align__(16) bf16_t ws[GT_WROWS * 32];
-  __shared__ int xrow[GT_ROWS], orow[GT_ROWS];
+#define GT_BK 64
+#define GT_STAGE(wrows) ((GT_ROWS + (wrows)) * GT_BK * 2)
+typedef const __attribute__((address_space(1))) void* gg_global_t;
+typedef __attribute__((address_space(3))) void* gg_lds_t;
+template <bool GLU, bool XF32, int WROWS>
+__global__ void __launch_bounds__(256, 2) grouped_gemm_tile_kernel(GroupedArgs a) {
+  static_assert(WROWS == 256 || (WROWS == 128 && !GLU), "a wave's 64 rows of W, for all or for half of the rows of X");
+  constexpr int STAGE = GT_STAGE(WROWS), XT = WROWS / 64, WL = WROWS / 32;   // tiles of 16 rows a wave, load instructions of W a wave
+  extern __shared__ __align__(256) unsigned char stages[];        // [2]: X [64][64], W [WROWS][64]
+  constexpr int COLS = GLU ? WROWS / 2 : WROWS;
+  // Blocks go to the eight XCDs in turn: each XCD gets a run of neighbours of the list [group, columns, rows]
+  // (routed: [columns, tile]), so that the tiles of a group that read the same rows of W do so through one L2.
+  const int col_tiles = (a.N + COLS - 1) / COLS, row_tiles = a.tiles ? *a.n_tiles : (a.M + GT_ROWS - 1) / GT_ROWS;
+  const long total = (long)row_tiles * col_tiles * (a.tiles ? 1 : a.G), share = (total + 7) / 8;
+  const long item = (long)(blockIdx.x % 8) * share + blockIdx.x / 8;
+  if ((long)(blockIdx.x / 8) >= share || item >= total) return;
+  const int row_tile = (int)(item % row_tiles), n0 = (int)(item / row_tiles % col_tiles) * COLS;
   int g, first, count;
   if (a.tiles) {
-    if ((int)blockIdx.x >= *a.n_tiles) return;
-    g = a.tiles[3 * blockIdx.x]; first = a.tiles[3 * blockIdx.x + 1]; count = a.tiles[3 * blockIdx.x + 2];
+    g = a.tiles[3 * row_tile]; first = a.tiles[3 * row_tile + 1]; count = a.tiles[3 * row_tile + 2];
   } else {
-    g = blockIdx.z; first = blockIdx.x * GT_ROWS; count = min(GT_ROWS, a.M - first);
+    g = (int)(item / row_tiles / col_tiles); first = row_tile * GT_ROWS; count = min(GT_ROWS, a.M - first);
   }
   if (count <= 0) return;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wr = wave >> 1, wc = wave & 1;
-  const int n0 = blockIdx.y * (GLU ? 64 : 128);
-  if (tid < GT_ROWS) {
-    const int r = first + min(tid, count - 1);
-    xrow[tid] = a.x_rows ? a.x_rows[r] : r;
-    orow[tid] = a.out_rows ? a.out_rows[r] : r;
-  }
-  __syncthreads();
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int w_rows = GLU ? 2 * a.N : a.N;
   const bf16_t* wg = a.w + (long)g * w_rows * a.K;
-  // staging: a thread brings 16 bytes of one row of X and of two rows of W a step
-  const int srow = tid >> 2, sk = (tid & 3) * 8;
-  const bool x_ok = srow < count;
-  const long x_at = (long)xrow[srow] * a.x_row_stride + (long)g * a.x_group_stride + sk;
-  const bf16_t* wsrc[2];
-  bool w_ok[2];
+  // a load instruction fills 8 rows: lane l row l / 8, slot l % 8.  A wave brings WROWS / 4 rows of W and 16 of X.
+  const int lrow = lane >> 3, lslot = lane & 7;
+  const int w_wave = WROWS == 256 ? wave : wave & 1, x_wave = WROWS == 256 ? 0 : 32 * (wave >> 1);   // what it multiplies
+  long w_at[WL];
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int slot = srow + 64 * h;
-    const int col = GLU ? n0 + srow : n0 + slot;
-    w_ok[h] = col < a.N;
-    wsrc[h] = wg + (long)((GLU && h) ? a.N + min(col, a.N - 1) : min(col, a.N - 1)) * a.K + sk;
+  for (int i = 0; i < WL; ++i) {
+    const int place = 8 * i + lrow;
+    const int col = GLU ? n0 + 32 * wave + (place & 31) : n0 + 8 * WL * wave + place;
+    w_at[i] = (long)(min(col, a.N - 1) + (GLU && place >= 32 ? a.N : 0)) * a.K + 8 * (lslot ^ (4 * (i & 1) + (lane >> 4)));
   }
-  const uint4 zero = make_uint4(0, 0, 0, 0);
-  uint4 px = gg_x_frag(a, x_at, x_ok), pw0 = w_ok[0] ? *reinterpret_cast<const uint4*>(wsrc[0]) : zero,
-        pw1 = w_ok[1] ? *reinterpret_cast<const uint4*>(wsrc[1]) : zero;
-  gg_f32x4 acc[2][4];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = gg_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  const int fr = lane & 15, fk = (lane >> 4) * 8;
-  for (int k0 = 0; k0 < a.K; k0 += 32) {
-    *reinterpret_cast<uint4*>(&xs[srow * 32 + sk]) = px;
-    *reinterpret_cast<uint4*>(&ws[srow * 32 + sk]) = pw0;
-    *reinterpret_cast<uint4*>(&ws[(srow + 64) * 32 + sk]) = pw1;
-    __syncthreads();
-    if (k0 + 32 < a.K) {
-      px = gg_x_frag(a, x_at + k0 + 32, x_ok);
-      pw0 = w_ok[0] ? *reinterpret_cast<const uint4*>(wsrc[0] + k0 + 32) : zero;
-      pw1 = w_ok[1] ? *reinterpret_cast<const uint4*>(wsrc[1] + k0 + 32) : zero;
-    }
-    uint4 xf[2], wf[4];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) xf[i] = *reinterpret_cast<const uint4*>(&xs[(32 * wr + 16 * i + fr) * 32 + fk]);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int slot = GLU ? (j < 2 ? 32 * wc + 16 * j : 64 + 32 * wc + 16 * (j - 2)) : 64 * wc + 16 * j;
-      wf[j] = *reinterpret_cast<const uint4*>(&ws[(slot + fr) * 32 + fk]);
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(gg_frag(wf[j]), gg_frag(xf[i]), acc[i][j], 0, 0, 0);
-    __syncthreads();
-  }
+  long x_at[2];
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
-    const int r = 32 * wr + 16 * i + fr;
+    const int r = first + min(16 * wave + 8 * i + lrow, count - 1);
+    x_at[i] = (long)(a.x_rows ? a.x_rows[r] : r) * a.x_row_stride + (long)g * a.x_group_stride + 8 * (lslot ^ (4 * (i & 1) + (lane >> 4)));
+  }
+  // the last 32 k of a K that is no multiple of 64: the slots behind them bring the ones before again (not used)
+  auto tail = [&](int k0, int i) {
+    const int chunk = lslot ^ (4 * (i & 1) + (lane >> 4));
+    return k0 + GT_BK > a.K && chunk >= 4 ? k0 - 32 : k0;
+  };
+  uint4 held[XF32 ? 4 : 1];
+  auto ask = [&](int k0, int which) {
+    unsigned char* st = stages + which * STAGE;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      if (XF32) {
+        const float* src = (const float*)a.x + x_at[i] + tail(k0, i);
+        held[XF32 ? 2 * i : 0] = *reinterpret_cast<const uint4*>(src);
+        held[XF32 ? 2 * i + 1 : 0] = *reinterpret_cast<const uint4*>(src + 4);
+      } else {
+        __builtin_amdgcn_global_load_lds((gg_global_t)((const bf16_t*)a.x + x_at[i] + tail(k0, i)),
+                                         (gg_lds_t)(st + (16 * wave + 8 * i) * 128), 16, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < WL; ++i)
+      __builtin_amdgcn_global_load_lds((gg_global_t)(wg + w_at[i] + tail(k0, i)),
+                                       (gg_lds_t)(st + (GT_ROWS + 8 * WL * wave + 8 * i) * 128), 16, 0, 0);
+  };
+  auto place_x = [&](int which) {                  // float32 rows, rounded, where a direct load would have put them
+    if (!XF32) return;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const float4 lo = __builtin_bit_cast(float4, held[XF32 ? 2 * i : 0]), hi = __builtin_bit_cast(float4, held[XF32 ? 2 * i + 1 : 0]);
+      *reinterpret_cast<uint4*>(stages + which * STAGE + (16 * wave + 8 * i) * 128 + 16 * lane) =
+          make_uint4(pack2_bf16(lo.x, lo.y), pack2_bf16(lo.z, lo.w), pack2_bf16(hi.x, hi.y), pack2_bf16(hi.z, hi.w));
+    }
+  };
+  gg_f32x4 acc[XT][4];
+#pragma unroll
+  for (int i = 0; i < XT; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = gg_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  const int fr = lane & 15, q = lane >> 4;
+  const unsigned lds0 = (unsigned)(size_t)(gg_lds_t)stages;
+  const unsigned at = lds0 + fr * 128 + ((q ^ (fr >> 1)) << 4);
+  const unsigned x_read = at + x_wave * 128, w_read = at + (GT_ROWS + 64 * w_wave) * 128;
+  const int n_steps = (a.K + GT_BK - 1) / GT_BK;
+  ask(0, 0);
+  for (int t = 0; t < n_steps; ++t) {
+    place_x(t & 1);
+    wait_vmcnt<0>();
+    __syncthreads();                               // this stage is there, and the other one's readers are done
+    if (t + 1 < n_steps) ask((t + 1) * GT_BK, (t + 1) & 1);
+    const unsigned xr = x_read + (t & 1) * STAGE, wr = w_read + (t & 1) * STAGE;
+    u32x4 xf[2][XT], wf[2][4];
+    read_frags<XT, 2048>(xf[0], xr);
+    read_frags<4, 2048>(wf[0], wr);
+    const bool both = t * GT_BK + 32 < a.K;
+    if (both) {
+      read_frags<XT, 2048>(xf[1], xr ^ 64);
+      read_frags<4, 2048>(wf[1], wr ^ 64);
+      wait_lgkmcnt<XT + 4>();
+    } else {
+      wait_lgkmcnt<0>();
+    }
+    use_frags<XT>(xf[0]);
+    use_frags<4>(wf[0]);
+#pragma unroll
+    for (int i = 0; i < XT; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gg_bf16x8, wf[0][j]), __builtin_bit_cast(gg_bf16x8, xf[0][i]),
+                                                            acc[i][j], 0, 0, 0);
+    if (both) {
+      wait_lgkmcnt<0>();
+      use_frags<XT>(xf[1]);
+      use_frags<4>(wf[1]);
+#pragma unroll
+      for (int i = 0; i < XT; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gg_bf16x8, wf[1][j]), __builtin_bit_cast(gg_bf16x8, xf[1][i]),
+                                                              acc[i][j], 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < XT; ++i) {
+    const int r = x_wave + 16 * i + fr;
     if (r >= count) continue;
+    const int orow = a.out_rows ? a.out_rows[first + r] : first + r;
 #pragma unroll
     for (int j = 0; j < (GLU ? 2 : 4); ++j)
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const int n = n0 + (GLU ? 32 * wc + 16 * j : 64 * wc + 16 * j) + (lane >> 4) * 4 + c;
-        if (n < a.N) gg_store(a, g, orow[r], n, acc[i][j][c], GLU ? acc[i][j + 2][c] : 0.0f);
-      }
+      gg_store4(a, g, orow, n0 + (GLU ? 32 : 64) * w_wave + 16 * j + 4 * q, acc[i][j], acc[i][GLU ? j + 2 : j]);
   }
+}
+
+template <bool GLU, bool XF32, int WROWS>
+int launch_tile(const GroupedArgs& a, dim3 grid, hipStream_t s) {
+  static bool configured = false;
+  if (!configured) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&grouped_gemm_tile_kernel<GLU, XF32, WROWS>),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, 2 * GT_STAGE(WROWS));
+    if (e != hipSuccess) {
+      axk_set_error("grouped_gemm: cannot reserve %d bytes of LDS: %s", 2 * GT_STAGE(WROWS), hipGetErrorString(e));
+      return -2;
+    }
+    configured = true;
+  }
+  grouped_gemm_tile_kernel<GLU, XF32, WROWS><<<grid, 256, 2 * GT_STAGE(WROWS), s>>>(a);
+  return 0;
 }
 #endif
 
@@ -337,7 +429,8 @@ extern "C" int axk_grouped_gemm(const void* x, int x_is_f32, long x_row_stride, 
   GroupedArgs a{x, x_is_f32, x_row_stride, x_group_stride, x_rows, (const elem_t*)w, bias, bias_is_f32, out, out_is_f32,
                 out_row_stride, out_group_stride, out_rows, gate, gate_row_stride, gate_per_group, row_scale, glu, glu_limit, glu_alpha,
                 glu_shift, tiles, n_tiles,
-                m, n, k, groups};
+                m, n, k, groups,
+                out_row_stride % 4 == 0 && out_group_stride % 4 == 0 && (uintptr_t)out % (out_is_f32 ? 16 : 8) == 0};
   dim3 grid(row_tiles, ceil_div(n, GG_COLS), tiles ? 1 : groups);
   hipStream_t s = (hipStream_t)stream;
 #if AXON_BF16
@@ -345,15 +438,32 @@ extern "C" int axk_grouped_gemm(const void* x, int x_is_f32, long x_row_stride, 
                     ((uintptr_t)w & 15) == 0;
   // many rows a group: tiles of 64 rows through LDS (a list of tiles says by its tile size which it was made for)
   if (mfma && (tiles ? tile_rows == 64 : m >= 256)) {
-    dim3 big(tiles ? max_tiles : ceil_div(m, GT_ROWS), ceil_div(n, glu ? 64 : 128), tiles ? 1 : groups);
-    if (glu) { AXK_INSTANCE(INST_GROUPED_GEMM, 2, 1); grouped_gemm_tile_kernel<true><<<big, 256, 0, s>>>(a); }
-    else { AXK_INSTANCE(INST_GROUPED_GEMM, 2, 0); grouped_gemm_tile_kernel<false><<<big, 256, 0, s>>>(a); }
+    // up to 128 columns a group (a head's values out of its latent): half the rows of W would be none
+    const bool narrow = !glu && n <= 128;
+    const long blocks = (long)(tiles ? max_tiles : ceil_div(m, GT_ROWS)) * ceil_div(n, glu || narrow ? 128 : 256) * (tiles ? 1 : groups);
+    AXK_REQUIRE(blocks < (1l << 31) - 8, "grouped_gemm: %ld blocks are more than one launch takes", blocks);
+    const dim3 big((unsigned)((blocks + 7) / 8 * 8));
+    int rc;
+    if (glu) { AXK_INSTANCE(INST_GROUPED_GEMM, 2, 1); rc = x_is_f32 ? launch_tile<true, true, 256>(a, big, s) : launch_tile<true, false, 256>(a, big, s); }
+    else {
+      AXK_INSTANCE(INST_GROUPED_GEMM, 2, 0);
+      if (narrow) rc = x_is_f32 ? launch_tile<false, true, 128>(a, big, s) : launch_tile<false, false, 128>(a, big, s);
+      else rc = x_is_f32 ? launch_tile<false, true, 256>(a, big, s) : launch_tile<false, false, 256>(a, big, s);
+    }
+    if (rc) return rc;
     AXK_LAUNCH_CHECK("grouped_gemm");
     return 0;
   }
   if (mfma) {
-    if (glu) { AXK_INSTANCE(INST_GROUPED_GEMM, 1, 1); grouped_gemm_mfma_kernel<true><<<grid, 256, 0, s>>>(a); }
-    else { AXK_INSTANCE(INST_GROUPED_GEMM, 1, 0); grouped_gemm_mfma_kernel<false><<<grid, 256, 0, s>>>(a); }
+    if (glu) {
+      AXK_INSTANCE(INST_GROUPED_GEMM, 1, 1);
+      if (x_is_f32) grouped_gemm_mfma_kernel<true, true><<<grid, 256, 0, s>>>(a);
+      else grouped_gemm_mfma_kernel<true, false><<<grid, 256, 0, s>>>(a);
+    } else {
+      AXK_INSTANCE(INST_GROUPED_GEMM, 1, 0);
+      if (x_is_f32) grouped_gemm_mfma_kernel<false, true><<<grid, 256, 0, s>>>(a);
+      else grouped_gemm_mfma_kernel<false, false><<<grid, 256, 0, s>>>(a);
+    }
     AXK_LAUNCH_CHECK("grouped_gemm");
     return 0;
   }

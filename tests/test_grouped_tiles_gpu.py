@@ -1,0 +1,56 @@
+"""The grouped products' two matrix-core kernels at the edges of their tiles: the one for many rows (64 x 256 or 64 x 128
+through LDS) gives the bits of the one for few, whatever the sizes, the type of X and the layout of the output."""
+import pytest
+import torch
+
+from axon_amd.kernels import kernels
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("N,K,G", [(8, 32, 2), (128, 96, 3), (129, 64, 2), (260, 160, 1), (300, 288, 2)])
+@pytest.mark.parametrize("x_f32", [False, True])
+@pytest.mark.parametrize("glu", [None, (1.5, 1.702)])
+def test_many_rows_have_the_bits_of_few(N, K, G, x_f32, glu):
+    k = kernels("bfloat16")
+    g = torch.Generator(device="cuda").manual_seed(N * K)
+    M = 321
+    x = torch.randn(M, G * K, generator=g, device="cuda")
+    x = x if x_f32 else x.bfloat16()
+    w = (torch.randn(G, (2 if glu else 1) * N, K, generator=g, device="cuda") * 0.2).bfloat16()
+    for out_dtype, pad in ((torch.float32, 0), (torch.bfloat16, 1), (torch.bfloat16, 4)):
+        ogs = N + pad
+        out = torch.full((M, G * ogs), float("nan"), dtype=out_dtype, device="cuda")
+        k.grouped_gemm(x, w, out, x_group_stride=K, out_group_stride=ogs, glu=glu)
+        for first, m in ((0, 200), (121, 200)):                      # few rows: the other kernel
+            few = torch.full((m, G * ogs), float("nan"), dtype=out_dtype, device="cuda")
+            k.grouped_gemm(x[first:first + m], w, few, x_group_stride=K, out_group_stride=ogs, glu=glu)
+            assert torch.equal(few.nan_to_num(9.0), out[first:first + m].nan_to_num(9.0))
+        cols = torch.arange(G * ogs, device="cuda") % ogs < N
+        assert not bool(out[:, cols].isnan().any()) and bool(out[:, ~cols].isnan().all())     # nothing beside the groups' columns
+        if glu is None and out_dtype == torch.float32:
+            want = torch.stack([x[:, i * K:(i + 1) * K].bfloat16().double() @ w[i].double().T for i in range(G)], 1).flatten(1)
+            # one chain of K / 32 products of 32, each rounding at most half a unit of the sum of magnitudes a step
+            bound = (K + 2) * 2.0 ** -24 * float(x.double().abs().max() * w.double().abs().max()) * K
+            assert float((out.double() - want).abs().max()) <= bound
+
+
+@pytest.mark.parametrize("T,E,top", [(70, 5, 3), (256, 8, 2)])
+def test_lists_of_64_and_of_16_rows_agree(T, E, top):
+    k = kernels("bfloat16")
+    g = torch.Generator(device="cuda").manual_seed(T)
+    H, F, P = 96, 136, T * top
+    h = torch.randn(T, H, generator=g, device="cuda").bfloat16()
+    wu = (torch.randn(E, 2 * F, H, generator=g, device="cuda") * 0.2).bfloat16()
+    chosen = torch.stack([torch.randperm(E, generator=g, device="cuda")[:top] for _ in range(T)]).int().contiguous()
+    scale = torch.rand(P, generator=g, device="cuda")
+    got = []
+    for rows in (16, 64):
+        most = k.route_max_tiles(P, E, rows)
+        pairs, tokens, tiles, n = (torch.zeros(s, dtype=torch.int32, device="cuda") for s in (P, P, 3 * most, 1))
+        k.route_sort(chosen, E, pairs, tokens, tiles, n, tile_rows=rows)
+        out = torch.full((P, F), float("nan"), dtype=torch.bfloat16, device="cuda")
+        k.grouped_gemm(h, wu, out, x_group_stride=0, out_group_stride=0, glu=(float("inf"), 1.0, 0.0),
+                       routed=(tiles, n, most, tokens, pairs, rows), rows=P, row_scale=scale)
+        got.append(out)
+    assert torch.equal(got[0], got[1]) and not bool(got[0].isnan().any())
