@@ -8,6 +8,8 @@
 // read), then [rank][page_size], the latents again with the positions of one dim side by side
 // (what the matrix cores want as the operand of the weighted sum; the same layout as the values of
 // the grouped-query attention's pages).  Scores, weights and sums are 32-bit.
+#include <type_traits>
+
 #include "api.h"
 #include "common.h"
 
@@ -174,13 +176,20 @@ __device__ inline la_bf16x8 la_frag(uint4 v) { return __builtin_bit_cast(la_bf16
 // lane) and the rounded weights, as they lie in the accumulators, as the second.  RT: tiles of 16
 // latent dims at most; QC: chunks of 32 key dims at most.  Pages hold a multiple of 64 positions.
 #define LAM_WAVES 2
+#define LAP_TOKENS 8                                  // tokens a block of the kernel for steps of many tokens
+__device__ __forceinline__ bool latent_one_request(const int32_t* __restrict__ seq_rows, int first, int last) {
+  bool same = true;
+  for (int u = first + 1; u <= last; ++u) same = same && seq_rows[u] == seq_rows[first];
+  return same;
+}
+
 template <int RT, int QC, bool SINK>
 __global__ void __launch_bounds__(LAM_WAVES * 64)
 latent_attention_mfma_kernel(const float* __restrict__ q_full, const bf16_t* __restrict__ cache,
                              const int32_t* __restrict__ block_table, int table_stride, const int32_t* __restrict__ positions,
                              const int32_t* __restrict__ seq_rows, float* __restrict__ o_lat, int n_tokens, int heads, int rank,
                              int rot, int page_size, int window, float scale, const float* __restrict__ sink,
-                             float* __restrict__ partial, int n_chunks) {
+                             float* __restrict__ partial, int n_chunks, bool mixed_only) {
   // the sixteen heads' queries as bfloat16 in LDS, rows 16 bytes longer than their chunks so that the
   // sixteen rows a product's operand is read from fall into different banks
   constexpr int QROW = QC * 32 + 8;
@@ -191,8 +200,12 @@ latent_attention_mfma_kernel(const float* __restrict__ q_full, const bf16_t* __r
   // should be the short ones; over a window most rows are equally long, and the tokens go in their order
   const long n_items = (long)n_tokens * groups, at = (long)blockIdx.x * LAM_WAVES + wave;
   const long item = window > 0 ? at : n_items - 1 - at;
-  const bool active = at < n_items;
+  bool active = at < n_items;
   const int t = active ? (int)(item / groups) : 0, hg = active ? (int)(item % groups) : 0;
+  if (mixed_only && active) {                         // beside the kernel for steps of many tokens: what it leaves
+    const int t_first = t / LAP_TOKENS * LAP_TOKENS;
+    active = !latent_one_request(seq_rows, t_first, min(t_first + LAP_TOKENS, n_tokens) - 1);
+  }
   const int width = rank + rot, qc = width / 32, rt = rank / 16;
   const int j = lane & 15, g = lane >> 4;
   bf16_t* qs = qs_all[wave];
@@ -321,218 +334,236 @@ latent_attention_mfma_kernel(const float* __restrict__ q_full, const bf16_t* __r
     if (dt < rt) *reinterpret_cast<float4*>(dst + 16 * dt) = make_float4(acc[dt][0] * inv, acc[dt][1] * inv, acc[dt][2] * inv, acc[dt][3] * inv);
 }
 
-// The same for steps of many tokens: four waves a block take four neighbouring tokens (and the same sixteen
-// heads).  Where these belong to one request (a prompt's portion) they read the same pages, and a block of
-// 64 positions is staged in LDS once for the four: its K rows [64][rank + rot] for the scores, then, in the
-// same buffer, its C^T rows [rank][64] for the weighted sums (rows 16 bytes longer than their content, as the
-// queries').  Each wave keeps its own mask, running pair and accumulators, and runs the chain of products
-// of the kernel above: the same bits.  Tokens of several requests in one block (decoding rows side by
-// side): every wave reads its own pages from memory, as above.
-#define LAS_WAVES 4
-#define LATENT_TOKENS_KERNEL_FROM 256           // (token, sixteen heads) items of a step from which four tokens share a block
-template <int RT, int QC, bool SHARED>
-__device__ __forceinline__ void latent_walk(const bf16_t* __restrict__ cache, const int32_t* __restrict__ pages, long page_elems,
-                                            int page_size, int width, int rank, int qc, int rt, int b_from, int b_to, bool active,
-                                            int lo, int pos, float scale, const bf16_t* qlane, bf16_t* stage, int j, int g,
-                                            float& m, float& l, la_f32x4 (&acc)[RT]) {
-  const int KROW = width + 8;
-  constexpr int VROW = 64 + 8;
-  for (int b = b_from; b <= b_to; ++b) {
-    const int p0 = b * 64, in0 = p0 % page_size;
-    const bf16_t* page = cache + (long)pages[p0 / page_size] * page_elems;
-    const bool mine = active && b >= lo / 64 && b <= pos / 64;
-    const bf16_t* kbase;
-    long krow_stride;
-    if constexpr (SHARED) {
-      __syncthreads();                               // the buffer's last readers are done
-      const uint4* src = reinterpret_cast<const uint4*>(page + (long)in0 * width);
-      const int per_row = width / 8, units = 64 * per_row;
-      {
-        // every load of the block's K rows in flight at once (the registers of the scores are free here)
-        uint4 held[QC];
-#pragma unroll
-        for (int e = 0; e < QC; ++e)
-          held[e] = src[min((int)threadIdx.x + e * LAS_WAVES * 64, units - 1)];
-#pragma unroll
-        for (int e = 0; e < QC; ++e) {
-          const int u = threadIdx.x + e * LAS_WAVES * 64;
-          if (u < units) *reinterpret_cast<uint4*>(stage + (u / per_row) * KROW + 8 * (u % per_row)) = held[e];
-        }
-      }
-      __syncthreads();
-      kbase = stage + 8 * g;
-      krow_stride = KROW;
-    } else {
-      kbase = page + (long)in0 * width + 8 * g;
-      krow_stride = width;
-    }
-    la_f32x4 s[4];
-    uint4 pf[2];
-    float fold = 1.0f;
-    if (mine) {
-#pragma unroll
-      for (int pt = 0; pt < 4; ++pt) {
-        s[pt] = la_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        const bf16_t* krow = kbase + (long)(16 * pt + j) * krow_stride;
-        constexpr int QB = SHARED ? (QC < 4 ? QC : 4) : (QC < 10 ? QC : 10);
-#pragma unroll
-        for (int k0 = 0; k0 < QC; k0 += QB) {
-          uint4 kf[QB];
-#pragma unroll
-          for (int e = 0; e < QB; ++e)
-            if (k0 + e < qc) kf[e] = *reinterpret_cast<const uint4*>(krow + 32 * (k0 + e));
-#pragma unroll
-          for (int e = 0; e < QB; ++e)
-            if (k0 + e < qc) s[pt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(la_frag(kf[e]), la_frag(*reinterpret_cast<const uint4*>(qlane + 32 * (k0 + e))), s[pt], 0, 0, 0);
-        }
-      }
-      float mx = -INFINITY;
-#pragma unroll
-      for (int pt = 0; pt < 4; ++pt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int p = p0 + 16 * pt + 4 * g + i;
-          const float v = (p >= lo && p <= pos) ? s[pt][i] * scale : -INFINITY;
-          s[pt][i] = v;
-          mx = fmaxf(mx, v);
-        }
-      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-      const float m_new = fmaxf(m, mx);
-      fold = expf(m - m_new);
-      float sum = 0.0f;
-#pragma unroll
-      for (int pt = 0; pt < 4; ++pt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float w = expf(s[pt][i] - m_new);        // 0 where the position is not seen
-          s[pt][i] = w;
-          sum += w;
-        }
-      sum += __shfl_xor(sum, 16, 64);
-      sum += __shfl_xor(sum, 32, 64);
-      l = fmaf(l, fold, sum);
-      m = m_new;
-#pragma unroll
-      for (int c = 0; c < 2; ++c)
-        pf[c] = make_uint4(pack2_bf16(s[2 * c][0], s[2 * c][1]), pack2_bf16(s[2 * c][2], s[2 * c][3]),
-                           pack2_bf16(s[2 * c + 1][0], s[2 * c + 1][1]), pack2_bf16(s[2 * c + 1][2], s[2 * c + 1][3]));
-    }
-    const bf16_t* vbase;
-    long vrow_stride;
-    if constexpr (SHARED) {
-      __syncthreads();                               // the K rows' readers are done
-      const bf16_t* src = page + (long)page_size * width + in0;
-      const int units = rank * 8;
-      {
-        constexpr int VU = (RT + 1) / 2;             // rank x 8 units of 16 bytes over 256 threads
-        uint4 held[VU];
-#pragma unroll
-        for (int e = 0; e < VU; ++e) {
-          const int u = min((int)threadIdx.x + e * LAS_WAVES * 64, units - 1);
-          held[e] = *reinterpret_cast<const uint4*>(src + (long)(u / 8) * page_size + 8 * (u % 8));
-        }
-#pragma unroll
-        for (int e = 0; e < VU; ++e) {
-          const int u = threadIdx.x + e * LAS_WAVES * 64;
-          if (u < units) *reinterpret_cast<uint4*>(stage + (u / 8) * VROW + 8 * (u % 8)) = held[e];
-        }
-      }
-      __syncthreads();
-      vbase = stage + 4 * g;
-      vrow_stride = VROW;
-    } else {
-      vbase = page + (long)page_size * width + in0 + 4 * g;
-      vrow_stride = page_size;
-    }
-    if (mine) {
-      constexpr int VB = SHARED ? 2 : 4;             // tiles of 16 dims whose rows are asked for together
-#pragma unroll
-      for (int d0 = 0; d0 < RT; d0 += VB) {
-        uint2 v[VB][4];
-#pragma unroll
-        for (int e = 0; e < VB; ++e) {
-          if (d0 + e < rt) {
-            const bf16_t* vrow = vbase + (long)(16 * (d0 + e) + j) * vrow_stride;
-#pragma unroll
-            for (int c = 0; c < 2; ++c) {
-              v[e][2 * c] = *reinterpret_cast<const uint2*>(vrow + 32 * c);
-              v[e][2 * c + 1] = *reinterpret_cast<const uint2*>(vrow + 32 * c + 16);
-            }
-          }
-        }
-#pragma unroll
-        for (int e = 0; e < VB; ++e) {
-          if (d0 + e < rt) {
-            acc[d0 + e] *= fold;
-#pragma unroll
-            for (int c = 0; c < 2; ++c)
-              acc[d0 + e] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                  la_frag(make_uint4(v[e][2 * c].x, v[e][2 * c].y, v[e][2 * c + 1].x, v[e][2 * c + 1].y)), la_frag(pf[c]), acc[d0 + e],
-                  0, 0, 0);
-          }
-        }
-      }
-    }
+#define LATENT_PROMPT_KERNEL_FROM 256           // (token, sixteen heads) items of a step from which eight tokens share a block
+typedef __attribute__((ext_vector_type(2))) unsigned la_u32x2;
+typedef const __attribute__((address_space(1))) void* la_global_t;
+typedef __attribute__((address_space(3))) void* la_lds_t;
+
+template <int OFFSET>
+__device__ __forceinline__ void la_read8(la_u32x2& dst, unsigned at) {
+  asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(dst) : "v"(at), "n"(OFFSET));
+}
+
+// body(0) .. body(N - 1), each with its number as a constant.
+template <int N, int I = 0, typename F>
+__device__ __forceinline__ void la_for(F&& body) {
+  if constexpr (I < N) {
+    body(std::integral_constant<int, I>());
+    la_for<N, I + 1>(body);
   }
 }
 
-template <int RT, int QC, bool SINK>
-__global__ void __launch_bounds__(LAS_WAVES * 64)
-latent_attention_mfma_tokens_kernel(const float* __restrict__ q_full, const bf16_t* __restrict__ cache,
-                                    const int32_t* __restrict__ block_table, int table_stride, const int32_t* __restrict__ positions,
-                                    const int32_t* __restrict__ seq_rows, float* __restrict__ o_lat, int n_tokens, int heads, int rank,
-                                    int rot, int page_size, int window, float scale, const float* __restrict__ sink) {
-  extern __shared__ __align__(16) bf16_t las_lds[];
-  bf16_t* stage = las_lds;                                                        // max(64 x (width + 8), rank x 72) elements
-  const int QROW = rank + rot + 8;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  bf16_t* qs = las_lds + max(64 * QROW, rank * 72) + wave * 16 * QROW;
-  const int groups = heads / 16;
-  const int n_tiles = (n_tokens + LAS_WAVES - 1) / LAS_WAVES;
-  // without a window the step's last tokens first (see the kernel above)
+// Steps of many tokens: a block takes eight neighbouring tokens (and the same sixteen heads), a wave each, its
+// queries in registers.  Where the eight belong to one request (a prompt's portion) a block of 64 positions goes
+// through LDS once for all of them, by direct loads: its K rows [64][rank + rot] while the block before is
+// summed, its C^T rows [rank][64] while the scores are worked out.  16-byte slots of a staged row are permuted by
+// slot ^ (row / 2 % 8), so that the sixteen rows of a read fall into different banks.  Each wave keeps its own
+// mask, running pair and accumulators and runs the chain of products of the kernels above: the same bits (sums
+// whose maximum stays are not multiplied by 1).  Tiles with tokens of several requests are left to a launch of
+// the kernel above (`mixed_only`).  Bound by the way out of LDS: a wave reads the block's 136 KB for 2,176 cycles of products.
+// 16 heads, latents of 512 and 64 rotated dims, 2,048 tokens over a window of 1,024: 638 -> 129 us (four tokens a
+// block, stages through registers, queries read from LDS beside the keys).
+template <int RT, int QC, bool EXACT, bool SINK>
+__global__ void __launch_bounds__(LAP_TOKENS * 64, 2)
+latent_attention_prompt_kernel(const float* __restrict__ q_full, const bf16_t* __restrict__ cache,
+                               const int32_t* __restrict__ block_table, int table_stride, const int32_t* __restrict__ positions,
+                               const int32_t* __restrict__ seq_rows, float* __restrict__ o_lat, int n_tokens, int heads, int rank,
+                               int rot, int page_size, int window, float scale, const float* __restrict__ sink) {
+  extern __shared__ __align__(256) unsigned char lap_lds[];                       // K [64][width], C^T [rank][64]
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int groups = heads / 16, n_tiles = (n_tokens + LAP_TOKENS - 1) / LAP_TOKENS;
+  // without a window the step's last tokens first (see above)
   const int at = (int)blockIdx.x / groups, hg = (int)blockIdx.x % groups;
   const int tile = window > 0 ? at : n_tiles - 1 - at;
-  const int t = tile * LAS_WAVES + wave;
-  const bool active = t < n_tokens;
+  if (EXACT) { rank = 16 * RT; rot = 32 * QC - 16 * RT; }
   const int width = rank + rot, qc = width / 32, rt = rank / 16;
-  const int j = lane & 15, g = lane >> 4;
-  if (active) {
-    const int per_row = width / 8;
-    for (int idx = lane; idx < 16 * per_row; idx += 64) {
-      const int row = idx / per_row, part = idx % per_row;
-      const float* src = q_full + ((long)t * heads + hg * 16 + row) * width + 8 * part;
-      const float4 a = *reinterpret_cast<const float4*>(src), b = *reinterpret_cast<const float4*>(src + 4);
-      *reinterpret_cast<uint4*>(qs + row * QROW + 8 * part) =
-          make_uint4(pack2_bf16(a.x, a.y), pack2_bf16(a.z, a.w), pack2_bf16(b.x, b.y), pack2_bf16(b.z, b.w));
-    }
-  }
-  // the block's tokens: one request (its pages staged once for all) or several (every wave on its own)
-  const int t_first = tile * LAS_WAVES, t_last = min(t_first + LAS_WAVES, n_tokens) - 1;
-  bool same = true;
+  const long page_elems = (long)page_size * (width + rank);
+  const int t_first = tile * LAP_TOKENS, t_last = min(t_first + LAP_TOKENS, n_tokens) - 1;
+  if (!latent_one_request(seq_rows, t_first, t_last)) return;       // (the same for the whole block)
   int b_from = 1 << 30, b_to = -1;
   for (int u = t_first; u <= t_last; ++u) {
-    same = same && seq_rows[u] == seq_rows[t_first];
     const int p = positions[u];
     b_from = min(b_from, (window > 0 ? max(0, p + 1 - window) : 0) / 64);
     b_to = max(b_to, p / 64);
   }
-  const bf16_t* qlane = qs + j * QROW + 8 * g;
-  const int pos = active ? positions[t] : 0;
-  const int lo = window > 0 ? max(0, pos + 1 - window) : 0;
-  const int32_t* pages = block_table + (long)seq_rows[active ? t : t_first] * table_stride;
-  const long page_elems = (long)page_size * (width + rank);
+  const bool active = t_first + wave <= t_last;
+  const int t = min(t_first + wave, t_last), j = lane & 15, g = lane >> 4;
+  const int pos = positions[t], lo = window > 0 ? max(0, pos + 1 - window) : 0;
+  const int32_t* pages = block_table + (long)seq_rows[t] * table_stride;
+  // Q^T: a lane's head j, 8 consecutive dims from 32 kc + 8 g, rounded
+  u32x4 qf[QC];
+  const float* qsrc = q_full + ((long)t * heads + hg * 16 + j) * width + 8 * g;
+#pragma unroll
+  for (int kc = 0; kc < QC; ++kc)
+    if (kc < qc) {
+      const float4 a = *reinterpret_cast<const float4*>(qsrc + 32 * kc), b = *reinterpret_cast<const float4*>(qsrc + 32 * kc + 4);
+      qf[kc] = u32x4{pack2_bf16(a.x, a.y), pack2_bf16(a.z, a.w), pack2_bf16(b.x, b.y), pack2_bf16(b.z, b.w)};
+    }
   la_f32x4 acc[RT];
 #pragma unroll
   for (int i = 0; i < RT; ++i) acc[i] = la_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  float m = (SINK && active) ? sink[hg * 16 + j] : -INFINITY, l = SINK ? 1.0f : 0.0f;
-  __syncthreads();
-  if (same)
-    latent_walk<RT, QC, true>(cache, pages, page_elems, page_size, width, rank, qc, rt, b_from, b_to, active, lo, pos, scale, qlane, stage,
-                              j, g, m, l, acc);
-  else if (active)
-    latent_walk<RT, QC, false>(cache, pages, page_elems, page_size, width, rank, qc, rt, lo / 64, pos / 64, true, lo, pos, scale, qlane,
-                               stage, j, g, m, l, acc);
+  float m = SINK ? sink[hg * 16 + j] : -INFINITY, l = SINK ? 1.0f : 0.0f;
+
+  // scores of a block (lane: positions p0 + 16 pt + 4 g + i of head j) to weights, the running pair, the operand
+  la_f32x4 s[4];
+  uint4 pf[2];
+  auto weigh = [&](int p0) {
+    float mx = -INFINITY;
+#pragma unroll
+    for (int pt = 0; pt < 4; ++pt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int p = p0 + 16 * pt + 4 * g + i;
+        const float v = (p >= lo && p <= pos) ? s[pt][i] * scale : -INFINITY;
+        s[pt][i] = v;
+        mx = fmaxf(mx, v);
+      }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    const float m_new = fmaxf(m, mx);
+    const float fold = expf(m - m_new);
+    float sum = 0.0f;
+#pragma unroll
+    for (int pt = 0; pt < 4; ++pt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float w = expf(s[pt][i] - m_new);        // 0 where the position is not seen
+        s[pt][i] = w;
+        sum += w;
+      }
+    sum += __shfl_xor(sum, 16, 64);
+    sum += __shfl_xor(sum, 32, 64);
+    l = fmaf(l, fold, sum);
+    m = m_new;
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+      pf[c] = make_uint4(pack2_bf16(s[2 * c][0], s[2 * c][1]), pack2_bf16(s[2 * c][2], s[2 * c][3]),
+                         pack2_bf16(s[2 * c + 1][0], s[2 * c + 1][1]), pack2_bf16(s[2 * c + 1][2], s[2 * c + 1][3]));
+    if (!__all(fold == 1.0f)) {
+#pragma unroll
+      for (int i = 0; i < RT; ++i) acc[i] *= fold;
+    }
+  };
+
+  const int per_row = width / 8, k_mask = per_row % 8 == 0 ? 7 : 3;
+  unsigned char* vstage = lap_lds + 128 * width;
+  const int first_slot = wave * 64 + lane, step_rows = LAP_TOKENS * 64 / per_row, step_slots = LAP_TOKENS * 64 % per_row;
+  const int row0 = first_slot / per_row, slot0 = first_slot % per_row;
+  auto ask_k = [&](int b) {
+    const int p0 = b * 64;
+    const bf16_t* src = cache + (long)pages[p0 / page_size] * page_elems + (long)(p0 % page_size) * width;
+    int row = row0, slot = slot0;
+    for (int n = wave; n < per_row; n += LAP_TOKENS) {
+      __builtin_amdgcn_global_load_lds((la_global_t)(src + row * width + 8 * (slot ^ ((row >> 1) & k_mask))), (la_lds_t)(lap_lds + n * 1024), 16, 0, 0);
+      row += step_rows;
+      slot += step_slots;
+      if (slot >= per_row) { slot -= per_row; ++row; }
+    }
+  };
+  auto ask_v = [&](int b) {
+    const int p0 = b * 64;
+    const bf16_t* src = cache + (long)pages[p0 / page_size] * page_elems + (long)page_size * width + p0 % page_size +
+                        8 * ((lane & 7) ^ (4 * (wave & 1) + (lane >> 4))) + (long)(lane >> 3) * page_size;
+    for (int n = wave; n < rank / 8; n += LAP_TOKENS)
+      __builtin_amdgcn_global_load_lds((la_global_t)(src + (long)n * 8 * page_size), (la_lds_t)(vstage + n * 1024), 16, 0, 0);
+  };
+  const int f = j >> 1;
+  const unsigned base = EXACT ? (unsigned)(size_t)(la_lds_t)lap_lds : 0u;       // (reads written as instructions: an LDS address)
+  const unsigned k_row = base + j * 2 * width;
+  // chunk kc of row j: k_at[kc % 2] + 128 (kc / 2); positions 16 x + 4 g .. + 3 of dim j: v_at[x].  Rows start at multiples
+  // of 64 bytes and of 128, so the second address differs from the first by a bit of it.
+  const unsigned k_first = k_row + ((k_mask == 7 ? g ^ f : g ^ (f & 3)) << 4);
+  const unsigned v_first = base + 128 * width + j * 128 + 8 * (g & 1) + (((g >> 1) ^ f) << 4);
+  ask_k(b_from);
+  for (int b = b_from; b <= b_to; ++b) {
+    wait_vmcnt<0>();
+    __syncthreads();                                // K of this block is there, C^T of the block before is read
+    ask_v(b);
+    const bool mine = active && b >= lo / 64 && b <= pos / 64;
+    if (mine) {
+#pragma unroll
+      for (int pt = 0; pt < 4; ++pt) s[pt] = la_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      unsigned k_base = k_first;
+      asm volatile("" : "+v"(k_base));              // (the others are worked out here: no registers of theirs across the loop)
+      const unsigned k_at[2] = {k_base, k_mask == 7 ? k_base ^ 64 : k_base + 64};
+      if constexpr (EXACT) {
+        u32x4 kf[2][2];                             // two of the four tiles of 16 positions, read one pair ahead
+        auto read_k = [&](auto u) {
+          constexpr int U = decltype(u)::value, KC = U / 2;
+          lds_read16<128 * (KC / 2) + 2 * (U & 1) * 1024 * QC>(kf[U & 1][0], k_at[KC & 1]);
+          lds_read16<128 * (KC / 2) + (2 * (U & 1) + 1) * 1024 * QC>(kf[U & 1][1], k_at[KC & 1]);
+        };
+        read_k(std::integral_constant<int, 0>());
+        la_for<2 * QC>([&](auto u) {
+          constexpr int U = decltype(u)::value;
+          if constexpr (U + 1 < 2 * QC) {
+            read_k(std::integral_constant<int, U + 1>());
+            wait_lgkmcnt<2>();
+          } else {
+            wait_lgkmcnt<0>();
+          }
+          use_frags<2>(kf[U & 1]);
+#pragma unroll
+          for (int e = 0; e < 2; ++e)
+            s[2 * (U & 1) + e] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(la_bf16x8, kf[U & 1][e]), __builtin_bit_cast(la_bf16x8, qf[U / 2]),
+                                                                         s[2 * (U & 1) + e], 0, 0, 0);
+        });
+      } else {
+#pragma unroll
+        for (int kc = 0; kc < QC; ++kc)
+          if (kc < qc)
+#pragma unroll
+            for (int pt = 0; pt < 4; ++pt) {
+              const uint4 kf = *reinterpret_cast<const uint4*>(lap_lds + k_at[kc & 1] + 128 * (kc / 2) + pt * 32 * width);
+              s[pt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(la_frag(kf), __builtin_bit_cast(la_bf16x8, qf[kc]), s[pt], 0, 0, 0);
+            }
+      }
+      weigh(b * 64);
+    }
+    wait_vmcnt<0>();
+    __syncthreads();                                // C^T of this block is there, its K is read
+    if (b < b_to) ask_k(b + 1);
+    if (mine) {
+      unsigned v_base = v_first;
+      asm volatile("" : "+v"(v_base));
+      const unsigned v_at[4] = {v_base, v_base ^ 32, v_base ^ 64, v_base ^ 96};
+      if constexpr (EXACT) {
+        la_u32x2 vf[2][4];                          // a tile of 16 dims, read one ahead
+        auto read_v = [&](auto d) {
+          constexpr int D = decltype(d)::value;
+#pragma unroll
+          for (int x = 0; x < 4; ++x) la_read8<2048 * D>(vf[D & 1][x], v_at[x]);
+        };
+        read_v(std::integral_constant<int, 0>());
+        la_for<RT>([&](auto d) {
+          constexpr int D = decltype(d)::value;
+          if constexpr (D + 1 < RT) {
+            read_v(std::integral_constant<int, D + 1>());
+            wait_lgkmcnt<4>();
+          } else {
+            wait_lgkmcnt<0>();
+          }
+#pragma unroll
+          for (int x = 0; x < 4; ++x) asm volatile("" : "+v"(vf[D & 1][x]));
+#pragma unroll
+          for (int c = 0; c < 2; ++c)
+            acc[D] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                la_frag(make_uint4(vf[D & 1][2 * c][0], vf[D & 1][2 * c][1], vf[D & 1][2 * c + 1][0], vf[D & 1][2 * c + 1][1])),
+                la_frag(pf[c]), acc[D], 0, 0, 0);
+        });
+      } else {
+#pragma unroll
+        for (int d = 0; d < RT; ++d)
+          if (d < rt)
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+              const uint2 a = *reinterpret_cast<const uint2*>(lap_lds + v_at[2 * c] + 2048 * d);
+              const uint2 e = *reinterpret_cast<const uint2*>(lap_lds + v_at[2 * c + 1] + 2048 * d);
+              acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(la_frag(make_uint4(a.x, a.y, e.x, e.y)), la_frag(pf[c]), acc[d], 0, 0, 0);
+            }
+      }
+    }
+  }
   if (!active) return;
   const float inv = 1.0f / l;
   float* dst = o_lat + ((long)t * heads + hg * 16 + j) * rank + 4 * g;
@@ -575,24 +606,20 @@ latent_attention_fold_kernel(const float* __restrict__ partial, float* __restric
   }
 }
 
-// Steps of many tokens (no blocks side by side): four tokens a block, their pages staged in LDS once.
-static long latent_tokens_lds(int rank, int rot) {
-  const long qrow = rank + rot + 8, stage = 64 * qrow > (long)rank * 72 ? 64 * qrow : (long)rank * 72;
-  return (stage + LAS_WAVES * 16 * qrow) * (long)sizeof(bf16_t);
-}
+// Steps of many tokens (no blocks side by side): eight tokens a block, their pages staged in LDS once.
 #define LATENT_LDS_MOST (160 * 1024)
 
-template <int RT, int QC>
-static int launch_latent_mfma_tokens(const float* q_full, const void* cache, const int32_t* block_table, int table_stride,
-                                     const int32_t* positions, const int32_t* seq_rows, float* o_lat, int n_tokens, int heads, int rank,
-                                     int rot, int page_size, int window, float scale, const float* sink, hipStream_t stream) {
-  const int lds = (int)latent_tokens_lds(rank, rot);
+template <int RT, int QC, bool EXACT>
+static int launch_latent_prompt(const float* q_full, const void* cache, const int32_t* block_table, int table_stride,
+                                const int32_t* positions, const int32_t* seq_rows, float* o_lat, int n_tokens, int heads, int rank,
+                                int rot, int page_size, int window, float scale, const float* sink, hipStream_t stream) {
+  const int lds = 128 * (rank + rot) + 128 * rank;
   static bool configured = false;
   if (!configured) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&latent_attention_mfma_tokens_kernel<RT, QC, true>),
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&latent_attention_prompt_kernel<RT, QC, EXACT, true>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, LATENT_LDS_MOST);
     if (e == hipSuccess)
-      e = hipFuncSetAttribute(reinterpret_cast<const void*>(&latent_attention_mfma_tokens_kernel<RT, QC, false>),
+      e = hipFuncSetAttribute(reinterpret_cast<const void*>(&latent_attention_prompt_kernel<RT, QC, EXACT, false>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, LATENT_LDS_MOST);
     if (e != hipSuccess) {
       axk_set_error("latent_attention: cannot reserve %d bytes of LDS: %s", LATENT_LDS_MOST, hipGetErrorString(e));
@@ -600,13 +627,13 @@ static int launch_latent_mfma_tokens(const float* q_full, const void* cache, con
     }
     configured = true;
   }
-  const unsigned grid = (unsigned)(((n_tokens + LAS_WAVES - 1) / LAS_WAVES) * (heads / 16));
+  const unsigned grid = (unsigned)(((n_tokens + LAP_TOKENS - 1) / LAP_TOKENS) * (heads / 16));
   if (sink)
-    latent_attention_mfma_tokens_kernel<RT, QC, true><<<grid, LAS_WAVES * 64, lds, stream>>>(
+    latent_attention_prompt_kernel<RT, QC, EXACT, true><<<grid, LAP_TOKENS * 64, lds, stream>>>(
         q_full, (const bf16_t*)cache, block_table, table_stride, positions, seq_rows, o_lat, n_tokens, heads, rank, rot, page_size, window,
         scale, sink);
   else
-    latent_attention_mfma_tokens_kernel<RT, QC, false><<<grid, LAS_WAVES * 64, lds, stream>>>(
+    latent_attention_prompt_kernel<RT, QC, EXACT, false><<<grid, LAP_TOKENS * 64, lds, stream>>>(
         q_full, (const bf16_t*)cache, block_table, table_stride, positions, seq_rows, o_lat, n_tokens, heads, rank, rot, page_size, window,
         scale, sink);
   return 0;
@@ -616,17 +643,17 @@ template <int RT, int QC>
 static void launch_latent_mfma(const float* q_full, const void* cache, const int32_t* block_table, int table_stride,
                                const int32_t* positions, const int32_t* seq_rows, float* o_lat, int n_tokens, int heads, int rank,
                                int rot, int page_size, int window, float scale, const float* sink, float* partial, int n_chunks,
-                               hipStream_t stream) {
+                               bool mixed_only, hipStream_t stream) {
   const long items = (long)n_tokens * (heads / 16);
   dim3 grid((unsigned)((items + LAM_WAVES - 1) / LAM_WAVES), partial ? n_chunks : 1);
   if (sink)
     latent_attention_mfma_kernel<RT, QC, true><<<grid, LAM_WAVES * 64, 0, stream>>>(
         q_full, (const bf16_t*)cache, block_table, table_stride, positions, seq_rows, o_lat, n_tokens, heads, rank, rot, page_size,
-        window, scale, sink, partial, n_chunks);
+        window, scale, sink, partial, n_chunks, mixed_only);
   else
     latent_attention_mfma_kernel<RT, QC, false><<<grid, LAM_WAVES * 64, 0, stream>>>(
         q_full, (const bf16_t*)cache, block_table, table_stride, positions, seq_rows, o_lat, n_tokens, heads, rank, rot, page_size,
-        window, scale, sink, partial, n_chunks);
+        window, scale, sink, partial, n_chunks, mixed_only);
   if (partial)
     latent_attention_fold_kernel<<<n_tokens * heads, min(512, (rank + 63) / 64 * 64), 3 * n_chunks * sizeof(float), stream>>>(
         partial, o_lat, rank, n_chunks, sink, heads);
@@ -712,30 +739,30 @@ extern "C" int axk_latent_attention(const float* q_full, const void* cache, cons
                 partial_floats, need);
     if (need == 0) partial = nullptr;
     const int n_chunks = latent_blocks_side_by_side(window, span);
-    if (partial == nullptr && (long)n_tokens * (heads / 16) >= LATENT_TOKENS_KERNEL_FROM && latent_tokens_lds(rank, rot) <= LATENT_LDS_MOST) {
+    const bool many = partial == nullptr && (long)n_tokens * (heads / 16) >= LATENT_PROMPT_KERNEL_FROM;
+    if (many) {
+#define LATENT_PROMPT(RT, QC, EXACT)                                                                                                      \
+  launch_latent_prompt<RT, QC, EXACT>(q_full, cache, block_table, table_stride, positions, seq_rows, o_lat, n_tokens, heads, rank, rot, page_size, \
+                               window, scale, sink, s)
       int rc;
-      if (rank <= 64 && rank + rot <= 128)
-        rc = launch_latent_mfma_tokens<4, 4>(q_full, cache, block_table, table_stride, positions, seq_rows, o_lat, n_tokens, heads, rank,
-                                             rot, page_size, window, scale, sink, s);
-      else if (rank <= 128 && rank + rot <= 256)
-        rc = launch_latent_mfma_tokens<8, 8>(q_full, cache, block_table, table_stride, positions, seq_rows, o_lat, n_tokens, heads, rank,
-                                             rot, page_size, window, scale, sink, s);
-      else
-        rc = launch_latent_mfma_tokens<32, 20>(q_full, cache, block_table, table_stride, positions, seq_rows, o_lat, n_tokens, heads,
-                                               rank, rot, page_size, window, scale, sink, s);
+      // a latent of 512 beside 64 rotated dims: every bound known when compiled, so that a block's reads of LDS can be one
+      // stretch of instructions (no branch may stand between such a read and its wait)
+      if (rank == 512 && rot == 64) rc = LATENT_PROMPT(32, 18, true);
+      else if (rank <= 64 && rank + rot <= 128) rc = LATENT_PROMPT(4, 4, false);
+      else if (rank <= 128 && rank + rot <= 256) rc = LATENT_PROMPT(8, 8, false);
+      else rc = LATENT_PROMPT(32, 20, false);
+#undef LATENT_PROMPT
       if (rc) return rc;
-      AXK_LAUNCH_CHECK("latent_attention");
-      return 0;
     }
     if (rank <= 64 && rank + rot <= 128)
       launch_latent_mfma<4, 4>(q_full, cache, block_table, table_stride, positions, seq_rows, o_lat, n_tokens, heads, rank, rot,
-                               page_size, window, scale, sink, partial, n_chunks, s);
+                               page_size, window, scale, sink, partial, n_chunks, many, s);
     else if (rank <= 128 && rank + rot <= 256)
       launch_latent_mfma<8, 8>(q_full, cache, block_table, table_stride, positions, seq_rows, o_lat, n_tokens, heads, rank, rot,
-                               page_size, window, scale, sink, partial, n_chunks, s);
+                               page_size, window, scale, sink, partial, n_chunks, many, s);
     else
       launch_latent_mfma<32, 20>(q_full, cache, block_table, table_stride, positions, seq_rows, o_lat, n_tokens, heads, rank, rot,
-                                 page_size, window, scale, sink, partial, n_chunks, s);
+                                 page_size, window, scale, sink, partial, n_chunks, many, s);
     AXK_LAUNCH_CHECK("latent_attention");
     return 0;
   }
