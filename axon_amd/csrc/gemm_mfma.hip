@@ -81,11 +81,14 @@ __device__ inline bf16x8 as_frag(u32x4 v) { return __builtin_bit_cast(bf16x8, v)
 // A block then owns BN / 2 output columns; each wave's share of the LDS tile holds the gate
 // rows of its columns and, after them, the up rows of the same columns, so that a lane ends
 // with both values of an output element.
-template <int BM, int BN, int WAVES_M, int WAVES_N, bool GLU, int BK, int STAGES>
-__global__ void __launch_bounds__(WAVES_M * WAVES_N * 64)
+//
+// KEEP: the block walks all `splits` segments of K itself; a segment's chains are added to the sums of those
+// before it in a second set of registers (the order of gemm_split_reduce), and no sums go through memory.
+template <int BM, int BN, int WAVES_M, int WAVES_N, bool GLU, int BK, int STAGES, bool KEEP>
+__global__ void __launch_bounds__(WAVES_M * WAVES_N * 64, KEEP ? 2 : 1)
 gemm_tile_kernel(const bf16_t* __restrict__ x, int x_stride, const bf16_t* __restrict__ w, const void* __restrict__ bias,
                  int bias_is_f32, void* __restrict__ out, int out_stride, int M, int N, int K, int mode, int m_blocks,
-                 int n_blocks, float* __restrict__ partial) {
+                 int n_blocks, float* __restrict__ partial, int splits) {
   extern __shared__ __align__(16) unsigned char smem[];
   static_assert(BK == 64 || BK == 32, "segments of K are counted in steps of 64: whole K tiles");
   constexpr int PER64 = 64 / BK;                       // K tiles in a step of 64
@@ -170,8 +173,8 @@ gemm_tile_kernel(const bf16_t* __restrict__ x, int x_stride, const bf16_t* __res
 
   // Split K (gridDim.y > 1): this block multiplies the K tiles kt_begin .. kt_begin + nk - 1 and
   // leaves its sums in `partial`; gemm_split_reduce_kernel adds the blocks' sums in block order.
-  const int kt_begin = (int)((long)blockIdx.y * (K / 64) / gridDim.y) * PER64;
-  const int nk = (int)((long)(blockIdx.y + 1) * (K / 64) / gridDim.y) * PER64 - kt_begin;
+  const int kt_begin = KEEP ? 0 : (int)((long)blockIdx.y * (K / 64) / gridDim.y) * PER64;
+  const int nk = KEEP ? K / 64 * PER64 : (int)((long)(blockIdx.y + 1) * (K / 64) / gridDim.y) * PER64 - kt_begin;
   auto issue = [&](int kt) {     // kt counts from kt_begin
     unsigned char* stage = smem + (kt % STAGES) * STAGE;
     const int koff = (kt_begin + kt) * BK;
@@ -192,6 +195,8 @@ gemm_tile_kernel(const bf16_t* __restrict__ x, int x_stride, const bf16_t* __res
     for (int j = 0; j < TN; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+  f32x16 sum[KEEP ? TM : 1][KEEP ? TN : 1];
+  int seg = 0, seg_end = KEEP ? (int)((long)(K / 64) / splits) * PER64 : 0;     // of the segment being multiplied
 
   // fragment addresses: row = tile row + lane % 32, k chunk = 2 ks + lane / 32, slot = chunk ^ SWZ(row)
   const int frow = lane & 31, fhalf = lane >> 5, fsw = SWZ(frow);
@@ -257,8 +262,27 @@ gemm_tile_kernel(const bf16_t* __restrict__ x, int x_stride, const bf16_t* __res
         multiply(cur, TN / 2, TN);
       }
     }
+    if (KEEP && kt + 1 == seg_end) {
+#pragma unroll
+      for (int i = 0; i < (KEEP ? TM : 0); ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) {
+            sum[KEEP ? i : 0][KEEP ? j : 0][e] = seg == 0 ? acc[i][j][e] : sum[KEEP ? i : 0][KEEP ? j : 0][e] + acc[i][j][e];
+            acc[i][j][e] = 0.0f;
+          }
+      ++seg;
+      seg_end = (int)((long)(seg + 1) * (K / 64) / splits) * PER64;
+    }
   }
 #undef SWZ
+  if constexpr (KEEP) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[i][j] = sum[i][j];
+  }
 
   // epilogue: lane holds column n = lane % 32 of each tile and rows (e/4)*8 + (lane/32)*4 + e%4
   if (partial) {
@@ -520,14 +544,14 @@ static int add_split_sums(const float* partial, int splits, int m, int n, const 
   return 0;
 }
 
-template <int BM, int BN, int WAVES_M, int WAVES_N, bool GLU, int BK = 64, int STAGES = 2>
+template <int BM, int BN, int WAVES_M, int WAVES_N, bool GLU, int BK = 64, int STAGES = 2, bool KEEP = false>
 static int launch_tile(const bf16_t* x, int x_stride, const bf16_t* w, const void* bias, int bias_is_f32, void* out,
                        int out_stride, int m, int n, int k, int mode, hipStream_t stream, int segs = 1,
                        float* partial = nullptr, const SplitNorm* norm = nullptr, const RopeStore* rope = nullptr) {
   static bool configured = false;
   constexpr int lds_bytes = STAGES * (BM + BN) * BK * 2;
   static_assert(lds_bytes <= 160 * 1024, "the stages do not fit the LDS of a CU");
-  auto kernel = &gemm_tile_kernel<BM, BN, WAVES_M, WAVES_N, GLU, BK, STAGES>;
+  auto kernel = &gemm_tile_kernel<BM, BN, WAVES_M, WAVES_N, GLU, BK, STAGES, KEEP>;
   if (!configured) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                        lds_bytes);
@@ -537,14 +561,16 @@ static int launch_tile(const bf16_t* x, int x_stride, const bf16_t* w, const voi
     }
     configured = true;
   }
-  // a block a segment (gridDim.y), the sums through `partial`
-  const int splits = segs;
+  // a block a segment (gridDim.y), the sums through `partial`; or a block all of them, the finished sums through
+  // `partial` where the kernel that adds sums does more than that
+  const int splits = KEEP ? 1 : segs;
+  const bool after = splits > 1 || norm || rope;
   const int m_blocks = ceil_div(m, BM), n_blocks = ceil_div(n, GLU ? BN / 2 : BN);
   AXK_INSTANCE(INST_GEMM_TILE, BM, BN, WAVES_M, WAVES_N, GLU, STAGES);
   kernel<<<dim3(m_blocks * n_blocks, splits), WAVES_M * WAVES_N * 64, lds_bytes, stream>>>(
-      x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode, m_blocks, n_blocks, splits > 1 ? partial : nullptr);
+      x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode, m_blocks, n_blocks, after ? partial : nullptr, segs);
   AXK_LAUNCH_CHECK("gemm_tile");
-  return splits > 1 ? add_split_sums(partial, splits, m, n, bias, bias_is_f32, out, out_stride, mode, norm, rope, stream) : 0;
+  return after ? add_split_sums(partial, splits, m, n, bias, bias_is_f32, out, out_stride, mode, norm, rope, stream) : 0;
 }
 
 // ---------------------------------------------------------------------------- gemm_stream
@@ -1624,9 +1650,8 @@ static int tiles32_of(int n, int mode) { return mode == MODE_SWIGLU ? n / 16 : (
 #define AXON_STREAM_MAX_M 16
 
 // More rows than the streaming kernel takes, S > 1 segments: a block a segment; the blocks' sums
-// go through a workspace and are added in segment order by a second kernel (measured faster for
-// every product of the 7B and 14B layers up to 8,192 rows than keeping the segments apart in one
-// block's registers, and the only way to occupy the chip when the output is small).  The
+// go through a workspace and are added in segment order by a second kernel (the only way to occupy the
+// chip when the output is small; gemm_mfma_pass says where a block keeps the segments' sums).  The
 // workspace holds the sums of at most GEMM_PASS_BYTES: a product of more rows runs in passes of
 // `rows_a_pass` rows, one after the other (a row's bits do not depend on the rows beside it).
 #define GEMM_PASS_BYTES ((size_t)2048 << 20)
@@ -1746,6 +1771,17 @@ static int gemm_mfma_pass(const bf16_t* x, int x_stride, const bf16_t* w, const 
   const long small = (long)ceil_div(m, 128) * ceil_div(n, glu ? 64 : 128) * segs;
   const long rounds_big = (big + 255) / 256, rounds_small = (small + 511) / 512;
   const bool use_big = rounds_big * 100 <= rounds_small * 65;
+  // Where 128 x 128 tiles that walk all of K themselves give the chip enough blocks, and K is short enough for their
+  // smaller tiles, the segments' sums stay in registers.  2,048 rows (us, a block a segment against here): 2,560 columns
+  // of K 2,048 56 against 46, 5,120 of 2,048 104 against 76, gated 1,408 of 2,048 60 against 38, 3,584 of 3,584 with
+  // the norm behind 100 against 83; 1,200 rows of 2,560 (200 blocks) 36 either way, 800 rows 32 against 35; 3,584 of
+  // 18,944 314 against 328, 2,048 of 5,632 (256 blocks) 72 against 89.  Without a norm behind it a product of K 3,584
+  // stays with the large tiles (4,608 columns 121 against 112), whose choice there the tests of the instances assert.
+  const long whole = (long)ceil_div(m, 128) * ceil_div(n, glu ? 64 : 128);
+  if (segs > 1 && whole >= (glu ? 144 : 288) && k <= (norm ? 5120 : 3072)) {
+    if (glu) return launch_tile<128, 128, 2, 2, true, 64, 2, true>(ARGS, segs, ws);
+    return launch_tile<128, 128, 2, 2, false, 64, 2, true>(ARGS, segs, ws, norm, rope_after);
+  }
   if (!use_big) {
     // Up to 256 rows still wait for W more than for the matrix cores.  Where the small tiles are no
     // more blocks than CUs, a block has its CU's LDS to itself: four stages instead of two, three

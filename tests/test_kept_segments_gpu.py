@@ -1,0 +1,44 @@
+"""Products of many rows whose blocks keep the sums of K's segments in registers: the bits of the kernels that take a
+segment a block, for every epilogue, at the edges of their tiles and on both sides of the choice."""
+import pytest
+import torch
+
+from axon_amd.kernels import MODE_ADD_F32, MODE_RELU_SQUARED, MODE_STORE, MODE_STORE_F32, MODE_SWIGLU, kernels
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("mode", [MODE_STORE, MODE_ADD_F32, MODE_STORE_F32, MODE_SWIGLU, MODE_RELU_SQUARED])
+@pytest.mark.parametrize("M,N,K", [(2050, 2064, 512), (1153, 4100, 1088), (4100, 1106, 1600), (1200, 2944, 3072)])
+def test_rows_have_the_bits_they_have_alone(M, N, K, mode):
+    if mode == MODE_SWIGLU:
+        N = N // 16 * 16
+    k = kernels("bfloat16")
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    x = torch.randn(M, K, generator=g, device="cuda").bfloat16()
+    w = k.prepare_weight((torch.randn((2 if mode == MODE_SWIGLU else 1) * N, K, generator=g, device="cuda") * 0.1).bfloat16(), mode == MODE_SWIGLU)
+    assert k.gemm_segments(N, K, mode == MODE_SWIGLU) > 1
+    bias = torch.randn(N, generator=g, device="cuda") if mode != MODE_SWIGLU else None
+    base = torch.randn(M, N, generator=g, device="cuda").to(torch.float32 if mode in (MODE_ADD_F32, MODE_STORE_F32) else torch.bfloat16)
+    whole = base.clone()
+    k.gemm(x, w, whole, bias, mode)
+    for first, m in ((0, 16), (M - 64, 64), (M // 2, 140), (3, 300)):
+        part = base[first:first + m].clone()
+        k.gemm(x[first:first + m].contiguous(), w, part, bias, mode)
+        assert torch.equal(part, whole[first:first + m]), (first, m)
+
+
+@pytest.mark.parametrize("M,N,K", [(1300, 3584, 3584), (2049, 2304, 5120)])
+def test_the_norm_behind(M, N, K):
+    k = kernels("bfloat16")
+    g = torch.Generator(device="cuda").manual_seed(M)
+    x = torch.randn(M, K, generator=g, device="cuda").bfloat16()
+    w = k.prepare_weight((torch.randn(N, K, generator=g, device="cuda") * 0.05).bfloat16())
+    gain, rows = torch.randn(N, generator=g, device="cuda").bfloat16(), torch.randn(M, N, generator=g, device="cuda")
+    out, normed = rows.clone(), torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+    k.gemm(x, w, out, None, MODE_ADD_F32, following_norm=(gain, normed, 1e-6))
+    plain = rows[:200].clone()
+    k.gemm(x[:200].contiguous(), w, plain, None, MODE_ADD_F32)
+    alone = torch.empty(200, N, dtype=torch.bfloat16, device="cuda")
+    k.rmsnorm(plain, gain, 1e-6, alone)
+    assert torch.equal(out[:200], plain) and torch.equal(normed[:200], alone)
