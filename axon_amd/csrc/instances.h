@@ -27,6 +27,7 @@ enum {
   INST_ATTENTION_DECODE,     // head_dim, waves a block
   INST_RMSNORM,              // 1: rows read as float4
   INST_GROUPED_GEMM,         // 2: matrix cores through LDS, 1: matrix cores from memory, 0: 32-bit FMA; gated epilogue
+  INST_CAUSAL_CONV,          // 1: runs of tokens, 0: a thread a (token, channel)
   INST_KINDS
 };
 

@@ -11,6 +11,7 @@
 // two tokens belong to one request iff their state slots (seq_rows) are equal.
 #include "api.h"
 #include "common.h"
+#include "instances.h"
 
 namespace {
 
@@ -44,7 +45,10 @@ __global__ void causal_conv_kernel(const elem_t* __restrict__ x, long x_stride, 
 
 // The same for many tokens: a thread takes four channels of CONV_RUN tokens, whose inputs (and the taps - 1 before them) it
 // asks for at once and keeps in registers, where a thread a (token, channel) reads each `taps` times and waits for its
-// row's slot first.  The sums in the same order.  2,048 tokens of 2,560 channels: 38 -> 24 us.
+// row's slot first.  Runs in which a request begins also ask for the kept inputs of all their tokens at once.  The sums in
+// the same order.  Bound by the three waits (slots, inputs, outputs) of the one round of blocks; 2,560 channels, us, a thread
+// a (token, channel) against here: 2,048 tokens of one request 38.7 / 13.4, of requests of 16 37.6 / 15.0, of 2,048 requests
+// 31.0 / 20.9; 512 of one 9.3 / 7.6.
 #define CONV_RUN 8
 #define CONV_TAPS 4           // at most
 __global__ void __launch_bounds__(128)
@@ -61,47 +65,58 @@ causal_conv_run_kernel(const elem_t* __restrict__ x, long x_stride, const elem_t
     slots[i] = t == t0 + i - (CONV_TAPS - 1) ? seq_rows[t] : -1;
     load4_guarded(x + (long)t * x_stride + c, 4, true, in[i]);
   }
-  float wk[4][CONV_TAPS];
+  float wb[CONV_TAPS][4];                            // the weights of the input `back` tokens before
 #pragma unroll
-  for (int e = 0; e < 4; ++e)
+  for (int back = 0; back < CONV_TAPS; ++back)
 #pragma unroll
-    for (int k = 0; k < CONV_TAPS; ++k) wk[e][k] = k < taps ? to_float(w[(long)(c + e) * taps + k]) : 0.0f;
+    for (int e = 0; e < 4; ++e) wb[back][e] = back < taps ? to_float(w[(long)(c + e) * taps + taps - 1 - back]) : 0.0f;
+  float added[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  if (bias)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) added[e] = load_vec(bias, bias_is_f32, c + e);
+
+  int inside[CONV_RUN];                              // earlier tokens of this step that belong to the same request
+  bool begins = false;
 #pragma unroll
   for (int r = 0; r < CONV_RUN; ++r) {
-    const int t = t0 + r;
-    if (t >= n_tokens) break;
-    const int slot = slots[r + CONV_TAPS - 1];
-    int inside = 0;                                  // earlier tokens of this step that belong to the same request
+    inside[r] = 0;
 #pragma unroll
     for (int b = 1; b < CONV_TAPS; ++b)
-      if (b < taps && inside == b - 1 && slots[r + CONV_TAPS - 1 - b] == slot) inside = b;
+      if (b < taps && inside[r] == b - 1 && slots[r + CONV_TAPS - 1 - b] == slots[r + CONV_TAPS - 1]) inside[r] = b;
+    begins |= t0 + r < n_tokens && inside[r] < taps - 1;
+  }
+  float kept[CONV_RUN][CONV_TAPS - 1][4];            // the inputs 1 .. CONV_TAPS - 1 tokens before, from the state
+  if (begins) {                                      // the same for the whole block
+#pragma unroll
+    for (int r = 0; r < CONV_RUN; ++r) {
+      const int t = min(t0 + r, n_tokens - 1);
+      const int before = (positions[t] - inside[r] + 1) & 1;
+      const float* row = state + (long)seq_rows[t] * state_stride + (long)before * taps * channels + channels + c;
+#pragma unroll
+      for (int back = 1; back < CONV_TAPS; ++back) {
+        const bool needed = back < taps && back > inside[r];       // (else any row that is there)
+        const float4 v = *reinterpret_cast<const float4*>(row + (needed ? (long)(taps - 1 - (back - inside[r])) * channels : -(long)channels));
+        kept[r][back - 1][0] = v.x; kept[r][back - 1][1] = v.y; kept[r][back - 1][2] = v.z; kept[r][back - 1][3] = v.w;
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < CONV_RUN; ++r) {
+    if (t0 + r >= n_tokens) break;
     float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (inside == taps - 1) {
 #pragma unroll
-      for (int k = 0; k < CONV_TAPS; ++k)
-        if (k < taps) {
-          // the input taps - 1 - k tokens before: its place in `in` by a constant, chosen among the taps there can be
+    for (int back = CONV_TAPS - 1; back >= 0; --back) {
+      if (back >= taps) continue;
 #pragma unroll
-          for (int back = 0; back < CONV_TAPS; ++back)
-            if (back == taps - 1 - k)
-#pragma unroll
-              for (int e = 0; e < 4; ++e) acc[e] = fmaf(wk[e][k], in[r + CONV_TAPS - 1 - back][e], acc[e]);
-        }
-    } else {
-      const int before = (positions[t] - inside + 1) & 1;
-      const float* kept = state + (long)slot * state_stride + (long)before * taps * channels + channels;
-      for (int k = 0; k < taps; ++k) {
-        const int back = taps - 1 - k;
-        for (int e = 0; e < 4; ++e) {
-          const float v = back <= inside ? to_float(x[(long)(t - back) * x_stride + c + e]) : kept[(long)(taps - 1 - (back - inside)) * channels + c + e];
-          acc[e] = fmaf(to_float(w[(long)(c + e) * taps + k]), v, acc[e]);
-        }
+      for (int e = 0; e < 4; ++e) {
+        const float v = back > 0 && begins && back > inside[r] ? kept[r][back > 0 ? back - 1 : 0][e] : in[r + CONV_TAPS - 1 - back][e];
+        acc[e] = fmaf(wb[back][e], v, acc[e]);
       }
     }
     if (bias)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) acc[e] += load_vec(bias, bias_is_f32, c + e);
-    *reinterpret_cast<float4*>(u + (long)t * channels + c) = make_float4(acc[0], acc[1], acc[2], acc[3]);
+      for (int e = 0; e < 4; ++e) acc[e] += added[e];
+    *reinterpret_cast<float4*>(u + (long)(t0 + r) * channels + c) = make_float4(acc[0], acc[1], acc[2], acc[3]);
   }
 }
 
@@ -254,15 +269,19 @@ extern "C" int axk_causal_conv(const void* x, long x_stride, const void* w, cons
               state_stride, taps, channels);
   AXK_REQUIRE(n_tokens <= 65535, "causal_conv: %d tokens in one step (at most 65535)", n_tokens);
   if (n_tokens == 0) return 0;
-  // runs of tokens once there are some of them for every CU and rows can be read four elements at a time; a step of
-  // fewer tokens is bound by its launch, and a thread a channel has less to wait for
-  if (n_tokens >= 64 && taps <= CONV_TAPS && channels % 4 == 0 && x_stride % 4 == 0 && (uintptr_t)x % (4 * sizeof(elem_t)) == 0 &&
-      ((uintptr_t)u & 15) == 0) {
+  // A step has to be long enough for a run to pay: blocks of 8 tokens x 512 channels wait one after another where a thread a
+  // (token, channel) has a wave for every wait.  2,560 channels (us, a thread each against runs): 64 tokens 3.6 / 6.8, 256
+  // 6.0 / 7.0, 512 9.3 / 7.6, 512 requests of a token 9.4 / 9.4; 512 channels: 2,048 tokens 8.0 / 7.0, 2,048 requests 6.9 / 7.7.
+  const bool by_fours = channels % 4 == 0 && x_stride % 4 == 0 && (uintptr_t)x % (4 * sizeof(elem_t)) == 0 && ((uintptr_t)u & 15) == 0 &&
+                        state_stride % 4 == 0 && ((uintptr_t)state & 15) == 0;
+  if (by_fours && taps <= CONV_TAPS && (long)n_tokens * channels >= 512 * 2560) {
+    AXK_INSTANCE(INST_CAUSAL_CONV, 1);
     causal_conv_run_kernel<<<dim3(ceil_div(channels / 4, 128), ceil_div(n_tokens, CONV_RUN)), 128, 0, (hipStream_t)stream>>>(
         (const elem_t*)x, x_stride, (const elem_t*)w, bias, bias_is_f32, state, state_stride, positions, seq_rows, u, n_tokens, channels, taps);
     AXK_LAUNCH_CHECK("causal_conv");
     return 0;
   }
+  AXK_INSTANCE(INST_CAUSAL_CONV, 0);
   dim3 grid(ceil_div(channels, 256), n_tokens);
   causal_conv_kernel<<<grid, 256, 0, (hipStream_t)stream>>>((const elem_t*)x, x_stride, (const elem_t*)w, bias, bias_is_f32,
                                                            state, state_stride, positions, seq_rows, u, channels, taps);

@@ -246,6 +246,29 @@ def check_grouped(dtype, M, G, N, K, glu):
     return hit
 
 
+def check_conv(dtype, T, C):
+    """The short causal convolution of one request that goes on, and of the tokens behind it, one request each."""
+    k = kernels(dtype)
+    td = torch.bfloat16 if dtype == "bfloat16" else torch.float32
+    taps, long_one = 4, T - 5
+    x = rnd(T, C, seed=70, device="cuda").to(td)
+    w, bias = rnd(C, taps, seed=71, device="cuda").to(td), rnd(C, seed=72, device="cuda")
+    state = rnd(6, 2 * taps * C, seed=73, device="cuda")
+    seq = torch.tensor([0] * long_one + [1, 2, 3, 4, 5], dtype=torch.int32).cuda()
+    pos = torch.tensor(list(range(9, 9 + long_one)) + [8, 9, 10, 11, 12], dtype=torch.int32).cuda()
+    u = torch.empty(T, C, device="cuda")
+    hit = launched(k, dtype, lambda: k.causal_conv(x, w, bias, state, pos, seq, u))
+    for first, n, slot, start in [(0, long_one, 0, 9)] + [(long_one + i, 1, 1 + i, 8 + i) for i in range(5)]:
+        before = (start - 1) & 1                             # the copy behind the position before the request's first
+        kept = state[slot, before * taps * C + C:(before + 1) * taps * C].view(taps - 1, C)
+        rows = torch.cat([kept.double(), x[first:first + n].double()])
+        want = bias.double() + sum(rows[i:i + n] * w.double()[:, i] for i in range(taps))
+        # four products and a bias, each sum rounded by at most half a unit of what it holds
+        bound = 6 * 2.0 ** -24 * (bias.double().abs() + sum((rows[i:i + n] * w.double()[:, i]).abs() for i in range(taps)))
+        assert bool(((u[first:first + n].double() - want).abs() <= bound).all())
+    return hit
+
+
 CASES = [
     # 32-bit FMA products: the float32 build's, and the bfloat16 build's for what cannot be packed
     (F32, ["gemm_fma<16,0>"], check_gemm, (F32, 5, 100, 70, MODE_STORE_F32, True)),
@@ -387,6 +410,11 @@ CASES = [
     (BF, ["grouped_gemm<2,1>"], check_grouped, (BF, 270, 2, 72, 160, True)),
     (F32, ["grouped_gemm<0,0>"], check_grouped, (F32, 50, 3, 40, 64, False)),
     (F32, ["grouped_gemm<0,1>"], check_grouped, (F32, 19, 2, 72, 160, True)),
+    # the short convolution: a thread a (token, channel), and runs of tokens in long steps
+    (BF, ["causal_conv<0>"], check_conv, (BF, 256, 2560)),
+    (BF, ["causal_conv<1>"], check_conv, (BF, 517, 2564)),
+    (F32, ["causal_conv<0>"], check_conv, (F32, 1023, 260)),
+    (F32, ["causal_conv<1>"], check_conv, (F32, 2049, 640)),
     # attention on the matrix cores: (head size, query heads a block, pages of 64 positions or more)
     # and (head size, waves a block) (one wave a block in the decoding kernel up to 2,560 blocks of
     # positions, four beyond; two heads a block in the prompt kernel where tiles x heads are more

@@ -20,7 +20,9 @@ def _rows(lengths, device):
 
 @pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
 @pytest.mark.parametrize("taps", [2, 3, 4])
-@pytest.mark.parametrize("lengths, channels", [([64], 4), ([1, 2, 3, 4, 5, 70], 520), ([33, 7, 1, 9, 8, 8, 15], 512), ([127, 2], 2564)])
+@pytest.mark.parametrize("lengths, channels", [([64], 4), ([1, 2, 3, 4, 5, 70], 520), ([33, 7, 1, 9, 8, 8, 15], 512), ([127, 2], 2564),
+                                               ([520], 2564), ([1] * 513, 2560), ([1, 2, 3, 4, 5, 1290, 33, 7, 1, 9, 8, 8, 15], 960),
+                                               ([5000, 246, 3], 252)])
 def test_convolution_by_runs(dtype, taps, lengths, channels):
     from axon_amd.kernels import kernels
     k, dev = kernels(dtype), "cuda:0"
@@ -35,7 +37,10 @@ def test_convolution_by_runs(dtype, taps, lengths, channels):
     state = torch.randn(len(lengths), 2 * taps * channels, device=dev)
     for bias in (None, torch.randn(channels, device=dev)):
         got, want = (torch.empty(T, channels, device=dev) for _ in range(2))
+        k.reset_instances()
         k.causal_conv(x, w, bias, state, pos, seq, got)
+        # a step of few (token, channel) pairs, a batch of decoding rows among them, keeps a thread each
+        assert k.instances(launched=True) == [f"causal_conv<{1 if T * channels >= 512 * 2560 else 0}>"]
         k.causal_conv(odd, w, bias, state, pos, seq, want)
         assert torch.equal(got, want)
 
