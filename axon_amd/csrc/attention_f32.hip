@@ -241,21 +241,97 @@ attention_f32_prefill_kernel(const float* __restrict__ q, int q_stride, const fl
 }
 
 // ============================================================================ decoding tokens
+// One block of 64 positions for the heads of a group; NT: its tiles of 16 positions up to the token's own.
+template <int HD, int NT>
+__device__ __forceinline__ void f32_decode_block(const float* __restrict__ qrow, const float* __restrict__ k_head,
+                                                 const float* __restrict__ v_head, const int32_t* __restrict__ table_row,
+                                                 size_t page_stride, int page_size, int p0, int lo, int pos, float scale, int r16,
+                                                 int g4, bool head_live, float* __restrict__ dst) {
+  constexpr int KG = HD / 16, DT = HD / 16;
+  f32x4 kf[NT][KG], vf[NT][DT], qf[KG];
+  int k_page[NT], v_page[NT];
+#pragma unroll
+  for (int i = 0; i < NT; ++i) {
+    k_page[i] = table_row[page_index(min(p0 + 16 * i + r16, pos), page_size)];
+    v_page[i] = table_row[page_index(min(p0 + 16 * i + 4 * g4, pos), page_size)];
+  }
+#pragma unroll
+  for (int i = 0; i < NT; ++i) {
+    const float* kr = k_head + (size_t)k_page[i] * page_stride + (size_t)page_offset(min(p0 + 16 * i + r16, pos), page_size) * HD;
+#pragma unroll
+    for (int g = 0; g < KG; ++g) kf[i][g] = *reinterpret_cast<const f32x4*>(kr + 16 * g + 4 * g4);
+  }
+#pragma unroll
+  for (int g = 0; g < KG; ++g) qf[g] = *reinterpret_cast<const f32x4*>(qrow + 16 * g + 4 * g4);
+#pragma unroll
+  for (int i = 0; i < NT; ++i) {
+    const float* vr = v_head + (size_t)v_page[i] * page_stride + (page_offset(min(p0 + 16 * i + 4 * g4, pos), page_size) & ~3);
+#pragma unroll
+    for (int d = 0; d < DT; ++d) vf[i][d] = *reinterpret_cast<const f32x4*>(vr + (size_t)(16 * d + r16) * page_size);
+  }
+
+  f32x4 s[4] = {F32_ZERO, F32_ZERO, F32_ZERO, F32_ZERO};
+#pragma unroll
+  for (int g = 0; g < KG; ++g) {
+    const f32x4 qo = f32_operand(qf[g]);
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+      const f32x4 a = f32_operand(kf[i][g]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) F32_STEP(s[i], a, qo, j);
+    }
+  }
+  float m_b, l_b;
+  f32_weights(s, p0, lo, pos, scale, g4, m_b, l_b);
+  // the weight of a position outside the token's range is 0, and so must be what it is multiplied with
+  if (p0 < lo || p0 + ATT_BLOCK - 1 > pos) {
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int p = p0 + 16 * i + 4 * g4 + e;
+        const bool live = p >= lo && p <= pos;
+#pragma unroll
+        for (int d = 0; d < DT; ++d) vf[i][d][e] = live ? vf[i][d][e] : 0.0f;
+      }
+  }
+  f32x4 o[DT];
+#pragma unroll
+  for (int d = 0; d < DT; ++d) o[d] = F32_ZERO;
+#pragma unroll
+  for (int i = 0; i < NT; ++i) {
+    const f32x4 pf = f32_operand(s[i]);
+#pragma unroll
+    for (int d = 0; d < DT; ++d) {
+      const f32x4 a = f32_operand(vf[i][d]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) F32_STEP(o[d], a, pf, j);
+    }
+  }
+  if (!head_live) return;
+#pragma unroll
+  for (int d = 0; d < DT; ++d) {
+    *reinterpret_cast<float2*>(dst + 16 * d + 4 * g4) = make_float2(o[d][0], o[d][1]);
+    *reinterpret_cast<float2*>(dst + 16 * d + 4 * g4 + 2) = make_float2(o[d][2], o[d][3]);
+  }
+  if (g4 == 0) *reinterpret_cast<float2*>(dst + HD) = make_float2(m_b, l_b);
+}
+
 // A wave takes one block of 64 positions of a (token, kv head), with the query heads of the group (up to
 // 16) as the columns; K and V^T go from the pages straight into registers, all 64 KB asked for at
 // once, and (o_b, m_b, l_b) of every head are left in `partial` for the fold (work list and layout as in
-// attention_mfma.hip).  A wave a block of threads: an even spread of the loads over the CUs.  Bound by the wait
-// for the pages: 8 tokens of 16 heads over 2 at 777 positions 64 -> 19 us with the fold, at 2,048 144 -> 17.
-template <int HD>
-__global__ void __launch_bounds__(64, 1)
+// attention_mfma.hip).  BW waves a block of threads.  Bound by the wait for the pages: 8 tokens of 16 heads over
+// 2 at 777 positions 64 -> 19 us with the fold, at 2,048 144 -> 17.
+template <int HD, int BW>
+__global__ void __launch_bounds__(64 * BW, 1)
 attention_f32_decode_kernel(const float* __restrict__ q, int q_stride, const float* __restrict__ k_cache,
                             const float* __restrict__ v_cache, const int32_t* __restrict__ block_table, int table_stride,
                             const int32_t* __restrict__ positions, const int32_t* __restrict__ seq_rows,
                             const int32_t* __restrict__ token_index, int n_tokens, const int32_t* __restrict__ work,
                             float* __restrict__ partial, int max_chunks, int n_heads, int n_kv_heads, int page_size,
                             int window, float scale) {
-  constexpr int KG = HD / 16, DT = HD / 16;
-  const int sub = blockIdx.x & 3, unit = blockIdx.x >> 2, lane = threadIdx.x, r16 = lane & 15, g4 = lane >> 4;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r16 = lane & 15, g4 = lane >> 4;
+  const int sub = BW == 4 ? wave : blockIdx.x & 3, unit = BW == 4 ? blockIdx.x : blockIdx.x >> 2;
   const int item = work[unit / n_kv_heads];
   if (item < 0) return;
   const int slot = item / CMB_MAX_CHUNKS, chunk = item % CMB_MAX_CHUNKS;
@@ -269,76 +345,17 @@ attention_f32_decode_kernel(const float* __restrict__ q, int q_stride, const flo
   const float* k_head = k_cache + (size_t)kvh * HD * page_size;
   const float* v_head = v_cache + (size_t)kvh * HD * page_size;
 
-  f32x4 kf[4][KG], vf[4][DT], qf[KG];
-  int k_page[4], v_page[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    k_page[i] = table_row[page_index(min(p0 + 16 * i + r16, pos), page_size)];
-    v_page[i] = table_row[page_index(min(p0 + 16 * i + 4 * g4, pos), page_size)];
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float* kr = k_head + (size_t)k_page[i] * page_stride + (size_t)page_offset(min(p0 + 16 * i + r16, pos), page_size) * HD;
-#pragma unroll
-    for (int g = 0; g < KG; ++g) kf[i][g] = *reinterpret_cast<const f32x4*>(kr + 16 * g + 4 * g4);
-  }
-  const float* qrow = q + (size_t)t * q_stride + (size_t)(kvh * group + min(r16, group - 1)) * HD;
-#pragma unroll
-  for (int g = 0; g < KG; ++g) qf[g] = *reinterpret_cast<const f32x4*>(qrow + 16 * g + 4 * g4);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float* vr = v_head + (size_t)v_page[i] * page_stride + (page_offset(min(p0 + 16 * i + 4 * g4, pos), page_size) & ~3);
-#pragma unroll
-    for (int d = 0; d < DT; ++d) vf[i][d] = *reinterpret_cast<const f32x4*>(vr + (size_t)(16 * d + r16) * page_size);
-  }
-
-  f32x4 s[4] = {F32_ZERO, F32_ZERO, F32_ZERO, F32_ZERO};
-#pragma unroll
-  for (int g = 0; g < KG; ++g) {
-    const f32x4 qo = f32_operand(qf[g]);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const f32x4 a = f32_operand(kf[i][g]);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) F32_STEP(s[i], a, qo, j);
-    }
-  }
-  float m_b, l_b;
-  f32_weights(s, p0, lo, pos, scale, g4, m_b, l_b);
-  // the weight of a position outside the token's range is 0, and so must be what it is multiplied with
-  if (p0 < lo || p0 + ATT_BLOCK - 1 > pos) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int p = p0 + 16 * i + 4 * g4 + e;
-        const bool live = p >= lo && p <= pos;
-#pragma unroll
-        for (int d = 0; d < DT; ++d) vf[i][d][e] = live ? vf[i][d][e] : 0.0f;
-      }
-  }
-  f32x4 o[DT];
-#pragma unroll
-  for (int d = 0; d < DT; ++d) o[d] = F32_ZERO;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const f32x4 pf = f32_operand(s[i]);
-#pragma unroll
-    for (int d = 0; d < DT; ++d) {
-      const f32x4 a = f32_operand(vf[i][d]);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) F32_STEP(o[d], a, pf, j);
-    }
-  }
-  if (r16 >= group) return;
-  float* dst = partial + (((size_t)slot * n_heads + kvh * group + r16) * (max_chunks * (DC_CHUNK / ATT_BLOCK)) +
+  float* dst = partial + (((size_t)slot * n_heads + kvh * group + min(r16, group - 1)) * (max_chunks * (DC_CHUNK / ATT_BLOCK)) +
                           chunk * (DC_CHUNK / ATT_BLOCK) + sub) * (HD + 2);
-#pragma unroll
-  for (int d = 0; d < DT; ++d) {
-    *reinterpret_cast<float2*>(dst + 16 * d + 4 * g4) = make_float2(o[d][0], o[d][1]);
-    *reinterpret_cast<float2*>(dst + 16 * d + 4 * g4 + 2) = make_float2(o[d][2], o[d][3]);
-  }
-  if (g4 == 0) *reinterpret_cast<float2*>(dst + HD) = make_float2(m_b, l_b);
+  const float* qrow = q + (size_t)t * q_stride + (size_t)(kvh * group + min(r16, group - 1)) * HD;
+  // A context's last block often holds a few positions: 32 heads over 32, 200 tokens at 10 positions 103 us with all four
+  // tiles, 40 with one; 1 token of 16 heads over 2 14 / 9.
+  if (pos - p0 < 16)
+    f32_decode_block<HD, 1>(qrow, k_head, v_head, table_row, page_stride, page_size, p0, lo, pos, scale, r16, g4, r16 < group, dst);
+  else if (pos - p0 < 32)
+    f32_decode_block<HD, 2>(qrow, k_head, v_head, table_row, page_stride, page_size, p0, lo, pos, scale, r16, g4, r16 < group, dst);
+  else
+    f32_decode_block<HD, 4>(qrow, k_head, v_head, table_row, page_stride, page_size, p0, lo, pos, scale, r16, g4, r16 < group, dst);
 }
 
 // The fold of a token's blocks in ascending order, thread d dim d.  The factors depend on the maxima
@@ -432,15 +449,20 @@ int launch_attention_f32_decode(const float* q, int q_stride, const float* k_cac
                                 const int32_t* seq_rows, float* out, const int32_t* token_index, int n_tokens,
                                 const int32_t* work, int n_work, float* partial, int max_chunks, int n_heads,
                                 int n_kv_heads, int head_dim, int page_size, int window, float scale, hipStream_t stream) {
-#define LAUNCH(HD)                                                                                                   \
+  // A wave a block spreads the loads evenly; where contexts end within their first chunk most of its blocks have nothing to
+  // do, and four waves a block are launched faster: 16 heads over 2, 128 tokens at 40 positions 26 / 16 us, 28 over 4, 64 at
+  // 30 25 / 16, 64 at 100 26 / 19, 32 over 32, 400 at 100 597 / 475; 28 over 4, 64 at 1,000 62 / 64, 9 at 4,000 48 / 51, 1 at 500 15 / 19.
+  const bool single = n_work >= 2 * n_tokens || (long)n_work * n_kv_heads * 4 <= 256;
+#define LAUNCH(HD, BW)                                                                                               \
   {                                                                                                                  \
-    attention_f32_decode_kernel<HD><<<(unsigned)n_work * n_kv_heads * 4, 64, 0, stream>>>(                           \
+    attention_f32_decode_kernel<HD, BW><<<(unsigned)n_work * n_kv_heads * (4 / BW), 64 * BW, 0, stream>>>(           \
         q, q_stride, k_cache, v_cache, block_table, table_stride, positions, seq_rows, token_index, n_tokens, work,  \
         partial, max_chunks, n_heads, n_kv_heads, page_size, window, scale);                                         \
     attention_f32_combine_kernel<HD><<<dim3(n_tokens, n_heads), HD, 0, stream>>>(partial, positions, token_index, out, \
                                                                                  max_chunks, n_heads, window);       \
   }
-  if (head_dim == 64) LAUNCH(64) else LAUNCH(128)
+  if (head_dim == 64) { if (single) LAUNCH(64, 1) else LAUNCH(64, 4) }
+  else { if (single) LAUNCH(128, 1) else LAUNCH(128, 4) }
 #undef LAUNCH
   AXK_LAUNCH_CHECK("attention_decode");
   return 0;

@@ -496,7 +496,8 @@ class Kernels:
         return out
 
     def attention_fast_ok(self, head_dim: int, page_size: int, n_heads: int, n_kv_heads: int) -> bool:
-        """Whether the matrix-core attention kernels take these sizes (never in float32)."""
+        """Whether the bfloat16 build's attention kernels on the matrix cores take these sizes (never in float32,
+        whose own `attention_blocks_ok` answers for)."""
         return bool(self.lib.axk_attention_fast_ok(head_dim, page_size, n_heads, n_kv_heads))
 
     def attention_blocks_ok(self, head_dim: int, page_size: int, n_heads: int, n_kv_heads: int) -> bool:

@@ -24,12 +24,26 @@ from ..kernels import MODE_ADD_F32, MODE_STORE, PackedMatrix
 from .base import CacheBinding, CacheSpec, Mixer, PrecedingNorm, TensorDecl, build_part, register_mixer
 
 
+def float32_as_single_tokens(spans, window: int, n_heads: int, n_kv_heads: int):
+    """The first tokens of the portions whose tokens the float32 decoding kernel takes one by one.  A block of the prompt
+    kernel, one a head, takes 8 us for 64 positions of 128 dims whatever the number of its tokens and walks its positions in
+    a row; a wave of the other, one a key head, takes one token's, side by side.  So portions of no more tokens than a group
+    has heads go there (us, prompt / decoding kernel: 32 portions of 5 tokens, 28 heads over 4 31 / 14), and up to 64 tokens
+    that see 256 positions or more, while tokens x key heads are few (28 over 4, 9 tokens at 4,000 positions 498 / 49, 64
+    tokens at 600 86 / 49; 8 over 8, 40 at 4,000 276 / 138; 32 over 32, 16 at 600 79 / 86, 40 at 4,000 522 / 1,178)."""
+    sees = lambda s: s.start_pos + s.q_len if window == 0 else min(s.start_pos + s.q_len, window + s.q_len)
+    long_way = [s for s in spans if 1 < s.q_len <= 64 and sees(s) >= 256]
+    few = sum(s.q_len for s in long_way) * n_kv_heads <= 256
+    return {s.q_start for s in spans if 1 < s.q_len <= n_heads // n_kv_heads} | {s.q_start for s in long_way if few}
+
+
 class AttentionPlan:
     """How the matrix-core kernels split a step: prompt portions (2 tokens or more) go to the
-    prompt kernel in tiles of up to 128 tokens, single tokens to the decoding kernel.  Made
-    once per step and window, shared by all layers."""
+    prompt kernel in tiles of up to 128 tokens, single tokens to the decoding kernel, and the tokens
+    of the portions in `as_singles` (their first tokens) too.  Made once per step and window, shared
+    by all layers."""
 
-    def __init__(self, ctx, window: int, n_heads: int, head_dim: int):
+    def __init__(self, ctx, window: int, n_heads: int, head_dim: int, as_singles=frozenset()):
         dev = ctx.rt.device
         self.tiles = None
         self.partial = None
@@ -43,17 +57,17 @@ class AttentionPlan:
             self.decode_work = ctx.decode_inputs[("attention_work", window)]
             n_single = ctx.n_tokens
         else:
-            tiles, seen, singles, chunks = [], [], [], 1
+            tiles, seen, singles, at = [], [], [], []
             tile = ctx.rt.k.attention_prefill_tile          # tokens of one request a tile of the prompt kernel holds
             for s in ctx.spans:
-                if s.q_len == 1:
-                    singles.append(s.q_start)
-                    chunks = max(chunks, decode_chunks_of(s.start_pos, window, ctx.rt.k.attention_decode_chunk))
+                if s.q_len == 1 or s.q_start in as_singles:
+                    singles += range(s.q_start, s.q_start + s.q_len)
+                    at += range(s.start_pos, s.start_pos + s.q_len)
                 else:
-                    for at in range(0, s.q_len, tile):
-                        n = min(tile, s.q_len - at)
-                        tiles.append((s.q_start + at, n))
-                        last = s.start_pos + at + n                 # positions the tile's last token sees
+                    for first in range(0, s.q_len, tile):
+                        n = min(tile, s.q_len - first)
+                        tiles.append((s.q_start + first, n))
+                        last = s.start_pos + first + n              # positions the tile's last token sees
                         seen.append(min(last, window + n) if window > 0 else last)
             # the kernels trust these indices: check them here, on the host
             if (any(a < 0 or n < 1 or a + n > ctx.n_tokens for a, n in tiles)
@@ -61,11 +75,10 @@ class AttentionPlan:
                 raise ValueError("attention plan: a span lies outside the tokens of the step")
             self.tiles = torch.tensor(pair_tiles(tiles, seen), dtype=torch.int32).to(dev) if tiles else None
             self.decode_tokens = torch.tensor(singles, dtype=torch.int32).to(dev) if singles else None
-            self.max_chunks = chunks
+            self.max_chunks = max([1] + [decode_chunks_of(p, window, ctx.rt.k.attention_decode_chunk) for p in at])
             n_single = len(singles)
             if singles:
-                at = {s.q_start: s.start_pos for s in ctx.spans if s.q_len == 1}
-                work = ctx.rt.k.attention_decode_work([at[t] for t in singles], window)
+                work = ctx.rt.k.attention_decode_work(at, window)
                 self.decode_work = torch.tensor(work, dtype=torch.int32).to(dev)
         if n_single:
             n = ctx.rt.k.attention_decode_workspace(n_single, n_heads, head_dim, self.max_chunks)
@@ -101,12 +114,19 @@ def decode_chunks_of(pos: int, window: int, chunk: int) -> int:
     return (pos - lo // chunk * chunk) // chunk + 1
 
 
-def attention_plan(ctx, window: int, n_heads: int, head_dim: int) -> AttentionPlan:
-    key = ("attention_plan", window, n_heads, head_dim)
-    plan = ctx.shared.get(key)
-    if plan is None:
-        plan = ctx.shared[key] = AttentionPlan(ctx, window, n_heads, head_dim)
-    return plan
+def attention_plan(ctx, window: int, n_heads: int, n_kv_heads: int, head_dim: int, page_size: int) -> Optional[AttentionPlan]:
+    """The step's split, or None where the kernel for tokens of any kind takes them all."""
+    key = ("attention_plan", window, n_heads, n_kv_heads, head_dim, page_size)
+    if key not in ctx.shared:
+        k = ctx.rt.k
+        if k.attention_fast_ok(head_dim, page_size, n_heads, n_kv_heads):
+            ctx.shared[key] = AttentionPlan(ctx, window, n_heads, head_dim)
+        elif k.attention_blocks_ok(head_dim, page_size, n_heads, n_kv_heads):
+            split = frozenset() if ctx.decode_only else float32_as_single_tokens(ctx.spans, window, n_heads, n_kv_heads)
+            ctx.shared[key] = AttentionPlan(ctx, window, n_heads, head_dim, split)
+        else:
+            ctx.shared[key] = None
+    return ctx.shared[key]
 
 
 class GQAttention(Mixer):
@@ -248,8 +268,8 @@ class GQAttention(Mixer):
             k.gemm(h, w, qkv[:, :w.shape[0]], bias, MODE_STORE)
             k.rope_kv_write(qkv, table, ctx.positions, ctx.seq_rows, *cache, rotary, group.page_size, binding.writes)
         att = ctx.ws.take((T, self.q_dim), ctx.rt.dtype)
-        if k.attention_blocks_ok(self.hd, group.page_size, self.nh, self.nkv):
-            plan = attention_plan(ctx, self.window, self.nh, self.hd)
+        plan = attention_plan(ctx, self.window, self.nh, self.nkv, self.hd, group.page_size)
+        if plan is not None:
             common = (k_cache, v_cache, group.block_table, ctx.positions, ctx.seq_rows, att)
             sizes = (self.nh, self.nkv, self.hd, group.page_size, self.window, self.scale)
             if plan.tiles is not None:

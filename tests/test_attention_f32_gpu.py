@@ -52,6 +52,24 @@ def test_prompts_and_decoding_have_the_bits_of_the_rows_kernel(nh, nkv, hd, page
     assert _same(out2[T - 1], want[T - 1]) and _same(out2[0], want[0])
 
 
+def test_blocks_of_four_waves_have_the_bits_too():
+    """Many tokens whose contexts end within a chunk, and more blocks than the chip has places for."""
+    k, nh, nkv, hd, page, T = kernels("float32"), 4, 4, 64, 16, 70
+    for starts in ([3] * T, [300] * T + [40] * 200):
+        n = len(starts)
+        g = torch.Generator().manual_seed(n)
+        q, keys, vals = (torch.randn(max(starts) + 1 if i else n, h, hd, generator=g) for i, h in ((0, nh), (1, nkv), (2, nkv)))
+        kc, vc, table = paged_cache(keys, vals, page, "float32")
+        q, pos, rows = q.cuda().view(n, nh * hd), torch.tensor(starts, dtype=torch.int32).cuda(), torch.zeros(n, dtype=torch.int32).cuda()
+        sizes = (nh, nkv, hd, page, 0, hd ** -0.5)
+        want, out = torch.empty_like(q), torch.full_like(q, 5.0)
+        k.attention(q, nh * hd, kc, vc, table, pos, rows, want, *sizes)
+        chunks = max(starts) // k.attention_decode_chunk + 1
+        partial = torch.full((k.attention_decode_workspace(n, nh, hd, chunks),), float("nan"), device="cuda")
+        k.attention_decode(q, nh * hd, kc, vc, table, pos, rows, out, n, partial, chunks, *sizes)
+        assert _same(out, want)
+
+
 def test_what_it_takes():
     k = kernels("float32")
     assert not k.attention_blocks_ok(80, 16, 4, 2) and not k.attention_blocks_ok(128, 2, 4, 2)
