@@ -112,6 +112,14 @@ class Engine:
             limit = b.mixer.max_context()
             if limit is not None and self.max_seq_len > limit:
                 raise StepError(f"max_seq_len {self.max_seq_len}: a mixer of this model takes contexts of up to {limit}")
+        # workspaces mixers want in decoding steps (Mixer.decode_scratch): one per name, sized for the
+        # most requests and the longest context, allocated at the first decoding step (the pool leaves room for them)
+        self._scratch_sizes: Dict = {}
+        for b in model.blocks:
+            asked = b.mixer.decode_scratch(cfg.max_seqs, self.max_seq_len)
+            if asked is not None:
+                self._scratch_sizes[asked[0]] = max(self._scratch_sizes.get(asked[0], 0), int(asked[1]))
+        self._scratch: Optional[Dict] = None
         self.ws = Workspace(rt.device)
         plans = model.group_plans(cfg.page_size, self._pool_size)
         self.cache = CacheManager(plans, model.cache_plan.state_elems, cfg.max_seqs, self.max_seq_len, rt.device,
@@ -155,14 +163,6 @@ class Engine:
                 self._input_mixers.append(b.mixer)
                 self._inputs[asked[0]] = torch.full((cap,), -1, dtype=torch.int32, device=rt.device)
                 self._input_hosts[asked[0]] = [torch.full((cap,), -1, dtype=torch.int32).pin_memory() for _ in range(4)]
-        # workspaces mixers want in decoding steps (Mixer.decode_scratch): one per name, sized for the
-        # most requests and the longest context, allocated at the first decoding step
-        self._scratch_sizes: Dict = {}
-        for b in model.blocks:
-            asked = b.mixer.decode_scratch(cfg.max_seqs, self.max_seq_len)
-            if asked is not None:
-                self._scratch_sizes[asked[0]] = max(self._scratch_sizes.get(asked[0], 0), int(asked[1]))
-        self._scratch: Optional[Dict] = None
         self._meta = torch.zeros((3, cfg.max_seqs), dtype=torch.int32, device=rt.device)
         # staging in pinned memory, a ring: a step's inputs and picks travel while the host
         # prepares the next step
@@ -185,8 +185,10 @@ class Engine:
             return cfg.num_pages
         if cfg.max_cache_tokens > 0:
             return max(1, -(-cfg.max_cache_tokens // page_size))
-        # from the memory that is free now: every group gets an equal share of the fraction
+        # from the memory that is free now and that no workspace of the decoding steps will take: every group gets an
+        # equal share of the fraction
         free, _ = torch.cuda.mem_get_info(self.rt.device)
+        free = max(0, free - 4 * sum(self._scratch_sizes.values()))
         n_groups = max(1, len(self.model.cache_plan.group_specs))
         elem = self.rt.elem_size if spec.dtype is None else torch.empty((), dtype=getattr(torch, spec.dtype)).element_size()
         per_page = n_layers * spec.entries * spec.heads * page_size * spec.head_dim * elem

@@ -24,6 +24,11 @@ from ..kernels import MODE_ADD_F32, MODE_STORE, PackedMatrix
 from .base import CacheBinding, CacheSpec, Mixer, PrecedingNorm, TensorDecl, build_part, register_mixer
 
 
+# The float32 build has a kernel for tokens of any kind that needs no workspace (`attention`), with the bits of its
+# prompt and decoding kernels; where the decoding kernel would want more memory than this, it is taken instead.
+FLOAT32_PARTIAL = 1 << 27         # floats of the decoding kernel's partial results (512 MiB)
+
+
 def float32_as_single_tokens(spans, window: int, n_heads: int, n_kv_heads: int):
     """The first tokens of the portions whose tokens the float32 decoding kernel takes one by one.  A block of the prompt
     kernel, one a head, takes 8 us for 64 positions of 128 dims whatever the number of its tokens and walks its positions in
@@ -122,11 +127,35 @@ def attention_plan(ctx, window: int, n_heads: int, n_kv_heads: int, head_dim: in
         if k.attention_fast_ok(head_dim, page_size, n_heads, n_kv_heads):
             ctx.shared[key] = AttentionPlan(ctx, window, n_heads, head_dim)
         elif k.attention_blocks_ok(head_dim, page_size, n_heads, n_kv_heads):
-            split = frozenset() if ctx.decode_only else float32_as_single_tokens(ctx.spans, window, n_heads, n_kv_heads)
-            ctx.shared[key] = AttentionPlan(ctx, window, n_heads, head_dim, split)
+            ctx.shared[key] = _float32_plan(ctx, window, n_heads, n_kv_heads, head_dim)
         else:
             ctx.shared[key] = None
     return ctx.shared[key]
+
+
+def _float32_plan(ctx, window: int, n_heads: int, n_kv_heads: int, head_dim: int) -> Optional[AttentionPlan]:
+    k = ctx.rt.k
+
+    def floats(n_tokens: int, longest: int) -> int:
+        chunks = decode_chunks_of(longest, window, k.attention_decode_chunk)
+        return k.attention_decode_workspace(n_tokens, n_heads, head_dim, chunks)
+    if ctx.decode_only:
+        # a captured step is replayed at any context: what the engine's largest would want decides (see `decode_scratch`)
+        most = decode_scratch_floats(k, window, n_heads, head_dim, ctx.cache.max_seqs, ctx.cache.max_seq_len)
+        return AttentionPlan(ctx, window, n_heads, head_dim) if most <= FLOAT32_PARTIAL and ctx.n_tokens <= 65535 else None
+    split = float32_as_single_tokens(ctx.spans, window, n_heads, n_kv_heads)
+    for as_singles in (split, frozenset()):
+        singles = [s for s in ctx.spans if s.q_len == 1 or s.q_start in as_singles]
+        n = sum(s.q_len for s in singles)
+        if n == 0 or n <= 65535 and floats(n, max(s.start_pos + s.q_len - 1 for s in singles)) <= FLOAT32_PARTIAL:
+            return AttentionPlan(ctx, window, n_heads, head_dim, as_singles)
+    return None
+
+
+def decode_scratch_floats(k, window: int, n_heads: int, head_dim: int, max_seqs: int, max_seq_len: int) -> int:
+    """The decoding kernel's partial results, laid out by the longest context in chunks rounded up to a power of two."""
+    most = decode_chunks_of(max(0, max_seq_len - 1), window, k.attention_decode_chunk)
+    return k.attention_decode_workspace(max_seqs, n_heads, head_dim, 1 << (most - 1).bit_length())
 
 
 class GQAttention(Mixer):
@@ -153,7 +182,7 @@ class GQAttention(Mixer):
         self.n = {k: base + names.get(k, k + "_proj") for k in ("q", "k", "v", "o")}
         self.w_qkv = self.b_qkv = self.w_o = self.b_o = None
         self._max_context = None
-        self._workspace = None
+        self._kernels = None                 # those that want a workspace in decoding steps
         self.decode_chunk = 1 << 30          # until `load` has asked the kernels: one chunk
         self._work_list = lambda positions, window: list(range(len(positions)))
 
@@ -196,20 +225,20 @@ class GQAttention(Mixer):
         return round_up_by_eighths(max_seqs * decode_chunks_of(max(0, max_seq_len - 1), 0, self.decode_chunk))
 
     def decode_scratch(self, max_seqs: int, max_seq_len: int):
-        """The blocks' partial results of the decoding kernel, laid out by the longest context in
-        chunks rounded up to a power of two (see `decode_shape`)."""
-        if self._workspace is None:              # no kernel of this build and these sizes wants one
+        """The blocks' partial results of the decoding kernel (see `decode_shape`)."""
+        if self._kernels is None:                # no kernel of this build and these sizes wants one
             return None
-        most = decode_chunks_of(max(0, max_seq_len - 1), self.window, self.decode_chunk)
-        chunks = 1 << (most - 1).bit_length()
-        return ("attention_partial", self.window, self.nh, self.hd), self._workspace(max_seqs, self.nh, self.hd, chunks)
+        floats = decode_scratch_floats(self._kernels, self.window, self.nh, self.hd, max_seqs, max_seq_len)
+        if floats > FLOAT32_PARTIAL and not self._kernels.attention_fast_ok(self.hd, 64, self.nh, self.nkv):
+            return None
+        return ("attention_partial", self.window, self.nh, self.hd), floats
 
     def load(self, store, rt) -> None:
         self.decode_chunk = rt.k.attention_decode_chunk
         self._work_list = rt.k.attention_decode_work
         self._max_context = rt.k.attention_decode_max_context
         if rt.k.attention_blocks_ok(self.hd, 64, self.nh, self.nkv):
-            self._workspace = rt.k.attention_decode_workspace
+            self._kernels = rt.k
         self.w_qkv = rt.k.prepare_weight(store.fused_matrix([self.n[k] + ".weight" for k in ("q", "k", "v")]))
         biases = [store.vector(self.n[k] + ".bias", optional=True) for k in ("q", "k", "v")] if self.qkv_bias else []
         present = [b is not None for b in biases]

@@ -70,6 +70,31 @@ def test_blocks_of_four_waves_have_the_bits_too():
         assert _same(out, want)
 
 
+def test_an_engine_of_any_capacity_decodes(tmp_path):
+    """So many and so long requests that the decoding kernel's partial results would take 17 GB: the engine runs without."""
+    import axon_amd
+    from axon_amd.config import config_from_dict
+    from axon_amd.engine import StepEntry
+    from axon_amd.weights import write_random_model
+    cfg = dict(architectures=["Qwen2ForCausalLM"], num_hidden_layers=2, hidden_size=256, intermediate_size=128, num_attention_heads=4,
+               num_key_value_heads=2, vocab_size=64, max_position_embeddings=131072, rope_theta=10000.0, rms_norm_eps=1e-6,
+               tie_word_embeddings=False)
+    write_random_model(config_from_dict(cfg), str(tmp_path), seed=1, std=0.3, storage="float32")
+    got = []
+    for max_seqs in (4, 8192):
+        llm = axon_amd.load(str(tmp_path), dtype="float32", max_seqs=max_seqs, num_pages=300, page_size=64)
+        torch.cuda.synchronize()
+        before = torch.cuda.memory_reserved()
+        llm.engine.step([StepEntry(id=0, tokens=list(range(40)) * 8, want=[319])])
+        rows = [llm.engine.step([StepEntry(id=0, tokens=[7 + i], want=[0])]).clone() for i in range(3)]
+        rows.append(llm.engine.step([StepEntry(id=0, tokens=[1, 2, 3], want=[0, 1, 2]), StepEntry(id=1, tokens=[5] * 9, want=[8])]).clone())
+        got.append(rows)
+        assert torch.cuda.memory_reserved() - before < 1 << 30
+        del llm
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+
+
 def test_what_it_takes():
     k = kernels("float32")
     assert not k.attention_blocks_ok(80, 16, 4, 2) and not k.attention_blocks_ok(128, 2, 4, 2)

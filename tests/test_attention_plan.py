@@ -1,10 +1,11 @@
 """How a step's tokens are split between the attention kernels, without a device: the float32 build's choice between its
-prompt and decoding kernels, which give the same bits, by what each is fast at."""
+prompt, decoding and any-token kernels, which give the same bits, by what each is fast at and how much memory it wants."""
 from types import SimpleNamespace
 
 import pytest
+import torch
 
-from axon_amd.engine.step import Span
+from axon_amd.engine.step import Engine, Span
 from axon_amd.kernels.lib import Kernels
 from axon_amd.parts import attention as A
 
@@ -72,3 +73,33 @@ def test_short_portions_go_token_by_token(spans, heads, singles):
 def test_a_window_bounds_what_a_portion_sees():
     assert _tokens(A.attention_plan(_ctx([(9, 4000)]), 100, 28, 4, 128, 64))[1] == []
     assert _tokens(A.attention_plan(_ctx([(9, 4000)]), 600, 28, 4, 128, 64))[1] == list(range(9))
+
+
+def test_float32_holds_no_workspace_beyond_its_limit():
+    """A float32 engine for so many and so long requests that the decoding kernel's partial results would take gigabytes
+    runs with the kernel that needs none, as it did before there was a decoding kernel."""
+    mixer = A.GQAttention(dict(hidden_size=64, num_heads=28, num_kv_heads=4, head_dim=128))
+    for float32 in (True, False):
+        mixer._kernels = _Kernels(float32=float32)
+        small, large = mixer.decode_scratch(64, 8192), mixer.decode_scratch(512, 131072)
+        assert small == (("attention_partial", 0, 28, 128), 64 * 28 * 32 * 4 * 130)
+        assert (large is None) == float32
+    assert A.attention_plan(_ctx([(1, 70)] * 3, decode_only=True, max_seqs=64), 0, 28, 4, 128, 64) is not None
+    assert A.attention_plan(_ctx([(1, 70)] * 3, decode_only=True, max_seqs=512, max_seq_len=131072), 0, 28, 4, 128, 64) is None
+    assert A.attention_plan(_ctx([(1, 70)] * 3, float32=False, decode_only=True, max_seqs=2, max_seq_len=4096), 0, 28, 4, 128, 64) is not None
+    # a step that feeds portions too: by what the step itself wants; portions go back to tiles before anything else
+    plan = A.attention_plan(_ctx([(7, 60000)] * 40 + [(1, 9)]), 0, 28, 4, 128, 64)
+    assert _tokens(plan)[1] == [280]
+    assert A.attention_plan(_ctx([(1, 60000)] * 60 + [(300, 0)]), 0, 28, 4, 128, 64) is None
+
+
+def test_the_cache_pool_leaves_room_for_the_decoding_steps_workspaces(monkeypatch):
+    monkeypatch.setattr(torch.cuda, "mem_get_info", lambda device=None: (1 << 30, 1 << 34))
+    spec = SimpleNamespace(dtype=None, entries=2, heads=4, head_dim=64)
+    cfg = SimpleNamespace(num_pages=0, max_cache_tokens=0, memory_fraction=1.0, max_seqs=1 << 20)
+    engine = SimpleNamespace(cfg=cfg, rt=SimpleNamespace(device=None, elem_size=4), max_seq_len=1 << 20,
+                             model=SimpleNamespace(cache_plan=SimpleNamespace(group_specs=[spec])), _scratch_sizes={})
+    page = 3 * 2 * 4 * 16 * 64 * 4
+    assert Engine._pool_size(engine, spec, 3, 16) == (1 << 30) // page
+    engine._scratch_sizes = {"a": 1 << 26, "b": 1 << 25}
+    assert Engine._pool_size(engine, spec, 3, 16) == ((1 << 30) - (3 << 27)) // page
