@@ -15,7 +15,8 @@ namespace {
 
 const char* const KIND_NAMES[INST_KINDS] = {"gemm_fma", "gemm_tile", "gemm_stream", "gemm_normed", "gemm_rows",
                                             "gemm_split_reduce", "attention_rows", "attention_prefill",
-                                            "attention_decode", "rmsnorm", "grouped_gemm", "causal_conv"};
+                                            "attention_decode", "rmsnorm", "grouped_gemm", "causal_conv",
+                                            "latent_prompt", "latent_tokens"};
 
 struct Registry {
   std::mutex lock;

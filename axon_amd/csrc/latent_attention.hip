@@ -12,6 +12,7 @@
 
 #include "api.h"
 #include "common.h"
+#include "instances.h"
 
 namespace {
 
@@ -177,10 +178,39 @@ __device__ inline la_bf16x8 la_frag(uint4 v) { return __builtin_bit_cast(la_bf16
 // latent dims at most; QC: chunks of 32 key dims at most.  Pages hold a multiple of 64 positions.
 #define LAM_WAVES 2
 #define LAP_TOKENS 8                                  // tokens a block of the kernel for steps of many tokens
-__device__ __forceinline__ bool latent_one_request(const int32_t* __restrict__ seq_rows, int first, int last) {
-  bool same = true;
-  for (int u = first + 1; u <= last; ++u) same = same && seq_rows[u] == seq_rows[first];
-  return same;
+// What the kernel for steps of many tokens walks of the tokens first .. last of a tile: up to two runs of neighbours of one
+// request, [from0, end0) and [from1, end1).  All of them where the tile holds no more than two requests; else those of
+// portions of two tokens or more (decoding rows beside them are left out), unless there are three of these.
+struct LatentRuns {
+  int from0, end0, from1, end1;
+  __device__ __forceinline__ bool hold(int t) const { return (t >= from0 && t < end0) || (t >= from1 && t < end1); }
+};
+__device__ __forceinline__ LatentRuns latent_runs(const int32_t* __restrict__ seq_rows, int n_tokens, int first, int last) {
+  const int n = last + 1 - first, whole = (1 << n) - 1;
+  int slot[LAP_TOKENS + 2];                             // of the tile's tokens and their neighbours, all asked for at once
+#pragma unroll
+  for (int i = 0; i < LAP_TOKENS + 2; ++i) slot[i] = seq_rows[min(max(first + i - 1, 0), n_tokens - 1)];
+  int same = 0;                                         // bit i: token i is of the request of the one before
+#pragma unroll
+  for (int i = 0; i <= LAP_TOKENS; ++i)
+    same |= (slot[i] == slot[i + 1] && first + i > 0 && first + i < n_tokens ? 1 : 0) << i;
+  const int starts = (~same | 1) & whole, portions = starts & (same | same >> 1);
+  auto behind = [&](int i) {                            // where the run that starts at i ends
+    const int later = starts & ~((2 << i) - 1);
+    return later ? __builtin_ctz(later) : n;
+  };
+  int a, b;                                             // the runs' first tokens (n: none)
+  if (__builtin_popcount(starts) <= 2) {
+    a = 0;
+    b = behind(0);
+  } else if (__builtin_popcount(portions) <= 2) {
+    const int second = portions & (portions - 1);
+    a = portions ? __builtin_ctz(portions) : n;
+    b = second ? __builtin_ctz(second) : n;
+  } else {
+    a = b = n;
+  }
+  return LatentRuns{first + a, first + (a < n ? behind(a) : n), first + b, first + (b < n ? behind(b) : n)};
 }
 
 template <int RT, int QC, bool SINK>
@@ -204,7 +234,7 @@ latent_attention_mfma_kernel(const float* __restrict__ q_full, const bf16_t* __r
   const int t = active ? (int)(item / groups) : 0, hg = active ? (int)(item % groups) : 0;
   if (mixed_only && active) {                         // beside the kernel for steps of many tokens: what it leaves
     const int t_first = t / LAP_TOKENS * LAP_TOKENS;
-    active = !latent_one_request(seq_rows, t_first, min(t_first + LAP_TOKENS, n_tokens) - 1);
+    active = !latent_runs(seq_rows, n_tokens, t_first, min(t_first + LAP_TOKENS, n_tokens) - 1).hold(t);
   }
   const int width = rank + rot, qc = width / 32, rt = rank / 16;
   const int j = lane & 15, g = lane >> 4;
@@ -359,10 +389,13 @@ __device__ __forceinline__ void la_for(F&& body) {
 // summed, its C^T rows [rank][64] while the scores are worked out.  16-byte slots of a staged row are permuted by
 // slot ^ (row / 2 % 8), so that the sixteen rows of a read fall into different banks.  Each wave keeps its own
 // mask, running pair and accumulators and runs the chain of products of the kernels above: the same bits (sums
-// whose maximum stays are not multiplied by 1).  Tiles with tokens of several requests are left to a launch of
-// the kernel above (`mixed_only`).  Bound by the way out of LDS: a wave reads the block's 136 KB for 2,176 cycles of products.
-// 16 heads, latents of 512 and 64 rotated dims, 2,048 tokens over a window of 1,024: 638 -> 129 us (four tokens a
-// block, stages through registers, queries read from LDS beside the keys).
+// whose maximum stays are not multiplied by 1).  A tile that lies across two requests walks the blocks of one and then
+// of the other; what `latent_runs` leaves out is left to a launch of the kernel above (`mixed_only`).  Bound by the way out of LDS: a wave reads the block's 136 KB for 2,176 cycles of products.
+// 16 heads, latents of 512 and 64 rotated dims, 2,048 tokens over a window of 1,024: 638 -> 123 us (four tokens a
+// block, stages through registers, queries read from LDS beside the keys); three requests of 701, 523 and 301 tokens
+// 232 -> 82, with the tiles across two of them left to the launch behind 260; two portions of 301 tokens at 6,000
+// positions 2,280 -> 839.  The launch behind comes after this one, not beside it: 64 decoding rows at 1,000 positions and a
+// prompt of 512 tokens 400 -> 335, but with latents of 64 dims 87 -> 92.
 template <int RT, int QC, bool EXACT, bool SINK>
 __global__ void __launch_bounds__(LAP_TOKENS * 64, 2)
 latent_attention_prompt_kernel(const float* __restrict__ q_full, const bf16_t* __restrict__ cache,
@@ -379,17 +412,11 @@ latent_attention_prompt_kernel(const float* __restrict__ q_full, const bf16_t* _
   const int width = rank + rot, qc = width / 32, rt = rank / 16;
   const long page_elems = (long)page_size * (width + rank);
   const int t_first = tile * LAP_TOKENS, t_last = min(t_first + LAP_TOKENS, n_tokens) - 1;
-  if (!latent_one_request(seq_rows, t_first, t_last)) return;       // (the same for the whole block)
-  int b_from = 1 << 30, b_to = -1;
-  for (int u = t_first; u <= t_last; ++u) {
-    const int p = positions[u];
-    b_from = min(b_from, (window > 0 ? max(0, p + 1 - window) : 0) / 64);
-    b_to = max(b_to, p / 64);
-  }
-  const bool active = t_first + wave <= t_last;
+  const LatentRuns runs = latent_runs(seq_rows, n_tokens, t_first, t_last);       // (the same for the whole block)
+  const bool active = runs.hold(t_first + wave);
   const int t = min(t_first + wave, t_last), j = lane & 15, g = lane >> 4;
   const int pos = positions[t], lo = window > 0 ? max(0, pos + 1 - window) : 0;
-  const int32_t* pages = block_table + (long)seq_rows[t] * table_stride;
+  const int32_t* pages = nullptr;                                  // of the request whose blocks are walked
   // Q^T: a lane's head j, 8 consecutive dims from 32 kc + 8 g, rounded
   u32x4 qf[QC];
   const float* qsrc = q_full + ((long)t * heads + hg * 16 + j) * width + 8 * g;
@@ -474,93 +501,105 @@ latent_attention_prompt_kernel(const float* __restrict__ q_full, const bf16_t* _
   // of 64 bytes and of 128, so the second address differs from the first by a bit of it.
   const unsigned k_first = k_row + ((k_mask == 7 ? g ^ f : g ^ (f & 3)) << 4);
   const unsigned v_first = base + 128 * width + j * 128 + 8 * (g & 1) + (((g >> 1) ^ f) << 4);
-  ask_k(b_from);
-  for (int b = b_from; b <= b_to; ++b) {
-    wait_vmcnt<0>();
-    __syncthreads();                                // K of this block is there, C^T of the block before is read
-    ask_v(b);
-    const bool mine = active && b >= lo / 64 && b <= pos / 64;
-    if (mine) {
-#pragma unroll
-      for (int pt = 0; pt < 4; ++pt) s[pt] = la_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-      unsigned k_base = k_first;
-      asm volatile("" : "+v"(k_base));              // (the others are worked out here: no registers of theirs across the loop)
-      const unsigned k_at[2] = {k_base, k_mask == 7 ? k_base ^ 64 : k_base + 64};
-      if constexpr (EXACT) {
-        u32x4 kf[2][2];                             // two of the four tiles of 16 positions, read one pair ahead
-        auto read_k = [&](auto u) {
-          constexpr int U = decltype(u)::value, KC = U / 2;
-          lds_read16<128 * (KC / 2) + 2 * (U & 1) * 1024 * QC>(kf[U & 1][0], k_at[KC & 1]);
-          lds_read16<128 * (KC / 2) + (2 * (U & 1) + 1) * 1024 * QC>(kf[U & 1][1], k_at[KC & 1]);
-        };
-        read_k(std::integral_constant<int, 0>());
-        la_for<2 * QC>([&](auto u) {
-          constexpr int U = decltype(u)::value;
-          if constexpr (U + 1 < 2 * QC) {
-            read_k(std::integral_constant<int, U + 1>());
-            wait_lgkmcnt<2>();
-          } else {
-            wait_lgkmcnt<0>();
-          }
-          use_frags<2>(kf[U & 1]);
-#pragma unroll
-          for (int e = 0; e < 2; ++e)
-            s[2 * (U & 1) + e] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(la_bf16x8, kf[U & 1][e]), __builtin_bit_cast(la_bf16x8, qf[U / 2]),
-                                                                         s[2 * (U & 1) + e], 0, 0, 0);
-        });
-      } else {
-#pragma unroll
-        for (int kc = 0; kc < QC; ++kc)
-          if (kc < qc)
-#pragma unroll
-            for (int pt = 0; pt < 4; ++pt) {
-              const uint4 kf = *reinterpret_cast<const uint4*>(lap_lds + k_at[kc & 1] + 128 * (kc / 2) + pt * 32 * width);
-              s[pt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(la_frag(kf), __builtin_bit_cast(la_bf16x8, qf[kc]), s[pt], 0, 0, 0);
-            }
-      }
-      weigh(b * 64);
+  for (int run = 0; run < 2; ++run) {
+    const int u0 = run ? runs.from1 : runs.from0, u1 = (run ? runs.end1 : runs.end0) - 1;
+    if (u0 > u1) continue;
+    int b_from = 1 << 30, b_to = -1;
+    for (int u = u0; u <= u1; ++u) {
+      const int p = positions[u];
+      b_from = min(b_from, (window > 0 ? max(0, p + 1 - window) : 0) / 64);
+      b_to = max(b_to, p / 64);
     }
-    wait_vmcnt<0>();
-    __syncthreads();                                // C^T of this block is there, its K is read
-    if (b < b_to) ask_k(b + 1);
-    if (mine) {
-      unsigned v_base = v_first;
-      asm volatile("" : "+v"(v_base));
-      const unsigned v_at[4] = {v_base, v_base ^ 32, v_base ^ 64, v_base ^ 96};
-      if constexpr (EXACT) {
-        la_u32x2 vf[2][4];                          // a tile of 16 dims, read one ahead
-        auto read_v = [&](auto d) {
-          constexpr int D = decltype(d)::value;
+    pages = block_table + (long)seq_rows[u0] * table_stride;
+    const bool walks = t_first + wave >= u0 && t_first + wave <= u1;
+    ask_k(b_from);
+    for (int b = b_from; b <= b_to; ++b) {
+      wait_vmcnt<0>();
+      __syncthreads();                                // K of this block is there, C^T of the block before is read
+      ask_v(b);
+      const bool mine = walks && b >= lo / 64 && b <= pos / 64;
+      if (mine) {
 #pragma unroll
-          for (int x = 0; x < 4; ++x) la_read8<2048 * D>(vf[D & 1][x], v_at[x]);
-        };
-        read_v(std::integral_constant<int, 0>());
-        la_for<RT>([&](auto d) {
-          constexpr int D = decltype(d)::value;
-          if constexpr (D + 1 < RT) {
-            read_v(std::integral_constant<int, D + 1>());
-            wait_lgkmcnt<4>();
-          } else {
-            wait_lgkmcnt<0>();
-          }
-#pragma unroll
-          for (int x = 0; x < 4; ++x) asm volatile("" : "+v"(vf[D & 1][x]));
-#pragma unroll
-          for (int c = 0; c < 2; ++c)
-            acc[D] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                la_frag(make_uint4(vf[D & 1][2 * c][0], vf[D & 1][2 * c][1], vf[D & 1][2 * c + 1][0], vf[D & 1][2 * c + 1][1])),
-                la_frag(pf[c]), acc[D], 0, 0, 0);
-        });
-      } else {
-#pragma unroll
-        for (int d = 0; d < RT; ++d)
-          if (d < rt)
-#pragma unroll
-            for (int c = 0; c < 2; ++c) {
-              const uint2 a = *reinterpret_cast<const uint2*>(lap_lds + v_at[2 * c] + 2048 * d);
-              const uint2 e = *reinterpret_cast<const uint2*>(lap_lds + v_at[2 * c + 1] + 2048 * d);
-              acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(la_frag(make_uint4(a.x, a.y, e.x, e.y)), la_frag(pf[c]), acc[d], 0, 0, 0);
+        for (int pt = 0; pt < 4; ++pt) s[pt] = la_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        unsigned k_base = k_first;
+        asm volatile("" : "+v"(k_base));              // (the others are worked out here: no registers of theirs across the loop)
+        const unsigned k_at[2] = {k_base, k_mask == 7 ? k_base ^ 64 : k_base + 64};
+        if constexpr (EXACT) {
+          u32x4 kf[2][2];                             // two of the four tiles of 16 positions, read one pair ahead
+          auto read_k = [&](auto u) {
+            constexpr int U = decltype(u)::value, KC = U / 2;
+            lds_read16<128 * (KC / 2) + 2 * (U & 1) * 1024 * QC>(kf[U & 1][0], k_at[KC & 1]);
+            lds_read16<128 * (KC / 2) + (2 * (U & 1) + 1) * 1024 * QC>(kf[U & 1][1], k_at[KC & 1]);
+          };
+          read_k(std::integral_constant<int, 0>());
+          la_for<2 * QC>([&](auto u) {
+            constexpr int U = decltype(u)::value;
+            if constexpr (U + 1 < 2 * QC) {
+              read_k(std::integral_constant<int, U + 1>());
+              wait_lgkmcnt<2>();
+            } else {
+              wait_lgkmcnt<0>();
             }
+            use_frags<2>(kf[U & 1]);
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+              s[2 * (U & 1) + e] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(la_bf16x8, kf[U & 1][e]), __builtin_bit_cast(la_bf16x8, qf[U / 2]),
+                                                                           s[2 * (U & 1) + e], 0, 0, 0);
+          });
+        } else {
+#pragma unroll
+          for (int kc = 0; kc < QC; ++kc)
+            if (kc < qc)
+#pragma unroll
+              for (int pt = 0; pt < 4; ++pt) {
+                const uint4 kf = *reinterpret_cast<const uint4*>(lap_lds + k_at[kc & 1] + 128 * (kc / 2) + pt * 32 * width);
+                s[pt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(la_frag(kf), __builtin_bit_cast(la_bf16x8, qf[kc]), s[pt], 0, 0, 0);
+              }
+        }
+        weigh(b * 64);
+      }
+      wait_vmcnt<0>();
+      __syncthreads();                                // C^T of this block is there, its K is read
+      if (b < b_to) ask_k(b + 1);
+      if (mine) {
+        unsigned v_base = v_first;
+        asm volatile("" : "+v"(v_base));
+        const unsigned v_at[4] = {v_base, v_base ^ 32, v_base ^ 64, v_base ^ 96};
+        if constexpr (EXACT) {
+          la_u32x2 vf[2][4];                          // a tile of 16 dims, read one ahead
+          auto read_v = [&](auto d) {
+            constexpr int D = decltype(d)::value;
+#pragma unroll
+            for (int x = 0; x < 4; ++x) la_read8<2048 * D>(vf[D & 1][x], v_at[x]);
+          };
+          read_v(std::integral_constant<int, 0>());
+          la_for<RT>([&](auto d) {
+            constexpr int D = decltype(d)::value;
+            if constexpr (D + 1 < RT) {
+              read_v(std::integral_constant<int, D + 1>());
+              wait_lgkmcnt<4>();
+            } else {
+              wait_lgkmcnt<0>();
+            }
+#pragma unroll
+            for (int x = 0; x < 4; ++x) asm volatile("" : "+v"(vf[D & 1][x]));
+#pragma unroll
+            for (int c = 0; c < 2; ++c)
+              acc[D] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                  la_frag(make_uint4(vf[D & 1][2 * c][0], vf[D & 1][2 * c][1], vf[D & 1][2 * c + 1][0], vf[D & 1][2 * c + 1][1])),
+                  la_frag(pf[c]), acc[D], 0, 0, 0);
+          });
+        } else {
+#pragma unroll
+          for (int d = 0; d < RT; ++d)
+            if (d < rt)
+#pragma unroll
+              for (int c = 0; c < 2; ++c) {
+                const uint2 a = *reinterpret_cast<const uint2*>(lap_lds + v_at[2 * c] + 2048 * d);
+                const uint2 e = *reinterpret_cast<const uint2*>(lap_lds + v_at[2 * c + 1] + 2048 * d);
+                acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(la_frag(make_uint4(a.x, a.y, e.x, e.y)), la_frag(pf[c]), acc[d], 0, 0, 0);
+              }
+        }
       }
     }
   }
@@ -628,6 +667,7 @@ static int launch_latent_prompt(const float* q_full, const void* cache, const in
     configured = true;
   }
   const unsigned grid = (unsigned)(((n_tokens + LAP_TOKENS - 1) / LAP_TOKENS) * (heads / 16));
+  if (sink) { AXK_INSTANCE(INST_LATENT_PROMPT, RT, QC, EXACT, 1); } else { AXK_INSTANCE(INST_LATENT_PROMPT, RT, QC, EXACT, 0); }
   if (sink)
     latent_attention_prompt_kernel<RT, QC, EXACT, true><<<grid, LAP_TOKENS * 64, lds, stream>>>(
         q_full, (const bf16_t*)cache, block_table, table_stride, positions, seq_rows, o_lat, n_tokens, heads, rank, rot, page_size, window,
@@ -646,6 +686,7 @@ static void launch_latent_mfma(const float* q_full, const void* cache, const int
                                bool mixed_only, hipStream_t stream) {
   const long items = (long)n_tokens * (heads / 16);
   dim3 grid((unsigned)((items + LAM_WAVES - 1) / LAM_WAVES), partial ? n_chunks : 1);
+  if (sink) { AXK_INSTANCE(INST_LATENT_TOKENS, RT, QC, 1); } else { AXK_INSTANCE(INST_LATENT_TOKENS, RT, QC, 0); }
   if (sink)
     latent_attention_mfma_kernel<RT, QC, true><<<grid, LAM_WAVES * 64, 0, stream>>>(
         q_full, (const bf16_t*)cache, block_table, table_stride, positions, seq_rows, o_lat, n_tokens, heads, rank, rot, page_size,

@@ -246,6 +246,38 @@ def check_grouped(dtype, M, G, N, K, glu):
     return hit
 
 
+def check_latent(rank, rot, sink):
+    """Latent attention of a portion of many tokens against the plain formula (weights and queries rounded as the kernel
+    does), and bit for bit as each token alone, a wave a token, gives it."""
+    k, T, heads, page = kernels("bfloat16"), 261, 16, 64
+    pages = -(-T // page)
+    cache = rnd(pages, 1, page, 2 * rank + rot, seed=80, device="cuda").bfloat16()
+    table = torch.arange(pages, device="cuda").flip(0).int().view(1, pages)
+    q = rnd(T, heads * (rank + rot), seed=81, scale=0.3, device="cuda")
+    pos = torch.arange(T, dtype=torch.int32, device="cuda")
+    sinks = rnd(heads, seed=82, device="cuda") if sink else None
+    scale = (rank + rot) ** -0.5
+
+    def attend(rows, tab):
+        out = torch.full((T, heads * rank), float("nan"), device="cuda")
+        k.latent_attention(q, cache, tab, pos, rows, out, heads, rank, rot, page, 0, scale, sink=sinks)
+        return out
+    got = {}
+    hit = launched(k, "bfloat16", lambda: got.setdefault("out", attend(torch.zeros(T, dtype=torch.int32, device="cuda"), table)))
+    assert torch.equal(got["out"], attend(torch.arange(T, dtype=torch.int32, device="cuda"), table.expand(T, pages).contiguous()))
+    lat, at = cache[table[0].long(), 0].reshape(pages, -1), torch.arange(T, device="cuda")
+    key = lat[:, :page * (rank + rot)].reshape(pages * page, rank + rot)[:T].double()
+    val = lat[:, page * (rank + rot):].reshape(pages, rank, page).transpose(1, 2).reshape(pages * page, rank)[:T].double()
+    s = torch.matmul(q.view(T, heads, -1).bfloat16().double().transpose(0, 1), key.T.contiguous()) * scale
+    s = s.masked_fill(at[None, :] > at[:, None], float("-inf"))
+    m = s.amax(-1, keepdim=True) if sinks is None else torch.maximum(s.amax(-1, keepdim=True), sinks.double()[:, None, None])
+    w = torch.exp(s - m)
+    want = torch.matmul(w, val) / (w.sum(-1, keepdim=True) + (0 if sinks is None else torch.exp(sinks.double()[:, None, None] - m)))
+    # the weights are rounded to 8 bits: each off by at most 2^-9 of itself
+    assert float((got["out"].view(T, heads, rank).transpose(0, 1).double() - want).abs().max()) <= 2.0 ** -8 * float(val.abs().max())
+    return hit
+
+
 def check_conv(dtype, T, C):
     """The short causal convolution of one request that goes on, and of the tokens behind it, one request each."""
     k = kernels(dtype)
@@ -415,6 +447,12 @@ CASES = [
     (BF, ["causal_conv<1>"], check_conv, (BF, 517, 2564)),
     (F32, ["causal_conv<0>"], check_conv, (F32, 1023, 260)),
     (F32, ["causal_conv<1>"], check_conv, (F32, 2049, 640)),
+    # latent attention: many tokens by (tiles of 16 latent dims, chunks of 32 key dims, bounds known when compiled, sink), and
+    # the kernel of a wave a token
+    *[(BF, [f"latent_prompt<{rt},{qc},1,{sink}>"], check_latent, (16 * rt, 32 * qc - 16 * rt, sink))
+      for rt, qcs in ((32, (18,)),) for qc in qcs for sink in (0, 1)],
+    *[(BF, [f"latent_prompt<{rt},{qc},0,{sink}>", f"latent_tokens<{rt},{qc},{sink}>"], check_latent, (rank, rot, sink))
+      for rt, qc, rank, rot in ((4, 4, 48, 16), (8, 8, 112, 48), (32, 20, 192, 64)) for sink in (0, 1)],
     # attention on the matrix cores: (head size, query heads a block, pages of 64 positions or more)
     # and (head size, waves a block) (one wave a block in the decoding kernel up to 2,560 blocks of
     # positions, four beyond; two heads a block in the prompt kernel where tiles x heads are more

@@ -1,5 +1,6 @@
 """Latent attention in steps of many tokens: eight tokens a block through LDS give the bits of a wave a token, for every
-size class, page, window and sink, with tokens of several requests side by side and runs that start anywhere."""
+size class, page, window and sink, with tokens of several requests side by side and runs that start anywhere: tiles of one
+request, of two, of decoding rows with the end or the start of a portion, of several short portions."""
 import pytest
 import torch
 
@@ -9,13 +10,18 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("rank,rot,page,window,heads", [(512, 64, 64, 0, 16), (512, 64, 128, 100, 16), (512, 128, 64, 70, 16), (48, 16, 64, 0, 32),
-                                                        (64, 64, 64, 65, 16), (128, 32, 192, 0, 16), (112, 48, 64, 1, 16), (256, 64, 64, 0, 16)])
+                                                        (64, 64, 64, 65, 16), (128, 32, 192, 0, 16), (112, 48, 64, 1, 16), (256, 64, 64, 0, 16),
+                                                        (512, 32, 64, 130, 16), (256, 32, 64, 50, 32), (64, 32, 128, 0, 32), (64, 128, 64, 200, 16)])
 @pytest.mark.parametrize("sink", [False, True])
 def test_many_tokens_have_the_bits_of_few(rank, rot, page, window, heads, sink):
     k = kernels("bfloat16")
-    assert k.latent_attention_uses_mfma(heads, rank, rot, page) if hasattr(k, "latent_attention_uses_mfma") else True
+    assert k.lib.axk_latent_attention_uses_mfma(heads, rank, rot, page)
     g = torch.Generator(device="cuda").manual_seed(rank + window)
-    runs = [(0, 0, 61), (1, 7, 3), (2, 130, 133), (1, 10, 1), (0, 61, 77), (3, 300, 38)]           # request, first position, tokens
+    # request, first position, tokens (tiles of eight: three requests in the eighth, a portion of one token more at its end)
+    runs = [(0, 0, 61), (1, 7, 3), (2, 130, 133), (1, 10, 1), (0, 61, 77), (3, 300, 38)]
+    if heads == 16:
+        # decoding rows, the end of a portion behind some and the start of one before others, portions of two and three tokens
+        runs += [(1, 40 + i, 1) if i % 2 else (2, 20 + i, 1) for i in range(13)] + [(3, 10, 3), (0, 9, 2), (1, 30, 2), (2, 50, 3), (3, 77, 1), (0, 200, 9), (1, 100, 190)]
     T, most = sum(n for _, _, n in runs), 400
     pages = -(-most // page)
     cache = torch.randn(4 * pages, 1, page, 2 * rank + rot, generator=g, device="cuda").bfloat16()
@@ -30,11 +36,19 @@ def test_many_tokens_have_the_bits_of_few(rank, rot, page, window, heads, sink):
         k.latent_attention(q[a:b].contiguous(), cache, table, pos[a:b].contiguous(), rows[a:b].contiguous(), out, heads, rank, rot, page, window,
                            (rank + rot) ** -0.5, sink=sinks)
         return out
-    assert T * (heads // 16) >= 256
+    assert T * (heads // 16) >= 512                                      # (from 256 on without a window)
+    k.reset_instances()
     whole, step = attend(0, T), 200 // (heads // 16)
+    assert any(name.startswith("latent_prompt<") for name in k.instances(launched=True))
+    # every token a request of its own: a wave each
+    alone = torch.full((T, heads * rank), float("nan"), device="cuda")
+    k.latent_attention(q, cache, table[rows.long()].contiguous(), pos, torch.arange(T, dtype=torch.int32, device="cuda"), alone, heads, rank,
+                       rot, page, window, (rank + rot) ** -0.5, sink=sinks)
+    assert torch.equal(whole, alone)
     if window == 0:                     # (over a window few rows run their blocks side by side, which is another order of sums)
+        k.reset_instances()
         few = torch.cat([attend(a, min(a + step, T)) for a in range(0, T, step)])
-        assert torch.equal(whole, few)
+        assert torch.equal(whole, few) and not any(name.startswith("latent_prompt<") for name in k.instances(launched=True))
     assert torch.equal(whole[5:], attend(5, T))                          # other tokens side by side
     lat = cache[:, 0, :, :].reshape(4 * pages, -1)
     for t in (0, 60, 62, 70, 197, T - 1):                                # against float64, weights and queries rounded as the kernel does
