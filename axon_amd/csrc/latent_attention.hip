@@ -786,10 +786,18 @@ extern "C" int axk_latent_attention(const float* q_full, const void* cache, cons
   launch_latent_prompt<RT, QC, EXACT>(q_full, cache, block_table, table_stride, positions, seq_rows, o_lat, n_tokens, heads, rank, rot, page_size, \
                                window, scale, sink, s)
       int rc;
-      // a latent of 512 beside 64 rotated dims: every bound known when compiled, so that a block's reads of LDS can be one
-      // stretch of instructions (no branch may stand between such a read and its wait)
-      if (rank == 512 && rot == 64) rc = LATENT_PROMPT(32, 18, true);
-      else if (rank <= 64 && rank + rot <= 128) rc = LATENT_PROMPT(4, 4, false);
+      const int rt = rank / 16, qc = (rank + rot) / 32;
+      // Latents of a power of two from 64 to 512 beside 32, 64 or 128 rotated dims: every bound known when compiled, so that a
+      // block's reads of LDS can be one stretch of instructions (no branch may stand between such a read and its wait).
+      // 2,048 tokens of 16 heads, bounds known when launched against here: 512 + 32 283 / 194 us, 512 + 128 299 / 227, 256 +
+      // 64 (32 heads) 242 / 162, 256 + 32 197 / 130, 128 + 64 118 / 96, 64 + 64 98 / 83, 64 + 32 85 / 77.
+#define LATENT_EXACT(RT, QC) if (rt == RT && qc == QC) rc = LATENT_PROMPT(RT, QC, true); else
+      LATENT_EXACT(32, 17) LATENT_EXACT(32, 18) LATENT_EXACT(32, 20)
+      LATENT_EXACT(16, 9) LATENT_EXACT(16, 10) LATENT_EXACT(16, 12)
+      LATENT_EXACT(8, 5) LATENT_EXACT(8, 6) LATENT_EXACT(8, 8)
+      LATENT_EXACT(4, 3) LATENT_EXACT(4, 4) LATENT_EXACT(4, 6)
+#undef LATENT_EXACT
+      if (rank <= 64 && rank + rot <= 128) rc = LATENT_PROMPT(4, 4, false);
       else if (rank <= 128 && rank + rot <= 256) rc = LATENT_PROMPT(8, 8, false);
       else rc = LATENT_PROMPT(32, 20, false);
 #undef LATENT_PROMPT

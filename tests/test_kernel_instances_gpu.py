@@ -450,7 +450,7 @@ CASES = [
     # latent attention: many tokens by (tiles of 16 latent dims, chunks of 32 key dims, bounds known when compiled, sink), and
     # the kernel of a wave a token
     *[(BF, [f"latent_prompt<{rt},{qc},1,{sink}>"], check_latent, (16 * rt, 32 * qc - 16 * rt, sink))
-      for rt, qcs in ((32, (18,)),) for qc in qcs for sink in (0, 1)],
+      for rt, qcs in ((32, (17, 18, 20)), (16, (9, 10, 12)), (8, (5, 6, 8)), (4, (3, 4, 6))) for qc in qcs for sink in (0, 1)],
     *[(BF, [f"latent_prompt<{rt},{qc},0,{sink}>", f"latent_tokens<{rt},{qc},{sink}>"], check_latent, (rank, rot, sink))
       for rt, qc, rank, rot in ((4, 4, 48, 16), (8, 8, 112, 48), (32, 20, 192, 64)) for sink in (0, 1)],
     # attention on the matrix cores: (head size, query heads a block, pages of 64 positions or more)
