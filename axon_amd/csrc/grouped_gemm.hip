@@ -343,14 +343,9 @@ __global__ void __launch_bounds__(256, 2) grouped_gemm_tile_kernel(GroupedArgs a
     u32x4 xf[2][XT], wf[2][4];
     read_frags<XT, 2048>(xf[0], xr);
     read_frags<4, 2048>(wf[0], wr);
-    const bool both = t * GT_BK + 32 < a.K;
-    if (both) {
-      read_frags<XT, 2048>(xf[1], xr ^ 64);
-      read_frags<4, 2048>(wf[1], wr ^ 64);
-      wait_lgkmcnt<XT + 4>();
-    } else {
-      wait_lgkmcnt<0>();
-    }
+    read_frags<XT, 2048>(xf[1], xr ^ 64);          // (no branch between a read and its wait: the half a short K lacks is read too)
+    read_frags<4, 2048>(wf[1], wr ^ 64);
+    wait_lgkmcnt<XT + 4>();
     use_frags<XT>(xf[0]);
     use_frags<4>(wf[0]);
 #pragma unroll
@@ -359,10 +354,10 @@ __global__ void __launch_bounds__(256, 2) grouped_gemm_tile_kernel(GroupedArgs a
       for (int j = 0; j < 4; ++j)
         acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gg_bf16x8, wf[0][j]), __builtin_bit_cast(gg_bf16x8, xf[0][i]),
                                                             acc[i][j], 0, 0, 0);
-    if (both) {
-      wait_lgkmcnt<0>();
-      use_frags<XT>(xf[1]);
-      use_frags<4>(wf[1]);
+    wait_lgkmcnt<0>();
+    use_frags<XT>(xf[1]);
+    use_frags<4>(wf[1]);
+    if (t * GT_BK + 32 < a.K) {
 #pragma unroll
       for (int i = 0; i < XT; ++i)
 #pragma unroll
