@@ -236,16 +236,15 @@ __global__ void __launch_bounds__(256) grouped_gemm_mfma_kernel(GroupedArgs a) {
 }
 
 // Many rows a group (a long prompt's pairs of an expert, the tokens of a prompt through a block of
-// channels): 64 rows x 256 rows of W a block, through two stages of 64 k of LDS that are filled by direct loads
-// (X in float32: through registers, where it is rounded).  Four waves, each the 64 rows x 64 rows of W
-// (4 x 4 products a step of 32 k); with the gated epilogue a wave's 64 rows of W are 32 gate rows and the 32
+// channels): 64 rows x 128 or 256 rows of W a block, through two stages of 64 k of LDS that are filled by direct loads
+// (X in float32: through registers, where it is rounded).  Four waves, each all or half of the 64 rows x 64 rows of W
+// (up to 4 x 4 products a step of 32 k); with the gated epilogue a wave's 64 rows of W are 32 gate rows and the 32
 // up rows of the same columns.  The next stage is on its way while this one is multiplied, and the two halves
 // of a stage are read one ahead of the products.  Rows of a stage are 128 bytes, their 16-byte slots permuted by
-// slot ^ (row / 2 % 8): the 16 rows a read takes at a time fall into 16 different slots of the 64 banks.  Bound by the
-// way into LDS and out of it (80 bytes a cycle in, 128 out at the matrix cores' full rate).  The chain of an
+// slot ^ (row / 2 % 8): the 16 rows a read takes at a time fall into 16 different slots of the 64 banks.  The chain of an
 // output is the one of the kernel above (16x16x32 products in ascending k), so which of the two runs changes no
-// bit.  2,048 tokens, 4 of 32 experts of [1,408, 2,048] and [2,048, 704]: 84 and 75 us (163 and 113 with stages of 32 k
-// through registers and 128 rows of W).
+// bit.  2,048 tokens, 4 of 32 experts of [1,408, 2,048] and [2,048, 704]: 81 and 63 us (163 and 113 with stages of 32 k
+// through registers).
 #define GT_ROWS 64
 #define GT_BK 64
 #define GT_STAGE(wrows) ((GT_ROWS + (wrows)) * GT_BK * 2)
@@ -253,7 +252,7 @@ typedef const __attribute__((address_space(1))) void* gg_global_t;
 typedef __attribute__((address_space(3))) void* gg_lds_t;
 template <bool GLU, bool XF32, int WROWS>
 __global__ void __launch_bounds__(256, 2) grouped_gemm_tile_kernel(GroupedArgs a) {
-  static_assert(WROWS == 256 || (WROWS == 128 && !GLU), "a wave's 64 rows of W, for all or for half of the rows of X");
+  static_assert(WROWS == 128 || (WROWS == 256 && GLU), "a wave's 64 rows of W, for half or for all of the rows of X");
   constexpr int STAGE = GT_STAGE(WROWS), XT = WROWS / 64, WL = WROWS / 32;   // tiles of 16 rows a wave, load instructions of W a wave
   extern __shared__ __align__(256) unsigned char stages[];        // [2]: X [64][64], W [WROWS][64]
   constexpr int COLS = GLU ? WROWS / 2 : WROWS;
@@ -280,9 +279,9 @@ __global__ void __launch_bounds__(256, 2) grouped_gemm_tile_kernel(GroupedArgs a
   long w_at[WL];
 #pragma unroll
   for (int i = 0; i < WL; ++i) {
-    const int place = 8 * i + lrow;
-    const int col = GLU ? n0 + 32 * wave + (place & 31) : n0 + 8 * WL * wave + place;
-    w_at[i] = (long)(min(col, a.N - 1) + (GLU && place >= 32 ? a.N : 0)) * a.K + 8 * (lslot ^ (4 * (i & 1) + (lane >> 4)));
+    const int row = 8 * WL * wave + 8 * i + lrow;                                // of the stage's W
+    const int col = GLU ? n0 + 32 * (row >> 6) + (row & 31) : n0 + row;
+    w_at[i] = (long)(min(col, a.N - 1) + (GLU && (row & 32) ? a.N : 0)) * a.K + 8 * (lslot ^ (4 * (i & 1) + (lane >> 4)));
   }
   long x_at[2];
 #pragma unroll
@@ -343,7 +342,7 @@ __global__ void __launch_bounds__(256, 2) grouped_gemm_tile_kernel(GroupedArgs a
     u32x4 xf[2][XT], wf[2][4];
     read_frags<XT, 2048>(xf[0], xr);
     read_frags<4, 2048>(wf[0], wr);
-    read_frags<XT, 2048>(xf[1], xr ^ 64);          // (no branch between a read and its wait: the half a short K lacks is read too)
+    read_frags<XT, 2048>(xf[1], xr ^ 64);          // (no branch between a read and its wait: the halves a short K lacks are read too)
     read_frags<4, 2048>(wf[1], wr ^ 64);
     wait_lgkmcnt<XT + 4>();
     use_frags<XT>(xf[0]);
@@ -389,6 +388,7 @@ int launch_tile(const GroupedArgs& a, dim3 grid, hipStream_t s) {
     }
     configured = true;
   }
+  AXK_INSTANCE(INST_GROUPED_GEMM, WROWS == 256 ? 2 : 3, GLU);
   grouped_gemm_tile_kernel<GLU, XF32, WROWS><<<grid, 256, 2 * GT_STAGE(WROWS), s>>>(a);
   return 0;
 }
@@ -433,18 +433,21 @@ extern "C" int axk_grouped_gemm(const void* x, int x_is_f32, long x_row_stride, 
                     ((uintptr_t)w & 15) == 0;
   // many rows a group: tiles of 64 rows through LDS (a list of tiles says by its tile size which it was made for)
   if (mfma && (tiles ? tile_rows == 64 : m >= 256)) {
-    // up to 128 columns a group (a head's values out of its latent): half the rows of W would be none
-    const bool narrow = !glu && n <= 128;
-    const long blocks = (long)(tiles ? max_tiles : ceil_div(m, GT_ROWS)) * ceil_div(n, glu || narrow ? 128 : 256) * (tiles ? 1 : groups);
+    // 128 rows of W a block, three blocks a CU, unless the gated product has two rounds of blocks of 256: those read
+    // X half as often, which pays where K is long.  us, 256 rows of W a block against 128: 10 blocks of channels [512, 256] at
+    // 256 rows 14.7 / 9.4, at 2,048 38 / 26; 16 heads [512, 128] at 2,048 41 / 27; 4 of 32 experts of 2,048 tokens
+    // [2,048, 704] 69 / 63, gated [1,408, 2,048] 81 / 85, of 1,024 tokens (576 blocks) 46 / 57, of 512 (384) 44 / 41, of
+    // 256 41 / 33; 2 of 8 of 128 tokens gated [1,024, 1,024] 20 / 16; 8 of 64 of 2,048 gated [512, 2,048] 74 / 67.
+    const long row_blocks = (long)(tiles ? max_tiles : ceil_div(m, GT_ROWS)) * (tiles ? 1 : groups);
+    const bool wide = glu && row_blocks * ceil_div(n, 128) >= 512;
+    const long blocks = row_blocks * ceil_div(n, glu && !wide ? 64 : 128);
     AXK_REQUIRE(blocks < (1l << 31) - 8, "grouped_gemm: %ld blocks are more than one launch takes", blocks);
     const dim3 big((unsigned)((blocks + 7) / 8 * 8));
     int rc;
-    if (glu) { AXK_INSTANCE(INST_GROUPED_GEMM, 2, 1); rc = x_is_f32 ? launch_tile<true, true, 256>(a, big, s) : launch_tile<true, false, 256>(a, big, s); }
-    else {
-      AXK_INSTANCE(INST_GROUPED_GEMM, 2, 0);
-      if (narrow) rc = x_is_f32 ? launch_tile<false, true, 128>(a, big, s) : launch_tile<false, false, 128>(a, big, s);
-      else rc = x_is_f32 ? launch_tile<false, true, 256>(a, big, s) : launch_tile<false, false, 256>(a, big, s);
-    }
+#define TILE(GLU, WROWS) (x_is_f32 ? launch_tile<GLU, true, WROWS>(a, big, s) : launch_tile<GLU, false, WROWS>(a, big, s))
+    if (wide) rc = TILE(true, 256);
+    else rc = glu ? TILE(true, 128) : TILE(false, 128);
+#undef TILE
     if (rc) return rc;
     AXK_LAUNCH_CHECK("grouped_gemm");
     return 0;

@@ -1,5 +1,6 @@
-"""The grouped products' two matrix-core kernels at the edges of their tiles: the one for many rows (64 x 256 or 64 x 128
-through LDS) gives the bits of the one for few, whatever the sizes, the type of X and the layout of the output."""
+"""The grouped products' two matrix-core kernels at the edges of their tiles: the one for many rows (64 x 128, or 64 x 256
+where a gated product has many of these, through LDS) gives the bits of the one for few, whatever the sizes, the type of X
+and the layout of the output."""
 import pytest
 import torch
 
@@ -8,20 +9,23 @@ from axon_amd.kernels import kernels
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("N,K,G", [(8, 32, 2), (128, 96, 3), (129, 64, 2), (260, 160, 1), (300, 288, 2)])
+@pytest.mark.parametrize("N,K,G,M", [(8, 32, 2, 321), (128, 96, 3, 321), (129, 64, 2, 321), (260, 160, 1, 321), (300, 288, 2, 321),
+                                     (64, 64, 2, 321), (65, 32, 1, 400), (200, 96, 16, 1030), (129, 32, 43, 321)])
 @pytest.mark.parametrize("x_f32", [False, True])
 @pytest.mark.parametrize("glu", [None, (1.5, 1.702)])
-def test_many_rows_have_the_bits_of_few(N, K, G, x_f32, glu):
+def test_many_rows_have_the_bits_of_few(N, K, G, M, x_f32, glu):
     k = kernels("bfloat16")
     g = torch.Generator(device="cuda").manual_seed(N * K)
-    M = 321
     x = torch.randn(M, G * K, generator=g, device="cuda")
     x = x if x_f32 else x.bfloat16()
     w = (torch.randn(G, (2 if glu else 1) * N, K, generator=g, device="cuda") * 0.2).bfloat16()
     for out_dtype, pad in ((torch.float32, 0), (torch.bfloat16, 1), (torch.bfloat16, 4)):
         ogs = N + pad
         out = torch.full((M, G * ogs), float("nan"), dtype=out_dtype, device="cuda")
+        k.reset_instances()
         k.grouped_gemm(x, w, out, x_group_stride=K, out_group_stride=ogs, glu=glu)
+        wide = glu is not None and -(-M // 64) * G * -(-N // 128) >= 512
+        assert k.instances(launched=True) == [f"grouped_gemm<{2 if wide else 3},{0 if glu is None else 1}>"]
         for first, m in ((0, 200), (121, 200)):                      # few rows: the other kernel
             few = torch.full((m, G * ogs), float("nan"), dtype=out_dtype, device="cuda")
             k.grouped_gemm(x[first:first + m], w, few, x_group_stride=K, out_group_stride=ogs, glu=glu)

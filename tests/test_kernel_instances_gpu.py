@@ -438,8 +438,9 @@ CASES = [
     (BF, ["grouped_gemm<1,1>"], check_grouped, (BF, 19, 2, 72, 160, True)),
     (BF, ["grouped_gemm<0,0>"], check_grouped, (BF, 50, 3, 40, 24, False)),
     (BF, ["grouped_gemm<0,1>"], check_grouped, (BF, 19, 2, 72, 40, True)),
-    (BF, ["grouped_gemm<2,0>"], check_grouped, (BF, 300, 3, 40, 64, False)),       # many rows: tiles of 64 through LDS
-    (BF, ["grouped_gemm<2,1>"], check_grouped, (BF, 270, 2, 72, 160, True)),
+    (BF, ["grouped_gemm<3,0>"], check_grouped, (BF, 300, 3, 40, 64, False)),       # many rows: tiles of 64 through LDS
+    (BF, ["grouped_gemm<3,1>"], check_grouped, (BF, 270, 2, 72, 160, True)),
+    (BF, ["grouped_gemm<2,1>"], check_grouped, (BF, 1030, 16, 200, 96, True)),     # gated, two rounds of large blocks
     (F32, ["grouped_gemm<0,0>"], check_grouped, (F32, 50, 3, 40, 64, False)),
     (F32, ["grouped_gemm<0,1>"], check_grouped, (F32, 19, 2, 72, 160, True)),
     # the short convolution: a thread a (token, channel), and runs of tokens in long steps
