@@ -176,12 +176,11 @@ __device__ inline void gg_store4(const GroupedArgs& a, int g, int orow, int n, c
 // 16 rows x 64 columns a block of four waves, a wave 16 columns: W rows as the MFMA's first
 // operand, X rows as its second, both straight from memory (lane l holds row l % 16, the eight k
 // from 8 (l / 16)); lane l ends with row l % 16 of the columns 4 (l / 16) .. + 3.  Such a product waits for W
-// alone, and an output is one chain over k, so a wave keeps GG_RING steps of 32 k under way: each is asked
+// alone, and an output is one chain over k, so a wave keeps RING steps of 32 k under way: each is asked
 // for again as soon as it is multiplied.  Rows and columns that do not exist read ones that do.  The 32 pairs
 // of 8 tokens over 32 experts of [1,408, 2,048] and [2,048, 704]: 42 and 19 us, launches included (120 and 45 with four steps
 // asked for at a time and waited for together).
-#define GG_RING 8
-template <bool GLU, bool XF32>
+template <bool GLU, bool XF32, int RING>
 __global__ void __launch_bounds__(256) grouped_gemm_mfma_kernel(GroupedArgs a) {
   int g, first, count;
   if (!gg_tile(a, g, first, count)) return;
@@ -197,7 +196,7 @@ __global__ void __launch_bounds__(256) grouped_gemm_mfma_kernel(GroupedArgs a) {
   const bf16_t* wrow = a.w + ((long)g * w_rows + min(n0 + r, a.N - 1)) * a.K + kq;
   const bf16_t* urow = wrow + (long)a.N * a.K;
   gg_f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f}, acc_up = {0.0f, 0.0f, 0.0f, 0.0f};
-  uint4 xf[GG_RING][XF32 ? 2 : 1], wf[GG_RING], uf[GLU ? GG_RING : 1];
+  uint4 xf[RING][XF32 ? 2 : 1], wf[RING], uf[GLU ? RING : 1];
   auto ask = [&](int s, int k) {
     if (XF32) {
       xf[s][0] = *reinterpret_cast<const uint4*>((const float*)a.x + x_at + k);
@@ -219,17 +218,17 @@ __global__ void __launch_bounds__(256) grouped_gemm_mfma_kernel(GroupedArgs a) {
   };
   // (a step behind the last asks for the last again: a branch would have every load under way waited for)
 #pragma unroll
-  for (int s = 0; s < GG_RING; ++s) ask(s, min(32 * s, a.K - 32));
+  for (int s = 0; s < RING; ++s) ask(s, min(32 * s, a.K - 32));
   int k0 = 0;
-  for (; k0 + 32 * GG_RING <= a.K; k0 += 32 * GG_RING) {
+  for (; k0 + 32 * RING <= a.K; k0 += 32 * RING) {
 #pragma unroll
-    for (int s = 0; s < GG_RING; ++s) {
+    for (int s = 0; s < RING; ++s) {
       multiply(s);
-      ask(s, min(k0 + 32 * (GG_RING + s), a.K - 32));
+      ask(s, min(k0 + 32 * (RING + s), a.K - 32));
     }
   }
 #pragma unroll
-  for (int s = 0; s < GG_RING; ++s)
+  for (int s = 0; s < RING; ++s)
     if (k0 + 32 * s < a.K) multiply(s);
   if (r >= count) return;
   gg_store4(a, g, orow, n0 + (lane >> 4) * 4, acc, acc_up);
@@ -453,15 +452,20 @@ extern "C" int axk_grouped_gemm(const void* x, int x_is_f32, long x_row_stride, 
     return 0;
   }
   if (mfma) {
+    // A K of up to 256 in a ring of four, beside whose registers more waves have room and which asks for little beyond it:
+    // 4 groups of [64, 32] at 130 rows 4.7 us with eight, 3.9 with four, 16 of [512, 96] at 255 21 / 13, 8 of 64
+    // experts of 128 tokens [2,048, 256] 46 / 37, 16 of [512, 128] at 8 rows 4.5 / 4.7; but 8 of 128 of 4 [1,536, 2,048] 76 / 103.
+#define FEW(GLU, RING)                                                                          \
+  if (x_is_f32) grouped_gemm_mfma_kernel<GLU, true, RING><<<grid, 256, 0, s>>>(a);              \
+  else grouped_gemm_mfma_kernel<GLU, false, RING><<<grid, 256, 0, s>>>(a);
     if (glu) {
-      AXK_INSTANCE(INST_GROUPED_GEMM, 1, 1);
-      if (x_is_f32) grouped_gemm_mfma_kernel<true, true><<<grid, 256, 0, s>>>(a);
-      else grouped_gemm_mfma_kernel<true, false><<<grid, 256, 0, s>>>(a);
+      if (k <= 256) { AXK_INSTANCE(INST_GROUPED_GEMM, 4, 1); FEW(true, 4) }
+      else { AXK_INSTANCE(INST_GROUPED_GEMM, 1, 1); FEW(true, 8) }
     } else {
-      AXK_INSTANCE(INST_GROUPED_GEMM, 1, 0);
-      if (x_is_f32) grouped_gemm_mfma_kernel<false, true><<<grid, 256, 0, s>>>(a);
-      else grouped_gemm_mfma_kernel<false, false><<<grid, 256, 0, s>>>(a);
+      if (k <= 256) { AXK_INSTANCE(INST_GROUPED_GEMM, 4, 0); FEW(false, 4) }
+      else { AXK_INSTANCE(INST_GROUPED_GEMM, 1, 0); FEW(false, 8) }
     }
+#undef FEW
     AXK_LAUNCH_CHECK("grouped_gemm");
     return 0;
   }

@@ -434,8 +434,10 @@ CASES = [
     (BF, ["gemm_tile<256,256,4,2,1,2>"], check_gemm, (BF, 200, 18944, 3584, MODE_SWIGLU)),              # a 7B layer's at 200 rows
     (BF, ["gemm_tile<256,256,4,2,0,2>", "gemm_split_reduce<2>"], check_qkv_rope, (2048, 28, 4, 128, 3584, 64)),
     # grouped products: (matrix cores or 32-bit FMA, gated epilogue)
-    (BF, ["grouped_gemm<1,0>"], check_grouped, (BF, 50, 3, 40, 64, False)),
-    (BF, ["grouped_gemm<1,1>"], check_grouped, (BF, 19, 2, 72, 160, True)),
+    (BF, ["grouped_gemm<4,0>"], check_grouped, (BF, 50, 3, 40, 64, False)),
+    (BF, ["grouped_gemm<4,1>"], check_grouped, (BF, 19, 2, 72, 160, True)),
+    (BF, ["grouped_gemm<1,0>"], check_grouped, (BF, 50, 3, 40, 288, False)),
+    (BF, ["grouped_gemm<1,1>"], check_grouped, (BF, 19, 2, 72, 544, True)),
     (BF, ["grouped_gemm<0,0>"], check_grouped, (BF, 50, 3, 40, 24, False)),
     (BF, ["grouped_gemm<0,1>"], check_grouped, (BF, 19, 2, 72, 40, True)),
     (BF, ["grouped_gemm<3,0>"], check_grouped, (BF, 300, 3, 40, 64, False)),       # many rows: tiles of 64 through LDS
