@@ -182,16 +182,17 @@ __device__ inline f32x4 fma_operand(const float (&v)[4]) {
 // chains of an output, which do not need each other, are shared out over its 8 waves: every wave
 // streams its chains' W from memory straight into operands, leaves the chains' sums in LDS, and a thread
 // an output adds them in ascending order.  MT tiles of 16 rows of X ride along with each W (a wave reads
-// them from L2 beside W: with 64 rows of X that is what bounds it).  5 rows: 2,560 x K 2,048 25 -> 16 us,
+// them from L2 beside W: with 64 rows of X that is what bounds it).  SHORT: a K of no more chains than waves, one
+// each (8 rows of 512 x K 256 6.5 us with all of them in one wave, 4.1 here).  5 rows: 2,560 x K 2,048 25 -> 16 us,
 // 2,048 x 5,632 63 -> 27, 32,000 x 2,048 (262 MB) 85 -> 61 us, 4.3 TB/s; 64 rows of 2,048 x 5,632 332 -> 63 us.
 #define FEW_WAVES 8
-template <int MT, int NR, bool GLU, bool VEC>
+template <int MT, int NR, bool GLU, bool VEC, bool SHORT>
 __global__ void __launch_bounds__(64 * FEW_WAVES, 2)
 gemm_fma_few_rows_kernel(const elem_t* __restrict__ x, int x_stride, const elem_t* __restrict__ w,
                          const void* __restrict__ bias, int bias_is_f32, void* __restrict__ out, int out_stride, int M,
                          int N, int K, int mode) {
   constexpr int NT = GLU ? 2 : 1;
-  constexpr int PW = MT * NT >= 8 ? 1 : MT * NT >= 3 ? 2 : MT * NT == 2 ? 4 : 8;   // chains of a wave in a round
+  constexpr int PW = SHORT || MT * NT >= 8 ? 1 : MT * NT >= 3 ? 2 : MT * NT == 2 ? 4 : 8;   // chains of a wave in a round
   constexpr int PARTS = FEW_WAVES * PW, OUTS = MT * 16 * NR;
   __shared__ __align__(16) float chains[PARTS * NT * OUTS];                        // [chain][gate, up][row][column]
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -278,12 +279,13 @@ static void launch_fma_few(const elem_t* x, int x_stride, const elem_t* w, const
                            int out_stride, int m, int n, int k, int mode, hipStream_t stream) {
   const int rows = ceil_div(m, 16 * MT);
   // blocks of 8 columns where blocks of 16 would leave CUs without one
-  if ((long)ceil_div(n, 16) * rows < 256)
-    gemm_fma_few_rows_kernel<MT, 8, GLU, VEC><<<dim3(ceil_div(n, 8), rows), 64 * FEW_WAVES, 0, stream>>>(
-        x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode);
-  else
-    gemm_fma_few_rows_kernel<MT, 16, GLU, VEC><<<dim3(ceil_div(n, 16), rows), 64 * FEW_WAVES, 0, stream>>>(
-        x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode);
+  const bool narrow = (long)ceil_div(n, 16) * rows < 256, brief = k <= FEW_WAVES * FMA_PART;
+#define FEW(NR, SHORT)                                                                                                \
+  gemm_fma_few_rows_kernel<MT, NR, GLU, VEC, SHORT><<<dim3(ceil_div(n, NR), rows), 64 * FEW_WAVES, 0, stream>>>(      \
+      x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode)
+  if (brief) { if (narrow) FEW(8, true); else FEW(16, true); }
+  else { if (narrow) FEW(8, false); else FEW(16, false); }
+#undef FEW
 }
 
 static int launch_fma(const elem_t* x, int x_stride, const elem_t* w, const void* bias, int bias_is_f32, void* out,
