@@ -294,19 +294,24 @@ static int launch_fma(const elem_t* x, int x_stride, const elem_t* w, const void
   const bool vec_w = (k % 4 == 0) && ((uintptr_t)w % vbytes == 0);
   const bool vec_x = (k % 4 == 0) && (x_stride % 4 == 0) && ((uintptr_t)x % vbytes == 0);
 #define FMA_ARGS x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode, stream
-// Up to 64 rows a product waits for W; from 65 to 128 so it does where the tiles would be fewer than
+// Up to 32 rows a product waits for W; from 33 to 128 so it does where the tiles would be fewer than
 // the CUs (2,048 columns of K 5,632 at 128 rows: 143 us with 64 tiles, 67 us with a wave a part of K), while
-// 352 tiles (a gated product of 5,632 columns) take 90 us against 117.
+// 352 tiles (a gated product of 5,632 columns at 128 rows) take 90 us against 117 and 500 (32,000 columns of K 2,048
+// at 33 and at 64 rows) 89 and 92 against 142 and 158.
 #define FMA_LAUNCH(GLU, VEC)                                                                  \
+  const dim3 tiles(ceil_div(n, GLU ? TILE_M / 2 : TILE_M), ceil_div(m, TILE_M));              \
   if (m <= 16) {                                                                              \
     AXK_INSTANCE(INST_GEMM_FMA, 16, GLU);                                                     \
     launch_fma_few<1, GLU, VEC>(FMA_ARGS);                                                    \
-  } else {                                                                                    \
+  } else if (m <= 32) {                                                                       \
+    AXK_INSTANCE(INST_GEMM_FMA, 32, GLU);                                                     \
+    launch_fma_few<2, GLU, VEC>(FMA_ARGS);                                                    \
+  } else if (m <= 128 && (long)tiles.x * tiles.y < 256) {                                     \
     AXK_INSTANCE(INST_GEMM_FMA, 64, GLU);                                                     \
-    const dim3 tiles(ceil_div(n, GLU ? TILE_M / 2 : TILE_M), ceil_div(m, TILE_M));            \
-    if (m <= 32) launch_fma_few<2, GLU, VEC>(FMA_ARGS);                                       \
-    else if (m <= 64 || (m <= 128 && (long)tiles.x * tiles.y < 256)) launch_fma_few<4, GLU, VEC>(FMA_ARGS); \
-    else gemm_fma_kernel<GLU, VEC><<<tiles, 256, 0, stream>>>(x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode); \
+    launch_fma_few<4, GLU, VEC>(FMA_ARGS);                                                    \
+  } else {                                                                                    \
+    AXK_INSTANCE(INST_GEMM_FMA, 128, GLU);                                                    \
+    gemm_fma_kernel<GLU, VEC><<<tiles, 256, 0, stream>>>(x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode); \
   }
   const bool glu = mode == MODE_SWIGLU;
   if (vec_x && vec_w) {

@@ -16,7 +16,7 @@
 #include <initializer_list>
 
 enum {
-  INST_GEMM_FMA = 0,
+  INST_GEMM_FMA = 0,         // rows of X a block (16, 32, 64: streaming W; 128: tiles through LDS), gated
   INST_GEMM_TILE,            // BM, BN, waves m, waves n, gated, stages
   INST_GEMM_STREAM,          // row tiles, tiles of X rows, segments, epilogue
   INST_GEMM_NORMED,          // tile pairs a wave, segments, epilogue, rows of X in LDS, float4 a lane

@@ -307,6 +307,10 @@ CASES = [
     (F32, ["gemm_fma<64,0>"], check_gemm, (F32, 70, 259, 130, MODE_ADD_F32)),
     (F32, ["gemm_fma<16,1>"], check_gemm, (F32, 9, 96, 70, MODE_SWIGLU)),
     (F32, ["gemm_fma<64,1>"], check_gemm, (F32, 33, 48, 100, MODE_SWIGLU)),
+    # (rows of X a block, gated; from 33 to 128 rows by how many tiles there would be)
+    *[(d, [f"gemm_fma<{rows},{int(mode == MODE_SWIGLU)}>"], check_gemm, (d, M, N, K, mode)) for d in (F32, BF)
+      for rows, M, N, K, mode in ((32, 20, 259, 290, MODE_STORE_F32), (128, 200, 259, 130, MODE_STORE_F32), (128, 40, 16390, 36, MODE_STORE_F32),
+                                  (32, 31, 48, 100, MODE_SWIGLU), (128, 129, 48, 100, MODE_SWIGLU), (64, 128, 96, 290, MODE_SWIGLU))],
     (BF, ["gemm_fma<16,0>"], check_gemm, (BF, 5, 100, 70, MODE_STORE, True)),
     (BF, ["gemm_fma<64,0>"], check_gemm, (BF, 70, 259, 130, MODE_STORE_F32)),
     (BF, ["gemm_fma<16,1>"], check_gemm, (BF, 9, 96, 70, MODE_SWIGLU)),
