@@ -1,5 +1,5 @@
-"""The 32-bit products on the matrix cores at the sizes where their blocks, chains and rows end: against float64, and a
-row's bits whatever the number of rows (which picks the kernel)."""
+"""The 32-bit products on the matrix cores at the sizes where their blocks, chains and rows end: against float64, bit for
+bit against chains of fmaf, and a row's bits whatever the number of rows (which picks the kernel)."""
 import pytest
 import torch
 
@@ -36,3 +36,48 @@ def test_edges_of_rows_columns_and_chains(N, K, x_stride, mode):
         rows[m] = out
     for m in rows:
         assert torch.equal(rows[m], rows[200][:m]), m
+
+
+def _by_chains(k, x, w):
+    """x w^T as chains of 32 fmaf in ascending k whose sums are added in ascending order: every chain by the grouped
+    product's kernel of 32-bit fmaf on the vector unit, one chain over its whole K, with the 32 k of the chain."""
+    M, K = x.shape
+    total = torch.zeros(M, w.shape[0], device="cuda")
+    for k0 in range(0, K, 32):
+        part = torch.full_like(total, float("nan"))
+        a, b = x[:, k0:k0 + 32].contiguous(), w[:, k0:k0 + 32].contiguous()
+        k.grouped_gemm(a, b[None], part, x_group_stride=a.shape[1], out_group_stride=w.shape[0])
+        total = total + part
+    return total
+
+
+@pytest.mark.parametrize("N,K", [(65, 64), (130, 257), (16390, 70), (48, 8), (33, 2052)])
+@pytest.mark.parametrize("values", ["ordinary", "denormal", "wide"])
+def test_the_bits_are_those_of_chains_of_fmaf(N, K, values):
+    k = kernels("float32")
+    g = torch.Generator(device="cuda").manual_seed(K)
+    x, w = torch.randn(140, K, generator=g, device="cuda"), torch.randn(N, K, generator=g, device="cuda")
+    if values == "denormal":            # products of 2^-140 or so, sums of them, and some operands below 2^-126
+        x, w = x * 2.0 ** -70, w * 2.0 ** -68
+        x[:, ::7] *= 2.0 ** -65
+        w[:, ::7] *= 2.0 ** 66
+    if values == "wide":                # magnitudes over 2^-30 .. 2^30: what is lost shows which k was added when
+        x = x * 2.0 ** torch.randint(-15, 16, x.shape, generator=g, device="cuda")
+        w = w * 2.0 ** torch.randint(-15, 16, w.shape, generator=g, device="cuda")
+    want = _by_chains(k, x, w)
+    assert values != "denormal" or (bool((want.abs() < 2.0 ** -126).any()) and bool((want != 0).any()))
+    k.reset_instances()
+    for m in (140, 128, 40, 20, 7):     # tiles, and the kernel that streams W by 64, 32 and 16 rows
+        out = torch.full((m, N), float("nan"), device="cuda")
+        k.gemm(x[:m], w, out, None, MODE_STORE_F32)
+        assert torch.equal(out, want[:m]), m
+    assert {"gemm_fma<16,0>", "gemm_fma<32,0>", "gemm_fma<128,0>"} <= set(k.instances(launched=True))
+    if values == "ordinary":            # gated: silu(gate) up of both products' bits
+        half = N // 2
+        gate, up = want[:, :half], want[:, half:2 * half]
+        for m in (140, 128, 20, 7):
+            out = torch.full((m, half), float("nan"), device="cuda")
+            k.gemm(x[:m], w[:2 * half], out, None, MODE_SWIGLU)
+            act = torch.empty_like(out)
+            k.swiglu(torch.cat([gate, up], 1)[:m].contiguous(), act)
+            assert torch.equal(out, act), m
