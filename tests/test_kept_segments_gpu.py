@@ -42,3 +42,24 @@ def test_the_norm_behind(M, N, K):
     alone = torch.empty(200, N, dtype=torch.bfloat16, device="cuda")
     k.rmsnorm(plain, gain, 1e-6, alone)
     assert torch.equal(out[:200], plain) and torch.equal(normed[:200], alone)
+
+
+@pytest.mark.parametrize("M,N,K", [(1100, 9300, 128), (129, 130, 192), (2051, 2309, 768), (1153, 2306, 1088)])
+def test_sums_added_into_rows(M, N, K):
+    """Whole tiles and remainders in both directions, rows that lie apart, one segment of K and several: what was there
+    plus the product, and nothing beside the columns that the product has."""
+    k = kernels("bfloat16")
+    g = torch.Generator(device="cuda").manual_seed(M)
+    x = torch.randn(M, K, generator=g, device="cuda").bfloat16()
+    w = (torch.randn(N, K, generator=g, device="cuda") * 0.1).bfloat16()
+    bias = torch.randn(N, generator=g, device="cuda")
+    wide = torch.randn(M, N + 24, generator=g, device="cuda")
+    packed, prod = k.prepare_weight(w), torch.empty(M, N, device="cuda")
+    got = wide.clone()
+    k.gemm(x, packed, got[:, :N], bias, MODE_ADD_F32)
+    k.gemm(x, packed, prod, bias, MODE_STORE_F32)
+    assert torch.equal(got[:, :N], wide[:, :N] + prod) and torch.equal(got[:, N:], wide[:, N:])
+    want = x.double() @ w.double().T + bias.double()
+    # a chain of K products and a bias, each sum off by at most a unit of what it holds
+    bound = (K + 1) * 2.0 ** -23 * (x.double().abs() @ w.double().abs().T + bias.double().abs())
+    assert bool(((prod.double() - want).abs() <= bound).all())
