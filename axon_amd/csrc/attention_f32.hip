@@ -16,6 +16,7 @@
 
 #include "api.h"
 #include "common.h"
+#include "instances.h"
 
 #define ATT_BLOCK 64
 #define DC_CHUNK 256
@@ -434,6 +435,7 @@ int launch_attention_f32_prefill(const float* q, int q_stride, const float* k_ca
       }                                                                                                              \
       configured = true;                                                                                             \
     }                                                                                                                \
+    AXK_INSTANCE(INST_ATTENTION_F32_PREFILL, HD);                                                                    \
     attention_f32_prefill_kernel<HD><<<dim3(n_tiles, n_heads, 4), 256, lds, stream>>>(                               \
         q, q_stride, k_cache, v_cache, block_table, table_stride, positions, seq_rows, out, tiles, n_heads,          \
         n_kv_heads, page_size, window, scale);                                                                       \
@@ -455,6 +457,7 @@ int launch_attention_f32_decode(const float* q, int q_stride, const float* k_cac
   const bool single = n_work >= 2 * n_tokens || (long)n_work * n_kv_heads * 4 <= 256;
 #define LAUNCH(HD, BW)                                                                                               \
   {                                                                                                                  \
+    AXK_INSTANCE(INST_ATTENTION_F32_DECODE, HD, BW);                                                                 \
     attention_f32_decode_kernel<HD, BW><<<(unsigned)n_work * n_kv_heads * (4 / BW), 64 * BW, 0, stream>>>(           \
         q, q_stride, k_cache, v_cache, block_table, table_stride, positions, seq_rows, token_index, n_tokens, work,  \
         partial, max_chunks, n_heads, n_kv_heads, page_size, window, scale);                                         \

@@ -588,7 +588,8 @@ static int launch_tile(const bf16_t* x, int x_stride, const bf16_t* w, const voi
   const int splits = KEEP ? 1 : segs;
   const bool after = splits > 1 || norm || rope;
   const int m_blocks = ceil_div(m, BM), n_blocks = ceil_div(n, GLU ? BN / 2 : BN);
-  AXK_INSTANCE(INST_GEMM_TILE, BM, BN, WAVES_M, WAVES_N, GLU, STAGES);
+  if constexpr (KEEP) AXK_INSTANCE(INST_GEMM_KEPT, GLU);
+  else AXK_INSTANCE(INST_GEMM_TILE, BM, BN, WAVES_M, WAVES_N, GLU, STAGES);
   kernel<<<dim3(m_blocks * n_blocks, splits), WAVES_M * WAVES_N * 64, lds_bytes, stream>>>(
       x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode, m_blocks, n_blocks, after ? partial : nullptr, segs);
   AXK_LAUNCH_CHECK("gemm_tile");

@@ -30,6 +30,9 @@ enum {
   INST_CAUSAL_CONV,          // 1: runs of tokens, 0: a thread a (token, channel)
   INST_LATENT_PROMPT,        // tiles of 16 latent dims, chunks of 32 key dims, bounds known when compiled, sink
   INST_LATENT_TOKENS,        // tiles of 16 latent dims, chunks of 32 key dims, sink
+  INST_GEMM_KEPT,            // tiles of 128 x 128 that keep the sums of K's segments; gated
+  INST_ATTENTION_F32_PREFILL,    // float32 build, head_dim
+  INST_ATTENTION_F32_DECODE,     // float32 build, head_dim, waves a block
   INST_KINDS
 };
 

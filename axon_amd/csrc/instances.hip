@@ -16,7 +16,8 @@ namespace {
 const char* const KIND_NAMES[INST_KINDS] = {"gemm_fma", "gemm_tile", "gemm_stream", "gemm_normed", "gemm_rows",
                                             "gemm_split_reduce", "attention_rows", "attention_prefill",
                                             "attention_decode", "rmsnorm", "grouped_gemm", "causal_conv",
-                                            "latent_prompt", "latent_tokens"};
+                                            "latent_prompt", "latent_tokens", "gemm_kept", "attention_f32_prefill",
+                                            "attention_f32_decode"};
 
 struct Registry {
   std::mutex lock;

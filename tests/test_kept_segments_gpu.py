@@ -8,6 +8,10 @@ from axon_amd.kernels import MODE_ADD_F32, MODE_RELU_SQUARED, MODE_STORE, MODE_S
 pytestmark = pytest.mark.gpu
 
 
+def _kept(m, n, gated):
+    return -(-m // 128) * -(-n // (64 if gated else 128)) >= (144 if gated else 288)
+
+
 @pytest.mark.parametrize("mode", [MODE_STORE, MODE_ADD_F32, MODE_STORE_F32, MODE_SWIGLU, MODE_RELU_SQUARED])
 @pytest.mark.parametrize("M,N,K", [(2050, 2064, 512), (1153, 4100, 1088), (4100, 1106, 1600), (1200, 2944, 3072)])
 def test_rows_have_the_bits_they_have_alone(M, N, K, mode):
@@ -21,10 +25,15 @@ def test_rows_have_the_bits_they_have_alone(M, N, K, mode):
     bias = torch.randn(N, generator=g, device="cuda") if mode != MODE_SWIGLU else None
     base = torch.randn(M, N, generator=g, device="cuda").to(torch.float32 if mode in (MODE_ADD_F32, MODE_STORE_F32) else torch.bfloat16)
     whole = base.clone()
+    k.reset_instances()
     k.gemm(x, w, whole, bias, mode)
+    gated = mode == MODE_SWIGLU
+    assert (k.instances(launched=True) == [f"gemm_kept<{int(gated)}>"]) == _kept(M, N, gated)
     for first, m in ((0, 16), (M - 64, 64), (M // 2, 140), (3, 300)):
         part = base[first:first + m].clone()
+        k.reset_instances()
         k.gemm(x[first:first + m].contiguous(), w, part, bias, mode)
+        assert (f"gemm_kept<{int(gated)}>" in k.instances(launched=True)) == _kept(m, N, gated)
         assert torch.equal(part, whole[first:first + m]), (first, m)
 
 
@@ -36,7 +45,9 @@ def test_the_norm_behind(M, N, K):
     w = k.prepare_weight((torch.randn(N, K, generator=g, device="cuda") * 0.05).bfloat16())
     gain, rows = torch.randn(N, generator=g, device="cuda").bfloat16(), torch.randn(M, N, generator=g, device="cuda")
     out, normed = rows.clone(), torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+    k.reset_instances()
     k.gemm(x, w, out, None, MODE_ADD_F32, following_norm=(gain, normed, 1e-6))
+    assert {"gemm_kept<0>", "gemm_split_reduce<1>"} == set(k.instances(launched=True))
     plain = rows[:200].clone()
     k.gemm(x[:200].contiguous(), w, plain, None, MODE_ADD_F32)
     alone = torch.empty(200, N, dtype=torch.bfloat16, device="cuda")

@@ -214,6 +214,26 @@ def check_attention_mfma(nh, nkv, hd, page, T, window, every=1):
     return hit
 
 
+def check_attention_f32(nh, nkv, hd, page, T, window, last):
+    """The float32 build's prompt kernel over the whole sequence and its decoding kernel for the `last` tokens against the
+    plain formula, each with the bits of a wave a (token, head)."""
+    k = kernels("float32")
+    q, kc, vc, table, pos, rows, ref = _attention_case(nh, nkv, hd, page, T, window, "float32")
+    sizes = (nh, nkv, hd, page, window, 1.0 / math.sqrt(hd))
+    want = k.attention(q, nh * hd, kc, vc, table, pos, rows, torch.empty_like(q), *sizes)
+    tiles = torch.tensor([(a, min(128, T - a)) for a in range(0, T, 128)], dtype=torch.int32).cuda()
+    prompt = torch.full_like(q, float("nan"))
+    hit = launched(k, "float32", lambda: k.attention_prefill(q, nh * hd, kc, vc, table, pos, rows, prompt, tiles, *sizes))
+    assert torch.equal(prompt, want)
+    assert (prompt.cpu().double() - ref).abs().max() <= tol("float32", ref, 2e-6)
+    idx, chunks = torch.arange(T - last, T, dtype=torch.int32).cuda(), -(-T // k.attention_decode_chunk)
+    partial = torch.empty(k.attention_decode_workspace(last, nh, hd, chunks), dtype=torch.float32, device="cuda")
+    decoded = torch.full_like(q, float("nan"))
+    hit |= launched(k, "float32", lambda: k.attention_decode(q, nh * hd, kc, vc, table, pos, rows, decoded, idx, partial, chunks, *sizes))
+    assert torch.equal(decoded[T - last:], want[T - last:])
+    return hit
+
+
 def check_rmsnorm(dtype, dim):
     k = kernels(dtype)
     x = rnd(5, dim, seed=60, scale=3.0)
@@ -437,6 +457,12 @@ CASES = [
     (BF, ["gemm_tile<128,128,2,2,0,4>", "gemm_split_reduce<1>"], check_then_norm, (150, 256, 1024)),
     (BF, ["gemm_tile<256,256,4,2,1,2>"], check_gemm, (BF, 200, 18944, 3584, MODE_SWIGLU)),              # a 7B layer's at 200 rows
     (BF, ["gemm_tile<256,256,4,2,0,2>", "gemm_split_reduce<2>"], check_qkv_rope, (2048, 28, 4, 128, 3584, 64)),
+    # the segments of K in one block, plain, gated, and with the norm and the rotary store behind
+    (BF, ["gemm_kept<0>"], check_gemm, (BF, 2050, 2308, 512, MODE_STORE, True)),
+    (BF, ["gemm_kept<0>"], check_gemm, (BF, 1153, 4102, 1088, MODE_ADD_F32, True)),
+    (BF, ["gemm_kept<1>"], check_gemm, (BF, 1153, 1040, 1024, MODE_SWIGLU)),
+    (BF, ["gemm_kept<0>", "gemm_split_reduce<1>"], check_then_norm, (2049, 2304, 1024)),
+    (BF, ["gemm_kept<0>", "gemm_split_reduce<2>"], check_qkv_rope, (2050, 16, 2, 128, 2048, 64)),
     # grouped products: (matrix cores or 32-bit FMA, gated epilogue)
     (BF, ["grouped_gemm<4,0>"], check_grouped, (BF, 50, 3, 40, 64, False)),
     (BF, ["grouped_gemm<4,1>"], check_grouped, (BF, 19, 2, 72, 160, True)),
@@ -460,6 +486,11 @@ CASES = [
       for rt, qcs in ((32, (17, 18, 20)), (16, (9, 10, 12)), (8, (5, 6, 8)), (4, (3, 4, 6))) for qc in qcs for sink in (0, 1)],
     *[(BF, [f"latent_prompt<{rt},{qc},0,{sink}>", f"latent_tokens<{rt},{qc},{sink}>"], check_latent, (rank, rot, sink))
       for rt, qc, rank, rot in ((4, 4, 48, 16), (8, 8, 112, 48), (32, 20, 192, 64)) for sink in (0, 1)],
+    # the float32 build's attention on the matrix cores: (head size) and (head size, waves a block)
+    (F32, ["attention_f32_prefill<64>", "attention_f32_decode<64,1>"], check_attention_f32, (4, 2, 64, 16, 333, 90, 5)),
+    (F32, ["attention_f32_prefill<128>", "attention_f32_decode<128,1>"], check_attention_f32, (7, 1, 128, 64, 600, 0, 7)),
+    (F32, ["attention_f32_decode<64,4>"], check_attention_f32, (8, 4, 64, 16, 140, 0, 40)),
+    (F32, ["attention_f32_decode<128,4>"], check_attention_f32, (8, 4, 128, 32, 150, 60, 33)),
     # attention on the matrix cores: (head size, query heads a block, pages of 64 positions or more)
     # and (head size, waves a block) (one wave a block in the decoding kernel up to 2,560 blocks of
     # positions, four beyond; two heads a block in the prompt kernel where tiles x heads are more
