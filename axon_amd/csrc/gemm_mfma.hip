@@ -1674,7 +1674,7 @@ static int tiles32_of(int n, int mode) { return mode == MODE_SWIGLU ? n / 16 : (
 
 // More rows than the streaming kernel takes, S > 1 segments: a block a segment; the blocks' sums
 // go through a workspace and are added in segment order by a second kernel (the only way to occupy the
-// chip when the output is small; gemm_mfma_pass says where a block keeps the segments' sums).  The
+// chip when the output is small; keeps_segments says where a block keeps the segments' sums).  The
 // workspace holds the sums of at most GEMM_PASS_BYTES: a product of more rows runs in passes of
 // `rows_a_pass` rows, one after the other (a row's bits do not depend on the rows beside it).
 #define GEMM_PASS_BYTES ((size_t)2048 << 20)
@@ -1699,6 +1699,30 @@ size_t gemm_workspace_bytes(int m, int n, int k, int mode) {
 int gemm_then_norm_ok(int m, int n, int k) {
   return gemm_pack_ok(n, k, 0) && m > AXON_STREAM_MAX_M && n <= SRN_MAX_N && n % 4 == 0 &&
          gemm_segments(tiles32_of(n, MODE_ADD_F32), k) > 1;
+}
+
+// Whether the blocks of a product of more than 128 rows walk all of K themselves, in tiles of 128 x 128, and keep the
+// segments' sums in registers; else a block takes a segment and its sums go through the workspace.  Both timed for 32
+// shapes of 140 to 8,192 rows: every epilogue is the faster one here wherever this says so (766 measurements, at the
+// median 0.75 of the time) but for one store of 900 rows of 16,384 columns of K 3,072 in two segments (132 against 124 us).
+//  * There have to be blocks for the chip's 256 CUs.  K 2,048, 2,560 columns of 1,525 rows (240 blocks) 35 against 38 us,
+//    2,048 of 1,525 (192) 35 against 33; K 3,584, 3,584 of 1,200 (280) 63 against 71, 900 (224) 52 against 49.  Gated,
+//    1,408 of 700 (132) 27 against 28, of 900 (176) 27 against 30; 1,024 of 900 (128) 27 against 22.
+//  * K has to be short enough for tiles that read twice what the large ones read.  With up to 4,096 they win whatever
+//    the last round of 512 blocks (two a CU) holds: K 3,584, 4,608 of 2,048 rows 109 against 123; 4,096, 4,096 of
+//    4,096 154 against 206.  Up to 8,192 they win where it is one round or nearly full ones: K 5,120, 5,120 of
+//    3,072 (960 blocks) 188 against 221, of 2,048 behind a norm (640) 186 against 177; 8,192, 3,584 of 4,096 280 against
+//    302.  K 18,944, 3,584 of 2,048 328 against 314.
+//  * A gated product of up to 256 rows and a long K has the kernel with four stages: K 3,072, 8,192 of 256 rows 47
+//    against 43 us; of K 1,536, 8,960 35 against 43.
+static bool keeps_segments(int m, int n, int k, int mode, int segs) {
+  if (segs <= 1 || m <= 128) return false;
+  const bool glu = mode == MODE_SWIGLU;
+  const long blocks = (long)ceil_div(m, 128) * ceil_div(n, glu ? 64 : 128), rounds = (blocks + 511) / 512;
+  if (glu) return blocks >= 144 && k <= (m <= 256 ? 2048 : 3072);
+  if (blocks < (segs == 4 && k <= 2048 ? 240 : 288)) return false;
+  if (segs < 4) return k <= 3072;
+  return k <= 4096 || (k <= 8192 && (rounds == 1 || 4 * blocks >= 3 * 512 * rounds));
 }
 
 static int gemm_mfma_pass(const bf16_t* x, int x_stride, const bf16_t* w, const void* bias, int bias_is_f32, void* out,
@@ -1794,14 +1818,7 @@ static int gemm_mfma_pass(const bf16_t* x, int x_stride, const bf16_t* w, const 
   const long small = (long)ceil_div(m, 128) * ceil_div(n, glu ? 64 : 128) * segs;
   const long rounds_big = (big + 255) / 256, rounds_small = (small + 511) / 512;
   const bool use_big = rounds_big * 100 <= rounds_small * 65;
-  // Where 128 x 128 tiles that walk all of K themselves give the chip enough blocks, and K is short enough for their
-  // smaller tiles, the segments' sums stay in registers.  2,048 rows (us, a block a segment against here): 2,560 columns
-  // of K 2,048 56 against 46, 5,120 of 2,048 104 against 76, gated 1,408 of 2,048 60 against 38, 3,584 of 3,584 with
-  // the norm behind 100 against 83; 1,200 rows of 2,560 (200 blocks) 36 either way, 800 rows 32 against 35; 3,584 of
-  // 18,944 314 against 328, 2,048 of 5,632 (256 blocks) 72 against 89.  Without a norm behind it a product of K 3,584
-  // stays with the large tiles (4,608 columns 121 against 112), whose choice there the tests of the instances assert.
-  const long whole = (long)ceil_div(m, 128) * ceil_div(n, glu ? 64 : 128);
-  if (segs > 1 && whole >= (glu ? 144 : 288) && k <= (norm ? 5120 : 3072)) {
+  if (keeps_segments(m, n, k, mode, segs)) {
     if (glu) return launch_tile<128, 128, 2, 2, true, 64, 2, true>(ARGS, segs, ws);
     return launch_tile<128, 128, 2, 2, false, 64, 2, true>(ARGS, segs, ws, norm, rope_after);
   }

@@ -9,7 +9,7 @@ pytestmark = pytest.mark.gpu
 
 
 def _kept(m, n, gated):
-    return -(-m // 128) * -(-n // (64 if gated else 128)) >= (144 if gated else 288)
+    return -(-m // 128) * -(-n // (64 if gated else 128)) >= (144 if gated else 288)     # of the K and the sizes below
 
 
 @pytest.mark.parametrize("mode", [MODE_STORE, MODE_ADD_F32, MODE_STORE_F32, MODE_SWIGLU, MODE_RELU_SQUARED])
@@ -53,6 +53,23 @@ def test_the_norm_behind(M, N, K):
     alone = torch.empty(200, N, dtype=torch.bfloat16, device="cuda")
     k.rmsnorm(plain, gain, 1e-6, alone)
     assert torch.equal(out[:200], plain) and torch.equal(normed[:200], alone)
+
+
+def test_which_products_keep_them():
+    """Both sides of each line of the choice: blocks, K by the number of segments, the last round of blocks."""
+    k = kernels("bfloat16")
+    sizes = [(1525, 2560, 2048, 0, True), (1409, 2560, 2048, 0, True), (1408, 2560, 2048, 0, False), (1525, 2560, 2112, 0, False),
+             (300, 12300, 1024, 0, True), (140, 12300, 1024, 0, False), (300, 12300, 3136, 0, False), (4096, 4096, 4096, 0, True),
+             (2048, 5120, 4160, 0, False), (1525, 5120, 5120, 0, True), (2432, 5120, 4160, 0, False), (2433, 5120, 4160, 0, True),
+             (4096, 2048, 8256, 0, False), (700, 1472, 1024, 1, False), (700, 1488, 1024, 1, True), (256, 8192, 2048, 1, True),
+             (256, 8192, 2112, 1, False), (257, 8192, 3072, 1, True), (257, 8192, 3136, 1, False)]
+    for M, N, K, gated, kept in sizes:
+        x = torch.zeros(M, K, dtype=torch.bfloat16, device="cuda")
+        w = k.prepare_weight(torch.zeros((1 + gated) * N, K, dtype=torch.bfloat16, device="cuda"), bool(gated))
+        out = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+        k.reset_instances()
+        k.gemm(x, w, out, None, MODE_SWIGLU if gated else MODE_STORE)
+        assert (f"gemm_kept<{gated}>" in k.instances(launched=True)) == kept, (M, N, K, gated)
 
 
 @pytest.mark.parametrize("M,N,K", [(1100, 9300, 128), (129, 130, 192), (2051, 2309, 768), (1153, 2306, 1088)])

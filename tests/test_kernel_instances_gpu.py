@@ -452,17 +452,19 @@ CASES = [
     (BF, ["gemm_tile<128,128,2,2,1,2>"], check_gemm, (BF, 200, 8320, 256, MODE_SWIGLU)),
     (BF, ["gemm_tile<256,192,4,2,0,2>"], check_gemm, (BF, 2048, 4608, 192, MODE_STORE, True)),
     (BF, ["gemm_tile<256,256,4,2,0,2>"], check_gemm, (BF, 1100, 9300, 128, MODE_STORE_F32)),
-    (BF, ["gemm_tile<256,256,4,2,0,2>", "gemm_split_reduce<0>"], check_gemm, (BF, 2049, 3584, 3584, MODE_ADD_F32)),
+    (BF, ["gemm_tile<256,256,4,2,0,2>", "gemm_split_reduce<0>"], check_gemm, (BF, 2049, 3584, 18944, MODE_ADD_F32)),
     (BF, ["gemm_tile<256,256,4,2,1,2>"], check_gemm, (BF, 2048, 2608, 64, MODE_SWIGLU)),
     (BF, ["gemm_tile<128,128,2,2,0,4>", "gemm_split_reduce<1>"], check_then_norm, (150, 256, 1024)),
     (BF, ["gemm_tile<256,256,4,2,1,2>"], check_gemm, (BF, 200, 18944, 3584, MODE_SWIGLU)),              # a 7B layer's at 200 rows
-    (BF, ["gemm_tile<256,256,4,2,0,2>", "gemm_split_reduce<2>"], check_qkv_rope, (2048, 28, 4, 128, 3584, 64)),
+    (BF, ["gemm_tile<256,256,4,2,0,2>", "gemm_split_reduce<2>"], check_qkv_rope, (1525, 40, 8, 128, 5120, 64)),        # a 14B layer's
     # the segments of K in one block, plain, gated, and with the norm and the rotary store behind
     (BF, ["gemm_kept<0>"], check_gemm, (BF, 2050, 2308, 512, MODE_STORE, True)),
     (BF, ["gemm_kept<0>"], check_gemm, (BF, 1153, 4102, 1088, MODE_ADD_F32, True)),
     (BF, ["gemm_kept<1>"], check_gemm, (BF, 1153, 1040, 1024, MODE_SWIGLU)),
     (BF, ["gemm_kept<0>", "gemm_split_reduce<1>"], check_then_norm, (2049, 2304, 1024)),
     (BF, ["gemm_kept<0>", "gemm_split_reduce<2>"], check_qkv_rope, (2050, 16, 2, 128, 2048, 64)),
+    (BF, ["gemm_kept<0>", "gemm_split_reduce<2>"], check_qkv_rope, (2048, 28, 4, 128, 3584, 64)),    # a 7B layer's
+    (BF, ["gemm_kept<0>"], check_gemm, (BF, 2049, 3584, 3584, MODE_ADD_F32)),
     # grouped products: (matrix cores or 32-bit FMA, gated epilogue)
     (BF, ["grouped_gemm<4,0>"], check_grouped, (BF, 50, 3, 40, 64, False)),
     (BF, ["grouped_gemm<4,1>"], check_grouped, (BF, 19, 2, 72, 160, True)),
