@@ -1679,28 +1679,6 @@ static int tiles32_of(int n, int mode) { return mode == MODE_SWIGLU ? n / 16 : (
 // `rows_a_pass` rows, one after the other (a row's bits do not depend on the rows beside it).
 #define GEMM_PASS_BYTES ((size_t)2048 << 20)
 
-static int rows_a_pass(int n, int mode, int segs) {
-  const size_t row_bytes = (size_t)segs * (mode == MODE_SWIGLU ? 2 : 1) * n * sizeof(float);
-  const size_t rows = GEMM_PASS_BYTES / row_bytes / 256 * 256;       // whole tiles of 256 rows
-  return (int)(rows < 256 ? 256 : rows > (1u << 30) ? (1u << 30) : rows);
-}
-
-size_t gemm_workspace_bytes(int m, int n, int k, int mode) {
-  if (k % 64 != 0 || m <= AXON_STREAM_MAX_M) return 0;
-  const int s = gemm_segments(tiles32_of(n, mode), k);
-  if (s <= 1) return 0;
-  const int rows = m < rows_a_pass(n, mode, s) ? m : rows_a_pass(n, mode, s);
-  return (size_t)s * (mode == MODE_SWIGLU ? 2 : 1) * rows * n * sizeof(float);
-}
-
-// Whether the product that adds into the rows runs with a block a segment, so that the kernel that
-// adds the segments' sums can also norm the finished rows (gemm_split_reduce_norm_kernel: rows of
-// up to SRN_MAX_N columns, in whole float4).
-int gemm_then_norm_ok(int m, int n, int k) {
-  return gemm_pack_ok(n, k, 0) && m > AXON_STREAM_MAX_M && n <= SRN_MAX_N && n % 4 == 0 &&
-         gemm_segments(tiles32_of(n, MODE_ADD_F32), k) > 1;
-}
-
 // Whether the blocks of a product of more than 128 rows walk all of K themselves, in tiles of 128 x 128, and keep the
 // segments' sums in registers; else a block takes a segment and its sums go through the workspace.  Both timed for 32
 // shapes of 140 to 8,192 rows: every epilogue is the faster one here wherever this says so (766 measurements, at the
@@ -1725,9 +1703,37 @@ static bool keeps_segments(int m, int n, int k, int mode, int segs) {
   return k <= 4096 || (k <= 8192 && (rounds == 1 || 4 * blocks >= 3 * 512 * rounds));
 }
 
+// How many sets of M x N sums go through the workspace: one a segment (twice for the gated product), none where
+// blocks keep them, but one for the modes behind which a norm or a rotary store may follow.
+static int sum_planes(int m, int n, int k, int mode, int segs) {
+  if (segs <= 1) return 0;
+  if (keeps_segments(m, n, k, mode, segs)) return mode == MODE_STORE || mode == MODE_ADD_F32 ? 1 : 0;
+  return segs * (mode == MODE_SWIGLU ? 2 : 1);
+}
+
+static int rows_a_pass(int n, int planes) {
+  if (planes == 0) return 1 << 30;
+  const size_t rows = GEMM_PASS_BYTES / ((size_t)planes * n * sizeof(float)) / 256 * 256;       // whole tiles of 256 rows
+  return (int)(rows < 256 ? 256 : rows > (1u << 30) ? (1u << 30) : rows);
+}
+
+size_t gemm_workspace_bytes(int m, int n, int k, int mode) {
+  if (k % 64 != 0 || m <= AXON_STREAM_MAX_M) return 0;
+  const int planes = sum_planes(m, n, k, mode, gemm_segments(tiles32_of(n, mode), k)), pass = rows_a_pass(n, planes);
+  return (size_t)planes * (m < pass ? m : pass) * n * sizeof(float);
+}
+
+// Whether the product that adds into the rows runs with a block a segment, so that the kernel that
+// adds the segments' sums can also norm the finished rows (gemm_split_reduce_norm_kernel: rows of
+// up to SRN_MAX_N columns, in whole float4).
+int gemm_then_norm_ok(int m, int n, int k) {
+  return gemm_pack_ok(n, k, 0) && m > AXON_STREAM_MAX_M && n <= SRN_MAX_N && n % 4 == 0 &&
+         gemm_segments(tiles32_of(n, MODE_ADD_F32), k) > 1;
+}
+
 static int gemm_mfma_pass(const bf16_t* x, int x_stride, const bf16_t* w, const void* bias, int bias_is_f32, void* out,
-                          int out_stride, int m, int n, int k, int mode, hipStream_t stream, int segs, const SplitNorm* norm,
-                          float* ws, const RopeStore* rope_after);
+                          int out_stride, int m, int n, int k, int mode, hipStream_t stream, int segs, bool keep,
+                          const SplitNorm* norm, float* ws, const RopeStore* rope_after);
 
 static int gemm_mfma_dispatch(const bf16_t* x, int x_stride, const bf16_t* w, const void* bias, int bias_is_f32, void* out,
                               int out_stride, int m, int n, int k, int mode, hipStream_t stream,
@@ -1763,9 +1769,11 @@ static int gemm_mfma_dispatch(const bf16_t* x, int x_stride, const bf16_t* w, co
                   workspace_bytes);
     return -1;
   }
-  const int pass = segs > 1 ? rows_a_pass(n, mode, segs) : m;
+  // what the whole product takes, its passes take: the workspace is of that size
+  const bool keep = keeps_segments(m, n, k, mode, segs);
+  const int pass = rows_a_pass(n, sum_planes(m, n, k, mode, segs));
   if (m <= pass)
-    return gemm_mfma_pass(x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode, stream, segs, norm,
+    return gemm_mfma_pass(x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode, stream, segs, keep, norm,
                           (float*)workspace, rope_after);
   // in passes: every operand that has a row per row of X moves on with it
   const size_t out_elem = mode_stores_elem(mode) || mode == MODE_SWIGLU ? sizeof(bf16_t) : sizeof(float);
@@ -1785,25 +1793,25 @@ static int gemm_mfma_dispatch(const bf16_t* x, int x_stride, const bf16_t* w, co
     }
     const int rc = gemm_mfma_pass(x + (size_t)m0 * x_stride, x_stride, w, bias, bias_is_f32,
                                   (char*)out + (size_t)m0 * out_stride * out_elem, out_stride, rows, n, k, mode, stream, segs,
-                                  norm ? &norm_at : nullptr, (float*)workspace, rope_after ? &rope_at : nullptr);
+                                  keep, norm ? &norm_at : nullptr, (float*)workspace, rope_after ? &rope_at : nullptr);
     if (rc != 0) return rc;
   }
   return 0;
 }
 
-// One pass: more than AXON_STREAM_MAX_M rows whose segments' sums (if S > 1) fit the workspace.
+// One pass: more than AXON_STREAM_MAX_M rows whose sums (if any go through it) fit the workspace.
 static int gemm_mfma_pass(const bf16_t* x, int x_stride, const bf16_t* w, const void* bias, int bias_is_f32, void* out,
-                          int out_stride, int m, int n, int k, int mode, hipStream_t stream, int segs, const SplitNorm* norm,
-                          float* ws, const RopeStore* rope_after) {
+                          int out_stride, int m, int n, int k, int mode, hipStream_t stream, int segs, bool keep,
+                          const SplitNorm* norm, float* ws, const RopeStore* rope_after) {
 #define ARGS x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode, stream
   const bool glu = mode == MODE_SWIGLU;
-  if (m <= 64) {
+  if (m <= 64 && !keep) {
     // W streamed, X shared through LDS; a block a segment.  Two row tiles a wave where the matrix is large.
     if (glu) return launch_rows<2, 4, EPI_GLU>(ARGS, segs, ws, nullptr, nullptr);
     if (n >= 32 * 512) return launch_rows<2, 4, EPI_PLAIN>(ARGS, segs, ws, norm, rope_after);
     return launch_rows<1, 4, EPI_PLAIN>(ARGS, segs, ws, norm, rope_after);
   }
-  if (m <= 128) {
+  if (m <= 128 && !keep) {
     // the same with 128 rows of X a step: still bound by reading W (a tile kernel's blocks are too few here)
     if (glu) return launch_rows<2, 8, EPI_GLU>(ARGS, segs, ws, nullptr, nullptr);
     if (n >= 32 * 512) return launch_rows<2, 8, EPI_PLAIN>(ARGS, segs, ws, norm, rope_after);
@@ -1818,7 +1826,7 @@ static int gemm_mfma_pass(const bf16_t* x, int x_stride, const bf16_t* w, const 
   const long small = (long)ceil_div(m, 128) * ceil_div(n, glu ? 64 : 128) * segs;
   const long rounds_big = (big + 255) / 256, rounds_small = (small + 511) / 512;
   const bool use_big = rounds_big * 100 <= rounds_small * 65;
-  if (keeps_segments(m, n, k, mode, segs)) {
+  if (keep) {
     if (glu) return launch_tile<128, 128, 2, 2, true, 64, 2, true>(ARGS, segs, ws);
     return launch_tile<128, 128, 2, 2, false, 64, 2, true>(ARGS, segs, ws, norm, rope_after);
   }

@@ -91,3 +91,31 @@ def test_sums_added_into_rows(M, N, K):
     # a chain of K products and a bias, each sum off by at most a unit of what it holds
     bound = (K + 1) * 2.0 ** -23 * (x.double().abs() @ w.double().abs().T + bias.double().abs())
     assert bool(((prod.double() - want).abs() <= bound).all())
+
+
+def test_what_goes_through_memory():
+    """A product that keeps its sums asks for no more than what a norm or a rotary store behind it reads."""
+    need = kernels("bfloat16").lib.axk_gemm_workspace
+    assert need(8192, 5120, 2048, MODE_STORE) == need(8192, 5120, 2048, MODE_ADD_F32) == 8192 * 5120 * 4
+    assert need(8192, 5120, 2048, MODE_STORE_F32) == need(8192, 5120, 2048, MODE_RELU_SQUARED) == 0
+    assert need(2048, 5632, 2048, MODE_SWIGLU) == 0 and need(2048, 3584, 18944, MODE_STORE) == 4 * 2048 * 3584 * 4
+    assert need(200, 5632, 4096, MODE_SWIGLU) == 4 * 2 * 200 * 5632 * 4 and need(2048, 30000, 2048, MODE_STORE) == 0
+
+
+def test_passes_of_a_product_that_keeps_them():
+    """More rows than the workspace holds sums of (2 GiB): a second pass of a few rows, with the norm behind."""
+    k, N, K = kernels("bfloat16"), 5120, 512
+    first = (2 << 30) // (N * 4) // 256 * 256
+    M = first + 70
+    assert k.lib.axk_gemm_workspace(M, N, K, MODE_ADD_F32) == first * N * 4
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x = torch.randn(M, K, generator=g, device="cuda").bfloat16()
+    w = k.prepare_weight((torch.randn(N, K, generator=g, device="cuda") * 0.1).bfloat16())
+    gain, out = torch.randn(N, generator=g, device="cuda").bfloat16(), torch.zeros(M, N, device="cuda")
+    normed = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+    k.gemm(x, w, out, None, MODE_ADD_F32, following_norm=(gain, normed, 1e-6))
+    for at, m in ((0, 100), (first - 60, 130), (first, 70), (M - 9, 9)):
+        part, alone = torch.zeros(m, N, device="cuda"), torch.empty(m, N, dtype=torch.bfloat16, device="cuda")
+        k.gemm(x[at:at + m].contiguous(), w, part, None, MODE_ADD_F32)
+        k.rmsnorm(part, gain, 1e-6, alone)
+        assert torch.equal(out[at:at + m], part) and torch.equal(normed[at:at + m], alone), at
