@@ -27,10 +27,15 @@ def _ptr(t: Optional[torch.Tensor]) -> c_void_p:
     return c_void_p(0 if t is None else t.data_ptr())
 
 
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream() -> c_void_p:
-    # what torch.cuda.current_stream().cuda_stream says, without the object made on the way: about 2.6 us a launch
-    # (a prompt of 3 tokens through the smoke run's model, 22 launches: 398 -> 339 us)
-    return c_void_p(torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()))
+    # torch.cuda.current_stream().cuda_stream, where torch has it without the object made on the way: about 2.6 us a
+    # launch (a prompt of 3 tokens through the smoke run's model, 22 launches: 398 -> 339 us)
+    if _raw_stream is None:
+        return c_void_p(torch.cuda.current_stream().cuda_stream)
+    return c_void_p(_raw_stream(torch._C._cuda_getDevice()))
 
 
 # for the callers of `Kernels.call`: a tensor's (or a packed matrix's) address, the current stream
