@@ -24,31 +24,8 @@
 
 #if !AXON_BF16
 
-typedef __attribute__((ext_vector_type(4))) float f32x4;
-
 #define F32_STEP(acc, a, b, j) acc = __builtin_amdgcn_mfma_f32_16x16x4f32((a)[j], (b)[j], acc, 0, 0, 0)
 #define F32_ZERO (f32x4{0.0f, 0.0f, 0.0f, 0.0f})
-
-// Lanes l, l + 16, l + 32, l + 48 hold k = 4 q + j in register j; afterwards k = 4 j + q.
-__device__ __forceinline__ f32x4 f32_operand(f32x4 v) {
-  unsigned r[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) r[j] = __float_as_uint(v[j]);
-#pragma unroll
-  for (int j = 0; j < 4; j += 2) {
-    const auto s = __builtin_amdgcn_permlane16_swap(r[j], r[j + 1], false, false);
-    r[j] = s[0];
-    r[j + 1] = s[1];
-  }
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const auto s = __builtin_amdgcn_permlane32_swap(r[j], r[j + 2], false, false);
-    r[j] = s[0];
-    r[j + 2] = s[1];
-  }
-  return f32x4{__builtin_bit_cast(float, r[0]), __builtin_bit_cast(float, r[1]), __builtin_bit_cast(float, r[2]),
-               __builtin_bit_cast(float, r[3])};
-}
 
 // A block's raw scores (tile t, register e: position p0 + 16 t + 4 q + e of the lane's column) to weights;
 // m_b and l_b in every lane of the column.

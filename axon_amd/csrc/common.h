@@ -165,6 +165,30 @@ __device__ inline void wait_lgkmcnt() {
 }
 
 typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+
+// Operands of v_mfma_f32_16x16x4_f32: lanes l, l + 16, l + 32, l + 48 hold k = 4 q + j of a row in v[j]; afterwards
+// k = 4 j + q in register j, a product's operand for each j.
+template <typename V>
+__device__ __forceinline__ f32x4 f32_operand(const V& v) {
+  unsigned r[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) r[j] = __float_as_uint(v[j]);
+#pragma unroll
+  for (int j = 0; j < 4; j += 2) {
+    const auto s = __builtin_amdgcn_permlane16_swap(r[j], r[j + 1], false, false);
+    r[j] = s[0];
+    r[j + 1] = s[1];
+  }
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const auto s = __builtin_amdgcn_permlane32_swap(r[j], r[j + 2], false, false);
+    r[j] = s[0];
+    r[j + 2] = s[1];
+  }
+  return f32x4{__builtin_bit_cast(float, r[0]), __builtin_bit_cast(float, r[1]), __builtin_bit_cast(float, r[2]),
+               __builtin_bit_cast(float, r[3])};
+}
 
 // 16 bytes a lane from LDS byte address `lds_address` + OFFSET.
 template <int OFFSET>

@@ -16,7 +16,6 @@
 #include "instances.h"
 
 #define FMA_PART 32    // k of one chain
-typedef __attribute__((ext_vector_type(4))) float f32x4;
 
 #define FMA_STEP(acc, a, b, j) acc = __builtin_amdgcn_mfma_f32_16x16x4f32((a)[j], (b)[j], acc, 0, 0, 0)
 
@@ -156,28 +155,6 @@ gemm_fma_kernel(const elem_t* __restrict__ x, int x_stride, const elem_t* __rest
       }
 }
 
-// Four lanes l, l + 16, l + 32, l + 48 hold k = 4 q + j of a row in register j: after this they hold
-// k = 4 j + q, a product's operand for each j.
-__device__ inline f32x4 fma_operand(const float (&v)[4]) {
-  unsigned r[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) r[j] = __float_as_uint(v[j]);
-#pragma unroll
-  for (int j = 0; j < 4; j += 2) {
-    const auto s = __builtin_amdgcn_permlane16_swap(r[j], r[j + 1], false, false);
-    r[j] = s[0];
-    r[j + 1] = s[1];
-  }
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const auto s = __builtin_amdgcn_permlane32_swap(r[j], r[j + 2], false, false);
-    r[j] = s[0];
-    r[j + 2] = s[1];
-  }
-  return f32x4{__builtin_bit_cast(float, r[0]), __builtin_bit_cast(float, r[1]), __builtin_bit_cast(float, r[2]),
-               __builtin_bit_cast(float, r[3])};
-}
-
 // Few rows (decoding): such a product only waits for W, so a block takes NR (16 or 8) columns and the
 // chains of an output, which do not need each other, are shared out over its 8 waves: every wave
 // streams its chains' W from memory straight into operands, leaves the chains' sums in LDS, and a thread
@@ -227,7 +204,7 @@ gemm_fma_few_rows_kernel(const elem_t* __restrict__ x, int x_stride, const elem_
 #pragma unroll
         for (int g = 0; g < 2; ++g) {
           if (k0 + FMA_PART > K) fma_clear(wv[t][p][g], k0 + 16 * g + 4 * q, K);
-          a[t][g] = fma_operand(wv[t][p][g]);
+          a[t][g] = f32_operand(wv[t][p][g]);
         }
 #pragma unroll
       for (int i = 0; i < MT; ++i) {
@@ -237,7 +214,7 @@ gemm_fma_few_rows_kernel(const elem_t* __restrict__ x, int x_stride, const elem_
           float xv[4];
           fma_load<VEC>(x_row[i], k0 + 16 * g + 4 * q, K, xv);
           if (k0 + FMA_PART > K) fma_clear(xv, k0 + 16 * g + 4 * q, K);
-          b[g] = fma_operand(xv);
+          b[g] = f32_operand(xv);
         }
 #pragma unroll
         for (int t = 0; t < NT; ++t) {

@@ -50,7 +50,6 @@
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
-typedef __attribute__((ext_vector_type(4))) float f32x4;
 
 __device__ inline bf16x8 as_frag(uint4 v) {
   union { uint4 u; bf16x8 f; } c;
