@@ -10,8 +10,9 @@
 // ONE ORDER OF ADDITION PER MATRIX.  Every output element of a product with a given W is
 //     ((c_0 + c_1) + c_2) + ... + c_(S-1),   then the bias and the epilogue,
 // where K is cut into S = gemm_segments(W's row tiles, K) contiguous segments (by the matrix
-// alone, never by the number of rows M of X), and c_s is one chain of 32x32x16 MFMAs over
-// the segment's k in ascending steps of 16, starting from zero.  Every kernel below computes
+// alone, never by the number of rows M of X), and c_s is one chain of 16x16x32 MFMAs over
+// the segment's k in ascending steps of 32, starting from zero (each gives the bits of two
+// 32x32x16 MFMAs over the same k).  Every kernel below computes
 // exactly this, whatever its tiles, its number of waves or the way it spreads the segments over
 // waves, blocks or registers: a row of X gives the same bits whether it comes alone, among 16
 // rows or among 4,096 (src/lm.rs:272-278 asks this of a step; the reference's integer products
@@ -19,9 +20,8 @@
 // speed alone:
 //
 // * gemm_stream (M <= 16): bound by reading W once.  A wave owns one or two tiles of 16 rows of W
-//   and one segment of K and streams its share from memory straight into 16x16x32 MFMA operands
-//   (one such MFMA gives the bits of two chained 32x32x16 ones over the same k), keeping a ring
-//   of steps in flight; W is the A operand, the rows of X the B operand.  The waves of a block
+//   and one segment of K and streams its share from memory straight into MFMA operands, keeping
+//   a ring of steps in flight; W is the A operand, the rows of X the B operand.  The waves of a block
 //   are the segments of its tiles; their sums are added in segment order through LDS.
 //   Epilogues: bias / residual add / SwiGLU, and the attention's qkv product with the rotary
 //   encoding and the store into the paged cache.
@@ -35,9 +35,8 @@
 //   through a workspace.
 //
 // * gemm_tile (M > 128): a block of 4 or 8 waves owns a BM x BN tile of the output, walks K in
-//   steps of 64 through LDS stages filled by direct global -> LDS loads (the next step's loads
-//   in flight while this one multiplies), and each wave keeps a tile of 32x32x16 MFMA
-//   accumulators.  With S > 1 segments each goes to blocks of its own (gridDim.y = S), whose sums
+//   steps of 32 through LDS stages filled by direct global -> LDS loads (the next steps' loads
+//   in flight while this one multiplies), and each wave keeps a tile of MFMA accumulators.  With S > 1 segments each goes to blocks of its own (gridDim.y = S), whose sums
 //   go through a workspace and are added in segment order by gemm_split_reduce, which also
 //   applies the epilogue.  X rows land in LDS with their 16-byte slots permuted so that fragment reads of
 //   neighbouring rows fall into different banks; W blocks land as they are.  Blocks are numbered
@@ -49,7 +48,6 @@
 #if AXON_BF16
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
-typedef __attribute__((ext_vector_type(16))) float f32x16;
 
 __device__ inline bf16x8 as_frag(uint4 v) {
   union { uint4 u; bf16x8 f; } c;
@@ -62,19 +60,47 @@ typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
 __device__ inline bf16x8 as_frag(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
 
+// A number that the type carries (a loop is written once for each of its values).
+template <int V>
+struct Number {
+  static constexpr int value = V;
+};
+
+// Waits until at most min(rounds, MAX) rounds of LOADS loads each are in flight.
+template <int MAX, int LOADS>
+__device__ inline void wait_rounds(int rounds) {
+  if constexpr (MAX <= 0) {
+    wait_vmcnt<0>();
+  } else {
+    if (rounds >= MAX) wait_vmcnt<MAX * LOADS>();
+    else wait_rounds<MAX - 1, LOADS>(rounds);
+  }
+}
+
 // ---------------------------------------------------------------------------- gemm_tile
-// LDS holds STAGES stages; a stage is BM rows of X and the BN / 16 x BK / 32 packed blocks of W,
-// written by direct global -> LDS loads of 16 bytes per lane (a wave instruction fills 1024
-// bytes: 8 rows of X, or one block of W).  Every stage is filled before the loop, and the loads
-// of step kt + STAGES go out as soon as step kt's stage is free, so the latency of L2 and of
-// the path into LDS is covered by STAGES - 1 steps of MFMAs.
+// LDS holds STAGES stages; a stage is 32 k: BM rows of X (64 bytes each) and the BN / 16 packed
+// blocks of W, written by direct global -> LDS loads of 16 bytes per lane (a wave instruction
+// fills 1024 bytes: 16 rows of X, or one block of W).  STAGES - 1 stages are under way, so the
+// latency of L2 and of the path into LDS is covered by as many blocks of products.
 //
-// A row of X in a stage is BK / 8 slots of 16 bytes, permuted so that fragment reads of
-// neighbouring rows at one k chunk fall into different banks without padding (which direct
-// loads could not skip).  LDS serves 256 bytes a cycle (64 banks): a 16-byte read of 16 consecutive lanes
-// (16 consecutive rows, the same k chunk) is conflict-free when the rows' 16-byte positions
-// modulo 256 differ.  With 128-byte rows (BK 64) that is slot = chunk ^ ((row >> 1) & 7); with
-// 64-byte rows (BK 32) slot = chunk ^ ((row >> 2) & 3).
+// A row of X in a stage is 4 slots of 16 bytes, permuted (slot = k chunk ^ (row / 4 % 4)) so that
+// fragment reads of 16 neighbouring rows at one k chunk fall into different banks without padding
+// (which direct loads could not skip): LDS serves 256 bytes a cycle (64 banks), and the 16
+// 16-byte positions are then distinct modulo 256.
+//
+// What bounds it, and why it is made so.  With every CU at work the card holds its power, not its
+// clock: 1.6 to 1.9 GHz instead of 2.4, so a product's energy counts like its cycles.
+//  * 16x16x32 MFMAs instead of pairs of 32x32x16 (the same bits): products alone, on operands in
+//    registers, run at 2.01 against 1.79 PFLOP/s (random values; 2.44 and 2.47 on zeros), since
+//    the sums are read and written once for 32 k instead of 16.
+//  * Loads and LDS reads go out one at a time between products.  A burst of a stage's loads held
+//    the wave at their issue until the path into LDS (some 59 bytes a cycle) had taken them: a
+//    block of 256 x 256 x 64 took 3,300 cycles of which 2,048 are products; loads spread 3,020,
+//    reads spread too 2,900.
+// [gate; up] of 8,192 rows (18,944 columns of K 3,584) 2,040 -> 1,803 us (1.23 PFLOP/s), of 2,048 rows 613 ->
+// 547; 3,584 columns of K 18,944 at 2,048 rows (with the sums' kernel) 381 -> 340; 2,048^3 38 -> 32 us, 1,500 rows
+// of 33,000 columns of K 1,024 208 -> 156 (four columns a store).  Slower: waves of 128 x 64 (573 against 547
+// us); four waves of 128 x 128 do not fit the registers beside their fragments.
 //
 // GLU: W holds 2 N rows (gate rows, then up rows) and the output is silu(gate) * up, N wide.
 // A block then owns BN / 2 output columns; each wave's share of the LDS tile holds the gate
@@ -83,27 +109,24 @@ __device__ inline bf16x8 as_frag(u32x4 v) { return __builtin_bit_cast(bf16x8, v)
 //
 // KEEP: the block walks all `splits` segments of K itself; a segment's chains are added to the sums of those
 // before it in a second set of registers (the order of gemm_split_reduce), and no sums go through memory.
-template <int BM, int BN, int WAVES_M, int WAVES_N, bool GLU, int BK, int STAGES, bool KEEP>
-__global__ void __launch_bounds__(WAVES_M * WAVES_N * 64, KEEP ? 2 : 1)
+template <int BM, int BN, int WAVES_M, int WAVES_N, bool GLU, int STAGES, bool KEEP>
+__global__ void __launch_bounds__(WAVES_M * WAVES_N * 64, KEEP || STAGES * (BM + BN) * 64 <= 80 * 1024 ? 2 : 1)
 gemm_tile_kernel(const bf16_t* __restrict__ x, int x_stride, const bf16_t* __restrict__ w, const void* __restrict__ bias,
                  int bias_is_f32, void* __restrict__ out, int out_stride, int M, int N, int K, int mode, int m_blocks,
                  int n_blocks, float* __restrict__ partial, int splits) {
   extern __shared__ __align__(16) unsigned char smem[];
-  static_assert(BK == 64 || BK == 32, "segments of K are counted in steps of 64: whole K tiles");
-  constexpr int PER64 = 64 / BK;                       // K tiles in a step of 64
   constexpr int NW = WAVES_M * WAVES_N;
   constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N;  // a wave's tile
-  constexpr int TM = WM / 32, TN = WN / 32;            // in 32 x 32 MFMA tiles
-  constexpr int ROW = BK * 2;                          // bytes of a row
-  constexpr int SLOTS = BK / 8;                        // 16-byte slots of a row
-  constexpr int RPI = 1024 / ROW;                      // rows one wave instruction fills
-  constexpr int KBT = BK / 32;                         // packed k blocks of a K tile
-  constexpr int XQ = BM / RPI / NW, WQ = BN / 16 * KBT / NW;  // load instructions per wave and stage
+  constexpr int TM = WM / 16, TN = WN / 16;            // in 16 x 16 MFMA tiles
+  constexpr int TH = TN / 2;                           // tiles of W read at a time
+  constexpr int ROW = 64;                              // bytes of a row: 32 k
+  constexpr int XQ = BM / 16 / NW;                     // load instructions of X per wave and stage: 16 rows each
+  constexpr int WC = BN / 16, WQ = (WC + NW - 1) / NW; // blocks of W in a stage; load instructions per wave
+  constexpr int LOADS = XQ + WQ;
   constexpr int STAGE = (BM + BN) * ROW;               // bytes per stage
-  static_assert(XQ >= 1 && WQ >= 1 && (STAGES - 2) * (XQ + WQ) < 64, "tile too small or too many loads in flight");
-  static_assert(BN / 16 * KBT % NW == 0 && WN % 32 == 0, "the 1 KB chunks of W are shared out evenly");
-  static_assert(!GLU || TN % 2 == 0, "a wave's gate columns and up columns are whole MFMA tiles");
-#define SWZ(row) (BK == 64 ? (((row) >> 1) & 7) : (((row) >> 2) & 3))
+  constexpr int AHEAD = STAGES - 1;                    // stages whose loads are under way
+  static_assert(XQ >= 1 && BM % (16 * NW) == 0 && (STAGES - 2) * LOADS < 64, "tile too small or too many loads in flight");
+  static_assert(WN % 32 == 0 && AHEAD % 2 == 0, "halves of a wave's W tiles; the loop takes two stages a turn");
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave / WAVES_N, wn = wave % WAVES_N;
@@ -141,24 +164,22 @@ gemm_tile_kernel(const bf16_t* __restrict__ x, int x_stride, const bf16_t* __res
   }
   const int m0 = mb * BM, n0 = nb * (GLU ? BN / 2 : BN);
 
-  // what this lane fetches: row r = (q * NW + wave) * RPI + lane / SLOTS of a tile; it fills slot
-  // lane % SLOTS of that row, which holds k chunk (lane % SLOTS) ^ SWZ(r)
-  const int lrow = lane / SLOTS, lslot = lane % SLOTS;
+  // what this lane fetches: row r = (q * NW + wave) * 16 + lane / 4 of a tile; it fills slot
+  // lane % 4 of that row, which holds k chunk (lane % 4) ^ (r / 4 % 4)
   unsigned xoff[XQ], woff[WQ];
 #pragma unroll
   for (int q = 0; q < XQ; ++q) {
-    const int r = (q * NW + wave) * RPI + lrow;
-    xoff[q] = (unsigned)min(m0 + r, M - 1) * (unsigned)x_stride + (lslot ^ SWZ(r)) * 8;
+    const int r = (q * NW + wave) * 16 + (lane >> 2);
+    xoff[q] = (unsigned)min(m0 + r, M - 1) * (unsigned)x_stride + ((lane & 3) ^ ((r >> 2) & 3)) * 8;
   }
-  // W: chunk c = q * NW + wave of a stage is the packed block (row tile c / KBT, k block c % KBT)
-  // of the tile, 1 KB as it lies in memory.  Row tiles past the matrix: its last one (the
-  // epilogue drops those columns).
+  // W: chunk c = (q * NW + wave) % WC of a stage is the packed block (row tile c, the stage's k block) of the tile, 1 KB
+  // as it lies in memory (where the waves do not divide the chunks, some twice: the same bytes to the same place).
+  // Row tiles past the matrix: its last one (the epilogue drops those columns).
   const int KB = K / 32;
   const int row_tiles = GLU ? N / 16 : (N + 15) / 16;          // GLU: per half, N a multiple of 16
 #pragma unroll
   for (int q = 0; q < WQ; ++q) {
-    const int c = q * NW + wave;
-    const int r = (c / KBT) * 16;                               // first row of the chunk in the LDS tile
+    const int r = (q * NW + wave) % WC * 16;                    // first row of the chunk in the LDS tile
     int tile;
     if (GLU) {
       const int owner = r / WN, within = r % WN;                // the wave whose columns these are
@@ -167,198 +188,254 @@ gemm_tile_kernel(const bf16_t* __restrict__ x, int x_stride, const bf16_t* __res
     } else {
       tile = min((n0 + r) / 16, row_tiles - 1);
     }
-    woff[q] = ((unsigned)tile * (unsigned)KB + (c % KBT)) * 512 + lane * 8;
+    woff[q] = (unsigned)tile * (unsigned)KB * 512 + lane * 8;
   }
 
-  // Split K (gridDim.y > 1): this block multiplies the K tiles kt_begin .. kt_begin + nk - 1 and
+  // Split K (gridDim.y > 1): this block multiplies the k blocks kt_begin .. kt_begin + nk - 1 and
   // leaves its sums in `partial`; gemm_split_reduce_kernel adds the blocks' sums in block order.
-  const int kt_begin = KEEP ? 0 : (int)((long)blockIdx.y * (K / 64) / gridDim.y) * PER64;
-  const int nk = KEEP ? K / 64 * PER64 : (int)((long)(blockIdx.y + 1) * (K / 64) / gridDim.y) * PER64 - kt_begin;
-  auto issue = [&](int kt) {     // kt counts from kt_begin
-    unsigned char* stage = smem + (kt % STAGES) * STAGE;
-    const int koff = (kt_begin + kt) * BK;
-#pragma unroll
-    for (int q = 0; q < XQ; ++q)
-      __builtin_amdgcn_global_load_lds((global_ptr_t)(x + xoff[q] + koff), (lds_ptr_t)(stage + (q * NW + wave) * 1024), 16,
-                                       0, 0);
-#pragma unroll
-    for (int q = 0; q < WQ; ++q)
-      __builtin_amdgcn_global_load_lds((global_ptr_t)(w + woff[q] + (kt_begin + kt) * (KBT * 512)),
-                                       (lds_ptr_t)(stage + BM * ROW + (q * NW + wave) * 1024), 16, 0, 0);
+  const int kt_begin = KEEP ? 0 : (int)((long)blockIdx.y * (K / 64) / gridDim.y) * 2;
+  const int nk = KEEP ? KB : (int)((long)(blockIdx.y + 1) * (K / 64) / gridDim.y) * 2 - kt_begin;       // even
+  // load instruction q of this wave for k block kt (counted from kt_begin) into stage `slot`
+  auto issue = [&](int slot, int kt, int q) {
+    unsigned char* stage = smem + slot * STAGE;
+    if (q < XQ)
+      __builtin_amdgcn_global_load_lds((global_ptr_t)(x + xoff[q < XQ ? q : 0] + (kt_begin + kt) * 32),
+                                       (lds_ptr_t)(stage + (q * NW + wave) * 1024), 16, 0, 0);
+    else
+      __builtin_amdgcn_global_load_lds((global_ptr_t)(w + woff[q < XQ ? 0 : q - XQ] + (kt_begin + kt) * 512),
+                                       (lds_ptr_t)(stage + BM * ROW + ((q - XQ) * NW + wave) % WC * 1024), 16, 0, 0);
   };
 
-  f32x16 acc[TM][TN];
+  f32x4 acc[TN][TM];
 #pragma unroll
-  for (int i = 0; i < TM; ++i)
+  for (int i = 0; i < TN; ++i)
 #pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
-  f32x16 sum[KEEP ? TM : 1][KEEP ? TN : 1];
-  int seg = 0, seg_end = KEEP ? (int)((long)(K / 64) / splits) * PER64 : 0;     // of the segment being multiplied
+    for (int j = 0; j < TM; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  f32x4 sum[KEEP ? TN : 1][KEEP ? TM : 1];
+  int seg = 0, seg_end = KEEP ? (int)((long)(K / 64) / splits) * 2 : 0;     // of the segment being multiplied
 
-  // fragment addresses: row = tile row + lane % 32, k chunk = 2 ks + lane / 32, slot = chunk ^ SWZ(row)
-  const int frow = lane & 31, fhalf = lane >> 5, fsw = SWZ(frow);
+  // X fragments: row = tile row + lane % 16, k chunk = lane / 16, at its permuted slot; W fragments: blocks as they are
+  const int frow = lane & 15;
   const unsigned lds0 = (unsigned)(size_t)(lds_ptr_t)smem;
-  const unsigned xbase = lds0 + (wm * WM + frow) * ROW;
-  // W fragment of k step ks: block (row tile of the lane's row, k block ks / 2), lane slot
-  // 16 (2 (ks % 2) + lane / 32) + row % 16 of it: no permutation, 16 lanes read 256 consecutive bytes
-  const unsigned wbase = lds0 + BM * ROW + ((wn * WN + frow) / 16) * KBT * 1024 + (fhalf * 16 + (frow & 15)) * 16;
-  // The fragments of k step ks of a stage into one of two register sets.  The reads are written
-  // as instructions: the compiler, which cannot tell the stage being read from the stage a
-  // direct load is filling, would wait for every load in flight before each of its own reads,
-  // and the loads of the next tile would never overlap the products of this one.
-  u32x4 a[2][TM], b[2][TN];
-  auto read_step = [&](int set, int stage_index, int ks) {
-    read_frags<TM, 32 * ROW>(a[set], xbase + stage_index * STAGE + ((((ks * 2 + fhalf) ^ fsw)) << 4));
-    read_frags<TN, 2 * KBT * 1024>(b[set], wbase + stage_index * STAGE + (ks / 2) * 1024 + (ks % 2) * 512);
-  };
-  auto multiply = [&](int set, int j_from, int j_to) {
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = j_from; j < j_to; ++j)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_frag(a[set][i]), as_frag(b[set][j]), acc[i][j], 0, 0, 0);
-  };
+  const unsigned xbase = lds0 + (wm * WM + frow) * ROW + (((lane >> 4) ^ ((frow >> 2) & 3)) << 4);
+  const unsigned wbase = lds0 + BM * ROW + wn * WN * ROW + lane * 16;
+  // The reads are written as instructions: the compiler, which cannot tell the stage being read
+  // from the stage a direct load is filling, would wait for every load in flight before each of
+  // its own reads, and the loads of later stages would never overlap the products of this one.
+  u32x4 xf[2][TM], wf[2][TH];
 
-  // Every stage is filled before the loop; tile kt + STAGES is fetched into tile kt's stage as
-  // soon as every wave has read that tile's last fragments, which is during its last k step:
-  // the wait for the next tile, the barrier and the first reads of the next tile are hidden
-  // behind that step's products (half of them before the barrier, half after the reads).
-  constexpr int KS = BK / 16;
-  static_assert(KS % 2 == 0, "the register sets alternate and start a tile at set 0");
 #pragma unroll
-  for (int d = 0; d < STAGES; ++d)
-    if (d < nk) issue(d);
-  if (nk >= STAGES) wait_vmcnt<(STAGES - 1) * (XQ + WQ)>();
-  else wait_vmcnt<0>();
-  __builtin_amdgcn_s_barrier();   // tile 0 is in LDS for every wave
-  read_step(0, 0, 0);
-  for (int kt = 0; kt < nk; ++kt) {
-    const int stage_index = kt % STAGES;
+  for (int d = 0; d < AHEAD; ++d)
+    if (d < nk) {
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      const int cur = ks & 1, nxt = cur ^ 1;
-      if (ks + 1 < KS) {
-        read_step(nxt, stage_index, ks + 1);
-        wait_lgkmcnt<TM + TN>();          // this step's fragments (reads return in order)
-        use_frags<TM>(a[cur]);
-        use_frags<TN>(b[cur]);
-        multiply(cur, 0, TN);
-      } else {
-        wait_lgkmcnt<0>();                // the last fragments of this tile: its stage is free
-        use_frags<TM>(a[cur]);
-        use_frags<TN>(b[cur]);
-        multiply(cur, 0, TN / 2);
-        if (kt + 1 < nk) {
-          // this wave's part of tile kt + 1 has landed when only younger tiles are outstanding
-          if (kt + STAGES < nk) wait_vmcnt<(STAGES - 2) * (XQ + WQ)>();
-          else wait_vmcnt<0>();
-          __builtin_amdgcn_s_barrier();   // tile kt + 1 is in LDS for every wave; nobody reads tile kt any more
-          if (kt + STAGES < nk) issue(kt + STAGES);
-          read_step(nxt, (kt + 1) % STAGES, 0);
+      for (int q = 0; q < LOADS; ++q) issue(d, d, q);
+    }
+  wait_rounds<STAGES - 2, LOADS>(nk - 1);
+  __builtin_amdgcn_s_barrier();   // stage 0 is in LDS for every wave
+  read_frags<TM, 16 * ROW>(xf[0], xbase);
+  read_frags<TH, 1024>(wf[0], wbase);
+  int slot = 0;
+  // One k block: the products with the first half of the wave's W tiles while the second half is read, then those with the
+  // second half; halfway through these the next block's reads.  A load instruction of the block AHEAD of this one goes out
+  // every few products (the stage it fills was last read before the barrier in the block before this one).
+  auto block = [&](int kt, auto set_of, auto fetch_of) {
+    constexpr int set = decltype(set_of)::value;
+    constexpr bool fetch = decltype(fetch_of)::value;
+    constexpr int HALF = TH * TM, BEFORE = HALF + HALF / 2;          // products before the barrier
+    constexpr int EACH = (TM + TH + HALF / 2 - 1) / (HALF / 2);      // reads behind each product after it
+    const int next = slot + 1 == STAGES ? 0 : slot + 1, free_slot = slot == 0 ? STAGES - 1 : slot - 1;
+    wait_lgkmcnt<0>();                  // X and the first half
+    use_frags<TM>(xf[set]);
+    use_frags<TH>(wf[0]);
+#pragma unroll
+    for (int t = 0; t < 2 * HALF; ++t) {
+      if (t == HALF) {
+        wait_lgkmcnt<0>();              // the last fragments of this stage
+        use_frags<TH>(wf[1]);
+      }
+      if (t == BEFORE && (fetch || kt + 1 < nk)) {
+        // this wave's part of block kt + 1 has landed when only younger blocks' loads are outstanding
+        if constexpr (fetch) wait_vmcnt<(STAGES - 2) * LOADS>();
+        else wait_rounds<STAGES - 2, LOADS>(nk - 2 - kt);
+        __builtin_amdgcn_s_barrier();   // block kt + 1 is in LDS for every wave; nobody reads block kt any more
+      }
+      const int i = t / TM, j = t % TM;
+      acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(wf[i / TH][i % TH]), as_frag(xf[set][j]), acc[i][j], 0, 0, 0);
+      // a read behind each product: the second half's behind the first ones, the next block's behind those after the barrier
+      if (t < TH) {
+        __builtin_amdgcn_sched_barrier(0);
+        lds_read16_step<1024, TH>(wf[1][t < TH ? t : 0], wbase + slot * STAGE + TH * 1024, t);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (t >= BEFORE && (fetch || kt + 1 < nk)) {
+#pragma unroll
+        for (int r = (t - BEFORE) * EACH; r < (t - BEFORE + 1) * EACH; ++r) {
+          if (r >= TM + TH) continue;
+          __builtin_amdgcn_sched_barrier(0);
+          if (r < TM) lds_read16_step<16 * ROW, TM>(xf[set ^ 1][r < TM ? r : 0], xbase + next * STAGE, r);
+          else lds_read16_step<1024, TH>(wf[0][r < TM ? 0 : r - TM], wbase + next * STAGE, r - TM);
+          __builtin_amdgcn_sched_barrier(0);
         }
-        multiply(cur, TN / 2, TN);
+      }
+      if constexpr (fetch) {
+#pragma unroll
+        for (int q = 0; q < LOADS; ++q)
+          if (t == (2 * q + 1) * BEFORE / (2 * LOADS)) {
+            __builtin_amdgcn_sched_barrier(0);
+            issue(free_slot, kt + AHEAD, q);
+            __builtin_amdgcn_sched_barrier(0);
+          }
       }
     }
-    if (KEEP && kt + 1 == seg_end) {
+    slot = next;
+  };
+  auto two_blocks = [&](int kt, auto fetch_of) {
+    block(kt, Number<0>(), fetch_of);
+    block(kt + 1, Number<1>(), fetch_of);
+    if (KEEP && kt + 2 == seg_end) {
 #pragma unroll
-      for (int i = 0; i < (KEEP ? TM : 0); ++i)
+      for (int i = 0; i < (KEEP ? TN : 0); ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j)
+        for (int j = 0; j < TM; ++j) {
+          f32x4& s = sum[KEEP ? i : 0][KEEP ? j : 0];
 #pragma unroll
-          for (int e = 0; e < 16; ++e) {
-            sum[KEEP ? i : 0][KEEP ? j : 0][e] = seg == 0 ? acc[i][j][e] : sum[KEEP ? i : 0][KEEP ? j : 0][e] + acc[i][j][e];
-            acc[i][j][e] = 0.0f;
-          }
+          for (int e = 0; e < 4; ++e) s[e] = seg == 0 ? acc[i][j][e] : s[e] + acc[i][j][e];
+          acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
       ++seg;
-      seg_end = (int)((long)(seg + 1) * (K / 64) / splits) * PER64;
+      seg_end = (int)((long)(seg + 1) * (K / 64) / splits) * 2;
     }
-  }
-#undef SWZ
+  };
+  int kt = 0;
+  for (; kt + AHEAD < nk; kt += 2) two_blocks(kt, Number<1>());
+  for (; kt < nk; kt += 2) two_blocks(kt, Number<0>());
   if constexpr (KEEP) {
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+    for (int i = 0; i < TN; ++i)
 #pragma unroll
-      for (int j = 0; j < TN; ++j) acc[i][j] = sum[i][j];
+      for (int j = 0; j < TM; ++j) acc[i][j] = sum[i][j];
   }
 
-  // epilogue: lane holds column n = lane % 32 of each tile and rows (e/4)*8 + (lane/32)*4 + e%4
+  // epilogue: a lane holds row m = lane % 16 and four consecutive columns n = 4 (lane / 16) .. of each tile
+  const int mrow = m0 + wm * WM + frow, ncol = n0 + wn * (GLU ? WN / 2 : WN) + (lane >> 4) * 4;
   if (partial) {
     // [split][gate | up][M][N] (one part without GLU), 32-bit sums as they are
     constexpr int PARTS = GLU ? 2 : 1;
 #pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const int part = GLU ? j / (TN / 2) : 0;
-      const int n = GLU ? n0 + wn * (WN / 2) + (j % (TN / 2)) * 32 + (lane & 31) : n0 + wn * WN + j * 32 + (lane & 31);
+    for (int i = 0; i < TN; ++i) {
+      const int part = GLU ? i / TH : 0, n = ncol + (GLU ? i % TH : i) * 16;
       if (n >= N) continue;
       float* dst = partial + ((size_t)blockIdx.y * PARTS + part) * M * N + n;
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
+      for (int j = 0; j < TM; ++j) {
+        const int m = mrow + j * 16;
+        if (m >= M) continue;
+        if (N % 4 == 0) {
+          *reinterpret_cast<f32x4*>(dst + (size_t)m * N) = acc[i][j];
+        } else {                                                   // rows of the workspace that are not 16-byte aligned
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int m = m0 + wm * WM + i * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
-          if (m < M) dst[(size_t)m * N] = acc[i][j][e];
+          for (int e = 0; e < 4; ++e)
+            if (n + e < N) dst[(size_t)m * N + e] = acc[i][j][e];
         }
+      }
     }
     return;
   }
+  // four columns in one store: where all exist and rows and `out` are aligned for it
+  const bool narrow = mode_stores_elem(mode) || GLU;
+  const bool vec = N % 4 == 0 && out_stride % 4 == 0 && ((uintptr_t)out & (narrow ? 7 : 15)) == 0;
   if (GLU) {
 #pragma unroll
-    for (int j = 0; j < TN / 2; ++j) {
-      const int n = n0 + wn * (WN / 2) + j * 32 + (lane & 31);
+    for (int i = 0; i < TH; ++i) {
+      const int n = ncol + i * 16;
       if (n >= N) continue;
 #pragma unroll
-      for (int i = 0; i < TM; ++i) {
+      for (int j = 0; j < TM; ++j) {
+        const int m = mrow + j * 16;
+        if (m >= M) continue;
+        float v[4];
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int m = m0 + wm * WM + i * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
-          if (m >= M) continue;
-          reinterpret_cast<bf16_t*>(out)[(size_t)m * out_stride + n] =
-              float_to_bf16(swiglu1(acc[i][j][e], acc[i][j + TN / 2][e]));
+        for (int e = 0; e < 4; ++e) v[e] = swiglu1(acc[i][j][e], acc[i + TH][j][e]);
+        bf16_t* dst = reinterpret_cast<bf16_t*>(out) + (size_t)m * out_stride + n;
+        if (vec) {
+          *reinterpret_cast<uint2*>(dst) = make_uint2(pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3]));
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) dst[e] = float_to_bf16(v[e]);           // N is a multiple of 16
         }
       }
     }
     return;
   }
 #pragma unroll
-  for (int j = 0; j < TN; ++j) {
-    const int n = n0 + wn * WN + j * 32 + (lane & 31);
+  for (int i = 0; i < TN; ++i) {
+    const int n = ncol + i * 16;
     if (n >= N) continue;
-    const float bv = bias ? load_vec(bias, bias_is_f32, n) : 0.0f;
+    float bv[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) bv[e] = bias && n + e < N ? load_vec(bias, bias_is_f32, n + e) : 0.0f;
     if (mode == MODE_ADD_F32) {
-      // All reads before the first store, which may alias the next read: element by element a lane waits for
-      // memory TM * 16 times in a row (kept segments, 700 rows of 12,288 columns of K 1,024: 82 us, 44 so;
-      // 4,096 rows of 1,152 of 896 45, 25 so; a block a segment, without this epilogue, 62 and 36).  Rows past M
-      // read the last row and store nothing.
+      // All reads of a tile column before its first store, which may alias the next read: element by element a lane
+      // waits for memory at every one.  Rows past M read the last row and store nothing.
       float* rows = reinterpret_cast<float*>(out) + n;
-      float before[TM][16];
+      float before[TM][4];
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
+      for (int j = 0; j < TM; ++j) {
+        const float* src = rows + (size_t)min(mrow + j * 16, M - 1) * out_stride;
+        if (vec) {
+          const f32x4 r = *reinterpret_cast<const f32x4*>(src);
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int m = m0 + wm * WM + i * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
-          before[i][e] = rows[(size_t)min(m, M - 1) * out_stride];
+          for (int e = 0; e < 4; ++e) before[j][e] = r[e];
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) before[j][e] = n + e < N ? src[e] : 0.0f;
         }
+      }
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
+      for (int j = 0; j < TM; ++j) {
+        const int m = mrow + j * 16;
+        if (m >= M) continue;
+        f32x4 v;
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int m = m0 + wm * WM + i * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
-          if (m < M) rows[(size_t)m * out_stride] = before[i][e] + (acc[i][j][e] + bv);
+        for (int e = 0; e < 4; ++e) v[e] = before[j][e] + (acc[i][j][e] + bv[e]);
+        if (vec) {
+          *reinterpret_cast<f32x4*>(rows + (size_t)m * out_stride) = v;
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (n + e < N) rows[(size_t)m * out_stride + e] = v[e];
         }
+      }
       continue;
     }
 #pragma unroll
-    for (int i = 0; i < TM; ++i) {
+    for (int j = 0; j < TM; ++j) {
+      const int m = mrow + j * 16;
+      if (m >= M) continue;
+      float v[4];
 #pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int m = m0 + wm * WM + i * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
-        if (m >= M) continue;
-        const float v = acc[i][j][e] + bv;
-        const size_t at = (size_t)m * out_stride + n;
-        if (mode_stores_elem(mode)) reinterpret_cast<bf16_t*>(out)[at] = float_to_bf16(mode_value(v, mode));
-        else reinterpret_cast<float*>(out)[at] = v;
+      for (int e = 0; e < 4; ++e) v[e] = acc[i][j][e] + bv[e];
+      const size_t at = (size_t)m * out_stride + n;
+      if (narrow) {
+        bf16_t* dst = reinterpret_cast<bf16_t*>(out) + at;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = mode_value(v[e], mode);
+        if (vec) {
+          *reinterpret_cast<uint2*>(dst) = make_uint2(pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3]));
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (n + e < N) dst[e] = float_to_bf16(v[e]);
+        }
+      } else {
+        float* dst = reinterpret_cast<float*>(out) + at;
+        if (vec) {
+          *reinterpret_cast<f32x4*>(dst) = f32x4{v[0], v[1], v[2], v[3]};
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (n + e < N) dst[e] = v[e];
+        }
       }
     }
   }
@@ -565,14 +642,14 @@ static int add_split_sums(const float* partial, int splits, int m, int n, const 
   return 0;
 }
 
-template <int BM, int BN, int WAVES_M, int WAVES_N, bool GLU, int BK = 64, int STAGES = 2, bool KEEP = false>
+template <int BM, int BN, int WAVES_M, int WAVES_N, bool GLU, int STAGES = 5, bool KEEP = false>
 static int launch_tile(const bf16_t* x, int x_stride, const bf16_t* w, const void* bias, int bias_is_f32, void* out,
                        int out_stride, int m, int n, int k, int mode, hipStream_t stream, int segs = 1,
                        float* partial = nullptr, const SplitNorm* norm = nullptr, const RopeStore* rope = nullptr) {
   static bool configured = false;
-  constexpr int lds_bytes = STAGES * (BM + BN) * BK * 2;
+  constexpr int lds_bytes = STAGES * (BM + BN) * 64;
   static_assert(lds_bytes <= 160 * 1024, "the stages do not fit the LDS of a CU");
-  auto kernel = &gemm_tile_kernel<BM, BN, WAVES_M, WAVES_N, GLU, BK, STAGES, KEEP>;
+  auto kernel = &gemm_tile_kernel<BM, BN, WAVES_M, WAVES_N, GLU, STAGES, KEEP>;
   if (!configured) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                        lds_bytes);
@@ -588,7 +665,7 @@ static int launch_tile(const bf16_t* x, int x_stride, const bf16_t* w, const voi
   const bool after = splits > 1 || norm || rope;
   const int m_blocks = ceil_div(m, BM), n_blocks = ceil_div(n, GLU ? BN / 2 : BN);
   if constexpr (KEEP) AXK_INSTANCE(INST_GEMM_KEPT, GLU);
-  else AXK_INSTANCE(INST_GEMM_TILE, BM, BN, WAVES_M, WAVES_N, GLU, STAGES);
+  else AXK_INSTANCE(INST_GEMM_TILE, BM, BN, WAVES_M, WAVES_N, GLU, STAGES / 2);
   kernel<<<dim3(m_blocks * n_blocks, splits), WAVES_M * WAVES_N * 64, lds_bytes, stream>>>(
       x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode, m_blocks, n_blocks, after ? partial : nullptr, segs);
   AXK_LAUNCH_CHECK("gemm_tile");
@@ -602,9 +679,7 @@ static int launch_tile(const bf16_t* x, int x_stride, const bf16_t* w, const voi
 // instruction), keeping a ring of steps in flight so that the memory pipe never drains, and
 // multiplying with the rows of X (the B operand: lane l holds row l % 16, 8 consecutive k
 // from (l / 16) * 8).  C[n][m] tiles of 16 x 16: a lane ends with 4 consecutive n of one m, one
-// vector store.  The segments' sums meet in LDS and are added in segment order.  A 16x16x32 MFMA
-// gives the bits of two chained 32x32x16 MFMAs over the same 32 k (measured over wide ranges of
-// exponents; the tests compare the kernels bit for bit), so the chain is the tile kernel's.
+// vector store.  The segments' sums meet in LDS and are added in segment order.
 // * GLU (NT16 = 2): the block's two tiles are the gate rows n0 .. n0 + 15 and the up rows of the
 //   same columns (W holds 2 N rows), and the output is silu(gate) * up.
 // * ROPE (NT16 = 2; the attention's fused [q; k; v] matrix, W's rows are heads of head_dim): a
@@ -954,7 +1029,7 @@ gemm_stream_kernel(const bf16_t* __restrict__ x, int x_stride, const bf16_t* __r
       xf[slot][j][1] = *reinterpret_cast<const uint4*>(xrow[j] + k0 + 32);
     }
   };
-  // one 16x16x32 MFMA is two chained 32x32x16 ones over the same k, bit for bit (the tile kernel's)
+  // the tile kernel's chain
   auto multiply = [&](int slot) {
 #pragma unroll
     for (int h = 0; h < 2; ++h)
@@ -1826,20 +1901,20 @@ static int gemm_mfma_pass(const bf16_t* x, int x_stride, const bf16_t* w, const 
   const long rounds_big = (big + 255) / 256, rounds_small = (small + 511) / 512;
   const bool use_big = rounds_big * 100 <= rounds_small * 65;
   if (keep) {
-    if (glu) return launch_tile<128, 128, 2, 2, true, 64, 2, true>(ARGS, segs, ws);
-    return launch_tile<128, 128, 2, 2, false, 64, 2, true>(ARGS, segs, ws, norm, rope_after);
+    if (glu) return launch_tile<128, 128, 2, 2, true, 5, true>(ARGS, segs, ws);
+    return launch_tile<128, 128, 2, 2, false, 5, true>(ARGS, segs, ws, norm, rope_after);
   }
   if (!use_big) {
     // Up to 256 rows still wait for W more than for the matrix cores.  Where the small tiles are no
-    // more blocks than CUs, a block has its CU's LDS to itself: four stages instead of two, three
-    // steps of loads in flight (the down projection of a 7B layer at 256 rows 79 -> 64 us); with
-    // more blocks two of them share a CU and cover each other's waits (four stages there: slower).
+    // more blocks than CUs, a block has its CU's LDS to itself: nine stages of 32 k instead of five
+    // (the down projection of a 7B layer at 256 rows: 64 us with four steps of 64 k, 79 with two); with
+    // more blocks two of them share a CU and cover each other's waits (more stages there: slower).
     const bool deep = m <= 256 && small <= 256;
     if (glu) {
-      if (deep) return launch_tile<128, 128, 2, 2, true, 64, 4>(ARGS, segs, ws);
+      if (deep) return launch_tile<128, 128, 2, 2, true, 9>(ARGS, segs, ws);
       return launch_tile<128, 128, 2, 2, true>(ARGS, segs, ws);
     }
-    if (deep) return launch_tile<128, 128, 2, 2, false, 64, 4>(ARGS, segs, ws, norm, rope_after);
+    if (deep) return launch_tile<128, 128, 2, 2, false, 9>(ARGS, segs, ws, norm, rope_after);
     return launch_tile<128, 128, 2, 2, false>(ARGS, segs, ws, norm, rope_after);
   }
   if (glu) return launch_tile<256, 256, 4, 2, true>(ARGS, segs, ws);
