@@ -234,6 +234,9 @@ gemm_tile_kernel(const bf16_t* __restrict__ x, int x_stride, const bf16_t* __res
   __builtin_amdgcn_s_barrier();   // stage 0 is in LDS for every wave
   read_frags<TM, 16 * ROW>(xf[0], xbase);
   read_frags<TH, 1024>(wf[0], wbase);
+  wait_lgkmcnt<0>();
+  use_frags<TM>(xf[0]);
+  use_frags<TH>(wf[0]);
   int slot = 0;
   // One k block: the products with the first half of the wave's W tiles while the second half is read, then those with the
   // second half; halfway through these the next block's reads.  A load instruction of the block AHEAD of this one goes out
@@ -244,21 +247,18 @@ gemm_tile_kernel(const bf16_t* __restrict__ x, int x_stride, const bf16_t* __res
     constexpr int HALF = TH * TM, BEFORE = HALF + HALF / 2;          // products before the barrier
     constexpr int EACH = (TM + TH + HALF / 2 - 1) / (HALF / 2);      // reads behind each product after it
     const int next = slot + 1 == STAGES ? 0 : slot + 1, free_slot = slot == 0 ? STAGES - 1 : slot - 1;
-    wait_lgkmcnt<0>();                  // X and the first half
-    use_frags<TM>(xf[set]);
-    use_frags<TH>(wf[0]);
 #pragma unroll
     for (int t = 0; t < 2 * HALF; ++t) {
       if (t == HALF) {
         wait_lgkmcnt<0>();              // the last fragments of this stage
         use_frags<TH>(wf[1]);
       }
-      if (t == BEFORE && (fetch || kt + 1 < nk)) {
+      if (t == BEFORE) {
         // this wave's part of block kt + 1 has landed when only younger blocks' loads are outstanding
         if constexpr (fetch) wait_vmcnt<(STAGES - 2) * LOADS>();
         else wait_rounds<STAGES - 2, LOADS>(nk - 2 - kt);
         __builtin_amdgcn_s_barrier();   // block kt + 1 is in LDS for every wave; nobody reads block kt any more
-      }
+      }                                 // (behind the last block: whatever the stage holds is read and not used)
       const int i = t / TM, j = t % TM;
       acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(wf[i / TH][i % TH]), as_frag(xf[set][j]), acc[i][j], 0, 0, 0);
       // a read behind each product: the second half's behind the first ones, the next block's behind those after the barrier
@@ -267,7 +267,7 @@ gemm_tile_kernel(const bf16_t* __restrict__ x, int x_stride, const bf16_t* __res
         lds_read16_step<1024, TH>(wf[1][t < TH ? t : 0], wbase + slot * STAGE + TH * 1024, t);
         __builtin_amdgcn_sched_barrier(0);
       }
-      if (t >= BEFORE && (fetch || kt + 1 < nk)) {
+      if (t >= BEFORE) {
 #pragma unroll
         for (int r = (t - BEFORE) * EACH; r < (t - BEFORE + 1) * EACH; ++r) {
           if (r >= TM + TH) continue;
@@ -288,6 +288,9 @@ gemm_tile_kernel(const bf16_t* __restrict__ x, int x_stride, const bf16_t* __res
       }
     }
     slot = next;
+    wait_lgkmcnt<0>();                  // the next block's X and first half: no read is under way across a branch
+    use_frags<TM>(xf[set ^ 1]);
+    use_frags<TH>(wf[0]);
   };
   auto two_blocks = [&](int kt, auto fetch_of) {
     block(kt, Number<0>(), fetch_of);

@@ -76,125 +76,19 @@ __device__ inline float ss_row_sum(float v) {
   return v;
 }
 
-// The walk.  grid (requests of the step, heads, blocks of 8 value dims); a block is 128 threads: sixteen
-// lanes side by side share a value dim p and hold the state's rows n = lane, lane + 16, ... of that
-// column (OWN each: N up to 16 OWN).  The operands of four tokens are asked for while the four before
-// them are worked on.  spans [n][3] = (slot, first token, tokens), or null: every token a request of its
-// own (a decoding step) in slot seq_rows[t].  u [T, channels] = [x: heads P | B: groups N | C: groups N]
-// behind the convolution; terms [T, heads, 2] = (dt, a).  y [T, heads P] float32.  The block (head 0,
-// dims 0) also brings the convolution's kept inputs up to date from conv_in (the convolution's inputs,
-// float32 rows conv_in_stride apart).  A sum over n is sixteen partial chains in ascending n folded in a
-// fixed order: the same for a token however the request was cut into steps.  FULL: N is 16 OWN, so no row
-// of a lane lies beyond the state (a lane's rows of B and C are then one address and constant offsets, and
-// nothing has to be kept at zero: a wave of this kernel is bound by the instructions it issues a token).
-#define SS_AHEAD 4
-#define SS_THREADS 128
-template <int OWN>
-struct SsOperands {
-  float x[SS_AHEAD], dt[SS_AHEAD], a[SS_AHEAD], B[SS_AHEAD][OWN], C[SS_AHEAD][OWN];
-};
+// The same over the thirty-two lanes of two neighbouring rows.
+__device__ inline float ss_two_rows_sum(float v) {
+  const unsigned r = __float_as_uint(ss_row_sum(v));
+  const auto s = __builtin_amdgcn_permlane16_swap(r, r, false, false);
+  const unsigned even = s[0], odd = s[1];
+  return __uint_as_float(even) + __uint_as_float(odd);
+}
 
-template <int OWN, bool FULL>
-__global__ void __launch_bounds__(SS_THREADS)
-state_space_scan_kernel(const float* __restrict__ u, const float* __restrict__ terms, const void* __restrict__ d_skip,
-                        int d_is_f32, float* __restrict__ state, long state_stride, long copy_elems, long tail_at,
-                        const int32_t* __restrict__ spans, const int32_t* __restrict__ positions,
-                        const int32_t* __restrict__ seq_rows, const float* __restrict__ conv_in, long conv_in_stride,
-                        float* __restrict__ y, int heads, int groups, int P, int N, int channels, int taps,
-                        const int32_t* __restrict__ segs, float* __restrict__ ends, float* __restrict__ cum) {
-  int slot, first, count;
-  bool from_state = true;
-  if (segs) {
-    slot = segs[4 * blockIdx.x]; first = segs[4 * blockIdx.x + 1]; count = segs[4 * blockIdx.x + 2];
-    from_state = segs[4 * blockIdx.x + 3] != 0;
-  } else if (spans) {
-    slot = spans[3 * blockIdx.x]; first = spans[3 * blockIdx.x + 1]; count = spans[3 * blockIdx.x + 2];
-  } else {
-    slot = seq_rows[blockIdx.x]; first = blockIdx.x; count = 1;
-  }
-  const int h = blockIdx.y, g = h / (heads / groups);
-  const int ns = threadIdx.x & 15, p = blockIdx.z * (SS_THREADS / 16) + (threadIdx.x >> 4);
-  const bool has_p = p < P;
-  const int start = positions[first];
-  const float* from = state + (long)slot * state_stride + (long)((start + 1) & 1) * copy_elems;
-  float* to = state + (long)slot * state_stride + (long)((start + count - 1) & 1) * copy_elems;
-  const int inner = heads * P;
-  const long s_at = (long)h * N * P;
-  float S[OWN];
-  int n_of[OWN];
-#pragma unroll
-  for (int i = 0; i < OWN; ++i) {
-    const int n = ns + 16 * i;
-    S[i] = from_state && has_p && n < N ? from[s_at + (long)n * P + p] : 0.0f;
-    n_of[i] = min(n, N - 1);            // rows beyond N hold zeros in S: what they meet does not count
-  }
-  const float dskip = load_vec(d_skip, d_is_f32, h);
-  const long x_col = (long)h * P + (has_p ? p : 0), b_col = inner + (long)g * N, c_col = inner + (long)groups * N + (long)g * N;
-  const int last = first + count;
-  const long lane_b = b_col + ns, lane_c = c_col + ns;
-  auto fetch = [&](SsOperands<OWN>& o, int t0) {
-#pragma unroll
-    for (int k = 0; k < SS_AHEAD; ++k) {
-      const int t = min(t0 + k, last - 1);             // behind the last token: the last again, not used
-      const float* row = u + (long)t * channels;
-      const float* bp = row + lane_b;
-      const float* cp = row + lane_c;
-      o.x[k] = row[x_col];
-      o.dt[k] = terms[((long)t * heads + h) * 2];
-      o.a[k] = terms[((long)t * heads + h) * 2 + 1];
-#pragma unroll
-      for (int i = 0; i < OWN; ++i) {
-        o.B[k][i] = FULL ? bp[16 * i] : row[b_col + n_of[i]];
-        o.C[k][i] = FULL ? cp[16 * i] : row[c_col + n_of[i]];
-      }
-    }
-  };
-  float decay = 1.0f;                  // of a segment: the product of its tokens' a so far
-  const bool tells_decay = cum != nullptr && blockIdx.z == 0 && threadIdx.x == 0;
-  auto work = [&](const SsOperands<OWN>& o, int t0) {
-#pragma unroll
-    for (int k = 0; k < SS_AHEAD; ++k) {
-      if (t0 + k < last) {
-        decay *= o.a[k];
-        if (tells_decay) cum[(long)(t0 + k) * heads + h] = decay;
-        const float dx = o.dt[k] * o.x[k];
-        float part = 0.0f;
-#pragma unroll
-        for (int i = 0; i < OWN; ++i) {
-          S[i] = FULL || ns + 16 * i < N ? fmaf(o.a[k], S[i], dx * o.B[k][i]) : 0.0f;
-          part = fmaf(S[i], o.C[k][i], part);
-        }
-        part = ss_row_sum(part);
-        if (ns == 0 && has_p) y[(long)(t0 + k) * inner + x_col] = fmaf(dskip, o.x[k], part);
-      }
-    }
-  };
-  SsOperands<OWN> even, odd;
-  fetch(even, first);
-  for (int t = first; t < last; t += 2 * SS_AHEAD) {
-    if (t + SS_AHEAD < last) fetch(odd, t + SS_AHEAD);
-    work(even, t);
-    if (t + SS_AHEAD >= last) break;
-    if (t + 2 * SS_AHEAD < last) fetch(even, t + 2 * SS_AHEAD);
-    work(odd, t + SS_AHEAD);
-  }
-  if (segs) {                          // a segment's end state goes to the workspace; the fold brings the request's state up to date
-    float* end = ends + ((long)blockIdx.x * heads + h) * N * P;
-#pragma unroll
-    for (int i = 0; i < OWN; ++i) {
-      const int n = ns + 16 * i;
-      if (has_p && n < N) end[(long)n * P + p] = S[i];
-    }
-    return;
-  }
-#pragma unroll
-  for (int i = 0; i < OWN; ++i) {
-    const int n = ns + 16 * i;
-    if (has_p && n < N) to[s_at + (long)n * P + p] = S[i];
-  }
-  if (blockIdx.y != 0 || blockIdx.z != 0) return;
-  // the convolution's last taps - 1 inputs: of (what was kept, this step's inputs) the last taps - 1; place
-  // i takes what lies `count` places later (where both copies are one: read before it is written, ascending)
+// A request's kept inputs of the convolution behind `count` tokens of this step: of (what was kept, this step's inputs) the
+// last taps - 1; place i takes what lies `count` places later (where both copies are one: read before it is written,
+// ascending).  By all threads of a block.
+__device__ inline void ss_keep_inputs(const float* from, float* to, long tail_at, const float* __restrict__ conv_in,
+                                      long conv_in_stride, int first, int count, int channels, int taps) {
   float* kept = to + tail_at;
   const float* kept_from = from + tail_at;
   for (int c = threadIdx.x; c < channels; c += blockDim.x)
@@ -205,7 +99,285 @@ state_space_scan_kernel(const float* __restrict__ u, const float* __restrict__ t
     }
 }
 
-// Long stretches of tokens in segments.  The scan above then runs every segment of a request side by side:
+// A decoding step.  grid (tokens, heads, blocks of 8 value dims), every token a request of its own in slot seq_rows[t]; a
+// block is 256 threads: thirty-two lanes side by side share a value dim p and hold the state's rows n = lane,
+// lane + 32, ... of that column (OWN each: N up to 32 OWN).  u [T, channels] = [x: heads P | B: groups N |
+// C: groups N] behind the convolution; terms [T, heads, 2] = (dt, a).  y [T, heads P] float32.  The block
+// (head 0, dims 0) also brings the convolution's kept inputs up to date from conv_in (the convolution's
+// inputs, float32 rows conv_in_stride apart).  A sum over n is thirty-two partial chains in ascending n
+// folded in a fixed order: the same for a token however the request was cut into steps.
+#define SS_DIMS 8          // value dims a block
+#define SS_LANES 32
+#define SS_WALKERS (SS_DIMS * SS_LANES)
+template <int OWN>
+__global__ void __launch_bounds__(SS_WALKERS)
+state_space_step_kernel(const float* __restrict__ u, const float* __restrict__ terms, const void* __restrict__ d_skip,
+                        int d_is_f32, float* __restrict__ state, long state_stride, long copy_elems, long tail_at,
+                        const int32_t* __restrict__ positions, const int32_t* __restrict__ seq_rows,
+                        const float* __restrict__ conv_in, long conv_in_stride, float* __restrict__ y, int heads, int groups,
+                        int P, int N, int channels, int taps) {
+  const int t = blockIdx.x, h = blockIdx.y, g = h / (heads / groups), slot = seq_rows[t];
+  const int ns = threadIdx.x % SS_LANES, p = blockIdx.z * SS_DIMS + threadIdx.x / SS_LANES;
+  const bool has_p = p < P;
+  const int start = positions[t];
+  const float* from = state + (long)slot * state_stride + (long)((start + 1) & 1) * copy_elems;
+  float* to = state + (long)slot * state_stride + (long)(start & 1) * copy_elems;
+  const int inner = heads * P;
+  const long s_at = (long)h * N * P, x_col = (long)h * P + (has_p ? p : 0);
+  const float* row = u + (long)t * channels;
+  const float* B = row + inner + (long)g * N;
+  const float* C = B + (long)groups * N;
+  const float x = row[x_col], dt = terms[((long)t * heads + h) * 2], a = terms[((long)t * heads + h) * 2 + 1];
+  const float dskip = load_vec(d_skip, d_is_f32, h);
+  float S[OWN], Bs[OWN], Cs[OWN];
+#pragma unroll
+  for (int i = 0; i < OWN; ++i) {
+    const int n = ns + SS_LANES * i, at = min(n, N - 1);       // rows beyond N: zeros in S, what they meet does not count
+    S[i] = has_p && n < N ? from[s_at + (long)n * P + p] : 0.0f;
+    Bs[i] = B[at];
+    Cs[i] = C[at];
+  }
+  const float dx = dt * x;
+  float part = 0.0f;
+#pragma unroll
+  for (int i = 0; i < OWN; ++i) {
+    S[i] = ns + SS_LANES * i < N ? fmaf(a, S[i], dx * Bs[i]) : 0.0f;
+    part = fmaf(S[i], Cs[i], part);
+  }
+  part = ss_two_rows_sum(part);
+  if (ns == 0 && has_p) y[(long)t * inner + x_col] = fmaf(dskip, x, part);
+#pragma unroll
+  for (int i = 0; i < OWN; ++i) {
+    const int n = ns + SS_LANES * i;
+    if (has_p && n < N) to[s_at + (long)n * P + p] = S[i];
+  }
+  if (blockIdx.y == 0 && blockIdx.z == 0) ss_keep_inputs(from, to, tail_at, conv_in, conv_in_stride, t, 1, channels, taps);
+}
+
+// The walk of stretches of tokens (a request's tokens of the step, or segments of them): the arithmetic and
+// the order of the kernel above, its operands through LDS.  SS_CHUNK tokens' B and C rows, the block's values
+// of x, and (dt, a) go to LDS by direct loads, a dword a lane, during the first half of the chunk before (one
+// barrier a chunk).  A lane's rows of B and C lie there side by side, so that it reads four at a time, conflict-
+// free, the operands of two tokens while the two before them are worked on.  A lane keeps the output of the
+// chunk's token that has its number; one store a chunk, while the next chunk is worked on.
+// What bounds it: a wave's own instructions and waits, a token after the other; more waves share a token's work,
+// and fewer of them are loads, than with sixteen lanes a value dim and a dword load a row of B and C a token (38
+// vector, 20 scalar and 17 memory instructions a token and wave, at 262 ns; here 125 to 135 ns).  32 heads of 64
+// dims, 128 rows, 2 groups (us, before and here): stretches of 311, 611 and 1,203 tokens 307 / 183, one of 1,024
+// 256 / 130, of 64 26 / 15, two of 1,024 270 / 142, 5 of 300 165 / 100, 32 of a token 44 / 41; 256 rows and 16
+// heads, 1,024 tokens 390 / 162; a decoding step of 8 tokens 17 / 13, of 32 44 / 36 (the kernel above).  Sixteen lanes
+// with the operands through LDS: 201 for the three stretches; two chunks ahead instead of one: 187.
+#define SS_CHUNK 16
+template <int OWN>
+struct SsChunk {
+  static constexpr int QUADS = OWN >= 4 ? OWN / 4 : 1;          // reads of four of a lane's rows
+  static constexpr int ROWS = SS_LANES * QUADS * 4;             // floats a token's B (or C) takes (OWN < 4: places unused)
+  static constexpr int WAVES = SS_WALKERS / AXON_WAVE, PIECES = ROWS / 64;
+  static constexpr int PER = 2 * PIECES / WAVES;                // loads of a wave and token
+  static constexpr int X_AT = SS_CHUNK * 2 * ROWS, TERMS_AT = X_AT + SS_DIMS * SS_CHUNK, FLOATS = TERMS_AT + AXON_WAVE;
+};
+
+template <int V>
+struct SsNumber {
+  static constexpr int value = V;
+};
+
+template <int OWN>
+struct SsStaged {
+  u32x4 B[2][SsChunk<OWN>::QUADS], C[2][SsChunk<OWN>::QUADS];
+  u32x4 x[1], terms[1];
+};
+
+template <int OWN, bool FULL, bool SEGMENTS>
+__global__ void __launch_bounds__(SS_WALKERS)
+state_space_walk_kernel(const float* __restrict__ u, const float* __restrict__ terms, const void* __restrict__ d_skip,
+                        int d_is_f32, float* __restrict__ state, long state_stride, long copy_elems, long tail_at,
+                        const int32_t* __restrict__ spans, const int32_t* __restrict__ positions,
+                        const float* __restrict__ conv_in, long conv_in_stride, float* __restrict__ y, int heads, int groups,
+                        int P, int N, int channels, int taps, const int32_t* __restrict__ segs, float* __restrict__ ends,
+                        float* __restrict__ cum) {
+  typedef SsChunk<OWN> Chunk;
+  constexpr int ROWS = Chunk::ROWS, QUADS = Chunk::QUADS, PER = Chunk::PER, WAVES = Chunk::WAVES, PIECES = Chunk::PIECES, SUB = 2;
+  static_assert(WAVES == 4 && SS_DIMS * SS_CHUNK == 2 * AXON_WAVE && 2 * SS_CHUNK <= AXON_WAVE, "who asks for the rest of a chunk");
+  __shared__ __align__(16) float lds[2][Chunk::FLOATS];
+  const int* stretch = SEGMENTS ? segs + 4 * blockIdx.x : spans + 3 * blockIdx.x;
+  const int slot = stretch[0], first = stretch[1], count = stretch[2];
+  const bool from_state = SEGMENTS ? stretch[3] != 0 : true;
+  const int h = blockIdx.y, g = h / (heads / groups);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ns = threadIdx.x % SS_LANES, p = blockIdx.z * SS_DIMS + threadIdx.x / SS_LANES;
+  const bool has_p = p < P;
+  const int start = positions[first];
+  const float* from = state + (long)slot * state_stride + (long)((start + 1) & 1) * copy_elems;
+  float* to = state + (long)slot * state_stride + (long)((start + count - 1) & 1) * copy_elems;
+  const int inner = heads * P;
+  const long s_at = (long)h * N * P, x_col = (long)h * P + (has_p ? p : 0);
+  const long b_col = inner + (long)g * N;
+  float S[OWN];
+#pragma unroll
+  for (int i = 0; i < OWN; ++i) {
+    const int n = ns + SS_LANES * i;
+    S[i] = from_state && has_p && n < N ? from[s_at + (long)n * P + p] : 0.0f;
+  }
+  const float dskip = load_vec(d_skip, d_is_f32, h);
+
+  // What this lane asks for of a token's row: load j of the wave is piece j WAVES + wave of (B's pieces, C's pieces), the
+  // c-th 64 of the places (quad, lane of the row set, place): row n = lane of the set + 32 (4 quad + place).
+  typedef const __attribute__((address_space(1))) void* from_t;
+  typedef __attribute__((address_space(3))) void* to_t;
+  unsigned col[PER];                   // in bytes from the row's B
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const int piece = j * WAVES + wave, c = piece % PIECES;
+    const int at = c * 64 + lane, n = at / 4 % SS_LANES + SS_LANES * (at / (4 * SS_LANES) * 4 + at % 4);
+    col[j] = (unsigned)((piece < PIECES ? 0 : groups * N) + min(n, N - 1)) * 4u;        // places beyond the state: any row
+  }
+  // COUNT tokens of the chunk that begins with token t0 of the stretch, from its token k on (behind the stretch: its last
+  // token again, not used)
+  const unsigned row_bytes = (unsigned)channels * 4u;
+  const char* rows = (const char*)(u + (long)first * channels + b_col);
+  auto ask = [&](int buffer, int t0, int k, auto how_many) {
+    constexpr int COUNT = decltype(how_many)::value;
+#pragma unroll
+    for (int i = 0; i < COUNT; ++i) {
+      const char* row = rows + (unsigned long)(unsigned)min(t0 + k + i, count - 1) * row_bytes;
+#pragma unroll
+      for (int j = 0; j < PER; ++j)
+        __builtin_amdgcn_global_load_lds((from_t)(row + col[j]), (to_t)(&lds[buffer][0] + (k + i) * 2 * ROWS + (j * WAVES + wave) * 64), 4, 0, 0);
+    }
+  };
+  // the rest of a chunk: x [value dim of the block][token] (waves 0 and 1), (dt, a) a token (waves 2 and 3, the same)
+  auto ask_rest = [&](int buffer, int t0) {
+    const int pp = blockIdx.z * SS_DIMS + (int)threadIdx.x / SS_CHUNK % SS_DIMS;
+    const long t = first + min(t0 + (wave < 2 ? lane : lane >> 1) % SS_CHUNK, count - 1);
+    const float* src = wave < 2 ? u + t * channels + (long)h * P + min(pp, P - 1) : terms + (t * heads + h) * 2 + (lane & 1);
+    __builtin_amdgcn_global_load_lds((from_t)src, (to_t)(&lds[buffer][0] + (wave < 2 ? Chunk::X_AT + wave * AXON_WAVE : Chunk::TERMS_AT)),
+                                     4, 0, 0);
+  };
+  ask_rest(0, 0);
+#pragma unroll
+  for (int k = 0; k < SS_CHUNK; ++k)
+    if (k < count) ask(0, 0, k, SsNumber<1>());
+
+  const unsigned lds0 = (unsigned)(size_t)(to_t)&lds[0][0];
+  const unsigned bc_at = lds0 + ns * 16, terms_at = lds0 + Chunk::TERMS_AT * 4;
+  const unsigned x_at = lds0 + (Chunk::X_AT + threadIdx.x / SS_LANES * SS_CHUNK) * 4;
+  float decay = 1.0f;                  // of a segment: the product of its tokens' a so far
+  float kept_y = 0.0f, kept_decay = 1.0f;      // of the chunk's token ns
+
+  // the operands of the chunk's tokens k0 + turn SUB ..: `turn` is known when compiled
+  auto read = [&](SsStaged<OWN>& o, unsigned at, int k0, int turn) {
+    const unsigned rows = bc_at + at + k0 * (2 * ROWS * 4);
+#pragma unroll
+    for (int k = 0; k < SUB; ++k)
+#pragma unroll
+      for (int q = 0; q < QUADS; ++q) {
+        lds_read16_step<16 * SS_LANES, 4 * SUB * QUADS>(o.B[k][q], rows, (turn * SUB + k) * 2 * QUADS + q);
+        lds_read16_step<16 * SS_LANES, 4 * SUB * QUADS>(o.C[k][q], rows, (turn * SUB + k) * 2 * QUADS + QUADS + q);
+      }
+    lds_read16_step<16, 2>(o.terms[0], terms_at + at + k0 * 8, turn);
+    lds_read16<0>(o.x[0], x_at + at + k0 * 4);
+    __builtin_amdgcn_sched_barrier(0);          // all of them ahead of the work that they are to be hidden behind
+  };
+  auto arrived = [&](SsStaged<OWN>& o) {
+    wait_lgkmcnt<0>();
+#pragma unroll
+    for (int k = 0; k < SUB; ++k) {
+      use_frags<QUADS>(o.B[k]);
+      use_frags<QUADS>(o.C[k]);
+    }
+    use_frags<1>(o.terms);
+    use_frags<1>(o.x);
+  };
+  // the work of SUB tokens from the chunk's token k0 + turn SUB on (left: the chunk's that exist; WHOLE: all of them)
+  auto work = [&](const SsStaged<OWN>& o, int k0, int turn, int left, auto whole) {
+    constexpr bool WHOLE = decltype(whole)::value != 0;
+    const int own = ns - k0;
+#pragma unroll
+    for (int k = 0; k < SUB; ++k) {
+      const int at = turn * SUB + k;
+      if (WHOLE || k0 + at < left) {
+        const float dt = __uint_as_float(o.terms[0][k * 2]), a = __uint_as_float(o.terms[0][k * 2 + 1]);
+        const float x = __uint_as_float(o.x[0][at]);
+        const float dx = dt * x;
+        float part = 0.0f;
+#pragma unroll
+        for (int i = 0; i < OWN; ++i) {
+          const float B = __uint_as_float(o.B[k][i / 4][i % 4]), C = __uint_as_float(o.C[k][i / 4][i % 4]);
+          S[i] = FULL || ns + SS_LANES * i < N ? fmaf(a, S[i], dx * B) : 0.0f;
+          part = fmaf(S[i], C, part);
+        }
+        part = ss_two_rows_sum(part);
+        kept_y = own == at ? fmaf(dskip, x, part) : kept_y;
+        if (SEGMENTS) {
+          decay *= a;
+          kept_decay = own == at ? decay : kept_decay;
+        }
+      }
+    }
+  };
+  // the outputs of the chunk before go out at the start of a chunk: they are on their way while it is worked on
+  auto put = [&](int at, int n) {
+    if (ns < n && has_p) y[(long)(at + ns) * inner + x_col] = kept_y;
+    if (SEGMENTS && blockIdx.z == 0 && (int)threadIdx.x < n) cum[(long)(at + ns) * heads + h] = kept_decay;
+  };
+
+  int buffer = 0;
+  for (int t0 = 0; t0 < count; t0 += SS_CHUNK) {
+    wait_vmcnt<0>();
+    __builtin_amdgcn_s_barrier();      // the chunk is in LDS for every wave; nobody reads the one before any more
+    const int left = min(SS_CHUNK, count - t0), ahead = t0 + SS_CHUNK;
+    const bool more = ahead < count;
+    const unsigned at = buffer * Chunk::FLOATS * 4;
+    if (t0 != 0) put(first + t0 - SS_CHUNK, SS_CHUNK);
+    if (more) ask_rest(buffer ^ 1, ahead);
+    SsStaged<OWN> even, odd;
+    if (left == SS_CHUNK) {
+      read(even, at, 0, 0);
+      arrived(even);
+#pragma unroll 1
+      for (int k0 = 0; k0 < SS_CHUNK; k0 += 2 * SUB) {      // no read is under way across a branch
+        read(odd, at, k0, 1);
+        work(even, k0, 0, left, SsNumber<1>());
+        arrived(odd);
+        if (more && k0 < SS_CHUNK / 2) ask(buffer ^ 1, ahead, 2 * k0, SsNumber<2 * SUB>());
+        read(even, at, k0 + 2 * SUB < SS_CHUNK ? k0 + 2 * SUB : 0, 0);
+        work(odd, k0, 1, left, SsNumber<1>());
+        arrived(even);
+        if (more && k0 < SS_CHUNK / 2) ask(buffer ^ 1, ahead, 2 * k0 + 2 * SUB, SsNumber<2 * SUB>());
+      }
+    } else {                                                // the last chunk: nothing is left to ask for
+#pragma unroll 1
+      for (int k0 = 0; k0 < left; k0 += 2 * SUB) {
+        read(even, at, k0, 0);
+        read(odd, at, k0, 1);                               // (places of the chunk that hold no token: not used)
+        arrived(even);
+        arrived(odd);
+        work(even, k0, 0, left, SsNumber<0>());
+        work(odd, k0, 1, left, SsNumber<0>());
+      }
+    }
+    buffer ^= 1;
+  }
+  put(first + (count - 1) / SS_CHUNK * SS_CHUNK, (count - 1) % SS_CHUNK + 1);
+  if (SEGMENTS) {                      // a segment's end state goes to the workspace; the fold brings the request's state up to date
+    float* end = ends + ((long)blockIdx.x * heads + h) * N * P;
+#pragma unroll
+    for (int i = 0; i < OWN; ++i) {
+      const int n = ns + SS_LANES * i;
+      if (has_p && n < N) end[(long)n * P + p] = S[i];
+    }
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < OWN; ++i) {
+    const int n = ns + SS_LANES * i;
+    if (has_p && n < N) to[s_at + (long)n * P + p] = S[i];
+  }
+  if (blockIdx.y == 0 && blockIdx.z == 0) ss_keep_inputs(from, to, tail_at, conv_in, conv_in_stride, first, count, channels, taps);
+}
+
+// Long stretches of tokens in segments.  The walk above then runs every segment of a request side by side:
 // the first from the request's state, the others from zero, each leaving its end state E_k in `ends` and
 // the running product of its tokens' a in `cum`.  Two more launches make the rest:
 //   the fold, per (request, head, eight value dims), over the request's segments in order: the state a
@@ -217,7 +389,9 @@ state_space_scan_kernel(const float* __restrict__ u, const float* __restrict__ t
 // The sums of a token then differ in order from the walk of one chain, by rounding, and which tokens share a
 // segment goes by how the request was cut into steps.
 // spans5 [n][5] = (slot, first token, tokens, first segment, segments).
+#define SS_THREADS 128      // of the fold and the carry: sixteen lanes a value dim
 #define SS_CARRY 32        // tokens of a segment a block of the carry takes
+#define SS_AHEAD 4         // tokens whose operands it asks for together
 template <int OWN>
 __global__ void __launch_bounds__(SS_THREADS)
 state_space_fold_kernel(float* __restrict__ ends, const float* __restrict__ cum, const int32_t* __restrict__ spans5,
@@ -258,15 +432,7 @@ state_space_fold_kernel(float* __restrict__ ends, const float* __restrict__ cum,
     const int n = ns + 16 * i;
     if (has_p && n < N) to[(long)h * N * P + (long)n * P + p] = I[i];
   }
-  if (blockIdx.y != 0 || blockIdx.z != 0) return;
-  float* kept = to + tail_at;
-  const float* kept_from = from + tail_at;
-  for (int c = threadIdx.x; c < channels; c += blockDim.x)
-    for (int i = 0; i < taps - 1; ++i) {
-      const int at = i + count;
-      kept[(long)i * channels + c] = at < taps - 1 ? kept_from[(long)at * channels + c]
-                                                   : conv_in[(long)(first + at - (taps - 1)) * conv_in_stride + c];
-    }
+  if (blockIdx.y == 0 && blockIdx.z == 0) ss_keep_inputs(from, to, tail_at, conv_in, conv_in_stride, first, count, channels, taps);
 }
 
 template <int OWN>
@@ -403,18 +569,27 @@ extern "C" int axk_state_space_scan(const float* u, const float* terms, const vo
   const int pieces = segs ? ceil_div(longest_seg, SS_CARRY) : 1;
   dim3 grid_carry((unsigned)((long)(segs ? n_segs : 1) * pieces), heads, ceil_div(vdim, SS_THREADS / 16));
   hipStream_t s = (hipStream_t)stream;
-#define SS_ARGS u, terms, d_skip, d_is_f32, state, state_stride, copy_elems, tail_at, spans, positions, seq_rows, conv_in, conv_in_stride, y, \
-                heads, groups, vdim, n_state, channels, taps, segs, ends, cum
 #define SS_LAUNCH(OWN)                                                                              \
   {                                                                                                 \
-    if (n_state == 16 * OWN) state_space_scan_kernel<OWN, true><<<grid, SS_THREADS, 0, s>>>(SS_ARGS); \
-    else state_space_scan_kernel<OWN, false><<<grid, SS_THREADS, 0, s>>>(SS_ARGS);                  \
+    if (spans == nullptr)                                                                           \
+      state_space_step_kernel<(OWN + 1) / 2><<<grid, SS_WALKERS, 0, s>>>(u, terms, d_skip, d_is_f32, state, state_stride, copy_elems, tail_at, \
+                                                               positions, seq_rows, conv_in, conv_in_stride, y, heads, groups, vdim, \
+                                                               n_state, channels, taps);            \
+    else if (segs) {                                                                                \
+      if (n_state == SS_LANES * ((OWN + 1) / 2)) state_space_walk_kernel<(OWN + 1) / 2, true, true><<<grid, SS_WALKERS, 0, s>>>(SS_ARGS); \
+      else state_space_walk_kernel<(OWN + 1) / 2, false, true><<<grid, SS_WALKERS, 0, s>>>(SS_ARGS);          \
+    } else {                                                                                        \
+      if (n_state == SS_LANES * ((OWN + 1) / 2)) state_space_walk_kernel<(OWN + 1) / 2, true, false><<<grid, SS_WALKERS, 0, s>>>(SS_ARGS); \
+      else state_space_walk_kernel<(OWN + 1) / 2, false, false><<<grid, SS_WALKERS, 0, s>>>(SS_ARGS);         \
+    }                                                                                               \
     if (segs) {                                                                                     \
       state_space_fold_kernel<OWN><<<grid_fold, SS_THREADS, 0, s>>>(ends, cum, spans5, segs, state, state_stride, copy_elems, tail_at, \
                                                                     positions, conv_in, conv_in_stride, heads, vdim, n_state, channels, taps); \
       state_space_carry_kernel<OWN><<<grid_carry, SS_THREADS, 0, s>>>(u, ends, cum, segs, y, heads, groups, vdim, n_state, channels, pieces); \
     }                                                                                               \
   }
+#define SS_ARGS u, terms, d_skip, d_is_f32, state, state_stride, copy_elems, tail_at, spans, positions, conv_in, conv_in_stride, y, \
+                heads, groups, vdim, n_state, channels, taps, segs, ends, cum
   if (n_state <= 16) SS_LAUNCH(1)
   else if (n_state <= 32) SS_LAUNCH(2)
   else if (n_state <= 64) SS_LAUNCH(4)

@@ -55,7 +55,9 @@ def unwaited(assembly, kernel):
 
 @pytest.mark.skipif(shutil.which("hipcc") is None and not os.path.exists("/opt/rocm/bin/hipcc"), reason="no compiler")
 @pytest.mark.parametrize("source, kernel", [("grouped_gemm.hip", "grouped_gemm_tile_kernel"),
-                                            ("latent_attention.hip", "latent_attention_prompt_kernel")])
+                                            ("latent_attention.hip", "latent_attention_prompt_kernel"),
+                                            ("gemm_mfma.hip", "gemm_tile_kernel"),
+                                            ("state_space.hip", "state_space_walk_kernel")])
 def test_nothing_comes_between_a_read_and_its_wait(tmp_path, source, kernel):
     out = tmp_path / "device.s"
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
