@@ -145,3 +145,29 @@ def test_attention_finds_loud_keys_across_9000_positions(hd, page):
     for h, p in enumerate(far):
         assert (got[h] - vb[p, 0].double()).abs().max() < 2e-2, (h, p)
     assert torch.equal(prompt[T - 1], decoded[T - 1])
+
+
+@pytest.mark.parametrize("hd,page,window", [(128, 64, 0), (64, 16, 0), (128, 16, 700)])
+def test_the_fold_of_a_decoding_token_at_the_edges_of_its_rounds(hd, page, window):
+    """Contexts that end in and beside the 16th, 32nd, 48th, 64th, 80th and 128th block of 64 positions, as one decoding
+    batch: the fold holds the first 64 blocks' values in rounds of 16, takes the others in rounds behind them and groups of
+    head size many; each row must have the bits that the prompt kernel gives the same token."""
+    k = kernels("bfloat16")
+    nh, nkv, T = 4, 2, 9300
+    g = torch.Generator().manual_seed(hd + page)
+    q, kk = torch.randn(T, nh, hd, generator=g).bfloat16(), torch.randn(T, nkv, hd, generator=g)
+    vv = torch.randn(T, nkv, hd, generator=g)
+    kc, vc, table = paged_cache(kk.bfloat16().double(), vv.bfloat16().double(), page, "bfloat16", seed=4)
+    ends = [0, 63, 64, 1023, 1024, 1087, 1088, 2047, 2048, 3071, 3136, 4031, 4032, 4095, 4096, 4159, 4160, 5119, 5184, 8191, 8192, 8256, 9299]
+    pos, rows = torch.arange(T, dtype=torch.int32).cuda(), torch.zeros(T, dtype=torch.int32).cuda()
+    qd = q.cuda().view(T, nh * hd)
+    chunks = -(-T // k.attention_decode_chunk)
+    partial = torch.full((k.attention_decode_workspace(len(ends), nh, hd, chunks),), float("nan"), device="cuda")   # nothing else is read
+    decoded, prompt = (torch.zeros(T, nh * hd, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    k.attention_decode(qd, nh * hd, kc, vc, table, pos, rows, decoded, torch.tensor(ends, dtype=torch.int32).cuda(), partial, chunks,
+                       nh, nkv, hd, page, window, hd ** -0.5)
+    for e in ends:
+        first = max(0, e - 3)
+        k.attention_prefill(qd, nh * hd, kc, vc, table, pos, rows, prompt, torch.tensor([[first, e + 1 - first]], dtype=torch.int32).cuda(),
+                            nh, nkv, hd, page, window, hd ** -0.5)
+    assert torch.equal(decoded[ends], prompt[ends])
