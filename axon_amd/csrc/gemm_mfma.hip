@@ -34,7 +34,7 @@
 //   same segment of K and share X through LDS; a block a segment, the sums of several segments
 //   through a workspace.
 //
-// * gemm_tile (M > 128): a block of 4 or 8 waves owns a BM x BN tile of the output, walks K in
+// * gemm_tile (M > 128; gemm_small_tile where the tiles are small and a block takes a segment): a block of 4 or 8 waves owns a BM x BN tile of the output, walks K in
 //   steps of 32 through LDS stages filled by direct global -> LDS loads (the next steps' loads
 //   in flight while this one multiplies), and each wave keeps a tile of MFMA accumulators.  With S > 1 segments each goes to blocks of its own (gridDim.y = S), whose sums
 //   go through a workspace and are added in segment order by gemm_split_reduce, which also
@@ -444,6 +444,265 @@ gemm_tile_kernel(const bf16_t* __restrict__ x, int x_stride, const bf16_t* __res
   }
 }
 
+// ---------------------------------------------------------------------------- gemm_small_tile
+// 128 x 128 outputs a block of four waves whose segments go to blocks of their own: products of some hundred rows, which wait
+// for their loads and barriers more than for the matrix cores or the card's power.  K tiles of 64 (one barrier for twice
+// the products of gemm_tile's stages), STAGES of them, every load of a stage issued at once when its place is free; 32x32x16
+// products (two of them give the bits of a 16x16x32 one).  us, here and with gemm_tile's walk: 3,584 columns of K 18,944 at
+// 256 rows 52 / 72, at 1,525 rows 259 / 292; of K 3,584 at 140 rows 18 / 23, at 1,024 52 / 58; gated 13,824 of K 5,120 at 256
+// rows 98 / 117; 2,048 of K 2,048 at 1,525 rows 33 / 35.
+typedef __attribute__((ext_vector_type(16))) float f32x16;
+template <bool GLU, int STAGES>
+__global__ void __launch_bounds__(256, 1)
+gemm_small_tile_kernel(const bf16_t* __restrict__ x, int x_stride, const bf16_t* __restrict__ w, const void* __restrict__ bias,
+                 int bias_is_f32, void* __restrict__ out, int out_stride, int M, int N, int K, int mode, int m_blocks,
+                       int n_blocks, float* __restrict__ partial) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  constexpr int BM = 128, BN = 128, WAVES_M = 2, WAVES_N = 2, BK = 64;
+  constexpr int NW = WAVES_M * WAVES_N;
+  constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N;  // a wave's tile
+  constexpr int TM = WM / 32, TN = WN / 32;            // in 32 x 32 MFMA tiles
+  constexpr int ROW = BK * 2;                          // bytes of a row
+  constexpr int SLOTS = BK / 8;                        // 16-byte slots of a row
+  constexpr int RPI = 1024 / ROW;                      // rows one wave instruction fills
+  constexpr int KBT = BK / 32;                         // packed k blocks of a K tile
+  constexpr int XQ = BM / RPI / NW, WQ = BN / 16 * KBT / NW;  // load instructions per wave and stage
+  constexpr int STAGE = (BM + BN) * ROW;               // bytes per stage
+  static_assert(XQ >= 1 && WQ >= 1 && (STAGES - 2) * (XQ + WQ) < 64, "tile too small or too many loads in flight");
+  static_assert(BN / 16 * KBT % NW == 0 && WN % 32 == 0, "the 1 KB chunks of W are shared out evenly");
+  static_assert(!GLU || TN % 2 == 0, "a wave's gate columns and up columns are whole MFMA tiles");
+#define SWZ(row) (((row) >> 1) & 7)
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wm = wave / WAVES_N, wn = wave % WAVES_N;
+
+  // (block numbering as in gemm_tile_kernel)
+  const int bid = blockIdx.x;
+  int mb, nb;
+  if (bid < (n_blocks / 8) * 8 * m_blocks) {
+    constexpr int GM = 8, GN = 4;
+    const int xcd = bid & 7, j = bid >> 3, mine = n_blocks / 8;       // this XCD's n blocks: xcd, xcd + 8, ...
+    const int whole_groups = mine / GN;
+    int g = j / (GN * m_blocks), rest = j % (GN * m_blocks), gn = GN;
+    if (g >= whole_groups) {                                          // the last, narrower group of n blocks
+      g = whole_groups;
+      rest = j - whole_groups * GN * m_blocks;
+      gn = mine - whole_groups * GN;
+    }
+    const int whole_rows = m_blocks / GM;
+    int ms = rest / (gn * GM), r = rest % (gn * GM), gm = GM;
+    if (ms >= whole_rows) {                                           // the last, shorter square
+      ms = whole_rows;
+      r = rest - whole_rows * gn * GM;
+      gm = m_blocks - whole_rows * GM;
+    }
+    mb = ms * GM + r % gm;
+    nb = (g * GN + r / gm) * 8 + xcd;
+  } else {  // the last, incomplete group of n blocks: plain order
+    const int r = bid - (n_blocks / 8) * 8 * m_blocks;
+    nb = (n_blocks / 8) * 8 + r / m_blocks;
+    mb = r % m_blocks;
+  }
+  const int m0 = mb * BM, n0 = nb * (GLU ? BN / 2 : BN);
+
+  // what this lane fetches: row r = (q * NW + wave) * RPI + lane / SLOTS of a tile; it fills slot
+  // lane % SLOTS of that row, which holds k chunk (lane % SLOTS) ^ SWZ(r)
+  const int lrow = lane / SLOTS, lslot = lane % SLOTS;
+  unsigned xoff[XQ], woff[WQ];
+#pragma unroll
+  for (int q = 0; q < XQ; ++q) {
+    const int r = (q * NW + wave) * RPI + lrow;
+    xoff[q] = (unsigned)min(m0 + r, M - 1) * (unsigned)x_stride + (lslot ^ SWZ(r)) * 8;
+  }
+  // W: chunk c = q * NW + wave of a stage is the packed block (row tile c / KBT, k block c % KBT)
+  // of the tile, 1 KB as it lies in memory.  Row tiles past the matrix: its last one (the
+  // epilogue drops those columns).
+  const int KB = K / 32;
+  const int row_tiles = GLU ? N / 16 : (N + 15) / 16;          // GLU: per half, N a multiple of 16
+#pragma unroll
+  for (int q = 0; q < WQ; ++q) {
+    const int c = q * NW + wave;
+    const int r = (c / KBT) * 16;                               // first row of the chunk in the LDS tile
+    int tile;
+    if (GLU) {
+      const int owner = r / WN, within = r % WN;                // the wave whose columns these are
+      const int col = n0 + owner * (WN / 2) + within % (WN / 2);
+      tile = (within >= WN / 2 ? row_tiles : 0) + min(col / 16, row_tiles - 1);   // up rows follow the N gate rows
+    } else {
+      tile = min((n0 + r) / 16, row_tiles - 1);
+    }
+    woff[q] = ((unsigned)tile * (unsigned)KB + (c % KBT)) * 512 + lane * 8;
+  }
+
+  // Split K (gridDim.y > 1): this block multiplies the K tiles kt_begin .. kt_begin + nk - 1 and
+  // leaves its sums in `partial`; gemm_split_reduce_kernel adds the blocks' sums in block order.
+  const int kt_begin = (int)((long)blockIdx.y * (K / 64) / gridDim.y);
+  const int nk = (int)((long)(blockIdx.y + 1) * (K / 64) / gridDim.y) - kt_begin;
+  auto issue = [&](int kt) {     // kt counts from kt_begin
+    unsigned char* stage = smem + (kt % STAGES) * STAGE;
+    const int koff = (kt_begin + kt) * BK;
+#pragma unroll
+    for (int q = 0; q < XQ; ++q)
+      __builtin_amdgcn_global_load_lds((global_ptr_t)(x + xoff[q] + koff), (lds_ptr_t)(stage + (q * NW + wave) * 1024), 16,
+                                       0, 0);
+#pragma unroll
+    for (int q = 0; q < WQ; ++q)
+      __builtin_amdgcn_global_load_lds((global_ptr_t)(w + woff[q] + (kt_begin + kt) * (KBT * 512)),
+                                       (lds_ptr_t)(stage + BM * ROW + (q * NW + wave) * 1024), 16, 0, 0);
+  };
+
+  f32x16 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+
+  // fragment addresses: row = tile row + lane % 32, k chunk = 2 ks + lane / 32, slot = chunk ^ SWZ(row)
+  const int frow = lane & 31, fhalf = lane >> 5, fsw = SWZ(frow);
+  const unsigned lds0 = (unsigned)(size_t)(lds_ptr_t)smem;
+  const unsigned xbase = lds0 + (wm * WM + frow) * ROW;
+  // W fragment of k step ks: block (row tile of the lane's row, k block ks / 2), lane slot
+  // 16 (2 (ks % 2) + lane / 32) + row % 16 of it: no permutation, 16 lanes read 256 consecutive bytes
+  const unsigned wbase = lds0 + BM * ROW + ((wn * WN + frow) / 16) * KBT * 1024 + (fhalf * 16 + (frow & 15)) * 16;
+  // The fragments of k step ks of a stage into one of two register sets.  The reads are written
+  // as instructions: the compiler, which cannot tell the stage being read from the stage a
+  // direct load is filling, would wait for every load in flight before each of its own reads,
+  // and the loads of the next tile would never overlap the products of this one.
+  u32x4 a[2][TM], b[2][TN];
+  auto read_step = [&](int set, int stage_index, int ks) {
+    read_frags<TM, 32 * ROW>(a[set], xbase + stage_index * STAGE + ((((ks * 2 + fhalf) ^ fsw)) << 4));
+    read_frags<TN, 2 * KBT * 1024>(b[set], wbase + stage_index * STAGE + (ks / 2) * 1024 + (ks % 2) * 512);
+  };
+  auto multiply = [&](int set, int j_from, int j_to) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = j_from; j < j_to; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_frag(a[set][i]), as_frag(b[set][j]), acc[i][j], 0, 0, 0);
+  };
+
+  // Every stage is filled before the loop; tile kt + STAGES is fetched into tile kt's stage as
+  // soon as every wave has read that tile's last fragments, which is during its last k step:
+  // the wait for the next tile, the barrier and the first reads of the next tile are hidden
+  // behind that step's products (half of them before the barrier, half after the reads).
+  constexpr int KS = BK / 16;
+  static_assert(KS % 2 == 0, "the register sets alternate and start a tile at set 0");
+#pragma unroll
+  for (int d = 0; d < STAGES; ++d)
+    if (d < nk) issue(d);
+  if (nk >= STAGES) wait_vmcnt<(STAGES - 1) * (XQ + WQ)>();
+  else wait_vmcnt<0>();
+  __builtin_amdgcn_s_barrier();   // tile 0 is in LDS for every wave
+  read_step(0, 0, 0);
+  for (int kt = 0; kt < nk; ++kt) {
+    const int stage_index = kt % STAGES;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const int cur = ks & 1, nxt = cur ^ 1;
+      if (ks + 1 < KS) {
+        read_step(nxt, stage_index, ks + 1);
+        wait_lgkmcnt<TM + TN>();          // this step's fragments (reads return in order)
+        use_frags<TM>(a[cur]);
+        use_frags<TN>(b[cur]);
+        multiply(cur, 0, TN);
+      } else {
+        wait_lgkmcnt<0>();                // the last fragments of this tile: its stage is free
+        use_frags<TM>(a[cur]);
+        use_frags<TN>(b[cur]);
+        multiply(cur, 0, TN / 2);
+        if (kt + 1 < nk) {
+          // this wave's part of tile kt + 1 has landed when only younger tiles are outstanding
+          if (kt + STAGES < nk) wait_vmcnt<(STAGES - 2) * (XQ + WQ)>();
+          else wait_vmcnt<0>();
+          __builtin_amdgcn_s_barrier();   // tile kt + 1 is in LDS for every wave; nobody reads tile kt any more
+          if (kt + STAGES < nk) issue(kt + STAGES);
+          read_step(nxt, (kt + 1) % STAGES, 0);
+        }
+        multiply(cur, TN / 2, TN);
+      }
+    }
+  }
+#undef SWZ
+  // epilogue: lane holds column n = lane % 32 of each tile and rows (e/4)*8 + (lane/32)*4 + e%4
+  if (partial) {
+    // [split][gate | up][M][N] (one part without GLU), 32-bit sums as they are
+    constexpr int PARTS = GLU ? 2 : 1;
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const int part = GLU ? j / (TN / 2) : 0;
+      const int n = GLU ? n0 + wn * (WN / 2) + (j % (TN / 2)) * 32 + (lane & 31) : n0 + wn * WN + j * 32 + (lane & 31);
+      if (n >= N) continue;
+      float* dst = partial + ((size_t)blockIdx.y * PARTS + part) * M * N + n;
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const int m = m0 + wm * WM + i * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
+          if (m < M) dst[(size_t)m * N] = acc[i][j][e];
+        }
+    }
+    return;
+  }
+  if (GLU) {
+#pragma unroll
+    for (int j = 0; j < TN / 2; ++j) {
+      const int n = n0 + wn * (WN / 2) + j * 32 + (lane & 31);
+      if (n >= N) continue;
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const int m = m0 + wm * WM + i * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
+          if (m >= M) continue;
+          reinterpret_cast<bf16_t*>(out)[(size_t)m * out_stride + n] =
+              float_to_bf16(swiglu1(acc[i][j][e], acc[i][j + TN / 2][e]));
+        }
+      }
+    }
+    return;
+  }
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+    const int n = n0 + wn * WN + j * 32 + (lane & 31);
+    if (n >= N) continue;
+    const float bv = bias ? load_vec(bias, bias_is_f32, n) : 0.0f;
+    if (mode == MODE_ADD_F32) {
+      // all reads before the first store, which may alias the next read; rows past M read the last row and store nothing
+      float* rows = reinterpret_cast<float*>(out) + n;
+      float before[TM][16];
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const int m = m0 + wm * WM + i * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
+          before[i][e] = rows[(size_t)min(m, M - 1) * out_stride];
+        }
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const int m = m0 + wm * WM + i * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
+          if (m < M) rows[(size_t)m * out_stride] = before[i][e] + (acc[i][j][e] + bv);
+        }
+      continue;
+    }
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int m = m0 + wm * WM + i * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
+        if (m >= M) continue;
+        const float v = acc[i][j][e] + bv;
+        const size_t at = (size_t)m * out_stride + n;
+        if (mode_stores_elem(mode)) reinterpret_cast<bf16_t*>(out)[at] = float_to_bf16(mode_value(v, mode));
+        else reinterpret_cast<float*>(out)[at] = v;
+      }
+    }
+  }
+}
+
 // The same for a width that is no multiple of 4 (rows of the workspace are then not 16-byte
 // aligned): a thread an element, the same additions in the same order.  No gated epilogue here: a
 // [gate; up] matrix has whole row tiles.
@@ -650,12 +909,14 @@ static int launch_tile(const bf16_t* x, int x_stride, const bf16_t* w, const voi
                        int out_stride, int m, int n, int k, int mode, hipStream_t stream, int segs = 1,
                        float* partial = nullptr, const SplitNorm* norm = nullptr, const RopeStore* rope = nullptr) {
   static bool configured = false;
-  constexpr int lds_bytes = STAGES * (BM + BN) * 64;
+  constexpr bool SMALL = BM == 128 && !KEEP;           // (kept segments fill the chip: 5,632 columns of K 2,048 at 688 rows 42 -> 37 us)
+  constexpr int lds_bytes = STAGES * (BM + BN) * (SMALL ? 128 : 64);
   static_assert(lds_bytes <= 160 * 1024, "the stages do not fit the LDS of a CU");
-  auto kernel = &gemm_tile_kernel<BM, BN, WAVES_M, WAVES_N, GLU, STAGES, KEEP>;
+  const void* kernel;
+  if constexpr (SMALL) kernel = reinterpret_cast<const void*>(&gemm_small_tile_kernel<GLU, STAGES>);
+  else kernel = reinterpret_cast<const void*>(&gemm_tile_kernel<BM, BN, WAVES_M, WAVES_N, GLU, STAGES, KEEP>);
   if (!configured) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       lds_bytes);
+    hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
     if (e != hipSuccess) {
       axk_set_error("gemm_tile: cannot reserve %d bytes of LDS: %s", lds_bytes, hipGetErrorString(e));
       return -2;
@@ -668,9 +929,15 @@ static int launch_tile(const bf16_t* x, int x_stride, const bf16_t* w, const voi
   const bool after = splits > 1 || norm || rope;
   const int m_blocks = ceil_div(m, BM), n_blocks = ceil_div(n, GLU ? BN / 2 : BN);
   if constexpr (KEEP) AXK_INSTANCE(INST_GEMM_KEPT, GLU);
-  else AXK_INSTANCE(INST_GEMM_TILE, BM, BN, WAVES_M, WAVES_N, GLU, STAGES / 2);
-  kernel<<<dim3(m_blocks * n_blocks, splits), WAVES_M * WAVES_N * 64, lds_bytes, stream>>>(
-      x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode, m_blocks, n_blocks, after ? partial : nullptr, segs);
+  else AXK_INSTANCE(INST_GEMM_TILE, BM, BN, WAVES_M, WAVES_N, GLU, SMALL ? STAGES : STAGES / 2);
+  const dim3 grid(m_blocks * n_blocks, splits);
+  float* sums = after ? partial : nullptr;
+  if constexpr (SMALL)
+    gemm_small_tile_kernel<GLU, STAGES><<<grid, 256, lds_bytes, stream>>>(x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode,
+                                                                          m_blocks, n_blocks, sums);
+  else
+    gemm_tile_kernel<BM, BN, WAVES_M, WAVES_N, GLU, STAGES, KEEP><<<grid, WAVES_M * WAVES_N * 64, lds_bytes, stream>>>(
+        x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode, m_blocks, n_blocks, sums, segs);
   AXK_LAUNCH_CHECK("gemm_tile");
   return after ? add_split_sums(partial, splits, m, n, bias, bias_is_f32, out, out_stride, mode, norm, rope, stream) : 0;
 }
@@ -708,81 +975,144 @@ enum { EPI_PLAIN = 0, EPI_GLU = 1, EPI_ROPE = 2 };
 
 // The sums of a split [q; k; v] product with the bias, the rotary encoding and the store into the
 // pages: what gemm_split_reduce_kernel (storing bfloat16) and the rotary kernel do one after the
-// other, bit for bit.  A block per token and group of head slots; a thread takes 4 consecutive dims
+// other, bit for bit.  A block per TOKENS tokens and group of head slots; a thread takes 4 consecutive dims
 // of a head's lower half and their partners in the upper half (every load a float4, all of a
 // thread's loads independent of each other); q heads go rotated to `out`, k heads rotated into the
 // request's page of keys, v heads as they are into its page of values.  Every head is rotated
 // over its whole width.
+//
+// Bound by memory once the stores of V are: values lie [dim][slot], so a token alone writes two bytes of a line that
+// seven other XCDs write their two bytes of.  A thread of the prompt form keeps eight neighbouring tokens and writes a
+// dim's eight slots at once where they are eight of one page (token by token where a request ends among them or the
+// tokens are not aligned to the page): 2,048 tokens of 36 heads, one sum each, 23.2 -> 17.2 us, 1,525 of 56, four sums each, 49 -> 45.
+template <int TOKENS>
 __global__ void __launch_bounds__(256)
 gemm_split_reduce_rope_kernel(const float* __restrict__ partial, int splits, int M, int N, const void* __restrict__ bias,
                               int bias_is_f32, bf16_t* __restrict__ out, int out_stride, RopeStore rope) {
   const int hd = rope.head_dim, half = hd / 2, per_head = half / 4;     // threads a head
   const int heads_a_block = 256 / per_head;
-  const int m = blockIdx.x, within = threadIdx.x / per_head, slot = blockIdx.y * heads_a_block + within;
+  const int m0 = blockIdx.x * TOKENS, within = threadIdx.x / per_head, slot = blockIdx.y * heads_a_block + within;
   const int d = (threadIdx.x % per_head) * 4;
   if (within >= heads_a_block || slot * hd >= N) return;
   const size_t plane = (size_t)M * N;
-  // four columns' sums, rounded as the product's own store rounds them
-  auto values = [&](int col, float (&v)[4]) {
-    const float* src = partial + (size_t)m * N + col;
-    float4 g = *reinterpret_cast<const float4*>(src);
-    for (int z = 1; z < splits; ++z) {
-      const float4 a = *reinterpret_cast<const float4*>(src + (size_t)z * plane);
-      g.x += a.x; g.y += a.y; g.z += a.z; g.w += a.w;
+  const int col = slot * hd + d;
+  // four columns' sums of every token (of tokens past the last the last's again), rounded as the product's own store
+  // rounds them
+  float a[TOKENS][4], b[TOKENS][4];
+  {
+    f32x4 lo[TOKENS], hi[TOKENS];
+#pragma unroll
+    for (int t = 0; t < TOKENS; ++t) {
+      const float* src = partial + (size_t)min(m0 + t, M - 1) * N + col;
+      lo[t] = *reinterpret_cast<const f32x4*>(src);
+      hi[t] = *reinterpret_cast<const f32x4*>(src + half);
     }
-    v[0] = g.x; v[1] = g.y; v[2] = g.z; v[3] = g.w;
+    for (int z = 1; z < splits; ++z) {
+#pragma unroll
+      for (int t = 0; t < TOKENS; ++t) {
+        const float* src = partial + (size_t)z * plane + (size_t)min(m0 + t, M - 1) * N + col;
+        lo[t] += *reinterpret_cast<const f32x4*>(src);
+        hi[t] += *reinterpret_cast<const f32x4*>(src + half);
+      }
+    }
+    float bl[4], bh[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      if (bias) v[e] += load_vec(bias, bias_is_f32, col + e);
-      v[e] = bf16_to_float(float_to_bf16(v[e]));
+      bl[e] = bias ? load_vec(bias, bias_is_f32, col + e) : 0.0f;
+      bh[e] = bias ? load_vec(bias, bias_is_f32, col + half + e) : 0.0f;
     }
-  };
-  float a[4], b[4];
-  values(slot * hd + d, a);
-  values(slot * hd + half + d, b);
-  bf16_t* dst;
-  if (slot < rope.n_heads) {
-    dst = out + (size_t)m * out_stride + (size_t)slot * hd;
-  } else {
-    const int pos = rope.positions[m];
-    const int page = rope.block_table[(size_t)rope.seq_rows[m] * rope.table_stride + pos / rope.page_size];
-    const int in_page = pos % rope.page_size;
-    if (slot >= rope.n_heads + rope.n_kv_heads) {
-      const int kvh = slot - rope.n_heads - rope.n_kv_heads;
-      bf16_t* vdst = rope.v_cache + ((size_t)page * rope.n_kv_heads + kvh) * hd * rope.page_size + in_page;
+#pragma unroll
+    for (int t = 0; t < TOKENS; ++t)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        vdst[(size_t)(d + e) * rope.page_size] = float_to_bf16(a[e]);
-        vdst[(size_t)(half + d + e) * rope.page_size] = float_to_bf16(b[e]);
+        a[t][e] = bf16_to_float(float_to_bf16(bias ? lo[t][e] + bl[e] : lo[t][e]));
+        b[t][e] = bf16_to_float(float_to_bf16(bias ? hi[t][e] + bh[e] : hi[t][e]));
       }
-      return;
-    }
-    dst = rope.k_cache + (((size_t)page * rope.n_kv_heads + (slot - rope.n_heads)) * rope.page_size + in_page) * hd;
   }
-  const float4* tab = reinterpret_cast<const float4*>(rope.table + ((size_t)m * half + d) * 2);
-  const float4 t0 = tab[0], t1 = tab[1];
-  const float sn[4] = {t0.x, t0.z, t1.x, t1.z}, cs[4] = {t0.y, t0.w, t1.y, t1.w};
-  float lo[4], hi[4];
+  int pos[TOKENS], page[TOKENS];
+  if (slot >= rope.n_heads) {
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    lo[e] = __fsub_rn(__fmul_rn(a[e], cs[e]), __fmul_rn(b[e], sn[e]));
-    hi[e] = __fadd_rn(__fmul_rn(a[e], sn[e]), __fmul_rn(b[e], cs[e]));
+    for (int t = 0; t < TOKENS; ++t) {
+      const int m = min(m0 + t, M - 1);
+      pos[t] = rope.positions[m];
+      page[t] = rope.block_table[(size_t)rope.seq_rows[m] * rope.table_stride + pos[t] / rope.page_size];
+    }
   }
-  uint2 pk;
-  pk.x = pack2_bf16(lo[0], lo[1]);
-  pk.y = pack2_bf16(lo[2], lo[3]);
-  *reinterpret_cast<uint2*>(dst + d) = pk;
-  pk.x = pack2_bf16(hi[0], hi[1]);
-  pk.y = pack2_bf16(hi[2], hi[3]);
-  *reinterpret_cast<uint2*>(dst + half + d) = pk;
+  if (slot >= rope.n_heads + rope.n_kv_heads) {
+    const int kvh = slot - rope.n_heads - rope.n_kv_heads;
+    const size_t head_at = (size_t)kvh * hd * rope.page_size, page_elems = (size_t)rope.n_kv_heads * hd * rope.page_size;
+    if (TOKENS == 8) {
+      // eight slots of one page, as 16 bytes of a dim (the pages' dims are then 16-byte aligned)
+      bool whole = m0 + TOKENS <= M && rope.page_size % 8 == 0 && pos[0] % 8 == 0 && ((uintptr_t)rope.v_cache & 15) == 0;
+#pragma unroll
+      for (int t = 1; t < TOKENS; ++t) whole = whole && pos[t] == pos[0] + t && page[t] == page[0];
+      if (whole) {
+        bf16_t* vdst = rope.v_cache + (size_t)page[0] * page_elems + head_at + pos[0] % rope.page_size;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          uint4 lo, hi;
+          lo.x = pack2_bf16(a[0][e], a[1 % TOKENS][e]);
+          lo.y = pack2_bf16(a[2 % TOKENS][e], a[3 % TOKENS][e]);
+          lo.z = pack2_bf16(a[4 % TOKENS][e], a[5 % TOKENS][e]);
+          lo.w = pack2_bf16(a[6 % TOKENS][e], a[7 % TOKENS][e]);
+          hi.x = pack2_bf16(b[0][e], b[1 % TOKENS][e]);
+          hi.y = pack2_bf16(b[2 % TOKENS][e], b[3 % TOKENS][e]);
+          hi.z = pack2_bf16(b[4 % TOKENS][e], b[5 % TOKENS][e]);
+          hi.w = pack2_bf16(b[6 % TOKENS][e], b[7 % TOKENS][e]);
+          *reinterpret_cast<uint4*>(vdst + (size_t)(d + e) * rope.page_size) = lo;
+          *reinterpret_cast<uint4*>(vdst + (size_t)(half + d + e) * rope.page_size) = hi;
+        }
+        return;
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < TOKENS; ++t) {
+      if (m0 + t >= M) break;
+      bf16_t* vdst = rope.v_cache + (size_t)page[t] * page_elems + head_at + pos[t] % rope.page_size;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        vdst[(size_t)(d + e) * rope.page_size] = float_to_bf16(a[t][e]);
+        vdst[(size_t)(half + d + e) * rope.page_size] = float_to_bf16(b[t][e]);
+      }
+    }
+    return;
+  }
+#pragma unroll
+  for (int t = 0; t < TOKENS; ++t) {
+    const int m = m0 + t;
+    if (m < M) {
+      bf16_t* dst = slot < rope.n_heads
+                        ? out + (size_t)m * out_stride + (size_t)slot * hd
+                        : rope.k_cache + (((size_t)page[t] * rope.n_kv_heads + (slot - rope.n_heads)) * rope.page_size +
+                                          pos[t] % rope.page_size) * hd;
+      const float4* tab = reinterpret_cast<const float4*>(rope.table + ((size_t)m * half + d) * 2);
+      const float4 t0 = tab[0], t1 = tab[1];
+      const float sn[4] = {t0.x, t0.z, t1.x, t1.z}, cs[4] = {t0.y, t0.w, t1.y, t1.w};
+      float lo[4], hi[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        lo[e] = __fsub_rn(__fmul_rn(a[t][e], cs[e]), __fmul_rn(b[t][e], sn[e]));
+        hi[e] = __fadd_rn(__fmul_rn(a[t][e], sn[e]), __fmul_rn(b[t][e], cs[e]));
+      }
+      *reinterpret_cast<uint2*>(dst + d) = make_uint2(pack2_bf16(lo[0], lo[1]), pack2_bf16(lo[2], lo[3]));
+      *reinterpret_cast<uint2*>(dst + half + d) = make_uint2(pack2_bf16(hi[0], hi[1]), pack2_bf16(hi[2], hi[3]));
+    }
+  }
 }
 
 static int launch_split_reduce_rope(const float* partial, int splits, int m, int n, const void* bias, int bias_is_f32,
                                     void* out, int out_stride, const RopeStore& rope, hipStream_t stream) {
   const int heads_a_block = 256 / (rope.head_dim / 8);
-  const dim3 grid(m, ceil_div(n / rope.head_dim, heads_a_block));
-  gemm_split_reduce_rope_kernel<<<grid, 256, 0, stream>>>(partial, splits, m, n, bias, bias_is_f32, (bf16_t*)out, out_stride,
-                                                          rope);
+  const int head_blocks = ceil_div(n / rope.head_dim, heads_a_block);
+  // Eight tokens a thread where that still is two and a half blocks a CU.  The product with its rotation, a token a thread
+  // against eight (us): 28 heads and 2 x 4 at 688 rows (258 blocks) 47 / 57, 16 and 2 x 2 at 1,024 (256) 34 / 46, at 2,048 (512)
+  // 48 / 50, 28 and 2 x 4 at 4,096 (1,536) 190 / 185.
+  if ((long)ceil_div(m, 8) * head_blocks >= 640)
+    gemm_split_reduce_rope_kernel<8><<<dim3(ceil_div(m, 8), head_blocks), 256, 0, stream>>>(partial, splits, m, n, bias, bias_is_f32,
+                                                                                            (bf16_t*)out, out_stride, rope);
+  else
+    gemm_split_reduce_rope_kernel<1><<<dim3(m, head_blocks), 256, 0, stream>>>(partial, splits, m, n, bias, bias_is_f32, (bf16_t*)out,
+                                                                               out_stride, rope);
   AXK_LAUNCH_CHECK("gemm_split_reduce_rope");
   return 0;
 }
@@ -1909,16 +2239,16 @@ static int gemm_mfma_pass(const bf16_t* x, int x_stride, const bf16_t* w, const 
   }
   if (!use_big) {
     // Up to 256 rows still wait for W more than for the matrix cores.  Where the small tiles are no
-    // more blocks than CUs, a block has its CU's LDS to itself: nine stages of 32 k instead of five
-    // (the down projection of a 7B layer at 256 rows: 64 us with four steps of 64 k, 79 with two); with
-    // more blocks two of them share a CU and cover each other's waits (more stages there: slower).
+    // more blocks than CUs, a block has its CU's LDS to itself: four stages instead of two, three
+    // steps of loads in flight (the down projection of a 7B layer at 256 rows 79 -> 64 us); with
+    // more blocks two of them share a CU and cover each other's waits (four stages there: slower).
     const bool deep = m <= 256 && small <= 256;
     if (glu) {
-      if (deep) return launch_tile<128, 128, 2, 2, true, 9>(ARGS, segs, ws);
-      return launch_tile<128, 128, 2, 2, true>(ARGS, segs, ws);
+      if (deep) return launch_tile<128, 128, 2, 2, true, 4>(ARGS, segs, ws);
+      return launch_tile<128, 128, 2, 2, true, 2>(ARGS, segs, ws);
     }
-    if (deep) return launch_tile<128, 128, 2, 2, false, 9>(ARGS, segs, ws, norm, rope_after);
-    return launch_tile<128, 128, 2, 2, false>(ARGS, segs, ws, norm, rope_after);
+    if (deep) return launch_tile<128, 128, 2, 2, false, 4>(ARGS, segs, ws, norm, rope_after);
+    return launch_tile<128, 128, 2, 2, false, 2>(ARGS, segs, ws, norm, rope_after);
   }
   if (glu) return launch_tile<256, 256, 4, 2, true>(ARGS, segs, ws);
   // one round of 256 x 256 tiles that leaves a quarter of the CUs idle, and N in whole tiles of
