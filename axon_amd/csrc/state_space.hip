@@ -76,13 +76,30 @@ __device__ inline float ss_row_sum(float v) {
   return v;
 }
 
-// The same over the thirty-two lanes of two neighbouring rows.
-__device__ inline float ss_two_rows_sum(float v) {
-  const unsigned r = __float_as_uint(ss_row_sum(v));
-  const auto s = __builtin_amdgcn_permlane16_swap(r, r, false, false);
-  const unsigned even = s[0], odd = s[1];
-  return __uint_as_float(even) + __uint_as_float(odd);
+// From the lanes of an even row of sixteen to those of the row behind it; zero in the even rows.
+__device__ inline float ss_hand_on(float v) {
+  const auto s = __builtin_amdgcn_permlane16_swap(0u, __float_as_uint(v), false, false);     // odd rows of the one, even rows of the other
+  const unsigned behind = s[0];
+  return __uint_as_float(behind);
 }
+
+// A value dim's N rows of the state lie in thirty-two lanes, two halves of sixteen, each with its ROWS rows a lane: lane l of
+// half f holds l + 16 (f ROWS + i).  A sum over n is sixteen partial chains l, l + 16, l + 32, ... in ascending n, folded in
+// a fixed order: the first half begins each chain, hands it on, and the second half ends it.  OWN: rows a chain has.
+template <int OWN>
+struct SsRows {
+  static constexpr int ROWS = OWN >= 2 ? OWN / 2 : 1;
+  static __device__ inline int row(int lane, int i) { return (lane & 15) + 16 * (lane / 16 * ROWS + i); }
+  // the chain goes on over this lane's rows (one row a chain: it has none in the second half)
+  static __device__ inline float chain(float part, int half, const float (&S)[ROWS], const float (&C)[ROWS]) {
+#pragma unroll
+    for (int i = 0; i < ROWS; ++i) {
+      const float on = fmaf(S[i], C[i], part);
+      part = OWN == 1 && half ? part : on;
+    }
+    return part;
+  }
+};
 
 // A request's kept inputs of the convolution behind `count` tokens of this step: of (what was kept, this step's inputs) the
 // last taps - 1; place i takes what lies `count` places later (where both copies are one: read before it is written,
@@ -100,12 +117,11 @@ __device__ inline void ss_keep_inputs(const float* from, float* to, long tail_at
 }
 
 // A decoding step.  grid (tokens, heads, blocks of 8 value dims), every token a request of its own in slot seq_rows[t]; a
-// block is 256 threads: thirty-two lanes side by side share a value dim p and hold the state's rows n = lane,
-// lane + 32, ... of that column (OWN each: N up to 32 OWN).  u [T, channels] = [x: heads P | B: groups N |
-// C: groups N] behind the convolution; terms [T, heads, 2] = (dt, a).  y [T, heads P] float32.  The block
-// (head 0, dims 0) also brings the convolution's kept inputs up to date from conv_in (the convolution's
-// inputs, float32 rows conv_in_stride apart).  A sum over n is thirty-two partial chains in ascending n
-// folded in a fixed order: the same for a token however the request was cut into steps.
+// block is 256 threads: thirty-two lanes side by side share a value dim p and hold that column of the state (N up to
+// 16 OWN rows) as SsRows says.  u [T, channels] = [x: heads P | B: groups N | C: groups N] behind the convolution;
+// terms [T, heads, 2] = (dt, a).  y [T, heads P] float32.  The block (head 0, dims 0) also brings the convolution's
+// kept inputs up to date from conv_in (the convolution's inputs, float32 rows conv_in_stride apart).  A token's sums do
+// not depend on how the request was cut into steps.
 #define SS_DIMS 8          // value dims a block
 #define SS_LANES 32
 #define SS_WALKERS (SS_DIMS * SS_LANES)
@@ -116,8 +132,10 @@ state_space_step_kernel(const float* __restrict__ u, const float* __restrict__ t
                         const int32_t* __restrict__ positions, const int32_t* __restrict__ seq_rows,
                         const float* __restrict__ conv_in, long conv_in_stride, float* __restrict__ y, int heads, int groups,
                         int P, int N, int channels, int taps) {
+  typedef SsRows<OWN> Rows;
+  constexpr int ROWS = Rows::ROWS;
   const int t = blockIdx.x, h = blockIdx.y, g = h / (heads / groups), slot = seq_rows[t];
-  const int ns = threadIdx.x % SS_LANES, p = blockIdx.z * SS_DIMS + threadIdx.x / SS_LANES;
+  const int lane = threadIdx.x % SS_LANES, half = lane / 16, p = blockIdx.z * SS_DIMS + threadIdx.x / SS_LANES;
   const bool has_p = p < P;
   const int start = positions[t];
   const float* from = state + (long)slot * state_stride + (long)((start + 1) & 1) * copy_elems;
@@ -129,52 +147,52 @@ state_space_step_kernel(const float* __restrict__ u, const float* __restrict__ t
   const float* C = B + (long)groups * N;
   const float x = row[x_col], dt = terms[((long)t * heads + h) * 2], a = terms[((long)t * heads + h) * 2 + 1];
   const float dskip = load_vec(d_skip, d_is_f32, h);
-  float S[OWN], Bs[OWN], Cs[OWN];
+  float S[ROWS], Bs[ROWS], Cs[ROWS];
 #pragma unroll
-  for (int i = 0; i < OWN; ++i) {
-    const int n = ns + SS_LANES * i, at = min(n, N - 1);       // rows beyond N: zeros in S, what they meet does not count
+  for (int i = 0; i < ROWS; ++i) {
+    const int n = Rows::row(lane, i), at = min(n, N - 1);      // rows beyond N: zeros in S, what they meet does not count
     S[i] = has_p && n < N ? from[s_at + (long)n * P + p] : 0.0f;
     Bs[i] = B[at];
     Cs[i] = C[at];
   }
   const float dx = dt * x;
-  float part = 0.0f;
 #pragma unroll
-  for (int i = 0; i < OWN; ++i) {
-    S[i] = ns + SS_LANES * i < N ? fmaf(a, S[i], dx * Bs[i]) : 0.0f;
-    part = fmaf(S[i], Cs[i], part);
-  }
-  part = ss_two_rows_sum(part);
-  if (ns == 0 && has_p) y[(long)t * inner + x_col] = fmaf(dskip, x, part);
+  for (int i = 0; i < ROWS; ++i) S[i] = Rows::row(lane, i) < N ? fmaf(a, S[i], dx * Bs[i]) : 0.0f;
+  const float begun = ss_hand_on(Rows::chain(0.0f, half, S, Cs));
+  const float part = ss_row_sum(Rows::chain(begun, half, S, Cs));
+  if (lane == 16 && has_p) y[(long)t * inner + x_col] = fmaf(dskip, x, part);
 #pragma unroll
-  for (int i = 0; i < OWN; ++i) {
-    const int n = ns + SS_LANES * i;
+  for (int i = 0; i < ROWS; ++i) {
+    const int n = Rows::row(lane, i);
     if (has_p && n < N) to[s_at + (long)n * P + p] = S[i];
   }
   if (blockIdx.y == 0 && blockIdx.z == 0) ss_keep_inputs(from, to, tail_at, conv_in, conv_in_stride, t, 1, channels, taps);
 }
 
 // The walk of stretches of tokens (a request's tokens of the step, or segments of them): the arithmetic and
-// the order of the kernel above, its operands through LDS.  SS_CHUNK tokens' B and C rows, the block's values
-// of x, and (dt, a) go to LDS by direct loads, a dword a lane, during the first half of the chunk before (one
-// barrier a chunk).  A lane's rows of B and C lie there side by side, so that it reads four at a time, conflict-
-// free, the operands of two tokens while the two before them are worked on.  A lane keeps the output of the
-// chunk's token that has its number; one store a chunk, while the next chunk is worked on.
-// What bounds it: a wave's own instructions and waits, a token after the other; more waves share a token's work,
-// and fewer of them are loads, than with sixteen lanes a value dim and a dword load a row of B and C a token (38
-// vector, 20 scalar and 17 memory instructions a token and wave, at 262 ns; here 125 to 135 ns).  32 heads of 64
-// dims, 128 rows, 2 groups (us, before and here): stretches of 311, 611 and 1,203 tokens 307 / 183, one of 1,024
-// 256 / 130, of 64 26 / 15, two of 1,024 270 / 142, 5 of 300 165 / 100, 32 of a token 44 / 41; 256 rows and 16
-// heads, 1,024 tokens 390 / 162; a decoding step of 8 tokens 17 / 13, of 32 44 / 36 (the kernel above).  Sixteen lanes
-// with the operands through LDS: 201 for the three stretches; two chunks ahead instead of one: 187.
+// the order of the kernel above, its operands through LDS.  The second half of a value dim's lanes is SS_BEHIND tokens behind
+// the first: in a turn the first begins the chains of token j while the second ends those of token j - 2, so that both halves
+// work in every turn and two neighbouring turns' chains do not wait for each other.
+// SS_CHUNK turns' B and C rows, the block's values of x, and (dt, a), each half's of its own token, go to LDS by direct
+// loads, a dword a lane, during the first half of the chunk before (one barrier a chunk).  A lane's rows of B and C lie
+// there side by side, so that it reads four at a time, conflict-free, the operands of two turns while the two before them
+// are worked on.  A lane of the second half keeps the output of the chunk's turn that has its number; one store a chunk,
+// while the next chunk is worked on.
+// What bounds it: a wave's own instructions and their latency, one token after the other (some 130 ns a turn).  32 heads of 64
+// dims, 128 rows, 2 groups, us, with sixteen lanes a value dim and a dword load a row of B and C a token / here: stretches of
+// 311, 611 and 1,203 tokens 308 / 196, one chain of 1,024 257 / 137, of 64 26 / 16, two of 1,024 270 / 155, five of 300 166 / 110,
+// 32 of a token 44 / 41; 256 rows and 16 heads, 1,024 tokens 390 / 179; a decoding step of 32 tokens 44 / 36 (the kernel
+// above).  Slower: one token behind (202 for the three stretches), two chunks ahead instead of one.  Thirty-two chains of half the
+// length take 183, but are other sums.
 #define SS_CHUNK 16
+#define SS_BEHIND 2
 template <int OWN>
 struct SsChunk {
-  static constexpr int QUADS = OWN >= 4 ? OWN / 4 : 1;          // reads of four of a lane's rows
-  static constexpr int ROWS = SS_LANES * QUADS * 4;             // floats a token's B (or C) takes (OWN < 4: places unused)
-  static constexpr int WAVES = SS_WALKERS / AXON_WAVE, PIECES = ROWS / 64;
-  static constexpr int PER = 2 * PIECES / WAVES;                // loads of a wave and token
-  static constexpr int X_AT = SS_CHUNK * 2 * ROWS, TERMS_AT = X_AT + SS_DIMS * SS_CHUNK, FLOATS = TERMS_AT + AXON_WAVE;
+  static constexpr int QUADS = SsRows<OWN>::ROWS >= 4 ? SsRows<OWN>::ROWS / 4 : 1;        // reads of four of a lane's rows
+  static constexpr int PLACES = SS_LANES * QUADS * 4;           // floats a turn's B (or C) takes (fewer than four rows: places unused)
+  static constexpr int WAVES = SS_WALKERS / AXON_WAVE, PIECES = PLACES / 64;
+  static constexpr int PER = 2 * PIECES / WAVES;                // loads of a wave and turn
+  static constexpr int X_AT = SS_CHUNK * 2 * PLACES, TERMS_AT = X_AT + 2 * SS_DIMS * SS_CHUNK, FLOATS = TERMS_AT + 4 * SS_CHUNK;
 };
 
 template <int V>
@@ -197,15 +215,20 @@ state_space_walk_kernel(const float* __restrict__ u, const float* __restrict__ t
                         int P, int N, int channels, int taps, const int32_t* __restrict__ segs, float* __restrict__ ends,
                         float* __restrict__ cum) {
   typedef SsChunk<OWN> Chunk;
-  constexpr int ROWS = Chunk::ROWS, QUADS = Chunk::QUADS, PER = Chunk::PER, WAVES = Chunk::WAVES, PIECES = Chunk::PIECES, SUB = 2;
-  static_assert(WAVES == 4 && SS_DIMS * SS_CHUNK == 2 * AXON_WAVE && 2 * SS_CHUNK <= AXON_WAVE, "who asks for the rest of a chunk");
+  typedef SsRows<OWN> Rows;
+  constexpr int ROWS = Rows::ROWS, PLACES = Chunk::PLACES, QUADS = Chunk::QUADS, PER = Chunk::PER, WAVES = Chunk::WAVES;
+  constexpr int PIECES = Chunk::PIECES, SUB = SS_BEHIND;
+  static_assert(WAVES == 4 && 2 * SS_DIMS * SS_CHUNK == WAVES * AXON_WAVE && 4 * SS_CHUNK == AXON_WAVE && PIECES % 2 == 0,
+                "who asks for what of a chunk");
+  static_assert(SUB == 2 && SS_CHUNK % (2 * SUB) == 0, "a turn's pair goes by the chunk's turn");
   __shared__ __align__(16) float lds[2][Chunk::FLOATS];
   const int* stretch = SEGMENTS ? segs + 4 * blockIdx.x : spans + 3 * blockIdx.x;
   const int slot = stretch[0], first = stretch[1], count = stretch[2];
   const bool from_state = SEGMENTS ? stretch[3] != 0 : true;
   const int h = blockIdx.y, g = h / (heads / groups);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int ns = threadIdx.x % SS_LANES, p = blockIdx.z * SS_DIMS + threadIdx.x / SS_LANES;
+  const int of_dim = threadIdx.x % SS_LANES, half = of_dim / 16, ns = of_dim & 15;
+  const int p = blockIdx.z * SS_DIMS + threadIdx.x / SS_LANES;
   const bool has_p = p < P;
   const int start = positions[first];
   const float* from = state + (long)slot * state_stride + (long)((start + 1) & 1) * copy_elems;
@@ -213,69 +236,75 @@ state_space_walk_kernel(const float* __restrict__ u, const float* __restrict__ t
   const int inner = heads * P;
   const long s_at = (long)h * N * P, x_col = (long)h * P + (has_p ? p : 0);
   const long b_col = inner + (long)g * N;
-  float S[OWN];
+  float S[ROWS], second[ROWS];         // the second half has no token in the first turns: its rows' beginning comes after them
 #pragma unroll
-  for (int i = 0; i < OWN; ++i) {
-    const int n = ns + SS_LANES * i;
-    S[i] = from_state && has_p && n < N ? from[s_at + (long)n * P + p] : 0.0f;
+  for (int i = 0; i < ROWS; ++i) {
+    const int n = Rows::row(of_dim, i);
+    second[i] = from_state && has_p && n < N ? from[s_at + (long)n * P + p] : 0.0f;
+    S[i] = half ? 0.0f : second[i];
   }
   const float dskip = load_vec(d_skip, d_is_f32, h);
+  const int turns = count + SS_BEHIND;
 
-  // What this lane asks for of a token's row: load j of the wave is piece j WAVES + wave of (B's pieces, C's pieces), the
-  // c-th 64 of the places (quad, lane of the row set, place): row n = lane of the set + 32 (4 quad + place).
+  // What this lane asks for of a turn: load j of the wave is piece j WAVES + wave of (B's pieces, C's pieces), the c-th 64
+  // of the places (quad, lane of the row set, place): the set's lane's row 4 quad + place.  Odd pieces are the second half's,
+  // and odd waves ask for odd pieces: their token is an earlier one.
   typedef const __attribute__((address_space(1))) void* from_t;
   typedef __attribute__((address_space(3))) void* to_t;
   unsigned col[PER];                   // in bytes from the row's B
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
     const int piece = j * WAVES + wave, c = piece % PIECES;
-    const int at = c * 64 + lane, n = at / 4 % SS_LANES + SS_LANES * (at / (4 * SS_LANES) * 4 + at % 4);
+    const int at = c * 64 + lane, n = Rows::row(at / 4 % SS_LANES, min(at / (4 * SS_LANES) * 4 + at % 4, ROWS - 1));
     col[j] = (unsigned)((piece < PIECES ? 0 : groups * N) + min(n, N - 1)) * 4u;        // places beyond the state: any row
   }
-  // COUNT tokens of the chunk that begins with token t0 of the stretch, from its token k on (behind the stretch: its last
-  // token again, not used)
+  // a half's token of a turn (before the first token and behind the last: that one, not used)
+  auto token = [&](int turn, int behind) { return max(min(turn - behind * SS_BEHIND, count - 1), 0); };
+  // COUNT turns of the chunk that begins with the stretch's turn t0, from its turn k on
   const unsigned row_bytes = (unsigned)channels * 4u;
   const char* rows = (const char*)(u + (long)first * channels + b_col);
   auto ask = [&](int buffer, int t0, int k, auto how_many) {
     constexpr int COUNT = decltype(how_many)::value;
 #pragma unroll
     for (int i = 0; i < COUNT; ++i) {
-      const char* row = rows + (unsigned long)(unsigned)min(t0 + k + i, count - 1) * row_bytes;
+      const char* row = rows + (unsigned long)(unsigned)token(t0 + k + i, wave & 1) * row_bytes;
 #pragma unroll
       for (int j = 0; j < PER; ++j)
-        __builtin_amdgcn_global_load_lds((from_t)(row + col[j]), (to_t)(&lds[buffer][0] + (k + i) * 2 * ROWS + (j * WAVES + wave) * 64), 4, 0, 0);
+        __builtin_amdgcn_global_load_lds((from_t)(row + col[j]), (to_t)(&lds[buffer][0] + (k + i) * 2 * PLACES + (j * WAVES + wave) * 64), 4, 0, 0);
     }
   };
-  // the rest of a chunk: x [value dim of the block][token] (waves 0 and 1), (dt, a) a token (waves 2 and 3, the same)
+  // the rest of a chunk: x [half][value dim of the block][turn] (a wave 64 of them), (dt, a) [half][turn] (one wave)
   auto ask_rest = [&](int buffer, int t0) {
-    const int pp = blockIdx.z * SS_DIMS + (int)threadIdx.x / SS_CHUNK % SS_DIMS;
-    const long t = first + min(t0 + (wave < 2 ? lane : lane >> 1) % SS_CHUNK, count - 1);
-    const float* src = wave < 2 ? u + t * channels + (long)h * P + min(pp, P - 1) : terms + (t * heads + h) * 2 + (lane & 1);
-    __builtin_amdgcn_global_load_lds((from_t)src, (to_t)(&lds[buffer][0] + (wave < 2 ? Chunk::X_AT + wave * AXON_WAVE : Chunk::TERMS_AT)),
-                                     4, 0, 0);
+    const int pp = blockIdx.z * SS_DIMS + (wave & 1) * (AXON_WAVE / SS_CHUNK) + lane / SS_CHUNK;
+    const long tx = first + token(t0 + lane % SS_CHUNK, wave >> 1), tt = first + token(t0 + (lane >> 1) % SS_CHUNK, lane / 32);
+    __builtin_amdgcn_global_load_lds((from_t)(u + tx * channels + (long)h * P + min(pp, P - 1)),
+                                     (to_t)(&lds[buffer][0] + Chunk::X_AT + wave * AXON_WAVE), 4, 0, 0);
+    if (wave == 0)
+      __builtin_amdgcn_global_load_lds((from_t)(terms + (tt * heads + h) * 2 + (lane & 1)), (to_t)(&lds[buffer][0] + Chunk::TERMS_AT), 4, 0, 0);
   };
   ask_rest(0, 0);
 #pragma unroll
   for (int k = 0; k < SS_CHUNK; ++k)
-    if (k < count) ask(0, 0, k, SsNumber<1>());
+    if (k < turns) ask(0, 0, k, SsNumber<1>());
 
   const unsigned lds0 = (unsigned)(size_t)(to_t)&lds[0][0];
-  const unsigned bc_at = lds0 + ns * 16, terms_at = lds0 + Chunk::TERMS_AT * 4;
-  const unsigned x_at = lds0 + (Chunk::X_AT + threadIdx.x / SS_LANES * SS_CHUNK) * 4;
-  float decay = 1.0f;                  // of a segment: the product of its tokens' a so far
-  float kept_y = 0.0f, kept_decay = 1.0f;      // of the chunk's token ns
+  const unsigned bc_at = lds0 + of_dim * 16, terms_at = lds0 + (Chunk::TERMS_AT + half * 2 * SS_CHUNK) * 4;
+  const unsigned x_at = lds0 + (Chunk::X_AT + (half * SS_DIMS + threadIdx.x / SS_LANES) * SS_CHUNK) * 4;
+  float decay = 1.0f;                  // of a segment: the product of its tokens' a so far (the first half's)
+  float kept_y = 0.0f, kept_decay = 1.0f;      // of the chunk's turn ns: the second half's token's, the first half's
+  float begun[SUB] = {};               // what the second half was handed
 
-  // the operands of the chunk's tokens k0 + turn SUB ..: `turn` is known when compiled
-  auto read = [&](SsStaged<OWN>& o, unsigned at, int k0, int turn) {
-    const unsigned rows = bc_at + at + k0 * (2 * ROWS * 4);
+  // the operands of the chunk's turns k0 + pair SUB ..: `pair` is known when compiled
+  auto read = [&](SsStaged<OWN>& o, unsigned at, int k0, int pair) {
+    const unsigned rows = bc_at + at + k0 * (2 * PLACES * 4);
 #pragma unroll
     for (int k = 0; k < SUB; ++k)
 #pragma unroll
       for (int q = 0; q < QUADS; ++q) {
-        lds_read16_step<16 * SS_LANES, 4 * SUB * QUADS>(o.B[k][q], rows, (turn * SUB + k) * 2 * QUADS + q);
-        lds_read16_step<16 * SS_LANES, 4 * SUB * QUADS>(o.C[k][q], rows, (turn * SUB + k) * 2 * QUADS + QUADS + q);
+        lds_read16_step<16 * SS_LANES, 4 * SUB * QUADS>(o.B[k][q], rows, (pair * SUB + k) * 2 * QUADS + q);
+        lds_read16_step<16 * SS_LANES, 4 * SUB * QUADS>(o.C[k][q], rows, (pair * SUB + k) * 2 * QUADS + QUADS + q);
       }
-    lds_read16_step<16, 2>(o.terms[0], terms_at + at + k0 * 8, turn);
+    lds_read16_step<16, 2>(o.terms[0], terms_at + at + k0 * 8, pair);
     lds_read16<0>(o.x[0], x_at + at + k0 * 4);
     __builtin_amdgcn_sched_barrier(0);          // all of them ahead of the work that they are to be hidden behind
   };
@@ -289,92 +318,99 @@ state_space_walk_kernel(const float* __restrict__ u, const float* __restrict__ t
     use_frags<1>(o.terms);
     use_frags<1>(o.x);
   };
-  // the work of SUB tokens from the chunk's token k0 + turn SUB on (left: the chunk's that exist; WHOLE: all of them)
-  auto work = [&](const SsStaged<OWN>& o, int k0, int turn, int left, auto whole) {
+  // the work of SUB turns from the chunk's turn k0 + pair SUB on (left: the chunk's turns in which the first half has a token,
+  // from where on its rows stay as they are; WHOLE: it has one in all; begins: the chunk's turn 0 is the stretch's)
+  auto work = [&](const SsStaged<OWN>& o, int k0, int pair, int left, bool begins, auto whole) {
     constexpr bool WHOLE = decltype(whole)::value != 0;
     const int own = ns - k0;
 #pragma unroll
     for (int k = 0; k < SUB; ++k) {
-      const int at = turn * SUB + k;
-      if (WHOLE || k0 + at < left) {
+      const int at = pair * SUB + k;
+      if (WHOLE || k0 + at < left + SS_BEHIND) {
         const float dt = __uint_as_float(o.terms[0][k * 2]), a = __uint_as_float(o.terms[0][k * 2 + 1]);
         const float x = __uint_as_float(o.x[0][at]);
         const float dx = dt * x;
-        float part = 0.0f;
+        float C[ROWS];
 #pragma unroll
-        for (int i = 0; i < OWN; ++i) {
-          const float B = __uint_as_float(o.B[k][i / 4][i % 4]), C = __uint_as_float(o.C[k][i / 4][i % 4]);
-          S[i] = FULL || ns + SS_LANES * i < N ? fmaf(a, S[i], dx * B) : 0.0f;
-          part = fmaf(S[i], C, part);
+        for (int i = 0; i < ROWS; ++i) {
+          const float B = __uint_as_float(o.B[k][i / 4][i % 4]);
+          C[i] = __uint_as_float(o.C[k][i / 4][i % 4]);
+          const float on = FULL || Rows::row(of_dim, i) < N ? fmaf(a, S[i], dx * B) : 0.0f;
+          S[i] = WHOLE || half || k0 + at < left ? on : S[i];
         }
-        part = ss_two_rows_sum(part);
-        kept_y = own == at ? fmaf(dskip, x, part) : kept_y;
+        const float part = Rows::chain(begun[k], half, S, C);
+        begun[k] = ss_hand_on(part);
+        const float sum = ss_row_sum(part);
+        kept_y = own == at ? fmaf(dskip, x, sum) : kept_y;
         if (SEGMENTS) {
           decay *= a;
           kept_decay = own == at ? decay : kept_decay;
         }
+        if (at == SS_BEHIND - 1) {
+          const bool enters = half && begins && k0 == 0;       // (chosen, not branched to: reads are under way)
+#pragma unroll
+          for (int i = 0; i < ROWS; ++i) S[i] = enters ? second[i] : S[i];
+        }
       }
     }
   };
-  // the outputs of the chunk before go out at the start of a chunk: they are on their way while it is worked on
-  auto put = [&](int at, int n) {
-    if (ns < n && has_p) y[(long)(at + ns) * inner + x_col] = kept_y;
-    if (SEGMENTS && blockIdx.z == 0 && (int)threadIdx.x < n) cum[(long)(at + ns) * heads + h] = kept_decay;
+  // the outputs of the chunk of turns t0 .. t0 + n - 1 go out at the start of the next: they are on their way while it is worked on
+  auto put = [&](int t0, int n) {
+    if (half && ns < n && t0 + ns >= SS_BEHIND && has_p) y[(long)(first + t0 + ns - SS_BEHIND) * inner + x_col] = kept_y;
+    if (SEGMENTS && blockIdx.z == 0 && (int)threadIdx.x < min(SS_CHUNK, count - t0)) cum[(long)(first + t0 + ns) * heads + h] = kept_decay;
   };
 
   int buffer = 0;
-  for (int t0 = 0; t0 < count; t0 += SS_CHUNK) {
+  for (int t0 = 0; t0 < turns; t0 += SS_CHUNK) {
     wait_vmcnt<0>();
     __builtin_amdgcn_s_barrier();      // the chunk is in LDS for every wave; nobody reads the one before any more
-    const int left = min(SS_CHUNK, count - t0), ahead = t0 + SS_CHUNK;
-    const bool more = ahead < count;
+    const int left = count - t0, ahead = t0 + SS_CHUNK;        // (left may be below 0: the second half's last tokens)
+    const bool more = ahead < turns, begins = t0 == 0;
     const unsigned at = buffer * Chunk::FLOATS * 4;
-    if (t0 != 0) put(first + t0 - SS_CHUNK, SS_CHUNK);
+    if (t0 != 0) put(t0 - SS_CHUNK, SS_CHUNK);
     if (more) ask_rest(buffer ^ 1, ahead);
     SsStaged<OWN> even, odd;
-    if (left == SS_CHUNK) {
+    if (left >= SS_CHUNK) {
       read(even, at, 0, 0);
       arrived(even);
 #pragma unroll 1
       for (int k0 = 0; k0 < SS_CHUNK; k0 += 2 * SUB) {      // no read is under way across a branch
         read(odd, at, k0, 1);
-        work(even, k0, 0, left, SsNumber<1>());
+        work(even, k0, 0, left, begins, SsNumber<1>());
         arrived(odd);
         if (more && k0 < SS_CHUNK / 2) ask(buffer ^ 1, ahead, 2 * k0, SsNumber<2 * SUB>());
         read(even, at, k0 + 2 * SUB < SS_CHUNK ? k0 + 2 * SUB : 0, 0);
-        work(odd, k0, 1, left, SsNumber<1>());
+        work(odd, k0, 1, left, begins, SsNumber<1>());
         arrived(even);
         if (more && k0 < SS_CHUNK / 2) ask(buffer ^ 1, ahead, 2 * k0 + 2 * SUB, SsNumber<2 * SUB>());
       }
-    } else {                                                // the last chunk: nothing is left to ask for
+    } else {                                                // the last chunk, or the last but one
+      if (more) {
+#pragma unroll
+        for (int k = 0; k < SS_BEHIND; ++k) ask(buffer ^ 1, ahead, k, SsNumber<1>());
+      }
 #pragma unroll 1
-      for (int k0 = 0; k0 < left; k0 += 2 * SUB) {
+      for (int k0 = 0; k0 < min(SS_CHUNK, left + SS_BEHIND); k0 += 2 * SUB) {
         read(even, at, k0, 0);
-        read(odd, at, k0, 1);                               // (places of the chunk that hold no token: not used)
+        read(odd, at, k0, 1);                               // (places of the chunk that nothing was asked for: not used)
         arrived(even);
         arrived(odd);
-        work(even, k0, 0, left, SsNumber<0>());
-        work(odd, k0, 1, left, SsNumber<0>());
+        work(even, k0, 0, left, begins, SsNumber<0>());
+        work(odd, k0, 1, left, begins, SsNumber<0>());
       }
     }
     buffer ^= 1;
   }
-  put(first + (count - 1) / SS_CHUNK * SS_CHUNK, (count - 1) % SS_CHUNK + 1);
-  if (SEGMENTS) {                      // a segment's end state goes to the workspace; the fold brings the request's state up to date
-    float* end = ends + ((long)blockIdx.x * heads + h) * N * P;
+  put((turns - 1) / SS_CHUNK * SS_CHUNK, (turns - 1) % SS_CHUNK + 1);
+  // a segment's end state goes to the workspace; the fold brings the request's state up to date
+  float* end = SEGMENTS ? ends + ((long)blockIdx.x * heads + h) * N * P : to + s_at;
 #pragma unroll
-    for (int i = 0; i < OWN; ++i) {
-      const int n = ns + SS_LANES * i;
-      if (has_p && n < N) end[(long)n * P + p] = S[i];
-    }
-    return;
+  for (int i = 0; i < ROWS; ++i) {
+    const int n = Rows::row(of_dim, i);
+    if (has_p && n < N) end[(long)n * P + p] = S[i];
   }
-#pragma unroll
-  for (int i = 0; i < OWN; ++i) {
-    const int n = ns + SS_LANES * i;
-    if (has_p && n < N) to[s_at + (long)n * P + p] = S[i];
-  }
-  if (blockIdx.y == 0 && blockIdx.z == 0) ss_keep_inputs(from, to, tail_at, conv_in, conv_in_stride, first, count, channels, taps);
+  if (!SEGMENTS && blockIdx.y == 0 && blockIdx.z == 0)
+    ss_keep_inputs(from, to, tail_at, conv_in, conv_in_stride, first, count, channels, taps);
 }
 
 // Long stretches of tokens in segments.  The walk above then runs every segment of a request side by side:
@@ -572,15 +608,15 @@ extern "C" int axk_state_space_scan(const float* u, const float* terms, const vo
 #define SS_LAUNCH(OWN)                                                                              \
   {                                                                                                 \
     if (spans == nullptr)                                                                           \
-      state_space_step_kernel<(OWN + 1) / 2><<<grid, SS_WALKERS, 0, s>>>(u, terms, d_skip, d_is_f32, state, state_stride, copy_elems, tail_at, \
+      state_space_step_kernel<OWN><<<grid, SS_WALKERS, 0, s>>>(u, terms, d_skip, d_is_f32, state, state_stride, copy_elems, tail_at, \
                                                                positions, seq_rows, conv_in, conv_in_stride, y, heads, groups, vdim, \
                                                                n_state, channels, taps);            \
     else if (segs) {                                                                                \
-      if (n_state == SS_LANES * ((OWN + 1) / 2)) state_space_walk_kernel<(OWN + 1) / 2, true, true><<<grid, SS_WALKERS, 0, s>>>(SS_ARGS); \
-      else state_space_walk_kernel<(OWN + 1) / 2, false, true><<<grid, SS_WALKERS, 0, s>>>(SS_ARGS);          \
+      if (n_state == 16 * OWN) state_space_walk_kernel<OWN, true, true><<<grid, SS_WALKERS, 0, s>>>(SS_ARGS); \
+      else state_space_walk_kernel<OWN, false, true><<<grid, SS_WALKERS, 0, s>>>(SS_ARGS);          \
     } else {                                                                                        \
-      if (n_state == SS_LANES * ((OWN + 1) / 2)) state_space_walk_kernel<(OWN + 1) / 2, true, false><<<grid, SS_WALKERS, 0, s>>>(SS_ARGS); \
-      else state_space_walk_kernel<(OWN + 1) / 2, false, false><<<grid, SS_WALKERS, 0, s>>>(SS_ARGS);         \
+      if (n_state == 16 * OWN) state_space_walk_kernel<OWN, true, false><<<grid, SS_WALKERS, 0, s>>>(SS_ARGS); \
+      else state_space_walk_kernel<OWN, false, false><<<grid, SS_WALKERS, 0, s>>>(SS_ARGS);         \
     }                                                                                               \
     if (segs) {                                                                                     \
       state_space_fold_kernel<OWN><<<grid_fold, SS_THREADS, 0, s>>>(ends, cum, spans5, segs, state, state_stride, copy_elems, tail_at, \

@@ -1,5 +1,6 @@
 """The state-space walk of stretches against the same recurrence a token at a time: the same bits, whatever the
 stretch's length is to the chunks that go through LDS, and whatever the state's rows are to the lanes that hold them."""
+import numpy as np
 import pytest
 import torch
 
@@ -81,3 +82,54 @@ def test_segments_of_a_stretch_add_up(heads, groups, P, N):
     assert float((got - want).abs().max()) <= bound
     assert torch.equal(got[:cut], want[:cut])
     assert float((many - one).abs().max()) <= 4 * N * 2.0 ** -24 * float(one.abs().max())
+
+
+def fma(a, b, c):
+    """a b + c of float32 values in one rounding: the sum in float64 rounded to odd, which the second rounding cannot see."""
+    p, c = np.float64(a) * np.float64(b), np.float64(c)            # the product of 24 bits and 24 bits is exact
+    s = p + c
+    t = s - p
+    err = (p - (s - t)) + (c - t)
+    bits = s.view(np.int64)
+    odd = np.where((err != 0) & (bits % 2 == 0), bits + np.where((err > 0) == (s > 0), 1, -1), bits)
+    return odd.view(np.float64).astype(np.float32)
+
+
+def sixteen_chains(x, dt, a, B, C, skip, S):
+    """A token of one head: x [P], B and C [N], the state S [N, P].  The outputs, and the state behind it."""
+    N, P = S.shape
+    S = fma(np.full((N, P), a, np.float32), S, (dt * x)[None] * B[:, None])
+    part = np.zeros((16, P), np.float32)
+    for at in range(0, N, 16):                                     # chain l: rows l, l + 16, ... in ascending order
+        rows = np.arange(at, min(at + 16, N))
+        part[rows - at] = fma(S[rows], np.broadcast_to(C[rows, None], (len(rows), P)), part[rows - at])
+    lanes = np.arange(16)
+    for with_lane in (lanes ^ 1, lanes ^ 2, lanes // 8 * 8 + 7 - lanes % 8, 15 - lanes):
+        part = part + part[with_lane]
+    return fma(np.full(P, skip, np.float32), x, part[0]), S
+
+
+@pytest.mark.parametrize("steps", [False, True])
+@pytest.mark.parametrize("P, N, tokens", [(8, 128, 37), (5, 100, 37), (3, 7, 37), (4, 16, 37), (2, 256, 37), (3, 33, 37), (2, 17, 37), (3, 32, 37)] +
+                         [(3, 128, n) for n in (1, 2, 3, 13, 14, 15, 16, 17, 29, 30, 31, 32)])
+def test_a_sum_over_the_state_is_sixteen_chains(P, N, tokens, steps):
+    """The order that a design's outputs have had in every form of this scan: bit for bit, in stretches and in single steps."""
+    heads = 2
+    d = case(heads, 1, P, N, tokens)
+    k = kernels("float32")
+    state = torch.randn(1, 2 * d["copy"], device="cuda")
+    at = d["tail"]
+    S = [state[0, d["copy"]:d["copy"] + at].view(heads, N, P)[h].cpu().numpy() for h in range(heads)]       # behind position -1
+    u, terms, skip = d["u"].cpu().numpy(), d["terms"].cpu().numpy(), d["skip"].cpu().numpy()
+    want = np.empty((tokens, heads * P), np.float32)
+    for t in range(tokens):
+        B, C = u[t, heads * P:heads * P + N], u[t, heads * P + N:]
+        for h in range(heads):
+            want[t, h * P:(h + 1) * P], S[h] = sixteen_chains(u[t, h * P:(h + 1) * P], terms[t, h, 0], terms[t, h, 1], B, C, skip[h], S[h])
+    if steps:
+        got = torch.cat([scan(k, d, state, None, i32([t]), i32([0]), [t]) for t in range(tokens)])
+    else:
+        got = scan(k, d, state, i32([[0, 0, tokens]]), i32(list(range(tokens))), i32([0] * tokens), list(range(tokens)))
+    assert np.array_equal(got.cpu().numpy(), want)
+    left = state[0, (tokens - 1) % 2 * d["copy"]:][:at].view(heads, N, P).cpu().numpy()
+    assert np.array_equal(left, np.stack(S))
