@@ -33,27 +33,25 @@ from .base import CacheBinding, Mixer, StateSpec, TensorDecl, register_mixer
 from .recurrent import step_spans
 
 SEGMENT = 128           # the fewest tokens a segment of a long stretch (a request's tokens of one step) holds
-TARGET_BLOCKS = 2048    # blocks a segmented scan of one or two waves a block launches: eight a compute unit
+TARGET_BLOCKS = 2048    # blocks the segmented scan launches: eight a compute unit
 FEW_BLOCKS = 256        # a walk of one chain a request that launches more blocks than this is left as it is
 
-# The state-space walk's blocks are four waves: 256 of them (a stretch of 32 heads of 64 dims) walk 1,024 tokens in 130 us as
-# one chain and in 147 in four segments with the two further launches, 2,048 in 257 against 254, 8,192 in 1,013 against 848
-# (eight); 64 blocks take 127 and 68 us for 1,024 tokens (eight segments), 252 and 105 for 2,048 (sixteen: 119).
-WALK_TARGET_BLOCKS = 512
-WALK_FEW_BLOCKS = 128
 
-
-def step_segments(ctx, blocks_a_stretch: int, few_blocks: int = FEW_BLOCKS, target_blocks: int = TARGET_BLOCKS):
+def step_segments(ctx, blocks_a_stretch: int):
     """The stretches of a step cut into segments, for the scan that runs a long stretch's segments side by side:
     (segs int32 [n, 4] = (slot, first token, tokens, whether the request's first), spans5 int32 [requests, 5] =
     (slot, first token, tokens, first segment, segments), the longest segment's tokens) on the device, made once a step and scan shape.  A walk
     of one chain a stretch launches `blocks_a_stretch` blocks a stretch; stretches are cut into as many equal
-    segments (of SEGMENT tokens at least) as brings the launch to `target_blocks`.  None where that is one segment
-    a stretch, where the walk of one chain a request fills the chip by itself (more than `few_blocks` blocks), and in
-    steps of single tokens: one walk a request then, whose sums do not depend on the cuts."""
-    if ctx.decode_only or blocks_a_stretch * len(ctx.spans) > few_blocks:
+    segments (of SEGMENT tokens at least) as brings the launch to TARGET_BLOCKS.  None where that is one segment
+    a stretch, where the walk of one chain a request fills the chip by itself (more than FEW_BLOCKS blocks), and in
+    steps of single tokens: one walk a request then, whose sums do not depend on the cuts.  At 256 blocks of the
+    state-space walk, whose blocks are four waves, one chain and eight segments with the two further launches take
+    72 and 94 us for 512 tokens (four segments), 137 and 154 for 1,024, 270 and 271 for 2,048, 1,061 and 914 for 8,192;
+    at 64 blocks 70 and 50, 135 and 72, 266 and 110.  (A line by length would give short stretches some 20 us back,
+    with the sums of one chain: a design's outputs do not change for that.)"""
+    if ctx.decode_only or blocks_a_stretch * len(ctx.spans) > FEW_BLOCKS:
         return None
-    most = target_blocks // max(1, blocks_a_stretch * len(ctx.spans))
+    most = TARGET_BLOCKS // max(1, blocks_a_stretch * len(ctx.spans))
     if most < 2 or all(s.q_len < 2 * SEGMENT for s in ctx.spans):
         return None
     key = ("state_space_segments", most)
@@ -133,7 +131,7 @@ class SelectiveStateSpace(Mixer):
         y = ctx.ws.take((T, self.inner), f32)
         k.state_space_scan(u, terms, self.d_skip, state, self.copy_elems, self.tail_at, step_spans(ctx), ctx.positions,
                            ctx.seq_rows, xbc, y, self.heads, self.groups, self.vdim, self.n_state, self.taps,
-                           segments=step_segments(ctx, self.heads * -(-self.vdim // 8), WALK_FEW_BLOCKS, WALK_TARGET_BLOCKS))
+                           segments=step_segments(ctx, self.heads * -(-self.vdim // 8)))
         normed = ctx.ws.take((T, self.inner), ctx.rt.dtype)
         k.gated_group_norm(y, z, self.gain, self.eps, normed, self.norm_groups)
         k.gemm(normed, self.w_o, out, None, MODE_ADD_F32 if accumulate else MODE_STORE_F32)
