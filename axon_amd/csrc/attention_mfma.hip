@@ -770,16 +770,18 @@ attention_decode_kernel(const bf16_t* __restrict__ q, int q_stride, const bf16_t
 // worked out for HD blocks at once, thread i those of block i (the running maximum before a block
 // is the largest of the maxima before it: no rounding, any order), and only the two multiply-adds
 // a block remain a chain: thread d folds dim d, every thread folds l for itself.
-// Bound by its waits (the position, the blocks' numbers, the scan through LDS), not by bytes.  The first COMBINE_AHEAD
-// blocks' values are asked for beside the maxima instead of behind the scan: 28 heads, contexts of 301 to 3,907 positions
-// of 8 tokens 7.25 -> 6.2 us, of 64 to 900 of 64 tokens 7.1 -> 6.5.
-#define COMBINE_AHEAD 64      // blocks whose values a thread holds (a context of 4,096 positions)
+// Bound by its waits (the position, the blocks' numbers, the scan of the maxima, one multiply-add behind another), not by
+// bytes.  At most 128 registers, so that four waves a SIMD fit: 64 tokens of 28 heads are 3,584 waves, and run at once.  28
+// heads, us, with the values behind the scan / here: 8 tokens of 301 to 3,907 positions 7.0 / 4.2, of 4,000 8.4 / 4.3, of
+// 32,900 23.6 / 21.8; 64 of 64 to 900 7.2 / 4.3, of 600 6.4 / 4.5, of 1,500 7.4 / 6.5, of 2,048 6.4 / 7.1 (30 MB at once), of 2,300
+// 7.7 / 7.9, of 3,000 12.8 / 9.9; one of 2,048 3.8 / 3.7, of 32,900 15.2 / 14.9.
+#define COMBINE_AHEAD 64      // blocks whose values a thread asks for beside the maxima, at most (4,096 positions)
 template <int HD>
-__global__ void __launch_bounds__(HD)
+__global__ void __launch_bounds__(HD, 4)
 attention_combine_kernel(const float* __restrict__ partial, const int32_t* __restrict__ positions,
                          const int32_t* __restrict__ token_index, bf16_t* __restrict__ out, int max_chunks, int n_heads,
                          int window) {
-  __shared__ float block_max[HD], block_sum[HD], wave_max[HD / 64];
+  __shared__ float wave_max[HD / 64];
   __shared__ __align__(16) float old_factor[HD], new_factor[HD], scaled_sum[HD];   // a, b, and l_b b, of the group's blocks
   const int t = token_index ? token_index[blockIdx.x] : blockIdx.x, head = blockIdx.y, d = threadIdx.x;
   const int pos = positions[t];
@@ -788,29 +790,41 @@ attention_combine_kernel(const float* __restrict__ partial, const int32_t* __res
   const int b0 = (lo - first) / ATT_BLOCK, b1 = (pos - first) / ATT_BLOCK;     // the blocks that hold seen positions
   const float* src = partial + ((size_t)blockIdx.x * n_heads + head) * (max_chunks * (DC_CHUNK / ATT_BLOCK)) * (HD + 2);
   float m = -INFINITY, l = 0.0f, o = 0.0f;     // m: the maximum of all blocks before this group
-  for (int g0 = b0; g0 <= b1; g0 += HD) {
-    const int n = min(HD, b1 - g0 + 1);        // blocks of this group
-    if (g0 > b0) __syncthreads();              // everyone has read the group before
-    // the first blocks' values are asked for beside the maxima (blocks that are not there: the last one's again), a
-    // round of sixteen where one is left: with them behind the scan a step waited for memory twice
-    float ahead[COMBINE_AHEAD];
-    const float* values = src + (size_t)g0 * (HD + 2) + d;
+  // four blocks of the chain, those from `n` on left out (whole: none are); the factors come from LDS four at a time
+  auto fold_four = [&](int i, int n, const float* values, auto whole) {
+    const float4 fa = *reinterpret_cast<const float4*>(&old_factor[i]);
+    const float4 fb = *reinterpret_cast<const float4*>(&new_factor[i]);
+    const float4 ls = *reinterpret_cast<const float4*>(&scaled_sum[i]);
+    const float a4[4] = {fa.x, fa.y, fa.z, fa.w}, b4[4] = {fb.x, fb.y, fb.z, fb.w}, l4[4] = {ls.x, ls.y, ls.z, ls.w};
 #pragma unroll
-    for (int i = 0; i < COMBINE_AHEAD; i += 16)
-      if (i < n) {
-#pragma unroll
-        for (int j = i; j < i + 16; ++j) ahead[j] = values[(size_t)min(j, n - 1) * (HD + 2)];
-      }
-    if (d < n) {
-      const float* p = src + (size_t)(g0 + d) * (HD + 2);
-      block_max[d] = p[HD];
-      block_sum[d] = p[HD + 1];
+    for (int e = 0; e < 4; ++e) {
+      float on = o;
+      attention_fold_into(on, a4[e], values[e], b4[e]);
+      const float sum = __builtin_fmaf(l, a4[e], l4[e]);
+      const bool there = decltype(whole)::value || i + e < n;      // chosen, not branched to
+      o = there ? on : o;
+      l = there ? sum : l;
     }
-    __syncthreads();
+  };
+  // the n blocks from g0 on; the first AHEAD blocks' values are asked for beside the maxima: behind the scan, a step waited for
+  // memory twice.  No branch lies between these loads and the scan, which so waits for the maxima alone, nor among the
+  // blocks of the chain that are sure to be there.
+  // full: n >= AHEAD; else the n blocks are among these AHEAD (for those that are not there the last one's value again).
+  auto fold_group = [&](int g0, int n, auto asked, auto full) {
+    constexpr int AHEAD = decltype(asked)::value;
+    constexpr bool FULL = decltype(full)::value;
+    const float* group = src + (size_t)g0 * (HD + 2);
+    const float* own = group + (size_t)min(d, n - 1) * (HD + 2) + HD;
+    const float block_max = own[0], block_sum = own[1];
+    float ahead[AHEAD];
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j)
+      ahead[j] = group[(size_t)(FULL ? j : min(j, n - 1)) * (HD + 2) + d];
+    __builtin_amdgcn_sched_barrier(0);         // nothing waits before all of them are under way
     {
       // the running maximum before block d: a scan over the lanes of each wave, then the waves before
       const int lane = d & 63, wave = d >> 6;
-      const float mine = d < n ? block_max[d] : -INFINITY;
+      const float mine = d < n ? block_max : -INFINITY;
       float upto = mine;                       // the largest of this wave's blocks up to d
 #pragma unroll
       for (int off = 1; off < 64; off <<= 1) {
@@ -828,58 +842,52 @@ attention_combine_kernel(const float* __restrict__ partial, const int32_t* __res
         attention_fold(before, unused, mine, 0.0f, fa, fb);
         old_factor[d] = fa;
         new_factor[d] = fb;
-        scaled_sum[d] = __fmul_rn(block_sum[d], fb);
+        scaled_sum[d] = __fmul_rn(block_sum, fb);
       }
     }
     __syncthreads();
-    // the fold is a chain, the loads are not: thirty-two blocks' values under way at a time where
-    // that many are left, then sixteen; the blocks' factors come from LDS four at a time (the first are there)
+    // the fold is a chain, the loads are not: behind the first blocks thirty-two blocks' values under way at a time where that
+    // many are left, then sixteen
 #pragma unroll
-    for (int r = 0; r < COMBINE_AHEAD; r += 16)
-      if (r < n) {
+    for (int r = 0; r < AHEAD; r += 16)
+      if (FULL || r + 16 <= n) {
 #pragma unroll
-        for (int j = r; j < r + 16; j += 4) {
-          const float4 fa = *reinterpret_cast<const float4*>(&old_factor[j]);
-          const float4 fb = *reinterpret_cast<const float4*>(&new_factor[j]);
-          const float4 ls = *reinterpret_cast<const float4*>(&scaled_sum[j]);
-          const float a4[4] = {fa.x, fa.y, fa.z, fa.w}, b4[4] = {fb.x, fb.y, fb.z, fb.w}, l4[4] = {ls.x, ls.y, ls.z, ls.w};
+        for (int j = r; j < r + 16; j += 4) fold_four(j, n, &ahead[j], std::true_type());
+      } else if (r < n) {
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (j + e < n) {
-              l = __builtin_fmaf(l, a4[e], l4[e]);
-              attention_fold_into(o, a4[e], ahead[j + e], b4[e]);
-            }
-        }
+        for (int j = r; j < r + 16; j += 4) fold_four(j, n, &ahead[j], std::false_type());
       }
-    int i = min(COMBINE_AHEAD, n);
-    auto fold_batch = [&](auto count) {
-      constexpr int COUNT = decltype(count)::value;
-      for (; i + COUNT - 1 < n; i += COUNT) {
-        float ob[COUNT];
+    if (FULL) {
+      int i = AHEAD;
+      auto fold_batch = [&](auto count) {
+        constexpr int COUNT = decltype(count)::value;
+        for (; i + COUNT - 1 < n; i += COUNT) {
+          float ob[COUNT];
 #pragma unroll
-        for (int j = 0; j < COUNT; ++j) ob[j] = src[(size_t)(g0 + i + j) * (HD + 2) + d];
+          for (int j = 0; j < COUNT; ++j) ob[j] = group[(size_t)(i + j) * (HD + 2) + d];
 #pragma unroll
-        for (int q = 0; q < COUNT / 4; ++q) {
-          const float4 fa = *reinterpret_cast<const float4*>(&old_factor[i + 4 * q]);
-          const float4 fb = *reinterpret_cast<const float4*>(&new_factor[i + 4 * q]);
-          const float4 ls = *reinterpret_cast<const float4*>(&scaled_sum[i + 4 * q]);
-          const float a4[4] = {fa.x, fa.y, fa.z, fa.w}, b4[4] = {fb.x, fb.y, fb.z, fb.w}, l4[4] = {ls.x, ls.y, ls.z, ls.w};
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            l = __builtin_fmaf(l, a4[e], l4[e]);
-            attention_fold_into(o, a4[e], ob[4 * q + e], b4[e]);
-          }
+          for (int q = 0; q < COUNT; q += 4) fold_four(i + q, n, &ob[q], std::true_type());
         }
+      };
+      fold_batch(std::integral_constant<int, 32>());
+      fold_batch(std::integral_constant<int, 16>());
+      for (; i < n; ++i) {
+        const float fa = old_factor[i], fb = new_factor[i];
+        l = __builtin_fmaf(l, fa, scaled_sum[i]);
+        attention_fold_into(o, fa, group[(size_t)i * (HD + 2) + d], fb);
       }
-    };
-    fold_batch(std::integral_constant<int, 32>());
-    fold_batch(std::integral_constant<int, 16>());
-    for (; i < n; ++i) {
-      const float fa = old_factor[i], fb = new_factor[i];
-      l = __builtin_fmaf(l, fa, scaled_sum[i]);
-      attention_fold_into(o, fa, src[(size_t)(g0 + i) * (HD + 2) + d], fb);
     }
     for (int w = 0; w < HD / 64; ++w) m = fmaxf(m, wave_max[w]);     // blocks past n count as -inf
+  };
+  for (int g0 = b0; g0 <= b1; g0 += HD) {
+    const int n = min(HD, b1 - g0 + 1);        // blocks of this group
+    if (g0 > b0) __syncthreads();              // everyone has read the group before
+    // (more blocks than a thread asks for at most: 32 ahead, as many as each batch behind them; with 64 ahead one token of
+    // 32,768 positions takes 14.1 us, eight 20.0)
+    if (n > COMBINE_AHEAD) fold_group(g0, n, std::integral_constant<int, COMBINE_AHEAD / 2>(), std::true_type());
+    else if (n > 32) fold_group(g0, n, std::integral_constant<int, COMBINE_AHEAD>(), std::false_type());
+    else if (n > 16) fold_group(g0, n, std::integral_constant<int, 32>(), std::false_type());
+    else fold_group(g0, n, std::integral_constant<int, 16>(), std::false_type());
   }
   out[(size_t)t * n_heads * HD + (size_t)head * HD + d] = float_to_bf16(__fmul_rn(o, attention_inverse(l)));
 }
