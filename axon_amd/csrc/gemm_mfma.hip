@@ -586,7 +586,8 @@ gemm_small_tile_kernel(const bf16_t* __restrict__ x, int x_stride, const bf16_t*
   // Every stage is filled before the loop; tile kt + STAGES is fetched into tile kt's stage as
   // soon as every wave has read that tile's last fragments, which is during its last k step:
   // the wait for the next tile, the barrier and the first reads of the next tile are hidden
-  // behind that step's products (half of them before the barrier, half after the reads).
+  // behind that step's products (half of them before the barrier, half after the reads).  No read is
+  // under way across a branch, where the compiler, which knows nothing of it, may move its registers.
   constexpr int KS = BK / 16;
   static_assert(KS % 2 == 0, "the register sets alternate and start a tile at set 0");
 #pragma unroll
@@ -596,34 +597,44 @@ gemm_small_tile_kernel(const bf16_t* __restrict__ x, int x_stride, const bf16_t*
   else wait_vmcnt<0>();
   __builtin_amdgcn_s_barrier();   // tile 0 is in LDS for every wave
   read_step(0, 0, 0);
-  for (int kt = 0; kt < nk; ++kt) {
+  wait_lgkmcnt<0>();
+  use_frags<TM>(a[0]);
+  use_frags<TN>(b[0]);
+  auto tile = [&](int kt, auto is_last) {
+    constexpr bool LAST = decltype(is_last)::value;
     const int stage_index = kt % STAGES;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       const int cur = ks & 1, nxt = cur ^ 1;
       if (ks + 1 < KS) {
         read_step(nxt, stage_index, ks + 1);
-        wait_lgkmcnt<TM + TN>();          // this step's fragments (reads return in order)
-        use_frags<TM>(a[cur]);
-        use_frags<TN>(b[cur]);
+        __builtin_amdgcn_sched_barrier(0);      // the next step's fragments: asked for ahead of this one's products, awaited behind them
         multiply(cur, 0, TN);
-      } else {
-        wait_lgkmcnt<0>();                // the last fragments of this tile: its stage is free
-        use_frags<TM>(a[cur]);
-        use_frags<TN>(b[cur]);
+        __builtin_amdgcn_sched_barrier(0);
+        wait_lgkmcnt<0>();
+      } else {                            // (the last fragments of this tile are read: its stage is free)
         multiply(cur, 0, TN / 2);
-        if (kt + 1 < nk) {
+        if (!LAST) {
           // this wave's part of tile kt + 1 has landed when only younger tiles are outstanding
           if (kt + STAGES < nk) wait_vmcnt<(STAGES - 2) * (XQ + WQ)>();
           else wait_vmcnt<0>();
           __builtin_amdgcn_s_barrier();   // tile kt + 1 is in LDS for every wave; nobody reads tile kt any more
           if (kt + STAGES < nk) issue(kt + STAGES);
           read_step(nxt, (kt + 1) % STAGES, 0);
+          __builtin_amdgcn_sched_barrier(0);
         }
         multiply(cur, TN / 2, TN);
+        __builtin_amdgcn_sched_barrier(0);
+        if (!LAST) wait_lgkmcnt<0>();
+      }
+      if (!LAST || ks + 1 < KS) {
+        use_frags<TM>(a[nxt]);
+        use_frags<TN>(b[nxt]);
       }
     }
-  }
+  };
+  for (int kt = 0; kt + 1 < nk; ++kt) tile(kt, Number<0>());
+  tile(nk - 1, Number<1>());
 #undef SWZ
   // epilogue: lane holds column n = lane % 32 of each tile and rows (e/4)*8 + (lane/32)*4 + e%4
   if (partial) {

@@ -53,17 +53,33 @@ def unwaited(assembly, kernel):
     return reads, faults
 
 
+@pytest.fixture(scope="module")
+def assembly(tmp_path_factory):
+    """The device code of a source, compiled once for all of its kernels."""
+    made = {}
+
+    def of(source):
+        if source not in made:
+            out = tmp_path_factory.mktemp("device") / (source + ".s")
+            hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+            subprocess.run([hipcc, *B.HIP_FLAGS, B.DTYPE_FLAG["bfloat16"], "-S", "--cuda-device-only", os.path.join(B.CSRC, source), "-o", str(out)],
+                           check=True, capture_output=True, timeout=600)
+            made[source] = out.read_text()
+        return made[source]
+    return of
+
+
 @pytest.mark.skipif(shutil.which("hipcc") is None and not os.path.exists("/opt/rocm/bin/hipcc"), reason="no compiler")
 @pytest.mark.parametrize("source, kernel", [("grouped_gemm.hip", "grouped_gemm_tile_kernel"),
                                             ("latent_attention.hip", "latent_attention_prompt_kernel"),
                                             ("gemm_mfma.hip", "gemm_tile_kernel"),
+                                            ("gemm_mfma.hip", "gemm_small_tile_kernel"),
+                                            ("gemm_mfma.hip", "gemm_rows_kernel"),
+                                            ("attention_mfma.hip", "attention_prefill_kernel"),
+                                            ("attention_mfma.hip", "attention_decode_kernel"),
                                             ("state_space.hip", "state_space_walk_kernel")])
-def test_nothing_comes_between_a_read_and_its_wait(tmp_path, source, kernel):
-    out = tmp_path / "device.s"
-    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
-    subprocess.run([hipcc, *B.HIP_FLAGS, B.DTYPE_FLAG["bfloat16"], "-S", "--cuda-device-only", os.path.join(B.CSRC, source), "-o", str(out)],
-                   check=True, capture_output=True, timeout=600)
-    reads, faults = unwaited(out.read_text(), kernel)
+def test_nothing_comes_between_a_read_and_its_wait(assembly, source, kernel):
+    reads, faults = unwaited(assembly(source), kernel)
     assert reads > 0 and not faults, faults[:5]
 
 
