@@ -34,11 +34,13 @@
 //   same segment of K and share X through LDS; a block a segment, the sums of several segments
 //   through a workspace.
 //
-// * gemm_tile (M > 128; gemm_small_tile where the tiles are small and a block takes a segment): a block of 4 or 8 waves owns a BM x BN tile of the output, walks K in
+// * gemm_tile (M > 128): a block of 4 or 8 waves owns a BM x BN tile of the output, walks K in
 //   steps of 32 through LDS stages filled by direct global -> LDS loads (the next steps' loads
-//   in flight while this one multiplies), and each wave keeps a tile of MFMA accumulators.  With S > 1 segments each goes to blocks of its own (gridDim.y = S), whose sums
-//   go through a workspace and are added in segment order by gemm_split_reduce, which also
-//   applies the epilogue.  X rows land in LDS with their 16-byte slots permuted so that fragment reads of
+//   in flight while this one multiplies), and each wave keeps a tile of MFMA accumulators; where
+//   128 x 128 tiles take a segment each, gemm_small_tile, in steps of 64.  With S > 1 segments each
+//   goes to blocks of its own (gridDim.y = S), whose sums go through a workspace and are added in
+//   segment order by gemm_split_reduce, which also applies the epilogue; or, where tiles of 128 x 128
+//   fill the chip (keeps_segments), a block walks them all.  X rows land in LDS with their 16-byte slots permuted so that fragment reads of
 //   neighbouring rows fall into different banks; W blocks land as they are.  Blocks are numbered
 //   so that the blocks of one XCD (every eighth block) share weight tiles in that XCD's L2.
 #include "api.h"
@@ -77,6 +79,143 @@ __device__ inline void wait_rounds(int rounds) {
   }
 }
 
+// ---------------------------------------------------------------------------- what the tile kernels share
+// Block numbering: every eighth block runs on the same XCD, 32 of them at a time.  An XCD takes
+// every eighth n block and walks its share in squares of up to 8 m blocks x 4 n blocks, so that
+// the 32 blocks at work share 12 tiles of operands in that XCD's L2 (with many m blocks, all m
+// blocks of one n block in a row would share 33), the squares of the same four n blocks one
+// after the other.
+__device__ inline void tile_of_block(int bid, int m_blocks, int n_blocks, int& mb, int& nb) {
+  if (bid < (n_blocks / 8) * 8 * m_blocks) {
+    constexpr int GM = 8, GN = 4;
+    const int xcd = bid & 7, j = bid >> 3, mine = n_blocks / 8;       // this XCD's n blocks: xcd, xcd + 8, ...
+    const int whole_groups = mine / GN;
+    int g = j / (GN * m_blocks), rest = j % (GN * m_blocks), gn = GN;
+    if (g >= whole_groups) {                                          // the last, narrower group of n blocks
+      g = whole_groups;
+      rest = j - whole_groups * GN * m_blocks;
+      gn = mine - whole_groups * GN;
+    }
+    const int whole_rows = m_blocks / GM;
+    int ms = rest / (gn * GM), r = rest % (gn * GM), gm = GM;
+    if (ms >= whole_rows) {                                           // the last, shorter square
+      ms = whole_rows;
+      r = rest - whole_rows * gn * GM;
+      gm = m_blocks - whole_rows * GM;
+    }
+    mb = ms * GM + r % gm;
+    nb = (g * GN + r / gm) * 8 + xcd;
+  } else {  // the last, incomplete group of n blocks: plain order
+    const int r = bid - (n_blocks / 8) * 8 * m_blocks;
+    nb = (n_blocks / 8) * 8 + r / m_blocks;
+    mb = r % m_blocks;
+  }
+}
+
+// The epilogue of a wave's tile whose columns lie across lanes.  Of each of COLS column tiles a lane holds one column, col(c),
+// and of that QUADS times four neighbouring rows from row(q) on: value(c, q, e).  Sixteen or 32 lanes side by side hold
+// neighbouring columns, so a store or read of 32-bit values is whole 64 or 128 bytes of each of a few rows; four columns a
+// lane (below) meet 64 lines in a 16-byte store where this meets 16.
+// With `partial`: the sums as they are to [split][gate | up][M][N] (one part without GLU).
+template <bool GLU, int COLS, int QUADS, class Value, class Col, class Row>
+__device__ __forceinline__ void tile_epilogue(Value value, Col col, Row row, const void* __restrict__ bias, int bias_is_f32,
+                                              void* __restrict__ out, int out_stride, int M, int N, int mode,
+                                              float* __restrict__ partial) {
+  if (partial) {
+#pragma unroll
+    for (int c = 0; c < COLS; ++c) {
+      const int n = col(c);
+      if (n >= N) continue;
+      float* dst = partial + ((size_t)blockIdx.y * (GLU ? 2 : 1) + (GLU ? c / (COLS / 2) : 0)) * M * N + n;
+#pragma unroll
+      for (int q = 0; q < QUADS; ++q)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (row(q) + e < M) dst[(size_t)(row(q) + e) * N] = value(c, q, e);
+    }
+    return;
+  }
+  if (GLU) {
+#pragma unroll
+    for (int c = 0; c < COLS / 2; ++c) {
+      const int n = col(c);
+      if (n >= N) continue;
+#pragma unroll
+      for (int q = 0; q < QUADS; ++q)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (row(q) + e < M)
+            reinterpret_cast<bf16_t*>(out)[(size_t)(row(q) + e) * out_stride + n] =
+                float_to_bf16(swiglu1(value(c, q, e), value(c + COLS / 2, q, e)));
+    }
+    return;
+  }
+#pragma unroll
+  for (int c = 0; c < COLS; ++c) {
+    const int n = col(c);
+    if (n >= N) continue;
+    const float bv = bias ? load_vec(bias, bias_is_f32, n) : 0.0f;
+    if (mode == MODE_ADD_F32) {
+      // all reads of a column before its first store, which may alias the next read; rows past M read the last row and store nothing
+      float* rows = reinterpret_cast<float*>(out) + n;
+      float before[QUADS][4];
+#pragma unroll
+      for (int q = 0; q < QUADS; ++q)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) before[q][e] = rows[(size_t)min(row(q) + e, M - 1) * out_stride];
+#pragma unroll
+      for (int q = 0; q < QUADS; ++q)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (row(q) + e < M) rows[(size_t)(row(q) + e) * out_stride] = before[q][e] + (value(c, q, e) + bv);
+      continue;
+    }
+#pragma unroll
+    for (int q = 0; q < QUADS; ++q)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (row(q) + e >= M) continue;
+        const float v = value(c, q, e) + bv;
+        const size_t at = (size_t)(row(q) + e) * out_stride + n;
+        if (mode_stores_elem(mode)) reinterpret_cast<bf16_t*>(out)[at] = float_to_bf16(mode_value(v, mode));
+        else reinterpret_cast<float*>(out)[at] = v;
+      }
+  }
+}
+
+// The same for 16-bit outputs with a lane's four neighbouring columns, col(c) .. col(c) + 3, of row(q): one store of 8 bytes
+// instead of four of 2.
+template <bool GLU, int COLS, int ROWS, class Value, class Col, class Row>
+__device__ __forceinline__ void tile_epilogue_narrow(Value value, Col col, Row row, const void* __restrict__ bias, int bias_is_f32,
+                                                     bf16_t* __restrict__ out, int out_stride, int M, int N, int mode) {
+  const bool vec = N % 4 == 0 && out_stride % 4 == 0 && ((uintptr_t)out & 7) == 0;     // all four exist, rows and `out` are aligned
+#pragma unroll
+  for (int c = 0; c < (GLU ? COLS / 2 : COLS); ++c) {
+    const int n = col(c);
+    if (n >= N) continue;
+    float bv[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) bv[e] = !GLU && bias && n + e < N ? load_vec(bias, bias_is_f32, n + e) : 0.0f;
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+      const int m = row(r);
+      if (m >= M) continue;
+      float v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        v[e] = GLU ? swiglu1(value(c, r, e), value(c + (GLU ? COLS / 2 : 0), r, e)) : mode_value(value(c, r, e) + bv[e], mode);
+      bf16_t* dst = out + (size_t)m * out_stride + n;
+      if (vec) {
+        *reinterpret_cast<uint2*>(dst) = make_uint2(pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3]));
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (n + e < N) dst[e] = float_to_bf16(v[e]);
+      }
+    }
+  }
+}
+
 // ---------------------------------------------------------------------------- gemm_tile
 // LDS holds STAGES stages; a stage is 32 k: BM rows of X (64 bytes each) and the BN / 16 packed
 // blocks of W, written by direct global -> LDS loads of 16 bytes per lane (a wave instruction
@@ -109,7 +248,10 @@ __device__ inline void wait_rounds(int rounds) {
 //
 // KEEP: the block walks all `splits` segments of K itself; a segment's chains are added to the sums of those
 // before it in a second set of registers (the order of gemm_split_reduce), and no sums go through memory.
-template <int BM, int BN, int WAVES_M, int WAVES_N, bool GLU, int STAGES, bool KEEP>
+//
+// ACROSS: which operand of a product X and W are (the same bits), and so whether a lane holds one column of four rows or
+// four columns of a row.  The former for 32-bit outputs, sums of segments among them, the latter for 16-bit ones.
+template <int BM, int BN, int WAVES_M, int WAVES_N, bool GLU, int STAGES, bool KEEP, bool ACROSS>
 __global__ void __launch_bounds__(WAVES_M * WAVES_N * 64, KEEP || STAGES * (BM + BN) * 64 <= 80 * 1024 ? 2 : 1)
 gemm_tile_kernel(const bf16_t* __restrict__ x, int x_stride, const bf16_t* __restrict__ w, const void* __restrict__ bias,
                  int bias_is_f32, void* __restrict__ out, int out_stride, int M, int N, int K, int mode, int m_blocks,
@@ -131,37 +273,8 @@ gemm_tile_kernel(const bf16_t* __restrict__ x, int x_stride, const bf16_t* __res
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave / WAVES_N, wn = wave % WAVES_N;
 
-  // Block numbering: every eighth block runs on the same XCD, 32 of them at a time.  An XCD takes
-  // every eighth n block and walks its share in squares of up to 8 m blocks x 4 n blocks, so that
-  // the 32 blocks at work share 12 tiles of operands in that XCD's L2 (with many m blocks, all m
-  // blocks of one n block in a row would share 33), the squares of the same four n blocks one
-  // after the other.
-  const int bid = blockIdx.x;
   int mb, nb;
-  if (bid < (n_blocks / 8) * 8 * m_blocks) {
-    constexpr int GM = 8, GN = 4;
-    const int xcd = bid & 7, j = bid >> 3, mine = n_blocks / 8;       // this XCD's n blocks: xcd, xcd + 8, ...
-    const int whole_groups = mine / GN;
-    int g = j / (GN * m_blocks), rest = j % (GN * m_blocks), gn = GN;
-    if (g >= whole_groups) {                                          // the last, narrower group of n blocks
-      g = whole_groups;
-      rest = j - whole_groups * GN * m_blocks;
-      gn = mine - whole_groups * GN;
-    }
-    const int whole_rows = m_blocks / GM;
-    int ms = rest / (gn * GM), r = rest % (gn * GM), gm = GM;
-    if (ms >= whole_rows) {                                           // the last, shorter square
-      ms = whole_rows;
-      r = rest - whole_rows * gn * GM;
-      gm = m_blocks - whole_rows * GM;
-    }
-    mb = ms * GM + r % gm;
-    nb = (g * GN + r / gm) * 8 + xcd;
-  } else {  // the last, incomplete group of n blocks: plain order
-    const int r = bid - (n_blocks / 8) * 8 * m_blocks;
-    nb = (n_blocks / 8) * 8 + r / m_blocks;
-    mb = r % m_blocks;
-  }
+  tile_of_block(blockIdx.x, m_blocks, n_blocks, mb, nb);
   const int m0 = mb * BM, n0 = nb * (GLU ? BN / 2 : BN);
 
   // what this lane fetches: row r = (q * NW + wave) * 16 + lane / 4 of a tile; it fills slot
@@ -260,7 +373,8 @@ gemm_tile_kernel(const bf16_t* __restrict__ x, int x_stride, const bf16_t* __res
         __builtin_amdgcn_s_barrier();   // block kt + 1 is in LDS for every wave; nobody reads block kt any more
       }                                 // (behind the last block: whatever the stage holds is read and not used)
       const int i = t / TM, j = t % TM;
-      acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(wf[i / TH][i % TH]), as_frag(xf[set][j]), acc[i][j], 0, 0, 0);
+      const u32x4 xs = xf[set][j], ws = wf[i / TH][i % TH];
+      acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(ACROSS ? xs : ws), as_frag(ACROSS ? ws : xs), acc[i][j], 0, 0, 0);
       // a read behind each product: the second half's behind the first ones, the next block's behind those after the barrier
       if (t < TH) {
         __builtin_amdgcn_sched_barrier(0);
@@ -319,129 +433,14 @@ gemm_tile_kernel(const bf16_t* __restrict__ x, int x_stride, const bf16_t* __res
       for (int j = 0; j < TM; ++j) acc[i][j] = sum[i][j];
   }
 
-  // epilogue: a lane holds row m = lane % 16 and four consecutive columns n = 4 (lane / 16) .. of each tile
-  const int mrow = m0 + wm * WM + frow, ncol = n0 + wn * (GLU ? WN / 2 : WN) + (lane >> 4) * 4;
-  if (partial) {
-    // [split][gate | up][M][N] (one part without GLU), 32-bit sums as they are
-    constexpr int PARTS = GLU ? 2 : 1;
-#pragma unroll
-    for (int i = 0; i < TN; ++i) {
-      const int part = GLU ? i / TH : 0, n = ncol + (GLU ? i % TH : i) * 16;
-      if (n >= N) continue;
-      float* dst = partial + ((size_t)blockIdx.y * PARTS + part) * M * N + n;
-#pragma unroll
-      for (int j = 0; j < TM; ++j) {
-        const int m = mrow + j * 16;
-        if (m >= M) continue;
-        if (N % 4 == 0) {
-          *reinterpret_cast<f32x4*>(dst + (size_t)m * N) = acc[i][j];
-        } else {                                                   // rows of the workspace that are not 16-byte aligned
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (n + e < N) dst[(size_t)m * N + e] = acc[i][j][e];
-        }
-      }
-    }
-    return;
-  }
-  // four columns in one store: where all exist and rows and `out` are aligned for it
-  const bool narrow = mode_stores_elem(mode) || GLU;
-  const bool vec = N % 4 == 0 && out_stride % 4 == 0 && ((uintptr_t)out & (narrow ? 7 : 15)) == 0;
-  if (GLU) {
-#pragma unroll
-    for (int i = 0; i < TH; ++i) {
-      const int n = ncol + i * 16;
-      if (n >= N) continue;
-#pragma unroll
-      for (int j = 0; j < TM; ++j) {
-        const int m = mrow + j * 16;
-        if (m >= M) continue;
-        float v[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = swiglu1(acc[i][j][e], acc[i + TH][j][e]);
-        bf16_t* dst = reinterpret_cast<bf16_t*>(out) + (size_t)m * out_stride + n;
-        if (vec) {
-          *reinterpret_cast<uint2*>(dst) = make_uint2(pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3]));
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) dst[e] = float_to_bf16(v[e]);           // N is a multiple of 16
-        }
-      }
-    }
-    return;
-  }
-#pragma unroll
-  for (int i = 0; i < TN; ++i) {
-    const int n = ncol + i * 16;
-    if (n >= N) continue;
-    float bv[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) bv[e] = bias && n + e < N ? load_vec(bias, bias_is_f32, n + e) : 0.0f;
-    if (mode == MODE_ADD_F32) {
-      // All reads of a tile column before its first store, which may alias the next read: element by element a lane
-      // waits for memory at every one.  Rows past M read the last row and store nothing.
-      float* rows = reinterpret_cast<float*>(out) + n;
-      float before[TM][4];
-#pragma unroll
-      for (int j = 0; j < TM; ++j) {
-        const float* src = rows + (size_t)min(mrow + j * 16, M - 1) * out_stride;
-        if (vec) {
-          const f32x4 r = *reinterpret_cast<const f32x4*>(src);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) before[j][e] = r[e];
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) before[j][e] = n + e < N ? src[e] : 0.0f;
-        }
-      }
-#pragma unroll
-      for (int j = 0; j < TM; ++j) {
-        const int m = mrow + j * 16;
-        if (m >= M) continue;
-        f32x4 v;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = before[j][e] + (acc[i][j][e] + bv[e]);
-        if (vec) {
-          *reinterpret_cast<f32x4*>(rows + (size_t)m * out_stride) = v;
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (n + e < N) rows[(size_t)m * out_stride + e] = v[e];
-        }
-      }
-      continue;
-    }
-#pragma unroll
-    for (int j = 0; j < TM; ++j) {
-      const int m = mrow + j * 16;
-      if (m >= M) continue;
-      float v[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = acc[i][j][e] + bv[e];
-      const size_t at = (size_t)m * out_stride + n;
-      if (narrow) {
-        bf16_t* dst = reinterpret_cast<bf16_t*>(out) + at;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = mode_value(v[e], mode);
-        if (vec) {
-          *reinterpret_cast<uint2*>(dst) = make_uint2(pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3]));
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (n + e < N) dst[e] = float_to_bf16(v[e]);
-        }
-      } else {
-        float* dst = reinterpret_cast<float*>(out) + at;
-        if (vec) {
-          *reinterpret_cast<f32x4*>(dst) = f32x4{v[0], v[1], v[2], v[3]};
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (n + e < N) dst[e] = v[e];
-        }
-      }
-    }
-  }
+  const int mrow = m0 + wm * WM, ncol = n0 + wn * (GLU ? WN / 2 : WN), four = (lane >> 4) * 4;
+  const auto value = [&](int c, int r, int e) { return acc[c][r][e]; };
+  if constexpr (ACROSS)       // a lane holds column lane % 16 and four rows from 4 (lane / 16) on of each tile
+    tile_epilogue<GLU, TN, TM>(value, [&](int c) { return ncol + (GLU ? c % TH : c) * 16 + frow; }, [&](int r) { return mrow + r * 16 + four; },
+                               bias, bias_is_f32, out, out_stride, M, N, mode, partial);
+  else                        // row lane % 16 and four columns from 4 (lane / 16) on
+    tile_epilogue_narrow<GLU, TN, TM>(value, [&](int c) { return ncol + c * 16 + four; }, [&](int r) { return mrow + r * 16 + frow; }, bias,
+                                      bias_is_f32, reinterpret_cast<bf16_t*>(out), out_stride, M, N, mode);
 }
 
 // ---------------------------------------------------------------------------- gemm_small_tile
@@ -455,7 +454,7 @@ typedef __attribute__((ext_vector_type(16))) float f32x16;
 template <bool GLU, int STAGES>
 __global__ void __launch_bounds__(256, 1)
 gemm_small_tile_kernel(const bf16_t* __restrict__ x, int x_stride, const bf16_t* __restrict__ w, const void* __restrict__ bias,
-                 int bias_is_f32, void* __restrict__ out, int out_stride, int M, int N, int K, int mode, int m_blocks,
+                       int bias_is_f32, void* __restrict__ out, int out_stride, int M, int N, int K, int mode, int m_blocks,
                        int n_blocks, float* __restrict__ partial) {
   extern __shared__ __align__(16) unsigned char smem[];
   constexpr int BM = 128, BN = 128, WAVES_M = 2, WAVES_N = 2, BK = 64;
@@ -476,33 +475,8 @@ gemm_small_tile_kernel(const bf16_t* __restrict__ x, int x_stride, const bf16_t*
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave / WAVES_N, wn = wave % WAVES_N;
 
-  // (block numbering as in gemm_tile_kernel)
-  const int bid = blockIdx.x;
   int mb, nb;
-  if (bid < (n_blocks / 8) * 8 * m_blocks) {
-    constexpr int GM = 8, GN = 4;
-    const int xcd = bid & 7, j = bid >> 3, mine = n_blocks / 8;       // this XCD's n blocks: xcd, xcd + 8, ...
-    const int whole_groups = mine / GN;
-    int g = j / (GN * m_blocks), rest = j % (GN * m_blocks), gn = GN;
-    if (g >= whole_groups) {                                          // the last, narrower group of n blocks
-      g = whole_groups;
-      rest = j - whole_groups * GN * m_blocks;
-      gn = mine - whole_groups * GN;
-    }
-    const int whole_rows = m_blocks / GM;
-    int ms = rest / (gn * GM), r = rest % (gn * GM), gm = GM;
-    if (ms >= whole_rows) {                                           // the last, shorter square
-      ms = whole_rows;
-      r = rest - whole_rows * gn * GM;
-      gm = m_blocks - whole_rows * GM;
-    }
-    mb = ms * GM + r % gm;
-    nb = (g * GN + r / gm) * 8 + xcd;
-  } else {  // the last, incomplete group of n blocks: plain order
-    const int r = bid - (n_blocks / 8) * 8 * m_blocks;
-    nb = (n_blocks / 8) * 8 + r / m_blocks;
-    mb = r % m_blocks;
-  }
+  tile_of_block(blockIdx.x, m_blocks, n_blocks, mb, nb);
   const int m0 = mb * BM, n0 = nb * (GLU ? BN / 2 : BN);
 
   // what this lane fetches: row r = (q * NW + wave) * RPI + lane / SLOTS of a tile; it fills slot
@@ -636,82 +610,11 @@ gemm_small_tile_kernel(const bf16_t* __restrict__ x, int x_stride, const bf16_t*
   for (int kt = 0; kt + 1 < nk; ++kt) tile(kt, Number<0>());
   tile(nk - 1, Number<1>());
 #undef SWZ
-  // epilogue: lane holds column n = lane % 32 of each tile and rows (e/4)*8 + (lane/32)*4 + e%4
-  if (partial) {
-    // [split][gate | up][M][N] (one part without GLU), 32-bit sums as they are
-    constexpr int PARTS = GLU ? 2 : 1;
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const int part = GLU ? j / (TN / 2) : 0;
-      const int n = GLU ? n0 + wn * (WN / 2) + (j % (TN / 2)) * 32 + (lane & 31) : n0 + wn * WN + j * 32 + (lane & 31);
-      if (n >= N) continue;
-      float* dst = partial + ((size_t)blockIdx.y * PARTS + part) * M * N + n;
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int m = m0 + wm * WM + i * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
-          if (m < M) dst[(size_t)m * N] = acc[i][j][e];
-        }
-    }
-    return;
-  }
-  if (GLU) {
-#pragma unroll
-    for (int j = 0; j < TN / 2; ++j) {
-      const int n = n0 + wn * (WN / 2) + j * 32 + (lane & 31);
-      if (n >= N) continue;
-#pragma unroll
-      for (int i = 0; i < TM; ++i) {
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int m = m0 + wm * WM + i * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
-          if (m >= M) continue;
-          reinterpret_cast<bf16_t*>(out)[(size_t)m * out_stride + n] =
-              float_to_bf16(swiglu1(acc[i][j][e], acc[i][j + TN / 2][e]));
-        }
-      }
-    }
-    return;
-  }
-#pragma unroll
-  for (int j = 0; j < TN; ++j) {
-    const int n = n0 + wn * WN + j * 32 + (lane & 31);
-    if (n >= N) continue;
-    const float bv = bias ? load_vec(bias, bias_is_f32, n) : 0.0f;
-    if (mode == MODE_ADD_F32) {
-      // all reads before the first store, which may alias the next read; rows past M read the last row and store nothing
-      float* rows = reinterpret_cast<float*>(out) + n;
-      float before[TM][16];
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int m = m0 + wm * WM + i * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
-          before[i][e] = rows[(size_t)min(m, M - 1) * out_stride];
-        }
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int m = m0 + wm * WM + i * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
-          if (m < M) rows[(size_t)m * out_stride] = before[i][e] + (acc[i][j][e] + bv);
-        }
-      continue;
-    }
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int m = m0 + wm * WM + i * 32 + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3);
-        if (m >= M) continue;
-        const float v = acc[i][j][e] + bv;
-        const size_t at = (size_t)m * out_stride + n;
-        if (mode_stores_elem(mode)) reinterpret_cast<bf16_t*>(out)[at] = float_to_bf16(mode_value(v, mode));
-        else reinterpret_cast<float*>(out)[at] = v;
-      }
-    }
-  }
+  // a lane holds column lane % 32 of each tile, and of it rows 4 (lane / 32) .. of every eight
+  const int mrow = m0 + wm * WM + fhalf * 4, ncol = n0 + wn * (GLU ? WN / 2 : WN) + frow;
+  tile_epilogue<GLU, TN, TM * 4>([&](int c, int q, int e) { return acc[q / 4][c][q % 4 * 4 + e]; },
+                                 [&](int c) { return ncol + (GLU ? c % (TN / 2) : c) * 32; },
+                                 [&](int q) { return mrow + q * 8; }, bias, bias_is_f32, out, out_stride, M, N, mode, partial);
 }
 
 // The same for a width that is no multiple of 4 (rows of the workspace are then not 16-byte
@@ -915,42 +818,70 @@ static int add_split_sums(const float* partial, int splits, int m, int n, const 
   return 0;
 }
 
-template <int BM, int BN, int WAVES_M, int WAVES_N, bool GLU, int STAGES = 5, bool KEEP = false>
+// Lets a kernel take more LDS than a launch gets unasked, once.
+template <auto KERNEL>
+static int reserve_lds(int bytes) {
+  static bool configured = false;
+  if (configured) return 0;
+  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(KERNEL), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  if (e != hipSuccess) {
+    axk_set_error("gemm_tile: cannot reserve %d bytes of LDS: %s", bytes, hipGetErrorString(e));
+    return -2;
+  }
+  configured = true;
+  return 0;
+}
+
+// The tiles of gemm_tile, STAGES stages of 32 k.  A block a segment (gridDim.y), the sums through `partial`; or, with KEEP, a
+// block all of them, the finished sums through `partial` where the kernel that adds sums does more than that.
+//
+// Which way round (us, four columns of a row in a lane / columns across lanes).  16-bit outputs: 33,000 columns of K 1,024 at
+// 1,500 rows 147 / 182, kept 5,632 of K 2,048 65 / 73, gated 18,944 of K 3,584 at 2,048 rows 462 / 469.  32-bit ones: segments' sums
+// of 5,632 of K 2,048 at 320 rows 30.5 / 26.5, of 3,584 of K 3,584 at 688 43.8 / 39.9, kept and added into rows 3,584 of K 3,584
+// at 2,048 65.8 / 64.5.  Kept gated products, whose waves own 32 columns of the output, go the second way, too (1,408 of K 2,048 at
+// 2,048 rows 37.7 / 36.4).
+template <int BM, int BN, int WAVES_M, int WAVES_N, bool GLU, bool KEEP = false, int STAGES = 5>
 static int launch_tile(const bf16_t* x, int x_stride, const bf16_t* w, const void* bias, int bias_is_f32, void* out,
                        int out_stride, int m, int n, int k, int mode, hipStream_t stream, int segs = 1,
                        float* partial = nullptr, const SplitNorm* norm = nullptr, const RopeStore* rope = nullptr) {
-  static bool configured = false;
-  constexpr bool SMALL = BM == 128 && !KEEP;           // (kept segments fill the chip: 5,632 columns of K 2,048 at 688 rows 42 -> 37 us)
-  constexpr int lds_bytes = STAGES * (BM + BN) * (SMALL ? 128 : 64);
+  constexpr int lds_bytes = STAGES * (BM + BN) * 64;
   static_assert(lds_bytes <= 160 * 1024, "the stages do not fit the LDS of a CU");
-  const void* kernel;
-  if constexpr (SMALL) kernel = reinterpret_cast<const void*>(&gemm_small_tile_kernel<GLU, STAGES>);
-  else kernel = reinterpret_cast<const void*>(&gemm_tile_kernel<BM, BN, WAVES_M, WAVES_N, GLU, STAGES, KEEP>);
-  if (!configured) {
-    hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
-    if (e != hipSuccess) {
-      axk_set_error("gemm_tile: cannot reserve %d bytes of LDS: %s", lds_bytes, hipGetErrorString(e));
-      return -2;
-    }
-    configured = true;
-  }
-  // a block a segment (gridDim.y), the sums through `partial`; or a block all of them, the finished sums through
-  // `partial` where the kernel that adds sums does more than that
   const int splits = KEEP ? 1 : segs;
   const bool after = splits > 1 || norm || rope;
   const int m_blocks = ceil_div(m, BM), n_blocks = ceil_div(n, GLU ? BN / 2 : BN);
   if constexpr (KEEP) AXK_INSTANCE(INST_GEMM_KEPT, GLU);
-  else AXK_INSTANCE(INST_GEMM_TILE, BM, BN, WAVES_M, WAVES_N, GLU, SMALL ? STAGES : STAGES / 2);
-  const dim3 grid(m_blocks * n_blocks, splits);
-  float* sums = after ? partial : nullptr;
-  if constexpr (SMALL)
-    gemm_small_tile_kernel<GLU, STAGES><<<grid, 256, lds_bytes, stream>>>(x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode,
-                                                                          m_blocks, n_blocks, sums);
-  else
-    gemm_tile_kernel<BM, BN, WAVES_M, WAVES_N, GLU, STAGES, KEEP><<<grid, WAVES_M * WAVES_N * 64, lds_bytes, stream>>>(
-        x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode, m_blocks, n_blocks, sums, segs);
-  AXK_LAUNCH_CHECK("gemm_tile");
+  else AXK_INSTANCE(INST_GEMM_TILE, BM, BN, WAVES_M, WAVES_N, GLU, STAGES * 32 / 64);
+  auto go = [&](auto across) {
+    constexpr auto kernel = &gemm_tile_kernel<BM, BN, WAVES_M, WAVES_N, GLU, STAGES, KEEP, decltype(across)::value>;
+    if (int rc = reserve_lds<kernel>(lds_bytes)) return rc;
+    kernel<<<dim3(m_blocks * n_blocks, splits), WAVES_M * WAVES_N * 64, lds_bytes, stream>>>(
+        x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode, m_blocks, n_blocks, after ? partial : nullptr, segs);
+    AXK_LAUNCH_CHECK("gemm_tile");
+    return 0;
+  };
+  int rc;
+  if constexpr (KEEP && GLU) rc = go(std::true_type());
+  else rc = after || !(GLU || mode_stores_elem(mode)) ? go(std::true_type()) : go(std::false_type());
+  if (rc) return rc;
   return after ? add_split_sums(partial, splits, m, n, bias, bias_is_f32, out, out_stride, mode, norm, rope, stream) : 0;
+}
+
+// The tiles of gemm_small_tile, STAGES stages of 64 k, a block a segment.
+template <bool GLU, int STAGES>
+static int launch_small_tile(const bf16_t* x, int x_stride, const bf16_t* w, const void* bias, int bias_is_f32, void* out,
+                             int out_stride, int m, int n, int k, int mode, hipStream_t stream, int segs,
+                             float* partial, const SplitNorm* norm = nullptr, const RopeStore* rope = nullptr) {
+  constexpr int lds_bytes = STAGES * (128 + 128) * 128;
+  static_assert(lds_bytes <= 160 * 1024, "the stages do not fit the LDS of a CU");
+  const bool after = segs > 1 || norm || rope;
+  const int m_blocks = ceil_div(m, 128), n_blocks = ceil_div(n, GLU ? 64 : 128);
+  AXK_INSTANCE(INST_GEMM_TILE, 128, 128, 2, 2, GLU, STAGES);
+  constexpr auto kernel = &gemm_small_tile_kernel<GLU, STAGES>;
+  if (int rc = reserve_lds<kernel>(lds_bytes)) return rc;
+  kernel<<<dim3(m_blocks * n_blocks, segs), 256, lds_bytes, stream>>>(x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode,
+                                                                      m_blocks, n_blocks, after ? partial : nullptr);
+  AXK_LAUNCH_CHECK("gemm_tile");
+  return after ? add_split_sums(partial, segs, m, n, bias, bias_is_f32, out, out_stride, mode, norm, rope, stream) : 0;
 }
 
 // ---------------------------------------------------------------------------- gemm_stream
@@ -2098,9 +2029,10 @@ static int tiles32_of(int n, int mode) { return mode == MODE_SWIGLU ? n / 16 : (
 #define GEMM_PASS_BYTES ((size_t)2048 << 20)
 
 // Whether the blocks of a product of more than 128 rows walk all of K themselves, in tiles of 128 x 128, and keep the
-// segments' sums in registers; else a block takes a segment and its sums go through the workspace.  Both timed for 32
-// shapes of 140 to 8,192 rows: every epilogue is the faster one here wherever this says so (766 measurements, at the
-// median 0.75 of the time) but for one store of 900 rows of 16,384 columns of K 3,072 in two segments (132 against 124 us).
+// segments' sums in registers; else a block takes a segment and its sums go through the workspace.  Where the lines
+// lie was found with tiles of 32x32x16 products (32 shapes of 140 to 8,192 rows, 766 measurements, of which the figures
+// below are), and the present tiles, which gained more here than there, were timed against it: of the products of 14 matrices
+// of 200 to 2,048 rows the 42 that keep their sums take 0.57 to 0.94 of the time.
 //  * There have to be blocks for the chip's 256 CUs.  K 2,048, 2,560 columns of 1,525 rows (240 blocks) 35 against 38 us,
 //    2,048 of 1,525 (192) 35 against 33; K 3,584, 3,584 of 1,200 (280) 63 against 71, 900 (224) 52 against 49.  Gated,
 //    1,408 of 700 (132) 27 against 28, of 900 (176) 27 against 30; 1,024 of 900 (128) 27 against 22.
@@ -2238,15 +2170,15 @@ static int gemm_mfma_pass(const bf16_t* x, int x_stride, const bf16_t* w, const 
   // 256 x 256 tiles (8 waves, a block a CU) or 128 x 128 tiles (4 waves, two blocks a CU, four
   // times as many blocks at twice the traffic from L2 per product): whichever takes the chip's 256
   // CUs fewer rounds, a round of the small tiles counted as 0.65 of a round of the large ones
-  // (measured on the four products of the 7B and 14B layers at 200 to 2,048 rows: the rule picks
-  // the faster tile in 66 of 70 cases and loses 7 % at most in the others).
+  // (both timed for 14 matrices, those of the 7B and 14B layers among them, at 200 to 2,048 rows: of 140
+  // products that do not keep their segments' sums one takes the slower tile, by 4 %, [gate; up] of 600 rows).
   const long big = (long)ceil_div(m, 256) * ceil_div(n, glu ? 128 : 256) * segs;
   const long small = (long)ceil_div(m, 128) * ceil_div(n, glu ? 64 : 128) * segs;
   const long rounds_big = (big + 255) / 256, rounds_small = (small + 511) / 512;
   const bool use_big = rounds_big * 100 <= rounds_small * 65;
   if (keep) {
-    if (glu) return launch_tile<128, 128, 2, 2, true, 5, true>(ARGS, segs, ws);
-    return launch_tile<128, 128, 2, 2, false, 5, true>(ARGS, segs, ws, norm, rope_after);
+    if (glu) return launch_tile<128, 128, 2, 2, true, true>(ARGS, segs, ws);
+    return launch_tile<128, 128, 2, 2, false, true>(ARGS, segs, ws, norm, rope_after);
   }
   if (!use_big) {
     // Up to 256 rows still wait for W more than for the matrix cores.  Where the small tiles are no
@@ -2255,11 +2187,11 @@ static int gemm_mfma_pass(const bf16_t* x, int x_stride, const bf16_t* w, const 
     // more blocks two of them share a CU and cover each other's waits (four stages there: slower).
     const bool deep = m <= 256 && small <= 256;
     if (glu) {
-      if (deep) return launch_tile<128, 128, 2, 2, true, 4>(ARGS, segs, ws);
-      return launch_tile<128, 128, 2, 2, true, 2>(ARGS, segs, ws);
+      if (deep) return launch_small_tile<true, 4>(ARGS, segs, ws);
+      return launch_small_tile<true, 2>(ARGS, segs, ws);
     }
-    if (deep) return launch_tile<128, 128, 2, 2, false, 4>(ARGS, segs, ws, norm, rope_after);
-    return launch_tile<128, 128, 2, 2, false, 2>(ARGS, segs, ws, norm, rope_after);
+    if (deep) return launch_small_tile<false, 4>(ARGS, segs, ws, norm, rope_after);
+    return launch_small_tile<false, 2>(ARGS, segs, ws, norm, rope_after);
   }
   if (glu) return launch_tile<256, 256, 4, 2, true>(ARGS, segs, ws);
   // one round of 256 x 256 tiles that leaves a quarter of the CUs idle, and N in whole tiles of

@@ -37,3 +37,25 @@ def model_dirs(tmp_path_factory):
         return made[key]
 
     return get
+
+
+@pytest.fixture(scope="session")
+def device_code(tmp_path_factory):
+    """The bfloat16 device code of a source under csrc, as text, compiled once a session; no GPU is needed."""
+    import shutil
+    import subprocess
+
+    from axon_amd.kernels import build as B
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not os.path.exists(hipcc):
+        pytest.skip("no compiler")
+    made = {}
+
+    def of(source):
+        if source not in made:
+            out = tmp_path_factory.mktemp("device") / (source + ".s")
+            subprocess.run([hipcc, *B.HIP_FLAGS, B.DTYPE_FLAG["bfloat16"], "-S", "--cuda-device-only", os.path.join(B.CSRC, source), "-o", str(out)],
+                           check=True, capture_output=True, timeout=600)
+            made[source] = out.read_text()
+        return made[source]
+    return of

@@ -1,27 +1,34 @@
-"""Kernels whose speed rests on how many of their waves a SIMD holds: their registers, from the device code's own notes.  A
-SIMD has 512 registers a lane and hands them out to a wave in eights, so 128 are four waves."""
-import os
+"""What the device code shows of kernels whose speed rests on it: how many waves a SIMD holds, and how outputs are stored."""
 import re
-import shutil
-import subprocess
 
 import pytest
 
-from axon_amd.kernels import build as B
+
+def functions(assembly, kernel):
+    """{an instance of the kernel: its instructions}."""
+    found = {name: body for name, body in re.findall(r"^(\w+):\s*; @\S+\n(.*?)^\.Lfunc_end", assembly, re.S | re.M) if kernel in name}
+    assert found
+    return found
 
 
-@pytest.mark.skipif(shutil.which("hipcc") is None and not os.path.exists("/opt/rocm/bin/hipcc"), reason="no compiler")
 @pytest.mark.parametrize("source, kernel, most", [("attention_mfma.hip", "attention_combine_kernel", 128)])
-def test_registers_leave_room_for_the_waves(tmp_path, source, kernel, most):
-    out = tmp_path / "device.s"
-    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
-    done = subprocess.run([hipcc, *B.HIP_FLAGS, B.DTYPE_FLAG["bfloat16"], "-I", B.CSRC, "-S", "--cuda-device-only", "-o", str(out),
-                           os.path.join(B.CSRC, source)], capture_output=True, text=True)
-    assert done.returncode == 0, done.stderr
+def test_registers_leave_room_for_the_waves(device_code, source, kernel, most):
+    """A SIMD has 512 registers a lane and hands them out to a wave in eights, so 128 are four waves."""
     seen = 0
-    for note in re.findall(r"- \.agpr_count:.*?\.wavefront_size:", out.read_text(), re.S):
+    for note in re.findall(r"- \.agpr_count:.*?\.wavefront_size:", device_code(source), re.S):
         field = {k: v for k, v in re.findall(r"\.(\w+):\s+(\S+)", note)}
         if kernel in field["symbol"]:
             seen += 1
             assert int(field["vgpr_count"]) <= most and int(field["private_segment_fixed_size"]) == 0, field
     assert seen
+
+
+def test_tiles_store_32_bit_values_across_lanes(device_code):
+    """A 16-byte store whose lanes hold four columns of sixteen rows each meets 64 lines, four stores of 4 bytes whose lanes hold
+    sixteen columns meet 16: 32-bit outputs and segments' sums leave the tiles that way, 16-bit ones in 8 bytes a lane."""
+    wide = 0
+    for name, body in functions(device_code("gemm_mfma.hip"), "gemm_tile_kernel").items():
+        stores = set(re.findall(r"\b(global_store_\w+)", body))
+        assert "global_store_dwordx4" not in stores, name
+        wide += "global_store_dword" in stores and "global_store_dwordx2" not in stores
+    assert wide >= 4                  # both tiles, gated and not, or kept

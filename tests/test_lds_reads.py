@@ -2,14 +2,9 @@
 once: nothing may touch these before the wait that the kernel writes behind them, and no branch may lie between, where the
 compiler is free to move registers.  The device code of the sources that write such reads is compiled to text and looked
 over, in straight lines; no GPU is needed."""
-import os
 import re
-import shutil
-import subprocess
 
 import pytest
-
-from axon_amd.kernels import build as B
 
 FUNCTION = re.compile(r"^(\w+):\s*; @\S+\n(.*?)^\.Lfunc_end", re.S | re.M)
 
@@ -53,23 +48,6 @@ def unwaited(assembly, kernel):
     return reads, faults
 
 
-@pytest.fixture(scope="module")
-def assembly(tmp_path_factory):
-    """The device code of a source, compiled once for all of its kernels."""
-    made = {}
-
-    def of(source):
-        if source not in made:
-            out = tmp_path_factory.mktemp("device") / (source + ".s")
-            hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
-            subprocess.run([hipcc, *B.HIP_FLAGS, B.DTYPE_FLAG["bfloat16"], "-S", "--cuda-device-only", os.path.join(B.CSRC, source), "-o", str(out)],
-                           check=True, capture_output=True, timeout=600)
-            made[source] = out.read_text()
-        return made[source]
-    return of
-
-
-@pytest.mark.skipif(shutil.which("hipcc") is None and not os.path.exists("/opt/rocm/bin/hipcc"), reason="no compiler")
 @pytest.mark.parametrize("source, kernel", [("grouped_gemm.hip", "grouped_gemm_tile_kernel"),
                                             ("latent_attention.hip", "latent_attention_prompt_kernel"),
                                             ("gemm_mfma.hip", "gemm_tile_kernel"),
@@ -78,8 +56,8 @@ def assembly(tmp_path_factory):
                                             ("attention_mfma.hip", "attention_prefill_kernel"),
                                             ("attention_mfma.hip", "attention_decode_kernel"),
                                             ("state_space.hip", "state_space_walk_kernel")])
-def test_nothing_comes_between_a_read_and_its_wait(assembly, source, kernel):
-    reads, faults = unwaited(assembly(source), kernel)
+def test_nothing_comes_between_a_read_and_its_wait(device_code, source, kernel):
+    reads, faults = unwaited(device_code(source), kernel)
     assert reads > 0 and not faults, faults[:5]
 
 
