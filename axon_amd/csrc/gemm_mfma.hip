@@ -924,44 +924,61 @@ enum { EPI_PLAIN = 0, EPI_GLU = 1, EPI_ROPE = 2 };
 // over its whole width.
 //
 // Bound by memory once the stores of V are: values lie [dim][slot], so a token alone writes two bytes of a line that
-// seven other XCDs write their two bytes of.  A thread of the prompt form keeps eight neighbouring tokens and writes a
-// dim's eight slots at once where they are eight of one page (token by token where a request ends among them or the
-// tokens are not aligned to the page): 2,048 tokens of 36 heads, one sum each, 23.2 -> 17.2 us, 1,525 of 56, four sums each, 49 -> 45.
+// seven other XCDs write their two bytes of.  In the prompt form a block takes eight neighbouring tokens, and of the values
+// the runs of slots that begin among them, wherever that is: a run is the tokens of one request from a position divisible by
+// eight (or the request's first of the step) up to the next such, so that up to seven of its tokens may lie in the
+// block behind.  A run of eight slots of a page leaves as 16 bytes of a dim, a shorter one slot by slot.  us, a token a thread /
+// eights counted from the step's first token, which only an aligned request fits / here: 28 and 2 x 4 heads, 2,048 tokens
+// 17.8 / 13.2 / 13.4, requests of 5 and 4,091 30.3 / 37.7 / 22.4; 40 and 2 x 8 heads, 2,048 tokens 31 / 18 / 18, 6,000 116 / 68 / 56,
+// 5 and 4,091 65 / 78 / 39, 110 of 37 68 / 74 / 46; four requests of 1,525 tokens in all, four sums each, 39.2 / 38.1 / 40.6.
 template <int TOKENS>
 __global__ void __launch_bounds__(256)
 gemm_split_reduce_rope_kernel(const float* __restrict__ partial, int splits, int M, int N, const void* __restrict__ bias,
                               int bias_is_f32, bf16_t* __restrict__ out, int out_stride, RopeStore rope) {
   const int hd = rope.head_dim, half = hd / 2, per_head = half / 4;     // threads a head
   const int heads_a_block = 256 / per_head;
-  const int m0 = blockIdx.x * TOKENS, within = threadIdx.x / per_head, slot = blockIdx.y * heads_a_block + within;
+  // (the last group of heads first: the values, whose waves wait for where their runs begin)
+  const int m0 = blockIdx.x * TOKENS, within = threadIdx.x / per_head, slot0 = (gridDim.y - 1 - blockIdx.y) * heads_a_block;
+  const int slot = slot0 + within, first_value = rope.n_heads + rope.n_kv_heads;
   const int d = (threadIdx.x % per_head) * 4;
+  // of the tokens from m0 on, one a lane (sixteen, again and again), in waves with value heads: position, page, and whether a
+  // run begins there
+  int pos_at = 0, page_at = 0;
+  unsigned begins = 1;                 // bit t: a run begins at token m0 + t (bit 16, and past the last token: set)
+  if (TOKENS == 8 && slot0 + (int)(threadIdx.x | 63) / per_head >= first_value) {
+    const int mine = m0 + (threadIdx.x & 15), at = min(mine, M - 1), before = max(at - 1, 0);
+    pos_at = rope.positions[at];
+    const int pos_before = rope.positions[before], seq_at = rope.seq_rows[at], seq_before = rope.seq_rows[before];
+    page_at = rope.block_table[(size_t)seq_at * rope.table_stride + pos_at / rope.page_size];
+    begins = (unsigned)(__ballot(mine >= M || pos_at % 8 == 0 || mine == 0 || seq_before != seq_at || pos_before != pos_at - 1) & 0xffff) | 0x10000;
+  }
   if (within >= heads_a_block || slot * hd >= N) return;
   const size_t plane = (size_t)M * N;
   const int col = slot * hd + d;
-  // four columns' sums of every token (of tokens past the last the last's again), rounded as the product's own store
-  // rounds them
+  float bl[4], bh[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    bl[e] = bias ? load_vec(bias, bias_is_f32, col + e) : 0.0f;
+    bh[e] = bias ? load_vec(bias, bias_is_f32, col + half + e) : 0.0f;
+  }
+  // four columns' sums of `count` tokens from `first` on (the last one's again past them), rounded as the product's own
+  // store rounds them
   float a[TOKENS][4], b[TOKENS][4];
-  {
+  auto sums = [&](int first, int count) {
     f32x4 lo[TOKENS], hi[TOKENS];
 #pragma unroll
     for (int t = 0; t < TOKENS; ++t) {
-      const float* src = partial + (size_t)min(m0 + t, M - 1) * N + col;
+      const float* src = partial + (size_t)(first + min(t, count - 1)) * N + col;
       lo[t] = *reinterpret_cast<const f32x4*>(src);
       hi[t] = *reinterpret_cast<const f32x4*>(src + half);
     }
     for (int z = 1; z < splits; ++z) {
 #pragma unroll
       for (int t = 0; t < TOKENS; ++t) {
-        const float* src = partial + (size_t)z * plane + (size_t)min(m0 + t, M - 1) * N + col;
+        const float* src = partial + (size_t)z * plane + (size_t)(first + min(t, count - 1)) * N + col;
         lo[t] += *reinterpret_cast<const f32x4*>(src);
         hi[t] += *reinterpret_cast<const f32x4*>(src + half);
       }
-    }
-    float bl[4], bh[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      bl[e] = bias ? load_vec(bias, bias_is_f32, col + e) : 0.0f;
-      bh[e] = bias ? load_vec(bias, bias_is_f32, col + half + e) : 0.0f;
     }
 #pragma unroll
     for (int t = 0; t < TOKENS; ++t)
@@ -970,55 +987,77 @@ gemm_split_reduce_rope_kernel(const float* __restrict__ partial, int splits, int
         a[t][e] = bf16_to_float(float_to_bf16(bias ? lo[t][e] + bl[e] : lo[t][e]));
         b[t][e] = bf16_to_float(float_to_bf16(bias ? hi[t][e] + bh[e] : hi[t][e]));
       }
-  }
-  int pos[TOKENS], page[TOKENS];
-  if (slot >= rope.n_heads) {
-#pragma unroll
-    for (int t = 0; t < TOKENS; ++t) {
-      const int m = min(m0 + t, M - 1);
-      pos[t] = rope.positions[m];
-      page[t] = rope.block_table[(size_t)rope.seq_rows[m] * rope.table_stride + pos[t] / rope.page_size];
-    }
-  }
-  if (slot >= rope.n_heads + rope.n_kv_heads) {
-    const int kvh = slot - rope.n_heads - rope.n_kv_heads;
+  };
+  auto page_of = [&](int m, int pos) {
+    return rope.block_table[(size_t)rope.seq_rows[m] * rope.table_stride + pos / rope.page_size];
+  };
+  if (slot >= first_value) {
+    const int kvh = slot - first_value;
     const size_t head_at = (size_t)kvh * hd * rope.page_size, page_elems = (size_t)rope.n_kv_heads * hd * rope.page_size;
-    if (TOKENS == 8) {
-      // eight slots of one page, as 16 bytes of a dim (the pages' dims are then 16-byte aligned)
-      bool whole = m0 + TOKENS <= M && rope.page_size % 8 == 0 && pos[0] % 8 == 0 && ((uintptr_t)rope.v_cache & 15) == 0;
+    // tokens `from` to `to` of those in a and b, the first of which is m0 + `first`, slot by slot
+    auto put = [&](int first, int from, int to) {
 #pragma unroll
-      for (int t = 1; t < TOKENS; ++t) whole = whole && pos[t] == pos[0] + t && page[t] == page[0];
-      if (whole) {
-        bf16_t* vdst = rope.v_cache + (size_t)page[0] * page_elems + head_at + pos[0] % rope.page_size;
+      for (int t = 0; t < TOKENS; ++t) {
+        if (t < from || t >= to) continue;
+        const int pos = TOKENS == 1 ? rope.positions[m0] : __builtin_amdgcn_readlane(pos_at, first + t);
+        const int page = TOKENS == 1 ? page_of(m0, pos) : __builtin_amdgcn_readlane(page_at, first + t);
+        bf16_t* vdst = rope.v_cache + (size_t)page * page_elems + head_at + pos % rope.page_size;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          uint4 lo, hi;
-          lo.x = pack2_bf16(a[0][e], a[1 % TOKENS][e]);
-          lo.y = pack2_bf16(a[2 % TOKENS][e], a[3 % TOKENS][e]);
-          lo.z = pack2_bf16(a[4 % TOKENS][e], a[5 % TOKENS][e]);
-          lo.w = pack2_bf16(a[6 % TOKENS][e], a[7 % TOKENS][e]);
-          hi.x = pack2_bf16(b[0][e], b[1 % TOKENS][e]);
-          hi.y = pack2_bf16(b[2 % TOKENS][e], b[3 % TOKENS][e]);
-          hi.z = pack2_bf16(b[4 % TOKENS][e], b[5 % TOKENS][e]);
-          hi.w = pack2_bf16(b[6 % TOKENS][e], b[7 % TOKENS][e]);
-          *reinterpret_cast<uint4*>(vdst + (size_t)(d + e) * rope.page_size) = lo;
-          *reinterpret_cast<uint4*>(vdst + (size_t)(half + d + e) * rope.page_size) = hi;
+          vdst[(size_t)(d + e) * rope.page_size] = float_to_bf16(a[t][e]);
+          vdst[(size_t)(half + d + e) * rope.page_size] = float_to_bf16(b[t][e]);
         }
-        return;
       }
+    };
+    if (TOKENS == 1) {
+      sums(m0, 1);
+      put(0, 0, 1);
+      return;
     }
-#pragma unroll
-    for (int t = 0; t < TOKENS; ++t) {
-      if (m0 + t >= M) break;
-      bf16_t* vdst = rope.v_cache + (size_t)page[t] * page_elems + head_at + pos[t] % rope.page_size;
+    const int tokens = min(TOKENS, M - m0);
+    const unsigned here = begins & ((1u << tokens) - 1);
+    if (here == 0) return;                                             // all of them belong to a run that the block before has
+    const int last = 31 - __builtin_clz(here), count = __builtin_ctz(begins >> (last + 1)) + 1;     // the last run that begins here
+    const bool apart = last + count > tokens || count == TOKENS;       // it goes on behind these tokens, or is a whole eight
+    const int to = apart ? last : last + count, from = __builtin_ctz(here);
+    if (from < to) {
+      sums(m0, tokens);
+      put(0, from, to);
+    }
+    if (!apart) return;
+    sums(m0 + last, count);
+    const int pos = __builtin_amdgcn_readlane(pos_at, last);
+    // (the pages' dims are 16-byte aligned if the first one's are)
+    if (count == TOKENS && pos % 8 == 0 && rope.page_size % 8 == 0 && ((uintptr_t)rope.v_cache & 15) == 0) {
+      bf16_t* vdst = rope.v_cache + (size_t)__builtin_amdgcn_readlane(page_at, last) * page_elems + head_at + pos % rope.page_size;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        vdst[(size_t)(d + e) * rope.page_size] = float_to_bf16(a[t][e]);
-        vdst[(size_t)(half + d + e) * rope.page_size] = float_to_bf16(b[t][e]);
+        uint4 lo, hi;
+        lo.x = pack2_bf16(a[0][e], a[1 % TOKENS][e]);
+        lo.y = pack2_bf16(a[2 % TOKENS][e], a[3 % TOKENS][e]);
+        lo.z = pack2_bf16(a[4 % TOKENS][e], a[5 % TOKENS][e]);
+        lo.w = pack2_bf16(a[6 % TOKENS][e], a[7 % TOKENS][e]);
+        hi.x = pack2_bf16(b[0][e], b[1 % TOKENS][e]);
+        hi.y = pack2_bf16(b[2 % TOKENS][e], b[3 % TOKENS][e]);
+        hi.z = pack2_bf16(b[4 % TOKENS][e], b[5 % TOKENS][e]);
+        hi.w = pack2_bf16(b[6 % TOKENS][e], b[7 % TOKENS][e]);
+        *reinterpret_cast<uint4*>(vdst + (size_t)(d + e) * rope.page_size) = lo;
+        *reinterpret_cast<uint4*>(vdst + (size_t)(half + d + e) * rope.page_size) = hi;
       }
+    } else {
+      put(last, 0, count);
     }
     return;
   }
+  int pos[TOKENS], page[TOKENS];       // of a key, ahead of the first store, which may alias the next read
+  if (slot >= rope.n_heads) {
+#pragma unroll
+    for (int t = 0; t < TOKENS; ++t) {
+      pos[t] = rope.positions[min(m0 + t, M - 1)];
+      page[t] = page_of(min(m0 + t, M - 1), pos[t]);
+    }
+  }
+  sums(m0, min(TOKENS, M - m0));
 #pragma unroll
   for (int t = 0; t < TOKENS; ++t) {
     const int m = m0 + t;
@@ -1047,14 +1086,16 @@ static int launch_split_reduce_rope(const float* partial, int splits, int m, int
   const int heads_a_block = 256 / (rope.head_dim / 8);
   const int head_blocks = ceil_div(n / rope.head_dim, heads_a_block);
   // Eight tokens a thread where that still is two and a half blocks a CU.  The product with its rotation, a token a thread
-  // against eight (us): 28 heads and 2 x 4 at 688 rows (258 blocks) 47 / 57, 16 and 2 x 2 at 1,024 (256) 34 / 46, at 2,048 (512)
-  // 48 / 50, 28 and 2 x 4 at 4,096 (1,536) 190 / 185.
-  if ((long)ceil_div(m, 8) * head_blocks >= 640)
+  // against eight (us, measured before the runs of slots): 28 heads and 2 x 4 at 688 rows (258 blocks) 47 / 57, 16 and 2 x 2 at
+  // 1,024 (256) 34 / 46, at 2,048 (512) 48 / 50, 28 and 2 x 4 at 4,096 (1,536) 190 / 185.
+  if ((long)ceil_div(m, 8) * head_blocks >= 640) {
+    AXK_INSTANCE(INST_GEMM_SPLIT_REDUCE, 2, 8);
     gemm_split_reduce_rope_kernel<8><<<dim3(ceil_div(m, 8), head_blocks), 256, 0, stream>>>(partial, splits, m, n, bias, bias_is_f32,
                                                                                             (bf16_t*)out, out_stride, rope);
-  else
+  } else {
     gemm_split_reduce_rope_kernel<1><<<dim3(m, head_blocks), 256, 0, stream>>>(partial, splits, m, n, bias, bias_is_f32, (bf16_t*)out,
                                                                                out_stride, rope);
+  }
   AXK_LAUNCH_CHECK("gemm_split_reduce_rope");
   return 0;
 }

@@ -415,6 +415,7 @@ CASES = [
     (BF, ["gemm_rows<1,4,2,0>", "gemm_split_reduce<3>"], check_gemm, (BF, 48, 130, 1024, MODE_STORE_F32, True)),   # N % 4 != 0
     (BF, ["gemm_rows<1,4,4,0>", "gemm_split_reduce<1>"], check_then_norm, (64, 3584, 1024)),
     (BF, ["gemm_rows<1,4,5,0>", "gemm_split_reduce<2>"], check_qkv_rope, (64, 28, 4, 128, 3584, 64)),
+    (BF, ["gemm_split_reduce<2,8>"], check_qkv_rope, (2056, 36, 4, 128, 512, 16)),
     # 65 to 128 rows: the same kernel with eight tiles of 16 rows of X a step
     (BF, ["gemm_rows<1,8,3,0>"], check_gemm, (BF, 65, 100, 128, MODE_STORE, True)),
     (BF, ["gemm_rows<1,8,3,0>", "gemm_split_reduce<0>"], check_gemm, (BF, 97, 4100, 512, MODE_STORE_F32, True)),
