@@ -108,7 +108,7 @@ int axk_pack_matrix(const void* src, void* dst, int rows, int k, void* stream);
 // through it (at most 2 GB: a product of more rows than that holds runs in passes).
 //
 // With a packed W every output element is the sum, in ascending order, of axk_gemm_segments(n, k,
-// gated) chains of 32x32x16 MFMAs over contiguous segments of K: the bits of a row do not depend on
+// gated) chains of 16x16x32 MFMAs over contiguous segments of K: the bits of a row do not depend on
 // M, that is, on what else is in the batch.
 long axk_gemm_workspace(int m, int n, int k, int mode);
 int axk_gemm_segments(int n, int k, int gated);

@@ -236,10 +236,11 @@ __device__ __forceinline__ void tile_epilogue_narrow(Value value, Col col, Row r
 //    the wave at their issue until the path into LDS (some 59 bytes a cycle) had taken them: a
 //    block of 256 x 256 x 64 took 3,300 cycles of which 2,048 are products; loads spread 3,020,
 //    reads spread too 2,900.
-// [gate; up] of 8,192 rows (18,944 columns of K 3,584) 2,040 -> 1,803 us (1.23 PFLOP/s), of 2,048 rows 613 ->
-// 547; 3,584 columns of K 18,944 at 2,048 rows (with the sums' kernel) 381 -> 340; 2,048^3 38 -> 32 us, 1,500 rows
-// of 33,000 columns of K 1,024 208 -> 156 (four columns a store).  Slower: waves of 128 x 64 (573 against 547
-// us); four waves of 128 x 128 do not fit the registers beside their fragments.
+// us, tiles of 32x32x16 products in steps of 64 k / here, in turn on one card: [gate; up] of 8,192 rows (18,944 columns of K
+// 3,584) 1,944 / 1,729 (1.29 PFLOP/s), of 2,048 rows 515 / 461; 3,584 columns of K 18,944 at 2,048 rows (with the
+// sums' kernel) 300 / 286; 2,048^3 37.0 / 29.5; 1,500 rows of 33,000 columns of K 1,024 190 / 133 (four columns a
+// store).  Where the output is narrow and K long it loses: 2,048 columns of K 8,448 at 8,192 rows 365 / 390.  Slower: waves
+// of 128 x 64 (573 against 547 us); four waves of 128 x 128 do not fit the registers beside their fragments.
 //
 // GLU: W holds 2 N rows (gate rows, then up rows) and the output is silu(gate) * up, N wide.
 // A block then owns BN / 2 output columns; each wave's share of the LDS tile holds the gate
@@ -447,7 +448,7 @@ gemm_tile_kernel(const bf16_t* __restrict__ x, int x_stride, const bf16_t* __res
 // 128 x 128 outputs a block of four waves whose segments go to blocks of their own: products of some hundred rows, which wait
 // for their loads and barriers more than for the matrix cores or the card's power.  K tiles of 64 (one barrier for twice
 // the products of gemm_tile's stages), STAGES of them, every load of a stage issued at once when its place is free; 32x32x16
-// products (two of them give the bits of a 16x16x32 one).  us, here and with gemm_tile's walk: 3,584 columns of K 18,944 at
+// products (two of them give the bits of a 16x16x32 one).  us, here and with gemm_tile's walk (sums stored with four columns a lane): 3,584 columns of K 18,944 at
 // 256 rows 52 / 72, at 1,525 rows 259 / 292; of K 3,584 at 140 rows 18 / 23, at 1,024 52 / 58; gated 13,824 of K 5,120 at 256
 // rows 98 / 117; 2,048 of K 2,048 at 1,525 rows 33 / 35.
 typedef __attribute__((ext_vector_type(16))) float f32x16;
