@@ -113,9 +113,7 @@ __device__ inline void tile_of_block(int bid, int m_blocks, int n_blocks, int& m
 }
 
 // The epilogue of a wave's tile whose columns lie across lanes.  Of each of COLS column tiles a lane holds one column, col(c),
-// and of that QUADS times four neighbouring rows from row(q) on: value(c, q, e).  Sixteen or 32 lanes side by side hold
-// neighbouring columns, so a store or read of 32-bit values is whole 64 or 128 bytes of each of a few rows; four columns a
-// lane (below) meet 64 lines in a 16-byte store where this meets 16.
+// and of that QUADS times four neighbouring rows from row(q) on: value(c, q, e).
 // With `partial`: the sums as they are to [split][gate | up][M][N] (one part without GLU).
 template <bool GLU, int COLS, int QUADS, class Value, class Col, class Row>
 __device__ __forceinline__ void tile_epilogue(Value value, Col col, Row row, const void* __restrict__ bias, int bias_is_f32,
@@ -150,26 +148,42 @@ __device__ __forceinline__ void tile_epilogue(Value value, Col col, Row row, con
     }
     return;
   }
+  if (mode == MODE_ADD_F32) {
+    // All reads of some columns before their first store, which may alias the next read: 32 values are under way at a time
+    // (with 16 a wave waits for memory once a column tile: kept 2,048 columns of K 2,048 at 2,048 rows 32.7 us, 30.1 so; 5,120 of
+    // K 512 at 4,096 rows 56.6, 48.7; 16,384 of K 256 154, 137).  Rows
+    // and columns past the end read the last one and store nothing.
+    constexpr int TOGETHER = QUADS >= 8 ? 1 : 2;
+    static_assert(COLS % TOGETHER == 0, "pairs of columns");
+    float* rows = reinterpret_cast<float*>(out);
+#pragma unroll
+    for (int c0 = 0; c0 < COLS; c0 += TOGETHER) {
+      float before[TOGETHER][QUADS][4], bv[TOGETHER];
+#pragma unroll
+      for (int i = 0; i < TOGETHER; ++i) {
+        const int n = min(col(c0 + i), N - 1);
+        bv[i] = bias ? load_vec(bias, bias_is_f32, n) : 0.0f;
+#pragma unroll
+        for (int q = 0; q < QUADS; ++q)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) before[i][q][e] = rows[(size_t)min(row(q) + e, M - 1) * out_stride + n];
+      }
+#pragma unroll
+      for (int i = 0; i < TOGETHER; ++i)
+#pragma unroll
+        for (int q = 0; q < QUADS; ++q)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (col(c0 + i) < N && row(q) + e < M)
+              rows[(size_t)(row(q) + e) * out_stride + col(c0 + i)] = before[i][q][e] + (value(c0 + i, q, e) + bv[i]);
+    }
+    return;
+  }
 #pragma unroll
   for (int c = 0; c < COLS; ++c) {
     const int n = col(c);
     if (n >= N) continue;
     const float bv = bias ? load_vec(bias, bias_is_f32, n) : 0.0f;
-    if (mode == MODE_ADD_F32) {
-      // all reads of a column before its first store, which may alias the next read; rows past M read the last row and store nothing
-      float* rows = reinterpret_cast<float*>(out) + n;
-      float before[QUADS][4];
-#pragma unroll
-      for (int q = 0; q < QUADS; ++q)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) before[q][e] = rows[(size_t)min(row(q) + e, M - 1) * out_stride];
-#pragma unroll
-      for (int q = 0; q < QUADS; ++q)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (row(q) + e < M) rows[(size_t)(row(q) + e) * out_stride] = before[q][e] + (value(c, q, e) + bv);
-      continue;
-    }
 #pragma unroll
     for (int q = 0; q < QUADS; ++q)
 #pragma unroll
@@ -183,12 +197,13 @@ __device__ __forceinline__ void tile_epilogue(Value value, Col col, Row row, con
   }
 }
 
-// The same for 16-bit outputs with a lane's four neighbouring columns, col(c) .. col(c) + 3, of row(q): one store of 8 bytes
-// instead of four of 2.
+// The same with a lane's four neighbouring columns, col(c) .. col(c) + 3, of row(q): one store of 8 or 16 bytes instead of four
+// of 2 or 4.  For outputs that are stored, not added into.
 template <bool GLU, int COLS, int ROWS, class Value, class Col, class Row>
-__device__ __forceinline__ void tile_epilogue_narrow(Value value, Col col, Row row, const void* __restrict__ bias, int bias_is_f32,
-                                                     bf16_t* __restrict__ out, int out_stride, int M, int N, int mode) {
-  const bool vec = N % 4 == 0 && out_stride % 4 == 0 && ((uintptr_t)out & 7) == 0;     // all four exist, rows and `out` are aligned
+__device__ __forceinline__ void tile_epilogue_four(Value value, Col col, Row row, const void* __restrict__ bias, int bias_is_f32,
+                                                   void* __restrict__ out, int out_stride, int M, int N, int mode) {
+  const bool narrow = GLU || mode_stores_elem(mode);
+  const bool vec = N % 4 == 0 && out_stride % 4 == 0 && ((uintptr_t)out & (narrow ? 7 : 15)) == 0;     // all four exist, rows and `out` are aligned
 #pragma unroll
   for (int c = 0; c < (GLU ? COLS / 2 : COLS); ++c) {
     const int n = col(c);
@@ -202,15 +217,29 @@ __device__ __forceinline__ void tile_epilogue_narrow(Value value, Col col, Row r
       if (m >= M) continue;
       float v[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        v[e] = GLU ? swiglu1(value(c, r, e), value(c + (GLU ? COLS / 2 : 0), r, e)) : mode_value(value(c, r, e) + bv[e], mode);
-      bf16_t* dst = out + (size_t)m * out_stride + n;
-      if (vec) {
-        *reinterpret_cast<uint2*>(dst) = make_uint2(pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3]));
-      } else {
+      for (int e = 0; e < 4; ++e) v[e] = GLU ? swiglu1(value(c, r, e), value(c + (GLU ? COLS / 2 : 0), r, e)) : value(c, r, e) + bv[e];
+      const size_t at = (size_t)m * out_stride + n;
+      if (narrow) {
+        bf16_t* dst = reinterpret_cast<bf16_t*>(out) + at;
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          if (n + e < N) dst[e] = float_to_bf16(v[e]);
+          if (!GLU) v[e] = mode_value(v[e], mode);
+        if (vec) {
+          *reinterpret_cast<uint2*>(dst) = make_uint2(pack2_bf16(v[0], v[1]), pack2_bf16(v[2], v[3]));
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (n + e < N) dst[e] = float_to_bf16(v[e]);
+        }
+      } else {
+        float* dst = reinterpret_cast<float*>(out) + at;
+        if (vec) {
+          *reinterpret_cast<f32x4*>(dst) = f32x4{v[0], v[1], v[2], v[3]};
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (n + e < N) dst[e] = v[e];
+        }
       }
     }
   }
@@ -251,7 +280,7 @@ __device__ __forceinline__ void tile_epilogue_narrow(Value value, Col col, Row r
 // before it in a second set of registers (the order of gemm_split_reduce), and no sums go through memory.
 //
 // ACROSS: which operand of a product X and W are (the same bits), and so whether a lane holds one column of four rows or
-// four columns of a row.  The former for 32-bit outputs, sums of segments among them, the latter for 16-bit ones.
+// four columns of a row (launch_tile says which for what).
 template <int BM, int BN, int WAVES_M, int WAVES_N, bool GLU, int STAGES, bool KEEP, bool ACROSS>
 __global__ void __launch_bounds__(WAVES_M * WAVES_N * 64, KEEP || STAGES * (BM + BN) * 64 <= 80 * 1024 ? 2 : 1)
 gemm_tile_kernel(const bf16_t* __restrict__ x, int x_stride, const bf16_t* __restrict__ w, const void* __restrict__ bias,
@@ -440,8 +469,8 @@ gemm_tile_kernel(const bf16_t* __restrict__ x, int x_stride, const bf16_t* __res
     tile_epilogue<GLU, TN, TM>(value, [&](int c) { return ncol + (GLU ? c % TH : c) * 16 + frow; }, [&](int r) { return mrow + r * 16 + four; },
                                bias, bias_is_f32, out, out_stride, M, N, mode, partial);
   else                        // row lane % 16 and four columns from 4 (lane / 16) on
-    tile_epilogue_narrow<GLU, TN, TM>(value, [&](int c) { return ncol + c * 16 + four; }, [&](int r) { return mrow + r * 16 + frow; }, bias,
-                                      bias_is_f32, reinterpret_cast<bf16_t*>(out), out_stride, M, N, mode);
+    tile_epilogue_four<GLU, TN, TM>(value, [&](int c) { return ncol + c * 16 + four; }, [&](int r) { return mrow + r * 16 + frow; }, bias,
+                                    bias_is_f32, out, out_stride, M, N, mode);
 }
 
 // ---------------------------------------------------------------------------- gemm_small_tile
@@ -453,7 +482,7 @@ gemm_tile_kernel(const bf16_t* __restrict__ x, int x_stride, const bf16_t* __res
 // rows 98 / 117; 2,048 of K 2,048 at 1,525 rows 33 / 35.
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 template <bool GLU, int STAGES>
-__global__ void __launch_bounds__(256, 1)
+__global__ void __launch_bounds__(256, 2)       // two waves a SIMD: two blocks a CU
 gemm_small_tile_kernel(const bf16_t* __restrict__ x, int x_stride, const bf16_t* __restrict__ w, const void* __restrict__ bias,
                        int bias_is_f32, void* __restrict__ out, int out_stride, int M, int N, int K, int mode, int m_blocks,
                        int n_blocks, float* __restrict__ partial) {
@@ -836,11 +865,13 @@ static int reserve_lds(int bytes) {
 // The tiles of gemm_tile, STAGES stages of 32 k.  A block a segment (gridDim.y), the sums through `partial`; or, with KEEP, a
 // block all of them, the finished sums through `partial` where the kernel that adds sums does more than that.
 //
-// Which way round (us, four columns of a row in a lane / columns across lanes).  16-bit outputs: 33,000 columns of K 1,024 at
-// 1,500 rows 147 / 182, kept 5,632 of K 2,048 65 / 73, gated 18,944 of K 3,584 at 2,048 rows 462 / 469.  32-bit ones: segments' sums
-// of 5,632 of K 2,048 at 320 rows 30.5 / 26.5, of 3,584 of K 3,584 at 688 43.8 / 39.9, kept and added into rows 3,584 of K 3,584
-// at 2,048 65.8 / 64.5.  Kept gated products, whose waves own 32 columns of the output, go the second way, too (1,408 of K 2,048 at
-// 2,048 rows 37.7 / 36.4).
+// Which way round (us, four columns of a row in a lane / columns across lanes).  Outputs that are stored go the first way: of
+// 16 bits 33,000 columns of K 1,024 at 1,500 rows 147 / 182, kept 5,632 of K 2,048 65 / 73, gated 18,944 of K 3,584 at 2,048
+// rows 462 / 469; of 32 bits kept 2,048 of K 2,048 at 2,048 rows 32 / 37, 5,632 65 / 74, 33,000 of K 1,024 at 1,525 142 / 170.
+// The second way: sums of segments, which are read again (5,632 of K 2,048 at 320 rows 30.5 / 26.5, 3,584 of K 3,584 at 688
+// 43.8 / 39.9); rows added into, where 16 bytes of sixteen rows meet 64 lines twice (kept 3,584 of K 3,584 at 2,048 65.6 /
+// 62.8, 3,333 of K 512 35 / 25); rows of 32 bits that are not aligned for 16 bytes (3,333 of K 512 26.6 / 23.1); kept gated
+// products, whose waves own 32 columns of the output (1,408 of K 2,048 at 2,048 rows 37.7 / 36.4).
 template <int BM, int BN, int WAVES_M, int WAVES_N, bool GLU, bool KEEP = false, int STAGES = 5>
 static int launch_tile(const bf16_t* x, int x_stride, const bf16_t* w, const void* bias, int bias_is_f32, void* out,
                        int out_stride, int m, int n, int k, int mode, hipStream_t stream, int segs = 1,
@@ -862,7 +893,9 @@ static int launch_tile(const bf16_t* x, int x_stride, const bf16_t* w, const voi
   };
   int rc;
   if constexpr (KEEP && GLU) rc = go(std::true_type());
-  else rc = after || !(GLU || mode_stores_elem(mode)) ? go(std::true_type()) : go(std::false_type());
+  else if (GLU || mode_stores_elem(mode)) rc = after ? go(std::true_type()) : go(std::false_type());
+  else if (!after && mode == MODE_STORE_F32 && n % 4 == 0 && out_stride % 4 == 0 && ((uintptr_t)out & 15) == 0) rc = go(std::false_type());
+  else rc = go(std::true_type());
   if (rc) return rc;
   return after ? add_split_sums(partial, splits, m, n, bias, bias_is_f32, out, out_stride, mode, norm, rope, stream) : 0;
 }
