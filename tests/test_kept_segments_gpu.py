@@ -119,3 +119,23 @@ def test_passes_of_a_product_that_keeps_them():
         k.gemm(x[at:at + m].contiguous(), w, part, None, MODE_ADD_F32)
         k.rmsnorm(part, gain, 1e-6, alone)
         assert torch.equal(out[at:at + m], part) and torch.equal(normed[at:at + m], alone), at
+
+
+@pytest.mark.parametrize("mode", [MODE_STORE, MODE_STORE_F32, MODE_ADD_F32, MODE_SWIGLU, MODE_RELU_SQUARED])
+@pytest.mark.parametrize("M,N,K", [(1300, 2576, 512), (700, 16416, 192), (2048, 4608, 192), (300, 16400, 256), (520, 5632, 2048)])
+def test_outputs_anywhere(M, N, K, mode):
+    """Outputs that are columns of wider rows, aligned for wide stores and not: the bits of a plain output, nothing beside it.
+    Kept segments, the three widths of tiles, and a segment a block."""
+    k = kernels("bfloat16")
+    g = torch.Generator(device="cuda").manual_seed(N)
+    x = torch.randn(M, K, generator=g, device="cuda").bfloat16()
+    w = k.prepare_weight((torch.randn((2 if mode == MODE_SWIGLU else 1) * N, K, generator=g, device="cuda") * 0.1).bfloat16(), mode == MODE_SWIGLU)
+    bias = None if mode == MODE_SWIGLU else torch.randn(N, generator=g, device="cuda")
+    dtype = torch.float32 if mode in (MODE_ADD_F32, MODE_STORE_F32) else torch.bfloat16
+    plain = torch.ones(M, N, dtype=dtype, device="cuda")
+    k.gemm(x, w, plain, bias, mode)
+    for wide, first in ((N + 8, 0), (N + 8, 4), (N + 8, 2), (N + 8, 1), (N + 3, 2), (N + 5, 0)):
+        rows = torch.ones(M, wide, dtype=dtype, device="cuda")
+        k.gemm(x, w, rows[:, first:first + N], bias, mode)
+        assert torch.equal(rows[:, first:first + N], plain), (wide, first)
+        assert bool((rows[:, :first] == 1).all()) and bool((rows[:, first + N:] == 1).all()), (wide, first)
