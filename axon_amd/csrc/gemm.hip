@@ -155,121 +155,222 @@ gemm_fma_kernel(const elem_t* __restrict__ x, int x_stride, const elem_t* __rest
       }
 }
 
-// Few rows (decoding): such a product only waits for W, so a block takes NR (16 or 8) columns and the
+// Few rows (decoding): such a product only waits for W, so a block takes up to 16 columns and the
 // chains of an output, which do not need each other, are shared out over its 8 waves: every wave
 // streams its chains' W from memory straight into operands, leaves the chains' sums in LDS, and a thread
 // an output adds them in ascending order.  MT tiles of 16 rows of X ride along with each W (a wave reads
-// them from L2 beside W: with 64 rows of X that is what bounds it).  SHORT: a K of no more chains than waves, one
-// each (8 rows of 512 x K 256 6.5 us with all of them in one wave, 4.1 here).  5 rows: 2,560 x K 2,048 25 -> 16 us,
-// 2,048 x 5,632 63 -> 27, 32,000 x 2,048 (262 MB) 85 -> 61 us, 4.3 TB/s; 64 rows of 2,048 x 5,632 332 -> 63 us.
+// them from L2 beside W, which is what bounds it from some 32 rows on).  What a wave multiplies next, W and X, is
+// asked for as soon as the registers are free, with no branch between, so that loads are under way through the
+// products, the barrier and the sums; they are buffer loads, whose k is in a scalar register, and the two halves of a
+// line (16 k) are asked for one behind the other (four loads apart they came from L2 twice: 2,048 x K 5,632 at 16 rows
+// 27 us, 22 so).  One chain of a wave at a time, or two where both operands are one tile: more of them (4 and 8)
+// only wait for each other (the same 22 us against 20; a gated 5,632 x 2,048 of 5 rows 26 against 23 us).
+// 5 rows, us, before (X asked for chain by chain between branches, a round's loads behind the last one's sums) / now:
+// 2,560 x K 2,048 15.3 / 8.5, 2,048 x 2,048 11.7 / 8.9, gated 5,632 x 2,048 33.1 / 21.0 (4.4 TB/s), 2,048 x 5,632 28.9 / 17.5,
+// 32,000 x 2,048 66 / 52 (5.0 TB/s); 32 rows of 2,560 x 2,048 23.3 / 13.5, of 32,000 x 2,048 102 / 90; 64 rows of
+// 2,048 x 5,632 65 / 56.  A K that is no multiple of four loads its numbers singly: 1,000 x K 1,001 of 5 rows 9.4 / 7.3, but of
+// 20 to 128 rows 5 to 7 % longer than before.
 #define FEW_WAVES 8
+#if AXON_BF16
+typedef __attribute__((ext_vector_type(2))) unsigned fma_quad;      // four numbers as they lie in memory
+#else
+typedef u32x4 fma_quad;
+#endif
+// Rows `stride` apart as a buffer: a row's place in it is in the lane's register and k in a scalar one, so that a load
+// needs no address of its own, and what lies behind the last row reads as zeros.
+struct FmaRows {
+  __amdgpu_buffer_rsrc_t rsrc;
+  const elem_t* base;
+};
+__device__ __forceinline__ FmaRows fma_rows(const elem_t* base, size_t elems) {
+  const size_t bytes = elems * sizeof(elem_t);
+  return {__builtin_amdgcn_make_buffer_rsrc((void*)base, 0, bytes < 0xffffffffu ? (unsigned)bytes : 0xffffffffu, 0x00027000), base};
+}
+// Four k of the row that begins `at` elements behind the first, k = k0 + in_chain .. + 3 (in_chain: this lane's place in
+// the chain that begins at k0).  Aligned operands read on into the next row behind K; others take the row's last number.
+template <bool VEC>
+__device__ __forceinline__ fma_quad fma_ask(const FmaRows& rows, unsigned at, int k0, int in_chain, int K) {
+  if (VEC) {
+    const int off = (int)((at + in_chain) * sizeof(elem_t)), s_off = (int)(k0 * sizeof(elem_t));
+#if AXON_BF16
+    return __builtin_amdgcn_raw_buffer_load_b64(rows.rsrc, off, s_off, 0);
+#else
+    return __builtin_amdgcn_raw_buffer_load_b128(rows.rsrc, off, s_off, 0);
+#endif
+  }
+  union { fma_quad q; elem_t e[4]; } c;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) c.e[e] = rows.base[(size_t)at + min(k0 + in_chain + e, K - 1)];
+  return c.q;
+}
+// What lies behind K of four k from `k` on becomes zeros.
+__device__ __forceinline__ void fma_clear(fma_quad& raw, int k, int K) {
+  union { fma_quad q; elem_t e[4]; } c;
+  c.q = raw;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) c.e[e] = k + e < K ? c.e[e] : from_float(0.0f);
+  raw = c.q;
+}
+__device__ __forceinline__ f32x4 fma_operand(const fma_quad& raw) {
+  union { fma_quad q; elem_t e[4]; } c;
+  c.q = raw;
+  float v[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = to_float(c.e[e]);
+  return f32_operand(v);
+}
+
 template <int MT, int NR, bool GLU, bool VEC, bool SHORT>
-__global__ void __launch_bounds__(64 * FEW_WAVES, 2)
+__global__ void __launch_bounds__(64 * FEW_WAVES, 4)
 gemm_fma_few_rows_kernel(const elem_t* __restrict__ x, int x_stride, const elem_t* __restrict__ w,
                          const void* __restrict__ bias, int bias_is_f32, void* __restrict__ out, int out_stride, int M,
-                         int N, int K, int mode) {
+                         int N, int K, int mode, int columns) {
   constexpr int NT = GLU ? 2 : 1;
-  constexpr int PW = SHORT || MT * NT >= 8 ? 1 : MT * NT >= 3 ? 2 : MT * NT == 2 ? 4 : 8;   // chains of a wave in a round
-  constexpr int PARTS = FEW_WAVES * PW, OUTS = MT * 16 * NR;
-  __shared__ __align__(16) float chains[PARTS * NT * OUTS];                        // [chain][gate, up][row][column]
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  constexpr int ROUND = SHORT || MT * NT >= (VEC ? 2 : 4) ? 1 : 2;
+  constexpr int PARTS = FEW_WAVES * ROUND, OUTS = MT * 16 * NR, ALL = NT * OUTS;
+  constexpr int BUFFERS = PARTS * ALL * 4 > 32768 ? 1 : 2;          // of chains: two where two blocks a CU leave room
+  __shared__ __align__(16) float chains[BUFFERS * PARTS * ALL];       // [chain][gate, up][row][NR columns]
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r16 = lane & 15, q = lane >> 4;
-  const int n0 = blockIdx.x * NR, m0 = blockIdx.y * MT * 16;
-  const elem_t* w_row = w + (size_t)min(n0 + min(r16, NR - 1), N - 1) * K;
-  const elem_t* x_row[MT];
+  const int n0 = blockIdx.x * columns, m0 = blockIdx.y * MT * 16;
+  FmaRows w_rows[NT];
 #pragma unroll
-  for (int i = 0; i < MT; ++i) x_row[i] = x + (size_t)min(m0 + 16 * i + r16, M - 1) * x_stride;
+  for (int t = 0; t < NT; ++t) w_rows[t] = fma_rows(w + (size_t)(n0 + t * N) * K, (size_t)(N - n0) * K);
+  const FmaRows x_rows = fma_rows(x + (size_t)m0 * x_stride, (size_t)(M - m0 - 1) * x_stride + K);
+  const unsigned w_at = (unsigned)min(min(r16, columns - 1), N - 1 - n0) * (unsigned)K;
+  unsigned x_at[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) x_at[i] = (unsigned)min(16 * i + r16, M - 1 - m0) * (unsigned)x_stride;
   const int n_parts = (K + FMA_PART - 1) / FMA_PART;
-  constexpr int MINE = (OUTS + 64 * FEW_WAVES - 1) / (64 * FEW_WAVES);
-  float sum[MINE], sum_up[MINE];
+  constexpr int MINE = (ALL + 64 * FEW_WAVES - 1) / (64 * FEW_WAVES);
+  float sum[MINE];
 #pragma unroll
-  for (int i = 0; i < MINE; ++i) sum[i] = sum_up[i] = 0.0f;
+  for (int i = 0; i < MINE; ++i) sum[i] = 0.0f;
 
-  for (int first = 0; first < n_parts; first += PARTS) {
-    float wv[NT][PW][2][4];
+  fma_quad wq[ROUND][NT][2], xq[ROUND][MT][2];
+  auto ask = [&](int p, int first) {
+    const int k0 = (first + p * FEW_WAVES + wave) * FMA_PART;
 #pragma unroll
-    for (int p = 0; p < PW; ++p)
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int g = 0; g < 2; ++g) wq[p][t][g] = fma_ask<VEC>(w_rows[t], w_at, k0, 16 * g + 4 * q, K);
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int g = 0; g < 2; ++g) xq[p][i][g] = fma_ask<VEC>(x_rows, x_at[i], k0, 16 * g + 4 * q, K);
+  };
+#pragma unroll
+  for (int p = 0; p < ROUND; ++p) ask(p, 0);
+  int buffer = 0;
+  auto round = [&](int first, bool more) {
+    float* to = chains + buffer * PARTS * ALL;
+#pragma unroll
+    for (int p = 0; p < ROUND; ++p) {
+      const int part = p * FEW_WAVES + wave, k0 = (first + part) * FMA_PART, k = k0 + 4 * q;
+      if (k0 < K && k0 + FMA_PART > K) {                   // K ends in this chain: the same for the whole wave
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+#pragma unroll
+          for (int t = 0; t < NT; ++t) fma_clear(wq[p][t][g], k + 16 * g, K);
+#pragma unroll
+          for (int i = 0; i < MT; ++i) fma_clear(xq[p][i][g], k + 16 * g, K);
+        }
+      }
+      f32x4 a[NT][2], b[MT][2];
+#pragma unroll
+      for (int g = 0; g < 2; ++g) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t) a[t][g] = fma_operand(wq[p][t][g]);
+#pragma unroll
+        for (int i = 0; i < MT; ++i) b[i][g] = fma_operand(xq[p][i][g]);
+      }
+      if (more) ask(p, first + PARTS);
+      f32x4 acc[MT][NT];
 #pragma unroll
       for (int g = 0; g < 2; ++g)
 #pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+          for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+              if (g == 0 && s == 0) acc[i][t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+              FMA_STEP(acc[i][t], a[t][g], b[i][g], s);
+            }
+      // columns 4 q .. 4 q + 3 of row 16 i + r16; of a chain behind the last one too: it is not added
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
         for (int t = 0; t < NT; ++t)
-          fma_load<VEC>(w_row + (size_t)t * N * K, (first + wave * PW + p) * FMA_PART + 16 * g + 4 * q, K, wv[t][p][g]);
-#pragma unroll
-    for (int p = 0; p < PW; ++p) {
-      const int part = wave * PW + p, k0 = (first + part) * FMA_PART;
-      if (k0 >= K) break;                            // the same for the whole wave
-      f32x4 a[NT][2];
-#pragma unroll
-      for (int t = 0; t < NT; ++t)
-#pragma unroll
-        for (int g = 0; g < 2; ++g) {
-          if (k0 + FMA_PART > K) fma_clear(wv[t][p][g], k0 + 16 * g + 4 * q, K);
-          a[t][g] = f32_operand(wv[t][p][g]);
-        }
-#pragma unroll
-      for (int i = 0; i < MT; ++i) {
-        f32x4 b[2];
-#pragma unroll
-        for (int g = 0; g < 2; ++g) {
-          float xv[4];
-          fma_load<VEC>(x_row[i], k0 + 16 * g + 4 * q, K, xv);
-          if (k0 + FMA_PART > K) fma_clear(xv, k0 + 16 * g + 4 * q, K);
-          b[g] = f32_operand(xv);
-        }
-#pragma unroll
-        for (int t = 0; t < NT; ++t) {
-          f32x4 acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-          for (int g = 0; g < 2; ++g)
-#pragma unroll
-            for (int s = 0; s < 4; ++s) FMA_STEP(acc, a[t][g], b[g], s);
-          // columns 4 q .. 4 q + 3 of row 16 i + r16
-          if (4 * q < NR) *reinterpret_cast<f32x4*>(&chains[(part * NT + t) * OUTS + (16 * i + r16) * NR + 4 * q]) = acc;
-        }
-      }
+          if (4 * q < NR) *reinterpret_cast<f32x4*>(&to[(part * NT + t) * OUTS + (16 * i + r16) * NR + 4 * q]) = acc[i][t];
     }
-    __syncthreads();
+    wait_lgkmcnt<0>();
+    __builtin_amdgcn_s_barrier();          // (loads stay under way)
+    asm volatile("" ::: "memory");
     const int count = min(PARTS, n_parts - first);
 #pragma unroll
     for (int i = 0; i < MINE; ++i) {
       const int o = tid + 64 * FEW_WAVES * i;
-      if (o < OUTS) {
-#pragma unroll 8
-        for (int p = 0; p < count; ++p) {
-          sum[i] += chains[p * NT * OUTS + o];
-          if (GLU) sum_up[i] += chains[(p * NT + NT - 1) * OUTS + o];
+      if (o < ALL) {
+        if (count == PARTS) {
+#pragma unroll
+          for (int p = 0; p < PARTS; ++p) sum[i] += to[p * ALL + o];
+        } else {
+          for (int p = 0; p < count; ++p) sum[i] += to[p * ALL + o];
         }
       }
     }
+    if (BUFFERS == 1) {
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+    }
+    if (BUFFERS == 2) buffer ^= 1;
+  };
+  int first = 0;
+  for (; first + PARTS < n_parts; first += PARTS) round(first, true);
+  round(first, false);
+
+  float up[MINE];
+  if (GLU) {                     // the up sums go to the threads that hold the gates'
     __syncthreads();
+#pragma unroll
+    for (int i = 0; i < MINE; ++i)
+      if (tid + 64 * FEW_WAVES * i < ALL) chains[tid + 64 * FEW_WAVES * i] = sum[i];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < MINE; ++i) up[i] = chains[(tid + 64 * FEW_WAVES * i) % OUTS + (NT - 1) * OUTS];
   }
 #pragma unroll
   for (int i = 0; i < MINE; ++i) {
-    const int o = tid + 64 * FEW_WAVES * i, m = m0 + o / NR, col = n0 + o % NR;
-    if (o < OUTS && m < M && col < N)
-      fma_store(sum[i], sum_up[i], GLU, bias, bias_is_f32, out, (size_t)m * out_stride + col, col, mode);
+    const int o = tid + 64 * FEW_WAVES * i, m = m0 + o / NR, c = o % NR, col = n0 + c;
+    if (o < OUTS && c < columns && m < M && col < N)
+      fma_store(sum[i], GLU ? up[i] : 0.0f, GLU, bias, bias_is_f32, out, (size_t)m * out_stride + col, col, mode);
   }
 }
 
 template <int MT, bool GLU, bool VEC>
 static void launch_fma_few(const elem_t* x, int x_stride, const elem_t* w, const void* bias, int bias_is_f32, void* out,
                            int out_stride, int m, int n, int k, int mode, hipStream_t stream) {
-  const int rows = ceil_div(m, 16 * MT);
-  // blocks of 8 columns where blocks of 16 would leave CUs without one
-  const bool narrow = (long)ceil_div(n, 16) * rows < 256, brief = k <= FEW_WAVES * FMA_PART;
-#define FEW(NR, SHORT)                                                                                                \
-  gemm_fma_few_rows_kernel<MT, NR, GLU, VEC, SHORT><<<dim3(ceil_div(n, NR), rows), 64 * FEW_WAVES, 0, stream>>>(      \
-      x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode)
-  if (brief) { if (narrow) FEW(8, true); else FEW(16, true); }
-  else { if (narrow) FEW(8, false); else FEW(16, false); }
+  // As many blocks as give every CU the same number of them, with at most 16 columns each (2,560 columns in 256 blocks of 10:
+  // 9.0 us, in 160 of 16 10.3; 11,264 gated in 512 of 11: 27.3, in 352 of 16 30.8), and so many that X counts less than W
+  const int rows = ceil_div(m, 16 * MT), each = ceil_div(ceil_div(n, 16) * rows, 256);
+  const int columns = max(MT == 1 ? 4 : 8, min(16, ceil_div(n * rows, 256 * each)));
+  const dim3 blocks(ceil_div(n, columns), rows);
+#define FEW(NR, SHORT)                                                                            \
+  gemm_fma_few_rows_kernel<MT, NR, GLU, VEC, SHORT><<<blocks, 64 * FEW_WAVES, 0, stream>>>(   \
+      x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode, columns)
+  if (k <= FEW_WAVES * FMA_PART) { if (columns <= 8) FEW(8, true); else FEW(16, true); }
+  else { if (columns <= 8) FEW(8, false); else FEW(16, false); }
 #undef FEW
 }
 
 static int launch_fma(const elem_t* x, int x_stride, const elem_t* w, const void* bias, int bias_is_f32, void* out,
                       int out_stride, int m, int n, int k, int mode, hipStream_t stream) {
   const size_t vbytes = 4 * sizeof(elem_t);
-  const bool vec_w = (k % 4 == 0) && ((uintptr_t)w % vbytes == 0);
-  const bool vec_x = (k % 4 == 0) && (x_stride % 4 == 0) && ((uintptr_t)x % vbytes == 0);
+  // (rows a block reads as a buffer lie within 4 GB)
+  const bool vec_w = (k % 4 == 0) && ((uintptr_t)w % vbytes == 0) && k < (1 << 23);
+  const bool vec_x = (k % 4 == 0) && (x_stride % 4 == 0) && ((uintptr_t)x % vbytes == 0) && x_stride < (1 << 23);
 #define FMA_ARGS x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode, stream
 // Up to 32 rows a product waits for W; from 33 to 128 so it does where the tiles would be fewer than
 // the CUs (2,048 columns of K 5,632 at 128 rows: 143 us with 64 tiles, 67 us with a wave a part of K), while

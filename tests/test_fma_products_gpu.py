@@ -81,3 +81,22 @@ def test_the_bits_are_those_of_chains_of_fmaf(N, K, values):
             act = torch.empty_like(out)
             k.swiglu(torch.cat([gate, up], 1)[:m].contiguous(), act)
             assert torch.equal(out, act), m
+
+
+@pytest.mark.parametrize("N,K", [(1030, 516), (2570, 1060), (4100, 292), (300, 545)])
+def test_columns_a_block_and_rounds_of_chains(N, K):
+    """Blocks of 4, 5, 8, 9, 11 and 16 columns, the last one short, and K of whole and broken rounds of chains."""
+    k = kernels("float32")
+    g = torch.Generator(device="cuda").manual_seed(N)
+    x, w = torch.randn(64, K, generator=g, device="cuda"), torch.randn(N, K, generator=g, device="cuda")
+    want = _by_chains(k, x, w)
+    for m in (1, 16, 17, 33, 64):
+        out = torch.full((m, N + 3), float("nan"), device="cuda")
+        k.gemm(x[:m], w, out[:, :N], None, MODE_STORE_F32)
+        assert torch.equal(out[:, :N], want[:m]) and bool(out[:, N:].isnan().all()), m
+    gate, up, half = want[:, :N // 2], want[:, N // 2:2 * (N // 2)], N // 2
+    for m in (3, 20, 64):
+        out, act = (torch.full((m, half), float("nan"), device="cuda") for _ in range(2))
+        k.gemm(x[:m], w[:2 * half], out, None, MODE_SWIGLU)
+        k.swiglu(torch.cat([gate, up], 1)[:m].contiguous(), act)
+        assert torch.equal(out, act), m
