@@ -40,7 +40,7 @@
 //   128 x 128 tiles take a segment each, gemm_small_tile, in steps of 64.  With S > 1 segments each
 //   goes to blocks of its own (gridDim.y = S), whose sums go through a workspace and are added in
 //   segment order by gemm_split_reduce, which also applies the epilogue; or, where tiles of 128 x 128
-//   fill the chip (keeps_segments), a block walks them all.  X rows land in LDS with their 16-byte slots permuted so that fragment reads of
+//   fill the chip (keeps_segments), a block walks them all (gemm_tile_kernel_kept).  X rows land in LDS with their 16-byte slots permuted so that fragment reads of
 //   neighbouring rows fall into different banks; W blocks land as they are.  Blocks are numbered
 //   so that the blocks of one XCD (every eighth block) share weight tiles in that XCD's L2.
 #include "api.h"
@@ -276,16 +276,13 @@ __device__ __forceinline__ void tile_epilogue_four(Value value, Col col, Row row
 // rows of its columns and, after them, the up rows of the same columns, so that a lane ends
 // with both values of an output element.
 //
-// KEEP: the block walks all `splits` segments of K itself; a segment's chains are added to the sums of those
-// before it in a second set of registers (the order of gemm_split_reduce), and no sums go through memory.
-//
 // ACROSS: which operand of a product X and W are (the same bits), and so whether a lane holds one column of four rows or
 // four columns of a row (launch_tile says which for what).
-template <int BM, int BN, int WAVES_M, int WAVES_N, bool GLU, int STAGES, bool KEEP, bool ACROSS>
-__global__ void __launch_bounds__(WAVES_M * WAVES_N * 64, KEEP || STAGES * (BM + BN) * 64 <= 80 * 1024 ? 2 : 1)
+template <int BM, int BN, int WAVES_M, int WAVES_N, bool GLU, int STAGES, bool ACROSS>
+__global__ void __launch_bounds__(WAVES_M * WAVES_N * 64, 1)
 gemm_tile_kernel(const bf16_t* __restrict__ x, int x_stride, const bf16_t* __restrict__ w, const void* __restrict__ bias,
                  int bias_is_f32, void* __restrict__ out, int out_stride, int M, int N, int K, int mode, int m_blocks,
-                 int n_blocks, float* __restrict__ partial, int splits) {
+                 int n_blocks, float* __restrict__ partial) {
   extern __shared__ __align__(16) unsigned char smem[];
   constexpr int NW = WAVES_M * WAVES_N;
   constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N;  // a wave's tile
@@ -336,8 +333,8 @@ gemm_tile_kernel(const bf16_t* __restrict__ x, int x_stride, const bf16_t* __res
 
   // Split K (gridDim.y > 1): this block multiplies the k blocks kt_begin .. kt_begin + nk - 1 and
   // leaves its sums in `partial`; gemm_split_reduce_kernel adds the blocks' sums in block order.
-  const int kt_begin = KEEP ? 0 : (int)((long)blockIdx.y * (K / 64) / gridDim.y) * 2;
-  const int nk = KEEP ? KB : (int)((long)(blockIdx.y + 1) * (K / 64) / gridDim.y) * 2 - kt_begin;       // even
+  const int kt_begin = (int)((long)blockIdx.y * (K / 64) / gridDim.y) * 2;
+  const int nk = (int)((long)(blockIdx.y + 1) * (K / 64) / gridDim.y) * 2 - kt_begin;       // even
   // load instruction q of this wave for k block kt (counted from kt_begin) into stage `slot`
   auto issue = [&](int slot, int kt, int q) {
     unsigned char* stage = smem + slot * STAGE;
@@ -354,8 +351,6 @@ gemm_tile_kernel(const bf16_t* __restrict__ x, int x_stride, const bf16_t* __res
   for (int i = 0; i < TN; ++i)
 #pragma unroll
     for (int j = 0; j < TM; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  f32x4 sum[KEEP ? TN : 1][KEEP ? TM : 1];
-  int seg = 0, seg_end = KEEP ? (int)((long)(K / 64) / splits) * 2 : 0;     // of the segment being multiplied
 
   // X fragments: row = tile row + lane % 16, k chunk = lane / 16, at its permuted slot; W fragments: blocks as they are
   const int frow = lane & 15;
@@ -439,30 +434,10 @@ gemm_tile_kernel(const bf16_t* __restrict__ x, int x_stride, const bf16_t* __res
   auto two_blocks = [&](int kt, auto fetch_of) {
     block(kt, Number<0>(), fetch_of);
     block(kt + 1, Number<1>(), fetch_of);
-    if (KEEP && kt + 2 == seg_end) {
-#pragma unroll
-      for (int i = 0; i < (KEEP ? TN : 0); ++i)
-#pragma unroll
-        for (int j = 0; j < TM; ++j) {
-          f32x4& s = sum[KEEP ? i : 0][KEEP ? j : 0];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) s[e] = seg == 0 ? acc[i][j][e] : s[e] + acc[i][j][e];
-          acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        }
-      ++seg;
-      seg_end = (int)((long)(seg + 1) * (K / 64) / splits) * 2;
-    }
   };
   int kt = 0;
   for (; kt + AHEAD < nk; kt += 2) two_blocks(kt, Number<1>());
   for (; kt < nk; kt += 2) two_blocks(kt, Number<0>());
-  if constexpr (KEEP) {
-#pragma unroll
-    for (int i = 0; i < TN; ++i)
-#pragma unroll
-      for (int j = 0; j < TM; ++j) acc[i][j] = sum[i][j];
-  }
-
   const int mrow = m0 + wm * WM, ncol = n0 + wn * (GLU ? WN / 2 : WN), four = (lane >> 4) * 4;
   const auto value = [&](int c, int r, int e) { return acc[c][r][e]; };
   if constexpr (ACROSS)       // a lane holds column lane % 16 and four rows from 4 (lane / 16) on of each tile
@@ -471,6 +446,184 @@ gemm_tile_kernel(const bf16_t* __restrict__ x, int x_stride, const bf16_t* __res
   else                        // row lane % 16 and four columns from 4 (lane / 16) on
     tile_epilogue_four<GLU, TN, TM>(value, [&](int c) { return ncol + c * 16 + four; }, [&](int r) { return mrow + r * 16 + frow; }, bias,
                                     bias_is_f32, out, out_stride, M, N, mode);
+}
+
+// ---------------------------------------------------------------------------- gemm_kept
+// 128 x 128 outputs a block of four waves of 64 x 64 (GLU: 64 columns), two blocks a CU.  The block walks all `splits`
+// segments of K itself; a segment's chains are added to the sums of those before it in a second set of registers (the order of
+// gemm_split_reduce), and no sums go through memory.
+//
+// Beside gemm_tile's way (steps of 32 k, direct loads, reads and loads between products):
+//  * X goes to LDS in pairs of steps, a row's 64 k, a whole line of 128 bytes: half lines were twice the requests of L2 (of
+//    9.3 M a launch 6.4 M; 16 channels an XCD answer one each a cycle).  Three pairs of X and four steps of W in
+//    80 KB: whatever is needed has had three steps to arrive.  A row's eight slots of 16 bytes are permuted by
+//    slot ^ (row / 2 % 8): LDS serves lanes 0-3, 12-15, 20-23 and 24-27 at a time, and those 16 fall on 256 different bytes.
+//  * A step's fragments are all in registers when it begins: the next step's are read behind the first products and have
+//    the other eight to arrive.
+// What bounds it: with one block a CU (of 2,048^3) a step takes some 600 cycles of which 256 are products, with two some 1,000 of
+// which 512 are; without its loads it would take 25 % less, without its reads of LDS 5.
+// us, half lines and half of a step's fragments ahead / here, 2,048 rows: 2,048 columns of K 2,048 31.6 / 27.3, 3,584 of 3,584
+// 67 / 58, 4,608 of 3,584 102 / 80, 5,632 of 2,048 66.6 / 56.8, 8,192 of 8,192 at 4,096 rows 596 / 499 (1.10 PFLOP/s), gated 1,408 of
+// 2,048 37.3 / 33.2; 5,120 of 5,120 added into 1,525 rows 99 / 82.  The fragments alone: 31.6 / 28.9, 67 / 66, 102 / 93.
+#define KEPT_X_PAIRS 3
+#define KEPT_W_STEPS 4
+#define KEPT_LDS (KEPT_X_PAIRS * 128 * 128 + KEPT_W_STEPS * 128 * 64)
+template <bool GLU, bool ACROSS>
+__global__ void __launch_bounds__(256, 2)
+gemm_tile_kernel_kept(const bf16_t* __restrict__ x, int x_stride, const bf16_t* __restrict__ w, const void* __restrict__ bias,
+                 int bias_is_f32, void* __restrict__ out, int out_stride, int M, int N, int K, int mode, int m_blocks,
+                 int n_blocks, float* __restrict__ partial, int splits) {
+  extern __shared__ __align__(128) unsigned char smem[];
+  constexpr int T = 4;                                 // 16 x 16 MFMA tiles a wave, both ways
+  constexpr int X_PAIR = 128 * 128, W_STEP = 128 * 64, W_AT = KEPT_X_PAIRS * X_PAIR;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+  int mb, nb;
+  tile_of_block(blockIdx.x, m_blocks, n_blocks, mb, nb);
+  const int m0 = mb * 128, n0 = nb * (GLU ? 64 : 128);
+
+  // A load of X fills 8 rows of a pair: lane l row l / 8, slot l % 8, which holds k chunk (l % 8) ^ (row / 2 % 8).  Load q of
+  // a wave: rows (q * 4 + wave) * 8 and on; the first two half a pair, the others the rest.
+  unsigned xoff[4], woff[2];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int r = (q * 4 + wave) * 8 + (lane >> 3);
+    xoff[q] = (unsigned)min(m0 + r, M - 1) * (unsigned)x_stride + ((lane & 7) ^ ((r >> 1) & 7)) * 8;
+  }
+  // W: packed blocks as they lie in memory, blocks q * 4 + wave of a step (see gemm_tile)
+  const int KB = K / 32, row_tiles = GLU ? N / 16 : (N + 15) / 16;
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int r = (q * 4 + wave) * 16;
+    int tile;
+    if (GLU) {
+      const int col = n0 + r / 64 * 32 + r % 32;
+      tile = (r % 64 >= 32 ? row_tiles : 0) + min(col / 16, row_tiles - 1);
+    } else {
+      tile = min((n0 + r) / 16, row_tiles - 1);
+    }
+    woff[q] = (unsigned)tile * (unsigned)KB * 512 + lane * 8;
+  }
+  auto ask_x = [&](int pair, int slot, int q) {
+    __builtin_amdgcn_global_load_lds((global_ptr_t)(x + xoff[q] + pair * 64), (lds_ptr_t)(smem + slot * X_PAIR + (q * 4 + wave) * 1024), 16, 0, 0);
+  };
+  auto ask_w = [&](int kt, int q) {
+    __builtin_amdgcn_global_load_lds((global_ptr_t)(w + woff[q] + kt * 512),
+                                     (lds_ptr_t)(smem + W_AT + (kt % KEPT_W_STEPS) * W_STEP + (q * 4 + wave) * 1024), 16, 0, 0);
+  };
+
+  f32x4 acc[T][T], sum[T][T];
+#pragma unroll
+  for (int i = 0; i < T; ++i)
+#pragma unroll
+    for (int j = 0; j < T; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  int seg = 0, seg_end = (int)((long)(K / 64) / splits) * 2;     // of the segment being multiplied
+
+  const int frow = lane & 15;
+  const unsigned lds0 = (unsigned)(size_t)(lds_ptr_t)smem;
+  const unsigned xbase = lds0 + (wm * 64 + frow) * 128 + (((lane >> 4) ^ (frow >> 1)) << 4);      // of the pair's first step; its second's: ^ 64
+  const unsigned wbase = lds0 + W_AT + wn * 4 * 1024 + lane * 16;
+  u32x4 xf[2][T], wf[2][T];
+
+  // What a step kt asks for: W of step kt + 4, and of the pair that takes the place of the one read last half the rows (kt odd: of
+  // pair (kt + 5) / 2; kt even: the other half, of pair (kt + 4) / 2).  So a step's barrier needs what steps up to kt - 3
+  // asked for; K is a multiple of 64, the steps an even number, and near the end step KB - 5 asks for W alone.
+  // First what steps before the first would have asked for, steps -3 to -1 last.
+#pragma unroll
+  for (int q = 0; q < 4; ++q) ask_x(0, 0, q);
+#pragma unroll
+  for (int q = 0; q < 2; ++q) ask_w(0, q);
+#pragma unroll
+  for (int d = 1; d < 4; ++d) {
+    if (d < KB) {
+      ask_w(d, 0);
+      ask_w(d, 1);
+    }
+    const int pair = d / 2 + d % 2;                      // 1, 1, 2
+    if (2 * pair < KB) {
+      ask_x(pair, pair, d == 2 ? 2 : 0);
+      ask_x(pair, pair, d == 2 ? 3 : 1);
+    }
+  }
+  if (KB >= 6) wait_vmcnt<12>();
+  else wait_vmcnt<0>();
+  __builtin_amdgcn_s_barrier();         // pair 0 and step 0 are in LDS for every wave
+  read_frags<T, 2048>(xf[0], xbase);
+  read_frags<T, 1024>(wf[0], wbase);
+  wait_lgkmcnt<0>();
+  use_frags<T>(xf[0]);
+  use_frags<T>(wf[0]);
+  int pair_slot = 0;                    // of the step being multiplied
+  // ODD, and what the step asks for: 2 W and X, 1 W alone, 0 nothing
+  auto step = [&](int kt, auto odd_of, auto asks_of) {
+    constexpr int odd = decltype(odd_of)::value, asks = decltype(asks_of)::value;
+    const int next_pair = pair_slot + 1 == KEPT_X_PAIRS ? 0 : pair_slot + 1, last_pair = pair_slot == 0 ? KEPT_X_PAIRS - 1 : pair_slot - 1;
+    if constexpr (asks != 0) {
+      wait_vmcnt<8>();
+    } else {
+      const int left = KB - kt;
+      if (left == 4) wait_vmcnt<6>();
+      else if (left == 3) wait_vmcnt<2>();
+      else wait_vmcnt<0>();
+    }
+    __builtin_amdgcn_s_barrier();       // step kt + 1 is in LDS for every wave; nobody reads step kt, or (odd) its pair, any more
+    const unsigned xr = odd ? xbase + next_pair * X_PAIR : (xbase ^ 64) + pair_slot * X_PAIR;
+    const unsigned wr = wbase + (kt + 1) % KEPT_W_STEPS * W_STEP;
+#pragma unroll
+    for (int t = 0; t < T * T; ++t) {
+      const int i = t / T, j = t % T;
+      const u32x4 xs = xf[odd][j], ws = wf[odd][i];
+      acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(ACROSS ? xs : ws), as_frag(ACROSS ? ws : xs), acc[i][j], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      if (t < T) lds_read16_step<2048, T>(xf[odd ^ 1][t % T], xr, t);
+      else if (t < 2 * T) lds_read16_step<1024, T>(wf[odd ^ 1][t % T], wr, t - T);
+      if (asks != 0 && t % 4 == 1) {
+        const int q = t / 4;            // W first: what the last asking step lacks is X
+        if (q < 2) ask_w(kt + 4, q % 2);
+        else if (asks == 2) {
+          if (odd) ask_x((kt + 5) / 2, pair_slot, q - 2);
+          else ask_x((kt + 4) / 2, last_pair, q);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (odd) pair_slot = next_pair;
+    wait_lgkmcnt<0>();                  // no read is under way across a branch
+    use_frags<T>(xf[odd ^ 1]);
+    use_frags<T>(wf[odd ^ 1]);
+  };
+  auto two_steps = [&](int kt, auto first_asks, auto second_asks) {
+    step(kt, Number<0>(), first_asks);
+    step(kt + 1, Number<1>(), second_asks);
+    if (kt + 2 == seg_end) {
+#pragma unroll
+      for (int i = 0; i < T; ++i)
+#pragma unroll
+        for (int j = 0; j < T; ++j) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) sum[i][j][e] = seg == 0 ? acc[i][j][e] : sum[i][j][e] + acc[i][j][e];
+          acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+      ++seg;
+      seg_end = (int)((long)(seg + 1) * (K / 64) / splits) * 2;
+    }
+  };
+  int kt = 0;
+  for (; kt + 6 < KB; kt += 2) two_steps(kt, Number<2>(), Number<2>());
+  if (kt + 4 < KB) {
+    two_steps(kt, Number<2>(), Number<1>());
+    kt += 2;
+  }
+  for (; kt < KB; kt += 2) two_steps(kt, Number<0>(), Number<0>());
+
+  const int mrow = m0 + wm * 64, ncol = n0 + wn * (GLU ? 32 : 64), four = (lane >> 4) * 4;
+  const auto value = [&](int c, int r, int e) { return sum[c][r][e]; };
+  if constexpr (ACROSS)
+    tile_epilogue<GLU, T, T>(value, [&](int c) { return ncol + (GLU ? c % 2 : c) * 16 + frow; }, [&](int r) { return mrow + r * 16 + four; },
+                             bias, bias_is_f32, out, out_stride, M, N, mode, partial);
+  else
+    tile_epilogue_four<GLU, T, T>(value, [&](int c) { return ncol + c * 16 + four; }, [&](int r) { return mrow + r * 16 + frow; }, bias,
+                                  bias_is_f32, out, out_stride, M, N, mode);
 }
 
 // ---------------------------------------------------------------------------- gemm_small_tile
@@ -867,7 +1020,8 @@ static int reserve_lds(int bytes) {
 //
 // Which way round (us, four columns of a row in a lane / columns across lanes).  Outputs that are stored go the first way: of
 // 16 bits 33,000 columns of K 1,024 at 1,500 rows 147 / 182, kept 5,632 of K 2,048 65 / 73, gated 18,944 of K 3,584 at 2,048
-// rows 462 / 469; of 32 bits kept 2,048 of K 2,048 at 2,048 rows 32 / 37, 5,632 65 / 74, 33,000 of K 1,024 at 1,525 142 / 170.
+// rows 462 / 469; of 32 bits kept 2,048 of K 2,048 at 2,048 rows 32 / 37, 5,632 65 / 74, 33,000 of K 1,024 at 1,525 142 / 170 (the
+// kept ones in steps of half lines).
 // The second way: sums of segments, which are read again (5,632 of K 2,048 at 320 rows 30.5 / 26.5, 3,584 of K 3,584 at 688
 // 43.8 / 39.9); rows added into, where 16 bytes of sixteen rows meet 64 lines twice (kept 3,584 of K 3,584 at 2,048 65.6 /
 // 62.8, 3,333 of K 512 35 / 25); rows of 32 bits that are not aligned for 16 bytes (3,333 of K 512 26.6 / 23.1); kept gated
@@ -876,7 +1030,8 @@ template <int BM, int BN, int WAVES_M, int WAVES_N, bool GLU, bool KEEP = false,
 static int launch_tile(const bf16_t* x, int x_stride, const bf16_t* w, const void* bias, int bias_is_f32, void* out,
                        int out_stride, int m, int n, int k, int mode, hipStream_t stream, int segs = 1,
                        float* partial = nullptr, const SplitNorm* norm = nullptr, const RopeStore* rope = nullptr) {
-  constexpr int lds_bytes = STAGES * (BM + BN) * 64;
+  static_assert(!KEEP || (BM == 128 && BN == 128 && WAVES_M == 2 && WAVES_N == 2), "the tiles of gemm_kept");
+  constexpr int lds_bytes = KEEP ? KEPT_LDS : STAGES * (BM + BN) * 64;
   static_assert(lds_bytes <= 160 * 1024, "the stages do not fit the LDS of a CU");
   const int splits = KEEP ? 1 : segs;
   const bool after = splits > 1 || norm || rope;
@@ -884,10 +1039,18 @@ static int launch_tile(const bf16_t* x, int x_stride, const bf16_t* w, const voi
   if constexpr (KEEP) AXK_INSTANCE(INST_GEMM_KEPT, GLU);
   else AXK_INSTANCE(INST_GEMM_TILE, BM, BN, WAVES_M, WAVES_N, GLU, STAGES * 32 / 64);
   auto go = [&](auto across) {
-    constexpr auto kernel = &gemm_tile_kernel<BM, BN, WAVES_M, WAVES_N, GLU, STAGES, KEEP, decltype(across)::value>;
-    if (int rc = reserve_lds<kernel>(lds_bytes)) return rc;
-    kernel<<<dim3(m_blocks * n_blocks, splits), WAVES_M * WAVES_N * 64, lds_bytes, stream>>>(
-        x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode, m_blocks, n_blocks, after ? partial : nullptr, segs);
+    constexpr bool ACROSS = decltype(across)::value;
+    if constexpr (KEEP) {
+      constexpr auto kernel = &gemm_tile_kernel_kept<GLU, ACROSS>;
+      if (int rc = reserve_lds<kernel>(lds_bytes)) return rc;
+      kernel<<<m_blocks * n_blocks, 256, lds_bytes, stream>>>(x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode, m_blocks,
+                                                              n_blocks, after ? partial : nullptr, segs);
+    } else {
+      constexpr auto kernel = &gemm_tile_kernel<BM, BN, WAVES_M, WAVES_N, GLU, STAGES, ACROSS>;
+      if (int rc = reserve_lds<kernel>(lds_bytes)) return rc;
+      kernel<<<dim3(m_blocks * n_blocks, splits), WAVES_M * WAVES_N * 64, lds_bytes, stream>>>(
+          x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode, m_blocks, n_blocks, after ? partial : nullptr);
+    }
     AXK_LAUNCH_CHECK("gemm_tile");
     return 0;
   };
