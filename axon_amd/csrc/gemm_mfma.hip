@@ -80,6 +80,19 @@ __device__ inline void wait_rounds(int rounds) {
 }
 
 // ---------------------------------------------------------------------------- what the tile kernels share
+// Memory from `base` on as a buffer: a load's place in it is a register of the lane's and a scalar one, with no address of its
+// own to work out, and what lies behind its `elems` elements reads as zeros.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_buffer(const bf16_t* base, size_t elems) {
+  return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, elems < 0x7fffffffu ? (unsigned)elems * 2u : 0xfffffffeu, 0x00027000);
+}
+// The rows of X from m on.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rows(const bf16_t* x, int x_stride, int m, int M, int K) {
+  return tile_buffer(x + (size_t)min(m, M - 1) * x_stride, m < M ? (size_t)(M - m - 1) * x_stride + K : 0);
+}
+__device__ __forceinline__ void tile_load(__amdgpu_buffer_rsrc_t rsrc, unsigned char* to, unsigned lane_bytes, unsigned bytes) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr_t)to, 16, (int)lane_bytes, (int)bytes, 0, 0);
+}
+
 // Block numbering: every eighth block runs on the same XCD, 32 of them at a time.  An XCD takes
 // every eighth n block and walks its share in squares of up to 8 m blocks x 4 n blocks, so that
 // the 32 blocks at work share 12 tiles of operands in that XCD's L2 (with many m blocks, all m
@@ -246,15 +259,15 @@ __device__ __forceinline__ void tile_epilogue_four(Value value, Col col, Row row
 }
 
 // ---------------------------------------------------------------------------- gemm_tile
-// LDS holds STAGES stages; a stage is 32 k: BM rows of X (64 bytes each) and the BN / 16 packed
-// blocks of W, written by direct global -> LDS loads of 16 bytes per lane (a wave instruction
-// fills 1024 bytes: 16 rows of X, or one block of W).  STAGES - 1 stages are under way, so the
-// latency of L2 and of the path into LDS is covered by as many blocks of products.
+// K is walked in steps of 32.  LDS holds three pairs of steps of X (BM rows of 128 bytes, a whole line each: half lines, a step
+// at a time, were twice the requests of L2) and four steps of W (the BN / 16 packed blocks), written by direct global ->
+// LDS loads of 16 bytes per lane (a wave instruction fills 1024 bytes: 8 rows of X, or one block of W).  Two to three steps
+// are under way, so the latency of L2 and of the path into LDS is covered by as many blocks of products.
 //
-// A row of X in a stage is 4 slots of 16 bytes, permuted (slot = k chunk ^ (row / 4 % 4)) so that
+// A row of X in a pair is 8 slots of 16 bytes, permuted (slot = k chunk ^ (row / 2 % 8)) so that
 // fragment reads of 16 neighbouring rows at one k chunk fall into different banks without padding
-// (which direct loads could not skip): LDS serves 256 bytes a cycle (64 banks), and the 16
-// 16-byte positions are then distinct modulo 256.
+// (which direct loads could not skip): LDS serves lanes 0-3, 12-15, 20-23 and 24-27 (4-11, 16-19 and 28-31, and so on) at a time, 256 bytes
+// a cycle, and their 16-byte positions are then distinct modulo 256.
 //
 // What bounds it, and why it is made so.  With every CU at work the card holds its power, not its
 // clock: 1.6 to 1.9 GHz instead of 2.4, so a product's energy counts like its cycles.
@@ -265,7 +278,11 @@ __device__ __forceinline__ void tile_epilogue_four(Value value, Col col, Row row
 //    the wave at their issue until the path into LDS (some 59 bytes a cycle) had taken them: a
 //    block of 256 x 256 x 64 took 3,300 cycles of which 2,048 are products; loads spread 3,020,
 //    reads spread too 2,900.
-// us, tiles of 32x32x16 products in steps of 64 k / here, in turn on one card: [gate; up] of 8,192 rows (18,944 columns of K
+//  * Loads are buffer loads with scalar places in rows and tiles: the address of a load in the vector unit was 4 % (of
+//    kept products, which have registers and issue slots to spare, nothing).
+// us, steps of half lines of X in five stages / whole lines / here, in turn: [gate; up] of a 7B layer (18,944 columns of K 3,584) at
+// 2,048 rows 478 / 442 / 424 (1.31 PFLOP/s), of a 14B layer (13,824 of K 5,120) at 1,525 rows 394 / 351 / 341, 3,584 columns of K 18,944 at
+// 2,048 rows with the sums' kernel 285 / 265 / 255.  Before that, tiles of 32x32x16 products in steps of 64 k / 16x16x32 products in those stages: [gate; up] of 8,192 rows (18,944 columns of K
 // 3,584) 1,944 / 1,729 (1.29 PFLOP/s), of 2,048 rows 515 / 461; 3,584 columns of K 18,944 at 2,048 rows (with the
 // sums' kernel) 300 / 286; 2,048^3 37.0 / 29.5; 1,500 rows of 33,000 columns of K 1,024 190 / 133 (four columns a
 // store).  Where the output is narrow and K long it loses: 2,048 columns of K 8,448 at 8,192 rows 365 / 390.  Slower: waves
@@ -278,41 +295,39 @@ __device__ __forceinline__ void tile_epilogue_four(Value value, Col col, Row row
 //
 // ACROSS: which operand of a product X and W are (the same bits), and so whether a lane holds one column of four rows or
 // four columns of a row (launch_tile says which for what).
-template <int BM, int BN, int WAVES_M, int WAVES_N, bool GLU, int STAGES, bool ACROSS>
+#define TILE_X_PAIRS 3
+#define TILE_W_STEPS 4
+template <int BM, int BN, int WAVES_M, int WAVES_N, bool GLU, bool ACROSS>
 __global__ void __launch_bounds__(WAVES_M * WAVES_N * 64, 1)
 gemm_tile_kernel(const bf16_t* __restrict__ x, int x_stride, const bf16_t* __restrict__ w, const void* __restrict__ bias,
                  int bias_is_f32, void* __restrict__ out, int out_stride, int M, int N, int K, int mode, int m_blocks,
                  int n_blocks, float* __restrict__ partial) {
-  extern __shared__ __align__(16) unsigned char smem[];
+  extern __shared__ __align__(128) unsigned char smem[];
   constexpr int NW = WAVES_M * WAVES_N;
   constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N;  // a wave's tile
   constexpr int TM = WM / 16, TN = WN / 16;            // in 16 x 16 MFMA tiles
   constexpr int TH = TN / 2;                           // tiles of W read at a time
-  constexpr int ROW = 64;                              // bytes of a row: 32 k
-  constexpr int XQ = BM / 16 / NW;                     // load instructions of X per wave and stage: 16 rows each
-  constexpr int WC = BN / 16, WQ = (WC + NW - 1) / NW; // blocks of W in a stage; load instructions per wave
+  constexpr int XQ = BM / 16 / NW;                     // load instructions of X per wave and half a pair: 8 rows each
+  constexpr int WC = BN / 16, WQ = (WC + NW - 1) / NW; // blocks of W in a step; load instructions per wave
   constexpr int LOADS = XQ + WQ;
-  constexpr int STAGE = (BM + BN) * ROW;               // bytes per stage
-  constexpr int AHEAD = STAGES - 1;                    // stages whose loads are under way
-  static_assert(XQ >= 1 && BM % (16 * NW) == 0 && (STAGES - 2) * LOADS < 64, "tile too small or too many loads in flight");
-  static_assert(WN % 32 == 0 && AHEAD % 2 == 0, "halves of a wave's W tiles; the loop takes two stages a turn");
+  constexpr int X_PAIR = BM * 128, W_STEP = BN * 64, W_AT = TILE_X_PAIRS * X_PAIR;      // bytes
+  static_assert(XQ >= 1 && BM % (16 * NW) == 0 && NW % 2 == 0 && 2 * LOADS < 64, "tile too small or too many loads in flight");
+  static_assert(WN % 32 == 0, "halves of a wave's W tiles");
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WAVES_N, wn = wave % WAVES_N;
 
   int mb, nb;
   tile_of_block(blockIdx.x, m_blocks, n_blocks, mb, nb);
   const int m0 = mb * BM, n0 = nb * (GLU ? BN / 2 : BN);
 
-  // what this lane fetches: row r = (q * NW + wave) * 16 + lane / 4 of a tile; it fills slot
-  // lane % 4 of that row, which holds k chunk (lane % 4) ^ (r / 4 % 4)
-  unsigned xoff[XQ], woff[WQ];
+  // what this lane fetches of X: row r = (q * NW + wave) * 8 + lane / 8 of a pair; it fills slot lane % 8 of that row, which
+  // holds k chunk (lane % 8) ^ (r / 2 % 8)
+  const unsigned x_lane = ((unsigned)(wave * 8 + (lane >> 3)) * (unsigned)x_stride + ((lane & 7) ^ ((4 * wave + (lane >> 4)) & 7)) * 8) * 2;
+  __amdgpu_buffer_rsrc_t x_rows[2 * XQ], w_tiles[WQ];
 #pragma unroll
-  for (int q = 0; q < XQ; ++q) {
-    const int r = (q * NW + wave) * 16 + (lane >> 2);
-    xoff[q] = (unsigned)min(m0 + r, M - 1) * (unsigned)x_stride + ((lane & 3) ^ ((r >> 2) & 3)) * 8;
-  }
-  // W: chunk c = (q * NW + wave) % WC of a stage is the packed block (row tile c, the stage's k block) of the tile, 1 KB
+  for (int q = 0; q < 2 * XQ; ++q) x_rows[q] = tile_rows(x, x_stride, m0 + q * NW * 8, M, K);
+  // W: chunk c = (q * NW + wave) % WC of a step is the packed block (row tile c, the step's k block) of the tile, 1 KB
   // as it lies in memory (where the waves do not divide the chunks, some twice: the same bytes to the same place).
   // Row tiles past the matrix: its last one (the epilogue drops those columns).
   const int KB = K / 32;
@@ -328,22 +343,18 @@ gemm_tile_kernel(const bf16_t* __restrict__ x, int x_stride, const bf16_t* __res
     } else {
       tile = min((n0 + r) / 16, row_tiles - 1);
     }
-    woff[q] = (unsigned)tile * (unsigned)KB * 512 + lane * 8;
+    w_tiles[q] = tile_buffer(w + (size_t)tile * KB * 512, (size_t)KB * 512);
   }
 
   // Split K (gridDim.y > 1): this block multiplies the k blocks kt_begin .. kt_begin + nk - 1 and
   // leaves its sums in `partial`; gemm_split_reduce_kernel adds the blocks' sums in block order.
   const int kt_begin = (int)((long)blockIdx.y * (K / 64) / gridDim.y) * 2;
   const int nk = (int)((long)(blockIdx.y + 1) * (K / 64) / gridDim.y) * 2 - kt_begin;       // even
-  // load instruction q of this wave for k block kt (counted from kt_begin) into stage `slot`
-  auto issue = [&](int slot, int kt, int q) {
-    unsigned char* stage = smem + slot * STAGE;
-    if (q < XQ)
-      __builtin_amdgcn_global_load_lds((global_ptr_t)(x + xoff[q < XQ ? q : 0] + (kt_begin + kt) * 32),
-                                       (lds_ptr_t)(stage + (q * NW + wave) * 1024), 16, 0, 0);
-    else
-      __builtin_amdgcn_global_load_lds((global_ptr_t)(w + woff[q < XQ ? 0 : q - XQ] + (kt_begin + kt) * 512),
-                                       (lds_ptr_t)(stage + BM * ROW + ((q - XQ) * NW + wave) % WC * 1024), 16, 0, 0);
+  auto ask_x = [&](int pair, int to, int q) {
+    tile_load(x_rows[q], smem + to * X_PAIR + (q * NW + wave) * 1024, x_lane, (kt_begin + 2 * pair) * 64);
+  };
+  auto ask_w = [&](int kt, int q) {
+    tile_load(w_tiles[q], smem + W_AT + (kt % TILE_W_STEPS) * W_STEP + (q * NW + wave) % WC * 1024, lane * 16, (kt_begin + kt) * 1024);
   };
 
   f32x4 acc[TN][TM];
@@ -352,58 +363,77 @@ gemm_tile_kernel(const bf16_t* __restrict__ x, int x_stride, const bf16_t* __res
 #pragma unroll
     for (int j = 0; j < TM; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
-  // X fragments: row = tile row + lane % 16, k chunk = lane / 16, at its permuted slot; W fragments: blocks as they are
+  // X fragments: row = tile row + lane % 16, k chunk = lane / 16 (+ 4 in a pair's second step), at its permuted slot; W
+  // fragments: blocks as they are
   const int frow = lane & 15;
   const unsigned lds0 = (unsigned)(size_t)(lds_ptr_t)smem;
-  const unsigned xbase = lds0 + (wm * WM + frow) * ROW + (((lane >> 4) ^ ((frow >> 2) & 3)) << 4);
-  const unsigned wbase = lds0 + BM * ROW + wn * WN * ROW + lane * 16;
+  const unsigned xbase = lds0 + (wm * WM + frow) * 128 + (((lane >> 4) ^ (frow >> 1)) << 4);
+  const unsigned wbase = lds0 + W_AT + wn * WN * 64 + lane * 16;
   // The reads are written as instructions: the compiler, which cannot tell the stage being read
   // from the stage a direct load is filling, would wait for every load in flight before each of
   // its own reads, and the loads of later stages would never overlap the products of this one.
   u32x4 xf[2][TM], wf[2][TH];
 
+  // What step kt asks for before its barrier: W of step kt + 3, and, into the place of the pair before its own, half the rows of
+  // a pair (kt even: of pair (kt + 4) / 2; kt odd: the other half, of pair (kt + 3) / 2).  A step's barrier needs what steps
+  // up to kt - 2 asked for (the pair of step kt + 1 and W of it); near the end step nk - 4 asks for W alone, those behind it for nothing.
+  // First what steps before the first would have asked for, -2 and -1 last.
 #pragma unroll
-  for (int d = 0; d < AHEAD; ++d)
-    if (d < nk) {
+  for (int q = 0; q < 2 * XQ; ++q) ask_x(0, 0, q);
 #pragma unroll
-      for (int q = 0; q < LOADS; ++q) issue(d, d, q);
-    }
-  wait_rounds<STAGES - 2, LOADS>(nk - 1);
-  __builtin_amdgcn_s_barrier();   // stage 0 is in LDS for every wave
-  read_frags<TM, 16 * ROW>(xf[0], xbase);
+  for (int q = 0; q < WQ; ++q) ask_w(0, q);
+#pragma unroll
+  for (int d = 1; d < 3; ++d) {
+#pragma unroll
+    for (int q = 0; q < WQ; ++q)
+      if (d < nk) ask_w(d, q);
+#pragma unroll
+    for (int q = 0; q < XQ; ++q)
+      if (2 < nk) ask_x(1, 1, (d - 1) * XQ + q);
+  }
+  if (nk >= 4) wait_vmcnt<2 * LOADS>();
+  else wait_vmcnt<0>();
+  __builtin_amdgcn_s_barrier();   // step 0 is in LDS for every wave
+  read_frags<TM, 2048>(xf[0], xbase);
   read_frags<TH, 1024>(wf[0], wbase);
   wait_lgkmcnt<0>();
   use_frags<TM>(xf[0]);
   use_frags<TH>(wf[0]);
-  int slot = 0;
-  // One k block: the products with the first half of the wave's W tiles while the second half is read, then those with the
-  // second half; halfway through these the next block's reads.  A load instruction of the block AHEAD of this one goes out
-  // every few products (the stage it fills was last read before the barrier in the block before this one).
-  auto block = [&](int kt, auto set_of, auto fetch_of) {
-    constexpr int set = decltype(set_of)::value;
-    constexpr bool fetch = decltype(fetch_of)::value;
+  int pair_slot = 0;              // of the step being multiplied
+  // One step: the products with the first half of the wave's W tiles while the second half is read, then those with the
+  // second half; halfway through these the next step's reads.  A load instruction goes out every few products (the place it
+  // fills was last read before the barrier in the step before this one).  asks: 2 W and X, 1 W alone, 0 nothing.
+  auto step = [&](int kt, auto odd_of, auto asks_of) {
+    constexpr int odd = decltype(odd_of)::value, asks = decltype(asks_of)::value;
     constexpr int HALF = TH * TM, BEFORE = HALF + HALF / 2;          // products before the barrier
     constexpr int EACH = (TM + TH + HALF / 2 - 1) / (HALF / 2);      // reads behind each product after it
-    const int next = slot + 1 == STAGES ? 0 : slot + 1, free_slot = slot == 0 ? STAGES - 1 : slot - 1;
+    const int next_pair = pair_slot + 1 == TILE_X_PAIRS ? 0 : pair_slot + 1, last_pair = pair_slot == 0 ? TILE_X_PAIRS - 1 : pair_slot - 1;
+    const unsigned xr = odd ? xbase + next_pair * X_PAIR : (xbase ^ 64) + pair_slot * X_PAIR;
+    const unsigned wr = wbase + kt % TILE_W_STEPS * W_STEP, wr_next = wbase + (kt + 1) % TILE_W_STEPS * W_STEP;
 #pragma unroll
     for (int t = 0; t < 2 * HALF; ++t) {
       if (t == HALF) {
-        wait_lgkmcnt<0>();              // the last fragments of this stage
+        wait_lgkmcnt<0>();              // the last fragments of this step
         use_frags<TH>(wf[1]);
       }
       if (t == BEFORE) {
-        // this wave's part of block kt + 1 has landed when only younger blocks' loads are outstanding
-        if constexpr (fetch) wait_vmcnt<(STAGES - 2) * LOADS>();
-        else wait_rounds<STAGES - 2, LOADS>(nk - 2 - kt);
-        __builtin_amdgcn_s_barrier();   // block kt + 1 is in LDS for every wave; nobody reads block kt any more
-      }                                 // (behind the last block: whatever the stage holds is read and not used)
+        if constexpr (asks == 2) {
+          wait_vmcnt<2 * LOADS>();
+        } else if constexpr (asks == 1) {
+          wait_vmcnt<LOADS + WQ>();
+        } else {
+          if (nk - kt == 3) wait_vmcnt<WQ>();
+          else wait_vmcnt<0>();
+        }
+        __builtin_amdgcn_s_barrier();   // step kt + 1 is in LDS for every wave; nobody reads step kt any more
+      }                                 // (behind the last step: whatever lies there is read and not used)
       const int i = t / TM, j = t % TM;
-      const u32x4 xs = xf[set][j], ws = wf[i / TH][i % TH];
+      const u32x4 xs = xf[odd][j], ws = wf[i / TH][i % TH];
       acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(ACROSS ? xs : ws), as_frag(ACROSS ? ws : xs), acc[i][j], 0, 0, 0);
-      // a read behind each product: the second half's behind the first ones, the next block's behind those after the barrier
+      // a read behind each product: the second half's behind the first ones, the next step's behind those after the barrier
       if (t < TH) {
         __builtin_amdgcn_sched_barrier(0);
-        lds_read16_step<1024, TH>(wf[1][t < TH ? t : 0], wbase + slot * STAGE + TH * 1024, t);
+        lds_read16_step<1024, TH>(wf[1][t < TH ? t : 0], wr + TH * 1024, t);
         __builtin_amdgcn_sched_barrier(0);
       }
       if (t >= BEFORE) {
@@ -411,33 +441,41 @@ gemm_tile_kernel(const bf16_t* __restrict__ x, int x_stride, const bf16_t* __res
         for (int r = (t - BEFORE) * EACH; r < (t - BEFORE + 1) * EACH; ++r) {
           if (r >= TM + TH) continue;
           __builtin_amdgcn_sched_barrier(0);
-          if (r < TM) lds_read16_step<16 * ROW, TM>(xf[set ^ 1][r < TM ? r : 0], xbase + next * STAGE, r);
-          else lds_read16_step<1024, TH>(wf[0][r < TM ? 0 : r - TM], wbase + next * STAGE, r - TM);
+          if (r < TM) lds_read16_step<2048, TM>(xf[odd ^ 1][r < TM ? r : 0], xr, r);
+          else lds_read16_step<1024, TH>(wf[0][r < TM ? 0 : r - TM], wr_next, r - TM);
           __builtin_amdgcn_sched_barrier(0);
         }
       }
-      if constexpr (fetch) {
 #pragma unroll
-        for (int q = 0; q < LOADS; ++q)
-          if (t == (2 * q + 1) * BEFORE / (2 * LOADS)) {
-            __builtin_amdgcn_sched_barrier(0);
-            issue(free_slot, kt + AHEAD, q);
-            __builtin_amdgcn_sched_barrier(0);
+      for (int q = 0; q < LOADS; ++q)
+        if (t == (2 * q + 1) * BEFORE / (2 * LOADS)) {
+          __builtin_amdgcn_sched_barrier(0);
+          if (q < WQ) {
+            if (asks != 0) ask_w(kt + 3, q < WQ ? q : 0);
+          } else if (asks == 2) {
+            ask_x(odd ? (kt + 3) / 2 : (kt + 4) / 2, last_pair, (odd ? XQ : 0) + (q < WQ ? 0 : q - WQ));
           }
-      }
+          __builtin_amdgcn_sched_barrier(0);
+        }
     }
-    slot = next;
-    wait_lgkmcnt<0>();                  // the next block's X and first half: no read is under way across a branch
-    use_frags<TM>(xf[set ^ 1]);
+    if (odd) pair_slot = next_pair;
+    wait_lgkmcnt<0>();                  // the next step's X and first half: no read is under way across a branch
+    use_frags<TM>(xf[odd ^ 1]);
     use_frags<TH>(wf[0]);
   };
-  auto two_blocks = [&](int kt, auto fetch_of) {
-    block(kt, Number<0>(), fetch_of);
-    block(kt + 1, Number<1>(), fetch_of);
-  };
   int kt = 0;
-  for (; kt + AHEAD < nk; kt += 2) two_blocks(kt, Number<1>());
-  for (; kt < nk; kt += 2) two_blocks(kt, Number<0>());
+  for (; kt + 4 < nk; kt += 2) {
+    step(kt, Number<0>(), Number<2>());
+    step(kt + 1, Number<1>(), Number<2>());
+  }
+  if (kt + 2 < nk) {
+    step(kt, Number<0>(), Number<1>());
+    step(kt + 1, Number<1>(), Number<0>());
+    kt += 2;
+  }
+  step(kt, Number<0>(), Number<0>());
+  step(kt + 1, Number<1>(), Number<0>());
+
   const int mrow = m0 + wm * WM, ncol = n0 + wn * (GLU ? WN / 2 : WN), four = (lane >> 4) * 4;
   const auto value = [&](int c, int r, int e) { return acc[c][r][e]; };
   if constexpr (ACROSS)       // a lane holds column lane % 16 and four rows from 4 (lane / 16) on of each tile
@@ -1026,18 +1064,18 @@ static int reserve_lds(int bytes) {
 // 43.8 / 39.9); rows added into, where 16 bytes of sixteen rows meet 64 lines twice (kept 3,584 of K 3,584 at 2,048 65.6 /
 // 62.8, 3,333 of K 512 35 / 25); rows of 32 bits that are not aligned for 16 bytes (3,333 of K 512 26.6 / 23.1); kept gated
 // products, whose waves own 32 columns of the output (1,408 of K 2,048 at 2,048 rows 37.7 / 36.4).
-template <int BM, int BN, int WAVES_M, int WAVES_N, bool GLU, bool KEEP = false, int STAGES = 5>
+template <int BM, int BN, int WAVES_M, int WAVES_N, bool GLU, bool KEEP = false>
 static int launch_tile(const bf16_t* x, int x_stride, const bf16_t* w, const void* bias, int bias_is_f32, void* out,
                        int out_stride, int m, int n, int k, int mode, hipStream_t stream, int segs = 1,
                        float* partial = nullptr, const SplitNorm* norm = nullptr, const RopeStore* rope = nullptr) {
   static_assert(!KEEP || (BM == 128 && BN == 128 && WAVES_M == 2 && WAVES_N == 2), "the tiles of gemm_kept");
-  constexpr int lds_bytes = KEEP ? KEPT_LDS : STAGES * (BM + BN) * 64;
+  constexpr int lds_bytes = KEEP ? KEPT_LDS : TILE_X_PAIRS * BM * 128 + TILE_W_STEPS * BN * 64;
   static_assert(lds_bytes <= 160 * 1024, "the stages do not fit the LDS of a CU");
   const int splits = KEEP ? 1 : segs;
   const bool after = splits > 1 || norm || rope;
   const int m_blocks = ceil_div(m, BM), n_blocks = ceil_div(n, GLU ? BN / 2 : BN);
   if constexpr (KEEP) AXK_INSTANCE(INST_GEMM_KEPT, GLU);
-  else AXK_INSTANCE(INST_GEMM_TILE, BM, BN, WAVES_M, WAVES_N, GLU, STAGES * 32 / 64);
+  else AXK_INSTANCE(INST_GEMM_TILE, BM, BN, WAVES_M, WAVES_N, GLU, TILE_W_STEPS * 32 / 64);
   auto go = [&](auto across) {
     constexpr bool ACROSS = decltype(across)::value;
     if constexpr (KEEP) {
@@ -1046,7 +1084,7 @@ static int launch_tile(const bf16_t* x, int x_stride, const bf16_t* w, const voi
       kernel<<<m_blocks * n_blocks, 256, lds_bytes, stream>>>(x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode, m_blocks,
                                                               n_blocks, after ? partial : nullptr, segs);
     } else {
-      constexpr auto kernel = &gemm_tile_kernel<BM, BN, WAVES_M, WAVES_N, GLU, STAGES, ACROSS>;
+      constexpr auto kernel = &gemm_tile_kernel<BM, BN, WAVES_M, WAVES_N, GLU, ACROSS>;
       if (int rc = reserve_lds<kernel>(lds_bytes)) return rc;
       kernel<<<dim3(m_blocks * n_blocks, splits), WAVES_M * WAVES_N * 64, lds_bytes, stream>>>(
           x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode, m_blocks, n_blocks, after ? partial : nullptr);

@@ -139,3 +139,25 @@ def test_outputs_anywhere(M, N, K, mode):
         k.gemm(x, w, rows[:, first:first + N], bias, mode)
         assert torch.equal(rows[:, first:first + N], plain), (wide, first)
         assert bool((rows[:, :first] == 1).all()) and bool((rows[:, first + N:] == 1).all()), (wide, first)
+
+
+@pytest.mark.parametrize("K", [64, 128, 192, 256, 320, 512, 576, 704])
+@pytest.mark.parametrize("N,M", [(9300, 1100), (4608, 2047)])
+def test_large_tiles_at_every_end_of_k(K, N, M):
+    """Steps of the tiles of 256 rows from one pair on, the last ones with less or nothing to ask for, and rows and columns past
+    the end: the bits of the streaming kernel's rows, whatever lies behind K and M in memory."""
+    k = kernels("bfloat16")
+    g = torch.Generator(device="cuda").manual_seed(K)
+    w = k.pack_matrix(torch.randn(N, K, generator=g, device="cuda").bfloat16())
+    x = torch.full((M + 1, K + 8), float("nan"), device="cuda", dtype=torch.bfloat16)
+    x[:M, :K] = torch.randn(M, K, generator=g, device="cuda").bfloat16()
+    for mode in (MODE_STORE_F32, MODE_STORE):
+        want = torch.empty(M, N, device="cuda", dtype=torch.float32 if mode == MODE_STORE_F32 else torch.bfloat16)
+        for at in range(0, M, 16):
+            k.gemm(x[at:min(at + 16, M), :K], w, want[at:at + 16], None, mode)
+        out = torch.full_like(want, float("nan"))
+        k.reset_instances()
+        k.gemm(x[:M, :K], w, out, None, mode)
+        assert torch.equal(out, want), mode
+        names = k.instances(launched=True)
+        assert any(name.startswith("gemm_tile<256") for name in names) or (K >= 512 and "gemm_kept<0>" in names), names
