@@ -26,6 +26,7 @@ import torch
 from ..cache.manager import CacheManager, host_lib
 from ..config.engine import EngineConfig
 from ..models.decoder import DecoderModel
+from ..upload import upload
 from .runtime import Runtime, Workspace
 
 
@@ -285,12 +286,11 @@ class Engine:
                 logits = self._decode_step(meta[0].tolist(), meta[1].tolist(), meta[2].tolist(), spans)
                 self._last_decode = [e.id for e in entries]
             else:
-                on_device = torch.from_numpy(np.ascontiguousarray(meta)).to(self.rt.device)
-                ctx = StepContext(self.rt, self.cache, self.ws, on_device, T, spans)
+                on_device = upload(np.concatenate([meta.reshape(-1), want_rows]), self.rt.device)
+                ctx = StepContext(self.rt, self.cache, self.ws, on_device[:3 * T].view(3, T), T, spans)
                 x = self.model.forward(ctx)
                 if len(want_rows):
-                    sel = torch.from_numpy(want_rows.copy()).to(self.rt.device)
-                    logits = self.model.logits(ctx, x, sel)
+                    logits = self.model.logits(ctx, x, on_device[3 * T:])
             for e, n in zip(entries, counts):
                 req = self.live[e.id]
                 req.n_cached += int(n)

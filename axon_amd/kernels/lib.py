@@ -23,8 +23,13 @@ class KernelError(RuntimeError):
     pass
 
 
-def _ptr(t: Optional[torch.Tensor]) -> c_void_p:
-    return c_void_p(0 if t is None else t.data_ptr())
+def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
+    # (a number: ctypes makes of it what the signature says, without the object made here)
+    return None if t is None else t.data_ptr()
+
+
+def ptr(t: Optional[torch.Tensor]) -> c_void_p:
+    return c_void_p(_ptr(t))
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
@@ -39,7 +44,7 @@ def _stream() -> c_void_p:
 
 
 # for the callers of `Kernels.call`: a tensor's (or a packed matrix's) address, the current stream
-ptr, current_stream = _ptr, _stream
+current_stream = _stream
 register_kernel_source = build.register_kernel_source
 
 

@@ -21,6 +21,7 @@ import torch
 
 from ..config.base import ConfigError
 from ..kernels import MODE_ADD_F32, MODE_STORE, PackedMatrix
+from ..upload import upload
 from .base import CacheBinding, CacheSpec, Mixer, PrecedingNorm, TensorDecl, build_part, register_mixer
 
 
@@ -78,13 +79,13 @@ class AttentionPlan:
             if (any(a < 0 or n < 1 or a + n > ctx.n_tokens for a, n in tiles)
                     or any(not 0 <= t < ctx.n_tokens for t in singles)):
                 raise ValueError("attention plan: a span lies outside the tokens of the step")
-            self.tiles = torch.tensor(pair_tiles(tiles, seen), dtype=torch.int32).to(dev) if tiles else None
-            self.decode_tokens = torch.tensor(singles, dtype=torch.int32).to(dev) if singles else None
+            self.tiles = upload(pair_tiles(tiles, seen), dev) if tiles else None
+            self.decode_tokens = upload(singles, dev) if singles else None
             self.max_chunks = max([1] + [decode_chunks_of(p, window, ctx.rt.k.attention_decode_chunk) for p in at])
             n_single = len(singles)
             if singles:
                 work = ctx.rt.k.attention_decode_work(at, window)
-                self.decode_work = torch.tensor(work, dtype=torch.int32).to(dev)
+                self.decode_work = upload(work, dev)
         if n_single:
             n = ctx.rt.k.attention_decode_workspace(n_single, n_heads, head_dim, self.max_chunks)
             lasting = ctx.decode_scratch.get(("attention_partial", window, n_heads, head_dim)) if ctx.decode_only else None

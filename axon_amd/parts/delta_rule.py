@@ -30,6 +30,7 @@ import torch
 
 from ..config.base import ConfigError
 from ..kernels import MODE_ADD_F32, MODE_STORE_F32
+from ..upload import upload
 from .base import CacheBinding, Mixer, StateSpec, TensorDecl, register_mixer
 from .recurrent import step_spans
 
@@ -53,7 +54,7 @@ def step_chunks(ctx) -> Optional[Tuple]:
                 continue
             spans5.append([s.slot, s.q_start, s.q_len, len(chunks), -(-s.q_len // CHUNK)])
             chunks += [[s.q_start + at, min(CHUNK, s.q_len - at)] for at in range(0, s.q_len, CHUNK)]
-        put = lambda rows, width: torch.tensor(rows, dtype=torch.int32).view(-1, width).to(ctx.rt.device)
+        put = lambda rows, width: upload(rows, ctx.rt.device).view(-1, width)
         made = ctx.shared["delta_rule_chunks"] = ((put(chunks, 2), put(spans5, 5)), put(rest, 3))
     return made
 

@@ -55,6 +55,7 @@ import torch
 
 from ..config.base import ConfigError
 from ..kernels import MODE_ADD_F32, MODE_STORE_F32, PackedMatrix
+from ..upload import upload
 from .base import CacheBinding, CacheSpec, Mixer, StateSpec, TensorDecl, build_part, register_mixer
 from .recurrent import step_spans
 
@@ -99,7 +100,7 @@ def attention_tiles(ctx, mask: str, size: int) -> Optional[torch.Tensor]:
         if any(a < 0 or n < 1 or a + n > ctx.n_tokens for _, a, n in rows):
             raise ValueError("attention tiles: a span lies outside the tokens of the step")
         rows.sort(key=lambda r: -r[0])
-        tiles = ctx.shared[key] = torch.tensor([(a, n) for _, a, n in rows], dtype=torch.int32).to(ctx.rt.device)
+        tiles = ctx.shared[key] = upload([(a, n) for _, a, n in rows], ctx.rt.device)
     return tiles
 
 

@@ -21,6 +21,7 @@ import torch
 
 from ..config.base import ConfigError
 from ..kernels import MODE_ADD_F32, MODE_STORE, MODE_STORE_F32
+from ..upload import upload
 from .base import CacheBinding, Mixer, StateSpec, TensorDecl, register_mixer
 
 
@@ -33,7 +34,7 @@ def step_spans(ctx) -> Optional[torch.Tensor]:
     spans = ctx.shared.get("step_spans")
     if spans is None:
         rows = [[s.slot, s.q_start, s.q_len] for s in ctx.spans]
-        spans = ctx.shared["step_spans"] = torch.tensor(rows, dtype=torch.int32).to(ctx.rt.device)
+        spans = ctx.shared["step_spans"] = upload(rows, ctx.rt.device)
     return spans
 
 

@@ -29,6 +29,7 @@ import torch
 
 from ..config.base import ConfigError
 from ..kernels import MODE_ADD_F32, MODE_STORE_F32
+from ..upload import upload
 from .base import CacheBinding, Mixer, StateSpec, TensorDecl, register_mixer
 from .recurrent import step_spans
 
@@ -64,8 +65,7 @@ def step_segments(ctx, blocks_a_stretch: int):
             spans5.append([s.slot, s.q_start, s.q_len, len(segs), -(-s.q_len // size)])
             for at in range(0, s.q_len, size):
                 segs.append([s.slot, s.q_start + at, min(size, s.q_len - at), 1 if at == 0 else 0])
-        made = ctx.shared[key] = (torch.tensor(segs, dtype=torch.int32).to(ctx.rt.device),
-                                  torch.tensor(spans5, dtype=torch.int32).to(ctx.rt.device), max(r[2] for r in segs))
+        made = ctx.shared[key] = (upload(segs, ctx.rt.device), upload(spans5, ctx.rt.device), max(r[2] for r in segs))
     return made
 
 
