@@ -45,7 +45,7 @@ __device__ inline void fma_store(float v, float up, bool glu, const void* bias, 
   else ((float*)out)[at] = v;
 }
 
-// Many rows: 64 x 64 outputs a block of 4 waves, each 2 x 2 tiles of 16 x 16 (gated: half of a wave's
+// Many rows (in the float32 build, those that gemm_fma_flow_kernel does not take): 64 x 64 outputs a block of 4 waves, each 2 x 2 tiles of 16 x 16 (gated: half of a wave's
 // columns are gate rows of W, half the up rows of the same outputs).  K is walked a chain at a time through
 // two stages of LDS; the stage's operands are read first, then the next stage is written and the one
 // after it asked for, all beside this stage's products.  A lane of a product holds k = 4 i + q of
@@ -349,6 +349,194 @@ gemm_fma_few_rows_kernel(const elem_t* __restrict__ x, int x_stride, const elem_
   }
 }
 
+#if !AXON_BF16
+// The same tiles and chains for rows of 32-bit numbers that are aligned: rows go to LDS as they lie in memory, by direct loads,
+// FLOW_STAGES stages ahead, and the numbers that a product wants of them (k = 4 s + q of row lane % 16) are read two tiles
+// at a time, two reads behind each of the first products of the step before.  So nothing is written to LDS, converted or cleared by the
+// vector unit, a wave waits for nothing that was not asked for half a step ago, and a chain's sums are added beside
+// the next chain's products.  A row of a stage is eight slots of 16 bytes, permuted by slot ^ (row / 2 % 8): the four k of 16
+// rows that a read takes fall on the 64 banks.
+// What bounds it: with four blocks a CU 83 % of what the products alone take (139 TFLOP/s at the clock that they leave); with one or two
+// blocks a CU also how they divide the rows (777 rows: 13 of 64, two rounds of 416 blocks or 1.6).
+// 777 rows, us, through registers / here: 2,560 x K 2,048 121 / 113, 2,048 x 2,048 90 / 77, 2,048 x 5,632 236 / 199, gated 5,632 x
+// 2,048 334 / 325, 32,000 x 2,048 947 / 930; 512 rows of 2,048 x 5,632 (a block a CU) 143 / 116, 2,048 rows 416 / 394.  With a read a
+// number (128 LDS instructions a block and step) 127 and 409 for the last two, three stages (three blocks a CU) 128 and 412.
+#define FLOW_STAGES 4
+#define FLOW_STAGE (2 * TILE_M * FMA_PART * 4)
+typedef const __attribute__((address_space(1))) void* fma_global_t;
+typedef __attribute__((address_space(3))) void* fma_lds_t;
+typedef __attribute__((ext_vector_type(2))) float f32x2;
+// The numbers at an address and 2 KB, 16 rows of a stage, behind it.
+__device__ __forceinline__ void lds_read_two(f32x2& dst, unsigned lds_address) {
+  asm volatile("ds_read2st64_b32 %0, %1 offset0:0 offset1:8" : "=v"(dst) : "v"(lds_address));
+}
+__device__ __forceinline__ void use_numbers(f32x2& v) { asm volatile("" : "+v"(v)); }
+template <int V>
+struct FmaNumber {
+  static constexpr int value = V;
+};
+template <bool GLU>
+__global__ void __launch_bounds__(256, 2)
+gemm_fma_flow_kernel(const float* __restrict__ x, int x_stride, const float* __restrict__ w, const void* __restrict__ bias,
+                     int bias_is_f32, void* __restrict__ out, int out_stride, int M, int N, int K, int mode) {
+  constexpr int R = 2, BM = TILE_M, BN = GLU ? BM / 2 : BM;
+  extern __shared__ __align__(128) unsigned char flow[];          // [stage]: X [64][32], W [64][32]
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
+  const int r16 = lane & 15, q = lane >> 4;
+  const int wm = (wave >> 1) * 16 * R, wn = (wave & 1) * 16 * R;
+
+  // A load fills 8 rows of a stage, lane l slot l % 8 of row l / 8, which holds k chunk slot ^ (row / 2 % 8): loads 0 and 1 rows
+  // 8 (4 j + wave) and on of X, loads 2 and 3 the same of W (gated: in a wave's 32 rows 16 gate rows, then the up rows of the same outputs)
+  const int lrow = lane >> 3, chunk = (lane & 7) ^ ((4 * wave + (lane >> 4)) & 7);
+  const bool up = GLU && (wave & 2);
+  const FmaRows x_rows = fma_rows(x + (size_t)m0 * x_stride, (size_t)(M - m0 - 1) * x_stride + K);
+  const FmaRows w_rows = fma_rows(w + (size_t)(n0 + (up ? N : 0)) * K, (size_t)(N - n0) * K);
+  unsigned at[4];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int row = 8 * (4 * j + wave) + lrow, col = GLU ? 16 * j + 8 * (wave & 1) + lrow : row;
+    at[j] = ((unsigned)min(row, M - 1 - m0) * (unsigned)x_stride + 4 * chunk) * 4;
+    at[2 + j] = ((unsigned)min(col, N - 1 - n0) * (unsigned)K + 4 * chunk) * 4;
+  }
+  auto ask = [&](int t, int j) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(j < 2 ? x_rows.rsrc : w_rows.rsrc,
+                                             (fma_lds_t)(flow + t % FLOW_STAGES * FLOW_STAGE + (j < 2 ? 0 : BM * 128) + (4 * (j & 1) + wave) * 1024), 16,
+                                             (int)at[j], t * FMA_PART * 4, 0, 0);
+  };
+  const unsigned lds0 = (unsigned)(size_t)(fma_lds_t)flow;
+  unsigned x_at[8], w_at[8];               // of product s of a chain: of X's first tile, of W's
+#pragma unroll
+  for (int s = 0; s < 8; ++s) {
+    x_at[s] = lds0 + (wm + r16) * 128 + ((s ^ (r16 >> 1)) << 4) + 4 * q;
+    w_at[s] = x_at[s] + BM * 128 + (wn - wm) * 128;
+  }
+  f32x2 a[2][8], b[2][8];                  // of a wave's two tiles
+  // read p of the 16 of a stage: X's and W's numbers of product p / 2
+  auto read = [&](auto set_of, unsigned stage, int p) {
+    constexpr int set = decltype(set_of)::value;
+    if (p % 2 == 0) lds_read_two(a[set][p / 2], x_at[p / 2] + stage);
+    else lds_read_two(b[set][p / 2], w_at[p / 2] + stage);
+  };
+  auto arrived = [&](auto set_of) {
+    constexpr int set = decltype(set_of)::value;
+    wait_lgkmcnt<0>();
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      use_numbers(a[set][s]);
+      use_numbers(b[set][s]);
+    }
+  };
+  f32x4 sum[R][R], acc[2][R][R];
+#pragma unroll
+  for (int i = 0; i < R; ++i)
+#pragma unroll
+    for (int j = 0; j < R; ++j) sum[i][j] = acc[1][i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+
+  const int n_steps = (K + FMA_PART - 1) / FMA_PART;
+#pragma unroll
+  for (int t = 0; t < FLOW_STAGES; ++t)
+    if (t < n_steps) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) ask(t, j);
+    }
+  if (n_steps >= FLOW_STAGES) wait_vmcnt<4 * (FLOW_STAGES - 1)>();
+  else wait_vmcnt<0>();
+  __builtin_amdgcn_s_barrier();            // stage 0 is in LDS for every wave
+#pragma unroll
+  for (int p = 0; p < 16; ++p) read(FmaNumber<0>(), 0u, p);
+  arrived(FmaNumber<0>());
+  // Step t, whose numbers are in registers: its stage is free behind the barrier.  asks: for stage t + FLOW_STAGES.
+  auto step = [&](int t, auto set_of, auto asks_of) {
+    constexpr int set = decltype(set_of)::value, other = set ^ 1;
+    constexpr bool asks = decltype(asks_of)::value != 0;
+    if constexpr (asks) {
+      wait_vmcnt<4 * (FLOW_STAGES - 2)>();
+    } else {
+      const int left = n_steps - t;        // of the stages behind the next, left - 2 may still be under way
+      if (FLOW_STAGES >= 4 && left >= 4) wait_vmcnt<8>();
+      else if (left >= 3) wait_vmcnt<4>();
+      else wait_vmcnt<0>();
+    }
+    __builtin_amdgcn_s_barrier();          // stage t + 1 is in LDS for every wave; nobody reads stage t any more
+    const unsigned next = (unsigned)((t + 1) % FLOW_STAGES * FLOW_STAGE);
+#pragma unroll
+    for (int p = 0; p < 8 * R * R; ++p) {
+      const int s = p / (R * R), i = p / R % R, j = p % R;
+      if (s == 0) acc[set][i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      acc[set][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[set][s][i], b[set][s][j], acc[set][i][j], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      if (p < 8) {                         // as soon as they go: spread over 16, 24 or 32 products they take 1 to 5 % longer
+        read(FmaNumber<other>(), next, 2 * p);
+        read(FmaNumber<other>(), next, 2 * p + 1);
+      }
+      if (p >= 16 && p < 20) sum[(p - 16) / R][p % R] += acc[other][(p - 16) / R][p % R];      // the chain before
+      if (asks && p >= 20 && p % 3 == 0) ask(t + FLOW_STAGES, (p - 21) / 3);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    arrived(FmaNumber<other>());           // (behind the last step: whatever lies there, not used)
+  };
+  const int whole = K / FMA_PART;          // the last step of a K that is no multiple of 32 has fewer products
+  int t = 0;
+  for (; t + 1 + FLOW_STAGES < n_steps; t += 2) {
+    step(t, FmaNumber<0>(), FmaNumber<1>());
+    step(t + 1, FmaNumber<1>(), FmaNumber<1>());
+  }
+  if (t + FLOW_STAGES < n_steps) {         // one more asks
+    step(t, FmaNumber<0>(), FmaNumber<1>());
+    step(t + 1, FmaNumber<1>(), FmaNumber<0>());
+    t += 2;
+  }
+  for (; t + 1 < whole; t += 2) {
+    step(t, FmaNumber<0>(), FmaNumber<0>());
+    step(t + 1, FmaNumber<1>(), FmaNumber<0>());
+  }
+  auto last = [&](auto set_of) {           // the products of the k that are left
+    constexpr int set = decltype(set_of)::value;
+    const int count = (K - whole * FMA_PART) / 4;
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+#pragma unroll
+      for (int j = 0; j < R; ++j) {
+        sum[i][j] += acc[set ^ 1][i][j];
+        acc[set][i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      }
+#pragma unroll
+    for (int s = 0; s < 8; ++s)
+      if (s < count) {
+#pragma unroll
+        for (int i = 0; i < R; ++i)
+#pragma unroll
+          for (int j = 0; j < R; ++j) acc[set][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[set][s][i], b[set][s][j], acc[set][i][j], 0, 0, 0);
+      }
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+#pragma unroll
+      for (int j = 0; j < R; ++j) sum[i][j] += acc[set][i][j];
+  };
+  if (t < whole) {                         // t is even: one whole step, and what may be left
+    step(t, FmaNumber<0>(), FmaNumber<0>());
+    last(FmaNumber<1>());
+  } else {
+    last(FmaNumber<0>());
+  }
+
+  constexpr int COLS = GLU ? R / 2 : R;
+#pragma unroll
+  for (int i = 0; i < R; ++i)
+#pragma unroll
+    for (int j = 0; j < COLS; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int m = m0 + wm + 16 * i + 4 * q + e;
+        const int n = n0 + (GLU ? wn / 2 : wn) + 16 * j + r16;
+        if (m < M && n < N)
+          fma_store(sum[i][j][e], GLU ? sum[i][j + (GLU ? COLS : 0)][e] : 0.0f, GLU, bias, bias_is_f32, out,
+                    (size_t)m * out_stride + n, n, mode);
+      }
+}
+#endif
+
 template <int MT, bool GLU, bool VEC>
 static void launch_fma_few(const elem_t* x, int x_stride, const elem_t* w, const void* bias, int bias_is_f32, void* out,
                            int out_stride, int m, int n, int k, int mode, hipStream_t stream) {
@@ -363,6 +551,19 @@ static void launch_fma_few(const elem_t* x, int x_stride, const elem_t* w, const
   if (k <= FEW_WAVES * FMA_PART) { if (columns <= 8) FEW(8, true); else FEW(16, true); }
   else { if (columns <= 8) FEW(8, false); else FEW(16, false); }
 #undef FEW
+}
+
+template <bool GLU, bool VEC>
+static void launch_fma_tiles(dim3 tiles, const elem_t* x, int x_stride, const elem_t* w, const void* bias, int bias_is_f32, void* out,
+                             int out_stride, int m, int n, int k, int mode, hipStream_t stream) {
+#if !AXON_BF16
+  if constexpr (VEC) {                       // FLOW_STAGES of 16 KB are what a launch gets unasked
+    static_assert(FLOW_STAGES * FLOW_STAGE <= 64 * 1024, "more LDS than a launch gets unasked");
+    gemm_fma_flow_kernel<GLU><<<tiles, 256, FLOW_STAGES * FLOW_STAGE, stream>>>(x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode);
+    return;
+  }
+#endif
+  gemm_fma_kernel<GLU, VEC><<<tiles, 256, 0, stream>>>(x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode);
 }
 
 static int launch_fma(const elem_t* x, int x_stride, const elem_t* w, const void* bias, int bias_is_f32, void* out,
@@ -389,7 +590,7 @@ static int launch_fma(const elem_t* x, int x_stride, const elem_t* w, const void
     launch_fma_few<4, GLU, VEC>(FMA_ARGS);                                                    \
   } else {                                                                                    \
     AXK_INSTANCE(INST_GEMM_FMA, 128, GLU);                                                    \
-    gemm_fma_kernel<GLU, VEC><<<tiles, 256, 0, stream>>>(x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode); \
+    launch_fma_tiles<GLU, VEC>(tiles, FMA_ARGS);                                              \
   }
   const bool glu = mode == MODE_SWIGLU;
   if (vec_x && vec_w) {

@@ -100,3 +100,24 @@ def test_columns_a_block_and_rounds_of_chains(N, K):
         k.gemm(x[:m], w[:2 * half], out, None, MODE_SWIGLU)
         k.swiglu(torch.cat([gate, up], 1)[:m].contiguous(), act)
         assert torch.equal(out, act), m
+
+
+@pytest.mark.parametrize("K", [4, 28, 32, 60, 64, 96, 124, 128, 132, 160, 188, 192, 224, 228, 1056])
+def test_tiles_at_every_end_of_k(K):
+    """Whole and broken last steps of K behind fewer and more stages than LDS holds, rows and columns past the end, and rows of X
+    with numbers that are none behind K: the bits of chains of fmaf."""
+    k = kernels("float32")
+    g = torch.Generator(device="cuda").manual_seed(K)
+    M, N = 201, 150
+    x = torch.full((M + 1, K + 4), float("nan"), device="cuda")
+    x[:M, :K] = torch.randn(M, K, generator=g, device="cuda")
+    w = torch.randn(N, K, generator=g, device="cuda")
+    want = _by_chains(k, x[:M, :K], w)
+    out = torch.full((M + 1, N + 2), float("nan"), device="cuda")
+    k.gemm(x[:M, :K], w, out[:M, :N], None, MODE_STORE_F32)
+    assert torch.equal(out[:M, :N], want) and bool(out[M:].isnan().all()) and bool(out[:, N:].isnan().all())
+    half = N // 2
+    got, act = (torch.full((M, half), float("nan"), device="cuda") for _ in range(2))
+    k.gemm(x[:M, :K], w, got, None, MODE_SWIGLU)
+    k.swiglu(want[:, :2 * half].contiguous(), act)
+    assert torch.equal(got, act)
