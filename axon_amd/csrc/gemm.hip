@@ -321,7 +321,7 @@ gemm_fma_few_rows_kernel(const elem_t* __restrict__ x, int x_stride, const elem_
       }
     }
     if (BUFFERS == 1) {
-      asm volatile("" ::: "memory");
+      wait_lgkmcnt<0>();                     // the sums' reads have run before another wave writes the next round's there
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
     }

@@ -1053,7 +1053,7 @@ static int reserve_lds(int bytes) {
   return 0;
 }
 
-// The tiles of gemm_tile, STAGES stages of 32 k.  A block a segment (gridDim.y), the sums through `partial`; or, with KEEP, a
+// The tiles of gemm_tile.  A block a segment (gridDim.y), the sums through `partial`; or, with KEEP, a
 // block all of them, the finished sums through `partial` where the kernel that adds sums does more than that.
 //
 // Which way round (us, four columns of a row in a lane / columns across lanes).  Outputs that are stored go the first way: of

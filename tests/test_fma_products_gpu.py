@@ -10,7 +10,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("mode", [MODE_STORE_F32, MODE_ADD_F32, MODE_SWIGLU])
 @pytest.mark.parametrize("N,K,x_stride", [(8, 4, 4), (63, 33, 33), (65, 64, 68), (257, 292, 292), (40, 2052, 2055), (4100, 36, 40),
-                                           (520, 256, 256), (24, 257, 260), (16390, 40, 44)])
+                                           (520, 256, 256), (24, 257, 260), (16390, 40, 44),
+                                           (4100, 2052, 2052)])
 def test_edges_of_rows_columns_and_chains(N, K, x_stride, mode):
     k = kernels("float32")
     g = torch.Generator(device="cuda").manual_seed(N + K)
