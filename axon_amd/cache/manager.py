@@ -26,7 +26,6 @@ import torch
 
 from ..kernels import build
 from ..parts.base import CacheSpec
-from ..upload import upload
 
 
 class CacheError(RuntimeError):
@@ -249,22 +248,25 @@ class CacheManager:
         if not self._dirty:
             return
         slots = sorted(self._dirty)
-        n = len(slots)
+        n, places, on_device_places = len(slots), torch.tensor(slots), None
         for gi, g in enumerate(self.groups):
             on_device = g.block_table is not None
             rows = torch.zeros((n, self.max_pages_per_seq), dtype=torch.int32, pin_memory=on_device)
+            at, row_bytes = rows.data_ptr(), 4 * self.max_pages_per_seq
             for i, slot in enumerate(slots):
-                got = self.lib.axh_cache_row(self._h, gi, slot, c_void_p(rows[i].data_ptr()), self.max_pages_per_seq)
+                got = self.lib.axh_cache_row(self._h, gi, slot, c_void_p(at + i * row_bytes), self.max_pages_per_seq)
                 if got < 0:
                     raise CacheError(f"no block table row for group {gi}, slot {slot}")
-                g.host_table[slot].copy_(rows[i])
+            g.host_table.index_copy_(0, places, rows)
             if not on_device:
                 continue
-            if n <= 4:              # four copies take the host as long as the scatter's three calls
+            if n <= 4:              # four copies take the host as long as the scatter and what it reads
                 for i, slot in enumerate(slots):
                     g.block_table[slot].copy_(rows[i], non_blocking=True)
             else:
-                g.block_table.index_copy_(0, upload(slots, self.device).long(), rows.to(self.device, non_blocking=True))
+                if on_device_places is None:
+                    on_device_places = places.pin_memory().to(self.device, non_blocking=True)
+                g.block_table.index_copy_(0, on_device_places, rows.to(self.device, non_blocking=True))
         self._dirty.clear()
 
     # ------------------------------------------------------------------ accounting
