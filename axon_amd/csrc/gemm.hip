@@ -12,6 +12,7 @@
 // what four fmaf in ascending k give (measured over random operands, denormals among them), at
 // twice the rate that the vector unit has without its packed instructions.
 #include "api.h"
+#include "buffer.h"
 #include "common.h"
 #include "instances.h"
 
@@ -161,7 +162,7 @@ gemm_fma_kernel(const elem_t* __restrict__ x, int x_stride, const elem_t* __rest
 // an output adds them in ascending order.  MT tiles of 16 rows of X ride along with each W (a wave reads
 // them from L2 beside W, which is what bounds it from some 32 rows on).  What a wave multiplies next, W and X, is
 // asked for as soon as the registers are free, with no branch between, so that loads are under way through the
-// products, the barrier and the sums; they are buffer loads, whose k is in a scalar register, and the two halves of a
+// products, the barrier and the sums; they are buffer loads, whose k is in scalar registers, and the two halves of a
 // line (16 k) are asked for one behind the other (four loads apart they came from L2 twice: 2,048 x K 5,632 at 16 rows
 // 27 us, 22 so).  One chain of a wave at a time, or two where both operands are one tile: more of them (4 and 8)
 // only wait for each other (the same 22 us against 20; a gated 5,632 x 2,048 of 5 rows 26 against 23 us).
@@ -176,26 +177,29 @@ typedef __attribute__((ext_vector_type(2))) unsigned fma_quad;      // four numb
 #else
 typedef u32x4 fma_quad;
 #endif
-// Rows `stride` apart as a buffer: a row's place in it is in the lane's register and k in a scalar one, so that a load
-// needs no address of its own, and what lies behind the last row reads as zeros.
+// Rows as a buffer (buffer.h): a row's place in it is in the lane's register and the buffer begins at the k that is asked for, so
+// that a load needs no address of its own, and what lies behind the last row reads as zeros.
 struct FmaRows {
-  __amdgpu_buffer_rsrc_t rsrc;
   const elem_t* base;
+  unsigned bytes;
+  __device__ __forceinline__ __amdgpu_buffer_rsrc_t from(int k) const {       // k: at most K
+    return __builtin_amdgcn_make_buffer_rsrc((void*)(base + k), 0, bytes - (unsigned)k * (unsigned)sizeof(elem_t), 0x00027000);
+  }
 };
-__device__ __forceinline__ FmaRows fma_rows(const elem_t* base, size_t elems) {
-  const size_t bytes = elems * sizeof(elem_t);
-  return {__builtin_amdgcn_make_buffer_rsrc((void*)base, 0, bytes < 0xffffffffu ? (unsigned)bytes : 0xffffffffu, 0x00027000), base};
+__device__ __forceinline__ FmaRows fma_rows(const elem_t* matrix, int m, int M, int stride, int K) {
+  const BufferRows rows = buffer_rows(m, M, stride, K, sizeof(elem_t));
+  return {matrix + rows.first, rows.bytes};
 }
 // Four k of the row that begins `at` elements behind the first, k = k0 + in_chain .. + 3 (in_chain: this lane's place in
 // the chain that begins at k0).  Aligned operands read on into the next row behind K; others take the row's last number.
 template <bool VEC>
 __device__ __forceinline__ fma_quad fma_ask(const FmaRows& rows, unsigned at, int k0, int in_chain, int K) {
   if (VEC) {
-    const int off = (int)((at + in_chain) * sizeof(elem_t)), s_off = (int)(k0 * sizeof(elem_t));
+    const int off = (int)((at + in_chain) * sizeof(elem_t));
 #if AXON_BF16
-    return __builtin_amdgcn_raw_buffer_load_b64(rows.rsrc, off, s_off, 0);
+    return __builtin_amdgcn_raw_buffer_load_b64(rows.from(min(k0, K)), off, 0, 0);
 #else
-    return __builtin_amdgcn_raw_buffer_load_b128(rows.rsrc, off, s_off, 0);
+    return __builtin_amdgcn_raw_buffer_load_b128(rows.from(min(k0, K)), off, 0, 0);
 #endif
   }
   union { fma_quad q; elem_t e[4]; } c;
@@ -235,8 +239,8 @@ gemm_fma_few_rows_kernel(const elem_t* __restrict__ x, int x_stride, const elem_
   const int n0 = blockIdx.x * columns, m0 = blockIdx.y * MT * 16;
   FmaRows w_rows[NT];
 #pragma unroll
-  for (int t = 0; t < NT; ++t) w_rows[t] = fma_rows(w + (size_t)(n0 + t * N) * K, (size_t)(N - n0) * K);
-  const FmaRows x_rows = fma_rows(x + (size_t)m0 * x_stride, (size_t)(M - m0 - 1) * x_stride + K);
+  for (int t = 0; t < NT; ++t) w_rows[t] = fma_rows(w + (size_t)t * N * K, n0, N, K, K);
+  const FmaRows x_rows = fma_rows(x, m0, M, x_stride, K);
   const unsigned w_at = (unsigned)min(min(r16, columns - 1), N - 1 - n0) * (unsigned)K;
   unsigned x_at[MT];
 #pragma unroll
@@ -390,8 +394,8 @@ gemm_fma_flow_kernel(const float* __restrict__ x, int x_stride, const float* __r
   // 8 (4 j + wave) and on of X, loads 2 and 3 the same of W (gated: in a wave's 32 rows 16 gate rows, then the up rows of the same outputs)
   const int lrow = lane >> 3, chunk = (lane & 7) ^ ((4 * wave + (lane >> 4)) & 7);
   const bool up = GLU && (wave & 2);
-  const FmaRows x_rows = fma_rows(x + (size_t)m0 * x_stride, (size_t)(M - m0 - 1) * x_stride + K);
-  const FmaRows w_rows = fma_rows(w + (size_t)(n0 + (up ? N : 0)) * K, (size_t)(N - n0) * K);
+  const FmaRows x_rows = fma_rows(x, m0, M, x_stride, K);
+  const FmaRows w_rows = fma_rows(w + (up ? (size_t)N * K : 0), n0, N, K, K);
   unsigned at[4];
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
@@ -400,9 +404,9 @@ gemm_fma_flow_kernel(const float* __restrict__ x, int x_stride, const float* __r
     at[2 + j] = ((unsigned)min(col, N - 1 - n0) * (unsigned)K + 4 * chunk) * 4;
   }
   auto ask = [&](int t, int j) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(j < 2 ? x_rows.rsrc : w_rows.rsrc,
+    __builtin_amdgcn_raw_ptr_buffer_load_lds((j < 2 ? x_rows : w_rows).from(t * FMA_PART),
                                              (fma_lds_t)(flow + t % FLOW_STAGES * FLOW_STAGE + (j < 2 ? 0 : BM * 128) + (4 * (j & 1) + wave) * 1024), 16,
-                                             (int)at[j], t * FMA_PART * 4, 0, 0);
+                                             (int)at[j], 0, 0, 0);
   };
   const unsigned lds0 = (unsigned)(size_t)(fma_lds_t)flow;
   unsigned x_at[8], w_at[8];               // of product s of a chain: of X's first tile, of W's

@@ -41,7 +41,8 @@ def model_dirs(tmp_path_factory):
 
 @pytest.fixture(scope="session")
 def device_code(tmp_path_factory):
-    """The bfloat16 device code of a source under csrc, as text, compiled once a session; no GPU is needed."""
+    """The device code of a source under csrc (of the bfloat16 build unless another is named), as text, compiled once a session; no GPU
+    is needed."""
     import shutil
     import subprocess
 
@@ -51,11 +52,11 @@ def device_code(tmp_path_factory):
         pytest.skip("no compiler")
     made = {}
 
-    def of(source):
-        if source not in made:
+    def of(source, dtype="bfloat16"):
+        if (source, dtype) not in made:
             out = tmp_path_factory.mktemp("device") / (source + ".s")
-            subprocess.run([hipcc, *B.HIP_FLAGS, B.DTYPE_FLAG["bfloat16"], "-S", "--cuda-device-only", os.path.join(B.CSRC, source), "-o", str(out)],
+            subprocess.run([hipcc, *B.HIP_FLAGS, B.DTYPE_FLAG[dtype], "-S", "--cuda-device-only", os.path.join(B.CSRC, source), "-o", str(out)],
                            check=True, capture_output=True, timeout=600)
-            made[source] = out.read_text()
-        return made[source]
+            made[source, dtype] = out.read_text()
+        return made[source, dtype]
     return of
