@@ -44,6 +44,7 @@
 //   neighbouring rows fall into different banks; W blocks land as they are.  Blocks are numbered
 //   so that the blocks of one XCD (every eighth block) share weight tiles in that XCD's L2.
 #include "api.h"
+#include "buffer.h"
 #include "common.h"
 #include "instances.h"
 
@@ -80,14 +81,11 @@ __device__ inline void wait_rounds(int rounds) {
 }
 
 // ---------------------------------------------------------------------------- what the tile kernels share
-// Memory from `base` on as a buffer: a load's place in it is a register of the lane's and a scalar one, with no address of its
-// own to work out, and what lies behind its `elems` elements reads as zeros.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_buffer(const bf16_t* base, size_t elems) {
-  return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, elems < 0x7fffffffu ? (unsigned)elems * 2u : 0xfffffffeu, 0x00027000);
-}
-// The rows of X from m on.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rows(const bf16_t* x, int x_stride, int m, int M, int K) {
-  return tile_buffer(x + (size_t)min(m, M - 1) * x_stride, m < M ? (size_t)(M - m - 1) * x_stride + K : 0);
+// Memory as a buffer (buffer.h): a load's place in it is a register of the lane's and a scalar one, with no address of its own to
+// work out; lanes whose row is behind the last one read nothing and get zeros.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rows(const bf16_t* matrix, int m, int M, int stride, int K) {
+  const BufferRows rows = buffer_rows(m, M, stride, K, 2);
+  return __builtin_amdgcn_make_buffer_rsrc((void*)(matrix + rows.first), 0, rows.bytes, 0x00027000);
 }
 __device__ __forceinline__ void tile_load(__amdgpu_buffer_rsrc_t rsrc, unsigned char* to, unsigned lane_bytes, unsigned bytes) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr_t)to, 16, (int)lane_bytes, (int)bytes, 0, 0);
@@ -326,7 +324,7 @@ gemm_tile_kernel(const bf16_t* __restrict__ x, int x_stride, const bf16_t* __res
   const unsigned x_lane = ((unsigned)(wave * 8 + (lane >> 3)) * (unsigned)x_stride + ((lane & 7) ^ ((4 * wave + (lane >> 4)) & 7)) * 8) * 2;
   __amdgpu_buffer_rsrc_t x_rows[2 * XQ], w_tiles[WQ];
 #pragma unroll
-  for (int q = 0; q < 2 * XQ; ++q) x_rows[q] = tile_rows(x, x_stride, m0 + q * NW * 8, M, K);
+  for (int q = 0; q < 2 * XQ; ++q) x_rows[q] = tile_rows(x, m0 + q * NW * 8, M, x_stride, K);
   // W: chunk c = (q * NW + wave) % WC of a step is the packed block (row tile c, the step's k block) of the tile, 1 KB
   // as it lies in memory (where the waves do not divide the chunks, some twice: the same bytes to the same place).
   // Row tiles past the matrix: its last one (the epilogue drops those columns).
@@ -343,7 +341,7 @@ gemm_tile_kernel(const bf16_t* __restrict__ x, int x_stride, const bf16_t* __res
     } else {
       tile = min((n0 + r) / 16, row_tiles - 1);
     }
-    w_tiles[q] = tile_buffer(w + (size_t)tile * KB * 512, (size_t)KB * 512);
+    w_tiles[q] = tile_rows(w, tile, tile + 1, KB * 512, KB * 512);
   }
 
   // Split K (gridDim.y > 1): this block multiplies the k blocks kt_begin .. kt_begin + nk - 1 and

@@ -59,3 +59,19 @@ def test_chains_read_their_rows_and_nothing_behind_the_last(buffer_rows, M, K, g
                 assert left >= 0 and (place + load <= left)[reads].all()
                 assert ((first + k) * size + place + load <= end)[reads].all()
                 assert reads[np.broadcast_to(32 * chain + in_chain < K, reads.shape)].all()
+
+
+@pytest.mark.parametrize("M, K, gap", [(1, 64, 0), (64, 128, 8), (65, 192, 0), (129, 320, 8), (200, 64, 64), (256, 128, 0), (333, 2048, 0)])
+def test_tiles_read_rows_that_there_are(buffer_rows, M, K, gap):
+    """Rows past M, whole groups of them too: a lane reads within the operand with its scalar place, or is stopped without it."""
+    stride, block_rows, group = K + gap, 256, 64                 # rows of X a block, rows that the waves load at a time
+    end = ((M - 1) * stride + K) * 2
+    row, slot = np.arange(group)[:, None], np.arange(8)[None, :]
+    place = (row * stride + slot * 8) * 2
+    for m in range(0, -(-M // block_rows) * block_rows, group):
+        first, total = buffer_rows(m, M, stride, K, 2)
+        reads = place < total
+        for k in range(0, K, 64):
+            assert (place + 2 * k + 16 <= total)[reads].all() and (first * 2 + place + 2 * k + 16 <= end)[reads].all()
+        assert (reads[np.broadcast_to(m + row < M, reads.shape)]).all()
+        assert total > 0, "nothing is known of a scalar place in a buffer of no bytes"
