@@ -169,8 +169,7 @@ gemm_fma_kernel(const elem_t* __restrict__ x, int x_stride, const elem_t* __rest
 // 5 rows, us, before (X asked for chain by chain between branches, a round's loads behind the last one's sums) / now:
 // 2,560 x K 2,048 15.3 / 8.5, 2,048 x 2,048 11.7 / 8.9, gated 5,632 x 2,048 33.1 / 21.0 (4.4 TB/s), 2,048 x 5,632 28.9 / 17.5,
 // 32,000 x 2,048 66 / 52 (5.0 TB/s); 32 rows of 2,560 x 2,048 23.3 / 13.5, of 32,000 x 2,048 102 / 90; 64 rows of
-// 2,048 x 5,632 65 / 56.  A K that is no multiple of four loads its numbers singly: 1,000 x K 1,001 of 5 rows 9.4 / 7.3, but of
-// 20 to 128 rows 5 to 7 % longer than before.
+// 2,048 x 5,632 65 / 56.
 #define FEW_WAVES 8
 #if AXON_BF16
 typedef __attribute__((ext_vector_type(2))) unsigned fma_quad;      // four numbers as they lie in memory
@@ -230,7 +229,7 @@ gemm_fma_few_rows_kernel(const elem_t* __restrict__ x, int x_stride, const elem_
                          const void* __restrict__ bias, int bias_is_f32, void* __restrict__ out, int out_stride, int M,
                          int N, int K, int mode, int columns) {
   constexpr int NT = GLU ? 2 : 1;
-  constexpr int ROUND = SHORT || MT * NT >= (VEC ? 2 : 4) ? 1 : 2;
+  constexpr int ROUND = SHORT || MT * NT >= 2 ? 1 : 2;
   constexpr int PARTS = FEW_WAVES * ROUND, OUTS = MT * 16 * NR, ALL = NT * OUTS;
   constexpr int BUFFERS = PARTS * ALL * 4 > 32768 ? 1 : 2;          // of chains: two where two blocks a CU leave room
   __shared__ __align__(16) float chains[BUFFERS * PARTS * ALL];       // [chain][gate, up][row][NR columns]
@@ -254,6 +253,7 @@ gemm_fma_few_rows_kernel(const elem_t* __restrict__ x, int x_stride, const elem_
   fma_quad wq[ROUND][NT][2], xq[ROUND][MT][2];
   auto ask = [&](int p, int first) {
     const int k0 = (first + p * FEW_WAVES + wave) * FMA_PART;
+    if (!VEC && k0 >= K) return;             // no chain, the same for the whole wave
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
@@ -271,6 +271,7 @@ gemm_fma_few_rows_kernel(const elem_t* __restrict__ x, int x_stride, const elem_
 #pragma unroll
     for (int p = 0; p < ROUND; ++p) {
       const int part = p * FEW_WAVES + wave, k0 = (first + part) * FMA_PART, k = k0 + 4 * q;
+      if (!more && k0 >= K) continue;                      // no chain: in the last round alone
       if (k0 < K && k0 + FMA_PART > K) {                   // K ends in this chain: the same for the whole wave
 #pragma unroll
         for (int g = 0; g < 2; ++g) {
@@ -301,7 +302,7 @@ gemm_fma_few_rows_kernel(const elem_t* __restrict__ x, int x_stride, const elem_
               if (g == 0 && s == 0) acc[i][t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
               FMA_STEP(acc[i][t], a[t][g], b[i][g], s);
             }
-      // columns 4 q .. 4 q + 3 of row 16 i + r16; of a chain behind the last one too: it is not added
+      // columns 4 q .. 4 q + 3 of row 16 i + r16
 #pragma unroll
       for (int i = 0; i < MT; ++i)
 #pragma unroll
@@ -353,8 +354,100 @@ gemm_fma_few_rows_kernel(const elem_t* __restrict__ x, int x_stride, const elem_
   }
 }
 
+// The same for numbers that have to be loaded singly (a K, rows or a base that are not aligned for four), but for the products of up to
+// 16 rows that launch_fma_few names: four loads take the place of one, with addresses of their own, so X is asked for chain by
+// chain, when it is multiplied, several chains of W before it, and a wave without a chain asks for nothing.  All of X ahead, as
+// above, does not fit the registers (gated, 64 rows).  us, all ahead / so: 20 rows of 1,000 x K 1,001 14.0 / 13.1, 40 of 2,048 x 2,047
+// 40.4 / 37.0, gated 5,632 x 2,049 5 rows 59.3 / 58.6, 32 91.5 / 86.5, 64 140 / 122; 256 x 127 of 5 rows 3.2 / 2.7, of 64 6.7 / 4.5.
+template <int MT, int NR, bool GLU, bool SHORT>
+__global__ void __launch_bounds__(64 * FEW_WAVES, 2)
+gemm_fma_singles_kernel(const elem_t* __restrict__ x, int x_stride, const elem_t* __restrict__ w, const void* __restrict__ bias,
+                        int bias_is_f32, void* __restrict__ out, int out_stride, int M, int N, int K, int mode) {
+  constexpr int NT = GLU ? 2 : 1;
+  constexpr int PW = SHORT || MT * NT >= 8 ? 1 : MT * NT >= 3 ? 2 : MT * NT == 2 ? 4 : 8;   // chains of a wave in a round
+  constexpr int PARTS = FEW_WAVES * PW, OUTS = MT * 16 * NR;
+  __shared__ __align__(16) float chains[PARTS * NT * OUTS];                        // [chain][gate, up][row][column]
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int r16 = lane & 15, q = lane >> 4;
+  const int n0 = blockIdx.x * NR, m0 = blockIdx.y * MT * 16;
+  const elem_t* w_row = w + (size_t)min(n0 + min(r16, NR - 1), N - 1) * K;
+  const elem_t* x_row[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) x_row[i] = x + (size_t)min(m0 + 16 * i + r16, M - 1) * x_stride;
+  const int n_parts = (K + FMA_PART - 1) / FMA_PART;
+  constexpr int MINE = (OUTS + 64 * FEW_WAVES - 1) / (64 * FEW_WAVES);
+  float sum[MINE], sum_up[MINE];
+#pragma unroll
+  for (int i = 0; i < MINE; ++i) sum[i] = sum_up[i] = 0.0f;
+
+  for (int first = 0; first < n_parts; first += PARTS) {
+    float wv[NT][PW][2][4];
+#pragma unroll
+    for (int p = 0; p < PW; ++p)
+#pragma unroll
+      for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+          fma_load<false>(w_row + (size_t)t * N * K, (first + wave * PW + p) * FMA_PART + 16 * g + 4 * q, K, wv[t][p][g]);
+#pragma unroll
+    for (int p = 0; p < PW; ++p) {
+      const int part = wave * PW + p, k0 = (first + part) * FMA_PART;
+      if (k0 >= K) break;                            // the same for the whole wave
+      f32x4 a[NT][2];
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+          if (k0 + FMA_PART > K) fma_clear(wv[t][p][g], k0 + 16 * g + 4 * q, K);
+          a[t][g] = f32_operand(wv[t][p][g]);
+        }
+#pragma unroll
+      for (int i = 0; i < MT; ++i) {
+        f32x4 b[2];
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+          float xv[4];
+          fma_load<false>(x_row[i], k0 + 16 * g + 4 * q, K, xv);
+          if (k0 + FMA_PART > K) fma_clear(xv, k0 + 16 * g + 4 * q, K);
+          b[g] = f32_operand(xv);
+        }
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          f32x4 acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+          for (int g = 0; g < 2; ++g)
+#pragma unroll
+            for (int s = 0; s < 4; ++s) FMA_STEP(acc, a[t][g], b[g], s);
+          // columns 4 q .. 4 q + 3 of row 16 i + r16
+          if (4 * q < NR) *reinterpret_cast<f32x4*>(&chains[(part * NT + t) * OUTS + (16 * i + r16) * NR + 4 * q]) = acc;
+        }
+      }
+    }
+    __syncthreads();
+    const int count = min(PARTS, n_parts - first);
+#pragma unroll
+    for (int i = 0; i < MINE; ++i) {
+      const int o = tid + 64 * FEW_WAVES * i;
+      if (o < OUTS) {
+#pragma unroll 8
+        for (int p = 0; p < count; ++p) {
+          sum[i] += chains[p * NT * OUTS + o];
+          if (GLU) sum_up[i] += chains[(p * NT + NT - 1) * OUTS + o];
+        }
+      }
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int i = 0; i < MINE; ++i) {
+    const int o = tid + 64 * FEW_WAVES * i, m = m0 + o / NR, col = n0 + o % NR;
+    if (o < OUTS && m < M && col < N)
+      fma_store(sum[i], sum_up[i], GLU, bias, bias_is_f32, out, (size_t)m * out_stride + col, col, mode);
+  }
+}
+
 #if !AXON_BF16
-// The same tiles and chains for rows of 32-bit numbers that are aligned: rows go to LDS as they lie in memory, by direct loads,
+// gemm_fma_kernel's tiles and chains for rows of 32-bit numbers that are aligned: rows go to LDS as they lie in memory, by direct loads,
 // FLOW_STAGES stages ahead, and the numbers that a product wants of them (k = 4 s + q of row lane % 16) are read two tiles
 // at a time, two reads behind each of the first products of the step before.  So nothing is written to LDS, converted or cleared by the
 // vector unit, a wave waits for nothing that was not asked for half a step ago, and a chain's sums are added beside
@@ -544,17 +637,44 @@ gemm_fma_flow_kernel(const float* __restrict__ x, int x_stride, const float* __r
 template <int MT, bool GLU, bool VEC>
 static void launch_fma_few(const elem_t* x, int x_stride, const elem_t* w, const void* bias, int bias_is_f32, void* out,
                            int out_stride, int m, int n, int k, int mode, hipStream_t stream) {
-  // As many blocks as give every CU the same number of them, with at most 16 columns each (2,560 columns in 256 blocks of 10:
-  // 9.0 us, in 160 of 16 10.3; 11,264 gated in 512 of 11: 27.3, in 352 of 16 30.8), and so many that X counts less than W
-  const int rows = ceil_div(m, 16 * MT), each = ceil_div(ceil_div(n, 16) * rows, 256);
-  const int columns = max(MT == 1 ? 4 : 8, min(16, ceil_div(n * rows, 256 * each)));
-  const dim3 blocks(ceil_div(n, columns), rows);
+  const int rows = ceil_div(m, 16 * MT);
+  const bool brief = k <= FEW_WAVES * FMA_PART;
+  // Numbers loaded singly: one tile of rows and one of W, in a K of more than a chain a wave, are asked for ahead like others (us,
+  // against chain by chain: 5 rows of 1,000 x K 1,001 7.5 / 9.5, of 300 x 5,631 31 / 40, of 2,048 x 515 6.0 / 8.4; 16 of 2,048 x 769 9.7 / 10.3,
+  // of 16,390 x 515 29.4 / 33.8)
+  constexpr bool AHEAD = VEC || (MT == 1 && !GLU);
+  if constexpr (!VEC) {
+    if (brief || !AHEAD) {
+      const bool narrow = (long)ceil_div(n, 16) * rows < 256;      // blocks of 8 columns where blocks of 16 would leave CUs without one
+#define SINGLES(NR, SHORT)                                                                                       \
+  gemm_fma_singles_kernel<MT, NR, GLU, SHORT><<<dim3(ceil_div(n, NR), rows), 64 * FEW_WAVES, 0, stream>>>(       \
+      x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode)
+      if (brief) { if (narrow) SINGLES(8, true); else SINGLES(16, true); }
+      else if constexpr (!AHEAD) { if (narrow) SINGLES(8, false); else SINGLES(16, false); }
+#undef SINGLES
+      return;
+    }
+  }
+  if constexpr (AHEAD) {
+    // As many blocks as give every CU the same number of them, with at most 16 columns each (2,560 columns in 256 blocks of 10:
+    // 9.0 us, in 160 of 16 10.3; 11,264 gated in 512 of 11: 27.3, in 352 of 16 30.8), and so many that X counts less than W.
+    // X that is loaded singly counts more than a last round: 16 columns from four blocks a CU on (16 rows of 16,390 x 1,001 in blocks
+    // of 13: 51.7, of 16 48.9)
+    const int each = ceil_div(ceil_div(n, 16) * rows, 256);
+    const int columns = !VEC && each >= 4 ? 16 : max(MT == 1 ? 4 : 8, min(16, ceil_div(n * rows, 256 * each)));
+    const dim3 blocks(ceil_div(n, columns), rows);
 #define FEW(NR, SHORT)                                                                            \
   gemm_fma_few_rows_kernel<MT, NR, GLU, VEC, SHORT><<<blocks, 64 * FEW_WAVES, 0, stream>>>(   \
       x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode, columns)
-  if (k <= FEW_WAVES * FMA_PART) { if (columns <= 8) FEW(8, true); else FEW(16, true); }
-  else { if (columns <= 8) FEW(8, false); else FEW(16, false); }
+    if constexpr (VEC) {
+      if (brief) {
+        if (columns <= 8) FEW(8, true); else FEW(16, true);
+        return;
+      }
+    }
+    if (columns <= 8) FEW(8, false); else FEW(16, false);
 #undef FEW
+  }
 }
 
 template <bool GLU, bool VEC>

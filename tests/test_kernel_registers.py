@@ -31,3 +31,15 @@ def test_sums_of_segments_leave_the_tiles_across_lanes(device_code):
         stores = set(re.findall(r"\b(global_store_\w+)", body))
         across += "global_store_dword" in stores and not stores & {"global_store_dwordx2", "global_store_dwordx4"}
     assert across >= 5                # 256 columns, gated and not, 192, and kept ones, gated and not
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_32_bit_products_of_few_rows_spill_nothing(device_code, dtype):
+    seen = set()
+    for note in re.findall(r"- \.agpr_count:.*?\.wavefront_size:", device_code("gemm.hip", dtype), re.S):
+        field = {k: v for k, v in re.findall(r"\.(\w+):\s+(\S+)", note)}
+        kernel = re.search(r"gemm_fma_(few_rows|singles)_kernel", field["symbol"])
+        if kernel:
+            seen.add(kernel[1])
+            assert int(field["vgpr_spill_count"]) == 0 and int(field["private_segment_fixed_size"]) == 0, field
+    assert seen == {"few_rows", "singles"}
