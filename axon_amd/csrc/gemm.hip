@@ -181,8 +181,9 @@ typedef u32x4 fma_quad;
 struct FmaRows {
   const elem_t* base;
   unsigned bytes;
-  __device__ __forceinline__ __amdgpu_buffer_rsrc_t from(int k) const {       // k: at most K
-    return __builtin_amdgcn_make_buffer_rsrc((void*)(base + k), 0, bytes - (unsigned)k * (unsigned)sizeof(elem_t), 0x00027000);
+  // From number k of the rows on; where there is no such number, of no bytes: nothing is read.
+  __device__ __forceinline__ __amdgpu_buffer_rsrc_t from(int k, bool any = true) const {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)(base + k), 0, any ? bytes - (unsigned)k * (unsigned)sizeof(elem_t) : 0u, 0x00027000);
   }
 };
 __device__ __forceinline__ FmaRows fma_rows(const elem_t* matrix, int m, int M, int stride, int K) {
@@ -196,9 +197,9 @@ __device__ __forceinline__ fma_quad fma_ask(const FmaRows& rows, unsigned at, in
   if (VEC) {
     const int off = (int)((at + in_chain) * sizeof(elem_t));
 #if AXON_BF16
-    return __builtin_amdgcn_raw_buffer_load_b64(rows.from(min(k0, K)), off, 0, 0);
+    return __builtin_amdgcn_raw_buffer_load_b64(rows.from(k0, k0 < K), off, 0, 0);
 #else
-    return __builtin_amdgcn_raw_buffer_load_b128(rows.from(min(k0, K)), off, 0, 0);
+    return __builtin_amdgcn_raw_buffer_load_b128(rows.from(k0, k0 < K), off, 0, 0);
 #endif
   }
   union { fma_quad q; elem_t e[4]; } c;
@@ -251,9 +252,10 @@ gemm_fma_few_rows_kernel(const elem_t* __restrict__ x, int x_stride, const elem_
   for (int i = 0; i < MINE; ++i) sum[i] = 0.0f;
 
   fma_quad wq[ROUND][NT][2], xq[ROUND][MT][2];
-  auto ask = [&](int p, int first) {
+  // whole: of a round whose chains all exist
+  auto ask = [&](int p, int first, bool whole) {
     const int k0 = (first + p * FEW_WAVES + wave) * FMA_PART;
-    if (!VEC && k0 >= K) return;             // no chain, the same for the whole wave
+    if (!VEC && !whole && k0 >= K) return;   // no chain, the same for the whole wave
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
@@ -264,9 +266,9 @@ gemm_fma_few_rows_kernel(const elem_t* __restrict__ x, int x_stride, const elem_
       for (int g = 0; g < 2; ++g) xq[p][i][g] = fma_ask<VEC>(x_rows, x_at[i], k0, 16 * g + 4 * q, K);
   };
 #pragma unroll
-  for (int p = 0; p < ROUND; ++p) ask(p, 0);
+  for (int p = 0; p < ROUND; ++p) ask(p, 0, false);
   int buffer = 0;
-  auto round = [&](int first, bool more) {
+  auto round = [&](int first, bool more, bool whole) {
     float* to = chains + buffer * PARTS * ALL;
 #pragma unroll
     for (int p = 0; p < ROUND; ++p) {
@@ -289,7 +291,7 @@ gemm_fma_few_rows_kernel(const elem_t* __restrict__ x, int x_stride, const elem_
 #pragma unroll
         for (int i = 0; i < MT; ++i) b[i][g] = fma_operand(xq[p][i][g]);
       }
-      if (more) ask(p, first + PARTS);
+      if (more) ask(p, first + PARTS, whole);
       f32x4 acc[MT][NT];
 #pragma unroll
       for (int g = 0; g < 2; ++g)
@@ -333,8 +335,16 @@ gemm_fma_few_rows_kernel(const elem_t* __restrict__ x, int x_stride, const elem_
     if (BUFFERS == 2) buffer ^= 1;
   };
   int first = 0;
-  for (; first + PARTS < n_parts; first += PARTS) round(first, true);
-  round(first, false);
+  if constexpr (VEC) {
+    for (; first + PARTS < n_parts; first += PARTS) round(first, true, false);
+  } else {                       // the check of every chain takes up to 7 % (a row of 300 x K 5,631)
+    for (; first + 2 * PARTS <= n_parts; first += PARTS) round(first, true, true);
+    if (first + PARTS < n_parts) {
+      round(first, true, false);
+      first += PARTS;
+    }
+  }
+  round(first, false, false);
 
   float up[MINE];
   if (GLU) {                     // the up sums go to the threads that hold the gates'
@@ -354,23 +364,26 @@ gemm_fma_few_rows_kernel(const elem_t* __restrict__ x, int x_stride, const elem_
   }
 }
 
-// The same for numbers that have to be loaded singly (a K, rows or a base that are not aligned for four), but for the products of up to
-// 16 rows that launch_fma_few names: four loads take the place of one, with addresses of their own, so X is asked for chain by
-// chain, when it is multiplied, several chains of W before it, and a wave without a chain asks for nothing.  All of X ahead, as
-// above, does not fit the registers (gated, 64 rows).  us, all ahead / so: 20 rows of 1,000 x K 1,001 14.0 / 13.1, 40 of 2,048 x 2,047
-// 40.4 / 37.0, gated 5,632 x 2,049 5 rows 59.3 / 58.6, 32 91.5 / 86.5, 64 140 / 122; 256 x 127 of 5 rows 3.2 / 2.7, of 64 6.7 / 4.5.
-template <int MT, int NR, bool GLU, bool SHORT>
+// The same with X asked for chain by chain, when it is multiplied, several chains of W before it; a wave without a chain asks for
+// nothing and multiplies nothing (launch_fma_few says for which products).
+//  * Numbers that have to be loaded singly (a K, rows or a base that are not aligned for four): four loads take the place of one, with
+//    addresses of their own, and all of X ahead does not fit the registers.  us, all ahead / so: 20 rows of 1,000 x K 1,001
+//    14.0 / 13.1, 40 of 2,048 x 2,047 40.4 / 37.0, gated 5,632 x 2,049 5 rows 59.3 / 58.6, 32 91.5 / 86.5, 64 140 / 122; 256 x 127 of
+//    5 rows 3.2 / 2.7, of 64 6.7 / 4.4.
+//  * Fewer chains than waves: 64 rows of 64 x K 96 4.0 / 3.0 us, of 256 x 128 4.6 / 3.4, of 4,096 x 192 8.2 / 7.2, gated 512 x 128
+//    5.9 / 4.2; 5 rows 2.4 / 2.2, 2.5 / 2.4, 3.6 / 3.6 and 3.3 / 2.8.
+template <int MT, int NR, bool GLU, bool VEC, bool SHORT>
 __global__ void __launch_bounds__(64 * FEW_WAVES, 2)
-gemm_fma_singles_kernel(const elem_t* __restrict__ x, int x_stride, const elem_t* __restrict__ w, const void* __restrict__ bias,
-                        int bias_is_f32, void* __restrict__ out, int out_stride, int M, int N, int K, int mode) {
+gemm_fma_by_chain_kernel(const elem_t* __restrict__ x, int x_stride, const elem_t* __restrict__ w, const void* __restrict__ bias,
+                         int bias_is_f32, void* __restrict__ out, int out_stride, int M, int N, int K, int mode, int columns) {
   constexpr int NT = GLU ? 2 : 1;
   constexpr int PW = SHORT || MT * NT >= 8 ? 1 : MT * NT >= 3 ? 2 : MT * NT == 2 ? 4 : 8;   // chains of a wave in a round
   constexpr int PARTS = FEW_WAVES * PW, OUTS = MT * 16 * NR;
   __shared__ __align__(16) float chains[PARTS * NT * OUTS];                        // [chain][gate, up][row][column]
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r16 = lane & 15, q = lane >> 4;
-  const int n0 = blockIdx.x * NR, m0 = blockIdx.y * MT * 16;
-  const elem_t* w_row = w + (size_t)min(n0 + min(r16, NR - 1), N - 1) * K;
+  const int n0 = blockIdx.x * columns, m0 = blockIdx.y * MT * 16;
+  const elem_t* w_row = w + (size_t)min(n0 + min(r16, columns - 1), N - 1) * K;
   const elem_t* x_row[MT];
 #pragma unroll
   for (int i = 0; i < MT; ++i) x_row[i] = x + (size_t)min(m0 + 16 * i + r16, M - 1) * x_stride;
@@ -388,7 +401,7 @@ gemm_fma_singles_kernel(const elem_t* __restrict__ x, int x_stride, const elem_t
       for (int g = 0; g < 2; ++g)
 #pragma unroll
         for (int t = 0; t < NT; ++t)
-          fma_load<false>(w_row + (size_t)t * N * K, (first + wave * PW + p) * FMA_PART + 16 * g + 4 * q, K, wv[t][p][g]);
+          fma_load<VEC>(w_row + (size_t)t * N * K, (first + wave * PW + p) * FMA_PART + 16 * g + 4 * q, K, wv[t][p][g]);
 #pragma unroll
     for (int p = 0; p < PW; ++p) {
       const int part = wave * PW + p, k0 = (first + part) * FMA_PART;
@@ -407,7 +420,7 @@ gemm_fma_singles_kernel(const elem_t* __restrict__ x, int x_stride, const elem_t
 #pragma unroll
         for (int g = 0; g < 2; ++g) {
           float xv[4];
-          fma_load<false>(x_row[i], k0 + 16 * g + 4 * q, K, xv);
+          fma_load<VEC>(x_row[i], k0 + 16 * g + 4 * q, K, xv);
           if (k0 + FMA_PART > K) fma_clear(xv, k0 + 16 * g + 4 * q, K);
           b[g] = f32_operand(xv);
         }
@@ -440,8 +453,8 @@ gemm_fma_singles_kernel(const elem_t* __restrict__ x, int x_stride, const elem_t
   }
 #pragma unroll
   for (int i = 0; i < MINE; ++i) {
-    const int o = tid + 64 * FEW_WAVES * i, m = m0 + o / NR, col = n0 + o % NR;
-    if (o < OUTS && m < M && col < N)
+    const int o = tid + 64 * FEW_WAVES * i, m = m0 + o / NR, c = o % NR, col = n0 + c;
+    if (o < OUTS && c < columns && m < M && col < N)
       fma_store(sum[i], sum_up[i], GLU, bias, bias_is_f32, out, (size_t)m * out_stride + col, col, mode);
   }
 }
@@ -637,44 +650,44 @@ gemm_fma_flow_kernel(const float* __restrict__ x, int x_stride, const float* __r
 template <int MT, bool GLU, bool VEC>
 static void launch_fma_few(const elem_t* x, int x_stride, const elem_t* w, const void* bias, int bias_is_f32, void* out,
                            int out_stride, int m, int n, int k, int mode, hipStream_t stream) {
-  const int rows = ceil_div(m, 16 * MT);
-  const bool brief = k <= FEW_WAVES * FMA_PART;
-  // Numbers loaded singly: one tile of rows and one of W, in a K of more than a chain a wave, are asked for ahead like others (us,
-  // against chain by chain: 5 rows of 1,000 x K 1,001 7.5 / 9.5, of 300 x 5,631 31 / 40, of 2,048 x 515 6.0 / 8.4; 16 of 2,048 x 769 9.7 / 10.3,
-  // of 16,390 x 515 29.4 / 33.8)
+  // As many blocks as give every CU the same number of them, with at most 16 columns each (2,560 columns in 256 blocks of 10:
+  // 9.0 us, in 160 of 16 10.3; 11,264 gated in 512 of 11: 27.3, in 352 of 16 30.8), and so many that X counts less than W.
+  // X that is loaded singly counts more than a last round: 16 columns from four blocks a CU on (16 rows of 16,390 x 1,001 in blocks
+  // of 13: 51.7, of 16 48.9), and whole or half tiles chain by chain.
+  const int rows = ceil_div(m, 16 * MT), tiles = ceil_div(n, 16) * rows, each = ceil_div(tiles, 256);
+  const int spread = max(MT == 1 ? 4 : 8, min(16, ceil_div(n * rows, 256 * each)));
+  // Which kernel.  Numbers loaded singly: one tile of rows and one of W, in a K of more than a chain a wave, are asked for ahead like
+  // others (us, against chain by chain: 5 rows of 1,000 x K 1,001 7.5 / 9.5, of 300 x 5,631 31 / 40, of 2,048 x 515 6.0 / 8.4; 16 of
+  // 2,048 x 769 9.7 / 10.3, of 16,390 x 515 29.4 / 33.8).  Aligned: fewer chains than waves go chain by chain,
+  // and 64 rows of as many (512 x K 256 4.6 / 4.3, 4,096 x 256 9.0 / 8.8; gated, and of fewer rows, asked for ahead is the faster: 5 rows of
+  // 2,048 x 256 3.2 / 3.5).
   constexpr bool AHEAD = VEC || (MT == 1 && !GLU);
-  if constexpr (!VEC) {
-    if (brief || !AHEAD) {
-      const bool narrow = (long)ceil_div(n, 16) * rows < 256;      // blocks of 8 columns where blocks of 16 would leave CUs without one
-#define SINGLES(NR, SHORT)                                                                                       \
-  gemm_fma_singles_kernel<MT, NR, GLU, SHORT><<<dim3(ceil_div(n, NR), rows), 64 * FEW_WAVES, 0, stream>>>(       \
-      x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode)
-      if (brief) { if (narrow) SINGLES(8, true); else SINGLES(16, true); }
-      else if constexpr (!AHEAD) { if (narrow) SINGLES(8, false); else SINGLES(16, false); }
-#undef SINGLES
-      return;
-    }
+  const bool brief = k <= FEW_WAVES * FMA_PART;
+#define FEW(KERNEL, SHORT, COLUMNS)                                                                                         \
+  {                                                                                                                         \
+    const int columns = COLUMNS;                                                                                            \
+    const dim3 blocks(ceil_div(n, columns), rows);                                                                          \
+    if (columns <= 8) KERNEL<MT, 8, GLU, VEC, SHORT><<<blocks, 64 * FEW_WAVES, 0, stream>>>(FEW_ARGS, columns);             \
+    else KERNEL<MT, 16, GLU, VEC, SHORT><<<blocks, 64 * FEW_WAVES, 0, stream>>>(FEW_ARGS, columns);                         \
   }
-  if constexpr (AHEAD) {
-    // As many blocks as give every CU the same number of them, with at most 16 columns each (2,560 columns in 256 blocks of 10:
-    // 9.0 us, in 160 of 16 10.3; 11,264 gated in 512 of 11: 27.3, in 352 of 16 30.8), and so many that X counts less than W.
-    // X that is loaded singly counts more than a last round: 16 columns from four blocks a CU on (16 rows of 16,390 x 1,001 in blocks
-    // of 13: 51.7, of 16 48.9)
-    const int each = ceil_div(ceil_div(n, 16) * rows, 256);
-    const int columns = !VEC && each >= 4 ? 16 : max(MT == 1 ? 4 : 8, min(16, ceil_div(n * rows, 256 * each)));
-    const dim3 blocks(ceil_div(n, columns), rows);
-#define FEW(NR, SHORT)                                                                            \
-  gemm_fma_few_rows_kernel<MT, NR, GLU, VEC, SHORT><<<blocks, 64 * FEW_WAVES, 0, stream>>>(   \
-      x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode, columns)
-    if constexpr (VEC) {
-      if (brief) {
-        if (columns <= 8) FEW(8, true); else FEW(16, true);
-        return;
-      }
-    }
-    if (columns <= 8) FEW(8, false); else FEW(16, false);
+#define BY_CHAIN(SHORT, COLUMNS)                              \
+  {                                                           \
+    AXK_INSTANCE(INST_GEMM_FMA_BY_CHAIN, 16 * MT, GLU, VEC);  \
+    FEW(gemm_fma_by_chain_kernel, SHORT, COLUMNS)             \
+  }
+#define FEW_ARGS x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode
+  if constexpr (VEC) {
+    if (k <= (FEW_WAVES - 1) * FMA_PART || (brief && MT == 4 && !GLU)) BY_CHAIN(true, spread)
+    else if (brief) FEW(gemm_fma_few_rows_kernel, true, spread)
+    else FEW(gemm_fma_few_rows_kernel, false, spread)
+  } else {
+    if (brief) BY_CHAIN(true, tiles < 256 ? 8 : 16)
+    else if constexpr (AHEAD) FEW(gemm_fma_few_rows_kernel, false, each >= 4 ? 16 : spread)
+    else BY_CHAIN(false, tiles < 256 ? 8 : 16)
+  }
+#undef FEW_ARGS
+#undef BY_CHAIN
 #undef FEW
-  }
 }
 
 template <bool GLU, bool VEC>

@@ -33,6 +33,7 @@ enum {
   INST_GEMM_KEPT,            // tiles of 128 x 128 that keep the sums of K's segments; gated
   INST_ATTENTION_F32_PREFILL,    // float32 build, head_dim
   INST_ATTENTION_F32_DECODE,     // float32 build, head_dim, waves a block
+  INST_GEMM_FMA_BY_CHAIN,    // beside gemm_fma: rows of X a block, gated, numbers loaded four at a time
   INST_KINDS
 };
 

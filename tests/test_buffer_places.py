@@ -52,8 +52,8 @@ def test_chains_read_their_rows_and_nothing_behind_the_last(buffer_rows, M, K, g
             row = np.minimum(np.arange(rows_a_block), M - 1 - m0)[:, None]
             in_chain = np.arange(0, 32, 4)[None, :]
             for chain in range(-(-K // 32) + 16):               # a round's chains behind the last one too
-                k = min(32 * chain, K)
-                left = total - k * size
+                k = 32 * chain
+                left = total - k * size if k < K else 0
                 place = (row * stride + in_chain) * size
                 reads = place < left
                 assert left >= 0 and (place + load <= left)[reads].all()

@@ -103,6 +103,11 @@ def test_columns_a_block_and_rounds_of_chains(N, K):
         assert torch.equal(out, act), m
 
 
+@pytest.mark.parametrize("N,K", [(1030, 224), (2570, 64), (4100, 128), (300, 256), (5640, 33), (16390, 8)])
+def test_columns_a_block_of_few_chains(N, K):
+    test_columns_a_block_and_rounds_of_chains(N, K)
+
+
 @pytest.mark.parametrize("K", [4, 28, 32, 60, 64, 96, 124, 128, 132, 160, 188, 192, 224, 228, 1056])
 def test_tiles_at_every_end_of_k(K):
     """Whole and broken last steps of K behind fewer and more stages than LDS holds, rows and columns past the end, and rows of X

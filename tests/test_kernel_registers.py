@@ -38,8 +38,8 @@ def test_32_bit_products_of_few_rows_spill_nothing(device_code, dtype):
     seen = set()
     for note in re.findall(r"- \.agpr_count:.*?\.wavefront_size:", device_code("gemm.hip", dtype), re.S):
         field = {k: v for k, v in re.findall(r"\.(\w+):\s+(\S+)", note)}
-        kernel = re.search(r"gemm_fma_(few_rows|singles)_kernel", field["symbol"])
+        kernel = re.search(r"gemm_fma_(few_rows|by_chain)_kernel", field["symbol"])
         if kernel:
             seen.add(kernel[1])
             assert int(field["vgpr_spill_count"]) == 0 and int(field["private_segment_fixed_size"]) == 0, field
-    assert seen == {"few_rows", "singles"}
+    assert seen == {"few_rows", "by_chain"}
