@@ -46,7 +46,7 @@ __device__ inline void fma_store(float v, float up, bool glu, const void* bias, 
   else ((float*)out)[at] = v;
 }
 
-// Many rows (in the float32 build, those that gemm_fma_flow_kernel does not take): 64 x 64 outputs a block of 4 waves, each 2 x 2 tiles of 16 x 16 (gated: half of a wave's
+// Many rows (in the float32 build those that launch_fma_tiles does not give to gemm_fma_flow_kernel): 64 x 64 outputs a block of 4 waves, each 2 x 2 tiles of 16 x 16 (gated: half of a wave's
 // columns are gate rows of W, half the up rows of the same outputs).  K is walked a chain at a time through
 // two stages of LDS; the stage's operands are read first, then the next stage is written and the one
 // after it asked for, all beside this stage's products.  A lane of a product holds k = 4 i + q of
@@ -473,6 +473,7 @@ gemm_fma_by_chain_kernel(const elem_t* __restrict__ x, int x_stride, const elem_
 // number (128 LDS instructions a block and step) 127 and 409 for the last two, three stages (three blocks a CU) 128 and 412.
 #define FLOW_STAGES 4
 #define FLOW_STAGE (2 * TILE_M * FMA_PART * 4)
+#define FLOW_LEAST_K 192      // (launch_fma_tiles)
 typedef const __attribute__((address_space(1))) void* fma_global_t;
 typedef __attribute__((address_space(3))) void* fma_lds_t;
 typedef __attribute__((ext_vector_type(2))) float f32x2;
@@ -544,14 +545,12 @@ gemm_fma_flow_kernel(const float* __restrict__ x, int x_stride, const float* __r
     for (int j = 0; j < R; ++j) sum[i][j] = acc[1][i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
   const int n_steps = (K + FMA_PART - 1) / FMA_PART;
+  static_assert(FLOW_LEAST_K > FLOW_STAGES * FMA_PART, "as many steps as stages");
 #pragma unroll
   for (int t = 0; t < FLOW_STAGES; ++t)
-    if (t < n_steps) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) ask(t, j);
-    }
-  if (n_steps >= FLOW_STAGES) wait_vmcnt<4 * (FLOW_STAGES - 1)>();
-  else wait_vmcnt<0>();
+    for (int j = 0; j < 4; ++j) ask(t, j);
+  wait_vmcnt<4 * (FLOW_STAGES - 1)>();
   __builtin_amdgcn_s_barrier();            // stage 0 is in LDS for every wave
 #pragma unroll
   for (int p = 0; p < 16; ++p) read(FmaNumber<0>(), 0u, p);
@@ -694,10 +693,17 @@ template <bool GLU, bool VEC>
 static void launch_fma_tiles(dim3 tiles, const elem_t* x, int x_stride, const elem_t* w, const void* bias, int bias_is_f32, void* out,
                              int out_stride, int m, int n, int k, int mode, hipStream_t stream) {
 #if !AXON_BF16
-  if constexpr (VEC) {                       // FLOW_STAGES of 16 KB are what a launch gets unasked
-    static_assert(FLOW_STAGES * FLOW_STAGE <= 64 * 1024, "more LDS than a launch gets unasked");
-    gemm_fma_flow_kernel<GLU><<<tiles, 256, FLOW_STAGES * FLOW_STAGE, stream>>>(x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode);
-    return;
+  // Short K: the stages that are filled before the first product count more than what they save, and where there are more
+  // than two blocks a CU these cover each other's waits.  us, through registers / by direct loads: up to 512 blocks, 400 rows of 1,000
+  // columns of K 64 4.8 / 5.4, 128 6.1 / 6.4, 192 7.3 / 7.3, 256 8.5 / 8.1; more, 777 rows of 4,096 of K 96 12.6 / 15.9, 256 27.5 / 29.2,
+  // 512 47.9 / 48.4, 640 57.9 / 57.4; of 32,000 of K 256 136 / 146, 640 1.02 times, 1,024 as long.
+  if constexpr (VEC) {
+    if (k >= ((long)tiles.x * tiles.y <= 512 ? FLOW_LEAST_K : 640)) {
+      static_assert(FLOW_STAGES * FLOW_STAGE <= 64 * 1024, "more LDS than a launch gets unasked");
+      AXK_INSTANCE(INST_GEMM_FMA_FLOW, GLU);
+      gemm_fma_flow_kernel<GLU><<<tiles, 256, FLOW_STAGES * FLOW_STAGE, stream>>>(x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode);
+      return;
+    }
   }
 #endif
   gemm_fma_kernel<GLU, VEC><<<tiles, 256, 0, stream>>>(x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode);

@@ -127,3 +127,18 @@ def test_tiles_at_every_end_of_k(K):
     k.gemm(x[:M, :K], w, got, None, MODE_SWIGLU)
     k.swiglu(want[:, :2 * half].contiguous(), act)
     assert torch.equal(got, act)
+
+
+@pytest.mark.parametrize("N,K,flows", [(150, 128, False), (150, 188, False), (150, 192, True), (150, 193, False), (150, 196, True), (150, 320, True),
+                                       (8150, 260, True), (8200, 260, False), (8200, 636, False), (8200, 640, True)])
+def test_short_and_long_k_have_their_kernels(N, K, flows):
+    """Up to 512 blocks of 64 rows and columns direct loads pay from a K of 192 on, with more of them from 640: the same bits on
+    both sides of the lines."""
+    k = kernels("float32")
+    g = torch.Generator(device="cuda").manual_seed(N + K)
+    x, w = torch.randn(220, K, generator=g, device="cuda"), torch.randn(N, K, generator=g, device="cuda")
+    out = torch.full((220, N), float("nan"), device="cuda")
+    k.reset_instances()
+    k.gemm(x, w, out, None, MODE_STORE_F32)
+    assert ("gemm_fma_flow<0>" in k.instances(launched=True)) == flows and "gemm_fma<128,0>" in k.instances(launched=True)
+    assert torch.equal(out, _by_chains(k, x, w))

@@ -331,6 +331,8 @@ CASES = [
     *[(d, [f"gemm_fma<{rows},{int(mode == MODE_SWIGLU)}>"], check_gemm, (d, M, N, K, mode)) for d in (F32, BF)
       for rows, M, N, K, mode in ((32, 20, 259, 290, MODE_STORE_F32), (128, 200, 259, 130, MODE_STORE_F32), (128, 40, 16390, 36, MODE_STORE_F32),
                                   (32, 31, 48, 100, MODE_SWIGLU), (128, 129, 48, 100, MODE_SWIGLU), (64, 128, 96, 290, MODE_SWIGLU))],
+    (F32, ["gemm_fma_flow<0>"], check_gemm, (F32, 200, 259, 260, MODE_STORE_F32)),
+    (F32, ["gemm_fma_flow<1>"], check_gemm, (F32, 129, 48, 292, MODE_SWIGLU)),
     # chain by chain: fewer chains than waves, and numbers loaded singly but for one tile of rows and W
     *[(d, [f"gemm_fma_by_chain<{rows},{int(mode == MODE_SWIGLU)},{int(K % 4 == 0)}>"], check_gemm, (d, M, N, K, mode)) for d in (F32, BF)
       for rows, M in ((16, 5), (32, 20), (64, 70)) for N, K, mode in ((259, 100, MODE_STORE_F32), (259, 70, MODE_STORE_F32), (48, 224, MODE_SWIGLU),
