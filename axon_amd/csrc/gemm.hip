@@ -192,8 +192,17 @@ __device__ __forceinline__ FmaRows fma_rows(const elem_t* matrix, int m, int M, 
 }
 // Four k of the row that begins `at` elements behind the first, k = k0 + in_chain .. + 3 (in_chain: this lane's place in
 // the chain that begins at k0).  Aligned operands read on into the next row behind K; others take the row's last number.
+// (A row's place: rows of numbers that are loaded singly may be any distance apart.)
 template <bool VEC>
-__device__ __forceinline__ fma_quad fma_ask(const FmaRows& rows, unsigned at, int k0, int in_chain, int K) {
+struct FmaPlace {
+  typedef unsigned type;
+};
+template <>
+struct FmaPlace<false> {
+  typedef size_t type;
+};
+template <bool VEC>
+__device__ __forceinline__ fma_quad fma_ask(const FmaRows& rows, typename FmaPlace<VEC>::type at, int k0, int in_chain, int K) {
   if (VEC) {
     const int off = (int)((at + in_chain) * sizeof(elem_t));
 #if AXON_BF16
@@ -204,7 +213,7 @@ __device__ __forceinline__ fma_quad fma_ask(const FmaRows& rows, unsigned at, in
   }
   union { fma_quad q; elem_t e[4]; } c;
 #pragma unroll
-  for (int e = 0; e < 4; ++e) c.e[e] = rows.base[(size_t)at + min(k0 + in_chain + e, K - 1)];
+  for (int e = 0; e < 4; ++e) c.e[e] = rows.base[at + min(k0 + in_chain + e, K - 1)];
   return c.q;
 }
 // What lies behind K of four k from `k` on becomes zeros.
@@ -241,10 +250,11 @@ gemm_fma_few_rows_kernel(const elem_t* __restrict__ x, int x_stride, const elem_
 #pragma unroll
   for (int t = 0; t < NT; ++t) w_rows[t] = fma_rows(w + (size_t)t * N * K, n0, N, K, K);
   const FmaRows x_rows = fma_rows(x, m0, M, x_stride, K);
-  const unsigned w_at = (unsigned)min(min(r16, columns - 1), N - 1 - n0) * (unsigned)K;
-  unsigned x_at[MT];
+  typedef typename FmaPlace<VEC>::type place_t;
+  const place_t w_at = (place_t)min(min(r16, columns - 1), N - 1 - n0) * (place_t)K;
+  place_t x_at[MT];
 #pragma unroll
-  for (int i = 0; i < MT; ++i) x_at[i] = (unsigned)min(16 * i + r16, M - 1 - m0) * (unsigned)x_stride;
+  for (int i = 0; i < MT; ++i) x_at[i] = (place_t)min(16 * i + r16, M - 1 - m0) * (place_t)x_stride;
   const int n_parts = (K + FMA_PART - 1) / FMA_PART;
   constexpr int MINE = (ALL + 64 * FEW_WAVES - 1) / (64 * FEW_WAVES);
   float sum[MINE];

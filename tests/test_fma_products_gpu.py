@@ -142,3 +142,16 @@ def test_short_and_long_k_have_their_kernels(N, K, flows):
     k.gemm(x, w, out, None, MODE_STORE_F32)
     assert ("gemm_fma_flow<0>" in k.instances(launched=True)) == flows and "gemm_fma<128,0>" in k.instances(launched=True)
     assert torch.equal(out, _by_chains(k, x, w))
+
+
+def test_rows_far_apart():
+    """Sixteen rows of X that lie 2^32 numbers from the first to the last."""
+    k, K, stride = kernels("bfloat16"), 301, 2 ** 32 // 15 + 1
+    g = torch.Generator(device="cuda").manual_seed(1)
+    x, w = torch.randn(16, K, generator=g, device="cuda").bfloat16(), torch.randn(40, K, generator=g, device="cuda").bfloat16()
+    far = torch.empty(15 * stride + K, dtype=torch.bfloat16, device="cuda").as_strided((16, K), (stride, 1))
+    far.copy_(x)
+    got, want = (torch.full((16, 40), float("nan"), device="cuda") for _ in range(2))
+    k.gemm(far, w, got, None, MODE_STORE_F32)
+    k.gemm(x, w, want, None, MODE_STORE_F32)
+    assert torch.equal(got, want)
