@@ -249,6 +249,8 @@ int axk_clamped_glu(const void* gate_up, void* out, int n_tokens, int n_ffn, flo
 // [out rows], or null): the sums of out row r are multiplied by row_scale[r] before bias and epilogue (a factor on
 // the row of X).
 int axk_grouped_gemm_uses_mfma(int k, int x_is_f32, long x_row_stride, long x_group_stride);
+// Whether the blocks of a list of 64-row tiles are numbered tile by tile, not column by column; it changes no bit.
+int axk_grouped_gemm_by_tile(int n, int k, int glu);
 int axk_grouped_gemm(const void* x, int x_is_f32, long x_row_stride, long x_group_stride, const int32_t* x_rows,
                      const void* w, const void* bias, int bias_is_f32, void* out, int out_is_f32, long out_row_stride,
                      long out_group_stride, const int32_t* out_rows, const float* gate, long gate_row_stride,

@@ -36,6 +36,7 @@ struct GroupedArgs {
   const int32_t* tiles; const int32_t* n_tiles;
   int M, N, K, G;
   bool vec_out;                         // four neighbouring outputs are one aligned store
+  bool by_tile;                         // a list of 64-row tiles is gone through tile by tile (axk_grouped_gemm_by_tile)
 };
 
 #define GG_ROWS 16
@@ -256,16 +257,13 @@ __global__ void __launch_bounds__(256, 2) grouped_gemm_tile_kernel(GroupedArgs a
   extern __shared__ __align__(256) unsigned char stages[];        // [2]: X [64][64], W [WROWS][64]
   constexpr int COLS = GLU ? WROWS / 2 : WROWS;
   // Blocks go to the eight XCDs in turn: each XCD gets a run of neighbours of the list [group, columns, rows]
-  // (routed and gated: [columns, tile]), so that the tiles of a group that read the same rows of W do so through one L2.  Routed
-  // and not gated, the list is [tile, columns]: an XCD has a group's tiles with all of their columns, so its rows of X and of the
-  // output stay there too (4 of 32 experts [2,048, 704] of 2,048 tokens 66.8 / 56.9 us, 8 of 64 [2,048, 256] 65.9 / 56.6; gated, whose W is
-  // twice as large, 78 / 80, 2 of 16 [2,816, 4,096] 171 / 202).
-  constexpr bool TILE_FIRST = !GLU;
+  // (routed: [columns, tile]), so that the tiles of a group that read the same rows of W do so through one L2; or, by_tile, of the list
+  // [tile, columns]: an XCD has a tile with all of its columns, so that its rows of X and of the output stay there.
   const int col_tiles = (a.N + COLS - 1) / COLS, row_tiles = a.tiles ? *a.n_tiles : (a.M + GT_ROWS - 1) / GT_ROWS;
   const long total = (long)row_tiles * col_tiles * (a.tiles ? 1 : a.G), share = (total + 7) / 8;
   const long item = (long)(blockIdx.x % 8) * share + blockIdx.x / 8;
   if ((long)(blockIdx.x / 8) >= share || item >= total) return;
-  const bool by_tile = TILE_FIRST && a.tiles;
+  const bool by_tile = !GLU && a.by_tile;
   const int row_tile = (int)(by_tile ? item / col_tiles : item % row_tiles);
   const int n0 = (int)(by_tile ? item % col_tiles : item / row_tiles % col_tiles) * COLS;
   int g, first, count;
@@ -410,6 +408,16 @@ extern "C" int axk_grouped_gemm_uses_mfma(int k, int x_is_f32, long x_row_stride
 #endif
 }
 
+// Whether a list of 64-row tiles is gone through tile by tile: not gated, where a group's W is no more than three of an XCD's L2 of 4 MB.
+// A tile that meets all of a larger W reads it from further away, again for each tile.  us, by columns / by tile: 4 of 32 experts
+// [2,048, 704] (2.9 MB) of 2,048 tokens 63.8 / 57.3, of 4,096 115 / 108, 8 of 64 [2,048, 256] (1 MB) 73.5 / 66.6, 2 of 8 [2,048, 1,408]
+// (5.8 MB) 51.0 / 42.0, 6 of 64 166 / 164, 4 of 16 [1,024, 1,024] 43.5 / 34.3; 2 of 16 [4,096, 1,408] (11.5 MB) 106 / 104, [4,096, 2,816]
+// (23 MB) 188 / 207, of 4,096 tokens 325 / 388, of 512 91 / 86, 2 of 8 [4,096, 14,336] (117 MB) 797 / 1,090.  Gated, whose W is twice as large for its columns:
+// 4 of 32 [1,408, 2,048] 78 / 80, 2 of 16 [2,816, 4,096] 171 / 202.
+extern "C" int axk_grouped_gemm_by_tile(int n, int k, int glu) {
+  return !glu && (size_t)n * k * sizeof(elem_t) <= (12u << 20);
+}
+
 extern "C" int axk_grouped_gemm(const void* x, int x_is_f32, long x_row_stride, long x_group_stride, const int32_t* x_rows,
                                 const void* w, const void* bias, int bias_is_f32, void* out, int out_is_f32,
                                 long out_row_stride, long out_group_stride, const int32_t* out_rows, const float* gate,
@@ -430,7 +438,8 @@ extern "C" int axk_grouped_gemm(const void* x, int x_is_f32, long x_row_stride, 
                 out_row_stride, out_group_stride, out_rows, gate, gate_row_stride, gate_per_group, row_scale, glu, glu_limit, glu_alpha,
                 glu_shift, tiles, n_tiles,
                 m, n, k, groups,
-                out_row_stride % 4 == 0 && out_group_stride % 4 == 0 && (uintptr_t)out % (out_is_f32 ? 16 : 8) == 0};
+                out_row_stride % 4 == 0 && out_group_stride % 4 == 0 && (uintptr_t)out % (out_is_f32 ? 16 : 8) == 0,
+                tiles != nullptr && axk_grouped_gemm_by_tile(n, k, glu)};
   dim3 grid(row_tiles, ceil_div(n, GG_COLS), tiles ? 1 : groups);
   hipStream_t s = (hipStream_t)stream;
 #if AXON_BF16

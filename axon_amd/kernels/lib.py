@@ -92,6 +92,7 @@ _SIGNATURES = {
     "axk_activation": [c_void_p, c_long, c_int, c_void_p],
     "axk_clamped_glu": [c_void_p, c_void_p, c_int, c_int, c_float, c_float, c_void_p],
     "axk_grouped_gemm_uses_mfma": [c_int, c_int, c_long, c_long],
+    "axk_grouped_gemm_by_tile": [c_int, c_int, c_int],
     "axk_grouped_gemm": [c_void_p, c_int, c_long, c_long, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int, c_long, c_long,
                          c_void_p, c_void_p, c_long, c_int, c_void_p, c_int, c_float, c_float, c_float, c_void_p, c_void_p, c_int, c_int,
                          c_int, c_int, c_int, c_int, c_void_p],

@@ -58,3 +58,26 @@ def test_lists_of_64_and_of_16_rows_agree(T, E, top):
                        routed=(tiles, n, most, tokens, pairs, rows), rows=P, row_scale=scale)
         got.append(out)
     assert torch.equal(got[0], got[1]) and not bool(got[0].isnan().any())
+
+
+@pytest.mark.parametrize("N,K,by_tile", [(136, 96, True), (2048, 704, True), (4096, 1408, True), (4100, 1568, False), (4096, 2816, False)])
+def test_lists_in_both_orders(N, K, by_tile):
+    """Groups whose W fits an XCD's cache, and larger ones: tiles of 64 rows, in the order that is the faster, have the bits of tiles
+    of 16."""
+    k, T, E, top = kernels("bfloat16"), 190, 5, 2
+    assert bool(k.lib.axk_grouped_gemm_by_tile(N, K, 0)) == by_tile and not k.lib.axk_grouped_gemm_by_tile(N, K, 1)
+    g = torch.Generator(device="cuda").manual_seed(N + K)
+    P = T * top
+    x = torch.randn(P, K, generator=g, device="cuda").bfloat16()
+    w = torch.randn(E, N, K, generator=g, device="cuda").mul_(0.2).bfloat16()
+    odds = torch.tensor([9.0, 4.0, 2.0, 0.0, 1.0], device="cuda").expand(T, E)            # uneven, one expert without a row
+    chosen = torch.multinomial(odds, top, generator=g).int().contiguous()
+    got = []
+    for rows in (16, 64):
+        most = k.route_max_tiles(P, E, rows)
+        pairs, tokens, tiles, n = (torch.zeros(s, dtype=torch.int32, device="cuda") for s in (P, P, 3 * most, 1))
+        k.route_sort(chosen, E, pairs, tokens, tiles, n, tile_rows=rows)
+        out = torch.full((P, N), float("nan"), device="cuda")
+        k.grouped_gemm(x, w, out, x_group_stride=0, out_group_stride=0, routed=(tiles, n, most, pairs, pairs, rows), rows=P)
+        got.append(out)
+    assert torch.equal(got[0], got[1]) and not bool(got[0].isnan().any())
