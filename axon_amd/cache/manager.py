@@ -244,29 +244,35 @@ class CacheManager:
     def sync_tables(self) -> None:
         """Upload the rows that changed since the last call, in stream order before the kernels
         that read them and without waiting for the device (through pinned memory, which torch's allocator gives out again when
-        the copies have run): a copy a row, or, of many rows, one copy and a scatter per group."""
+        the copies have run): a copy a row, or, of many rows, one copy for all groups and a scatter for each."""
         if not self._dirty:
             return
         slots = sorted(self._dirty)
-        n, places, on_device_places = len(slots), torch.tensor(slots), None
+        n, n_groups, width = len(slots), len(self.groups), self.max_pages_per_seq
+        places, on_device = torch.tensor(slots), self.device is not None
+        scatter = on_device and n * n_groups > 4        # four copies take the host as long as a scatter and what it reads
+        # every group's rows in one piece of pinned memory (a new one takes the host 100 us) and, to be scattered, their places behind
+        # them (64 bits wide)
+        n_rows = n_groups * n
+        rows_staged = n_rows - (-2 * n // width) if scatter else n_rows
+        staged = torch.zeros((rows_staged, width), dtype=torch.int32, pin_memory=on_device)
+        at = staged.data_ptr()
         for gi, g in enumerate(self.groups):
-            on_device = g.block_table is not None
-            rows = torch.zeros((n, self.max_pages_per_seq), dtype=torch.int32, pin_memory=on_device)
-            at, row_bytes = rows.data_ptr(), 4 * self.max_pages_per_seq
-            for i, slot in enumerate(slots):
-                got = self.lib.axh_cache_row(self._h, gi, slot, c_void_p(at + i * row_bytes), self.max_pages_per_seq)
-                if got < 0:
+            for slot in slots:
+                if self.lib.axh_cache_row(self._h, gi, slot, c_void_p(at), width) < 0:
                     raise CacheError(f"no block table row for group {gi}, slot {slot}")
-            g.host_table.index_copy_(0, places, rows)
-            if not on_device:
-                continue
-            if n <= 4:              # four copies take the host as long as the scatter and what it reads
+                at += 4 * width
+            g.host_table.index_copy_(0, places, staged if rows_staged == n else staged[gi * n:gi * n + n])
+        if scatter:
+            staged[n_rows:].view(-1)[:2 * n].view(torch.int64).copy_(places)
+            staged = staged.to(self.device, non_blocking=True)
+            places = staged[n_rows:].view(-1)[:2 * n].view(torch.int64)
+            for gi, g in enumerate(self.groups):
+                g.block_table.index_copy_(0, places, staged[gi * n:gi * n + n])
+        elif on_device:
+            for gi, g in enumerate(self.groups):
                 for i, slot in enumerate(slots):
-                    g.block_table[slot].copy_(rows[i], non_blocking=True)
-            else:
-                if on_device_places is None:
-                    on_device_places = places.pin_memory().to(self.device, non_blocking=True)
-                g.block_table.index_copy_(0, on_device_places, rows.to(self.device, non_blocking=True))
+                    g.block_table[slot].copy_(staged[gi * n + i], non_blocking=True)
         self._dirty.clear()
 
     # ------------------------------------------------------------------ accounting

@@ -4,7 +4,9 @@ import pytest
 import torch
 
 import axon_amd
+from axon_amd.cache.manager import CacheManager, GroupPlan
 from axon_amd.engine import StepEntry
+from axon_amd.parts.base import CacheSpec
 
 pytestmark = pytest.mark.gpu
 
@@ -33,3 +35,25 @@ def test_queued_steps_give_what_waited_ones_give(dtype, requests):
     want, got = run(True), run(False)
     for i, (a, b) in enumerate(zip(want, got)):
         assert torch.equal(a, b), i
+
+
+@pytest.mark.parametrize("groups", [1, 3])
+@pytest.mark.parametrize("changed", [1, 2, 4, 5, 16])
+@pytest.mark.parametrize("length", [64, 4000])              # rows shorter and longer than the places of sixteen
+def test_changed_rows_of_all_groups_travel_together(groups, changed, length):
+    """However many groups and rows: what the device holds is what the host holds, from one piece of pinned memory."""
+    plans = [GroupPlan(CacheSpec(entries=2, heads=1, head_dim=8, window=0 if i == 0 else 48 + 16 * i), 1, 16, 6000) for i in range(groups)]
+    cache = CacheManager(plans, [], 20, length, device="cuda:0", dtype=torch.float32)
+    slots = [cache.open() for _ in range(20)]
+    cache.reserve_many([(s, 16) for s in slots])
+    cache.sync_tables()
+    for s in slots[3:3 + changed]:
+        cache.reserve(s, length)
+    asked = torch.cuda.host_memory_stats()["active_requests.allocated"]
+    cache.sync_tables()
+    assert torch.cuda.host_memory_stats()["active_requests.allocated"] - asked == 1
+    for gi, g in enumerate(cache.groups):
+        assert torch.equal(g.block_table.cpu(), g.host_table)
+        for s in slots:
+            row = cache.row(gi, s)
+            assert g.host_table[s, :len(row)].tolist() == row and not bool(g.host_table[s, len(row):].any())
