@@ -251,24 +251,25 @@ class CacheManager:
         n, n_groups, width = len(slots), len(self.groups), self.max_pages_per_seq
         places, on_device = torch.tensor(slots), self.device is not None
         scatter = on_device and n * n_groups > 4        # four copies take the host as long as a scatter and what it reads
-        # every group's rows in one piece of pinned memory (a new one takes the host 100 us) and, to be scattered, their places behind
-        # them (64 bits wide)
-        n_rows = n_groups * n
-        rows_staged = n_rows - (-2 * n // width) if scatter else n_rows
-        staged = torch.zeros((rows_staged, width), dtype=torch.int32, pin_memory=on_device)
-        at = staged.data_ptr()
+        # one piece of pinned memory (a new one takes the host 100 us): to be scattered, the rows' places (64 bits wide), then the
+        # rows of every group
+        head = -(-2 * n // width) if scatter else 0
+        staged = torch.zeros((head + n_groups * n, width), dtype=torch.int32, pin_memory=on_device)
+        at = staged.data_ptr() + 4 * head * width
         for gi, g in enumerate(self.groups):
             for slot in slots:
                 if self.lib.axh_cache_row(self._h, gi, slot, c_void_p(at), width) < 0:
                     raise CacheError(f"no block table row for group {gi}, slot {slot}")
                 at += 4 * width
-            g.host_table.index_copy_(0, places, staged if rows_staged == n else staged[gi * n:gi * n + n])
+            first = head + gi * n
+            g.host_table.index_copy_(0, places, staged if n_groups == 1 and not head else staged[first:first + n])
         if scatter:
-            staged[n_rows:].view(-1)[:2 * n].view(torch.int64).copy_(places)
+            staged[:head].view(-1)[:2 * n].view(torch.int64).copy_(places)
             staged = staged.to(self.device, non_blocking=True)
-            places = staged[n_rows:].view(-1)[:2 * n].view(torch.int64)
+            places = staged[:head].view(-1)[:2 * n].view(torch.int64)
             for gi, g in enumerate(self.groups):
-                g.block_table.index_copy_(0, places, staged[gi * n:gi * n + n])
+                first = head + gi * n
+                g.block_table.index_copy_(0, places, staged[first:first + n])
         elif on_device:
             for gi, g in enumerate(self.groups):
                 for i, slot in enumerate(slots):

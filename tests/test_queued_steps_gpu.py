@@ -39,7 +39,7 @@ def test_queued_steps_give_what_waited_ones_give(dtype, requests):
 
 @pytest.mark.parametrize("groups", [1, 3])
 @pytest.mark.parametrize("changed", [1, 2, 4, 5, 16])
-@pytest.mark.parametrize("length", [64, 4000])              # rows shorter and longer than the places of sixteen
+@pytest.mark.parametrize("length", [64, 72, 4000])          # rows shorter and longer than the places of sixteen, even and odd
 def test_changed_rows_of_all_groups_travel_together(groups, changed, length):
     """However many groups and rows: what the device holds is what the host holds, from one piece of pinned memory."""
     plans = [GroupPlan(CacheSpec(entries=2, heads=1, head_dim=8, window=0 if i == 0 else 48 + 16 * i), 1, 16, 6000) for i in range(groups)]
