@@ -7,6 +7,7 @@ import axon_amd
 from axon_amd.cache.manager import CacheManager, GroupPlan
 from axon_amd.engine import StepEntry
 from axon_amd.parts.base import CacheSpec
+from axon_amd.upload import upload
 
 pytestmark = pytest.mark.gpu
 
@@ -57,3 +58,19 @@ def test_changed_rows_of_all_groups_travel_together(groups, changed, length):
         for s in slots:
             row = cache.row(gi, s)
             assert g.host_table[s, :len(row)].tolist() == row and not bool(g.host_table[s, len(row):].any())
+
+
+def test_uploads_are_not_captured():
+    """The pinned memory of an upload serves the next one when its copy has run: a graph must not come to read it."""
+    kept = upload([1, 2, 3], "cuda:0")                       # a piece that a captured upload would find at hand
+    torch.cuda.synchronize()
+    a = torch.zeros(4, device="cuda:0")
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        a += 1
+        with pytest.raises(RuntimeError, match="captured"):
+            upload([4, 5, 6], "cuda:0")
+        a += 1
+    for i in range(3):
+        graph.replay()
+        assert a.tolist() == [2.0 * (i + 1)] * 4 and upload([7, i], "cuda:0").tolist() == [7, i] and kept.tolist() == [1, 2, 3]
