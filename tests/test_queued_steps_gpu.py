@@ -16,26 +16,52 @@ CONFIG = dict(architectures=["Qwen2ForCausalLM"], model_type="qwen2", num_hidden
               rope_theta=10000.0, rms_norm_eps=1e-6, tie_word_embeddings=False)
 
 
+def _busy():
+    """Half a second of the device's time on the stream (its last product's event)."""
+    a = torch.ones(8192, 8192, device="cuda")
+    for _ in range(60):                                     # 1.1 TFLOP each, and no more than 157 TFLOP/s
+        torch.mm(a, a)
+    event = torch.cuda.Event()
+    event.record()
+    return event
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("requests", [1, 4, 5, 9])          # up to four changed rows of a table are copied singly
 def test_queued_steps_give_what_waited_ones_give(dtype, requests):
     engine = axon_amd.load(CONFIG, dtype=dtype, random_seed=1, init_std=0.05, page_size=16, num_pages=400, max_seqs=12,
                            max_seq_len=512).engine
     g = torch.Generator().manual_seed(requests)
-    steps = [[torch.randint(0, 512, (int(torch.randint(3, 60, (1,), generator=g)),), generator=g).tolist() for _ in range(requests)]
-             for _ in range(12)]
+
+    def tokens(n):
+        return torch.randint(0, 512, (n,), generator=g).tolist()
+    steps = [[tokens(int(torch.randint(3, 60, (1,), generator=g))) for _ in range(requests)] for _ in range(12)]
+    whole = [tokens(16 * (1 + i % 3)) for i in range(requests)]        # whole pages: the next token of each takes a new one
+    further = [[tokens(1) for _ in range(requests)] for _ in range(3)]
 
     def run(wait):
         rows = []
-        for i, prompts in enumerate(steps):
-            ids = [(wait, i, j) for j in range(requests)]
-            rows.append(engine.step([StepEntry(r, p, [0, len(p) - 1]) for r, p in zip(ids, prompts)], end=ids))
+
+        def step(entries, end=()):
+            rows.append(engine.step(entries, end=end).clone())
             if wait:
                 torch.cuda.synchronize()
+        for i, prompts in enumerate(steps):
+            ids = [(wait, i, j) for j in range(requests)]
+            step([StepEntry(r, p, [0, len(p) - 1]) for r, p in zip(ids, prompts)], ids)
+        ids = [(wait, "on", j) for j in range(requests)]
+        step([StepEntry(r, p, [len(p) - 1]) for r, p in zip(ids, whole)])
+        for i, new in enumerate(further):
+            step([StepEntry(r, t, [0]) for r, t in zip(ids, new)], ids if i == len(further) - 1 else ())
         return rows
-    want, got = run(True), run(False)
+    run(True)                                               # whatever happens once
+    want = run(True)
+    behind = _busy()
+    got = run(False)
+    assert not behind.query(), "the device was to be busy with other work until the last step was queued"
     for i, (a, b) in enumerate(zip(want, got)):
         assert torch.equal(a, b), i
+    assert len(want) == 16
 
 
 @pytest.mark.parametrize("groups", [1, 3])
