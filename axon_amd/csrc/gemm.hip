@@ -167,10 +167,10 @@ gemm_fma_kernel(const elem_t* __restrict__ x, int x_stride, const elem_t* __rest
 // 27 us, 22 so).  One chain of a wave at a time, or two where both operands are one tile: more of them (4 and 8)
 // only wait for each other (the same 22 us against 20; a gated 5,632 x 2,048 of 5 rows 26 against 23 us).
 // 5 rows, us, before (X asked for chain by chain between branches, a round's loads behind the last one's sums) / now:
-// 2,560 x K 2,048 15.3 / 8.5, 2,048 x 2,048 11.7 / 8.9, gated 5,632 x 2,048 33.1 / 21.0 (4.4 TB/s), 2,048 x 5,632 28.9 / 17.5,
-// 32,000 x 2,048 66 / 52 (5.0 TB/s); 32 rows of 2,560 x 2,048 23.3 / 13.5, of 32,000 x 2,048 102 / 90; 64 rows of
-// 2,048 x 5,632 65 / 56.
+// 2,560 x K 2,048 15.7 / 8.2, 2,048 x 2,048 11.7 / 8.9, gated 5,632 x 2,048 33.6 / 21.3 (4.3 TB/s), 2,048 x 5,632 29.2 / 17.2,
+// 32,000 x 2,048 69 / 53 (4.9 TB/s); 32 rows of 2,560 x 2,048 23.7 / 14.3; 64 rows of 2,048 x 5,632 65 / 57.
 #define FEW_WAVES 8
+#define FEW_BRIEF (AXON_BF16 ? 4 : 7)      // so many chains, of all that the waves could take, go chain by chain (launch_fma_few)
 #if AXON_BF16
 typedef __attribute__((ext_vector_type(2))) unsigned fma_quad;      // four numbers as they lie in memory
 #else
@@ -380,8 +380,8 @@ gemm_fma_few_rows_kernel(const elem_t* __restrict__ x, int x_stride, const elem_
 //    addresses of their own, and all of X ahead does not fit the registers.  us, all ahead / so: 20 rows of 1,000 x K 1,001
 //    14.0 / 13.1, 40 of 2,048 x 2,047 40.4 / 37.0, gated 5,632 x 2,049 5 rows 59.3 / 58.6, 32 91.5 / 86.5, 64 140 / 122; 256 x 127 of
 //    5 rows 3.2 / 2.7, of 64 6.7 / 4.4.
-//  * Fewer chains than waves: 64 rows of 64 x K 96 4.0 / 3.0 us, of 256 x 128 4.6 / 3.4, of 4,096 x 192 8.2 / 7.2, gated 512 x 128
-//    5.9 / 4.2; 5 rows 2.4 / 2.2, 2.5 / 2.4, 3.6 / 3.6 and 3.3 / 2.8.
+//  * Fewer chains than waves: 64 rows of 64 x K 96 4.5 / 3.3 us, of 256 x 128 4.6 / 3.4, of 4,096 x 192 5.7 / 5.0, gated 512 x 128
+//    5.9 / 4.2; 5 rows 2.5 / 2.3, 2.5 / 2.4, 3.4 / 3.3 and 3.4 / 2.7.
 template <int MT, int NR, bool GLU, bool VEC, bool SHORT>
 __global__ void __launch_bounds__(64 * FEW_WAVES, 2)
 gemm_fma_by_chain_kernel(const elem_t* __restrict__ x, int x_stride, const elem_t* __restrict__ w, const void* __restrict__ bias,
@@ -478,9 +478,9 @@ gemm_fma_by_chain_kernel(const elem_t* __restrict__ x, int x_stride, const elem_
 // rows that a read takes fall on the 64 banks.
 // What bounds it: with four blocks a CU 83 % of what the products alone take (139 TFLOP/s at the clock that they leave); with one or two
 // blocks a CU also how they divide the rows (777 rows: 13 of 64, two rounds of 416 blocks or 1.6).
-// 777 rows, us, through registers / here: 2,560 x K 2,048 121 / 113, 2,048 x 2,048 90 / 77, 2,048 x 5,632 236 / 199, gated 5,632 x
-// 2,048 334 / 325, 32,000 x 2,048 947 / 930; 512 rows of 2,048 x 5,632 (a block a CU) 143 / 116, 2,048 rows 416 / 394.  With a read a
-// number (128 LDS instructions a block and step) 127 and 409 for the last two, three stages (three blocks a CU) 128 and 412.
+// 777 rows, us, through registers / here: 2,560 x K 2,048 121 / 114, 2,048 x 2,060 89 / 76, 2,048 x 5,632 234 / 198, gated 5,632 x
+// 2,048 338 / 329, 32,000 x 2,048 960 / 942; 512 rows of 2,048 x 5,632 (a block a CU) 142 / 116, 2,048 rows 414 / 393.  With a read a
+// number (128 LDS instructions a block and step) 409 for the last, three stages (three blocks a CU) 412.
 #define FLOW_STAGES 4
 #define FLOW_STAGE (2 * TILE_M * FMA_PART * 4)
 #define FLOW_LEAST_K 192      // (launch_fma_tiles)
@@ -659,17 +659,19 @@ gemm_fma_flow_kernel(const float* __restrict__ x, int x_stride, const float* __r
 template <int MT, bool GLU, bool VEC>
 static void launch_fma_few(const elem_t* x, int x_stride, const elem_t* w, const void* bias, int bias_is_f32, void* out,
                            int out_stride, int m, int n, int k, int mode, hipStream_t stream) {
-  // As many blocks as give every CU the same number of them, with at most 16 columns each (2,560 columns in 256 blocks of 10:
-  // 9.0 us, in 160 of 16 10.3; 11,264 gated in 512 of 11: 27.3, in 352 of 16 30.8), and so many that X counts less than W.
+  // As many blocks as give every CU the same number of them, with at most 16 columns each, and so many that X counts less than W
+  // (5 rows of 2,560 columns of K 2,048 in 256 blocks of 10: 7.6 us, in 160 of 16 8.1; of gated 5,632 in 512 of 11: 20.1, in 352 of 16
+  // 23.9).
   // X that is loaded singly counts more than a last round: 16 columns from four blocks a CU on (16 rows of 16,390 x 1,001 in blocks
   // of 13: 51.7, of 16 48.9), and whole or half tiles chain by chain.
   const int rows = ceil_div(m, 16 * MT), tiles = ceil_div(n, 16) * rows, each = ceil_div(tiles, 256);
   const int spread = max(MT == 1 ? 4 : 8, min(16, ceil_div(n * rows, 256 * each)));
   // Which kernel.  Numbers loaded singly: one tile of rows and one of W, in a K of more than a chain a wave, are asked for ahead like
   // others (us, against chain by chain: 5 rows of 1,000 x K 1,001 7.5 / 9.5, of 300 x 5,631 31 / 40, of 2,048 x 515 6.0 / 8.4; 16 of
-  // 2,048 x 769 9.7 / 10.3, of 16,390 x 515 29.4 / 33.8).  Aligned: fewer chains than waves go chain by chain,
-  // and 64 rows of as many (512 x K 256 4.6 / 4.3, 4,096 x 256 9.0 / 8.8; gated, and of fewer rows, asked for ahead is the faster: 5 rows of
-  // 2,048 x 256 3.2 / 3.5).
+  // 2,048 x 769 9.7 / 10.3, of 16,390 x 515 27.5 / 33.7).  Aligned: fewer chains than waves go chain by chain,
+  // and 64 rows of as many (us, ahead / so: 512 x K 256 4.5 / 4.3, 2,048 x 256 5.0 / 4.9; gated, and of fewer rows, ahead is the faster: 5 rows of
+  // 2,048 x 256 3.0 / 3.2, of gated 5,632 x 256 a fifth).  In the bfloat16 build, whose numbers are half as long, up to half the waves
+  // (ahead / so: 5 rows of 512 x 192 2.7 / 2.8, 40 of 2,048 x 224 4.4 / 4.8, 40 of 512 x 256 4.1 / 4.6).
   constexpr bool AHEAD = VEC || (MT == 1 && !GLU);
   const bool brief = k <= FEW_WAVES * FMA_PART;
 #define FEW(KERNEL, SHORT, COLUMNS)                                                                                         \
@@ -686,7 +688,7 @@ static void launch_fma_few(const elem_t* x, int x_stride, const elem_t* w, const
   }
 #define FEW_ARGS x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode
   if constexpr (VEC) {
-    if (k <= (FEW_WAVES - 1) * FMA_PART || (brief && MT == 4 && !GLU)) BY_CHAIN(true, spread)
+    if (k <= FEW_BRIEF * FMA_PART || (!AXON_BF16 && brief && MT == 4 && !GLU)) BY_CHAIN(true, max(8, spread))
     else if (brief) FEW(gemm_fma_few_rows_kernel, true, spread)
     else FEW(gemm_fma_few_rows_kernel, false, spread)
   } else {
@@ -705,8 +707,8 @@ static void launch_fma_tiles(dim3 tiles, const elem_t* x, int x_stride, const el
 #if !AXON_BF16
   // Short K: the stages that are filled before the first product count more than what they save, and where there are more
   // than two blocks a CU these cover each other's waits.  us, through registers / by direct loads: up to 512 blocks, 400 rows of 1,000
-  // columns of K 64 4.8 / 5.4, 128 6.1 / 6.4, 192 7.3 / 7.3, 256 8.5 / 8.1; more, 777 rows of 4,096 of K 96 12.6 / 15.9, 256 27.5 / 29.2,
-  // 512 47.9 / 48.4, 640 57.9 / 57.4; of 32,000 of K 256 136 / 146, 640 1.02 times, 1,024 as long.
+  // columns of K 64 4.8 / 5.4, 128 6.6 / 6.9, 192 8.4 / 8.3, 256 10.0 / 9.6; more, 777 rows of 4,096 of K 96 12.6 / 15.9, 256 24.0 / 25.5,
+  // 512 42.3 / 42.8, 640 51.4 / 51.0; of 32,000 of K 256 136 / 146, 640 309 / 314, as long from 1,024 on.
   if constexpr (VEC) {
     if (k >= ((long)tiles.x * tiles.y <= 512 ? FLOW_LEAST_K : 640)) {
       static_assert(FLOW_STAGES * FLOW_STAGE <= 64 * 1024, "more LDS than a launch gets unasked");
@@ -726,10 +728,10 @@ static int launch_fma(const elem_t* x, int x_stride, const elem_t* w, const void
   const bool vec_w = (k % 4 == 0) && ((uintptr_t)w % vbytes == 0) && k < (1 << 23);
   const bool vec_x = (k % 4 == 0) && (x_stride % 4 == 0) && ((uintptr_t)x % vbytes == 0) && x_stride < (1 << 23);
 #define FMA_ARGS x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode, stream
-// Up to 32 rows a product waits for W; from 33 to 128 so it does where the tiles would be fewer than
-// the CUs (2,048 columns of K 5,632 at 128 rows: 143 us with 64 tiles, 67 us with a wave a part of K), while
-// 352 tiles (a gated product of 5,632 columns at 128 rows) take 90 us against 117 and 500 (32,000 columns of K 2,048
-// at 33 and at 64 rows) 89 and 92 against 142 and 158.
+// Up to 32 rows a product waits for W; from 33 to 128 so it does where the tiles would be fewer than the CUs.  us, a wave a
+// chain / tiles: 128 rows of 2,048 columns of K 5,632 (64 tiles) 58 / 114, 64 of 8,192 of K 2,048 (128) 42 / 45, 65 of them (256) 67 / 46, of gated
+// 5,632 (352) 78 / 75, 33 and 64 of 32,000 (500) 119 / 78 and 153 / 81.  From some 170 tiles on the line is on the slow side: 64 rows
+// of gated 5,632 of K 2,048 (176) 54 / 46, of 16,000 of K 1,024 (250) 44 / 26.
 #define FMA_LAUNCH(GLU, VEC)                                                                  \
   const dim3 tiles(ceil_div(n, GLU ? TILE_M / 2 : TILE_M), ceil_div(m, TILE_M));              \
   if (m <= 16) {                                                                              \

@@ -335,8 +335,11 @@ CASES = [
     (F32, ["gemm_fma_flow<1>"], check_gemm, (F32, 129, 48, 292, MODE_SWIGLU)),
     # chain by chain: fewer chains than waves, and numbers loaded singly but for one tile of rows and W
     *[(d, [f"gemm_fma_by_chain<{rows},{int(mode == MODE_SWIGLU)},{int(K % 4 == 0)}>"], check_gemm, (d, M, N, K, mode)) for d in (F32, BF)
-      for rows, M in ((16, 5), (32, 20), (64, 70)) for N, K, mode in ((259, 100, MODE_STORE_F32), (259, 70, MODE_STORE_F32), (48, 224, MODE_SWIGLU),
+      for rows, M in ((16, 5), (32, 20), (64, 70)) for N, K, mode in ((259, 100, MODE_STORE_F32), (259, 70, MODE_STORE_F32), (48, 96, MODE_SWIGLU),
                                                                       (48, 290, MODE_SWIGLU))],
+    # as many chains as waves, or nearly, asked for ahead
+    *[(BF, [f"gemm_fma<{rows},{int(mode == MODE_SWIGLU)}>"], check_gemm, (BF, M, N, 224, mode)) for rows, M in ((16, 5), (32, 20), (64, 70))
+      for N, mode in ((259, MODE_STORE_F32), (48, MODE_SWIGLU))],
     (BF, ["gemm_fma<16,0>"], check_gemm, (BF, 5, 100, 70, MODE_STORE, True)),
     (BF, ["gemm_fma<64,0>"], check_gemm, (BF, 70, 259, 130, MODE_STORE_F32)),
     (BF, ["gemm_fma<16,1>"], check_gemm, (BF, 9, 96, 70, MODE_SWIGLU)),
