@@ -69,17 +69,6 @@ struct Number {
   static constexpr int value = V;
 };
 
-// Waits until at most min(rounds, MAX) rounds of LOADS loads each are in flight.
-template <int MAX, int LOADS>
-__device__ inline void wait_rounds(int rounds) {
-  if constexpr (MAX <= 0) {
-    wait_vmcnt<0>();
-  } else {
-    if (rounds >= MAX) wait_vmcnt<MAX * LOADS>();
-    else wait_rounds<MAX - 1, LOADS>(rounds);
-  }
-}
-
 // ---------------------------------------------------------------------------- what the tile kernels share
 // Memory as a buffer (buffer.h): a load's place in it is a register of the lane's and a scalar one, with no address of its own to
 // work out; lanes whose row is behind the last one read nothing and get zeros.
@@ -2304,9 +2293,12 @@ static int tiles32_of(int n, int mode) { return mode == MODE_SWIGLU ? n / 16 : (
 
 // Whether the blocks of a product of more than 128 rows walk all of K themselves, in tiles of 128 x 128, and keep the
 // segments' sums in registers; else a block takes a segment and its sums go through the workspace.  Where the lines
-// lie was found with tiles of 32x32x16 products (32 shapes of 140 to 8,192 rows, 766 measurements, of which the figures
-// below are), and the present tiles, which gained more here than there, were timed against it: of the products of 14 matrices
-// of 200 to 2,048 rows the 42 that keep their sums take 0.57 to 0.94 of the time.
+// lie was found with former tiles (32x32x16 products; 32 shapes of 140 to 8,192 rows, 766 measurements, of which the figures
+// below are).  The present ones, of which these gained more than the others, were timed both ways for 21 matrices of the 2,048,
+// 4,096, 7B and 14B widths at 150 to 3,072 rows: of 106 products that keep their sums 102 are the faster for it (down to 0.40 of the
+// time), and of 164 that do not 69 would be too, by up to 1.8 times: the lines are on the safe side.  us, kept / as they run: K 2,048,
+// 2,048 columns of 1,525 rows 23 / 40, of 1,024 22 / 27; 3,584 of K 3,584 of 1,024 rows 34 / 50; gated 4,096 of K 4,096 of 1,024 70 / 101;
+// kept and the slower for it 5,120 of K 13,824 of 1,024 rows 209, with large tiles 180.
 //  * There have to be blocks for the chip's 256 CUs.  K 2,048, 2,560 columns of 1,525 rows (240 blocks) 35 against 38 us,
 //    2,048 of 1,525 (192) 35 against 33; K 3,584, 3,584 of 1,200 (280) 63 against 71, 900 (224) 52 against 49.  Gated,
 //    1,408 of 700 (132) 27 against 28, of 900 (176) 27 against 30; 1,024 of 900 (128) 27 against 22.
@@ -2443,9 +2435,11 @@ static int gemm_mfma_pass(const bf16_t* x, int x_stride, const bf16_t* w, const 
   }
   // 256 x 256 tiles (8 waves, a block a CU) or 128 x 128 tiles (4 waves, two blocks a CU, four
   // times as many blocks at twice the traffic from L2 per product): whichever takes the chip's 256
-  // CUs fewer rounds, a round of the small tiles counted as 0.65 of a round of the large ones
-  // (both timed for 14 matrices, those of the 7B and 14B layers among them, at 200 to 2,048 rows: of 140
-  // products that do not keep their segments' sums one takes the slower tile, by 4 %, [gate; up] of 600 rows).
+  // CUs fewer rounds, a round of the small tiles counted as 0.65 of a round of the large ones: found with tiles that both have
+  // 32x32x16 products.  With the present large ones a round of the small is 0.5 to 0.9 of theirs, and of 209 products of 21 matrices at
+  // 150 to 3,072 rows that do not keep their segments' sums 21 take the slower tile by more than 3 %, most of them three rounds of the
+  // small for two of the large: us, small / large, [gate; up] of a 7B layer of 600 rows 196 / 161, of a 14B layer of 777 265 / 215, 32,000
+  // columns of K 2,048 of 600 124 / 101.
   const long big = (long)ceil_div(m, 256) * ceil_div(n, glu ? 128 : 256) * segs;
   const long small = (long)ceil_div(m, 128) * ceil_div(n, glu ? 64 : 128) * segs;
   const long rounds_big = (big + 255) / 256, rounds_small = (small + 511) / 512;

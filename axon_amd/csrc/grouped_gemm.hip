@@ -243,8 +243,8 @@ __global__ void __launch_bounds__(256) grouped_gemm_mfma_kernel(GroupedArgs a) {
 // of a stage are read one ahead of the products.  Rows of a stage are 128 bytes, their 16-byte slots permuted by
 // slot ^ (row / 2 % 8): the 16 rows a read takes at a time fall into 16 different slots of the 64 banks.  The chain of an
 // output is the one of the kernel above (16x16x32 products in ascending k), so which of the two runs changes no
-// bit.  2,048 tokens, 4 of 32 experts of [1,408, 2,048] and [2,048, 704]: 81 and 63 us (163 and 113 with stages of 32 k
-// through registers).
+// bit.  2,048 tokens, 4 of 32 experts of [1,408, 2,048] and [2,048, 704]: 81 and 57 us (163 and 113 with stages of 32 k
+// through registers, by columns).
 #define GT_ROWS 64
 #define GT_BK 64
 #define GT_STAGE(wrows) ((GT_ROWS + (wrows)) * GT_BK * 2)
@@ -450,7 +450,7 @@ extern "C" int axk_grouped_gemm(const void* x, int x_is_f32, long x_row_stride, 
     // 128 rows of W a block, three blocks a CU, unless the gated product has two rounds of blocks of 256: those read
     // X half as often, which pays where K is long.  us, 256 rows of W a block against 128: 10 blocks of channels [512, 256] at
     // 256 rows 14.7 / 9.4, at 2,048 38 / 26; 16 heads [512, 128] at 2,048 41 / 27; 4 of 32 experts of 2,048 tokens
-    // [2,048, 704] 69 / 63, gated [1,408, 2,048] 81 / 85, of 1,024 tokens (576 blocks) 46 / 57, of 512 (384) 44 / 41, of
+    // [2,048, 704] (by columns) 69 / 63, gated [1,408, 2,048] 81 / 85, of 1,024 tokens (576 blocks) 46 / 57, of 512 (384) 44 / 41, of
     // 256 41 / 33; 2 of 8 of 128 tokens gated [1,024, 1,024] 20 / 16; 8 of 64 of 2,048 gated [512, 2,048] 74 / 67.
     const long row_blocks = (long)(tiles ? max_tiles : ceil_div(m, GT_ROWS)) * (tiles ? 1 : groups);
     const bool wide = glu && row_blocks * ceil_div(n, 128) >= 512;

@@ -155,3 +155,12 @@ def test_rows_far_apart():
     k.gemm(far, w, got, None, MODE_STORE_F32)
     k.gemm(x, w, want, None, MODE_STORE_F32)
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("K", [192, 196, 204, 216, 220, 224, 232, 252, 256, 284, 316, 320, 1052])
+def test_direct_loads_at_every_end_of_k(K):
+    """The same for a K that the tiles take by direct loads."""
+    k = kernels("float32")
+    k.reset_instances()
+    test_tiles_at_every_end_of_k(K)
+    assert {"gemm_fma_flow<0>", "gemm_fma_flow<1>"} <= set(k.instances(launched=True))

@@ -48,7 +48,8 @@ def unwaited(assembly, kernel):
     return reads, faults
 
 
-@pytest.mark.parametrize("source, kernel", [("grouped_gemm.hip", "grouped_gemm_tile_kernel"),
+@pytest.mark.parametrize("source, kernel", [("gemm.hip", "gemm_fma_flow_kernel"),
+                                            ("grouped_gemm.hip", "grouped_gemm_tile_kernel"),
                                             ("latent_attention.hip", "latent_attention_prompt_kernel"),
                                             ("gemm_mfma.hip", "gemm_tile_kernel"),
                                             ("gemm_mfma.hip", "gemm_small_tile_kernel"),
@@ -57,7 +58,7 @@ def unwaited(assembly, kernel):
                                             ("attention_mfma.hip", "attention_decode_kernel"),
                                             ("state_space.hip", "state_space_walk_kernel")])
 def test_nothing_comes_between_a_read_and_its_wait(device_code, source, kernel):
-    reads, faults = unwaited(device_code(source), kernel)
+    reads, faults = unwaited(device_code(source, "float32" if source == "gemm.hip" else "bfloat16"), kernel)
     assert reads > 0 and not faults, faults[:5]
 
 
