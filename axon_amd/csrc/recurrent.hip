@@ -178,84 +178,140 @@ __global__ void gated_scan_kernel(const float* __restrict__ gates, const float* 
   }
 }
 
-// The same recurrence for long stretches of tokens, in two launches.  First, for every (token,
-// channel) at once, what does not depend on the state: a, b = (sqrt(1 - a^2) i) u and gelu(y), the
-// very operations of the kernel above, kept in 32-bit.  Then a thread per (request, channel) walks
-// S = a S + b with 32 steps' operands under way while the 32 before them are walked (2,048 tokens of 2,560 channels,
-// 40 waves: 109 -> 91 us with the walk waiting for sixteen at a time).  Bound by what a wave issues: 21 instructions a
-// step, half of them scalar, at four clocks and more each, in 84 % of its cycles.  The bits are those of the kernel above.
-__global__ void gated_scan_terms_kernel(const float* __restrict__ gates, const float* __restrict__ u,
-                                        const elem_t* __restrict__ y, long y_stride, const void* __restrict__ lam,
-                                        int lam_is_f32, float decay, float* __restrict__ terms, int channels, int block_width) {
-  const int t = blockIdx.y;
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= channels) return;
-  const float l = load_vec(lam, lam_is_f32, c);
+// The same recurrence for stretches of tokens: a block has `width` channels of a request.  One wave walks S = a S + b, a lane a
+// channel, and does nothing else; the others work out, a (token, channel) a lane, what it walks with and what comes of it: a,
+// b = (sqrt(1 - a^2) i) u and gelu(y) of the chunk ahead, the outputs of the chunk behind, through LDS, a barrier a chunk.  The
+// operations are those of the kernel above, and so are the bits.  Bound by the exponentials and the tangent, some 200 vector
+// instructions a (token, channel): 2,048 tokens of 2,560 channels 47 us, where the terms in a launch of their own through memory and
+// a walk bound by what one wave issues took 35 + 91; 4,096 243 -> 87, 512 37 -> 16, 64 15 -> 10; five requests of 300 46 -> 34, 64
+// of 32 48 -> 40; 5,120 channels 157 -> 67, 1,024 106 -> 40.
+#define SCAN_FEEDERS 512
+#define SCAN_EACH 2                               // tokens of a chunk that a feeding thread has
+#define SCAN_WIDEST 64
+// Tokens that the feeding threads have side by side: four at a time, since the walk reads four.
+__host__ __device__ inline int scan_rows(int width) { return SCAN_FEEDERS / width / 4 * 4; }
+// Channels a block has: of a lone request as many as give every CU a block, 16 of each of several, 64 of those that are short
+// (the blocks that are too many then leave at once).  us by width, 2,560 channels: 2,048 tokens of a request 53.5 with 8, 46.8 with
+// 10, 50.0 with 16, 91.9 with 32 (5,120 channels 64.1 with 10, 67.1 with 20, 79.1 with 16); requests of 1,000, 700 and 400 38.9 with 10, 35.7 with
+// 16, 48.5 with 32; five of 300 39.8, 33.8, 28.7, and 31.7 with 64; 64 of 32 tokens 93.0 with 16, 39.7 with 64.
+#define SCAN_SHORT 128
+__host__ inline int scan_width(int channels, int requests) {
+  const int width = requests > 1 ? 16 : (channels + 255) / 256;
+  return width < 8 ? 8 : width <= 16 ? (width + 1) / 2 * 2 : width <= 20 ? 20 : 32;
+}
+// Floats a channel has in LDS: four more than its tokens, so that lanes side by side meet different banks.
+#define SCAN_FLOATS (SCAN_FEEDERS * SCAN_EACH + 4 * SCAN_WIDEST)
+
+__device__ inline void scan_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }   // loads stay under way
+
+__global__ void __launch_bounds__(SCAN_FEEDERS + AXON_WAVE)
+gated_scan_stretch_kernel(const float* __restrict__ gates, const float* __restrict__ u, const elem_t* __restrict__ y, long y_stride,
+                          const elem_t* __restrict__ x, long x_stride, const void* __restrict__ lam, int lam_is_f32, float decay,
+                          float* __restrict__ state, long state_stride, const int32_t* __restrict__ spans,
+                          const int32_t* __restrict__ positions, elem_t* __restrict__ out, int channels, int block_width, int taps,
+                          int width) {
+  __shared__ __align__(16) float as[2][SCAN_FLOATS], bs[2][SCAN_FLOATS], ss[2][SCAN_FLOATS];
+  const int slot = spans[3 * blockIdx.y], first = spans[3 * blockIdx.y + 1], count = spans[3 * blockIdx.y + 2];
+  if (gridDim.y > 1 && count <= SCAN_SHORT) width = SCAN_WIDEST;
+  // neighbouring channels on one XCD: their rows share cache lines
+  const int per_xcd = ((channels + width - 1) / width + 7) / 8, c0 = ((blockIdx.x % 8) * per_xcd + blockIdx.x / 8) * width;
+  if ((int)blockIdx.x / 8 >= per_xcd || c0 >= channels || count <= 0) return;
+  const int rows = scan_rows(width), chunk = SCAN_EACH * rows, pitch = chunk + 4, chunks = (count + chunk - 1) / chunk;
+  if (threadIdx.x >= SCAN_FEEDERS) {
+    const int lane = threadIdx.x - SCAN_FEEDERS, c = c0 + lane;
+    const bool has = lane < width && c < channels;
+    const int start = positions[first];
+    const float* from = state + (long)slot * state_stride + (long)((start + 1) & 1) * taps * channels;
+    float* row = state + (long)slot * state_stride + (long)((start + count - 1) & 1) * taps * channels;
+    float S = has ? from[c] : 0.0f;
+    for (int it = 0; it < chunks + 2; ++it) {
+      if (it > 0 && it <= chunks && has) {
+        const int left = count - (it - 1) * chunk, at = lane * pitch;
+        const float* A = as[(it - 1) & 1] + at;
+        const float* B = bs[(it - 1) & 1] + at;
+        float* to = ss[(it - 1) & 1] + at;
+        if (left >= chunk) {
+          float4 a0 = *reinterpret_cast<const float4*>(A), b0 = *reinterpret_cast<const float4*>(B);
+          for (int j = 0; j < chunk; j += 4) {
+            const int ahead = min(j + 4, chunk - 4);
+            const float4 a1 = *reinterpret_cast<const float4*>(A + ahead), b1 = *reinterpret_cast<const float4*>(B + ahead);
+            float4 v;
+            S = fmaf(a0.x, S, b0.x); v.x = S;
+            S = fmaf(a0.y, S, b0.y); v.y = S;
+            S = fmaf(a0.z, S, b0.z); v.z = S;
+            S = fmaf(a0.w, S, b0.w); v.w = S;
+            *reinterpret_cast<float4*>(to + j) = v;
+            a0 = a1; b0 = b1;
+          }
+        } else {
+          for (int j = 0; j < left; ++j) {
+            S = fmaf(A[j], S, B[j]);
+            to[j] = S;
+          }
+        }
+      }
+      scan_barrier();
+    }
+    if (!has) return;
+    row[c] = S;
+    float* kept = row + channels;
+    const float* kept_from = from + channels;
+    for (int i = 0; i < taps - 1; ++i) {
+      const int at = i + count;
+      kept[(long)i * channels + c] = at < taps - 1 ? kept_from[(long)at * channels + c]
+                                                   : to_float(x[(long)(first + at - (taps - 1)) * x_stride + c]);
+    }
+    return;
+  }
+
+  const int ch = threadIdx.x % width, tok = threadIdx.x / width, c = c0 + ch;
+  const bool has = tok < rows && c < channels;
+  const int cc = min(c, channels - 1);
+  const float l = load_vec(lam, lam_is_f32, cc);
   const float softplus = l > 20.0f ? l : log1pf(expf(l));
   const float rate = -decay * softplus;
-  const int b = c / block_width, j = c % block_width;
-  const float* g = gates + (long)t * 2 * channels + (long)b * 2 * block_width + j;
-  const float r = sigmoid32(g[0]), i = sigmoid32(g[block_width]);
-  const float log_a = rate * r;
-  const float mult = sqrtf(-expm1f(2.0f * log_a));
-  float* dst = terms + (long)t * 3 * channels + c;
-  dst[0] = expf(log_a);
-  dst[channels] = (mult * i) * u[(long)t * channels + c];
-  dst[2 * channels] = gelu_tanh32(to_float(y[(long)t * y_stride + c]));
-}
-
-#define SCAN_AHEAD 32
-__global__ void __launch_bounds__(64) gated_scan_walk_kernel(const float* __restrict__ terms, const elem_t* __restrict__ x, long x_stride,
-                                       float* __restrict__ state, long state_stride, const int32_t* __restrict__ spans,
-                                       const int32_t* __restrict__ positions, elem_t* __restrict__ out, int channels, int taps) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= channels) return;
-  const int slot = spans[3 * blockIdx.y], first = spans[3 * blockIdx.y + 1], count = spans[3 * blockIdx.y + 2];
-  const int start = positions[first];
-  const float* from = state + (long)slot * state_stride + (long)((start + 1) & 1) * taps * channels;
-  float* row = state + (long)slot * state_stride + (long)((start + count - 1) & 1) * taps * channels;
-  float S = from[c];
-  int t = first;
-  // SCAN_AHEAD steps' operands asked for while the SCAN_AHEAD before them are walked
-  float even[3][SCAN_AHEAD], odd[3][SCAN_AHEAD];
-  const int whole = first + count / SCAN_AHEAD * SCAN_AHEAD;
-  auto ask = [&](float (&o)[3][SCAN_AHEAD], int t0) {
-    if (t0 >= whole) return;
+  const long gate_at = (long)(cc / block_width) * 2 * block_width + cc % block_width;
+  struct Inputs { float r, i, u; elem_t y; };
+  Inputs next[SCAN_EACH];
+  auto ask = [&](int it) {                         // (behind the last token: that one, not used)
 #pragma unroll
-    for (int i = 0; i < SCAN_AHEAD; ++i) {
-      const float* src = terms + (long)(t0 + i) * 3 * channels + c;
-      o[0][i] = src[0]; o[1][i] = src[channels]; o[2][i] = src[2 * channels];
+    for (int e = 0; e < SCAN_EACH; ++e) {
+      const long t = first + min(it * chunk + e * rows + tok, count - 1);
+      const float* g = gates + t * 2 * channels + gate_at;
+      next[e] = Inputs{g[0], g[block_width], u[t * channels + cc], y[t * y_stride + cc]};
     }
   };
-  auto walk = [&](const float (&o)[3][SCAN_AHEAD], int t0) {
+  ask(0);
+  float gelu[3][SCAN_EACH] = {};                   // of the chunk now fed, of the one walked, of the one put out
+  for (int it = 0; it < chunks + 2; ++it) {
 #pragma unroll
-    for (int i = 0; i < SCAN_AHEAD; ++i) {
-      S = fmaf(o[0][i], S, o[1][i]);
-      out[(long)(t0 + i) * channels + c] = from_float(S * o[2][i]);
+    for (int e = 0; e < SCAN_EACH; ++e) { gelu[2][e] = gelu[1][e]; gelu[1][e] = gelu[0][e]; }
+    if (it < chunks) {
+      Inputs now[SCAN_EACH];
+#pragma unroll
+      for (int e = 0; e < SCAN_EACH; ++e) now[e] = next[e];
+      if (it + 1 < chunks) ask(it + 1);
+#pragma unroll
+      for (int e = 0; e < SCAN_EACH; ++e) {
+        const float r = sigmoid32(now[e].r), i = sigmoid32(now[e].i);
+        const float log_a = rate * r;
+        const float mult = sqrtf(-expm1f(2.0f * log_a));
+        const float a = expf(log_a), b = (mult * i) * now[e].u;
+        gelu[0][e] = gelu_tanh32(to_float(now[e].y));
+        if (has) {
+          as[it & 1][ch * pitch + e * rows + tok] = a;
+          bs[it & 1][ch * pitch + e * rows + tok] = b;
+        }
+      }
     }
-  };
-  ask(even, t);
-  while (t < whole) {
-    ask(odd, t + SCAN_AHEAD);
-    walk(even, t);
-    t += SCAN_AHEAD;
-    if (t >= whole) break;
-    ask(even, t + SCAN_AHEAD);
-    walk(odd, t);
-    t += SCAN_AHEAD;
-  }
-  for (; t < first + count; ++t) {
-    const float* src = terms + (long)t * 3 * channels + c;
-    S = fmaf(src[0], S, src[channels]);
-    out[(long)t * channels + c] = from_float(S * src[2 * channels]);
-  }
-  row[c] = S;
-  float* kept = row + channels;
-  const float* kept_from = from + channels;
-  for (int i = 0; i < taps - 1; ++i) {
-    const int at = i + count;
-    kept[(long)i * channels + c] = at < taps - 1 ? kept_from[(long)at * channels + c]
-                                                 : to_float(x[(long)(first + at - (taps - 1)) * x_stride + c]);
+    if (it >= 2 && has) {
+#pragma unroll
+      for (int e = 0; e < SCAN_EACH; ++e) {
+        const int j = (it - 2) * chunk + e * rows + tok;
+        if (j < count) out[(long)(first + j) * channels + c] = from_float(ss[it & 1][ch * pitch + e * rows + tok] * gelu[2][e]);
+      }
+    }
+    scan_barrier();
   }
 }
 
@@ -302,19 +358,29 @@ extern "C" int axk_gated_scan(const float* gates, const float* u, const void* y,
   AXK_REQUIRE(n_spans <= 65535, "gated_scan: %d requests in one step (at most 65535)", n_spans);
   if (n_spans == 0) return 0;
   dim3 grid(ceil_div(channels, 64), n_spans);
-  if (terms != nullptr && spans != nullptr && n_tokens > 0) {
-    AXK_REQUIRE(n_tokens <= 65535, "gated_scan: %d tokens in one step (at most 65535)", n_tokens);
-    dim3 wide(ceil_div(channels, 256), n_tokens);
-    gated_scan_terms_kernel<<<wide, 256, 0, (hipStream_t)stream>>>(gates, u, (const elem_t*)y, y_stride, lam, lam_is_f32, decay,
-                                                                  terms, channels, block_width);
-    gated_scan_walk_kernel<<<grid, 64, 0, (hipStream_t)stream>>>(terms, (const elem_t*)x, x_stride, state, state_stride, spans,
-                                                                positions, (elem_t*)out, channels, taps);
-    AXK_LAUNCH_CHECK("gated_scan");
-    return 0;
-  }
   gated_scan_kernel<<<grid, 64, 0, (hipStream_t)stream>>>(gates, u, (const elem_t*)y, y_stride, (const elem_t*)x, x_stride, lam,
                                                          lam_is_f32, decay, state, state_stride, spans, positions,
                                                          seq_rows, (elem_t*)out, channels, block_width, taps);
   AXK_LAUNCH_CHECK("gated_scan");
+  return 0;
+}
+
+extern "C" int axk_gated_scan_stretches(const float* gates, const float* u, const void* y, long y_stride, const void* x, long x_stride,
+                                        const void* lam, int lam_is_f32, float decay, float* state, long state_stride,
+                                        const int32_t* spans, int n_spans, const int32_t* positions, void* out, int channels,
+                                        int block_width, int taps, void* stream) {
+  AXK_REQUIRE(n_spans >= 0 && channels > 0 && block_width > 0 && channels % block_width == 0 && taps >= 1,
+              "gated_scan: bad sizes spans=%d channels=%d block width=%d taps=%d", n_spans, channels, block_width, taps);
+  AXK_REQUIRE(state_stride >= 2L * taps * channels, "gated_scan: a state row of %ld floats does not hold 2 x %d x %d",
+              state_stride, taps, channels);
+  AXK_REQUIRE(spans != nullptr && positions != nullptr, "gated_scan: no spans or no positions");
+  AXK_REQUIRE(n_spans <= 65535, "gated_scan: %d requests in one step (at most 65535)", n_spans);
+  if (n_spans == 0) return 0;
+  const int width = scan_width(channels, n_spans);
+  const dim3 grid(8 * ceil_div(ceil_div(channels, width), 8), n_spans);
+  gated_scan_stretch_kernel<<<grid, SCAN_FEEDERS + AXON_WAVE, 0, (hipStream_t)stream>>>(
+      gates, u, (const elem_t*)y, y_stride, (const elem_t*)x, x_stride, lam, lam_is_f32, decay, state, state_stride, spans, positions,
+      (elem_t*)out, channels, block_width, taps, width);
+  AXK_LAUNCH_CHECK("gated_scan_stretches");
   return 0;
 }

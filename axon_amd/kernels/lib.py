@@ -110,6 +110,8 @@ _SIGNATURES = {
                         c_int, c_void_p],
     "axk_gated_scan": [c_void_p, c_void_p, c_void_p, c_long, c_void_p, c_long, c_void_p, c_int, c_float, c_void_p, c_long,
                        c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_int, c_void_p],
+    "axk_gated_scan_stretches": [c_void_p, c_void_p, c_void_p, c_long, c_void_p, c_long, c_void_p, c_int, c_float, c_void_p, c_long,
+                                 c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p],
     "axk_state_conv": [c_void_p, c_long, c_void_p, c_void_p, c_int, c_int, c_void_p, c_long, c_long, c_long, c_void_p, c_void_p,
                        c_void_p, c_int, c_int, c_int, c_void_p, c_long, c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p],
     "axk_state_space_scan": [c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_long, c_long, c_long, c_void_p, c_int, c_void_p,
@@ -1041,18 +1043,20 @@ class Kernels:
         if (gates.shape != (T, 2 * C) and gates.numel() != T * 2 * C) or y.shape != (T, C) or x.shape != (T, C) or out.shape != (T, C) \
                 or y.stride(1) != 1 or x.stride(1) != 1 or not out.is_contiguous() or lam.numel() != C or seq_rows.numel() != T:
             raise KernelError(f"gated_scan: gates {tuple(gates.shape)}, u {tuple(u.shape)}, y {tuple(y.shape)}, out {tuple(out.shape)}")
-        terms = None
+        n = T
         if spans is not None:
             self._i32(spans, "scan spans")
             n = spans.shape[0]
-            if T > 4 * n:            # stretches of tokens: the state-free terms for all tokens at once, then a lean walk
-                terms = torch.empty((T, 3, C), dtype=torch.float32, device=u.device)
-        else:
-            n = T
+            if T > 4 * n:            # stretches of tokens
+                self._check(self.lib.axk_gated_scan_stretches(
+                    _ptr(gates), _ptr(u), _ptr(y), y.stride(0), _ptr(x), x.stride(0), _ptr(lam), self._vec_flag(lam, "scan lam"),
+                    float(decay), _ptr(state), state.stride(0), _ptr(spans), n, _ptr(positions), _ptr(out), C, int(block_width),
+                    int(taps), _stream()))
+                return out
         self._check(self.lib.axk_gated_scan(_ptr(gates), _ptr(u), _ptr(y), y.stride(0), _ptr(x), x.stride(0), _ptr(lam),
                                             self._vec_flag(lam, "scan lam"), float(decay), _ptr(state), state.stride(0),
                                             _ptr(spans), n, _ptr(positions), _ptr(seq_rows), _ptr(out), C, int(block_width),
-                                            int(taps), _ptr(terms), T, _stream()))
+                                            int(taps), None, T, _stream()))
         return out
 
     # ------------------------------------------------------------------ a state-space mixer with per-request state

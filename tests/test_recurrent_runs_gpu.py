@@ -67,3 +67,27 @@ def test_long_walk(dtype, lengths):
     assert k.lib.axk_gated_scan(_ptr(gates), _ptr(u), _ptr(y), C, _ptr(x), C, _ptr(lam), 1, 8.0, _ptr(kept), kept.stride(0),
                                 _ptr(spans), len(lengths), _ptr(pos), _ptr(seq), _ptr(want), C, width, taps, None, T, _stream()) == 0
     assert torch.equal(got, want) and torch.equal(state, kept)
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
+@pytest.mark.parametrize("lengths, channels", [([6], 8), ([95], 2560), ([96], 2560), ([193], 2570), ([400], 4200), ([131], 5130), ([70], 8200),
+                                               ([128, 129, 127, 64, 65, 1], 1290), ([9, 300], 20)])
+def test_long_walk_by_width(dtype, lengths, channels):
+    """Blocks of 8, 10, 16, 20, 32 and 64 channels, the last ones of a row narrower, around whole chunks of each."""
+    from axon_amd.kernels import kernels
+    from axon_amd.kernels.lib import _ptr, _stream
+    k, dev, C, width, taps = kernels(dtype), "cuda:0", channels, channels // 2, 3
+    elem = getattr(torch, dtype)
+    torch.manual_seed(6)
+    seq, pos, spans = _rows(lengths, dev)
+    T = sum(lengths)
+    gates, u = torch.randn(T, 2 * C, device=dev), torch.randn(T, C, device=dev)
+    yx = torch.randn(T, 2 * C, device=dev).to(elem)
+    lam = torch.rand(C, device=dev)
+    state = torch.randn(len(lengths), 2 * taps * C, device=dev)
+    kept = state.clone()
+    got, want = (torch.full((T, C), float("nan"), dtype=elem, device=dev) for _ in range(2))
+    k.gated_scan(gates, u, yx[:, :C], yx[:, C:], lam, 8.0, state, spans, pos, seq, got, width, taps)
+    assert k.lib.axk_gated_scan(_ptr(gates), _ptr(u), _ptr(yx), 2 * C, _ptr(yx[:, C:]), 2 * C, _ptr(lam), 1, 8.0, _ptr(kept), kept.stride(0),
+                                _ptr(spans), len(lengths), _ptr(pos), _ptr(seq), _ptr(want), C, width, taps, None, T, _stream()) == 0
+    assert torch.equal(got, want) and torch.equal(state, kept)
