@@ -355,16 +355,35 @@ struct MaState {
 // row, rows vstride apart, the block's positions side by side; both already moved to the lane's
 // slice (8 g, 4 g).  qfrag(mp, c): the lane's query operand of map mp, chunk c.  full: every column
 // sees every position of the block (no mask to apply).  The running maximum is kept in units of log2 e.
-template <int MAPS, int DT, int KC, class PTR, class QF>
+// AHEAD: every load of the block goes out before the first product (a wave that has one block waits for memory once), loaded()
+// behind them.
+template <int MAPS, int DT, int KC, bool AHEAD, class PTR, class QF, class LOADED>
 __device__ inline void ma_block(MaState<MAPS, DT>& st, PTR kbase, int kstride, PTR vbase, int vstride,
                                 QF qfrag, int p0, int my_lo, int my_pos, int keep, bool full, int dim, int dt_n, float scale, float softcap,
-                                int j, int g) {
+                                int j, int g, LOADED loaded) {
   const int kc = (dim + 31) / 32;
   // the bend's constants: scale 2 log2(e) / c into the exponential; c log2(e) and twice that out of it
   const float bend_in = softcap > 0.0f ? scale * 2.8853900817779268f / softcap : 0.0f, scale_log2 = scale * 1.4426950408889634f;
   const float softcap_log2 = softcap * 1.4426950408889634f, bend_out = 2.0f * softcap_log2;
   uint4 pf[MAPS][2];
   float fold[MAPS];
+  uint4 kall[AHEAD ? MAPS * 4 : 1][KC];
+  uint2 vall[AHEAD ? DT : 1][4];
+  if (AHEAD) {                         // (chunks and tiles that the sizes lack: the last again, not used)
+#pragma unroll
+    for (int r = 0; r < MAPS * 4; ++r)
+#pragma unroll
+      for (int c = 0; c < KC; ++c)
+        kall[AHEAD ? r : 0][c] = ma_load16(kbase + (16 * (r % 4) + j) * kstride + r / 4 * dim + 32 * min(c, kc - 1));
+#pragma unroll
+    for (int e = 0; e < DT; ++e) {
+      const PTR vrow = vbase + (16 * min(e, dt_n - 1) + j) * vstride;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) vall[AHEAD ? e : 0][c] = ma_load8(vrow + 16 * c);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    loaded();
+  }
 #pragma unroll
   for (int mp = 0; mp < MAPS; ++mp) {
     ma_f32x4 s[4];
@@ -375,7 +394,7 @@ __device__ inline void ma_block(MaState<MAPS, DT>& st, PTR kbase, int kstride, P
       uint4 kf[KC];
 #pragma unroll
       for (int c = 0; c < KC; ++c)
-        if (c < kc) kf[c] = ma_load16(krow + 32 * c);      // beyond dim the query's operand is zero and the row's neighbours are finite
+        if (c < kc) kf[c] = AHEAD ? kall[AHEAD ? mp * 4 + pt : 0][c] : ma_load16(krow + 32 * c);      // beyond dim the query's operand is zero and the row's neighbours are finite
 #pragma unroll
       for (int c = 0; c < KC; ++c)
         if (c < kc) s[pt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ma_frag(kf[c]), ma_frag(qfrag(mp, c)), s[pt], 0, 0, 0);
@@ -441,10 +460,7 @@ __device__ inline void ma_block(MaState<MAPS, DT>& st, PTR kbase, int kstride, P
       if (d0 + e < dt_n) {
         const PTR vrow = vbase + (16 * (d0 + e) + j) * vstride;
 #pragma unroll
-        for (int c = 0; c < 2; ++c) {
-          v[e][2 * c] = ma_load8(vrow + 32 * c);
-          v[e][2 * c + 1] = ma_load8(vrow + 32 * c + 16);
-        }
+        for (int c = 0; c < 4; ++c) v[e][c] = AHEAD ? vall[AHEAD ? d0 + e : 0][c] : ma_load8(vrow + 16 * c);
       }
     }
 #pragma unroll
@@ -579,10 +595,10 @@ masked_attention_mfma_kernel(const bf16_t* __restrict__ q, const bf16_t* __restr
     const int b = nth_block(nb, kept, lo_block);
     const int p0 = b * 64, in0 = p0 % page_size;
     const bf16_t* page = cache + (long)pages[p0 / page_size] * page_elems;
-    ma_block<MAPS, DT, KC, const bf16_t*>(st, page + (long)in0 * kw + (long)gk * MAPS * dim + 8 * g, kw,
+    ma_block<MAPS, DT, KC, false, const bf16_t*>(st, page + (long)in0 * kw + (long)gk * MAPS * dim + 8 * g, kw,
                            page + (long)page_size * kw + (long)gk * vdim * page_size + in0 + 4 * g, page_size, qfrag, p0, my_lo,
                            my_pos, keep, ncols == 16 && (p0 >= lo_last || p0 + 63 < keep) && p0 + 63 <= pos_first, dim, dt_n, scale,
-                           softcap, j, g);
+                           softcap, j, g, [] {});
   }
   if (split) {
     if (!my_col) return;
@@ -606,63 +622,152 @@ masked_attention_mfma_kernel(const bf16_t* __restrict__ q, const bf16_t* __restr
                       gate_per_head);
 }
 
+// The same for a step of single tokens whose blocks of positions run side by side: a wave has one block of one token's
+// key/value head, and asks for all of it before its first product.  grid (tokens, kv_heads x sixteens of query heads, chunks).
+// A step of 16 tokens has some 300 such waves, so it waits for memory, once: us at 90 to 1,700 positions, the walk's kernel (a
+// round of loads for every 16 rows of keys and 64 dims of values) / here: 16 heads on 2 of 128 17.7 / 11.7, two maps of 64 over 128 17.1 / 10.2,
+// 8 heads on 2, values of 256 16.8 / 16.4 (64 loads of 8 bytes a lane); the fold behind it, which read eight dims a lane
+// whatever the head has and rows of blocks that do not exist, 6.3 / 5.3, 11.9 / 8.2, 7.9 / 5.9.
+template <int MAPS, int DT, int KC>
+__global__ void __launch_bounds__(64)
+masked_attention_blocks_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ cache, const int32_t* __restrict__ block_table,
+                               int table_stride, const int32_t* __restrict__ positions, const int32_t* __restrict__ seq_rows, int heads,
+                               int kv_heads, int dim, int vdim, int page_size, int mask_kind, int mask_size, float scale, float softcap,
+                               float* __restrict__ partial, int n_chunks, int keep) {
+  constexpr int QMAP = KC * 32, QROW = MAPS * QMAP + 8;
+  constexpr bool AHEAD = MAPS * 4 * KC * 4 + DT * 8 <= 256;       // the registers that a block's keys and values take
+  __shared__ __align__(16) bf16_t qs[16 * QROW];
+  const int lane = threadIdx.x, j = lane & 15, g = lane >> 4, t = blockIdx.x;
+  const int grp = heads / kv_heads, hc = min(grp, 16), per_kv = (grp + hc - 1) / hc;
+  const int gk = blockIdx.y / per_kv, first = blockIdx.y % per_kv * hc, h0 = gk * grp + first, ncols = min(hc, grp - first);
+  const bool my_col = j < ncols;
+  const int pos = positions[t], lo = first_seen(pos, mask_kind, mask_size), lo_block = lo / 64, kept = kept_blocks(keep, lo_block);
+  float* dst = partial + (((long)t * heads + h0 + j) * n_chunks + blockIdx.z) * MAPS * (vdim + 2);
+  if ((int)blockIdx.z >= kept + pos / 64 - lo_block + 1) {        // no such block: nothing seen
+    if (my_col && g < MAPS) {
+      dst[g * (vdim + 2) + vdim] = -INFINITY;
+      dst[g * (vdim + 2) + vdim + 1] = 0.0f;
+    }
+    return;
+  }
+  const int b = nth_block(blockIdx.z, kept, lo_block), p0 = b * 64, in0 = p0 % page_size;
+  uint4 qv[MAPS * KC];                 // all of them asked for at once, ahead of the page's number
+#pragma unroll
+  for (int i = 0; i < MAPS * KC; ++i) {
+    const int idx = lane + 64 * i, col = idx / (MAPS * KC * 4), rest = idx % (MAPS * KC * 4), mp = rest / (KC * 4), sl = rest % (KC * 4);
+    qv[i] = make_uint4(0u, 0u, 0u, 0u);
+    if (col < ncols && 8 * sl < dim) qv[i] = *reinterpret_cast<const uint4*>(q + ((long)t * heads + h0 + col) * (MAPS * dim) + mp * dim + 8 * sl);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  const int kw = kv_heads * MAPS * dim, dt_n = vdim / 16;
+  const bf16_t* page = cache + (long)block_table[(long)seq_rows[t] * table_stride + p0 / page_size] * ((long)page_size * (kw + kv_heads * vdim));
+  const bf16_t* qlane = qs + j * QROW + 8 * g;
+  auto qfrag = [&](int mp, int c) { return *reinterpret_cast<const uint4*>(qlane + mp * QMAP + 32 * c); };
+  MaState<MAPS, DT> st;
+  st.clear();
+  auto stage_q = [&]() {               // behind the block's loads (one wave: its own writes are there when it reads)
+#pragma unroll
+    for (int i = 0; i < MAPS * KC; ++i) {
+      const int idx = lane + 64 * i, col = idx / (MAPS * KC * 4), rest = idx % (MAPS * KC * 4), mp = rest / (KC * 4), sl = rest % (KC * 4);
+      *reinterpret_cast<uint4*>(qs + col * QROW + mp * QMAP + 8 * sl) = qv[i];
+    }
+  };
+  if (!AHEAD) stage_q();
+  ma_block<MAPS, DT, KC, AHEAD, const bf16_t*>(st, page + (long)in0 * kw + (long)gk * MAPS * dim + 8 * g, kw,
+                         page + (long)page_size * kw + (long)gk * vdim * page_size + in0 + 4 * g, page_size, qfrag, p0, my_col ? lo : 0,
+                         my_col ? pos : -1, keep, ncols == 16 && (p0 >= lo || p0 + 63 < keep) && p0 + 63 <= pos, dim, dt_n, scale,
+                         softcap, j, g, stage_q);
+  if (!my_col) return;
+#pragma unroll
+  for (int mp = 0; mp < MAPS; ++mp) {
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+      if (dt < dt_n)
+        *reinterpret_cast<float2*>(dst + mp * (vdim + 2) + 16 * dt + 4 * g) = make_float2(st.acc[mp][dt][0], st.acc[mp][dt][1]),
+        *reinterpret_cast<float2*>(dst + mp * (vdim + 2) + 16 * dt + 4 * g + 2) = make_float2(st.acc[mp][dt][2], st.acc[mp][dt][3]);
+    if (g == 0) {
+      dst[mp * (vdim + 2) + vdim] = st.m[mp];
+      dst[mp * (vdim + 2) + vdim + 1] = st.l[mp];
+    }
+  }
+}
+
 // The blocks of a single token's (head, map) folded in ascending order, a_mp = sum_c e^(m_c - M) o_c /
 // sum_c e^(m_c - M) l_c (M the largest m_c; a block that saw nothing has l = 0 and weighs nothing), then
-// the maps combined, normed, gated and stored.  One wave per (tile, head); tiles of several tokens were
-// finished by the attention kernel itself.
-template <int MAPS>
+// the maps combined, normed, gated and stored.  One wave per (tile, head), OWN dims a lane; tiles of several tokens were
+// finished by the attention kernel itself.  Rows of blocks are asked for ROWS at a time, the first of them beside the weights.
+template <int MAPS, int OWN>
 __global__ void __launch_bounds__(64)
 masked_attention_fold_kernel(const float* __restrict__ partial, int n_chunks, const int32_t* __restrict__ tiles,
                              const float* __restrict__ gate, long gate_stride, bf16_t* __restrict__ out, int heads, int vdim,
                              float lambda, float out_scale, float eps, float sink_log2, int gate_per_head,
                              const float* __restrict__ sinks) {
+  constexpr int ROWS = OWN <= 4 ? 16 : 8;
   const int t = tiles ? tiles[2 * blockIdx.x] : (int)blockIdx.x, n = tiles ? tiles[2 * blockIdx.x + 1] : 1;
   if (n != 1) return;
   const int h = blockIdx.y, lane = threadIdx.x;
   if (sinks) sink_log2 = sinks[h] * 1.4426950408889634f;
-  float o[MA_OWN];
+  float gates[OWN];
+  if (gate != nullptr) {
 #pragma unroll
-  for (int i = 0; i < MA_OWN; ++i) o[i] = 0.0f;
+    for (int i = 0; i < OWN; ++i)
+      gates[i] = gate[(long)t * gate_stride + (gate_per_head ? (long)h : (long)h * vdim + min(lane + 64 * i, vdim - 1))];
+  }
+  float o[OWN];
+#pragma unroll
+  for (int i = 0; i < OWN; ++i) o[i] = 0.0f;
   for (int mp = 0; mp < MAPS; ++mp) {
     const float* src = partial + (((long)t * heads + h) * n_chunks * MAPS + mp) * (vdim + 2);
     const long step = (long)MAPS * (vdim + 2);
     // the blocks' (m, l) a lane each, 64 at a time; the largest maximum first, then weights handed round by lane
-    float M = -INFINITY;
-    for (int c0 = 0; c0 < n_chunks; c0 += 64) {
+    float m_first = -INFINITY, l_first = 0.0f;
+    if (lane < n_chunks) {
+      m_first = src[lane * step + vdim];
+      l_first = src[lane * step + vdim + 1];
+    }
+    float rows[ROWS][OWN];
+    auto ask = [&](int c0, int n_here) {      // (a row behind the last is the last again)
+#pragma unroll
+      for (int k = 0; k < ROWS; ++k) {
+        const float* row = src + (c0 + min(k, n_here - 1)) * step;
+#pragma unroll
+        for (int i = 0; i < OWN; ++i) rows[k][i] = row[min(lane + 64 * i, vdim - 1)];
+      }
+    };
+    ask(0, n_chunks);
+    float M = l_first > 0.0f ? m_first : -INFINITY;
+    for (int c0 = 64; c0 < n_chunks; c0 += 64) {
       const int c = c0 + lane;
       if (c < n_chunks && src[c * step + vdim + 1] > 0.0f) M = fmaxf(M, src[c * step + vdim]);
     }
     M = wave_max(M);
-    float L = 0.0f, acc[MA_OWN];
+    float L = 0.0f, acc[OWN];
 #pragma unroll
-    for (int i = 0; i < MA_OWN; ++i) acc[i] = 0.0f;
+    for (int i = 0; i < OWN; ++i) acc[i] = 0.0f;
     for (int c0 = 0; c0 < n_chunks; c0 += 64) {
       const int c = c0 + lane;
-      const float lc = c < n_chunks ? src[c * step + vdim + 1] : 0.0f;
-      const float w = lc > 0.0f ? exp2f(src[c * step + vdim] - M) : 0.0f;      // the blocks' maxima are in units of log2 e
+      const float lc = c0 == 0 ? l_first : c < n_chunks ? src[c * step + vdim + 1] : 0.0f;
+      const float w = lc > 0.0f ? exp2f((c0 == 0 ? m_first : src[c * step + vdim]) - M) : 0.0f;      // the blocks' maxima are in units of log2 e
       L += wave_sum(w * lc);
-      // eight blocks' rows asked for together (a row beyond the last is the last again and weighs nothing)
-      const int n_here = min(64, n_chunks - c0);
-      for (int k0 = 0; k0 < n_here; k0 += 8) {
-        float rows[8][MA_OWN];
+      // the rows of blocks behind the last that saw something were not written
+      const unsigned long long some = __ballot(lc > 0.0f);
+      const int n_here = some == 0 ? 0 : 64 - __builtin_clzll(some);
+      for (int k0 = 0; k0 < n_here; k0 += ROWS) {
+        if (c0 + k0 > 0) ask(c0 + k0, n_here - k0);
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-          const float* row = src + (c0 + min(k0 + k, n_here - 1)) * step;
+        for (int k = 0; k < ROWS; ++k) {
+          const float wk = __shfl(w, k0 + k, 64);
+          if (k0 + k < n_here) {
 #pragma unroll
-          for (int i = 0; i < MA_OWN; ++i) rows[k][i] = row[min(lane + 64 * i, vdim - 1)];
-        }
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-          const float wk = k0 + k < n_here ? __shfl(w, k0 + k, 64) : 0.0f;
-#pragma unroll
-          for (int i = 0; i < MA_OWN; ++i) acc[i] = fmaf(wk, rows[k][i], acc[i]);
+            for (int i = 0; i < OWN; ++i) acc[i] = fmaf(wk, rows[k][i], acc[i]);
+          }
         }
       }
     }
     if (sink_log2 > -INFINITY) L += exp2f(sink_log2 - M);
     const float inv = 1.0f / L;
 #pragma unroll
-    for (int i = 0; i < MA_OWN; ++i) {
+    for (int i = 0; i < OWN; ++i) {
       const float a = lane + 64 * i < vdim ? acc[i] * inv : 0.0f;      // places beyond vdim hold copies: they count as 0
       o[i] = mp == 0 ? a : o[i] - lambda * a;
     }
@@ -670,18 +775,18 @@ masked_attention_fold_kernel(const float* __restrict__ partial, int n_chunks, co
   if (MAPS > 1) {
     float ss = 0.0f;
 #pragma unroll
-    for (int i = 0; i < MA_OWN; ++i) ss = fmaf(o[i], o[i], ss);
+    for (int i = 0; i < OWN; ++i) ss = fmaf(o[i], o[i], ss);
     const float inv = 1.0f / sqrtf(wave_sum(ss) / (float)vdim + eps);
 #pragma unroll
-    for (int i = 0; i < MA_OWN; ++i) o[i] = (o[i] * inv) * out_scale;
+    for (int i = 0; i < OWN; ++i) o[i] = (o[i] * inv) * out_scale;
   }
   bf16_t* dst = out + ((long)t * heads + h) * vdim;
 #pragma unroll
-  for (int i = 0; i < MA_OWN; ++i) {
+  for (int i = 0; i < OWN; ++i) {
     const int d = lane + 64 * i;
     if (d >= vdim) continue;
     float v = o[i];
-    if (gate != nullptr) v *= 1.0f / (1.0f + expf(-gate[(long)t * gate_stride + (gate_per_head ? (long)h : (long)h * vdim + d)]));
+    if (gate != nullptr) v *= 1.0f / (1.0f + expf(-gates[i]));
     dst[d] = from_float(v);
   }
 }
@@ -789,9 +894,9 @@ masked_attention_staged_kernel(const bf16_t* __restrict__ q, const bf16_t* __res
     if (nb + 1 < n_blocks) fetch(nth_block(nb + 1, kept, lo_block));
     const int p0 = nth_block(nb, kept, lo_block) * 64;
     if (active)
-      ma_block<MAPS, DT, KC, ma_lds_cptr>(st, ks + 8 * g, krow, vs + 4 * g, vrow, qfrag, p0, my_lo, my_pos,
+      ma_block<MAPS, DT, KC, false, ma_lds_cptr>(st, ks + 8 * g, krow, vs + 4 * g, vrow, qfrag, p0, my_lo, my_pos,
                              keep, ncols == 16 && (p0 >= lo_last || p0 + 63 < keep) && p0 + 63 <= pos_first, dim, dt_n, scale, softcap,
-                             j, g);
+                             j, g, [] {});
   }
   if (active)
     ma_finish<MAPS, DT>(st, my_col, my_tok, my_head, heads, vdim, dt_n, gate, gate_stride, out, lambda, out_scale, eps, g, sink_log2,
@@ -833,14 +938,27 @@ static int launch_masked_mfma(const void* q, const void* cache, const int32_t* b
     return 0;
   }
   const int n_chunks = partial ? masked_chunks(mask_kind, mask_size, keep, span) : 1;
-  masked_attention_mfma_kernel<MAPS, DT, KC><<<dim3(n_tiles, heads, n_chunks), 64, 0, stream>>>(
-      (const bf16_t*)q, (const bf16_t*)cache, block_table, table_stride, positions, seq_rows, gate, gate_stride, (bf16_t*)out, tiles,
-      heads, kv_heads, dim, vdim, page_size, mask_kind, mask_size, scale, softcap, lambda, out_scale, eps, partial, n_chunks,
-      sink_log2, gate_per_head, keep, sinks);
-  if (partial)
-    masked_attention_fold_kernel<MAPS><<<dim3(n_tiles, heads), 64, 0, stream>>>(partial, n_chunks, tiles, gate, gate_stride,
-                                                                              (bf16_t*)out, heads, vdim, lambda, out_scale, eps,
-                                                                              sink_log2, gate_per_head, sinks);
+  if (tiles == nullptr && partial != nullptr) {
+    const int hc = grp < 16 ? grp : 16;
+    masked_attention_blocks_kernel<MAPS, DT, KC><<<dim3(n_tiles, kv_heads * ((grp + hc - 1) / hc), n_chunks), 64, 0, stream>>>(
+        (const bf16_t*)q, (const bf16_t*)cache, block_table, table_stride, positions, seq_rows, heads, kv_heads, dim, vdim, page_size,
+        mask_kind, mask_size, scale, softcap, partial, n_chunks, keep);
+  } else {
+    masked_attention_mfma_kernel<MAPS, DT, KC><<<dim3(n_tiles, heads, n_chunks), 64, 0, stream>>>(
+        (const bf16_t*)q, (const bf16_t*)cache, block_table, table_stride, positions, seq_rows, gate, gate_stride, (bf16_t*)out, tiles,
+        heads, kv_heads, dim, vdim, page_size, mask_kind, mask_size, scale, softcap, lambda, out_scale, eps, partial, n_chunks,
+        sink_log2, gate_per_head, keep, sinks);
+  }
+  if (partial) {
+#define MA_FOLD(OWN)                                                                                                            \
+  masked_attention_fold_kernel<MAPS, OWN><<<dim3(n_tiles, heads), 64, 0, stream>>>(partial, n_chunks, tiles, gate, gate_stride, \
+                                                                                   (bf16_t*)out, heads, vdim, lambda, out_scale, eps, \
+                                                                                   sink_log2, gate_per_head, sinks)
+    if (vdim <= 64) MA_FOLD(1);
+    else if (vdim <= 128) MA_FOLD(2);
+    else MA_FOLD(4);
+#undef MA_FOLD
+  }
   return 0;
 }
 #endif
