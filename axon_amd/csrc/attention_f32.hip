@@ -64,13 +64,17 @@ __device__ __forceinline__ int page_index(int p, int page_size) { return p >> (3
 __device__ __forceinline__ int page_offset(int p, int page_size) { return p & (page_size - 1); }
 
 // ============================================================================ prompt portions
-// A block takes 64 tokens (four waves of 16) of a tile and one query head and walks their blocks of
+// A block takes 32 tokens of a tile and one query head and walks their blocks of
 // positions; a block's K [64][HD] and V^T [HD][64] go through LDS, rows in the order [16 k][q][i] so that
 // a 16-byte read is a lane's operand of four products, rows a multiple of 16 bytes and an odd number
 // of them apart (16 rows fall into 16 slots of the 64 banks).  The next block's numbers are asked for
-// while this one is multiplied.  grid (pairs of tiles, heads, 4): which tile of the pair and which half of it.
-// Bound by the products (2 x 128 of 32 cycles a wave and block at head size 128) of the tokens that see most:
-// 16 heads, 777 tokens 806 -> 95 us (the kernel of a wave a token and head before), 2,048 tokens 4,514 -> 258 us, 67 TFLOP/s.
+// while this one is multiplied.  Sixteen tokens have two waves: each scores half of the positions, the scores meet in LDS, both
+// work out the weights and each sums half of the dims, so that the tokens that see most, which a prompt waits for, take half as
+// long.  grid (pairs of tiles, heads, 8): which tile of the pair and which quarter of it.
+// Bound by the tokens that see most: a wave's 128 products of 32 cycles a block of positions (head size 128) are a third of its
+// time, behind them stand the stage's writes, the exponentials and three barriers.  16 heads, us, 64 tokens a block and a wave
+// for sixteen of them / here: 777 tokens 105 / 70, three requests of 100 to 341 53 / 37, 200 tokens 36 / 23, 2,048 tokens 260 / 257
+// (67 TFLOP/s; twice the stages, no more blocks than the chip holds).
 template <int HD>
 __global__ void __launch_bounds__(256, 2)
 attention_f32_prefill_kernel(const float* __restrict__ q, int q_stride, const float* __restrict__ k_cache,
@@ -78,18 +82,20 @@ attention_f32_prefill_kernel(const float* __restrict__ q, int q_stride, const fl
                              const int32_t* __restrict__ positions, const int32_t* __restrict__ seq_rows,
                              float* __restrict__ out, const int32_t* __restrict__ tiles, int n_heads, int n_kv_heads,
                              int page_size, int window, float scale) {
-  constexpr int KG = HD / 16, DT = HD / 16, K_LD = HD + 4, V_LD = ATT_BLOCK + 4, LOADS = ATT_BLOCK * HD / 4 / 256;
-  extern __shared__ __align__(16) float smem[];      // K [64][K_LD], V^T [HD][V_LD]
+  constexpr int KG = HD / 16, DT = HD / 16, K_LD = HD + 4, V_LD = ATT_BLOCK + 4, DH = DT / 2, LOADS = ATT_BLOCK * HD / 4 / 256;
+  extern __shared__ __align__(16) float smem[];      // K [64][K_LD], V^T [HD][V_LD], the scores of the waves' tiles [4][2][64][4]
   float* ks = smem;
   float* vs = smem + ATT_BLOCK * K_LD;
-  const int32_t* mine = tiles + 4 * blockIdx.x + 2 * (blockIdx.z >> 1);
-  const int skip = 64 * (blockIdx.z & 1), count = mine[1] - skip, t0 = mine[0] + skip;
+  f32x4* scores = reinterpret_cast<f32x4*>(vs + HD * V_LD);
+  const int32_t* mine = tiles + 4 * blockIdx.x + 2 * (blockIdx.z >> 2);
+  const int skip = 32 * (blockIdx.z & 3), count = mine[1] - skip, t0 = mine[0] + skip;
   if (count <= 0) return;                            // the same for the whole block
   const int head = blockIdx.y, kvh = head / (n_heads / n_kv_heads);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r16 = lane & 15, g4 = lane >> 4;
-  const int n = min(count, 64), first_pos = positions[t0], last_pos = positions[t0 + n - 1];
-  const bool wave_live = 16 * wave < n;
-  const int row = t0 + min(16 * wave + r16, n - 1), pos = positions[row];
+  const int group = wave >> 1, half = __builtin_amdgcn_readfirstlane(wave & 1), d0 = half * DH;
+  const int n = min(count, 32), first_pos = positions[t0], last_pos = positions[t0 + n - 1];
+  const bool wave_live = 16 * group < n;
+  const int row = t0 + min(16 * group + r16, n - 1), pos = positions[row];
   const int lo = window > 0 ? max(0, pos + 1 - window) : 0;
   const int from = window > 0 ? max(0, first_pos + 1 - window) : 0, upto = window > 0 ? max(0, last_pos + 1 - window) : 0;
   const int32_t* table_row = block_table + (size_t)seq_rows[t0] * table_stride;
@@ -118,9 +124,9 @@ attention_f32_prefill_kernel(const float* __restrict__ q, int q_stride, const fl
     }
   };
   float M = -INFINITY, L = 0.0f;
-  f32x4 O[DT];
+  f32x4 O[DH];
 #pragma unroll
-  for (int d = 0; d < DT; ++d) O[d] = F32_ZERO;
+  for (int d = 0; d < DH; ++d) O[d] = F32_ZERO;
 
   const int b_end = last_pos / ATT_BLOCK;
   fetch(from / ATT_BLOCK * ATT_BLOCK);
@@ -150,43 +156,50 @@ attention_f32_prefill_kernel(const float* __restrict__ q, int q_stride, const fl
     const bool spoiled = whole ? (__syncthreads(), false) : __syncthreads_or(odd);
     if (b < b_end) fetch(p0 + ATT_BLOCK);
     const bool seen = p0 <= pos && p0 + ATT_BLOCK - 1 >= lo;               // by this lane's token
-    if (!wave_live || !__any(seen)) continue;
+    const bool works = wave_live && __any(seen);                           // the same for both waves of sixteen tokens
 
     f32x4 s[4] = {F32_ZERO, F32_ZERO, F32_ZERO, F32_ZERO};
+    if (works) {
+      f32x4 part[2] = {F32_ZERO, F32_ZERO};
 #pragma unroll
-    for (int g = 0; g < KG; ++g) {
-      f32x4 a[4];
+      for (int g = 0; g < KG; ++g) {
+        f32x4 a[2];
 #pragma unroll
-      for (int t = 0; t < 4; ++t) a[t] = *reinterpret_cast<const f32x4*>(&ks[(16 * t + r16) * K_LD + 16 * g + 4 * g4]);
+        for (int t = 0; t < 2; ++t) a[t] = *reinterpret_cast<const f32x4*>(&ks[(32 * half + 16 * t + r16) * K_LD + 16 * g + 4 * g4]);
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int t = 0; t < 4; ++t) F32_STEP(s[t], a[t], qf[g], i);
+          for (int t = 0; t < 2; ++t) F32_STEP(part[t], a[t], qf[g], i);
+      }
+#pragma unroll
+      for (int t = 0; t < 2; ++t) scores[(2 * wave + t) * 64 + lane] = part[t];
     }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");        // the next block's loads stay under way
+    if (!works) continue;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) s[t] = scores[(4 * group + t) * 64 + lane];
     float m_b, l_b;
     f32_weights(s, p0, lo, pos, scale, g4, m_b, l_b);
-    f32x4 o[DT];
+    f32x4 o[DH];
     if (!spoiled) {
       f32x4 pf[4];
 #pragma unroll
       for (int t = 0; t < 4; ++t) pf[t] = f32_operand(s[t]);
 #pragma unroll
-      for (int d = 0; d < DT; ++d) o[d] = F32_ZERO;
+      for (int d = 0; d < DH; ++d) o[d] = F32_ZERO;
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
+      for (int t = 0; t < 4; ++t) {
+        f32x4 a[DH];
 #pragma unroll
-        for (int dh = 0; dh < DT; dh += 4) {
-          f32x4 a[4];
+        for (int d = 0; d < DH; ++d) a[d] = *reinterpret_cast<const f32x4*>(&vs[(16 * (d0 + d) + r16) * V_LD + 16 * t + 4 * g4]);
 #pragma unroll
-          for (int d = 0; d < 4; ++d) a[d] = *reinterpret_cast<const f32x4*>(&vs[(16 * (dh + d) + r16) * V_LD + 16 * t + 4 * g4]);
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int d = 0; d < 4; ++d) F32_STEP(o[dh + d], a[d], pf[t], i);
-        }
+          for (int d = 0; d < DH; ++d) F32_STEP(o[d], a[d], pf[t], i);
+      }
     } else {
 #pragma unroll
-      for (int d = 0; d < DT; ++d) o[d] = F32_ZERO;
+      for (int d = 0; d < DH; ++d) o[d] = F32_ZERO;
 #pragma unroll
       for (int t = 0; t < 4; ++t)
         for (int g = 0; g < 4; ++g)
@@ -196,9 +209,9 @@ attention_f32_prefill_kernel(const float* __restrict__ q, int q_stride, const fl
             const float w = __shfl(s[t][e], r16 + 16 * g, AXON_WAVE);
             if (p0 + place < lo || p0 + place > pos) continue;
 #pragma unroll
-            for (int d = 0; d < DT; ++d)
+            for (int d = 0; d < DH; ++d)
 #pragma unroll
-              for (int r = 0; r < 4; ++r) o[d][r] = fmaf(w, vs[(16 * d + 4 * g4 + r) * V_LD + 16 * t + 4 * e + g], o[d][r]);
+              for (int r = 0; r < 4; ++r) o[d][r] = fmaf(w, vs[(16 * (d0 + d) + 4 * g4 + r) * V_LD + 16 * t + 4 * e + g], o[d][r]);
           }
     }
     const float mn = fmaxf(M, m_b), alpha = expf(M - mn), wgt = expf(m_b - mn);
@@ -206,16 +219,16 @@ attention_f32_prefill_kernel(const float* __restrict__ q, int q_stride, const fl
       L = fmaf(l_b, wgt, L * alpha);
       M = mn;
 #pragma unroll
-      for (int d = 0; d < DT; ++d)
+      for (int d = 0; d < DH; ++d)
 #pragma unroll
         for (int r = 0; r < 4; ++r) O[d][r] = fmaf(o[d][r], wgt, O[d][r] * alpha);
     }
   }
-  if (16 * wave + r16 >= n) return;
+  if (16 * group + r16 >= n) return;
   float* orow = out + ((size_t)row * n_heads + head) * HD;
 #pragma unroll
-  for (int d = 0; d < DT; ++d)
-    *reinterpret_cast<f32x4*>(orow + 16 * d + 4 * g4) = f32x4{O[d][0] / L, O[d][1] / L, O[d][2] / L, O[d][3] / L};
+  for (int d = 0; d < DH; ++d)
+    *reinterpret_cast<f32x4*>(orow + 16 * (d0 + d) + 4 * g4) = f32x4{O[d][0] / L, O[d][1] / L, O[d][2] / L, O[d][3] / L};
 }
 
 // ============================================================================ decoding tokens
@@ -401,7 +414,7 @@ int launch_attention_f32_prefill(const float* q, int q_stride, const float* k_ca
                                  int n_kv_heads, int head_dim, int page_size, int window, float scale, hipStream_t stream) {
 #define LAUNCH(HD)                                                                                                   \
   {                                                                                                                  \
-    constexpr int lds = (ATT_BLOCK * (HD + 4) + HD * (ATT_BLOCK + 4)) * (int)sizeof(float);                          \
+    constexpr int lds = (ATT_BLOCK * (HD + 4) + HD * (ATT_BLOCK + 4) + 4 * 2 * 64 * 4) * (int)sizeof(float);                          \
     static bool configured = lds <= 48 * 1024;                                                                       \
     if (!configured) {                                                                                               \
       hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attention_f32_prefill_kernel<HD>),           \
@@ -413,7 +426,7 @@ int launch_attention_f32_prefill(const float* q, int q_stride, const float* k_ca
       configured = true;                                                                                             \
     }                                                                                                                \
     AXK_INSTANCE(INST_ATTENTION_F32_PREFILL, HD);                                                                    \
-    attention_f32_prefill_kernel<HD><<<dim3(n_tiles, n_heads, 4), 256, lds, stream>>>(                               \
+    attention_f32_prefill_kernel<HD><<<dim3(n_tiles, n_heads, 8), 256, lds, stream>>>(                               \
         q, q_stride, k_cache, v_cache, block_table, table_stride, positions, seq_rows, out, tiles, n_heads,          \
         n_kv_heads, page_size, window, scale);                                                                       \
   }
