@@ -477,52 +477,77 @@ gemm_fma_by_chain_kernel(const elem_t* __restrict__ x, int x_stride, const elem_
 // the next chain's products.  A row of a stage is eight slots of 16 bytes, permuted by slot ^ (row / 2 % 8): the four k of 16
 // rows that a read takes fall on the 64 banks.
 // What bounds it: with four blocks a CU 83 % of what the products alone take (139 TFLOP/s at the clock that they leave); with one or two
-// blocks a CU also how they divide the rows (777 rows: 13 of 64, two rounds of 416 blocks or 1.6).
+// blocks a CU also how they divide the rows, so a block has 32 to 96 of them (flow_rows).
 // 777 rows, us, through registers / here: 2,560 x K 2,048 121 / 114, 2,048 x 2,060 89 / 76, 2,048 x 5,632 234 / 198, gated 5,632 x
 // 2,048 338 / 329, 32,000 x 2,048 960 / 942; 512 rows of 2,048 x 5,632 (a block a CU) 142 / 116, 2,048 rows 414 / 393.  With a read a
 // number (128 LDS instructions a block and step) 409 for the last, three stages (three blocks a CU) 412.
 #define FLOW_STAGES 4
-#define FLOW_STAGE (2 * TILE_M * FMA_PART * 4)
+#define FLOW_STAGE(rows) (((rows) + TILE_M) * FMA_PART * 4)
 #define FLOW_LEAST_K 192      // (launch_fma_tiles)
 typedef const __attribute__((address_space(1))) void* fma_global_t;
 typedef __attribute__((address_space(3))) void* fma_lds_t;
 typedef __attribute__((ext_vector_type(2))) float f32x2;
-// The numbers at an address and 2 KB, 16 rows of a stage, behind it.
-__device__ __forceinline__ void lds_read_two(f32x2& dst, unsigned lds_address) {
-  asm volatile("ds_read2st64_b32 %0, %1 offset0:0 offset1:8" : "=v"(dst) : "v"(lds_address));
-}
-__device__ __forceinline__ void use_numbers(f32x2& v) { asm volatile("" : "+v"(v)); }
+// A product's operand of TILES tiles: a lane's number of each, read two tiles at a time, 2 KB (16 rows of a stage) apart, and the
+// last of an odd number alone.
+template <int TILES>
+struct FmaOperand {
+  static constexpr int PAIRS = (TILES + 1) / 2;
+  f32x2 two[TILES > 1 ? TILES / 2 : 1];
+  float one;
+  __device__ __forceinline__ float number(int i) const { return TILES % 2 && i == TILES - 1 ? one : two[i / 2][i % 2]; }
+  // read `pair` of the PAIRS
+  template <int I = PAIRS - 1>
+  __device__ __forceinline__ void read(unsigned lds_address, int pair) {
+    if (pair == I) {
+      if constexpr (TILES % 2 && I == PAIRS - 1) asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(one) : "v"(lds_address), "n"(I * 4096));
+      else asm volatile("ds_read2st64_b32 %0, %1 offset0:%2 offset1:%3" : "=v"(two[I]) : "v"(lds_address), "n"(I * 16), "n"(I * 16 + 8));
+    } else if constexpr (I > 0) {
+      read<I - 1>(lds_address, pair);
+    }
+  }
+  __device__ __forceinline__ void use() {
+#pragma unroll
+    for (int i = 0; i < TILES / 2; ++i) asm volatile("" : "+v"(two[i]));
+    if constexpr (TILES % 2) asm volatile("" : "+v"(one));
+  }
+};
 template <int V>
 struct FmaNumber {
   static constexpr int value = V;
 };
-template <bool GLU>
-__global__ void __launch_bounds__(256, 2)
+// WAVES_M x (4 / WAVES_M) waves, each TM x TN tiles of 16 x 16: 16 WAVES_M TM rows by 64 rows of W a block.
+template <bool GLU, int WAVES_M, int TM, int TN>
+__global__ void __launch_bounds__(256, TM * TN <= 6 ? 2 : 1)
 gemm_fma_flow_kernel(const float* __restrict__ x, int x_stride, const float* __restrict__ w, const void* __restrict__ bias,
                      int bias_is_f32, void* __restrict__ out, int out_stride, int M, int N, int K, int mode) {
-  constexpr int R = 2, BM = TILE_M, BN = GLU ? BM / 2 : BM;
-  extern __shared__ __align__(128) unsigned char flow[];          // [stage]: X [64][32], W [64][32]
+  constexpr int BM = 16 * WAVES_M * TM, BN = GLU ? TILE_M / 2 : TILE_M, STAGE = FLOW_STAGE(BM), PRODUCTS = 8 * TM * TN;
+  constexpr int XL = (BM / 8 + 3) / 4, LOADS = XL + 2;           // load instructions of a wave and stage: of X, with W's two
+  constexpr int PAIRS = FmaOperand<TM>::PAIRS, READS = 8 * (PAIRS + 1), EACH = (2 * READS + PRODUCTS - 1) / PRODUCTS;
+  static_assert(4 / WAVES_M * TN * 16 == TILE_M && (!GLU || TN == 2) && LOADS * FLOW_STAGES < 64, "64 rows of W a block");
+  extern __shared__ __align__(128) unsigned char flow[];          // [stage]: X [BM][32], W [64][32]
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
   const int r16 = lane & 15, q = lane >> 4;
-  const int wm = (wave >> 1) * 16 * R, wn = (wave & 1) * 16 * R;
+  const int wm = WAVES_M == 2 ? (wave >> 1) * 16 * TM : 0, wn = (WAVES_M == 2 ? wave & 1 : wave) * 16 * TN;
 
-  // A load fills 8 rows of a stage, lane l slot l % 8 of row l / 8, which holds k chunk slot ^ (row / 2 % 8): loads 0 and 1 rows
-  // 8 (4 j + wave) and on of X, loads 2 and 3 the same of W (gated: in a wave's 32 rows 16 gate rows, then the up rows of the same outputs)
-  const int lrow = lane >> 3, chunk = (lane & 7) ^ ((4 * wave + (lane >> 4)) & 7);
+  // A load fills 8 rows of a stage, lane l slot l % 8 of row l / 8, which holds k chunk slot ^ (row / 2 % 8): loads 0 .. XL - 1 rows
+  // 8 (4 j + wave) and on of X (where there are none: some twice), the last two the same of W (gated: in a wave's 32 rows 16 gate
+  // rows, then the up rows of the same outputs)
+  const int lrow = lane >> 3;
   const bool up = GLU && (wave & 2);
   const FmaRows x_rows = fma_rows(x, m0, M, x_stride, K);
   const FmaRows w_rows = fma_rows(w + (up ? (size_t)N * K : 0), n0, N, K, K);
-  unsigned at[4];
+  auto group = [&](int j) { return j < XL ? min(4 * j + wave, BM / 8 - 1) : 4 * (j - XL) + wave; };
+  unsigned at[LOADS];
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int row = 8 * (4 * j + wave) + lrow, col = GLU ? 16 * j + 8 * (wave & 1) + lrow : row;
-    at[j] = ((unsigned)min(row, M - 1 - m0) * (unsigned)x_stride + 4 * chunk) * 4;
-    at[2 + j] = ((unsigned)min(col, N - 1 - n0) * (unsigned)K + 4 * chunk) * 4;
+  for (int j = 0; j < LOADS; ++j) {
+    const int row = 8 * group(j) + lrow, chunk = (lane & 7) ^ ((4 * group(j) + (lane >> 4)) & 7);
+    const int col = GLU ? 16 * (j - XL) + 8 * (wave & 1) + lrow : row;
+    at[j] = (j < XL ? (unsigned)min(row, M - 1 - m0) * (unsigned)x_stride : (unsigned)min(col, N - 1 - n0) * (unsigned)K) * 4 + 16 * chunk;
   }
   auto ask = [&](int t, int j) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds((j < 2 ? x_rows : w_rows).from(t * FMA_PART),
-                                             (fma_lds_t)(flow + t % FLOW_STAGES * FLOW_STAGE + (j < 2 ? 0 : BM * 128) + (4 * (j & 1) + wave) * 1024), 16,
+    __builtin_amdgcn_raw_ptr_buffer_load_lds((j < XL ? x_rows : w_rows).from(t * FMA_PART),
+                                             (fma_lds_t)(flow + t % FLOW_STAGES * STAGE + (j < XL ? 0 : BM * 128) + group(j) * 1024), 16,
                                              (int)at[j], 0, 0, 0);
   };
   const unsigned lds0 = (unsigned)(size_t)(fma_lds_t)flow;
@@ -532,65 +557,67 @@ gemm_fma_flow_kernel(const float* __restrict__ x, int x_stride, const float* __r
     x_at[s] = lds0 + (wm + r16) * 128 + ((s ^ (r16 >> 1)) << 4) + 4 * q;
     w_at[s] = x_at[s] + BM * 128 + (wn - wm) * 128;
   }
-  f32x2 a[2][8], b[2][8];                  // of a wave's two tiles
-  // read p of the 16 of a stage: X's and W's numbers of product p / 2
+  FmaOperand<TM> a[2][8];                  // of a wave's tiles
+  FmaOperand<TN> b[2][8];
+  // read p of those of a stage: X's and W's numbers of product p / (PAIRS + 1)
   auto read = [&](auto set_of, unsigned stage, int p) {
     constexpr int set = decltype(set_of)::value;
-    if (p % 2 == 0) lds_read_two(a[set][p / 2], x_at[p / 2] + stage);
-    else lds_read_two(b[set][p / 2], w_at[p / 2] + stage);
+    const int s = p / (PAIRS + 1), of = p % (PAIRS + 1);
+    if (of < PAIRS) a[set][s].read(x_at[s] + stage, of);
+    else b[set][s].read(w_at[s] + stage, 0);
   };
   auto arrived = [&](auto set_of) {
     constexpr int set = decltype(set_of)::value;
     wait_lgkmcnt<0>();
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
-      use_numbers(a[set][s]);
-      use_numbers(b[set][s]);
+      a[set][s].use();
+      b[set][s].use();
     }
   };
-  f32x4 sum[R][R], acc[2][R][R];
+  f32x4 sum[TM][TN], acc[2][TM][TN];
 #pragma unroll
-  for (int i = 0; i < R; ++i)
+  for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < R; ++j) sum[i][j] = acc[1][i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int j = 0; j < TN; ++j) sum[i][j] = acc[1][i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
   const int n_steps = (K + FMA_PART - 1) / FMA_PART;
   static_assert(FLOW_LEAST_K > FLOW_STAGES * FMA_PART, "as many steps as stages");
 #pragma unroll
   for (int t = 0; t < FLOW_STAGES; ++t)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) ask(t, j);
-  wait_vmcnt<4 * (FLOW_STAGES - 1)>();
+    for (int j = 0; j < LOADS; ++j) ask(t, j);
+  wait_vmcnt<LOADS*(FLOW_STAGES - 1)>();
   __builtin_amdgcn_s_barrier();            // stage 0 is in LDS for every wave
 #pragma unroll
-  for (int p = 0; p < 16; ++p) read(FmaNumber<0>(), 0u, p);
+  for (int p = 0; p < READS; ++p) read(FmaNumber<0>(), 0u, p);
   arrived(FmaNumber<0>());
   // Step t, whose numbers are in registers: its stage is free behind the barrier.  asks: for stage t + FLOW_STAGES.
   auto step = [&](int t, auto set_of, auto asks_of) {
     constexpr int set = decltype(set_of)::value, other = set ^ 1;
     constexpr bool asks = decltype(asks_of)::value != 0;
     if constexpr (asks) {
-      wait_vmcnt<4 * (FLOW_STAGES - 2)>();
+      wait_vmcnt<LOADS*(FLOW_STAGES - 2)>();
     } else {
       const int left = n_steps - t;        // of the stages behind the next, left - 2 may still be under way
-      if (FLOW_STAGES >= 4 && left >= 4) wait_vmcnt<8>();
-      else if (left >= 3) wait_vmcnt<4>();
+      if (FLOW_STAGES >= 4 && left >= 4) wait_vmcnt<2 * LOADS>();
+      else if (left >= 3) wait_vmcnt<LOADS>();
       else wait_vmcnt<0>();
     }
     __builtin_amdgcn_s_barrier();          // stage t + 1 is in LDS for every wave; nobody reads stage t any more
-    const unsigned next = (unsigned)((t + 1) % FLOW_STAGES * FLOW_STAGE);
+    const unsigned next = (unsigned)((t + 1) % FLOW_STAGES * STAGE);
 #pragma unroll
-    for (int p = 0; p < 8 * R * R; ++p) {
-      const int s = p / (R * R), i = p / R % R, j = p % R;
+    for (int p = 0; p < PRODUCTS; ++p) {
+      const int s = p / (TM * TN), i = p / TN % TM, j = p % TN;
       if (s == 0) acc[set][i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-      acc[set][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[set][s][i], b[set][s][j], acc[set][i][j], 0, 0, 0);
+      acc[set][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[set][s].number(i), b[set][s].number(j), acc[set][i][j], 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
-      if (p < 8) {                         // as soon as they go: spread over 16, 24 or 32 products they take 1 to 5 % longer
-        read(FmaNumber<other>(), next, 2 * p);
-        read(FmaNumber<other>(), next, 2 * p + 1);
-      }
-      if (p >= 16 && p < 20) sum[(p - 16) / R][p % R] += acc[other][(p - 16) / R][p % R];      // the chain before
-      if (asks && p >= 20 && p % 3 == 0) ask(t + FLOW_STAGES, (p - 21) / 3);
+#pragma unroll
+      for (int r = p * EACH; r < (p + 1) * EACH; ++r)      // as soon as they go: spread over more products they take 1 to 5 % longer
+        if (r < READS) read(FmaNumber<other>(), next, r);
+      constexpr int HALF = PRODUCTS / 2;
+      if (p >= HALF && p < HALF + TM * TN) sum[(p - HALF) / TN][p % TN] += acc[other][(p - HALF) / TN][p % TN];      // the chain before
+      if (asks && (PRODUCTS - 1 - p) % 3 == 0 && (PRODUCTS - 1 - p) / 3 < LOADS) ask(t + FLOW_STAGES, LOADS - 1 - (PRODUCTS - 1 - p) / 3);
       __builtin_amdgcn_sched_barrier(0);
     }
     arrived(FmaNumber<other>());           // (behind the last step: whatever lies there, not used)
@@ -614,9 +641,9 @@ gemm_fma_flow_kernel(const float* __restrict__ x, int x_stride, const float* __r
     constexpr int set = decltype(set_of)::value;
     const int count = (K - whole * FMA_PART) / 4;
 #pragma unroll
-    for (int i = 0; i < R; ++i)
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int j = 0; j < R; ++j) {
+      for (int j = 0; j < TN; ++j) {
         sum[i][j] += acc[set ^ 1][i][j];
         acc[set][i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
       }
@@ -624,14 +651,15 @@ gemm_fma_flow_kernel(const float* __restrict__ x, int x_stride, const float* __r
     for (int s = 0; s < 8; ++s)
       if (s < count) {
 #pragma unroll
-        for (int i = 0; i < R; ++i)
+        for (int i = 0; i < TM; ++i)
 #pragma unroll
-          for (int j = 0; j < R; ++j) acc[set][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[set][s][i], b[set][s][j], acc[set][i][j], 0, 0, 0);
+          for (int j = 0; j < TN; ++j)
+            acc[set][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[set][s].number(i), b[set][s].number(j), acc[set][i][j], 0, 0, 0);
       }
 #pragma unroll
-    for (int i = 0; i < R; ++i)
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int j = 0; j < R; ++j) sum[i][j] += acc[set][i][j];
+      for (int j = 0; j < TN; ++j) sum[i][j] += acc[set][i][j];
   };
   if (t < whole) {                         // t is even: one whole step, and what may be left
     step(t, FmaNumber<0>(), FmaNumber<0>());
@@ -640,9 +668,9 @@ gemm_fma_flow_kernel(const float* __restrict__ x, int x_stride, const float* __r
     last(FmaNumber<0>());
   }
 
-  constexpr int COLS = GLU ? R / 2 : R;
+  constexpr int COLS = GLU ? TN / 2 : TN;
 #pragma unroll
-  for (int i = 0; i < R; ++i)
+  for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < COLS; ++j)
 #pragma unroll
@@ -701,8 +729,54 @@ static void launch_fma_few(const elem_t* x, int x_stride, const elem_t* w, const
 #undef FEW
 }
 
+#if !AXON_BF16
+// Rows a block of gemm_fma_flow_kernel: what takes least by how many blocks the fullest CU then has: of one `alone`, of more
+// `each` for every one and `odd` where one stays without its neighbour (us for K 2,048, measured with 2,048, 2,560 and 8,192
+// columns and gated 5,632 at 129 to 2,048 rows, all within 5 % of it; of 32 rows the first three blocks take 5 more).  64 rows of all / so, K 2,048: 2,048
+// columns, 129 and 200 rows 47 / 30, 300 48 / 40, 626 76 / 56, 1,500 118 / 105; 2,560 columns, 430 rows 76 / 56, 777 117 / 84, 1,024
+// 117 / 101; gated 5,632, 129 rows 117 / 86, 900 405 / 367, 1,500 620 / 570.  Blocks of 112 and of 128 rows, one a CU, are the best of none.
+static int flow_rows(int columns, int m, bool glu) {
+  int best = 0;
+  double least = 0.0;
+  auto is = [&](int rows, double alone, double each, double odd) {
+    const long blocks = ((long)columns * ceil_div(m, rows) + 255) / 256;
+    const double cost = blocks == 1 ? alone : blocks * each + (blocks % 2 ? odd : 0.0) + (rows == 32 && blocks <= 3 ? 5.0 : 0.0);
+    if (best == 0 || cost < least) {
+      best = rows;
+      least = cost;
+    }
+  };
+  is(64, 47.0, 36.7, 5.0);
+  is(32, 30.0, 19.7, 0.0);
+  is(96, 62.0, 51.8, 8.0);
+  if (!glu) {
+    is(48, 39.0, 29.4, 2.0);
+    is(80, 55.0, 45.3, 7.0);
+  }
+  return best;
+}
+
+template <bool GLU, int WAVES_M, int TM, int TN>
+static int launch_flow(unsigned columns, const float* x, int x_stride, const float* w, const void* bias, int bias_is_f32, void* out,
+                       int out_stride, int m, int n, int k, int mode, hipStream_t stream) {
+  constexpr int rows = 16 * WAVES_M * TM, lds = FLOW_STAGES * FLOW_STAGE(rows);
+  constexpr auto kernel = &gemm_fma_flow_kernel<GLU, WAVES_M, TM, TN>;
+  static bool configured = lds <= 64 * 1024;
+  if (!configured) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (e != hipSuccess) {
+      axk_set_error("gemm_fma: cannot reserve %d bytes of LDS: %s", lds, hipGetErrorString(e));
+      return -2;
+    }
+    configured = true;
+  }
+  kernel<<<dim3(columns, ceil_div(m, rows)), 256, lds, stream>>>(x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode);
+  return 0;
+}
+#endif
+
 template <bool GLU, bool VEC>
-static void launch_fma_tiles(dim3 tiles, const elem_t* x, int x_stride, const elem_t* w, const void* bias, int bias_is_f32, void* out,
+static int launch_fma_tiles(dim3 tiles, const elem_t* x, int x_stride, const elem_t* w, const void* bias, int bias_is_f32, void* out,
                              int out_stride, int m, int n, int k, int mode, hipStream_t stream) {
 #if !AXON_BF16
   // Short K: the stages that are filled before the first product count more than what they save, and where there are more
@@ -711,14 +785,31 @@ static void launch_fma_tiles(dim3 tiles, const elem_t* x, int x_stride, const el
   // 512 42.3 / 42.8, 640 51.4 / 51.0; of 32,000 of K 256 136 / 146, 640 309 / 314, as long from 1,024 on.
   if constexpr (VEC) {
     if (k >= ((long)tiles.x * tiles.y <= 512 ? FLOW_LEAST_K : 640)) {
-      static_assert(FLOW_STAGES * FLOW_STAGE <= 64 * 1024, "more LDS than a launch gets unasked");
       AXK_INSTANCE(INST_GEMM_FMA_FLOW, GLU);
-      gemm_fma_flow_kernel<GLU><<<tiles, 256, FLOW_STAGES * FLOW_STAGE, stream>>>(x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode);
-      return;
+#define FLOW(WAVES_M, TM, TN) return launch_flow<GLU, WAVES_M, TM, TN>(tiles.x, x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode, stream)
+      const int rows = flow_rows(tiles.x, m, GLU);
+      if (rows == 32) FLOW(2, 1, 2);
+      if (rows == 96) FLOW(2, 3, 2);
+      if constexpr (!GLU) {
+        if (rows == 48) FLOW(1, 3, 1);
+        if (rows == 80) FLOW(1, 5, 1);
+      }
+      FLOW(2, 2, 2);
+#undef FLOW
     }
   }
 #endif
   gemm_fma_kernel<GLU, VEC><<<tiles, 256, 0, stream>>>(x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode);
+  return 0;
+}
+
+// Whether 33 to 128 rows of aligned 32-bit numbers go to the tiles though these are fewer than the CUs: where a wave a chain
+// would give a CU two blocks, tiles of 32 rows are the faster.  us, K 2,048: one block a CU, 2,048 columns of 64 rows 20.5 / 28.7, of 128
+// 22.7 / 29.3; two, 2,560 of 65 33.6 / 28.8, of 128 39 / 29, 8,192 of 33 32.5 / 29.6, of 64 40.5 / 29.6, gated 5,632 of 64 53 / 46; four, 16,000 of
+// K 1,024 of 64 42 / 27.
+template <bool VEC>
+static bool tiles_of_few_rows(int m, int n, int k) {
+  return !AXON_BF16 && VEC && k >= 512 && (long)ceil_div(n, 16) * ceil_div(m, 64) > 256;
 }
 
 static int launch_fma(const elem_t* x, int x_stride, const elem_t* w, const void* bias, int bias_is_f32, void* out,
@@ -730,8 +821,7 @@ static int launch_fma(const elem_t* x, int x_stride, const elem_t* w, const void
 #define FMA_ARGS x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode, stream
 // Up to 32 rows a product waits for W; from 33 to 128 so it does where the tiles would be fewer than the CUs.  us, a wave a
 // chain / tiles: 128 rows of 2,048 columns of K 5,632 (64 tiles) 58 / 114, 64 of 8,192 of K 2,048 (128) 42 / 45, 65 of them (256) 67 / 46, of gated
-// 5,632 (352) 78 / 75, 33 and 64 of 32,000 (500) 119 / 78 and 153 / 81.  From some 170 tiles on the line is on the slow side: 64 rows
-// of gated 5,632 of K 2,048 (176) 54 / 46, of 16,000 of K 1,024 (250) 44 / 26.
+// 5,632 (352) 78 / 75, 33 and 64 of 32,000 (500) 119 / 78 and 153 / 81.
 #define FMA_LAUNCH(GLU, VEC)                                                                  \
   const dim3 tiles(ceil_div(n, GLU ? TILE_M / 2 : TILE_M), ceil_div(m, TILE_M));              \
   if (m <= 16) {                                                                              \
@@ -740,12 +830,12 @@ static int launch_fma(const elem_t* x, int x_stride, const elem_t* w, const void
   } else if (m <= 32) {                                                                       \
     AXK_INSTANCE(INST_GEMM_FMA, 32, GLU);                                                     \
     launch_fma_few<2, GLU, VEC>(FMA_ARGS);                                                    \
-  } else if (m <= 128 && (long)tiles.x * tiles.y < 256) {                                     \
+  } else if (m <= 128 && (long)tiles.x * tiles.y < 256 && !tiles_of_few_rows<VEC>(m, n, k)) { \
     AXK_INSTANCE(INST_GEMM_FMA, 64, GLU);                                                     \
     launch_fma_few<4, GLU, VEC>(FMA_ARGS);                                                    \
   } else {                                                                                    \
     AXK_INSTANCE(INST_GEMM_FMA, 128, GLU);                                                    \
-    launch_fma_tiles<GLU, VEC>(tiles, FMA_ARGS);                                              \
+    if (const int rc = launch_fma_tiles<GLU, VEC>(tiles, FMA_ARGS)) return rc;                \
   }
   const bool glu = mode == MODE_SWIGLU;
   if (vec_x && vec_w) {

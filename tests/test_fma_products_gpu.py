@@ -164,3 +164,23 @@ def test_direct_loads_at_every_end_of_k(K):
     k.reset_instances()
     test_tiles_at_every_end_of_k(K)
     assert {"gemm_fma_flow<0>", "gemm_fma_flow<1>"} <= set(k.instances(launched=True))
+
+
+@pytest.mark.parametrize("M,N,K", [(129, 2048, 644), (97, 2560, 512), (300, 2050, 192), (626, 2048, 228), (777, 2560, 644), (1500, 2048, 640),
+                                   (64, 8200, 516), (65, 4100, 512), (1025, 1000, 196)])
+def test_rows_a_block_by_what_the_cus_get(M, N, K):
+    """Tiles of 32, 48, 64, 80 and 96 rows, the last ones of a product among them: the bits of chains of fmaf."""
+    k = kernels("float32")
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    x, w = torch.randn(M, K, generator=g, device="cuda"), torch.randn(N, K, generator=g, device="cuda")
+    out = torch.full((M + 1, N), float("nan"), device="cuda")
+    k.reset_instances()
+    k.gemm(x, w, out[:M], None, MODE_STORE_F32)
+    assert "gemm_fma_flow<0>" in k.instances(launched=True)
+    want = _by_chains(k, x, w)
+    assert torch.equal(out[:M], want) and bool(out[M:].isnan().all())
+    half = N // 2
+    got, act = (torch.full((M, half), float("nan"), device="cuda") for _ in range(2))
+    k.gemm(x, w[:2 * half], got, None, MODE_SWIGLU)
+    k.swiglu(want[:, :2 * half].contiguous(), act)
+    assert torch.equal(got, act)
