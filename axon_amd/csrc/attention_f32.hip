@@ -308,13 +308,93 @@ __device__ __forceinline__ void f32_decode_block(const float* __restrict__ qrow,
   if (g4 == 0) *reinterpret_cast<float2*>(dst + HD) = make_float2(m_b, l_b);
 }
 
-// A wave takes one block of 64 positions of a (token, kv head), with the query heads of the group (up to
+// The same work shared by the four waves of a block: each scores sixteen of the positions, the scores meet in LDS, every wave works
+// out the weights from all of them and sums a quarter of the dims.  A wave alone had the pages' 64 KB to wait for, 256 products of 32
+// cycles and some thousand lane exchanges one after the other.
+template <int HD>
+__device__ __forceinline__ void f32_decode_shared(const float* __restrict__ qrow, const float* __restrict__ k_head,
+                                                  const float* __restrict__ v_head, const int32_t* __restrict__ table_row,
+                                                  size_t page_stride, int page_size, int p0, int lo, int pos, float scale, int r16,
+                                                  int g4, int wave, bool head_live, float* __restrict__ dst) {
+  constexpr int KG = HD / 16, DH = HD / 64;            // chunks of 16 dims of a key; tiles of 16 dims a wave
+  __shared__ __align__(16) f32x4 scores[4][64];
+  const int nt = min(4, (pos - p0) / 16 + 1), d0 = wave * DH, lane = r16 + 16 * g4;
+  f32x4 kf[KG], vf[4][DH], qf[KG];
+  int v_page[4];
+  const int kp = min(p0 + 16 * wave + r16, pos), k_page = table_row[page_index(kp, page_size)];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v_page[i] = table_row[page_index(min(p0 + 16 * i + 4 * g4, pos), page_size)];
+#pragma unroll
+  for (int g = 0; g < KG; ++g) qf[g] = *reinterpret_cast<const f32x4*>(qrow + 16 * g + 4 * g4);
+  const float* kr = k_head + (size_t)k_page * page_stride + (size_t)page_offset(kp, page_size) * HD;
+#pragma unroll
+  for (int g = 0; g < KG; ++g) kf[g] = *reinterpret_cast<const f32x4*>(kr + 16 * g + 4 * g4);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {                        // (tiles behind the token's own: its last positions again, not used)
+    const float* vr = v_head + (size_t)v_page[i] * page_stride + (page_offset(min(p0 + 16 * i + 4 * g4, pos), page_size) & ~3);
+#pragma unroll
+    for (int d = 0; d < DH; ++d) vf[i][d] = *reinterpret_cast<const f32x4*>(vr + (size_t)(16 * (d0 + d) + r16) * page_size);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  f32x4 mine = F32_ZERO;
+#pragma unroll
+  for (int g = 0; g < KG; ++g) {
+    const f32x4 qo = f32_operand(qf[g]), a = f32_operand(kf[g]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) F32_STEP(mine, a, qo, j);
+  }
+  scores[wave][lane] = mine;
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  f32x4 s[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) s[t] = scores[t][lane];
+  float m_b, l_b;
+  f32_weights(s, p0, lo, pos, scale, g4, m_b, l_b);
+  // the weight of a position outside the token's range is 0, and so must be what it is multiplied with
+  if (p0 < lo || p0 + ATT_BLOCK - 1 > pos) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int p = p0 + 16 * i + 4 * g4 + e;
+        const bool live = p >= lo && p <= pos;
+#pragma unroll
+        for (int d = 0; d < DH; ++d) vf[i][d][e] = live ? vf[i][d][e] : 0.0f;
+      }
+  }
+  f32x4 o[DH];
+#pragma unroll
+  for (int d = 0; d < DH; ++d) o[d] = F32_ZERO;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if (i >= nt) break;
+    const f32x4 pf = f32_operand(s[i]);
+#pragma unroll
+    for (int d = 0; d < DH; ++d) {
+      const f32x4 a = f32_operand(vf[i][d]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) F32_STEP(o[d], a, pf, j);
+    }
+  }
+  if (!head_live) return;
+#pragma unroll
+  for (int d = 0; d < DH; ++d) {
+    *reinterpret_cast<float2*>(dst + 16 * (d0 + d) + 4 * g4) = make_float2(o[d][0], o[d][1]);
+    *reinterpret_cast<float2*>(dst + 16 * (d0 + d) + 4 * g4 + 2) = make_float2(o[d][2], o[d][3]);
+  }
+  if (wave == 0 && g4 == 0) *reinterpret_cast<float2*>(dst + HD) = make_float2(m_b, l_b);
+}
+
+// One block of 64 positions of a (token, kv head), with the query heads of the group (up to
 // 16) as the columns; K and V^T go from the pages straight into registers, all 64 KB asked for at
 // once, and (o_b, m_b, l_b) of every head are left in `partial` for the fold (work list and layout as in
-// attention_mfma.hip).  BW waves a block of threads.  Bound by the wait for the pages: 8 tokens of 16 heads over
+// attention_mfma.hip).  BW blocks of positions a block of threads: four of a wave each, or one, which at head size 128 four waves
+// share (us with the fold, a wave alone / so: 5 tokens of 16 heads over 2 at 800 positions 15.0 / 12.4, 8 at 2,048 18.3 / 14.5, 9 of 28 over 4
+// at 4,000 44.6 / 38.2, 64 at 1,000 58 / 53; of 64, half as much to wait for: 32 over 32 at 1,500 156 / 181, 16 over 16 at 500 18.7 / 21.3).
+// Bound by the wait for the pages: 8 tokens of 16 heads over
 // 2 at 777 positions 64 -> 19 us with the fold, at 2,048 144 -> 17.
 template <int HD, int BW>
-__global__ void __launch_bounds__(64 * BW, 1)
+__global__ void __launch_bounds__(BW == 4 || HD == 128 ? 256 : 64, 1)
 attention_f32_decode_kernel(const float* __restrict__ q, int q_stride, const float* __restrict__ k_cache,
                             const float* __restrict__ v_cache, const int32_t* __restrict__ block_table, int table_stride,
                             const int32_t* __restrict__ positions, const int32_t* __restrict__ seq_rows,
@@ -339,14 +419,18 @@ attention_f32_decode_kernel(const float* __restrict__ q, int q_stride, const flo
   float* dst = partial + (((size_t)slot * n_heads + kvh * group + min(r16, group - 1)) * (max_chunks * (DC_CHUNK / ATT_BLOCK)) +
                           chunk * (DC_CHUNK / ATT_BLOCK) + sub) * (HD + 2);
   const float* qrow = q + (size_t)t * q_stride + (size_t)(kvh * group + min(r16, group - 1)) * HD;
-  // A context's last block often holds a few positions: 32 heads over 32, 200 tokens at 10 positions 103 us with all four
-  // tiles, 40 with one; 1 token of 16 heads over 2 14 / 9.
-  if (pos - p0 < 16)
-    f32_decode_block<HD, 1>(qrow, k_head, v_head, table_row, page_stride, page_size, p0, lo, pos, scale, r16, g4, r16 < group, dst);
-  else if (pos - p0 < 32)
-    f32_decode_block<HD, 2>(qrow, k_head, v_head, table_row, page_stride, page_size, p0, lo, pos, scale, r16, g4, r16 < group, dst);
-  else
-    f32_decode_block<HD, 4>(qrow, k_head, v_head, table_row, page_stride, page_size, p0, lo, pos, scale, r16, g4, r16 < group, dst);
+  if constexpr (BW == 1 && HD == 128) {
+    f32_decode_shared<HD>(qrow, k_head, v_head, table_row, page_stride, page_size, p0, lo, pos, scale, r16, g4, wave, r16 < group, dst);
+  } else {
+    // A context's last block often holds a few positions: 32 heads over 32, 200 tokens at 10 positions 103 us with all four
+    // tiles, 40 with one; 1 token of 16 heads over 2 14 / 9.
+    if (pos - p0 < 16)
+      f32_decode_block<HD, 1>(qrow, k_head, v_head, table_row, page_stride, page_size, p0, lo, pos, scale, r16, g4, r16 < group, dst);
+    else if (pos - p0 < 32)
+      f32_decode_block<HD, 2>(qrow, k_head, v_head, table_row, page_stride, page_size, p0, lo, pos, scale, r16, g4, r16 < group, dst);
+    else
+      f32_decode_block<HD, 4>(qrow, k_head, v_head, table_row, page_stride, page_size, p0, lo, pos, scale, r16, g4, r16 < group, dst);
+  }
 }
 
 // The fold of a token's blocks in ascending order, thread d dim d.  The factors depend on the maxima
@@ -448,7 +532,7 @@ int launch_attention_f32_decode(const float* q, int q_stride, const float* k_cac
 #define LAUNCH(HD, BW)                                                                                               \
   {                                                                                                                  \
     AXK_INSTANCE(INST_ATTENTION_F32_DECODE, HD, BW);                                                                 \
-    attention_f32_decode_kernel<HD, BW><<<(unsigned)n_work * n_kv_heads * (4 / BW), 64 * BW, 0, stream>>>(           \
+    attention_f32_decode_kernel<HD, BW><<<(unsigned)n_work * n_kv_heads * (4 / BW), BW == 4 || HD == 128 ? 256 : 64, 0, stream>>>(           \
         q, q_stride, k_cache, v_cache, block_table, table_stride, positions, seq_rows, token_index, n_tokens, work,  \
         partial, max_chunks, n_heads, n_kv_heads, page_size, window, scale);                                         \
     attention_f32_combine_kernel<HD><<<dim3(n_tokens, n_heads), HD, 0, stream>>>(partial, positions, token_index, out, \
