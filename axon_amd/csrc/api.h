@@ -251,6 +251,8 @@ int axk_clamped_glu(const void* gate_up, void* out, int n_tokens, int n_ffn, flo
 int axk_grouped_gemm_uses_mfma(int k, int x_is_f32, long x_row_stride, long x_group_stride);
 // Whether the blocks of a list of 64-row tiles are numbered tile by tile, not column by column; it changes no bit.
 int axk_grouped_gemm_by_tile(int n, int k, int glu);
+// Whether a gated routed product of `pairs` rows is the faster for a list of tiles of 128 rows (bfloat16 build); it changes no bit.
+int axk_grouped_gemm_wide(int pairs, int groups, int n, int k);
 int axk_grouped_gemm(const void* x, int x_is_f32, long x_row_stride, long x_group_stride, const int32_t* x_rows,
                      const void* w, const void* bias, int bias_is_f32, void* out, int out_is_f32, long out_row_stride,
                      long out_group_stride, const int32_t* out_rows, const float* gate, long gate_row_stride,
@@ -271,7 +273,7 @@ int axk_grouped_gemm(const void* x, int x_is_f32, long x_row_stride, long x_grou
 // sorted_tokens) and the tiles (of up to tile_rows rows) of the grouped product, at most
 // axk_route_max_tiles of them; pairs of experts from n_experts on (identities) are not listed.
 // place_of [n_pairs] (or null): where each pair stands in `sorted`; first_of [n_experts + 1] (or
-// null): where each expert's pairs start there.
+// null): where each expert's pairs start there.  wide_tiles (or null): the same rows in tiles of up to wide_rows too, *n_wide of them.
 // axk_route_combine: y[t, :] (+)= sum_k weights[t, k] rows[t top + k, :], k ascending (with
 // place_of: rows[place_of[t top + k], :]); weights may be null (all 1); extra (float32 [n_tokens, width], or null) is
 // a further row a token, times sigmoid(extra_gate[t extra_gate_stride]) if extra_gate is given; input (elem rows, or
@@ -281,7 +283,8 @@ int axk_route_scored(const float* logits, long logits_stride, const float* corre
                      int groups, int keep, float scale, int normalize, int softmax, int32_t* experts, float* weights, void* stream);
 int axk_route_max_tiles(int n_pairs, int n_experts, int tile_rows);
 int axk_route_sort(const int32_t* experts, int n_pairs, int n_experts, int top, int32_t* sorted, int32_t* sorted_tokens,
-                   int32_t* tiles, int32_t* n_tiles, int32_t* place_of, int32_t* first_of, int tile_rows, void* stream);
+                   int32_t* tiles, int32_t* n_tiles, int32_t* place_of, int32_t* first_of, int tile_rows, int32_t* wide_tiles,
+                   int32_t* n_wide, int wide_rows, void* stream);
 int axk_route_combine(const float* rows, const float* weights, float* y, int n_tokens, int top, int width, int accumulate,
                       const int32_t* place_of, const float* extra, const float* extra_gate, long extra_gate_stride, const int32_t* experts,
                       int n_experts, const void* input, long input_stride, void* stream);

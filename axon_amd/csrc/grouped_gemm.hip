@@ -20,6 +20,8 @@
 // The K-reduction of one output is one chain in ascending k that depends on K and the build alone
 // (32-bit FMA, or 16x16x32 MFMAs where the bfloat16 build can use them: K a multiple of 32 and
 // 16-byte aligned rows), never on which other rows share the tile.
+#include <type_traits>
+
 #include "api.h"
 #include "common.h"
 #include "instances.h"
@@ -379,6 +381,148 @@ __global__ void __launch_bounds__(256, 2) grouped_gemm_tile_kernel(GroupedArgs a
   }
 }
 
+// The gated product of more rows still: 128 rows x 256 rows of W a block of eight waves, each 64 x 64 (a wave's 64 rows of W are 32 gate rows
+// and the up rows of the same columns).  Stages of 64 k as above, three of them (144 KB, a block a CU): a step's fragments are in
+// registers when it begins, the next step's are read behind its first products, and a stage's loads go out between the products of the
+// stage two before it.  The chains are the same.  Lists of tiles of 128 rows, K a multiple of 64, X in the compute dtype.
+// Waves whose 64 rows a tile lacks only bring operands.  Bound by LDS, which is filled and read for 1,400 cycles a stage of 1,024 cycles of
+// products, and by what the last round leaves idle: 256 blocks take 36 us at K 2,048 (0.97 PFLOP/s).  us, tiles of 64 rows / here: 4 of 32
+// experts of [1,408, 2,048], 2,048 tokens 82 / 71 (104 / 84 in a step, which reads W from HBM), 4,096 151 / 133; 6 of 64 of [2,816,
+// 4,096], 2,048 tokens 480 / 420, 256 288 / 265; 2 of 16 of [5,632, 4,096], 2,048 tokens 328 / 269.  Products that are not gated lose with
+// short K (4 of 32 of [2,048, 704] 56 / 70: nobody multiplies while a block stores).
+#define GW_ROWS 128
+#define GW_COLS 256                                    // rows of W
+#define GW_STAGES 3
+#define GW_STAGE ((GW_ROWS + GW_COLS) * GT_BK * 2)
+__global__ void __launch_bounds__(512, 1) grouped_gemm_wide_kernel(GroupedArgs a) {
+  constexpr int COLS = GW_COLS / 2, LOADS = (GW_ROWS + GW_COLS) / 64;       // load instructions of a wave and stage
+  extern __shared__ __align__(256) unsigned char stages[];        // [3]: X [128][64], W [256][64]
+  const int col_tiles = (a.N + COLS - 1) / COLS, row_tiles = *a.n_tiles;
+  const long total = (long)row_tiles * col_tiles, share = (total + 7) / 8, item = (long)(blockIdx.x % 8) * share + blockIdx.x / 8;
+  if ((long)(blockIdx.x / 8) >= share || item >= total) return;       // (the order of blocks: as above)
+  const int row_tile = (int)(item % row_tiles), n0 = (int)(item / row_tiles) * COLS;
+  const int g = a.tiles[3 * row_tile], first = a.tiles[3 * row_tile + 1], count = a.tiles[3 * row_tile + 2];
+  if (count <= 0) return;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave >> 2, wn = wave & 3;
+  const bf16_t* wg = a.w + (long)g * 2 * a.N * a.K;
+  // a load instruction fills 8 rows: lane l row l / 8, slot l % 8; a wave's i-th the rows 8 (8 i + wave) and on, of X and then of W
+  const int lrow = lane >> 3, chunk = (lane & 7) ^ (4 * (wave & 1) + (lane >> 4));
+  const bf16_t* from[LOADS];
+#pragma unroll
+  for (int i = 0; i < LOADS; ++i) {
+    if (i < GW_ROWS / 64) {
+      const int r = first + min(8 * (8 * i + wave) + lrow, count - 1);
+      from[i] = (const bf16_t*)a.x + (long)(a.x_rows ? a.x_rows[r] : r) * a.x_row_stride + (long)g * a.x_group_stride + 8 * chunk;
+    } else {
+      const int row = 8 * (8 * (i - GW_ROWS / 64) + wave) + lrow;
+      from[i] = wg + (long)(min(n0 + 32 * (row >> 6) + (row & 31), a.N - 1) + (row & 32 ? a.N : 0)) * a.K + 8 * chunk;
+    }
+  }
+  auto ask = [&](int t, int i) {
+    __builtin_amdgcn_global_load_lds((gg_global_t)(from[i] + t * GT_BK), (gg_lds_t)(stages + t % GW_STAGES * GW_STAGE + (8 * i + wave) * 1024), 16, 0, 0);
+  };
+  const int n_stages = a.K / GT_BK;
+#pragma unroll
+  for (int i = 0; i < LOADS; ++i) ask(0, i);
+  if (n_stages > 1) {
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) ask(1, i);
+    wait_vmcnt<LOADS>();
+  } else {
+    wait_vmcnt<0>();
+  }
+  __builtin_amdgcn_s_barrier();                        // stage 0 is there for every wave
+  if (64 * wm >= count) {                              // nothing to multiply: its share of the loads, and the barriers
+    for (int t = 0; t + 1 < n_stages; ++t) {
+      if (t + 2 < n_stages) {
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) ask(t + 2, i);
+        wait_vmcnt<LOADS>();
+      } else {
+        wait_vmcnt<0>();
+      }
+      __builtin_amdgcn_s_barrier();
+    }
+    return;
+  }
+  gg_f32x4 acc[4][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = gg_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  const int fr = lane & 15, q = lane >> 4;
+  const unsigned lds0 = (unsigned)(size_t)(gg_lds_t)stages;
+  const unsigned at = lds0 + fr * 128 + ((q ^ (fr >> 1)) << 4);
+  const unsigned x_read = at + wm * 64 * 128, w_read = at + (GW_ROWS + 64 * wn) * 128;
+  u32x4 xf[2][4], wf[2][4];
+  read_frags<4, 2048>(xf[0], x_read);
+  read_frags<4, 2048>(wf[0], w_read);
+  wait_lgkmcnt<0>();
+  use_frags<4>(xf[0]);
+  use_frags<4>(wf[0]);
+  // A stage's two steps.  NEXT: there is one behind it; ASKS: and one behind that, whose place nobody reads any more.
+  auto stage = [&](int t, auto next_of, auto asks_of) {
+    constexpr bool NEXT = decltype(next_of)::value, ASKS = decltype(asks_of)::value;
+    const unsigned here = t % GW_STAGES * GW_STAGE, behind = (t + 1) % GW_STAGES * GW_STAGE;
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      if (half == 1 && NEXT) {
+        if (ASKS) wait_vmcnt<LOADS>();
+        else wait_vmcnt<0>();
+        __builtin_amdgcn_s_barrier();                  // the next stage is there for every wave; nobody reads the one before this one
+      }
+      const unsigned xr = half ? x_read + behind : (x_read ^ 64) + here, wr = half ? w_read + behind : (w_read ^ 64) + here;
+#pragma unroll
+      for (int p = 0; p < 16; ++p) {
+        const int i = p / 4, j = p % 4;
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gg_bf16x8, wf[half][j]), __builtin_bit_cast(gg_bf16x8, xf[half][i]),
+                                                            acc[i][j], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (half == 0 || NEXT) {
+          if (p < 4) lds_read16_step<2048, 4>(xf[half ^ 1][p % 4], xr, p);
+          else if (p < 8) lds_read16_step<2048, 4>(wf[half ^ 1][p % 4], wr, p - 4);
+        }
+        if (ASKS && half == 0 && p % 2 == 1 && p / 2 < LOADS) ask(t + 2, p / 2);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (half == 0 || NEXT) {
+        wait_lgkmcnt<0>();
+        use_frags<4>(xf[half ^ 1]);
+        use_frags<4>(wf[half ^ 1]);
+      }
+    }
+  };
+  int t = 0;
+  for (; t + 2 < n_stages; ++t) stage(t, std::true_type(), std::true_type());
+  if (t + 1 < n_stages) stage(t++, std::true_type(), std::false_type());
+  stage(t, std::false_type(), std::false_type());
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = 64 * wm + 16 * i + fr;
+    if (r >= count) continue;
+    const int orow = a.out_rows ? a.out_rows[first + r] : first + r;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) gg_store4(a, g, orow, n0 + 32 * wn + 16 * j + 4 * q, acc[i][j], acc[i][j + 2]);
+  }
+}
+
+int launch_wide(const GroupedArgs& a, dim3 grid, hipStream_t s) {
+  constexpr int lds = GW_STAGES * GW_STAGE;
+  static_assert(lds <= 160 * 1024, "the stages do not fit the LDS of a CU");
+  static bool configured = false;
+  if (!configured) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&grouped_gemm_wide_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (e != hipSuccess) {
+      axk_set_error("grouped_gemm: cannot reserve %d bytes of LDS: %s", lds, hipGetErrorString(e));
+      return -2;
+    }
+    configured = true;
+  }
+  AXK_INSTANCE(INST_GROUPED_GEMM, 2, 1);
+  grouped_gemm_wide_kernel<<<grid, 512, lds, s>>>(a);
+  return 0;
+}
+
 template <bool GLU, bool XF32, int WROWS>
 int launch_tile(const GroupedArgs& a, dim3 grid, hipStream_t s) {
   static bool configured = false;
@@ -418,6 +562,18 @@ extern "C" int axk_grouped_gemm_by_tile(int n, int k, int glu) {
   return !glu && (size_t)n * k * sizeof(elem_t) <= (12u << 20);
 }
 
+// Whether a gated routed product takes a list of tiles of 128 rows: where those of 64 are more than a round of two blocks a CU (an
+// expert's last tile half full).  us, 64 / 128 rows: 4 of 32 experts of [1,408, 2,048] of 1,024 tokens (480 blocks) 45 / 62, of
+// 2,048 (864) 82 / 71; 6 of 64 of [2,816, 4,096] of 256 (616) 288 / 265; 2 of 16 of [5,632, 4,096] of 256 (352) 150 / 160, of 512 (528) 203 / 168;
+// 2 of 8 of [2,048, 1,024] of 1,024 (288) 21 / 23, of 2,048 (544) 42 / 37; 8 of 64 of [512, 512] of 2,048 (576) 33.5 / 32.7.
+extern "C" int axk_grouped_gemm_wide(int pairs, int groups, int n, int k) {
+#if AXON_BF16
+  return k % GT_BK == 0 && (long)(pairs / 64 + groups / 2) * ceil_div(n, 128) > 512;
+#else
+  return 0;
+#endif
+}
+
 extern "C" int axk_grouped_gemm(const void* x, int x_is_f32, long x_row_stride, long x_group_stride, const int32_t* x_rows,
                                 const void* w, const void* bias, int bias_is_f32, void* out, int out_is_f32,
                                 long out_row_stride, long out_group_stride, const int32_t* out_rows, const float* gate,
@@ -430,7 +586,7 @@ extern "C" int axk_grouped_gemm(const void* x, int x_is_f32, long x_row_stride, 
               "grouped_gemm: a list of tiles comes with its length and the most tiles there can be");
   AXK_REQUIRE(tiles != nullptr || (x_rows == nullptr && out_rows == nullptr),
               "grouped_gemm: rows are named only beside a list of tiles");
-  AXK_REQUIRE(tile_rows == 16 || tile_rows == 64, "grouped_gemm: tiles of %d rows (16 or 64)", tile_rows);
+  AXK_REQUIRE(tile_rows == 16 || tile_rows == 64 || (tile_rows == 128 && tiles != nullptr), "grouped_gemm: tiles of %d rows (16, 64 or 128)", tile_rows);
   const int row_tiles = tiles ? max_tiles : ceil_div(m, GG_ROWS);
   if (row_tiles == 0) return 0;
   AXK_REQUIRE(groups <= 65535 && ceil_div(n, GG_COLS) <= 65535, "grouped_gemm: %d groups of %d columns are too many", groups, n);
@@ -445,6 +601,17 @@ extern "C" int axk_grouped_gemm(const void* x, int x_is_f32, long x_row_stride, 
 #if AXON_BF16
   const bool mfma = axk_grouped_gemm_uses_mfma(k, x_is_f32, x_row_stride, x_group_stride) && ((uintptr_t)x & 15) == 0 &&
                     ((uintptr_t)w & 15) == 0;
+  if (mfma && tile_rows == 128) {
+    AXK_REQUIRE(glu && !x_is_f32 && k % GT_BK == 0,
+                "grouped_gemm: tiles of 128 rows are for gated products of a K of a multiple of 64, not float32 X (K=%d)", k);
+    const long blocks = (long)max_tiles * ceil_div(n, GW_COLS / 2);
+    AXK_REQUIRE(blocks < (1l << 31) - 8, "grouped_gemm: %ld blocks are more than one launch takes", blocks);
+    const dim3 big((unsigned)((blocks + 7) / 8 * 8));
+    if (const int rc = launch_wide(a, big, s)) return rc;
+    AXK_LAUNCH_CHECK("grouped_gemm");
+    return 0;
+  }
+  AXK_REQUIRE(tile_rows != 128, "grouped_gemm: tiles of 128 rows are the matrix cores' (K a multiple of 64, operands aligned for 16 bytes)");
   // many rows a group: tiles of 64 rows through LDS (a list of tiles says by its tile size which it was made for)
   if (mfma && (tiles ? tile_rows == 64 : m >= 256)) {
     // 128 rows of W a block, three blocks a CU, unless the gated product has two rounds of blocks of 256: those read

@@ -145,43 +145,111 @@ __global__ void route_scored_wave_kernel(const float* __restrict__ logits, long 
 }
 
 // One block.  pairs p = t top + k in expert order -> sorted [n_pairs], with the token of each
-// (sorted_tokens); tiles [.][3] = (expert, first place in sorted, count <= tile_rows), *n_tiles of them.
+// (sorted_tokens); tiles [.][3] = (expert, first place in sorted, count <= tile_rows), *n_tiles of them; if given,
+// the same rows in tiles of wide_rows too (wide_tiles, *n_wide of them).
 // Which place a pair gets inside its expert's stretch is not fixed (atomic counters); no result
 // depends on it: every row of a product is a chain of its own.  Pairs whose expert is n_experts or more (an
 // identity, which has no matrices) are not listed.
-__global__ void __launch_bounds__(1024)
+// Bound by its waits: the first SORT_KEPT pairs a thread are read at once and keep the place that counting them gave, so that they
+// are neither read nor counted again; the experts' stretches and tiles are summed up by all threads; and the lists are put in order in
+// LDS where they fit (`staged`), since two scattered words a pair are as many lines.  us, two counts a pair, one thread for the stretches
+// and scattered words / here: 2,048 tokens, 4 of 32 13.2 / 8.2, 6 of 64 21.9 / 8.3, 8 of 64 (too many to be staged) 26.8 / 16.5.
+#define SORT_THREADS 1024
+#define SORT_KEPT 16
+__global__ void __launch_bounds__(SORT_THREADS)
 route_sort_kernel(const int32_t* __restrict__ experts, int n_pairs, int n_experts, int top, int32_t* __restrict__ sorted,
                   int32_t* __restrict__ sorted_tokens, int32_t* __restrict__ tiles, int32_t* __restrict__ n_tiles,
-                  int32_t* __restrict__ place_of, int32_t* __restrict__ first_of, int tile_rows) {
-  extern __shared__ int counts[];              // [n_experts] counts, then [n_experts] next free places
-  int* next = counts + n_experts;
-  for (int e = threadIdx.x; e < n_experts; e += blockDim.x) counts[e] = 0;
+                  int32_t* __restrict__ place_of, int32_t* __restrict__ first_of, int tile_rows, int32_t* __restrict__ wide_tiles,
+                  int32_t* __restrict__ n_wide, int wide_rows, bool staged) {
+  extern __shared__ int counts[];              // [n_experts] counts, [n_experts] where a stretch begins, [n_experts] next free places, staged: [n_pairs]
+  __shared__ int waves[3][SORT_THREADS / AXON_WAVE], all;
+  int *first = counts + n_experts, *next = first + n_experts;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  int expert[SORT_KEPT], rank[SORT_KEPT];
+#pragma unroll
+  for (int i = 0; i < SORT_KEPT; ++i) expert[i] = tid + SORT_THREADS * i < n_pairs ? experts[tid + SORT_THREADS * i] : n_experts;
+  for (int e = tid; e < n_experts; e += SORT_THREADS) counts[e] = 0;
   __syncthreads();
-  for (int p = threadIdx.x; p < n_pairs; p += blockDim.x)
-    if (experts[p] < n_experts) atomicAdd(&counts[experts[p]], 1);
+#pragma unroll
+  for (int i = 0; i < SORT_KEPT; ++i)
+    if (expert[i] < n_experts) rank[i] = atomicAdd(&counts[expert[i]], 1);
   __syncthreads();
-  if (threadIdx.x == 0) {
-    int at = 0, tile = 0;
-    for (int e = 0; e < n_experts; ++e) {
-      const int n = counts[e];
-      next[e] = at;
-      if (first_of) first_of[e] = at;
-      for (int i = 0; i < n; i += tile_rows) {
-        tiles[3 * tile] = e; tiles[3 * tile + 1] = at + i; tiles[3 * tile + 2] = min(tile_rows, n - i);
-        ++tile;
-      }
-      at += n;
+  const bool more = n_pairs > SORT_THREADS * SORT_KEPT;
+  if (more) {
+    for (int e = tid; e < n_experts; e += SORT_THREADS) next[e] = counts[e];
+    __syncthreads();
+    for (int p = tid + SORT_THREADS * SORT_KEPT; p < n_pairs; p += SORT_THREADS)
+      if (experts[p] < n_experts) atomicAdd(&counts[experts[p]], 1);
+    __syncthreads();
+  }
+  // a thread's neighbouring experts; pairs, tiles and wide tiles before them
+  const int each = (n_experts + SORT_THREADS - 1) / SORT_THREADS, e0 = min(tid * each, n_experts), e1 = min(e0 + each, n_experts);
+  int sums[3] = {0, 0, 0}, before[3];
+  for (int e = e0; e < e1; ++e) {
+    sums[0] += counts[e];
+    sums[1] += (counts[e] + tile_rows - 1) / tile_rows;
+    sums[2] += (counts[e] + wide_rows - 1) / wide_rows;
+  }
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    int upto = sums[k];
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int other = __shfl_up(upto, off, 64);
+      upto += lane >= off ? other : 0;
     }
-    *n_tiles = tile;
-    if (first_of) first_of[n_experts] = at;
+    before[k] = upto - sums[k];
+    if (lane == 63) waves[k][wave] = upto;
+  }
+  if (n_experts > 64) {                        // (else the first wave has them all)
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      for (int w = 0; w < wave; ++w) before[k] += waves[k][w];
+  }
+  for (int e = e0; e < e1; ++e) {
+    const int n = counts[e];
+    first[e] = before[0];
+    if (more) next[e] += before[0];
+    if (first_of) first_of[e] = before[0];
+    for (int i = 0; i < n; i += tile_rows, ++before[1]) {
+      tiles[3 * before[1]] = e; tiles[3 * before[1] + 1] = before[0] + i; tiles[3 * before[1] + 2] = min(tile_rows, n - i);
+    }
+    if (wide_tiles)
+      for (int i = 0; i < n; i += wide_rows, ++before[2]) {
+        wide_tiles[3 * before[2]] = e; wide_tiles[3 * before[2] + 1] = before[0] + i; wide_tiles[3 * before[2] + 2] = min(wide_rows, n - i);
+      }
+    before[0] += n;
+  }
+  if (tid == (n_experts > 64 ? SORT_THREADS - 1 : 63)) {       // (its experts are the last, or it has none)
+    *n_tiles = before[1];
+    if (wide_tiles) *n_wide = before[2];
+    if (first_of) first_of[n_experts] = before[0];
+    all = before[0];
   }
   __syncthreads();
-  for (int p = threadIdx.x; p < n_pairs; p += blockDim.x) {
-    if (experts[p] >= n_experts) continue;
-    const int place = atomicAdd(&next[experts[p]], 1);
-    sorted[place] = p;
-    sorted_tokens[place] = p / top;
+  const int listed = all;
+  int* order = next + n_experts;
+  auto put = [&](int p, int place) {
+    if (staged) {
+      order[place] = p;
+    } else {
+      sorted[place] = p;
+      sorted_tokens[place] = p / top;
+    }
     if (place_of) place_of[p] = place;
+  };
+#pragma unroll
+  for (int i = 0; i < SORT_KEPT; ++i)
+    if (expert[i] < n_experts) put(tid + SORT_THREADS * i, first[expert[i]] + rank[i]);
+  for (int p = tid + SORT_THREADS * SORT_KEPT; p < n_pairs; p += SORT_THREADS)
+    if (experts[p] < n_experts) put(p, atomicAdd(&next[experts[p]], 1));
+  if (!staged) return;
+  __syncthreads();
+  for (int i = tid; i < listed; i += SORT_THREADS) {
+    const int p = order[i];
+    sorted[i] = p;
+    sorted_tokens[i] = p / top;
   }
 }
 
@@ -267,11 +335,16 @@ extern "C" int axk_gather_rows(const void* x, long x_stride, const int32_t* rows
 
 extern "C" int axk_route_sort(const int32_t* experts, int n_pairs, int n_experts, int top, int32_t* sorted,
                               int32_t* sorted_tokens, int32_t* tiles, int32_t* n_tiles, int32_t* place_of, int32_t* first_of,
-                              int tile_rows, void* stream) {
+                              int tile_rows, int32_t* wide_tiles, int32_t* n_wide, int wide_rows, void* stream) {
   AXK_REQUIRE(n_pairs >= 0 && n_experts > 0 && top > 0 && n_experts <= 4096 && tile_rows > 0,
               "route_sort: %d pairs, %d experts, tiles of %d", n_pairs, n_experts, tile_rows);
-  route_sort_kernel<<<1, 1024, 2 * n_experts * sizeof(int), (hipStream_t)stream>>>(experts, n_pairs, n_experts, top, sorted,
-                                                                                  sorted_tokens, tiles, n_tiles, place_of, first_of, tile_rows);
+  AXK_REQUIRE((wide_tiles == nullptr) == (n_wide == nullptr) && (wide_tiles == nullptr || wide_rows > 0),
+              "route_sort: a second list of tiles (of %d) comes with its length", wide_rows);
+  const long lists = 3l * n_experts * (long)sizeof(int), order = (long)n_pairs * (long)sizeof(int);
+  const bool staged = n_pairs > SORT_THREADS && lists + order <= 60 * 1024;       // (a launch gets 64 KB unasked)
+  route_sort_kernel<<<1, SORT_THREADS, lists + (staged ? order : 0), (hipStream_t)stream>>>(
+      experts, n_pairs, n_experts, top, sorted, sorted_tokens, tiles, n_tiles, place_of, first_of, tile_rows, wide_tiles, n_wide,
+      wide_tiles ? wide_rows : tile_rows, staged);
   AXK_LAUNCH_CHECK("route_sort");
   return 0;
 }

@@ -99,7 +99,9 @@ _SIGNATURES = {
     "axk_route_topk": [c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p],
     "axk_route_scored": [c_void_p, c_long, c_void_p, c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_int, c_void_p, c_void_p, c_void_p],
     "axk_route_max_tiles": [c_int, c_int, c_int],
-    "axk_route_sort": [c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p],
+    "axk_grouped_gemm_wide": [c_int, c_int, c_int, c_int],
+    "axk_route_sort": [c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p,
+                             c_void_p, c_int, c_void_p],
     "axk_route_combine": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_long, c_void_p, c_int,
                           c_void_p, c_long, c_void_p],
     "axk_tanh_norm": [c_void_p, c_void_p, c_float, c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_int, c_void_p],
@@ -874,8 +876,8 @@ class Kernels:
         and u clamped by limit, shift 1 unless given; (inf, 1, 0) is silu(gate) up) in the compute dtype; out float32 or
         compute dtype.  Block-diagonal: every row meets every group.  `routed` = (tiles, n_tiles,
         max_tiles, x_rows, out_rows[, tile_rows]), int32 on the device: the listed rows (`rows` of them at
-        most) meet the group their tile names; tile_rows (16, or 64: many rows a group) is what the list
-        was made for.  `gate` (float32, out's shape): out is multiplied
+        most) meet the group their tile names; tile_rows (16; 64: many rows a group; 128: more still, with `glu`, see
+        `grouped_gemm_wide`) is what the list was made for.  `gate` (float32, out's shape): out is multiplied
         by its sigmoid; with `gate_per_group` the gate holds one number a group, [rows, >= G].  `row_scale`
         (float32, one number an out row): the sums are multiplied by it before bias and epilogue, as if the
         row of x had been."""
@@ -920,6 +922,10 @@ class Kernels:
             _ptr(row_scale), 1 if glu else 0, float(limit), float(alpha), float(shift), _ptr(tiles), _ptr(n_tiles), int(max_tiles), int(tile_rows), M, N, K, G, _stream()))
         return out
 
+    def grouped_gemm_wide(self, pairs: int, groups: int, n: int, k: int) -> bool:
+        """Whether a gated routed product of `pairs` rows over `groups` matrices [2 n, k] is the faster for a list of tiles of 128 rows."""
+        return bool(self.lib.axk_grouped_gemm_wide(pairs, groups, n, k))
+
     # ------------------------------------------------------------------ routing
     def route_topk(self, logits: torch.Tensor, top: int, experts: torch.Tensor, weights: torch.Tensor) -> None:
         self._f32(logits, "router logits"); self._i32(experts, "chosen experts"); self._f32(weights, "router weights")
@@ -954,18 +960,23 @@ class Kernels:
         return int(self.lib.axk_route_max_tiles(n_pairs, n_experts, tile_rows))
 
     def route_sort(self, experts: torch.Tensor, n_experts: int, sorted_pairs, sorted_tokens, tiles, n_tiles, place_of=None,
-                   first_of=None, tile_rows: int = 16) -> None:
+                   first_of=None, tile_rows: int = 16, wide=None) -> None:
         """The pairs in expert order, their tokens, the grouped product's tiles; optionally where each
-        pair stands (place_of [pairs]) and where each expert's pairs start (first_of [experts + 1])."""
-        for t in (experts, sorted_pairs, sorted_tokens, tiles, n_tiles) + tuple(t for t in (place_of, first_of) if t is not None):
+        pair stands (place_of [pairs]) and where each expert's pairs start (first_of [experts + 1]), and a second list
+        of tiles, `wide` = (tiles, n_tiles, tile_rows)."""
+        wide_tiles, n_wide, wide_rows = wide if wide is not None else (None, None, 0)
+        for t in (experts, sorted_pairs, sorted_tokens, tiles, n_tiles) + tuple(t for t in (place_of, first_of, wide_tiles, n_wide) if t is not None):
             self._i32(t, "route_sort")
         if (place_of is not None and place_of.numel() < experts.numel()) or (first_of is not None and first_of.numel() < n_experts + 1):
             raise KernelError("route_sort: place_of or first_of is too short")
         P = experts.numel()
         if sorted_pairs.numel() < P or sorted_tokens.numel() < P or tiles.numel() < 3 * self.route_max_tiles(P, n_experts, tile_rows):
             raise KernelError(f"route_sort: lists too short for {P} pairs of {n_experts} experts")
+        if wide is not None and wide_tiles.numel() < 3 * self.route_max_tiles(P, n_experts, wide_rows):
+            raise KernelError(f"route_sort: the second list is too short for {P} pairs of {n_experts} experts")
         self._check(self.lib.axk_route_sort(_ptr(experts), P, n_experts, experts.shape[-1], _ptr(sorted_pairs), _ptr(sorted_tokens),
-                                            _ptr(tiles), _ptr(n_tiles), _ptr(place_of), _ptr(first_of), int(tile_rows), _stream()))
+                                                  _ptr(tiles), _ptr(n_tiles), _ptr(place_of), _ptr(first_of), int(tile_rows),
+                                                  _ptr(wide_tiles), _ptr(n_wide), int(wide_rows), _stream()))
 
     def gather_rows(self, x: torch.Tensor, rows: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
         self._elem(x, "gather x"); self._elem(out, "gather out"); self._i32(rows, "gather rows")

@@ -157,11 +157,17 @@ class RoutedExperts(FeedForward):
         max_tiles = k.route_max_tiles(P, E, tile_rows)
         pairs, tokens = ctx.ws.take((P,), i32), ctx.ws.take((P,), i32)
         tiles, n_tiles = ctx.ws.take((3 * max_tiles,), i32), ctx.ws.take((1,), i32)
-        k.route_sort(chosen, E, pairs, tokens, tiles, n_tiles, tile_rows=tile_rows)
+        gated = (tiles, n_tiles, max_tiles, tile_rows)      # the tiles of the gated product: larger ones where it has many
+        wide = None
+        if tile_rows == 64 and k.grouped_gemm_wide(P, E, self.ff, self.hidden):
+            most = k.route_max_tiles(P, E, 128)
+            gated = (ctx.ws.take((3 * most,), i32), ctx.ws.take((1,), i32), most, 128)
+            wide = (gated[0], gated[1], 128)
+        k.route_sort(chosen, E, pairs, tokens, tiles, n_tiles, tile_rows=tile_rows, wide=wide)
         act = ctx.ws.take((P, self.ff), ctx.rt.dtype)
         on_input = self.weight_on == "input"        # act row p is the unit of (weight of pair p) x (the token's row)
         k.grouped_gemm(h, self.w_gate_up, act, x_group_stride=0, out_group_stride=0, glu=(self.limit, self.alpha, self.shift),
-                       routed=(tiles, n_tiles, max_tiles, tokens, pairs, tile_rows), rows=P,
+                       routed=(*gated[:3], tokens, pairs, gated[3]), rows=P,
                        row_scale=weights.view(-1) if on_input else None)
         rows = ctx.ws.take((P, self.hidden), torch.float32)
         k.grouped_gemm(act, self.w_down, rows, x_group_stride=0, out_group_stride=0,

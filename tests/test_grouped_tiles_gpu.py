@@ -81,3 +81,50 @@ def test_lists_in_both_orders(N, K, by_tile):
         k.grouped_gemm(x, w, out, x_group_stride=0, out_group_stride=0, routed=(tiles, n, most, pairs, pairs, rows), rows=P)
         got.append(out)
     assert torch.equal(got[0], got[1]) and not bool(got[0].isnan().any())
+
+
+@pytest.mark.parametrize("T,H,F", [(1, 64, 40), (65, 128, 128), (190, 192, 129), (260, 704, 300), (700, 256, 72)])
+def test_lists_of_128_rows(T, H, F):
+    """Gated products: a tile's second 64 rows there, partly and not at all, one and two stages of K and more, columns past the end,
+    and the second list of a sort against one of its own."""
+    k, E, top = kernels("bfloat16"), 5, 2
+    g = torch.Generator(device="cuda").manual_seed(T + H)
+    P = T * top
+    h = torch.randn(T, H, generator=g, device="cuda").bfloat16()
+    wu = (torch.randn(E, 2 * F, H, generator=g, device="cuda") * 0.2).bfloat16()
+    odds = torch.tensor([9.0, 4.0, 2.0, 0.0, 0.3], device="cuda").expand(T, E)
+    chosen = torch.multinomial(odds, top, generator=g).int().contiguous()
+    scale = torch.rand(P, generator=g, device="cuda")
+    most, most128 = k.route_max_tiles(P, E, 16), k.route_max_tiles(P, E, 128)
+    pairs, tokens, tiles, n, tiles128, n128 = (torch.zeros(s, dtype=torch.int32, device="cuda") for s in (P, P, 3 * most, 1, 3 * most128, 1))
+    k.route_sort(chosen, E, pairs, tokens, tiles, n, tile_rows=16, wide=(tiles128, n128, 128))
+    got = []
+    for listed, count, at_most, rows in ((tiles, n, most, 16), (tiles128, n128, most128, 128)):
+        out = torch.full((P + 1, F), float("nan"), dtype=torch.bfloat16, device="cuda")
+        k.grouped_gemm(h, wu, out[:P], x_group_stride=0, out_group_stride=0, glu=(float("inf"), 1.0, 0.0),
+                       routed=(listed, count, at_most, tokens, pairs, rows), rows=P, row_scale=scale)
+        assert bool(out[P:].isnan().all())
+        got.append(out[:P])
+    assert torch.equal(got[0], got[1]) and not bool(got[0].isnan().any())
+
+
+@pytest.mark.parametrize("T,E,top,identities", [(1, 1, 1, 0), (300, 7, 3, 2), (2050, 1500, 8, 0), (9000, 40, 2, 8), (5000, 4096, 4, 0), (2048, 32, 4, 0), (1024, 64, 8, 1)])
+def test_sorting_pairs(T, E, top, identities):
+    """More pairs than the block keeps, more experts than it has threads, experts without a pair, and pairs that are not listed."""
+    k, P = kernels("bfloat16"), T * top
+    g = torch.Generator(device="cuda").manual_seed(P)
+    chosen = (torch.rand(T, top, generator=g, device="cuda") ** 2 * (E + identities)).int()
+    sizes = (P, P, 3 * k.route_max_tiles(P, E, 64), 1, 3 * k.route_max_tiles(P, E, 128), 1, P, E + 1)
+    pairs, tokens, tiles, n, wide, n_wide, place_of, first_of = (torch.full((s,), -7, dtype=torch.int32, device="cuda") for s in sizes)
+    k.route_sort(chosen, E, pairs, tokens, tiles, n, place_of, first_of, tile_rows=64, wide=(wide, n_wide, 128))
+    flat, pairs, tokens, place_of = (v.long().cpu() for v in (chosen.view(-1), pairs, tokens, place_of))
+    count = torch.bincount(flat[flat < E], minlength=E)
+    total = int(count.sum())
+    first = [0] + count.cumsum(0).tolist()
+    assert first_of.tolist() == first and bool((pairs[total:] == -7).all())
+    assert pairs[:total].sort().values.tolist() == (flat < E).nonzero().view(-1).tolist()
+    assert torch.equal(flat[pairs[:total]], torch.arange(E).repeat_interleave(count)) and torch.equal(tokens[:total], pairs[:total] // top)
+    assert torch.equal(place_of[pairs[:total]], torch.arange(total))
+    for listed, made, rows in ((tiles, n, 64), (wide, n_wide, 128)):
+        want = [[e, first[e] + i, min(rows, int(count[e]) - i)] for e in range(E) for i in range(0, int(count[e]), rows)]
+        assert int(made) == len(want) and listed.view(-1, 3)[:len(want)].tolist() == want
