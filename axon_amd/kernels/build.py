@@ -6,6 +6,7 @@ Two kinds of library are built from `axon_amd/csrc`:
   (`bfloat16`, `float32`), compiled with hipcc.  A call that needs a dtype compiles that
   dtype only.
 * `libaxon_host.so`: the host runtime (cache manager, scheduler), plain C++.
+* `axon_calls.<interpreter>.so`: the kernel libraries' entry points as callables of this Python, where its headers are there.
 * `libaxon_ext_<name>_<dtype>.so`: one library per kernel source that a part outside the package
   registered (`register_kernel_source`), built like the kernel library, with this package's
   headers on the include path.
@@ -22,6 +23,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 import tempfile
 import time
 from concurrent.futures import ThreadPoolExecutor
@@ -37,6 +39,7 @@ KERNEL_SOURCES = ["elementwise.hip", "gemm.hip", "gemm_mfma.hip", "attention.hip
 # what a library built from a part's own kernel sources gets beside them (the error channel, the
 # list of its kernel instances)
 EXTENSION_SUPPORT = ["support.hip", "instances.hip"]
+CALLS_SOURCES = ["host/calls.cpp"]
 HOST_SOURCES = ["host/cache.cpp", "host/scheduler.cpp", "host/sampler.cpp", "host/step.cpp"]
 
 # Packed 32-bit float instructions are switched off for all device code.  No contraction of a
@@ -207,6 +210,18 @@ def build_host(force: bool = False) -> str:
     return _build("libaxon_host.so", HOST_SOURCES, cxx, HOST_FLAGS, ["-fPIC"], force)
 
 
+def build_calls(force: bool = False) -> str:
+    """The entry points as Python callables (an extension of the interpreter that runs)."""
+    include = sysconfig.get_paths()["include"]
+    name = f"axon_calls{sysconfig.get_config_var('EXT_SUFFIX')}"
+    flags = HOST_FLAGS + ["-I", include]
+    if not force and _fresh(name, CALLS_SOURCES, flags):
+        return os.path.join(built_dir(), name)
+    if not os.path.exists(os.path.join(include, "Python.h")):
+        raise BuildError(f"no Python.h in {include}")
+    return _build(name, CALLS_SOURCES, _find("g++", ["/usr/bin/g++", "/usr/bin/c++"]), flags, ["-fPIC"], force)
+
+
 def _fresh(lib_name: str, sources: List[str], flags: List[str]) -> bool:
     lib = os.path.join(built_dir(), lib_name)
     try:
@@ -218,4 +233,9 @@ def _fresh(lib_name: str, sources: List[str], flags: List[str]) -> bool:
 
 def build_all(force: bool = True) -> List[str]:
     """Everything: the host runtime and both kernel libraries."""
-    return [build_host(force), build_kernels("float32", force), build_kernels("bfloat16", force)]
+    built = [build_host(force), build_kernels("float32", force), build_kernels("bfloat16", force)]
+    try:
+        built.append(build_calls(force))
+    except BuildError as e:                      # the calls go through ctypes then
+        _say(str(e))
+    return built

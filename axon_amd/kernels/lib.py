@@ -8,6 +8,9 @@ other implementation behind these calls: without the library they fail.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
+import types
 from ctypes import c_char_p, c_float, c_int, c_long, c_void_p
 from typing import Dict, List, Optional, Sequence
 
@@ -41,6 +44,11 @@ def _stream() -> c_void_p:
     if _raw_stream is None:
         return c_void_p(torch.cuda.current_stream().cuda_stream)
     return c_void_p(_raw_stream(torch._C._cuda_getDevice()))
+
+
+def _queue() -> int:
+    """The current stream as a number, for the calls of this file."""
+    return torch.cuda.current_stream().cuda_stream if _raw_stream is None else _raw_stream(torch._C._cuda_getDevice())
 
 
 # for the callers of `Kernels.call`: a tensor's (or a packed matrix's) address, the current stream
@@ -169,6 +177,28 @@ _SIGNATURES = {
 }
 
 
+# entry points beside those of _SIGNATURES that the methods call
+_PLAIN = ["axk_argmax_workspace", "axk_attention_decode_chunk", "axk_attention_decode_item_factor", "axk_attention_decode_workspace",
+          "axk_attention_prefill_tile", "axk_delta_chunked_workspace", "axk_gemm_workspace", "axk_latent_attention_workspace",
+          "axk_masked_attention_workspace", "axk_packed_elems"]
+
+
+def _calls_module():
+    """The native callables of this interpreter (see csrc/host/calls.cpp), or None where they cannot be built."""
+    global _calls
+    if _calls is False:
+        try:
+            loader = importlib.machinery.ExtensionFileLoader("axon_calls", build.build_calls())
+            _calls = importlib.util.module_from_spec(importlib.util.spec_from_loader("axon_calls", loader))
+            loader.exec_module(_calls)
+        except (build.BuildError, ImportError):
+            _calls = None
+    return _calls
+
+
+_calls = False
+
+
 class PackedMatrix:
     """A [rows, cols] matrix in the layout the matrix-core products read: blocks of 16 rows x 32
     columns, each 1 KB in the order in which a wave holds them as an MFMA operand, ordered
@@ -232,8 +262,20 @@ class Kernels:
         self.lib.axk_instances_reset.restype = None
         if bool(self.lib.axk_is_bf16()) != (dtype_name == "bfloat16"):
             raise KernelError(f"{self.path} was not built for {dtype_name}")
+        self.run = self._callables()
         self._extensions: Dict[str, ctypes.CDLL] = {}      # a registered source's path -> its library
         self._chunk_factor = None
+
+    def _callables(self):
+        """The library's entry points as the methods call them: bound natively where that module is there (csrc/host/calls.cpp), else
+        through ctypes."""
+        run = types.SimpleNamespace()
+        calls = _calls_module()
+        native = set(calls.names()) if calls is not None else set()
+        for name in native | set(_SIGNATURES) | set(_PLAIN):
+            fn = getattr(self.lib, name)
+            setattr(run, name, calls.bind(name, ctypes.cast(fn, c_void_p).value) if name in native else fn)
+        return run
 
     # ------------------------------------------------------------------ a part's own kernels
     def call(self, name: str, *args) -> None:
@@ -356,8 +398,8 @@ class Kernels:
         vocab, dim = table.shape
         if out.shape != (tokens.numel(), dim) or not (packed or table.is_contiguous()):
             raise KernelError(f"embed: out {tuple(out.shape)} does not fit {tokens.numel()} tokens of width {dim}")
-        self._check(self.lib.axk_embed_scaled(_ptr(tokens), _ptr(table), 1 if packed else 0, _ptr(out), tokens.numel(), dim,
-                                              vocab, float(scale), _stream()))
+        self._check(self.run.axk_embed_scaled(_ptr(tokens), _ptr(table), 1 if packed else 0, _ptr(out), tokens.numel(), dim,
+                                              vocab, float(scale), _queue()))
         return out
 
     def rmsnorm(self, x: torch.Tensor, gain: torch.Tensor, eps: float, out: torch.Tensor,
@@ -373,8 +415,8 @@ class Kernels:
             raise KernelError(f"rmsnorm: {x.shape[0]} rows in, {n} rows out")
         if gain.numel() != dim or out.shape[-1] != dim or not out.is_contiguous():
             raise KernelError(f"rmsnorm: width {dim}, gain {gain.numel()}, out {tuple(out.shape)}")
-        self._check(self.lib.axk_rmsnorm(_ptr(x), _ptr(rows), _ptr(gain), self._vec_flag(gain, "rmsnorm gain"),
-                                         _ptr(out), n, dim, float(eps), _stream()))
+        self._check(self.run.axk_rmsnorm(_ptr(x), _ptr(rows), _ptr(gain), self._vec_flag(gain, "rmsnorm gain"),
+                                         _ptr(out), n, dim, float(eps), _queue()))
         return out
 
     def rope_table(self, positions: torch.Tensor, freqs: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
@@ -383,8 +425,8 @@ class Kernels:
             raise KernelError("rope_table: frequencies must be float64 on the device")
         if out.shape != (positions.numel(), freqs.numel(), 2):
             raise KernelError(f"rope_table: table {tuple(out.shape)} for {positions.numel()} x {freqs.numel()} pairs")
-        self._check(self.lib.axk_rope_table(_ptr(positions), _ptr(freqs), _ptr(out), positions.numel(), freqs.numel(),
-                                            _stream()))
+        self._check(self.run.axk_rope_table(_ptr(positions), _ptr(freqs), _ptr(out), positions.numel(), freqs.numel(),
+                                            _queue()))
         return out
 
     def rope_kv_write(self, qkv, table, positions, seq_rows, block_table, k_cache, v_cache, n_heads, n_kv_heads,
@@ -399,14 +441,14 @@ class Kernels:
             raise KernelError(f"rope_kv_write: table {tuple(table.shape)} for rotary_dim {rotary_dim}")
         if write_kv:
             self._check_caches(k_cache, v_cache, n_kv_heads, page_size, head_dim)
-        self._check(self.lib.axk_rope_kv_write(
+        self._check(self.run.axk_rope_kv_write(
             _ptr(qkv), _ptr(table), _ptr(positions), _ptr(seq_rows), _ptr(block_table), block_table.shape[-1],
             _ptr(k_cache if write_kv else None), _ptr(v_cache if write_kv else None), T, n_heads, n_kv_heads, head_dim,
-            rotary_dim, page_size, 1 if write_kv else 0, _stream()))
+            rotary_dim, page_size, 1 if write_kv else 0, _queue()))
 
     def gemm_qkv_rope_ok(self, m: int, n: int, k: int, head_dim: int, rotary_dim: int) -> bool:
         """Whether `gemm_qkv_rope` takes a step of m tokens and a matrix of n rows of these sizes."""
-        return bool(self.lib.axk_gemm_qkv_rope_ok(m, n, k, head_dim, rotary_dim))
+        return bool(self.run.axk_gemm_qkv_rope_ok(m, n, k, head_dim, rotary_dim))
 
     def gemm_qkv_rope(self, x, w, bias, qkv, table, positions, seq_rows, block_table, k_cache, v_cache, n_heads,
                       n_kv_heads, head_dim, page_size, write_kv=True) -> None:
@@ -431,13 +473,13 @@ class Kernels:
             raise KernelError(f"gemm_qkv_rope: bias of {bias.numel()} for {rows} rows")
         if write_kv:
             self._check_caches(k_cache, v_cache, n_kv_heads, page_size, head_dim)
-        need = self.lib.axk_gemm_workspace(M, rows, K, MODE_STORE)
+        need = self.run.axk_gemm_workspace(M, rows, K, MODE_STORE)
         work = torch.empty(need // 4, dtype=torch.float32, device=x.device) if need > 0 else None
-        self._check(self.lib.axk_gemm_qkv_rope(
+        self._check(self.run.axk_gemm_qkv_rope(
             _ptr(x), x.stride(0), _ptr(w), _ptr(bias), self._vec_flag(bias, "qkv bias"), _ptr(qkv), qkv.stride(0), M, K,
             _ptr(table), _ptr(positions), _ptr(seq_rows), _ptr(block_table),
             block_table.shape[-1], _ptr(k_cache if write_kv else None), _ptr(v_cache if write_kv else None), n_heads,
-            n_kv_heads, head_dim, page_size, 1 if write_kv else 0, _ptr(work), need, _stream()))
+            n_kv_heads, head_dim, page_size, 1 if write_kv else 0, _ptr(work), need, _queue()))
 
     def gemm_normed_ok(self, m: int, n: int, k: int, gated: bool = False, gain=None) -> bool:
         """Whether the product of m rows with a packed [n, k] matrix (gated: [gate; up] of 2 n rows)
@@ -445,7 +487,7 @@ class Kernels:
         `gain`, also whether that gain is one the kernels take (bfloat16)."""
         if gain is not None and gain.dtype != torch.bfloat16:
             return False
-        return bool(self.lib.axk_gemm_normed_ok(m, n, k, 1 if gated else 0))
+        return bool(self.run.axk_gemm_normed_ok(m, n, k, 1 if gated else 0))
 
     def _normed_rows(self, rows, gain, K, what):
         if rows.dtype != torch.float32 or not rows.is_cuda:
@@ -465,8 +507,8 @@ class Kernels:
         self._elem(w.data, "gate|up w"); self._elem(out, "gate|up out")
         if w.shape != (2 * N, K) or out.shape != (M, N) or out.stride(1) != 1:
             raise KernelError(f"gemm_normed_glu: w {tuple(w.shape)} out {tuple(out.shape)} for rows {tuple(rows.shape)}")
-        self._check(self.lib.axk_gemm_normed_glu(_ptr(rows), rows.stride(0), _ptr(gain), self._vec_flag(gain, "norm gain"),
-                                                 float(eps), _ptr(w), _ptr(out), out.stride(0), M, N, K, _stream()))
+        self._check(self.run.axk_gemm_normed_glu(_ptr(rows), rows.stride(0), _ptr(gain), self._vec_flag(gain, "norm gain"),
+                                                 float(eps), _ptr(w), _ptr(out), out.stride(0), M, N, K, _queue()))
         return out
 
     def gemm_normed_qkv_rope(self, rows, gain, eps, w, bias, qkv, table, positions, seq_rows, block_table, k_cache, v_cache,
@@ -490,11 +532,11 @@ class Kernels:
             raise KernelError(f"gemm_normed_qkv_rope: bias of {bias.numel()} for {n} rows")
         if write_kv:
             self._check_caches(k_cache, v_cache, n_kv_heads, page_size, head_dim)
-        self._check(self.lib.axk_gemm_normed_qkv_rope(
+        self._check(self.run.axk_gemm_normed_qkv_rope(
             _ptr(rows), rows.stride(0), _ptr(gain), self._vec_flag(gain, "norm gain"), float(eps), _ptr(w), _ptr(bias),
             self._vec_flag(bias, "qkv bias"), _ptr(qkv), qkv.stride(0), M, K, _ptr(table), _ptr(positions), _ptr(seq_rows),
             _ptr(block_table), block_table.shape[-1], _ptr(k_cache if write_kv else None),
-            _ptr(v_cache if write_kv else None), n_heads, n_kv_heads, head_dim, page_size, 1 if write_kv else 0, _stream()))
+            _ptr(v_cache if write_kv else None), n_heads, n_kv_heads, head_dim, page_size, 1 if write_kv else 0, _queue()))
 
     def attention(self, q, q_stride, k_cache, v_cache, block_table, positions, seq_rows, out, n_heads, n_kv_heads,
                   head_dim, page_size, window, scale) -> torch.Tensor:
@@ -505,20 +547,20 @@ class Kernels:
         if out.shape != (T, n_heads * head_dim) or not out.is_contiguous():
             raise KernelError(f"attention: out {tuple(out.shape)} is not [{T}, {n_heads * head_dim}]")
         self._check_caches(k_cache, v_cache, n_kv_heads, page_size, head_dim)
-        self._check(self.lib.axk_attention(
+        self._check(self.run.axk_attention(
             _ptr(q), q_stride, _ptr(k_cache), _ptr(v_cache), _ptr(block_table), block_table.shape[-1], _ptr(positions),
-            _ptr(seq_rows), _ptr(out), T, n_heads, n_kv_heads, head_dim, page_size, window, float(scale), _stream()))
+            _ptr(seq_rows), _ptr(out), T, n_heads, n_kv_heads, head_dim, page_size, window, float(scale), _queue()))
         return out
 
     def attention_fast_ok(self, head_dim: int, page_size: int, n_heads: int, n_kv_heads: int) -> bool:
         """Whether the bfloat16 build's attention kernels on the matrix cores take these sizes (never in float32,
         whose own `attention_blocks_ok` answers for)."""
-        return bool(self.lib.axk_attention_fast_ok(head_dim, page_size, n_heads, n_kv_heads))
+        return bool(self.run.axk_attention_fast_ok(head_dim, page_size, n_heads, n_kv_heads))
 
     def attention_blocks_ok(self, head_dim: int, page_size: int, n_heads: int, n_kv_heads: int) -> bool:
         """Whether `attention_prefill` and `attention_decode` take these sizes in this build (float32: on the
         32-bit matrix cores, with the bits of `attention`)."""
-        return bool(self.lib.axk_attention_blocks_ok(head_dim, page_size, n_heads, n_kv_heads))
+        return bool(self.run.axk_attention_blocks_ok(head_dim, page_size, n_heads, n_kv_heads))
 
     def attention_prefill(self, q, q_stride, k_cache, v_cache, block_table, positions, seq_rows, out, tiles, n_heads,
                           n_kv_heads, head_dim, page_size, window, scale) -> torch.Tensor:
@@ -534,35 +576,35 @@ class Kernels:
         if (out.shape[1] != n_heads * head_dim or not out.is_contiguous() or tiles.dim() != 2 or tiles.shape[1] != 4
                 or not tiles.is_contiguous()):
             raise KernelError(f"attention_prefill: out {tuple(out.shape)}, tiles {tuple(tiles.shape)}")
-        self._check(self.lib.axk_attention_prefill(
+        self._check(self.run.axk_attention_prefill(
             _ptr(q), q_stride, _ptr(k_cache), _ptr(v_cache), _ptr(block_table), block_table.shape[-1], _ptr(positions),
             _ptr(seq_rows), _ptr(out), _ptr(tiles), tiles.shape[0], n_heads, n_kv_heads, head_dim, page_size, window,
-            float(scale), _stream()))
+            float(scale), _queue()))
         return out
 
     @property
     def attention_prefill_tile(self) -> int:
         """The most consecutive tokens of one request in a run of `attention_prefill`'s tiles."""
-        return int(self.lib.axk_attention_prefill_tile())
+        return int(self.run.axk_attention_prefill_tile())
 
     def _decode_chunk_and_factor(self):
         if self._chunk_factor is None:
-            self._chunk_factor = (int(self.lib.axk_attention_decode_chunk()), int(self.lib.axk_attention_decode_item_factor()))
+            self._chunk_factor = (int(self.run.axk_attention_decode_chunk()), int(self.run.axk_attention_decode_item_factor()))
         return self._chunk_factor
 
     @property
     def attention_decode_chunk(self) -> int:
         """Positions of one chunk of the decoding kernel: a token's range (from the chunk that
         holds the window's first position, or 0) is cut into chunks of this size."""
-        return int(self.lib.axk_attention_decode_chunk())
+        return int(self.run.axk_attention_decode_chunk())
 
     @property
     def attention_decode_max_context(self) -> int:
         """The longest context the decoding kernel's work list can name."""
-        return self.attention_decode_chunk * int(self.lib.axk_attention_decode_item_factor())
+        return self.attention_decode_chunk * int(self.run.axk_attention_decode_item_factor())
 
     def attention_decode_workspace(self, n_tokens: int, n_heads: int, head_dim: int, max_chunks: int) -> int:
-        return int(self.lib.axk_attention_decode_workspace(n_tokens, n_heads, head_dim, max_chunks))
+        return int(self.run.axk_attention_decode_workspace(n_tokens, n_heads, head_dim, max_chunks))
 
     def attention_decode_work(self, positions: Sequence[int], window: int, pad_to: int = 0) -> List[int]:
         """The work list of the decoding kernel for single tokens at `positions` (in the order
@@ -609,25 +651,25 @@ class Kernels:
         self._i32(work, "attention work list")
         if work.dim() != 1 or not work.is_contiguous():
             raise KernelError(f"attention_decode: work list {tuple(work.shape)}")
-        self._check(self.lib.axk_attention_decode(
+        self._check(self.run.axk_attention_decode(
             _ptr(q), q_stride, _ptr(k_cache), _ptr(v_cache), _ptr(block_table), block_table.shape[-1], _ptr(positions),
             _ptr(seq_rows), _ptr(out), _ptr(token_index), n, _ptr(work), work.numel(),
             _ptr(partial), max_chunks, n_heads, n_kv_heads, head_dim, page_size, window,
-            float(scale), _stream()))
+            float(scale), _queue()))
         return out
 
     def pack_ok(self, rows: int, cols: int, gated: bool = False) -> bool:
         """Whether a [rows, cols] matrix can be packed for the matrix-core products (gated: a
         [gate; up] matrix for the SwiGLU epilogue).  Never in the float32 build."""
-        return bool(self.lib.axk_pack_ok(rows, cols, 1 if gated else 0))
+        return bool(self.run.axk_pack_ok(rows, cols, 1 if gated else 0))
 
     def pack_matrix(self, w: torch.Tensor) -> PackedMatrix:
         self._elem(w, "pack_matrix")
         if w.dim() != 2 or not w.is_contiguous() or not self.pack_ok(w.shape[0], w.shape[1]):
             raise KernelError(f"pack_matrix: {tuple(w.shape)} cannot be packed")
         rows, cols = w.shape
-        out = torch.empty(self.lib.axk_packed_elems(rows, cols), dtype=w.dtype, device=w.device)
-        self._check(self.lib.axk_pack_matrix(_ptr(w), _ptr(out), rows, cols, _stream()))
+        out = torch.empty(self.run.axk_packed_elems(rows, cols), dtype=w.dtype, device=w.device)
+        self._check(self.run.axk_pack_matrix(_ptr(w), _ptr(out), rows, cols, _queue()))
         return PackedMatrix(out, rows, cols)
 
     def prepare_weight(self, w: torch.Tensor, gated: bool = False):
@@ -640,13 +682,13 @@ class Kernels:
     def gemm_then_norm_ok(self, m: int, n: int, k: int) -> bool:
         """Whether the product that adds into [m, n] float32 rows can also write the RMS norm of
         the new rows (see `gemm`: `following_norm`)."""
-        return bool(self.lib.axk_gemm_then_norm_ok(m, n, k))
+        return bool(self.run.axk_gemm_then_norm_ok(m, n, k))
 
     def gemm_segments(self, n: int, k: int, gated: bool = False) -> int:
         """The number of contiguous segments of K whose sums a product with a packed [n, k]
         matrix adds in ascending order (gated: a [gate; up] matrix for n output columns).  It
         depends on the matrix alone: a row's bits do not depend on the other rows of a step."""
-        return int(self.lib.axk_gemm_segments(n, k, 1 if gated else 0))
+        return int(self.run.axk_gemm_segments(n, k, 1 if gated else 0))
 
     def gemm(self, x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, bias: Optional[torch.Tensor] = None,
              mode: int = MODE_STORE, following_norm=None) -> torch.Tensor:
@@ -675,12 +717,12 @@ class Kernels:
             raise KernelError(f"gemm: mode {mode} writes {want}, out is {out.dtype}")
         if bias is not None and bias.numel() != N:
             raise KernelError(f"gemm: bias of {bias.numel()} for {N} columns")
-        need = self.lib.axk_gemm_workspace(M, N, K, mode) if packed else 0
+        need = self.run.axk_gemm_workspace(M, N, K, mode) if packed else 0
         work = torch.empty(need // 4, dtype=torch.float32, device=x.device) if need > 0 else None
         if following_norm is None:
-            self._check(self.lib.axk_gemm(_ptr(x), x.stride(0), _ptr(w), 1 if packed else 0, _ptr(bias),
+            self._check(self.run.axk_gemm(_ptr(x), x.stride(0), _ptr(w), 1 if packed else 0, _ptr(bias),
                                           self._vec_flag(bias, "gemm bias"), _ptr(out), out.stride(0), M, N, K, mode,
-                                          _ptr(work), need, _stream()))
+                                          _ptr(work), need, _queue()))
             return out
         gain, values, norm_eps = following_norm
         self._elem(values, "gemm norm values")
@@ -689,10 +731,10 @@ class Kernels:
         if gain.numel() != N or values.shape != (M, N) or not values.is_contiguous():
             raise KernelError(f"gemm: the following norm's gain {tuple(gain.shape)} or values "
                               f"{tuple(values.shape)} do not fit [{M}, {N}]")
-        self._check(self.lib.axk_gemm_then_norm(
+        self._check(self.run.axk_gemm_then_norm(
             _ptr(x), x.stride(0), _ptr(w), _ptr(bias), self._vec_flag(bias, "gemm bias"), _ptr(out), out.stride(0),
             M, N, K, _ptr(gain), self._vec_flag(gain, "gemm norm gain"), float(norm_eps), _ptr(values), _ptr(work),
-            need, _stream()))
+            need, _queue()))
         return out
 
     def swiglu(self, gate_up: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
@@ -700,7 +742,7 @@ class Kernels:
         T, F = out.shape
         if gate_up.shape != (T, 2 * F) or not gate_up.is_contiguous() or not out.is_contiguous():
             raise KernelError(f"swiglu: in {tuple(gate_up.shape)} out {tuple(out.shape)}")
-        self._check(self.lib.axk_swiglu(_ptr(gate_up), _ptr(out), T, F, _stream()))
+        self._check(self.run.axk_swiglu(_ptr(gate_up), _ptr(out), T, F, _queue()))
         return out
 
     def argmax(self, logits: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
@@ -708,8 +750,8 @@ class Kernels:
         if logits.dtype != torch.float32 or not logits.is_cuda or logits.stride(1) != 1 or out.numel() != logits.shape[0]:
             raise KernelError(f"argmax: logits {tuple(logits.shape)} {logits.dtype}, picks {out.numel()}")
         rows, n = logits.shape
-        work = torch.empty(max(1, self.lib.axk_argmax_workspace(rows, n) // 8), dtype=torch.int64, device=logits.device)
-        self._check(self.lib.axk_argmax(_ptr(logits), logits.stride(0), _ptr(out), rows, n, _ptr(work), _stream()))
+        work = torch.empty(max(1, self.run.axk_argmax_workspace(rows, n) // 8), dtype=torch.int64, device=logits.device)
+        self._check(self.run.axk_argmax(_ptr(logits), logits.stride(0), _ptr(out), rows, n, _ptr(work), _queue()))
         return out
 
     def topk(self, logits, recent, n_recent, penalty, k_of_row, cands, k_max: Optional[int] = None) -> torch.Tensor:
@@ -725,11 +767,11 @@ class Kernels:
             k_max = int(k_of_row.max())
         if k_max > cands.shape[1]:
             raise KernelError(f"topk: k up to {k_max} for {cands.shape[1]} candidate places")
-        need = self.lib.axk_topk_workspace(rows, n, cands.shape[1])
+        need = self.run.axk_topk_workspace(rows, n, cands.shape[1])
         work = torch.empty(max(need, 8) // 8, dtype=torch.int64, device=logits.device)
-        self._check(self.lib.axk_topk(_ptr(logits), logits.stride(0), _ptr(recent), recent.shape[1], _ptr(n_recent),
+        self._check(self.run.axk_topk(_ptr(logits), logits.stride(0), _ptr(recent), recent.shape[1], _ptr(n_recent),
                                       _ptr(penalty), _ptr(k_of_row), _ptr(cands), cands.shape[1], rows, n, _ptr(work),
-                                      _stream()))
+                                      _queue()))
         return cands
 
     # ------------------------------------------------------------------ a norm on a sublayer's output, roundings, activations
@@ -743,8 +785,8 @@ class Kernels:
             self._elem(rounded, "norm_add rounded")
             if rounded.shape != x.shape or not rounded.is_contiguous():
                 raise KernelError(f"norm_add: rounded {tuple(rounded.shape)} is not {tuple(x.shape)} contiguous")
-        self._check(self.lib.axk_norm_add(_ptr(y), _ptr(gain), self._vec_flag(gain, "norm_add gain"), float(eps), float(mult),
-                                          _ptr(x), _ptr(rounded), x.shape[0], x.shape[1], _stream()))
+        self._check(self.run.axk_norm_add(_ptr(y), _ptr(gain), self._vec_flag(gain, "norm_add gain"), float(eps), float(mult),
+                                          _ptr(x), _ptr(rounded), x.shape[0], x.shape[1], _queue()))
         return x
 
     def tanh_norm(self, x: torch.Tensor, norm, out: torch.Tensor, rows: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -757,8 +799,8 @@ class Kernels:
             n = rows.numel()
         if x.dim() != 2 or out.shape != (n, x.shape[1]) or not out.is_contiguous() or w.numel() != x.shape[1] or b.numel() != x.shape[1]:
             raise KernelError(f"tanh_norm: x {tuple(x.shape)}, out {tuple(out.shape)}, vectors of {w.numel()} and {b.numel()}")
-        self._check(self.lib.axk_tanh_norm(_ptr(x), _ptr(rows), float(alpha), _ptr(w), self._vec_flag(w, "tanh_norm w"), _ptr(b),
-                                           self._vec_flag(b, "tanh_norm b"), _ptr(out), n, x.shape[1], _stream()))
+        self._check(self.run.axk_tanh_norm(_ptr(x), _ptr(rows), float(alpha), _ptr(w), self._vec_flag(w, "tanh_norm w"), _ptr(b),
+                                           self._vec_flag(b, "tanh_norm b"), _ptr(out), n, x.shape[1], _queue()))
         return out
 
     def tanh_norm_add(self, y: torch.Tensor, norm, x: torch.Tensor, following=None) -> torch.Tensor:
@@ -773,10 +815,10 @@ class Kernels:
             if values.shape != x.shape or not values.is_contiguous():
                 raise KernelError(f"tanh_norm_add: values {tuple(values.shape)} are not {tuple(x.shape)} contiguous")
         flag = lambda v: self._vec_flag(v, "tanh_norm_add vector")
-        self._check(self.lib.axk_tanh_norm_add(
+        self._check(self.run.axk_tanh_norm_add(
             _ptr(y), float(norm[0]), _ptr(norm[1]), flag(norm[1]), _ptr(norm[2]), flag(norm[2]), _ptr(x), _ptr(values),
             float(next_norm[0]), _ptr(next_norm[1]), flag(next_norm[1]), _ptr(next_norm[2]), flag(next_norm[2]), x.shape[0],
-            x.shape[1], _stream()))
+            x.shape[1], _queue()))
         return x
 
     NORM_KINDS = {"rms": 0, "layer": 1}
@@ -792,8 +834,8 @@ class Kernels:
             self._elem(rounded, "sum_norm rounded")
             if rounded.shape != x.shape or not rounded.is_contiguous():
                 raise KernelError(f"sum_norm: rounded {tuple(rounded.shape)} is not {tuple(x.shape)} contiguous")
-        self._check(self.lib.axk_sum_norm(_ptr(y), float(alpha), _ptr(gain), self._vec_flag(gain, "sum_norm gain"), float(eps),
-                                          self.NORM_KINDS[kind], _ptr(x), _ptr(rounded), x.shape[0], x.shape[1], _stream()))
+        self._check(self.run.axk_sum_norm(_ptr(y), float(alpha), _ptr(gain), self._vec_flag(gain, "sum_norm gain"), float(eps),
+                                          self.NORM_KINDS[kind], _ptr(x), _ptr(rounded), x.shape[0], x.shape[1], _queue()))
         return x
 
     def layernorm(self, x: torch.Tensor, gain: torch.Tensor, eps: float, out: torch.Tensor,
@@ -806,22 +848,22 @@ class Kernels:
             n = rows.numel()
         if x.dim() != 2 or out.shape != (n, x.shape[1]) or not out.is_contiguous() or gain.numel() != x.shape[1]:
             raise KernelError(f"layernorm: x {tuple(x.shape)}, out {tuple(out.shape)}, a gain of {gain.numel()}")
-        self._check(self.lib.axk_layernorm(_ptr(x), _ptr(rows), _ptr(gain), self._vec_flag(gain, "layernorm gain"), _ptr(out), n,
-                                           x.shape[1], float(eps), _stream()))
+        self._check(self.run.axk_layernorm(_ptr(x), _ptr(rows), _ptr(gain), self._vec_flag(gain, "layernorm gain"), _ptr(out), n,
+                                           x.shape[1], float(eps), _queue()))
         return out
 
     def softcap(self, v: torch.Tensor, cap: float) -> torch.Tensor:
         """v = cap tanh(v / cap) in place on float32 rows."""
         if v.dtype != torch.float32 or not v.is_cuda or v.dim() != 2 or v.stride(1) != 1:
             raise KernelError(f"softcap: {tuple(v.shape)} {v.dtype} with strides {v.stride()}")
-        self._check(self.lib.axk_softcap(_ptr(v), v.stride(0), v.shape[0], v.shape[1], float(cap), _stream()))
+        self._check(self.run.axk_softcap(_ptr(v), v.stride(0), v.shape[0], v.shape[1], float(cap), _queue()))
         return v
 
     def scale_rows(self, v: torch.Tensor, factor: float) -> torch.Tensor:
         """v *= factor in place on float32 rows."""
         if v.dtype != torch.float32 or not v.is_cuda or v.dim() != 2 or v.stride(1) != 1:
             raise KernelError(f"scale_rows: {tuple(v.shape)} {v.dtype} with strides {v.stride()}")
-        self._check(self.lib.axk_scale_rows(_ptr(v), v.stride(0), v.shape[0], v.shape[1], float(factor), _stream()))
+        self._check(self.run.axk_scale_rows(_ptr(v), v.stride(0), v.shape[0], v.shape[1], float(factor), _queue()))
         return v
 
     def add_scaled(self, x: torch.Tensor, y: torch.Tensor, factor: float = 1.0) -> torch.Tensor:
@@ -829,14 +871,14 @@ class Kernels:
         self._f32(x, "add_scaled x"); self._f32(y, "add_scaled y")
         if x.shape != y.shape or not x.is_contiguous() or not y.is_contiguous():
             raise KernelError(f"add_scaled: {tuple(x.shape)} and {tuple(y.shape)}")
-        self._check(self.lib.axk_add_scaled(_ptr(x), _ptr(y), float(factor), x.numel(), _stream()))
+        self._check(self.run.axk_add_scaled(_ptr(x), _ptr(y), float(factor), x.numel(), _queue()))
         return x
 
     def round_rows(self, x: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
         self._f32(x, "round_rows x"); self._elem(out, "round_rows out")
         if out.numel() != x.numel() or not out.is_contiguous():
             raise KernelError(f"round_rows: {tuple(x.shape)} into {tuple(out.shape)}")
-        self._check(self.lib.axk_round_rows(_ptr(x), _ptr(out), x.numel(), _stream()))
+        self._check(self.run.axk_round_rows(_ptr(x), _ptr(out), x.numel(), _queue()))
         return out
 
     ACTIVATIONS = {"gelu_tanh": 0, "gelu_erf": 1, "relu_squared": 2}
@@ -845,7 +887,7 @@ class Kernels:
         self._elem(v, "activation")
         if kind not in self.ACTIVATIONS or not v.is_contiguous():
             raise KernelError(f"activation: '{kind}' on a tensor of strides {v.stride()}")
-        self._check(self.lib.axk_activation(_ptr(v), v.numel(), self.ACTIVATIONS[kind], _stream()))
+        self._check(self.run.axk_activation(_ptr(v), v.numel(), self.ACTIVATIONS[kind], _queue()))
         return v
 
     def concat_round(self, a: torch.Tensor, b: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
@@ -854,7 +896,7 @@ class Kernels:
         if a.dim() != 2 or b.dim() != 2 or a.shape[0] != b.shape[0] or out.shape != (a.shape[0], a.shape[1] + b.shape[1]) \
                 or not out.is_contiguous():
             raise KernelError(f"concat_round: {tuple(a.shape)} and {tuple(b.shape)} into {tuple(out.shape)}")
-        self._check(self.lib.axk_concat_round(_ptr(a), a.shape[1], _ptr(b), b.shape[1], _ptr(out), a.shape[0], _stream()))
+        self._check(self.run.axk_concat_round(_ptr(a), a.shape[1], _ptr(b), b.shape[1], _ptr(out), a.shape[0], _queue()))
         return out
 
     def clamped_glu(self, gate_up: torch.Tensor, out: torch.Tensor, limit: float, alpha: float) -> torch.Tensor:
@@ -862,7 +904,7 @@ class Kernels:
         T, F = out.shape
         if gate_up.shape != (T, 2 * F) or not gate_up.is_contiguous() or not out.is_contiguous():
             raise KernelError(f"clamped_glu: in {tuple(gate_up.shape)} out {tuple(out.shape)}")
-        self._check(self.lib.axk_clamped_glu(_ptr(gate_up), _ptr(out), T, F, float(limit), float(alpha), _stream()))
+        self._check(self.run.axk_clamped_glu(_ptr(gate_up), _ptr(out), T, F, float(limit), float(alpha), _queue()))
         return out
 
     # ------------------------------------------------------------------ grouped products
@@ -915,16 +957,16 @@ class Kernels:
             if not row_scale.is_contiguous() or row_scale.numel() < (M if routed is not None else out.shape[0]):
                 raise KernelError(f"grouped_gemm: {row_scale.numel()} row factors for {M} rows")
         limit, alpha, shift = (tuple(glu) + (1.0,))[:3] if glu else (0.0, 0.0, 0.0)
-        self._check(self.lib.axk_grouped_gemm(
+        self._check(self.run.axk_grouped_gemm(
             _ptr(x), 1 if x.dtype == torch.float32 else 0, x.stride(0), x_group_stride, _ptr(x_rows), _ptr(w), _ptr(bias),
             self._vec_flag(bias, "grouped bias"), _ptr(out), 1 if out.dtype == torch.float32 else 0, out.stride(0),
             out_group_stride, _ptr(out_rows), _ptr(gate), 0 if gate is None else gate.stride(0), 1 if gate_per_group else 0,
-            _ptr(row_scale), 1 if glu else 0, float(limit), float(alpha), float(shift), _ptr(tiles), _ptr(n_tiles), int(max_tiles), int(tile_rows), M, N, K, G, _stream()))
+            _ptr(row_scale), 1 if glu else 0, float(limit), float(alpha), float(shift), _ptr(tiles), _ptr(n_tiles), int(max_tiles), int(tile_rows), M, N, K, G, _queue()))
         return out
 
     def grouped_gemm_wide(self, pairs: int, groups: int, n: int, k: int) -> bool:
         """Whether a gated routed product of `pairs` rows over `groups` matrices [2 n, k] is the faster for a list of tiles of 128 rows."""
-        return bool(self.lib.axk_grouped_gemm_wide(pairs, groups, n, k))
+        return bool(self.run.axk_grouped_gemm_wide(pairs, groups, n, k))
 
     # ------------------------------------------------------------------ routing
     def route_topk(self, logits: torch.Tensor, top: int, experts: torch.Tensor, weights: torch.Tensor) -> None:
@@ -932,7 +974,7 @@ class Kernels:
         T, E = logits.shape
         if experts.shape != (T, top) or weights.shape != (T, top):
             raise KernelError(f"route_topk: {tuple(experts.shape)} / {tuple(weights.shape)} for {T} x {top}")
-        self._check(self.lib.axk_route_topk(_ptr(logits), T, E, top, _ptr(experts), _ptr(weights), _stream()))
+        self._check(self.run.axk_route_topk(_ptr(logits), T, E, top, _ptr(experts), _ptr(weights), _queue()))
 
     def route_scored(self, logits: torch.Tensor, correction: Optional[torch.Tensor], top: int, groups: int, keep: int, scale: float,
                      experts: torch.Tensor, weights: torch.Tensor, normalize: bool = True, n_experts: Optional[int] = None,
@@ -953,11 +995,11 @@ class Kernels:
             self._f32(correction, "router correction")
             if correction.numel() != E:
                 raise KernelError(f"route_scored: a correction of {correction.numel()} for {E} experts")
-        self._check(self.lib.axk_route_scored(_ptr(logits), logits.stride(0), _ptr(correction), T, E, top, int(groups), int(keep),
-                                              float(scale), 1 if normalize else 0, 1 if softmax else 0, _ptr(experts), _ptr(weights), _stream()))
+        self._check(self.run.axk_route_scored(_ptr(logits), logits.stride(0), _ptr(correction), T, E, top, int(groups), int(keep),
+                                              float(scale), 1 if normalize else 0, 1 if softmax else 0, _ptr(experts), _ptr(weights), _queue()))
 
     def route_max_tiles(self, n_pairs: int, n_experts: int, tile_rows: int = 16) -> int:
-        return int(self.lib.axk_route_max_tiles(n_pairs, n_experts, tile_rows))
+        return int(self.run.axk_route_max_tiles(n_pairs, n_experts, tile_rows))
 
     def route_sort(self, experts: torch.Tensor, n_experts: int, sorted_pairs, sorted_tokens, tiles, n_tiles, place_of=None,
                    first_of=None, tile_rows: int = 16, wide=None) -> None:
@@ -974,15 +1016,15 @@ class Kernels:
             raise KernelError(f"route_sort: lists too short for {P} pairs of {n_experts} experts")
         if wide is not None and wide_tiles.numel() < 3 * self.route_max_tiles(P, n_experts, wide_rows):
             raise KernelError(f"route_sort: the second list is too short for {P} pairs of {n_experts} experts")
-        self._check(self.lib.axk_route_sort(_ptr(experts), P, n_experts, experts.shape[-1], _ptr(sorted_pairs), _ptr(sorted_tokens),
+        self._check(self.run.axk_route_sort(_ptr(experts), P, n_experts, experts.shape[-1], _ptr(sorted_pairs), _ptr(sorted_tokens),
                                                   _ptr(tiles), _ptr(n_tiles), _ptr(place_of), _ptr(first_of), int(tile_rows),
-                                                  _ptr(wide_tiles), _ptr(n_wide), int(wide_rows), _stream()))
+                                                  _ptr(wide_tiles), _ptr(n_wide), int(wide_rows), _queue()))
 
     def gather_rows(self, x: torch.Tensor, rows: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
         self._elem(x, "gather x"); self._elem(out, "gather out"); self._i32(rows, "gather rows")
         if out.shape != (rows.numel(), x.shape[1]) or x.stride(1) != 1 or not out.is_contiguous():
             raise KernelError(f"gather_rows: {rows.numel()} rows of {tuple(x.shape)} into {tuple(out.shape)}")
-        self._check(self.lib.axk_gather_rows(_ptr(x), x.stride(0), _ptr(rows), _ptr(out), rows.numel(), x.shape[1], _stream()))
+        self._check(self.run.axk_gather_rows(_ptr(x), x.stride(0), _ptr(rows), _ptr(out), rows.numel(), x.shape[1], _queue()))
         return out
 
     def route_combine(self, rows: torch.Tensor, weights: Optional[torch.Tensor], y: torch.Tensor, accumulate: bool = False,
@@ -1020,9 +1062,9 @@ class Kernels:
             self._i32(chosen, "combine experts"); self._elem(given, "combine input")
             if chosen.numel() != T * top or given.shape != y.shape or given.stride(1) != 1:
                 raise KernelError(f"route_combine: experts {tuple(chosen.shape)}, input {tuple(given.shape)} for y {tuple(y.shape)}")
-        self._check(self.lib.axk_route_combine(_ptr(rows), _ptr(weights), _ptr(y), T, top, y.shape[1], 1 if accumulate else 0,
+        self._check(self.run.axk_route_combine(_ptr(rows), _ptr(weights), _ptr(y), T, top, y.shape[1], 1 if accumulate else 0,
                                                _ptr(place_of), _ptr(extra), _ptr(extra_gate), gate_stride, _ptr(chosen), int(n_listed), _ptr(given),
-                                               0 if given is None else given.stride(0), _stream()))
+                                               0 if given is None else given.stride(0), _queue()))
         return y
 
     # ------------------------------------------------------------------ convolution and recurrence with per-request state
@@ -1038,9 +1080,9 @@ class Kernels:
             raise KernelError(f"causal_conv: x {tuple(x.shape)}, w {tuple(w.shape)}, u {tuple(u.shape)}")
         if bias is not None and bias.numel() != C:
             raise KernelError(f"causal_conv: a bias of {bias.numel()} for {C} channels")
-        self._check(self.lib.axk_causal_conv(_ptr(x), x.stride(0), _ptr(w), _ptr(bias), self._vec_flag(bias, "conv bias"),
+        self._check(self.run.axk_causal_conv(_ptr(x), x.stride(0), _ptr(w), _ptr(bias), self._vec_flag(bias, "conv bias"),
                                              _ptr(state), state.stride(0), _ptr(positions), _ptr(seq_rows), _ptr(u), T, C,
-                                             w.shape[1], _stream()))
+                                             w.shape[1], _queue()))
         return u
 
     def gated_scan(self, gates, u, y, x, lam, decay: float, state, spans, positions, seq_rows, out, block_width: int, taps: int):
@@ -1059,15 +1101,15 @@ class Kernels:
             self._i32(spans, "scan spans")
             n = spans.shape[0]
             if T > 4 * n:            # stretches of tokens
-                self._check(self.lib.axk_gated_scan_stretches(
+                self._check(self.run.axk_gated_scan_stretches(
                     _ptr(gates), _ptr(u), _ptr(y), y.stride(0), _ptr(x), x.stride(0), _ptr(lam), self._vec_flag(lam, "scan lam"),
                     float(decay), _ptr(state), state.stride(0), _ptr(spans), n, _ptr(positions), _ptr(out), C, int(block_width),
-                    int(taps), _stream()))
+                    int(taps), _queue()))
                 return out
-        self._check(self.lib.axk_gated_scan(_ptr(gates), _ptr(u), _ptr(y), y.stride(0), _ptr(x), x.stride(0), _ptr(lam),
+        self._check(self.run.axk_gated_scan(_ptr(gates), _ptr(u), _ptr(y), y.stride(0), _ptr(x), x.stride(0), _ptr(lam),
                                             self._vec_flag(lam, "scan lam"), float(decay), _ptr(state), state.stride(0),
                                             _ptr(spans), n, _ptr(positions), _ptr(seq_rows), _ptr(out), C, int(block_width),
-                                            int(taps), None, T, _stream()))
+                                            int(taps), None, T, _queue()))
         return out
 
     # ------------------------------------------------------------------ a state-space mixer with per-request state
@@ -1091,11 +1133,11 @@ class Kernels:
             if raw.shape[0] != T or raw.stride(1) != 1 or terms.shape != (T, heads, 2) or not terms.is_contiguous() \
                     or dt_bias.numel() != heads or a_log.numel() != heads:
                 raise KernelError(f"state_conv: raw {tuple(raw.shape)}, terms {tuple(terms.shape)} for {heads} heads")
-        self._check(self.lib.axk_state_conv(
+        self._check(self.run.axk_state_conv(
             _ptr(x), x.stride(0), _ptr(w), _ptr(bias), self._vec_flag(bias, "conv bias"), 1 if silu else 0, _ptr(state),
             state.stride(0), int(copy_elems), int(tail_at), _ptr(positions), _ptr(seq_rows), _ptr(u), T, C, w.shape[1],
             _ptr(raw), 0 if raw is None else raw.stride(0), _ptr(dt_bias), self._vec_flag(dt_bias, "dt bias"), _ptr(a_log),
-            self._vec_flag(a_log, "A_log"), _ptr(terms), heads, _stream()))
+            self._vec_flag(a_log, "A_log"), _ptr(terms), heads, _queue()))
         return u
 
     def state_space_scan(self, u, terms, d_skip, state, copy_elems: int, tail_at: int, spans, positions, seq_rows, conv_in, y,
@@ -1131,10 +1173,10 @@ class Kernels:
                 raise KernelError(f"state_space_scan: segments {tuple(segs.shape)} of requests {tuple(spans5.shape)} for {n} requests")
             ends = torch.empty((n_segs, heads, n_state, vdim), dtype=torch.float32, device=u.device)
             cum = torch.empty((T, heads), dtype=torch.float32, device=u.device)
-        self._check(self.lib.axk_state_space_scan(
+        self._check(self.run.axk_state_space_scan(
             _ptr(u), _ptr(terms), _ptr(d_skip), self._vec_flag(d_skip, "D"), _ptr(state), state.stride(0), int(copy_elems),
             int(tail_at), _ptr(spans), n, _ptr(positions), _ptr(seq_rows), _ptr(conv_in), conv_in.stride(0), _ptr(y), heads,
-            groups, vdim, n_state, taps, _ptr(segs), n_segs, int(longest), _ptr(spans5), _ptr(ends), _ptr(cum), _stream()))
+            groups, vdim, n_state, taps, _ptr(segs), n_segs, int(longest), _ptr(spans5), _ptr(ends), _ptr(cum), _queue()))
         return y
 
     def gated_group_norm(self, y, z, gain, eps: float, out, parts: int) -> torch.Tensor:
@@ -1145,8 +1187,8 @@ class Kernels:
         if z.shape != (T, W) or z.stride(1) != 1 or out.shape != (T, W) or not y.is_contiguous() or not out.is_contiguous() \
                 or gain.numel() != W or parts < 1 or W % parts:
             raise KernelError(f"gated_group_norm: y {tuple(y.shape)}, z {tuple(z.shape)}, out {tuple(out.shape)}, {parts} parts")
-        self._check(self.lib.axk_gated_group_norm(_ptr(y), _ptr(z), z.stride(0), _ptr(gain), self._vec_flag(gain, "group norm gain"),
-                                                  float(eps), _ptr(out), T, W, int(parts), _stream()))
+        self._check(self.run.axk_gated_group_norm(_ptr(y), _ptr(z), z.stride(0), _ptr(gain), self._vec_flag(gain, "group norm gain"),
+                                                  float(eps), _ptr(out), T, W, int(parts), _queue()))
         return out
 
     # ------------------------------------------------------------------ time mixing and the delta rule, with per-request state
@@ -1163,8 +1205,8 @@ class Kernels:
         self._state_rows(state, seq_rows, positions, T, "token_shift")
         if not h.is_contiguous() or mu.dim() != 2 or mu.shape[1] != W or out.shape != (mu.shape[0], T, W) or not out.is_contiguous():
             raise KernelError(f"token_shift: h {tuple(h.shape)}, mu {tuple(mu.shape)}, out {tuple(out.shape)}")
-        self._check(self.lib.axk_token_shift(_ptr(h), _ptr(mu), mu.shape[0], _ptr(state), state.stride(0), int(copy_elems), int(tail_at),
-                                             _ptr(positions), _ptr(seq_rows), _ptr(out), T, W, _stream()))
+        self._check(self.run.axk_token_shift(_ptr(h), _ptr(mu), mu.shape[0], _ptr(state), state.stride(0), int(copy_elems), int(tail_at),
+                                             _ptr(positions), _ptr(seq_rows), _ptr(out), T, W, _queue()))
         return out
 
     def time_mix_decay(self, low, w2, w0, w) -> torch.Tensor:
@@ -1174,8 +1216,8 @@ class Kernels:
         T, C = w.shape
         if low.dim() != 2 or low.shape[0] != T or w2.shape != (C, low.shape[1]) or not w2.is_contiguous() or w0.numel() != C:
             raise KernelError(f"time_mix_decay: low {tuple(low.shape)}, w2 {tuple(w2.shape)}, w {tuple(w.shape)}")
-        self._check(self.lib.axk_time_mix_decay(_ptr(low), _ptr(w2), _ptr(w0), self._vec_flag(w0, "decay w0"), _ptr(w), T, C,
-                                                low.shape[1], _stream()))
+        self._check(self.run.axk_time_mix_decay(_ptr(low), _ptr(w2), _ptr(w0), self._vec_flag(w0, "decay w0"), _ptr(w), T, C,
+                                                low.shape[1], _queue()))
         return w
 
     def wkv_scan(self, rows, r_at: int, k_at: int, v_at: int, w, u, state, copy_elems: int, tail_at: int, spans, positions, seq_rows,
@@ -1206,10 +1248,10 @@ class Kernels:
                 raise KernelError(f"wkv_scan: segments {tuple(segs.shape)} of requests {tuple(spans5.shape)} for {n} requests")
             take = lambda *shape: torch.empty(shape, dtype=torch.float32, device=y.device)
             ends, decays, rc = take(n_segs, heads, values, keys), take(n_segs, heads, keys), take(T, heads * keys)
-        self._check(self.lib.axk_wkv_scan(
+        self._check(self.run.axk_wkv_scan(
             _ptr(rows), rows.stride(0), int(r_at), int(k_at), int(v_at), _ptr(w), _ptr(u), _ptr(state), state.stride(0), int(copy_elems),
             int(tail_at), _ptr(spans), n, _ptr(positions), _ptr(seq_rows), _ptr(h_in), h_in.shape[1], _ptr(y), heads, keys, values,
-            _ptr(segs), n_segs, int(longest), _ptr(spans5), _ptr(ends), _ptr(decays), _ptr(rc), _stream()))
+            _ptr(segs), n_segs, int(longest), _ptr(spans5), _ptr(ends), _ptr(decays), _ptr(rc), _queue()))
         return y
 
     def delta_prepare(self, rows, w, state, copy_elems: int, tail_at: int, positions, seq_rows, beta_at: int, decay_at: int, a_log,
@@ -1223,10 +1265,10 @@ class Kernels:
         if C != 2 * kv_heads * keys + heads * values or rows.shape[0] != T or w.dim() != 2 or w.shape[0] != C or not w.is_contiguous() \
                 or terms.shape != (T, heads, 2) or (a_log is not None and (a_log.numel() != heads or dt_bias.numel() != heads)):
             raise KernelError(f"delta_prepare: rows {tuple(rows.shape)}, conv {tuple(w.shape)}, u {tuple(u.shape)}, terms {tuple(terms.shape)}")
-        self._check(self.lib.axk_delta_prepare(
+        self._check(self.run.axk_delta_prepare(
             _ptr(rows), rows.stride(0), _ptr(w), w.shape[1], _ptr(state), state.stride(0), int(copy_elems), int(tail_at), _ptr(positions),
             _ptr(seq_rows), int(beta_at), int(decay_at), _ptr(a_log), self._vec_flag(a_log, "A_log"), _ptr(dt_bias),
-            self._vec_flag(dt_bias, "dt bias"), _ptr(u), _ptr(terms), T, heads, kv_heads, keys, values, float(q_scale), _stream()))
+            self._vec_flag(dt_bias, "dt bias"), _ptr(u), _ptr(terms), T, heads, kv_heads, keys, values, float(q_scale), _queue()))
 
     def delta_scan(self, u, terms, state, copy_elems: int, tail_at: int, spans, positions, seq_rows, conv_in, y, heads: int,
                    kv_heads: int, keys: int, values: int, taps: int, chunks=None, decay=None) -> torch.Tensor:
@@ -1257,22 +1299,22 @@ class Kernels:
             self._i32(list_, "delta chunks"); self._i32(spans5, "delta requests")
             if spans is None or list_.dim() != 2 or list_.shape[1] != 2 or spans5.dim() != 2 or spans5.shape[1] != 5:
                 raise KernelError(f"delta_scan: chunks {tuple(list_.shape)} of requests {tuple(spans5.shape)}")
-            need = int(self.lib.axk_delta_chunked_workspace(list_.shape[0], heads, keys, values))
+            need = int(self.run.axk_delta_chunked_workspace(list_.shape[0], heads, keys, values))
             work = torch.empty(need, dtype=torch.float32, device=y.device)
-            self._check(self.lib.axk_delta_chunked(
+            self._check(self.run.axk_delta_chunked(
                 _ptr(u), _ptr(terms), _ptr(decay), _ptr(state), state.stride(0), int(copy_elems), int(tail_at), _ptr(list_), list_.shape[0], _ptr(spans5),
                 spans5.shape[0], _ptr(positions), _ptr(conv_in), conv_in.stride(0), _ptr(y), heads, kv_heads, keys, values, int(taps),
-                _ptr(work), need, _stream()))
+                _ptr(work), need, _queue()))
             if n == 0:
                 return y
-        self._check(self.lib.axk_delta_scan(
+        self._check(self.run.axk_delta_scan(
             _ptr(u), _ptr(terms), _ptr(decay), _ptr(state), state.stride(0), int(copy_elems), int(tail_at), _ptr(spans), n, _ptr(positions),
-            _ptr(seq_rows), _ptr(conv_in), conv_in.stride(0), _ptr(y), heads, kv_heads, keys, values, int(taps), _stream()))
+            _ptr(seq_rows), _ptr(conv_in), conv_in.stride(0), _ptr(y), heads, kv_heads, keys, values, int(taps), _queue()))
         return y
 
     def delta_chunked_ok(self, kv_heads: int, heads: int, keys: int, values: int) -> bool:
         """Whether `delta_scan` takes `chunks` at these sizes."""
-        return bool(self.lib.axk_delta_chunked_ok(kv_heads, heads, keys, values))
+        return bool(self.run.axk_delta_chunked_ok(kv_heads, heads, keys, values))
 
     def delta_low_rank(self, rows, decay=None, gate=None) -> None:
         """Decays and gates of low rank, from columns of the projections' float32 rows [T, .]: decay = (first column, w
@@ -1291,10 +1333,10 @@ class Kernels:
         if d_w is not None and (d_bias.numel() != d_w.shape[0] or d_w.shape[0] % a_log.numel()):
             raise KernelError(f"delta_low_rank: {d_bias.numel()} biases and {a_log.numel()} heads for {d_w.shape[0]} decays")
         size = lambda w, i: 0 if w is None else w.shape[i]
-        self._check(self.lib.axk_delta_low_rank(
+        self._check(self.run.axk_delta_low_rank(
             _ptr(rows), rows.stride(0), int(d_at), size(d_w, 1), _ptr(d_w), _ptr(d_bias), self._vec_flag(d_bias, "dt bias"), _ptr(a_log),
             self._vec_flag(a_log, "A_log"), 1 if d_w is None else d_w.shape[0] // a_log.numel(), _ptr(d_out), size(d_w, 0), int(g_at),
-            size(g_w, 1), _ptr(g_w), _ptr(g_out), size(g_w, 0), T, _stream()))
+            size(g_w, 1), _ptr(g_w), _ptr(g_out), size(g_w, 0), T, _queue()))
 
     GATES = {"silu": 0, "sigmoid": 1}
 
@@ -1305,21 +1347,21 @@ class Kernels:
         T, W = y.shape
         if W % heads or gate.shape != (T, W) or out.shape != (T, W) or not out.is_contiguous() or gain.numel() not in (W, W // heads):
             raise KernelError(f"head_norm_gate: y {tuple(y.shape)}, gate {tuple(gate.shape)}, a gain of {gain.numel()}, {heads} heads")
-        self._check(self.lib.axk_head_norm_gate(_ptr(y), _ptr(gate), gate.stride(0), _ptr(gain), self._vec_flag(gain, "head norm gain"),
+        self._check(self.run.axk_head_norm_gate(_ptr(y), _ptr(gate), gate.stride(0), _ptr(gain), self._vec_flag(gain, "head norm gain"),
                                                 1 if gain.numel() == W else 0, self.GATES[act], float(eps), _ptr(out), T, heads, W // heads,
-                                                _stream()))
+                                                _queue()))
         return out
 
     # ------------------------------------------------------------------ linear attention with a constant decay a head
     def silu_rows(self, rows, columns: int) -> torch.Tensor:
         """silu in place over the first `columns` numbers of float32 rows."""
         self._f32_rows(rows, "silu rows")
-        self._check(self.lib.axk_silu_rows(_ptr(rows), rows.stride(0), int(columns), rows.shape[0], _stream()))
+        self._check(self.run.axk_silu_rows(_ptr(rows), rows.stride(0), int(columns), rows.shape[0], _queue()))
         return rows
 
     def lightning_chunked_ok(self, heads: int, keys: int, values: int, stride: int, q_at: int, k_at: int) -> bool:
         """Whether `lightning_scan` takes `chunks` at these sizes."""
-        return bool(self.lib.axk_lightning_chunked_ok(heads, keys, values, int(stride), int(q_at), int(k_at)))
+        return bool(self.run.axk_lightning_chunked_ok(heads, keys, values, int(stride), int(q_at), int(k_at)))
 
     def lightning_scan(self, rows, q_at: int, k_at: int, v_at: int, silu: bool, decay, state, copy_elems: int, spans, positions, seq_rows,
                        y, heads: int, keys: int, values: int, chunks=None) -> torch.Tensor:
@@ -1343,15 +1385,15 @@ class Kernels:
                 raise KernelError(f"lightning_scan: chunks {tuple(list_.shape)} of requests {tuple(spans5.shape)}")
             need = list_.shape[0] * heads * keys * values
             ends = torch.empty(need, dtype=torch.float32, device=y.device)
-            self._check(self.lib.axk_lightning_chunked(
+            self._check(self.run.axk_lightning_chunked(
                 _ptr(rows), rows.stride(0), int(q_at), int(k_at), int(v_at), _ptr(decay), _ptr(state), state.stride(0), int(copy_elems),
                 _ptr(list_), list_.shape[0], _ptr(spans5), spans5.shape[0], _ptr(positions), _ptr(y), heads, keys, values, _ptr(ends), need,
-                _stream()))
+                _queue()))
             if n == 0:
                 return y
-        self._check(self.lib.axk_lightning_scan(
+        self._check(self.run.axk_lightning_scan(
             _ptr(rows), rows.stride(0), int(q_at), int(k_at), int(v_at), 1 if silu else 0, _ptr(decay), _ptr(state), state.stride(0),
-            int(copy_elems), _ptr(spans), n, _ptr(positions), _ptr(seq_rows), _ptr(y), heads, keys, values, _stream()))
+            int(copy_elems), _ptr(spans), n, _ptr(positions), _ptr(seq_rows), _ptr(y), heads, keys, values, _queue()))
         return y
 
     # ------------------------------------------------------------------ passes over the residual stream
@@ -1366,9 +1408,9 @@ class Kernels:
         if out.shape != (T, dim) or pairs.dim() != 2 or pairs.shape[1] != dim or pairs.shape[0] < 2 or not pairs.is_contiguous() \
                 or not (packed or table.is_contiguous()) or state.dim() != 2 or state.shape[1] != 2:
             raise KernelError(f"embed_pairs: pairs {tuple(pairs.shape)}, out {tuple(out.shape)} for {T} tokens of width {dim}")
-        self._check(self.lib.axk_embed_pairs(
+        self._check(self.run.axk_embed_pairs(
             _ptr(tokens), _ptr(table), 1 if packed else 0, float(scale), _ptr(pairs), pairs.shape[0] - 1, int(mul_prev), int(mul_cur),
-            _ptr(state), _ptr(positions), _ptr(seq_rows), _ptr(out), T, dim, vocab, _stream()))
+            _ptr(state), _ptr(positions), _ptr(seq_rows), _ptr(out), T, dim, vocab, _queue()))
         return out
 
     def scaled_sum(self, terms, x, norm=None, shift=None) -> torch.Tensor:
@@ -1394,8 +1436,8 @@ class Kernels:
                 raise KernelError(f"scaled_sum: a gain of {gain.numel()}, out {tuple(out.shape)} for x {tuple(x.shape)}")
         if shift is not None:
             self._f32(share, "scaled_sum share"); self._state_rows(state, seq_rows, positions, T, "scaled_sum")
-        self._check(self.lib.axk_scaled_sum(*args, _ptr(x), _ptr(gain), float(eps), _ptr(out), _ptr(share), _ptr(state),
-                                            0 if state is None else state.stride(0), _ptr(positions), _ptr(seq_rows), T, W, _stream()))
+        self._check(self.run.axk_scaled_sum(*args, _ptr(x), _ptr(gain), float(eps), _ptr(out), _ptr(share), _ptr(state),
+                                            0 if state is None else state.stride(0), _ptr(positions), _ptr(seq_rows), T, W, _queue()))
         return x
 
     def shifted_norm(self, x, gain, eps: float, share, state, positions, seq_rows, out) -> torch.Tensor:
@@ -1407,8 +1449,8 @@ class Kernels:
         self._state_rows(state, seq_rows, positions, T, "shifted_norm")
         if gain.numel() != W or share.numel() != W or out.shape != (T, W) or not out.is_contiguous():
             raise KernelError(f"shifted_norm: x {tuple(x.shape)}, gain {gain.numel()}, share {share.numel()}, out {tuple(out.shape)}")
-        self._check(self.lib.axk_shifted_norm(_ptr(x), _ptr(gain), float(eps), _ptr(share), _ptr(state), state.stride(0), _ptr(positions),
-                                              _ptr(seq_rows), _ptr(out), T, W, _stream()))
+        self._check(self.run.axk_shifted_norm(_ptr(x), _ptr(gain), float(eps), _ptr(share), _ptr(state), state.stride(0), _ptr(positions),
+                                              _ptr(seq_rows), _ptr(out), T, W, _queue()))
         return out
 
     # ------------------------------------------------------------------ attention over a latent cache
@@ -1427,12 +1469,12 @@ class Kernels:
                 raise KernelError(f"latent_prepare: cq {tuple(cq.shape)} for a query latent of {q_rank}")
         if kv_gain.numel() != rank:
             raise KernelError(f"latent_prepare: a gain of {kv_gain.numel()} for a latent of {rank}")
-        self._check(self.lib.axk_latent_prepare(
+        self._check(self.run.axk_latent_prepare(
             _ptr(fused), fused.stride(0), q_at, q_rank, kv_at, rank, rot, rot_dims, 1 if neighbours else 0, float(magnitude),
             _ptr(q_gain if q_rank else None), self._vec_flag(q_gain if q_rank else None, "q gain"),
             _ptr(kv_gain), self._vec_flag(kv_gain, "kv gain"), float(eps), _ptr(table), _ptr(positions), _ptr(seq_rows),
             _ptr(block_table), block_table.shape[-1], _ptr(cache), page_size, _ptr(cq if q_rank else None), T,
-            1 if write_kv else 0, _stream()))
+            1 if write_kv else 0, _queue()))
 
     def latent_query_rope(self, q, dim, rot, rot_dims, table, q_full, rank, heads, neighbours=False, magnitude=1.0) -> None:
         """q: float32 [T, >= heads (dim + rot)], rows may be strided (a view into a wider product's rows)."""
@@ -1441,8 +1483,8 @@ class Kernels:
         if q.dtype != torch.float32 or not q.is_cuda or q.dim() != 2 or q.shape[1] < heads * (dim + rot) or q.stride(1) != 1 or q_full.shape != (T, heads * (rank + rot)) \
                 or not q_full.is_contiguous():
             raise KernelError(f"latent_query_rope: q {tuple(q.shape)}, q_full {tuple(q_full.shape)}")
-        self._check(self.lib.axk_latent_query_rope(_ptr(q), q.stride(0), dim, rot, rot_dims, 1 if neighbours else 0, float(magnitude),
-                                                   _ptr(table), _ptr(q_full), rank, heads, T, _stream()))
+        self._check(self.run.axk_latent_query_rope(_ptr(q), q.stride(0), dim, rot, rot_dims, 1 if neighbours else 0, float(magnitude),
+                                                   _ptr(table), _ptr(q_full), rank, heads, T, _queue()))
 
     def latent_attention(self, q_full, cache, block_table, positions, seq_rows, o_lat, heads, rank, rot, page_size, window,
                          scale, sink=None, span: int = 0) -> torch.Tensor:
@@ -1460,11 +1502,11 @@ class Kernels:
             self._f32(sink, "latent sink")
             if sink.numel() != heads:
                 raise KernelError(f"latent_attention: {sink.numel()} sinks for {heads} heads")
-        need = int(self.lib.axk_latent_attention_workspace(T, heads, rank, rot, page_size, int(window), int(span)))
+        need = int(self.run.axk_latent_attention_workspace(T, heads, rank, rot, page_size, int(window), int(span)))
         partial = torch.empty(need, dtype=torch.float32, device=o_lat.device) if need else None
-        self._check(self.lib.axk_latent_attention(_ptr(q_full), _ptr(cache), _ptr(block_table), block_table.shape[-1],
+        self._check(self.run.axk_latent_attention(_ptr(q_full), _ptr(cache), _ptr(block_table), block_table.shape[-1],
                                                   _ptr(positions), _ptr(seq_rows), _ptr(o_lat), T, heads, rank, rot, page_size,
-                                                  int(window), int(span), float(scale), _ptr(sink), _ptr(partial), need, _stream()))
+                                                  int(window), int(span), float(scale), _ptr(sink), _ptr(partial), need, _queue()))
         return o_lat
 
     # ------------------------------------------------------------------ attention with maps, masks and bent scores
@@ -1504,16 +1546,16 @@ class Kernels:
                 raise KernelError(f"heads_prepare: a convolution {tuple(w.shape)} of {(n_q + n_k) * dim + v_width} channels")
             if spans is not None:
                 self._i32(spans, "conv spans")
-        self._check(self.lib.axk_heads_prepare(
+        self._check(self.run.axk_heads_prepare(
             _ptr(proj), proj.stride(0), q_at, n_q, k_at, n_k, v_at, v_width, dim, _ptr(q_gain), self._vec_flag(q_gain, "q gain"),
             _ptr(k_gain), self._vec_flag(k_gain, "k gain"), float(eps), rot, 1 if neighbours else 0, float(magnitude), _ptr(table),
             _ptr(positions), _ptr(seq_rows), _ptr(block_table), block_table.shape[-1], _ptr(cache), page_size, _ptr(q_out), T,
             1 if write_kv else 0, float(q_temp[0]) if q_temp else 0.0, int(q_temp[1]) if q_temp else 0, 1 if norm_rows else 0,
             _ptr(w), 0 if w is None else w.shape[1], _ptr(state), 0 if state is None else state.stride(0), int(copy_elems), _ptr(spans),
-            0 if spans is None else spans.shape[0], _stream()))
+            0 if spans is None else spans.shape[0], _queue()))
 
     def masked_attention_uses_mfma(self, heads, kv_heads, maps, dim, vdim, page_size) -> bool:
-        return bool(self.lib.axk_masked_attention_uses_mfma(heads, kv_heads, maps, dim, vdim, page_size))
+        return bool(self.run.axk_masked_attention_uses_mfma(heads, kv_heads, maps, dim, vdim, page_size))
 
     def masked_attention(self, q, cache, block_table, positions, seq_rows, out, heads, kv_heads, maps, dim, vdim, page_size,
                          mask, mask_size, scale, softcap=0.0, lam=0.0, out_scale=1.0, eps=0.0, gate=None, tiles=None,
@@ -1543,7 +1585,7 @@ class Kernels:
         if tiles is not None:
             self._i32(tiles, "attention tiles")
             n_tiles = tiles.shape[0]
-        need = int(self.lib.axk_masked_attention_workspace(T, heads, kv_heads, maps, dim, vdim, page_size, self.MASKS[mask],
+        need = int(self.run.axk_masked_attention_workspace(T, heads, kv_heads, maps, dim, vdim, page_size, self.MASKS[mask],
                                                            int(mask_size), int(keep), int(span)))
         sinks = sink if isinstance(sink, torch.Tensor) else None
         if sinks is not None:
@@ -1551,21 +1593,21 @@ class Kernels:
             if sinks.numel() != heads:
                 raise KernelError(f"masked_attention: {sinks.numel()} sinks for {heads} heads")
         partial = torch.empty(need, dtype=torch.float32, device=out.device) if need else None
-        self._check(self.lib.axk_masked_attention(
+        self._check(self.run.axk_masked_attention(
             _ptr(q), _ptr(cache), _ptr(block_table), block_table.shape[-1], _ptr(positions), _ptr(seq_rows), _ptr(gate),
             gate_stride, _ptr(out), T, heads, kv_heads, maps, dim, vdim, page_size, self.MASKS[mask], int(mask_size), float(scale),
             float(softcap), float(lam), float(out_scale), float(eps), _ptr(tiles), n_tiles, _ptr(partial), need,
             float("-inf") if sink is None or sinks is not None else float(sink), _ptr(sinks), 1 if gate_per_head else 0, int(keep),
-            int(span), _stream()))
+            int(span), _queue()))
         return out
 
     def fill_i32(self, dst: torch.Tensor, value: int) -> None:
         self._i32(dst, "fill")
-        self._check(self.lib.axk_fill_i32(_ptr(dst), int(value), dst.numel(), _stream()))
+        self._check(self.run.axk_fill_i32(_ptr(dst), int(value), dst.numel(), _queue()))
 
     def fill_f32(self, dst: torch.Tensor, value: float) -> None:
         self._f32(dst, "fill")
-        self._check(self.lib.axk_fill_f32(_ptr(dst), float(value), dst.numel(), _stream()))
+        self._check(self.run.axk_fill_f32(_ptr(dst), float(value), dst.numel(), _queue()))
 
 
 _LOADED: Dict[str, Kernels] = {}
