@@ -259,20 +259,48 @@ extern "C" int axk_swiglu(const void* gate_up, void* out, int n_tokens, int n_ff
 // ---------------------------------------------------------------------------- a norm on a sublayer's output
 // x[r, :] += mult * ((y[r, :] * inv_rms(y[r, :])) * gain), and rounded[r, :] = x[r, :] in the compute
 // dtype if asked for (what the next sublayer's products read).  The sum of squares as in rmsnorm_kernel.
+// A row of few others is bound by how often it waits for memory: all that a thread needs of rows of up to
+// KEPT x 256 values (y, x, gain) is asked for at once, where y was read twice and x and the gain only behind
+// the sum.  With the rounding of the stream for the next block in the same pass, a decoding step of 8 rows of 2,048
+// values, eight of these passes: 538 -> 532 us; a prompt step of 2,048 rows 0.906 -> 0.897 of the same yardstick.
+template <int KEPT>
 __global__ void __launch_bounds__(NORM_THREADS)
 norm_add_kernel(const float* __restrict__ y, const void* __restrict__ gain, int gain_is_f32, float eps, float mult,
                 float* __restrict__ x, elem_t* __restrict__ rounded, int dim) {
   __shared__ float partial[NORM_THREADS / AXON_WAVE];
   const int r = blockIdx.x;
   const float* src = y + (size_t)r * dim;
-  float ss = 0.0f;
-  for (int i = threadIdx.x; i < dim; i += NORM_THREADS) ss = fmaf(src[i], src[i], ss);
-  const float inv = 1.0f / sqrtf(block_sum_256(ss, partial) / (float)dim + eps);
   float* dst = x + (size_t)r * dim;
-  for (int i = threadIdx.x; i < dim; i += NORM_THREADS) {
-    const float v = dst[i] + mult * ((src[i] * inv) * load_vec(gain, gain_is_f32, i));
-    dst[i] = v;
-    if (rounded) rounded[(size_t)r * dim + i] = from_float(v);
+  float ss = 0.0f;
+  if constexpr (KEPT > 0) {
+    float v[KEPT], was[KEPT], g[KEPT];
+#pragma unroll
+    for (int c = 0; c < KEPT; ++c) {
+      const int i = threadIdx.x + c * NORM_THREADS;
+      v[c] = i < dim ? src[i] : 0.0f;
+      was[c] = i < dim ? dst[i] : 0.0f;
+      g[c] = i < dim ? load_vec(gain, gain_is_f32, i) : 0.0f;
+    }
+#pragma unroll
+    for (int c = 0; c < KEPT; ++c) ss = fmaf(v[c], v[c], ss);
+    const float inv = 1.0f / sqrtf(block_sum_256(ss, partial) / (float)dim + eps);
+#pragma unroll
+    for (int c = 0; c < KEPT; ++c) {
+      const int i = threadIdx.x + c * NORM_THREADS;
+      if (i < dim) {
+        const float sum = was[c] + mult * ((v[c] * inv) * g[c]);
+        dst[i] = sum;
+        if (rounded) rounded[(size_t)r * dim + i] = from_float(sum);
+      }
+    }
+  } else {
+    for (int i = threadIdx.x; i < dim; i += NORM_THREADS) ss = fmaf(src[i], src[i], ss);
+    const float inv = 1.0f / sqrtf(block_sum_256(ss, partial) / (float)dim + eps);
+    for (int i = threadIdx.x; i < dim; i += NORM_THREADS) {
+      const float v = dst[i] + mult * ((src[i] * inv) * load_vec(gain, gain_is_f32, i));
+      dst[i] = v;
+      if (rounded) rounded[(size_t)r * dim + i] = from_float(v);
+    }
   }
 }
 
@@ -280,7 +308,9 @@ extern "C" int axk_norm_add(const float* y, const void* gain, int gain_is_f32, f
                             int n_rows, int dim, void* stream) {
   AXK_REQUIRE(n_rows >= 0 && dim > 0, "norm_add: bad sizes rows=%d dim=%d", n_rows, dim);
   if (n_rows == 0) return 0;
-  norm_add_kernel<<<n_rows, NORM_THREADS, 0, (hipStream_t)stream>>>(y, gain, gain_is_f32, eps, mult, x, (elem_t*)rounded, dim);
+  auto kernel = dim <= 4 * NORM_THREADS ? norm_add_kernel<4> : dim <= 8 * NORM_THREADS ? norm_add_kernel<8>
+              : dim <= 16 * NORM_THREADS ? norm_add_kernel<16> : norm_add_kernel<0>;
+  kernel<<<n_rows, NORM_THREADS, 0, (hipStream_t)stream>>>(y, gain, gain_is_f32, eps, mult, x, (elem_t*)rounded, dim);
   AXK_LAUNCH_CHECK("norm_add");
   return 0;
 }

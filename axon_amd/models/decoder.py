@@ -149,6 +149,7 @@ class DecoderModel:
     def forward_runs(self, ctx, x: torch.Tensor, first: int, end: int) -> None:
         """Runs first .. end - 1 of the execution order on the residual stream x, in place."""
         normed = None        # the next block's first norm, where the block before it did its work
+        ctx.shared[ROUNDED_STREAM] = None            # what other runs left of the stream may be older than the stream
         for i in range(first, end):
             run, binding = self.order[i], self.cache_plan.bindings[i]
             block = self.blocks[run.layer]
@@ -163,6 +164,8 @@ class DecoderModel:
                 block.forward(ctx, binding, x)          # a block that knows nothing of this is called plainly
             else:
                 block.forward(ctx, binding, x, normed, following)
+            if not getattr(block, "leaves_rounded_stream", False):
+                ctx.shared[ROUNDED_STREAM] = None
             normed = None if following is None else following.values
 
     def run_is_graph_safe(self, i: int) -> bool:

@@ -105,9 +105,10 @@ class SublayerNormBlock(Block):
     outputs, the sublayers read the residual stream itself (rounded to the compute dtype for their
     products), and a layer may have no feed-forward.  The norm, the scaling and the sum are one
     32-bit pass over the sublayer's 32-bit output, which also leaves the new rows rounded for the
-    next sublayer.  The norms are RMS norms (they hand over a gain and an eps).  `residual_mult`
-    comes with the norm's parameters."""
+    next sublayer, the next block's too.  The norms are RMS norms (they hand over a gain and an eps).
+    `residual_mult` comes with the norm's parameters."""
     graph_safe = True
+    leaves_rounded_stream = True
     norm1_name = "norm1"
     norm2_name = "norm2"
 
@@ -142,16 +143,21 @@ class SublayerNormBlock(Block):
     def forward(self, ctx, binding: CacheBinding, x, normed=None, following=None) -> None:
         k, rt = ctx.rt.k, ctx.rt
         exact = rt.dtype == torch.float32            # the 32-bit path: the sublayers read x as it is
-        h = x if exact else k.round_rows(x, ctx.ws.take(tuple(x.shape), rt.dtype))
+        h = x if exact else self.rounded(ctx, x)
         y = ctx.ws.take(tuple(x.shape), torch.float32)
         self._run(self.mixer, ctx, y, binding, h)
-        if self.feed_forward is None:
-            k.norm_add(y, self.norm1.gain, self.norm1.eps, self.mult, x)
-            return
-        h = x if exact else ctx.ws.take(tuple(x.shape), rt.dtype)
-        k.norm_add(y, self.norm1.gain, self.norm1.eps, self.mult, x, None if exact else h)
-        self._run(self.feed_forward, ctx, y, h)
-        k.norm_add(y, self.norm2.gain, self.norm2.eps, self.mult, x)
+        h = None if exact else ctx.ws.take(tuple(x.shape), rt.dtype)
+        k.norm_add(y, self.norm1.gain, self.norm1.eps, self.mult, x, h)
+        if self.feed_forward is not None:
+            self._run(self.feed_forward, ctx, y, x if exact else h)
+            k.norm_add(y, self.norm2.gain, self.norm2.eps, self.mult, x, h)
+        ctx.shared[ROUNDED_STREAM] = None if exact else (x, h)
+
+    @staticmethod
+    def rounded(ctx, x):
+        """x in the compute dtype: the rows that the block before left where it wrote x, or rounded here."""
+        left = ctx.shared.get(ROUNDED_STREAM)
+        return left[1] if left is not None and left[0] is x else ctx.rt.k.round_rows(x, ctx.ws.take(tuple(x.shape), ctx.rt.dtype))
 
 
 class PostNormBlock(Block):
@@ -185,14 +191,12 @@ class PostNormBlock(Block):
             part.load(store, rt)
 
     _run = staticmethod(SublayerNormBlock._run)
+    rounded = staticmethod(SublayerNormBlock.rounded)
 
     def forward(self, ctx, binding: CacheBinding, x, normed=None, following=None) -> None:
         k, rt = ctx.rt.k, ctx.rt
         exact = rt.dtype == torch.float32            # the 32-bit path: the sublayers read x as it is
-        h = x
-        if not exact:
-            left = ctx.shared.get(ROUNDED_STREAM)    # the block before left the rows it wrote, rounded
-            h = left[1] if left is not None and left[0] is x else k.round_rows(x, ctx.ws.take(tuple(x.shape), rt.dtype))
+        h = x if exact else self.rounded(ctx, x)
         y = ctx.ws.take(tuple(x.shape), torch.float32)
         self._run(self.mixer, ctx, y, binding, h)
         h = None if exact else ctx.ws.take(tuple(x.shape), rt.dtype)
@@ -269,6 +273,7 @@ class SandwichNormBlock(Block):
         return norm.following_values(ctx, n_rows) if hasattr(norm, "following_values") else None
 
     _run = staticmethod(SublayerNormBlock._run)
+    rounded = staticmethod(SublayerNormBlock.rounded)
 
     def forward(self, ctx, binding: CacheBinding, x, normed=None, following=None) -> None:
         h = normed if normed is not None else self.norms[0].forward(ctx, x)
