@@ -2291,32 +2291,60 @@ static int tiles32_of(int n, int mode) { return mode == MODE_SWIGLU ? n / 16 : (
 // `rows_a_pass` rows, one after the other (a row's bits do not depend on the rows beside it).
 #define GEMM_PASS_BYTES ((size_t)2048 << 20)
 
-// Whether the blocks of a product of more than 128 rows walk all of K themselves, in tiles of 128 x 128, and keep the
-// segments' sums in registers; else a block takes a segment and its sums go through the workspace.  Where the lines
-// lie was found with former tiles (32x32x16 products; 32 shapes of 140 to 8,192 rows, 766 measurements, of which the figures
-// below are).  The present ones, of which these gained more than the others, were timed both ways for 21 matrices of the 2,048,
-// 4,096, 7B and 14B widths at 150 to 3,072 rows: of 106 products that keep their sums 102 are the faster for it (down to 0.40 of the
-// time), and of 164 that do not 69 would be too, by up to 1.8 times: the lines are on the safe side.  us, kept / as they run: K 2,048,
-// 2,048 columns of 1,525 rows 23 / 40, of 1,024 22 / 27; 3,584 of K 3,584 of 1,024 rows 34 / 50; gated 4,096 of K 4,096 of 1,024 70 / 101;
-// kept and the slower for it 5,120 of K 13,824 of 1,024 rows 209, with large tiles 180.
-//  * There have to be blocks for the chip's 256 CUs.  K 2,048, 2,560 columns of 1,525 rows (240 blocks) 35 against 38 us,
-//    2,048 of 1,525 (192) 35 against 33; K 3,584, 3,584 of 1,200 (280) 63 against 71, 900 (224) 52 against 49.  Gated,
-//    1,408 of 700 (132) 27 against 28, of 900 (176) 27 against 30; 1,024 of 900 (128) 27 against 22.
+// The tiles of a product of more than 128 rows.  KEPT: 128 x 128, two blocks a CU, a block walks all of K and keeps the
+// segments' sums in registers.  The others take a segment a block and its sums go through the workspace (the same bits).
+//
+// Where the lines of the kept ones lie was found with former tiles (32x32x16 products; 32 shapes of 140 to 8,192 rows, 766
+// measurements) and moved with the present ones (28 matrices of the widths 1,024 to 5,120, K up to 27,648, 17 row counts of 150 to
+// 4,096, the sums' kernel included; us, kept / a segment a block).
+//  * There have to be blocks for the chip's 256 CUs.  Four segments of a long K: for all but eight.  4,608 columns of K 3,584 of
+//    777 rows (252 blocks) 35 / 51, 4,096 of K 4,096 of 1,024 (256) 51 / 59, 2,048 of K 5,632 of 2,048 (256) 63 / 70 (6,144 of K
+//    4,096 of 600, 240 blocks, 37 / 54: on the safe side).  Of a short K, former tiles: K 2,048, 2,560 columns of 1,525 rows (240 blocks) 35 against 38, 2,048 of 1,525 (192) 35 against 33 (with
+//    the present ones 32 / 40: the line is on the safe side).  Gated, former: 1,408 of 700 (132) 27 against 28, of 900 (176) 27 against 30.
 //  * K has to be short enough for tiles that read twice what the large ones read.  With up to 4,096 they win whatever
 //    the last round of 512 blocks (two a CU) holds: K 3,584, 4,608 of 2,048 rows 109 against 123; 4,096, 4,096 of
 //    4,096 154 against 206.  Up to 8,192 they win where it is one round or nearly full ones: K 5,120, 5,120 of
 //    3,072 (960 blocks) 188 against 221, of 2,048 behind a norm (640) 186 against 177; 8,192, 3,584 of 4,096 280 against
 //    302.  K 18,944, 3,584 of 2,048 328 against 314.
 //  * A gated product of up to 256 rows and a long K has the kernel with four stages: K 3,072, 8,192 of 256 rows 47
-//    against 43 us; of K 1,536, 8,960 35 against 43.
+//    against 43 us; of K 1,536, 8,960 35 against 43.  With more rows and four segments the kept ones save eight sets of sums:
+//    4,096 of K 4,096 of 300 rows 34 / 39, of 1,024 67 / 101, of 4,096 235 / 472; they cost 0.4 us more a step of 64 k and round of
+//    256 large tiles, the sums of such a round some 87, so 8,192 is well inside.
 static bool keeps_segments(int m, int n, int k, int mode, int segs) {
   if (segs <= 1 || m <= 128) return false;
   const bool glu = mode == MODE_SWIGLU;
   const long blocks = (long)ceil_div(m, 128) * ceil_div(n, glu ? 64 : 128), rounds = (blocks + 511) / 512;
-  if (glu) return blocks >= 144 && k <= (m <= 256 ? 2048 : 3072);
-  if (blocks < (segs == 4 && k <= 2048 ? 240 : 288)) return false;
+  if (glu) return blocks >= 144 && k <= (m <= 256 ? 2048 : segs == 4 ? 8192 : 3072);
+  if (blocks < (segs < 4 ? 288 : k <= 2048 ? 240 : 248)) return false;
   if (segs < 4) return k <= 3072;
   return k <= 4096 || (k <= 8192 && (rounds == 1 || 4 * blocks >= 3 * 512 * rounds));
+}
+
+// The tiles of a segment a block: 128 x 128, two blocks a CU, or DEEP, the same with four stages instead of two and a block
+// a CU, or LARGE, 256 x 256, a block a CU, half the traffic from L2 per product.
+//  * DEEP: up to 256 rows still wait for W more than for the matrix cores.  Where the small tiles are no more blocks than CUs, a
+//    block has its CU's LDS to itself and three steps of loads in flight (the down projection of a 7B layer at 256 rows 79 ->
+//    64 us); with more blocks two of them share a CU and cover each other's waits (four stages there: slower).
+//  * else what takes less by an estimate: the steps of 64 k of the fullest CU (two small blocks side by side take 1.05 us a
+//    step, one alone 0.73, a large one 1.2), a start a round of the large, M x N numbers out and the segments' sums out and in.  The
+//    constants (us) are fitted to the 950 measurements of both.  A count of rounds, one of the small as 0.65 of the large, as it was
+//    before, took three rounds of the small for two of the large: 18,944 gated columns of K 3,584 of 512 rows 192, here 158;
+//    27,648 of K 5,120 of 777 536, 435; 5,120 of K 13,824 of 1,024 214, 184; 32,000 of K 2,048 of 600 128, 101.  Of 465 products 76 take
+//    less by over 3 % by this and the lines above, two more by 3 and 6 %.
+enum TileKind { TILES_SMALL, TILES_DEEP, TILES_LARGE };
+
+static TileKind split_tiles(int m, int n, int k, int mode, int segs) {
+  const bool glu = mode == MODE_SWIGLU;
+  const long small = (long)ceil_div(m, 128) * ceil_div(n, glu ? 64 : 128) * segs;
+  const long large = (long)ceil_div(m, 256) * ceil_div(n, glu ? 128 : 256) * segs;
+  const long fullest = (small + 255) / 256, rounds = (large + 255) / 256;
+  const float steps = (float)k / 64.0f / (float)segs, out = (float)m * (float)n * 1e-6f;
+  const float sums = segs > 1 ? (glu ? 2.0f : 1.0f) * (float)segs * out : 0.0f;
+  const bool deep = m <= 256 && small <= 256;
+  const float with_small = deep ? 6.2f + steps * 0.53f + 1.4f * out + 1.1f * sums
+                                : 6.2f + steps * (1.05f * (float)(fullest / 2) + 0.73f * (float)(fullest % 2)) + 1.4f * out + 1.1f * sums;
+  const float with_large = 3.7f + (float)rounds * (steps * 1.2f + 3.6f) + 1.15f * out + 1.3f * sums;
+  return with_large < with_small ? TILES_LARGE : deep ? TILES_DEEP : TILES_SMALL;
 }
 
 // How many sets of M x N sums go through the workspace: one a segment (twice for the gated product), none where
@@ -2433,35 +2461,21 @@ static int gemm_mfma_pass(const bf16_t* x, int x_stride, const bf16_t* w, const 
     if (n >= 32 * 512) return launch_rows<2, 8, EPI_PLAIN>(ARGS, segs, ws, norm, rope_after);
     return launch_rows<1, 8, EPI_PLAIN>(ARGS, segs, ws, norm, rope_after);
   }
-  // 256 x 256 tiles (8 waves, a block a CU) or 128 x 128 tiles (4 waves, two blocks a CU, four
-  // times as many blocks at twice the traffic from L2 per product): whichever takes the chip's 256
-  // CUs fewer rounds, a round of the small tiles counted as 0.65 of a round of the large ones: found with tiles that both have
-  // 32x32x16 products.  With the present large ones a round of the small is 0.5 to 0.9 of theirs, and of 209 products of 21 matrices at
-  // 150 to 3,072 rows that do not keep their segments' sums 21 take the slower tile by more than 3 %, most of them three rounds of the
-  // small for two of the large: us, small / large, [gate; up] of a 7B layer of 600 rows 196 / 161, of a 14B layer of 777 265 / 215, 32,000
-  // columns of K 2,048 of 600 124 / 101.
-  const long big = (long)ceil_div(m, 256) * ceil_div(n, glu ? 128 : 256) * segs;
-  const long small = (long)ceil_div(m, 128) * ceil_div(n, glu ? 64 : 128) * segs;
-  const long rounds_big = (big + 255) / 256, rounds_small = (small + 511) / 512;
-  const bool use_big = rounds_big * 100 <= rounds_small * 65;
   if (keep) {
     if (glu) return launch_tile<128, 128, 2, 2, true, true>(ARGS, segs, ws);
     return launch_tile<128, 128, 2, 2, false, true>(ARGS, segs, ws, norm, rope_after);
   }
-  if (!use_big) {
-    // Up to 256 rows still wait for W more than for the matrix cores.  Where the small tiles are no
-    // more blocks than CUs, a block has its CU's LDS to itself: four stages instead of two, three
-    // steps of loads in flight (the down projection of a 7B layer at 256 rows 79 -> 64 us); with
-    // more blocks two of them share a CU and cover each other's waits (four stages there: slower).
-    const bool deep = m <= 256 && small <= 256;
-    if (glu) {
-      if (deep) return launch_small_tile<true, 4>(ARGS, segs, ws);
-      return launch_small_tile<true, 2>(ARGS, segs, ws);
-    }
-    if (deep) return launch_small_tile<false, 4>(ARGS, segs, ws, norm, rope_after);
+  const TileKind kind = split_tiles(m, n, k, mode, segs);
+  if (kind == TILES_DEEP) {
+    if (glu) return launch_small_tile<true, 4>(ARGS, segs, ws);
+    return launch_small_tile<false, 4>(ARGS, segs, ws, norm, rope_after);
+  }
+  if (kind == TILES_SMALL) {
+    if (glu) return launch_small_tile<true, 2>(ARGS, segs, ws);
     return launch_small_tile<false, 2>(ARGS, segs, ws, norm, rope_after);
   }
   if (glu) return launch_tile<256, 256, 4, 2, true>(ARGS, segs, ws);
+  const long big = (long)ceil_div(m, 256) * ceil_div(n, 256) * segs;
   // one round of 256 x 256 tiles that leaves a quarter of the CUs idle, and N in whole tiles of
   // 192 columns that still fit one round: the narrower tile (measured 1.1 times the cost per
   // product, three quarters of the products per block).
