@@ -82,6 +82,24 @@ __device__ inline float4 load_vec4(const void* p, int is_f32, int i) {
   return make_float4(a.f, b.f, c.f, d.f);
 }
 
+// GROUPS groups of COUNT neighbouring numbers of such a vector, `stride` apart from number `first` on; for those from `end` on the last
+// one again.  All are asked for before the first is widened: where load_vec's choice of type stands between two loads, each is
+// waited for.
+template <int GROUPS, int COUNT>
+__device__ inline void load_vec_apart(const void* p, int is_f32, int first, int stride, int end, float (&out)[GROUPS][COUNT]) {
+  if (is_f32) {
+#pragma unroll
+    for (int c = 0; c < GROUPS * COUNT; ++c)
+      out[c / COUNT][c % COUNT] = ((const float*)p)[min(first + c / COUNT * stride + c % COUNT, end - 1)];
+  } else {
+    bf16_t raw[GROUPS * COUNT];
+#pragma unroll
+    for (int c = 0; c < GROUPS * COUNT; ++c) raw[c] = ((const bf16_t*)p)[min(first + c / COUNT * stride + c % COUNT, end - 1)];
+#pragma unroll
+    for (int c = 0; c < GROUPS * COUNT; ++c) out[c / COUNT][c % COUNT] = bf16_to_float(raw[c]);
+  }
+}
+
 // Four consecutive elements as floats: one 8- or 16-byte load where `vec` says the address is
 // aligned for it and all four exist, else the `valid` first ones singly and zeros behind them.
 __device__ inline void load4_guarded(const elem_t* __restrict__ p, int valid, bool vec, float out[4]) {

@@ -844,10 +844,27 @@ gemm_split_reduce_any_kernel(const float* __restrict__ partial, int splits, int 
   else reinterpret_cast<float*>(out)[at] = v;
 }
 
+// The sums of a product's segments in their order: SPLITS sets (gemm_segments: 1, 2 or 4), `step` numbers apart, all asked for
+// together.  (A loop over a number of sets that is not known when compiled waits for each before it asks for the next: a row of
+// four sets took four trips to memory.  us, so / here: 64 rows of 4,608 with the rotary store 6.7 / 6.1; of 1,525 rows, bound by bytes,
+// 5,120 with the norm 29.8 / 29.2, 7,168 with the rotary store 48.4 / 43.3.)
+template <int SPLITS>
+__device__ inline float4 summed_segments(const float* __restrict__ src, size_t step) {
+  float4 a[SPLITS];
+#pragma unroll
+  for (int z = 0; z < SPLITS; ++z) a[z] = *reinterpret_cast<const float4*>(src + (size_t)z * step);
+#pragma unroll
+  for (int z = 1; z < SPLITS; ++z) {
+    a[0].x += a[z].x; a[0].y += a[z].y; a[0].z += a[z].z; a[0].w += a[z].w;
+  }
+  return a[0];
+}
+
 // The sums of the split-K blocks, added in block order, then the epilogue of the product.
 // One thread per 4 consecutive columns of a row (N a multiple of 4).
+template <int SPLITS>
 __global__ void __launch_bounds__(256)
-gemm_split_reduce_kernel(const float* __restrict__ partial, int splits, int M, int N, const void* __restrict__ bias,
+gemm_split_reduce_kernel(const float* __restrict__ partial, int M, int N, const void* __restrict__ bias,
                          int bias_is_f32, void* __restrict__ out, int out_stride, int mode) {
   const int idx = blockIdx.x * 256 + threadIdx.x;
   const int n4 = N / 4;
@@ -855,28 +872,8 @@ gemm_split_reduce_kernel(const float* __restrict__ partial, int splits, int M, i
   const int m = idx / n4, n = (idx % n4) * 4;
   const size_t plane = (size_t)M * N, at_in = (size_t)m * N + n;
   const int parts = mode == MODE_SWIGLU ? 2 : 1;
-  // the blocks' sums in block order; four loads under way at a time
-  auto summed = [&](const float* src, size_t step) {
-    float4 g = *reinterpret_cast<const float4*>(src);
-    int z = 1;
-    for (; z + 3 < splits; z += 4) {
-      const float4 a0 = *reinterpret_cast<const float4*>(src + (size_t)z * step);
-      const float4 a1 = *reinterpret_cast<const float4*>(src + (size_t)(z + 1) * step);
-      const float4 a2 = *reinterpret_cast<const float4*>(src + (size_t)(z + 2) * step);
-      const float4 a3 = *reinterpret_cast<const float4*>(src + (size_t)(z + 3) * step);
-      g.x += a0.x; g.y += a0.y; g.z += a0.z; g.w += a0.w;
-      g.x += a1.x; g.y += a1.y; g.z += a1.z; g.w += a1.w;
-      g.x += a2.x; g.y += a2.y; g.z += a2.z; g.w += a2.w;
-      g.x += a3.x; g.y += a3.y; g.z += a3.z; g.w += a3.w;
-    }
-    for (; z < splits; ++z) {
-      const float4 a = *reinterpret_cast<const float4*>(src + (size_t)z * step);
-      g.x += a.x; g.y += a.y; g.z += a.z; g.w += a.w;
-    }
-    return g;
-  };
-  const float4 g = summed(partial + at_in, (size_t)parts * plane);
-  const float4 u = parts == 2 ? summed(partial + plane + at_in, (size_t)parts * plane) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  const float4 g = summed_segments<SPLITS>(partial + at_in, (size_t)parts * plane);
+  const float4 u = parts == 2 ? summed_segments<SPLITS>(partial + plane + at_in, (size_t)parts * plane) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   float v[4] = {g.x, g.y, g.z, g.w};
   const size_t at = (size_t)m * out_stride + n;
   if (mode == MODE_SWIGLU) {
@@ -912,51 +909,38 @@ struct SplitNorm {
 #define SRN_THREADS 1024
 #define SRN_MAX_N 8192
 
+template <int SPLITS>
 __global__ void __launch_bounds__(SRN_THREADS)
-gemm_split_reduce_norm_kernel(const float* __restrict__ partial, int splits, int M, int N, const void* __restrict__ bias,
+gemm_split_reduce_norm_kernel(const float* __restrict__ partial, int M, int N, const void* __restrict__ bias,
                               int bias_is_f32, float* __restrict__ out, int out_stride, SplitNorm norm) {
   __shared__ float4 row[SRN_MAX_N / 4];
   __shared__ float sums[4];
   const int m = blockIdx.x, n4 = N / 4, tid = threadIdx.x;
   const size_t plane = (size_t)M * N;
-  auto added = [&](int i) {
+  auto added = [&](int i, float (&gain)[1][4]) {
     const int n = i * 4;
-    const float* src = partial + (size_t)m * N + n;
-    float4 g = *reinterpret_cast<const float4*>(src);
-    int z = 1;
-    for (; z + 3 < splits; z += 4) {           // four loads under way at a time; added in block order
-      const float4 a0 = *reinterpret_cast<const float4*>(src + (size_t)z * plane);
-      const float4 a1 = *reinterpret_cast<const float4*>(src + (size_t)(z + 1) * plane);
-      const float4 a2 = *reinterpret_cast<const float4*>(src + (size_t)(z + 2) * plane);
-      const float4 a3 = *reinterpret_cast<const float4*>(src + (size_t)(z + 3) * plane);
-      g.x += a0.x; g.y += a0.y; g.z += a0.z; g.w += a0.w;
-      g.x += a1.x; g.y += a1.y; g.z += a1.z; g.w += a1.w;
-      g.x += a2.x; g.y += a2.y; g.z += a2.z; g.w += a2.w;
-      g.x += a3.x; g.y += a3.y; g.z += a3.z; g.w += a3.w;
-    }
-    for (; z < splits; ++z) {
-      const float4 a = *reinterpret_cast<const float4*>(src + (size_t)z * plane);
-      g.x += a.x; g.y += a.y; g.z += a.z; g.w += a.w;
-    }
+    float4* dst = reinterpret_cast<float4*>(out + (size_t)m * out_stride + n);
+    float4 r = *dst;
+    load_vec_apart<1, 4>(norm.gain, norm.gain_is_f32, n, 0, N, gain);
+    float4 g = summed_segments<SPLITS>(partial + (size_t)m * N + n, plane);
     if (bias) {
       g.x += load_vec(bias, bias_is_f32, n);
       g.y += load_vec(bias, bias_is_f32, n + 1);
       g.z += load_vec(bias, bias_is_f32, n + 2);
       g.w += load_vec(bias, bias_is_f32, n + 3);
     }
-    float4* dst = reinterpret_cast<float4*>(out + (size_t)m * out_stride + n);
-    float4 r = *dst;
     r.x += g.x; r.y += g.y; r.z += g.z; r.w += g.w;
     *dst = r;
     return r;
   };
   constexpr int MINE = SRN_MAX_N / 4 / SRN_THREADS;
   float4 mine[MINE];
+  float gain[MINE][1][4];              // asked for beside the sums, not behind the norm's
 #pragma unroll
   for (int c = 0; c < MINE; ++c) {
     const int i = tid + c * SRN_THREADS;
     if (i < n4) {
-      mine[c] = added(i);
+      mine[c] = added(i, gain[c]);
       row[i] = mine[c];
     }
   }
@@ -984,10 +968,8 @@ gemm_split_reduce_norm_kernel(const float* __restrict__ partial, int splits, int
       const int e = i * 4;
       const float4 v = mine[c];
       uint2 pk;
-      pk.x = pack2_bf16((v.x * inv) * load_vec(norm.gain, norm.gain_is_f32, e),
-                        (v.y * inv) * load_vec(norm.gain, norm.gain_is_f32, e + 1));
-      pk.y = pack2_bf16((v.z * inv) * load_vec(norm.gain, norm.gain_is_f32, e + 2),
-                        (v.w * inv) * load_vec(norm.gain, norm.gain_is_f32, e + 3));
+      pk.x = pack2_bf16((v.x * inv) * gain[c][0][0], (v.y * inv) * gain[c][0][1]);
+      pk.y = pack2_bf16((v.z * inv) * gain[c][0][2], (v.w * inv) * gain[c][0][3]);
       *reinterpret_cast<uint2*>(dst + e) = pk;
     }
   }
@@ -1001,14 +983,18 @@ static int launch_split_reduce_rope(const float* partial, int splits, int m, int
 // order, then the epilogue (with the rotary store, or the norm of the new rows, where asked).
 static int add_split_sums(const float* partial, int splits, int m, int n, const void* bias, int bias_is_f32, void* out,
                           int out_stride, int mode, const SplitNorm* norm, const RopeStore* rope, hipStream_t stream) {
+  if (splits != 1 && splits != 2 && splits != 4) {
+    axk_set_error("gemm: the sums of %d segments (1, 2 or 4)", splits);
+    return -1;
+  }
   if (rope != nullptr) {
     AXK_INSTANCE(INST_GEMM_SPLIT_REDUCE, 2);
     return launch_split_reduce_rope(partial, splits, m, n, bias, bias_is_f32, out, out_stride, *rope, stream);
   }
   if (norm != nullptr) {
     AXK_INSTANCE(INST_GEMM_SPLIT_REDUCE, 1);
-    gemm_split_reduce_norm_kernel<<<m, SRN_THREADS, 0, stream>>>(partial, splits, m, n, bias, bias_is_f32, (float*)out,
-                                                                 out_stride, *norm);
+    auto kernel = splits == 1 ? gemm_split_reduce_norm_kernel<1> : splits == 2 ? gemm_split_reduce_norm_kernel<2> : gemm_split_reduce_norm_kernel<4>;
+    kernel<<<m, SRN_THREADS, 0, stream>>>(partial, m, n, bias, bias_is_f32, (float*)out, out_stride, *norm);
     AXK_LAUNCH_CHECK("gemm_split_reduce_norm");
     return 0;
   }
@@ -1020,8 +1006,8 @@ static int add_split_sums(const float* partial, int splits, int m, int n, const 
     return 0;
   }
   AXK_INSTANCE(INST_GEMM_SPLIT_REDUCE, 0);
-  gemm_split_reduce_kernel<<<ceil_div(m * (n / 4), 256), 256, 0, stream>>>(partial, splits, m, n, bias, bias_is_f32, out,
-                                                                          out_stride, mode);
+  auto kernel = splits == 1 ? gemm_split_reduce_kernel<1> : splits == 2 ? gemm_split_reduce_kernel<2> : gemm_split_reduce_kernel<4>;
+  kernel<<<ceil_div(m * (n / 4), 256), 256, 0, stream>>>(partial, m, n, bias, bias_is_f32, out, out_stride, mode);
   AXK_LAUNCH_CHECK("gemm_split_reduce");
   return 0;
 }
@@ -1153,9 +1139,9 @@ enum { EPI_PLAIN = 0, EPI_GLU = 1, EPI_ROPE = 2 };
 // eights counted from the step's first token, which only an aligned request fits / here: 28 and 2 x 4 heads, 2,048 tokens
 // 17.8 / 13.2 / 13.4, requests of 5 and 4,091 30.3 / 37.7 / 22.4; 40 and 2 x 8 heads, 2,048 tokens 31 / 18 / 18, 6,000 116 / 68 / 56,
 // 5 and 4,091 65 / 78 / 39, 110 of 37 68 / 74 / 46; four requests of 1,525 tokens in all, four sums each, 39.2 / 38.1 / 40.6.
-template <int TOKENS>
+template <int TOKENS, int SPLITS>
 __global__ void __launch_bounds__(256)
-gemm_split_reduce_rope_kernel(const float* __restrict__ partial, int splits, int M, int N, const void* __restrict__ bias,
+gemm_split_reduce_rope_kernel(const float* __restrict__ partial, int M, int N, const void* __restrict__ bias,
                               int bias_is_f32, bf16_t* __restrict__ out, int out_stride, RopeStore rope) {
   const int hd = rope.head_dim, half = hd / 2, per_head = half / 4;     // threads a head
   const int heads_a_block = 256 / per_head;
@@ -1188,18 +1174,26 @@ gemm_split_reduce_rope_kernel(const float* __restrict__ partial, int splits, int
   float a[TOKENS][4], b[TOKENS][4];
   auto sums = [&](int first, int count) {
     f32x4 lo[TOKENS], hi[TOKENS];
-#pragma unroll
-    for (int t = 0; t < TOKENS; ++t) {
-      const float* src = partial + (size_t)(first + min(t, count - 1)) * N + col;
-      lo[t] = *reinterpret_cast<const f32x4*>(src);
-      hi[t] = *reinterpret_cast<const f32x4*>(src + half);
-    }
-    for (int z = 1; z < splits; ++z) {
+    if constexpr (TOKENS == 1) {
+      const float* src = partial + (size_t)first * N + col;
+      const float4 l = summed_segments<SPLITS>(src, plane), h = summed_segments<SPLITS>(src + half, plane);
+      lo[0] = f32x4{l.x, l.y, l.z, l.w};
+      hi[0] = f32x4{h.x, h.y, h.z, h.w};
+    } else {
 #pragma unroll
       for (int t = 0; t < TOKENS; ++t) {
-        const float* src = partial + (size_t)z * plane + (size_t)(first + min(t, count - 1)) * N + col;
-        lo[t] += *reinterpret_cast<const f32x4*>(src);
-        hi[t] += *reinterpret_cast<const f32x4*>(src + half);
+        const float* src = partial + (size_t)(first + min(t, count - 1)) * N + col;
+        lo[t] = *reinterpret_cast<const f32x4*>(src);
+        hi[t] = *reinterpret_cast<const f32x4*>(src + half);
+      }
+#pragma unroll
+      for (int z = 1; z < SPLITS; ++z) {
+#pragma unroll
+        for (int t = 0; t < TOKENS; ++t) {
+          const float* src = partial + (size_t)z * plane + (size_t)(first + min(t, count - 1)) * N + col;
+          lo[t] += *reinterpret_cast<const f32x4*>(src);
+          hi[t] += *reinterpret_cast<const f32x4*>(src + half);
+        }
       }
     }
 #pragma unroll
@@ -1221,8 +1215,8 @@ gemm_split_reduce_rope_kernel(const float* __restrict__ partial, int splits, int
 #pragma unroll
       for (int t = 0; t < TOKENS; ++t) {
         if (t < from || t >= to) continue;
-        const int pos = TOKENS == 1 ? rope.positions[m0] : __builtin_amdgcn_readlane(pos_at, first + t);
-        const int page = TOKENS == 1 ? page_of(m0, pos) : __builtin_amdgcn_readlane(page_at, first + t);
+        const int pos = TOKENS == 1 ? pos_at : __builtin_amdgcn_readlane(pos_at, first + t);
+        const int page = TOKENS == 1 ? page_at : __builtin_amdgcn_readlane(page_at, first + t);
         bf16_t* vdst = rope.v_cache + (size_t)page * page_elems + head_at + pos % rope.page_size;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -1232,6 +1226,8 @@ gemm_split_reduce_rope_kernel(const float* __restrict__ partial, int splits, int
       }
     };
     if (TOKENS == 1) {
+      pos_at = rope.positions[m0];       // and the page beside the sums, not behind them
+      page_at = page_of(m0, pos_at);
       sums(m0, 1);
       put(0, 0, 1);
       return;
@@ -1279,6 +1275,12 @@ gemm_split_reduce_rope_kernel(const float* __restrict__ partial, int splits, int
       page[t] = page_of(min(m0 + t, M - 1), pos[t]);
     }
   }
+  float4 turn[TOKENS == 1 ? 2 : 1];      // of one token: asked for beside the sums
+  if (TOKENS == 1) {
+    const float4* tab = reinterpret_cast<const float4*>(rope.table + ((size_t)m0 * half + d) * 2);
+    turn[0] = tab[0];
+    turn[TOKENS == 1 ? 1 : 0] = tab[1];
+  }
   sums(m0, min(TOKENS, M - m0));
 #pragma unroll
   for (int t = 0; t < TOKENS; ++t) {
@@ -1289,7 +1291,7 @@ gemm_split_reduce_rope_kernel(const float* __restrict__ partial, int splits, int
                         : rope.k_cache + (((size_t)page[t] * rope.n_kv_heads + (slot - rope.n_heads)) * rope.page_size +
                                           pos[t] % rope.page_size) * hd;
       const float4* tab = reinterpret_cast<const float4*>(rope.table + ((size_t)m * half + d) * 2);
-      const float4 t0 = tab[0], t1 = tab[1];
+      const float4 t0 = TOKENS == 1 ? turn[0] : tab[0], t1 = TOKENS == 1 ? turn[TOKENS == 1 ? 1 : 0] : tab[1];
       const float sn[4] = {t0.x, t0.z, t1.x, t1.z}, cs[4] = {t0.y, t0.w, t1.y, t1.w};
       float lo[4], hi[4];
 #pragma unroll
@@ -1312,11 +1314,13 @@ static int launch_split_reduce_rope(const float* partial, int splits, int m, int
   // 1,024 (256) 34 / 46, at 2,048 (512) 48 / 50, 28 and 2 x 4 at 4,096 (1,536) 190 / 185.
   if ((long)ceil_div(m, 8) * head_blocks >= 640) {
     AXK_INSTANCE(INST_GEMM_SPLIT_REDUCE, 2, 8);
-    gemm_split_reduce_rope_kernel<8><<<dim3(ceil_div(m, 8), head_blocks), 256, 0, stream>>>(partial, splits, m, n, bias, bias_is_f32,
-                                                                                            (bf16_t*)out, out_stride, rope);
+    auto kernel = splits == 1 ? gemm_split_reduce_rope_kernel<8, 1> : splits == 2 ? gemm_split_reduce_rope_kernel<8, 2>
+                                                                                 : gemm_split_reduce_rope_kernel<8, 4>;
+    kernel<<<dim3(ceil_div(m, 8), head_blocks), 256, 0, stream>>>(partial, m, n, bias, bias_is_f32, (bf16_t*)out, out_stride, rope);
   } else {
-    gemm_split_reduce_rope_kernel<1><<<dim3(m, head_blocks), 256, 0, stream>>>(partial, splits, m, n, bias, bias_is_f32, (bf16_t*)out,
-                                                                               out_stride, rope);
+    auto kernel = splits == 1 ? gemm_split_reduce_rope_kernel<1, 1> : splits == 2 ? gemm_split_reduce_rope_kernel<1, 2>
+                                                                                 : gemm_split_reduce_rope_kernel<1, 4>;
+    kernel<<<dim3(m, head_blocks), 256, 0, stream>>>(partial, m, n, bias, bias_is_f32, (bf16_t*)out, out_stride, rope);
   }
   AXK_LAUNCH_CHECK("gemm_split_reduce_rope");
   return 0;
@@ -2329,7 +2333,7 @@ static bool keeps_segments(int m, int n, int k, int mode, int segs) {
 //    step, one alone 0.73, a large one 1.2), a start a round of the large, M x N numbers out and the segments' sums out and in.  The
 //    constants (us) are fitted to the 950 measurements of both.  A count of rounds, one of the small as 0.65 of the large, as it was
 //    before, took three rounds of the small for two of the large: 18,944 gated columns of K 3,584 of 512 rows 192, here 158;
-//    27,648 of K 5,120 of 777 536, 435; 5,120 of K 13,824 of 1,024 214, 184; 32,000 of K 2,048 of 600 128, 101.  Of 465 products 76 take
+//    27,648 of K 5,120 of 777 536, 435; 5,120 of K 13,824 of 1,024 214, 184; 32,000 of K 2,048 of 600 128, 101.  Of 476 products 76 take
 //    less by over 3 % by this and the lines above, two more by 3 and 6 %.
 enum TileKind { TILES_SMALL, TILES_DEEP, TILES_LARGE };
 
