@@ -10,19 +10,28 @@
 // (src/model.rs:2657-2675).
 // A tied head's matrix is kept packed for the products (see axk_pack_matrix): element (row, i) is
 // then at ((row / 16 * dim / 32 + i / 32) * 64 + row % 16 + 16 (i % 32 / 8)) * 8 + i % 8.
+// VEC: eight neighbouring numbers a thread, which either layout has side by side (widths that are a multiple of 8, 16-byte
+// aligned tables and rows): a row's numbers one at a time were fourteen loads a thread behind one another at 3,584 of them.
+// us, so / here: 64 tokens of 3,584 9.0 / 3.4, 8 of 2,048 6.5 / 3.4, 2,126 of 2,048 19.0 / 16.7, 1,525 of 5,120 20.9 / 14.7.
+template <bool VEC>
 __global__ void embed_kernel(const int32_t* __restrict__ tokens, const elem_t* __restrict__ table, int packed,
                              float* __restrict__ x, int dim, float scale) {
   const int t = blockIdx.x;
   const int token = tokens[t];
   float* dst = x + (size_t)t * dim;
-  if (packed) {
-    const elem_t* tile = table + (size_t)(token / 16) * (dim / 32) * 512 + (token % 16) * 8;
-    for (int i = threadIdx.x; i < dim; i += blockDim.x)
-      dst[i] = to_float(tile[(size_t)(i / 32) * 512 + ((i % 32) / 8) * 128 + i % 8]) * scale;
-    return;
+  const elem_t* row = packed ? table + (size_t)(token / 16) * (dim / 32) * 512 + (token % 16) * 8 : table + (size_t)token * dim;
+  auto place = [&](int i) { return packed ? (size_t)(i / 32) * 512 + ((i % 32) / 8) * 128 + i % 8 : (size_t)i; };
+  if constexpr (VEC) {
+    for (int i = 8 * (blockIdx.y * blockDim.x + threadIdx.x); i < dim; i += 8 * gridDim.y * blockDim.x) {
+      float v[8];
+      load4_guarded(row + place(i), 4, true, v);
+      load4_guarded(row + place(i) + 4, 4, true, v + 4);
+      *reinterpret_cast<float4*>(dst + i) = make_float4(v[0] * scale, v[1] * scale, v[2] * scale, v[3] * scale);
+      *reinterpret_cast<float4*>(dst + i + 4) = make_float4(v[4] * scale, v[5] * scale, v[6] * scale, v[7] * scale);
+    }
+  } else {
+    for (int i = threadIdx.x; i < dim; i += blockDim.x) dst[i] = to_float(row[place(i)]) * scale;
   }
-  const elem_t* row = table + (size_t)token * dim;
-  for (int i = threadIdx.x; i < dim; i += blockDim.x) dst[i] = to_float(row[i]) * scale;
 }
 
 extern "C" int axk_embed_scaled(const int32_t* tokens, const void* table, int packed, float* x, int n_tokens, int dim,
@@ -30,7 +39,10 @@ extern "C" int axk_embed_scaled(const int32_t* tokens, const void* table, int pa
   AXK_REQUIRE(n_tokens >= 0 && dim > 0 && vocab > 0, "embed: bad sizes T=%d dim=%d vocab=%d", n_tokens, dim, vocab);
   AXK_REQUIRE(!packed || dim % 32 == 0, "embed: a packed table has rows of whole blocks of 32, not %d", dim);
   if (n_tokens == 0) return 0;
-  embed_kernel<<<n_tokens, 256, 0, (hipStream_t)stream>>>(tokens, (const elem_t*)table, packed, x, dim, scale);
+  if (dim % 8 == 0 && (((uintptr_t)table | (uintptr_t)x) & 15) == 0)
+    embed_kernel<true><<<dim3(n_tokens, ceil_div(dim, 8 * 256)), 256, 0, (hipStream_t)stream>>>(tokens, (const elem_t*)table, packed, x, dim, scale);
+  else
+    embed_kernel<false><<<n_tokens, 256, 0, (hipStream_t)stream>>>(tokens, (const elem_t*)table, packed, x, dim, scale);
   AXK_LAUNCH_CHECK("embed");
   return 0;
 }
@@ -70,11 +82,16 @@ rmsnorm_vec_kernel(const float* __restrict__ x, const int32_t* __restrict__ rows
   const int r = blockIdx.x, n4 = dim >> 2;
   const float4* src = reinterpret_cast<const float4*>(x + (size_t)(rows ? rows[r] : r) * dim);
   float4 kept[NORM_CACHED];
-  float ss = 0.0f;
+  float g[NORM_CACHED][4];                           // the gain is asked for beside the row, not behind its sum
 #pragma unroll
   for (int c = 0; c < NORM_CACHED; ++c) {
     const int i = threadIdx.x + c * NORM_THREADS;
     kept[c] = i < n4 ? src[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  }
+  load_vec_apart<NORM_CACHED, 4>(gain, gain_is_f32, 4 * threadIdx.x, 4 * NORM_THREADS, dim, g);
+  float ss = 0.0f;
+#pragma unroll
+  for (int c = 0; c < NORM_CACHED; ++c) {
     ss = fmaf(kept[c].x, kept[c].x, ss);
     ss = fmaf(kept[c].y, kept[c].y, ss);
     ss = fmaf(kept[c].z, kept[c].z, ss);
@@ -95,8 +112,7 @@ rmsnorm_vec_kernel(const float* __restrict__ x, const int32_t* __restrict__ rows
     const int i = threadIdx.x + c * NORM_THREADS;
     if (i < n4) {
       const int e = i * 4;
-      store4(dst + e, (kept[c].x * inv) * load_vec(gain, gain_is_f32, e), (kept[c].y * inv) * load_vec(gain, gain_is_f32, e + 1),
-             (kept[c].z * inv) * load_vec(gain, gain_is_f32, e + 2), (kept[c].w * inv) * load_vec(gain, gain_is_f32, e + 3));
+      store4(dst + e, (kept[c].x * inv) * g[c][0], (kept[c].y * inv) * g[c][1], (kept[c].z * inv) * g[c][2], (kept[c].w * inv) * g[c][3]);
     }
   }
   for (int i = threadIdx.x + NORM_CACHED * NORM_THREADS; i < n4; i += NORM_THREADS) {
@@ -261,8 +277,7 @@ extern "C" int axk_swiglu(const void* gate_up, void* out, int n_tokens, int n_ff
 // dtype if asked for (what the next sublayer's products read).  The sum of squares as in rmsnorm_kernel.
 // A row of few others is bound by how often it waits for memory: all that a thread needs of rows of up to
 // KEPT x 256 values (y, x, gain) is asked for at once, where y was read twice and x and the gain only behind
-// the sum.  With the rounding of the stream for the next block in the same pass, a decoding step of 8 rows of 2,048
-// values, eight of these passes: 538 -> 532 us; a prompt step of 2,048 rows 0.906 -> 0.897 of the same yardstick.
+// the sum.  Rows of 2,048 values, us, so / here: 8 rows 7.1 / 4.4, 2,048 rows 13.8 / 11.4.
 template <int KEPT>
 __global__ void __launch_bounds__(NORM_THREADS)
 norm_add_kernel(const float* __restrict__ y, const void* __restrict__ gain, int gain_is_f32, float eps, float mult,
@@ -273,22 +288,25 @@ norm_add_kernel(const float* __restrict__ y, const void* __restrict__ gain, int 
   float* dst = x + (size_t)r * dim;
   float ss = 0.0f;
   if constexpr (KEPT > 0) {
-    float v[KEPT], was[KEPT], g[KEPT];
+    float v[KEPT], was[KEPT], g[KEPT][1];
 #pragma unroll
     for (int c = 0; c < KEPT; ++c) {
-      const int i = threadIdx.x + c * NORM_THREADS;
-      v[c] = i < dim ? src[i] : 0.0f;
-      was[c] = i < dim ? dst[i] : 0.0f;
-      g[c] = i < dim ? load_vec(gain, gain_is_f32, i) : 0.0f;
+      const int i = min((int)threadIdx.x + c * NORM_THREADS, dim - 1);
+      v[c] = src[i];
+      was[c] = dst[i];
     }
+    load_vec_apart<KEPT, 1>(gain, gain_is_f32, threadIdx.x, NORM_THREADS, dim, g);
 #pragma unroll
-    for (int c = 0; c < KEPT; ++c) ss = fmaf(v[c], v[c], ss);
+    for (int c = 0; c < KEPT; ++c) {
+      v[c] = (int)threadIdx.x + c * NORM_THREADS < dim ? v[c] : 0.0f;
+      ss = fmaf(v[c], v[c], ss);
+    }
     const float inv = 1.0f / sqrtf(block_sum_256(ss, partial) / (float)dim + eps);
 #pragma unroll
     for (int c = 0; c < KEPT; ++c) {
       const int i = threadIdx.x + c * NORM_THREADS;
       if (i < dim) {
-        const float sum = was[c] + mult * ((v[c] * inv) * g[c]);
+        const float sum = was[c] + mult * ((v[c] * inv) * g[c][0]);
         dst[i] = sum;
         if (rounded) rounded[(size_t)r * dim + i] = from_float(sum);
       }

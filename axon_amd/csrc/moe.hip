@@ -2,6 +2,8 @@
 // and the (token, chosen expert) pairs listed expert by expert in tiles of up to 16 rows, which
 // the grouped product takes as its work list.  Everything stays on the device: the launches of a
 // step depend on the number of tokens alone.
+#include <type_traits>
+
 #include "api.h"
 #include "common.h"
 
@@ -257,26 +259,76 @@ route_sort_kernel(const int32_t* __restrict__ experts, int n_pairs, int n_expert
 // itself, or place_of[pair]; without weights the rows are added as they are.  extra (or null): a further
 // row a token, added last, times sigmoid(extra_gate[t extra_gate_stride]) if a gate is given.  input (or null): a pair
 // whose expert (experts[pair]) is n_experts or more is an identity, its row is input[t, :].
-__global__ void route_combine_kernel(const float* __restrict__ rows, const float* __restrict__ weights, float* __restrict__ y,
-                                     int top, int width, int accumulate, const int32_t* __restrict__ place_of,
-                                     const float* __restrict__ extra, const float* __restrict__ extra_gate, long extra_gate_stride,
-                                     const int32_t* __restrict__ experts, int n_experts, const elem_t* __restrict__ input,
-                                     long input_stride) {
+// G neighbouring columns a thread (4 where width and addresses allow), the rows of four, two and then one pair asked for together:
+// one after another, each waited for where its row lies and then for the row.
+// Four pairs and a further row of 2,048 columns, us, so / here: 2,126 tokens 31.3 / 19.4, 2,048 21.9 / 14.6, 8 4.7 / 4.6.
+template <int G>
+__global__ void __launch_bounds__(256)
+route_combine_kernel(const float* __restrict__ rows, const float* __restrict__ weights, float* __restrict__ y,
+                     int top, int width, int accumulate, const int32_t* __restrict__ place_of,
+                     const float* __restrict__ extra, const float* __restrict__ extra_gate, long extra_gate_stride,
+                     const int32_t* __restrict__ experts, int n_experts, const elem_t* __restrict__ input,
+                     long input_stride) {
   const int t = blockIdx.y;
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
+  const int c = G * (blockIdx.x * blockDim.x + threadIdx.x);
   if (c >= width) return;
-  float acc = accumulate ? y[(long)t * width + c] : 0.0f;
-  for (int k = 0; k < top; ++k) {
-    const long pair = (long)t * top + k;
-    const float row = input && experts[pair] >= n_experts ? to_float(input[(long)t * input_stride + c])
-                                                          : rows[(place_of ? (long)place_of[pair] : pair) * width + c];
-    acc = weights ? fmaf(weights[pair], row, acc) : acc + row;
+  auto load = [&](const float* from, float (&v)[G]) {
+    if constexpr (G == 4) {
+      const float4 q = *reinterpret_cast<const float4*>(from);
+      v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
+    } else {
+      v[0] = from[0];
+    }
+  };
+  float acc[G], more[G];
+  if (accumulate) load(y + (long)t * width + c, acc);
+  if (extra) load(extra + (long)t * width + c, more);
+  if (!accumulate) {
+#pragma unroll
+    for (int e = 0; e < G; ++e) acc[e] = 0.0f;
   }
+  const float gate = extra && extra_gate ? extra_gate[(long)t * extra_gate_stride] : 0.0f;
+  auto add = [&](int first, auto how_many) {
+    constexpr int PAIRS = decltype(how_many)::value;
+    const long pair = (long)t * top + first;
+    float row[PAIRS][G], weight[PAIRS];
+    long at[PAIRS];
+    bool own[PAIRS];                   // the pair's row is the token's input
+#pragma unroll
+    for (int j = 0; j < PAIRS; ++j) {
+      own[j] = input && experts[pair + j] >= n_experts;
+      at[j] = place_of ? (long)place_of[pair + j] : pair + j;
+      weight[j] = weights ? weights[pair + j] : 1.0f;
+    }
+#pragma unroll
+    for (int j = 0; j < PAIRS; ++j) {
+      if (own[j]) {
+#pragma unroll
+        for (int e = 0; e < G; ++e) row[j][e] = to_float(input[(long)t * input_stride + c + e]);
+      } else {
+        load(rows + at[j] * width + c, row[j]);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < PAIRS; ++j)
+#pragma unroll
+      for (int e = 0; e < G; ++e) acc[e] = weights ? fmaf(weight[j], row[j][e], acc[e]) : acc[e] + row[j][e];
+  };
+  int k = 0;
+  for (; k + 4 <= top; k += 4) add(k, std::integral_constant<int, 4>());
+  if (k + 2 <= top) {
+    add(k, std::integral_constant<int, 2>());
+    k += 2;
+  }
+  if (k < top) add(k, std::integral_constant<int, 1>());
   if (extra) {
-    const float e = extra[(long)t * width + c];
-    acc = extra_gate ? fmaf(1.0f / (1.0f + expf(-extra_gate[(long)t * extra_gate_stride])), e, acc) : acc + e;
+    const float share = 1.0f / (1.0f + expf(-gate));
+#pragma unroll
+    for (int e = 0; e < G; ++e) acc[e] = extra_gate ? fmaf(share, more[e], acc[e]) : acc[e] + more[e];
   }
-  y[(long)t * width + c] = acc;
+  float* to = y + (long)t * width + c;
+  if constexpr (G == 4) *reinterpret_cast<float4*>(to) = make_float4(acc[0], acc[1], acc[2], acc[3]);
+  else to[0] = acc[0];
 }
 
 // out[r, :] = x[rows[r], :] (rows of the compute dtype).
@@ -357,10 +409,13 @@ extern "C" int axk_route_combine(const float* rows, const float* weights, float*
               width);
   AXK_REQUIRE(input == nullptr || (experts != nullptr && input_stride >= width), "route_combine: identities need the chosen experts and rows of %d", width);
   if (n_tokens == 0) return 0;
-  dim3 grid(ceil_div(width, 256), n_tokens);
-  route_combine_kernel<<<grid, 256, 0, (hipStream_t)stream>>>(rows, weights, y, top, width, accumulate, place_of, extra,
-                                                              extra_gate, extra_gate_stride, experts, n_experts,
-                                                              (const elem_t*)input, input_stride);
+  const bool vec = width % 4 == 0 && (((uintptr_t)rows | (uintptr_t)y | (uintptr_t)extra) & 15) == 0;
+  auto kernel = vec ? route_combine_kernel<4> : route_combine_kernel<1>;
+  // (few tokens: blocks of a wave, so that a token's columns are on several CUs)
+  const int threads = vec && n_tokens < 256 ? 64 : 256;
+  kernel<<<dim3(ceil_div(width, (vec ? 4 : 1) * threads), n_tokens), threads, 0, (hipStream_t)stream>>>(
+      rows, weights, y, top, width, accumulate, place_of, extra, extra_gate, extra_gate_stride, experts, n_experts,
+      (const elem_t*)input, input_stride);
   AXK_LAUNCH_CHECK("route_combine");
   return 0;
 }

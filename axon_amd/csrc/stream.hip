@@ -32,6 +32,8 @@ __device__ inline int last_of_request(const int32_t* __restrict__ seq_rows, int 
   return in;
 }
 
+// VEC: eight neighbouring numbers a thread (as the embedding without pairs takes them).
+template <bool VEC>
 __global__ void __launch_bounds__(ST_THREADS)
 embed_pairs_kernel(const int32_t* __restrict__ tokens, const elem_t* __restrict__ table, int packed, float scale,
                    const elem_t* __restrict__ pairs, int buckets, long mul_prev, long mul_cur, int32_t* __restrict__ state,
@@ -39,6 +41,18 @@ embed_pairs_kernel(const int32_t* __restrict__ tokens, const elem_t* __restrict_
                    int dim) {
   __shared__ int pair_row;
   const int t = blockIdx.x, token = tokens[t];
+  float* dst = x + (size_t)t * dim;
+  const elem_t* row = packed ? table + (size_t)(token / 16) * (dim / 32) * 512 + (token % 16) * 8 : table + (size_t)token * dim;
+  auto place = [&](int i) { return packed ? (size_t)(i / 32) * 512 + ((i % 32) / 8) * 128 + i % 8 : (size_t)i; };
+  float mine[2][8];                    // the token's own numbers, under way while the pair's row is looked up
+  if constexpr (VEC) {
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const int i = min(8 * ((int)threadIdx.x + c * ST_THREADS), dim - 8);
+      load4_guarded(row + place(i), 4, true, mine[c]);
+      load4_guarded(row + place(i) + 4, 4, true, mine[c] + 4);
+    }
+  }
   if (threadIdx.x == 0) {
     const int slot = seq_rows[t], pos = positions[t];
     int before = -1;
@@ -53,15 +67,31 @@ embed_pairs_kernel(const int32_t* __restrict__ tokens, const elem_t* __restrict_
   }
   __syncthreads();
   const elem_t* pair = pairs + (size_t)pair_row * dim;
-  float* dst = x + (size_t)t * dim;
-  if (packed) {
-    const elem_t* tile = table + (size_t)(token / 16) * (dim / 32) * 512 + (token % 16) * 8;
-    for (int i = threadIdx.x; i < dim; i += ST_THREADS)
-      dst[i] = fmaf(to_float(tile[(size_t)(i / 32) * 512 + ((i % 32) / 8) * 128 + i % 8]), scale, to_float(pair[i]));
-    return;
+  auto put = [&](int i, const float* v) {
+    float p[8];
+    load4_guarded(pair + i, 4, true, p);
+    load4_guarded(pair + i + 4, 4, true, p + 4);
+    float sum[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) sum[e] = fmaf(v[e], scale, p[e]);
+    *reinterpret_cast<float4*>(dst + i) = make_float4(sum[0], sum[1], sum[2], sum[3]);
+    *reinterpret_cast<float4*>(dst + i + 4) = make_float4(sum[4], sum[5], sum[6], sum[7]);
+  };
+  if constexpr (VEC) {
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const int i = 8 * (threadIdx.x + c * ST_THREADS);
+      if (i < dim) put(i, mine[c]);
+    }
+    for (int i = 8 * (threadIdx.x + 2 * ST_THREADS); i < dim; i += 8 * ST_THREADS) {
+      float v[8];
+      load4_guarded(row + place(i), 4, true, v);
+      load4_guarded(row + place(i) + 4, 4, true, v + 4);
+      put(i, v);
+    }
+  } else {
+    for (int i = threadIdx.x; i < dim; i += ST_THREADS) dst[i] = fmaf(to_float(row[place(i)]), scale, to_float(pair[i]));
   }
-  const elem_t* row = table + (size_t)token * dim;
-  for (int i = threadIdx.x; i < dim; i += ST_THREADS) dst[i] = fmaf(to_float(row[i]), scale, to_float(pair[i]));
 }
 
 // G neighbouring numbers (4 where the width and the addresses allow, else 1).
@@ -104,7 +134,10 @@ __device__ inline float inverse_rms(const float* __restrict__ row, int dim, floa
 
 // A block a row.  y1 may be null; scales are float32 [dim]; norm_eps < 0: that output is taken as it is.  h null: no
 // norm behind the sum; share null: no shift.  With a shift every row is a request of its own.
-template <int G>
+// Few rows wait for memory and do little else, so rows of up to KEPT x 256 G numbers are asked for at once, with everything that the
+// sums and the shift want of them, and are not read again behind them (KEPT 0: any width, read as often as used).
+// 16 rows of 2,048, us, read again / here: 5.6 / 4.5.
+template <int G, int KEPT>
 __global__ void __launch_bounds__(ST_THREADS)
 scaled_sum_kernel(const float* __restrict__ y0, const float* __restrict__ s0, float norm_eps0, const float* __restrict__ y1,
                   const float* __restrict__ s1, float norm_eps1, float* __restrict__ x, const float* __restrict__ gain, float eps,
@@ -113,50 +146,106 @@ scaled_sum_kernel(const float* __restrict__ y0, const float* __restrict__ s0, fl
   __shared__ float partial[3][ST_THREADS / AXON_WAVE];
   const int t = blockIdx.x;
   const size_t at = (size_t)t * dim;
-  const float inv0 = norm_eps0 >= 0.0f ? inverse_rms<G>(y0 + at, dim, norm_eps0, partial[0]) : 1.0f;
-  const float inv1 = y1 != nullptr && norm_eps1 >= 0.0f ? inverse_rms<G>(y1 + at, dim, norm_eps1, partial[1]) : 1.0f;
-  float ss = 0.0f;
-  for (int i = G * threadIdx.x; i < dim; i += G * ST_THREADS) {
-    float v[G], y[G], s[G];
-    st_load<G>(x + at + i, v);
-    st_load<G>(y0 + at + i, y);
-    st_load<G>(s0 + i, s);
-#pragma unroll
-    for (int e = 0; e < G; ++e) y[e] = (y[e] * inv0) * s[e];
-    if (y1 != nullptr) {
-      float z[G];
-      st_load<G>(y1 + at + i, z);
-      st_load<G>(s1 + i, s);
-#pragma unroll
-      for (int e = 0; e < G; ++e) y[e] = fmaf(z[e] * inv1, s[e], y[e]);
-    }
-#pragma unroll
-    for (int e = 0; e < G; ++e) { v[e] += y[e]; ss = fmaf(v[e], v[e], ss); }
-    st_store<G>(x + at + i, v);
-  }
-  if (h == nullptr) return;
-  const float inv = 1.0f / sqrtf(block_sum_256(ss, partial[2]) / (float)dim + eps);
   const float* kept = nullptr;
   float* keep = nullptr;
   if (share != nullptr) {
     kept = rec_copy_before(state, state_stride, dim, seq_rows[t], positions[t]);
     keep = rec_copy_behind(state, state_stride, dim, seq_rows[t], positions[t]);
   }
-  for (int i = G * threadIdx.x; i < dim; i += G * ST_THREADS) {
-    float v[G], g[G];
-    st_load<G>(x + at + i, v);                     // what this thread stored above
-    st_load<G>(gain + i, g);
+  // (y0 + y1) of a row, added to x; the result's squares go on in ss
+  auto add = [&](float (&v)[G], float (&y)[G], const float (&z)[G], const float (&scale0)[G], const float (&scale1)[G], float inv0,
+                 float inv1, float& ss) {
+#pragma unroll
+    for (int e = 0; e < G; ++e) y[e] = (y[e] * inv0) * scale0[e];
+    if (y1 != nullptr) {
+#pragma unroll
+      for (int e = 0; e < G; ++e) y[e] = fmaf(z[e] * inv1, scale1[e], y[e]);
+    }
+#pragma unroll
+    for (int e = 0; e < G; ++e) { v[e] += y[e]; ss = fmaf(v[e], v[e], ss); }
+  };
+  // the norm of a row's numbers, and with a shift what goes to the state and comes from it
+  auto finish = [&](int i, float (&v)[G], const float (&g)[G], const float (&p)[G], const float (&m)[G], float inv) {
 #pragma unroll
     for (int e = 0; e < G; ++e) v[e] = (v[e] * inv) * g[e];
     if (share != nullptr) {
-      float p[G], m[G];
-      st_load<G>(kept + i, p);
-      st_load<G>(share + i, m);
       st_store<G>(keep + i, v);
 #pragma unroll
       for (int e = 0; e < G; ++e) v[e] = fmaf(p[e] - v[e], m[e], v[e]);
     }
     st_store_elem<G>(h + at + i, v);
+  };
+  float ss = 0.0f;
+  if constexpr (KEPT > 0) {
+    float v[KEPT][G], y[KEPT][G], z[KEPT][G], sc0[KEPT][G], sc1[KEPT][G], g[KEPT][G], p[KEPT][G], m[KEPT][G];
+#pragma unroll
+    for (int c = 0; c < KEPT; ++c) {
+      const int i = G * (threadIdx.x + c * ST_THREADS);
+      if (i >= dim) continue;
+      st_load<G>(y0 + at + i, y[c]);
+      if (y1 != nullptr) st_load<G>(y1 + at + i, z[c]);
+      st_load<G>(x + at + i, v[c]);
+      st_load<G>(s0 + i, sc0[c]);
+      if (y1 != nullptr) st_load<G>(s1 + i, sc1[c]);
+      if (h != nullptr) st_load<G>(gain + i, g[c]);
+      if (share != nullptr) {
+        st_load<G>(kept + i, p[c]);
+        st_load<G>(share + i, m[c]);
+      }
+    }
+    auto inverse = [&](const float (&row)[KEPT][G], float norm_eps, float* sums) {      // the order of inverse_rms
+      float squares = 0.0f;
+#pragma unroll
+      for (int c = 0; c < KEPT; ++c)
+        if (G * ((int)threadIdx.x + c * ST_THREADS) < dim) {
+#pragma unroll
+          for (int e = 0; e < G; ++e) squares = fmaf(row[c][e], row[c][e], squares);
+        }
+      return 1.0f / sqrtf(block_sum_256(squares, sums) / (float)dim + norm_eps);
+    };
+    const float inv0 = norm_eps0 >= 0.0f ? inverse(y, norm_eps0, partial[0]) : 1.0f;
+    const float inv1 = y1 != nullptr && norm_eps1 >= 0.0f ? inverse(z, norm_eps1, partial[1]) : 1.0f;
+#pragma unroll
+    for (int c = 0; c < KEPT; ++c) {
+      const int i = G * (threadIdx.x + c * ST_THREADS);
+      if (i >= dim) continue;
+      add(v[c], y[c], z[c], sc0[c], sc1[c], inv0, inv1, ss);
+      st_store<G>(x + at + i, v[c]);
+    }
+    if (h == nullptr) return;
+    const float inv = 1.0f / sqrtf(block_sum_256(ss, partial[2]) / (float)dim + eps);
+#pragma unroll
+    for (int c = 0; c < KEPT; ++c) {
+      const int i = G * (threadIdx.x + c * ST_THREADS);
+      if (i < dim) finish(i, v[c], g[c], p[c], m[c], inv);
+    }
+  } else {
+    const float inv0 = norm_eps0 >= 0.0f ? inverse_rms<G>(y0 + at, dim, norm_eps0, partial[0]) : 1.0f;
+    const float inv1 = y1 != nullptr && norm_eps1 >= 0.0f ? inverse_rms<G>(y1 + at, dim, norm_eps1, partial[1]) : 1.0f;
+    for (int i = G * threadIdx.x; i < dim; i += G * ST_THREADS) {
+      float v[G], y[G], z[G] = {}, sc0[G], sc1[G] = {};
+      st_load<G>(x + at + i, v);
+      st_load<G>(y0 + at + i, y);
+      st_load<G>(s0 + i, sc0);
+      if (y1 != nullptr) {
+        st_load<G>(y1 + at + i, z);
+        st_load<G>(s1 + i, sc1);
+      }
+      add(v, y, z, sc0, sc1, inv0, inv1, ss);
+      st_store<G>(x + at + i, v);
+    }
+    if (h == nullptr) return;
+    const float inv = 1.0f / sqrtf(block_sum_256(ss, partial[2]) / (float)dim + eps);
+    for (int i = G * threadIdx.x; i < dim; i += G * ST_THREADS) {
+      float v[G], g[G], p[G] = {}, m[G] = {};
+      st_load<G>(x + at + i, v);                     // what this thread stored above
+      st_load<G>(gain + i, g);
+      if (share != nullptr) {
+        st_load<G>(kept + i, p);
+        st_load<G>(share + i, m);
+      }
+      finish(i, v, g, p, m, inv);
+    }
   }
 }
 
@@ -221,9 +310,10 @@ extern "C" int axk_embed_pairs(const int32_t* tokens, const void* table, int pac
   AXK_REQUIRE(mul_prev < (1L << 31) && mul_cur < (1L << 31), "embed_pairs: multipliers %ld and %ld", mul_prev, mul_cur);
   AXK_REQUIRE(!packed || dim % 32 == 0, "embed_pairs: a packed table has rows of whole blocks of 32, not %d", dim);
   if (n_tokens == 0) return 0;
-  embed_pairs_kernel<<<n_tokens, ST_THREADS, 0, (hipStream_t)stream>>>(tokens, (const elem_t*)table, packed, scale, (const elem_t*)pairs,
-                                                                       buckets, mul_prev, mul_cur, state, positions, seq_rows, x,
-                                                                       n_tokens, dim);
+  const bool vec = dim % 8 == 0 && (((uintptr_t)table | (uintptr_t)pairs | (uintptr_t)x) & 15) == 0;
+  auto kernel = vec ? embed_pairs_kernel<true> : embed_pairs_kernel<false>;
+  kernel<<<n_tokens, ST_THREADS, 0, (hipStream_t)stream>>>(tokens, (const elem_t*)table, packed, scale, (const elem_t*)pairs, buckets,
+                                                           mul_prev, mul_cur, state, positions, seq_rows, x, n_tokens, dim);
   AXK_LAUNCH_CHECK("embed_pairs");
   return 0;
 }
@@ -240,7 +330,9 @@ extern "C" int axk_scaled_sum(const float* y0, const float* s0, float norm_eps0,
   const bool vec = dim % 4 == 0 && state_stride % 4 == 0 &&
                    (((uintptr_t)y0 | (uintptr_t)s0 | (uintptr_t)y1 | (uintptr_t)s1 | (uintptr_t)x | (uintptr_t)gain | (uintptr_t)h |
                      (uintptr_t)share | (uintptr_t)state) & 15) == 0;
-  auto kernel = vec ? scaled_sum_kernel<4> : scaled_sum_kernel<1>;
+  const int kept = dim <= 4 * ST_THREADS ? 1 : dim <= 8 * ST_THREADS ? 2 : dim <= 16 * ST_THREADS ? 4 : 0;
+  auto kernel = !vec ? scaled_sum_kernel<1, 0> : kept == 1 ? scaled_sum_kernel<4, 1> : kept == 2 ? scaled_sum_kernel<4, 2>
+              : kept == 4 ? scaled_sum_kernel<4, 4> : scaled_sum_kernel<4, 0>;
   kernel<<<n_tokens, ST_THREADS, 0, (hipStream_t)stream>>>(y0, s0, norm_eps0, y1, s1, norm_eps1, x, gain, eps, (elem_t*)h, share, state,
                                                            state_stride, positions, seq_rows, dim);
   AXK_LAUNCH_CHECK("scaled_sum");
