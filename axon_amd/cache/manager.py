@@ -154,6 +154,12 @@ class CacheManager:
         sized = [(e, "float32") if isinstance(e, int) else (int(e[0]), str(e[1])) for e in state_elems]
         self.states = [torch.zeros((max_seqs, max(e, 1)), dtype=getattr(torch, dt), device=device) if device is not None
                        else None for e, dt in sized]
+        # a new request's rows are cleared by a launch a type, not one a run (4.3 us each on the device, as much on the host)
+        by_type: dict = {}
+        for s in self.states:
+            if s is not None:
+                by_type.setdefault(s.dtype, []).append(s)
+        self._states_by_type = list(by_type.values())
         self._dirty: set = set()
 
     def __del__(self):
@@ -178,9 +184,8 @@ class CacheManager:
         slot = self.lib.axh_cache_open(self._h)
         if slot < 0:
             raise CacheError(self._error())
-        for s in self.states:
-            if s is not None:
-                s[slot].zero_()
+        for states in self._states_by_type:
+            torch._foreach_zero_([s[slot] for s in states])
         return slot
 
     def close(self, slot: int) -> int:
