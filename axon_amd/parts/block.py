@@ -151,7 +151,9 @@ class SublayerNormBlock(Block):
         if self.feed_forward is not None:
             self._run(self.feed_forward, ctx, y, x if exact else h)
             k.norm_add(y, self.norm2.gain, self.norm2.eps, self.mult, x, h)
-        ctx.shared[ROUNDED_STREAM] = None if exact else (x, h)
+        # (a subclass's forward may go on behind this one and rewrite the stream: it leaves what it knows to be its rows itself)
+        whole = getattr(self.forward, "__func__", None) is SublayerNormBlock.forward
+        ctx.shared[ROUNDED_STREAM] = (x, h) if whole and not exact else None
 
     @staticmethod
     def rounded(ctx, x):
