@@ -160,11 +160,12 @@ class DecoderModel:
             if i + 1 < end and self.order[i + 1].enter is None:     # a rewritten stream is normed by its own pass
                 after = self.blocks[self.order[i + 1].layer]
                 following = block.following_of(ctx, block.last_part(), after.entry_norm(self.cache_plan.bindings[i + 1]), x.shape[0])
+            found = ctx.shared.get(ROUNDED_STREAM)
             if normed is None and following is None:
                 block.forward(ctx, binding, x)          # a block that knows nothing of this is called plainly
             else:
                 block.forward(ctx, binding, x, normed, following)
-            if not getattr(block, "leaves_rounded_stream", False):
+            if ctx.shared.get(ROUNDED_STREAM) is found:     # nothing of its own: what was there is older than the stream
                 ctx.shared[ROUNDED_STREAM] = None
             normed = None if following is None else following.values
 

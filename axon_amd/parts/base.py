@@ -272,9 +272,10 @@ class StreamEntry(Part):
         raise NotImplementedError
 
 
-# A block that says `leaves_rounded_stream` leaves in ctx.shared, under this key, (the stream, its rows in the compute
-# dtype) for the block after it; whatever else rewrites the stream sets the value to None.  What runs in order leaves
-# it among itself only: another call of the decoder's `forward_runs` does not find it.
+# A block may leave in ctx.shared, under this key, (the stream, its rows in the compute dtype) for the block after it;
+# whatever else rewrites the stream between two blocks sets the value to None, and behind a block that left nothing of
+# its own the decoder does.  What runs in order leaves it among itself only: another call of the decoder's
+# `forward_runs` does not find it.
 ROUNDED_STREAM = "rounded rows of the stream"
 
 
@@ -284,7 +285,6 @@ class Block(Part):
     A block that wants the speed of norms finished by the product before them calls
     `run_part` for its mixer and feed-forward and `normed` for its norms (below); one that does
     not calls the parts plainly, and everything still works."""
-    leaves_rounded_stream = False
 
     def __init__(self, norm_factory: Callable[[str], Norm], mixer: Mixer, feed_forward: FeedForward, prefix: str):
         super().__init__({}, prefix)

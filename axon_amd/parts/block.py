@@ -108,7 +108,6 @@ class SublayerNormBlock(Block):
     next sublayer, the next block's too.  The norms are RMS norms (they hand over a gain and an eps).
     `residual_mult` comes with the norm's parameters."""
     graph_safe = True
-    leaves_rounded_stream = True
     norm1_name = "norm1"
     norm2_name = "norm2"
 
@@ -275,7 +274,6 @@ class SandwichNormBlock(Block):
         return norm.following_values(ctx, n_rows) if hasattr(norm, "following_values") else None
 
     _run = staticmethod(SublayerNormBlock._run)
-    rounded = staticmethod(SublayerNormBlock.rounded)
 
     def forward(self, ctx, binding: CacheBinding, x, normed=None, following=None) -> None:
         h = normed if normed is not None else self.norms[0].forward(ctx, x)

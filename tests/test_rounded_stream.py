@@ -3,7 +3,8 @@ only those.  The real blocks over a stand-in for the kernels, on the CPU."""
 import torch
 
 from axon_amd.models.decoder import DecoderModel
-from axon_amd.parts.block import SublayerNormBlock
+from axon_amd.parts.base import ROUNDED_STREAM
+from axon_amd.parts.block import PostNormBlock, SublayerNormBlock
 
 WIDTH = 8
 
@@ -78,6 +79,26 @@ def run(blocks):
     ctx.stream = torch.randn(3, WIDTH, generator=torch.Generator().manual_seed(1))
     model_of(blocks).forward_runs(ctx, ctx.stream, 0, len(blocks))
     return ctx.k.rounded
+
+
+def test_a_run_of_blocks_rounds_the_stream_once():
+    for kind in (SublayerNormBlock, PostNormBlock):
+        assert run([block_of(kind), block_of(kind, False), block_of(kind), block_of(kind)]) == 1, kind
+    assert run([block_of(SublayerNormBlock), block_of(PostNormBlock), block_of(SublayerNormBlock)]) == 1
+
+
+def test_a_block_of_another_part_that_leaves_rows_is_heard():
+    class Leaves(PostNormBlock):
+        def forward(self, ctx, binding, x, normed=None, following=None):
+            x.mul_(0.5)
+            ctx.shared[ROUNDED_STREAM] = (x, x.to(torch.bfloat16))
+
+    class Silent(PostNormBlock):
+        def forward(self, ctx, binding, x, normed=None, following=None):
+            x.mul_(0.5)
+    for kind in (SublayerNormBlock, PostNormBlock):
+        assert run([block_of(kind), block_of(Leaves), block_of(kind)]) == 1
+        assert run([block_of(kind), block_of(Silent), block_of(kind)]) == 2
 
 
 def test_a_subclass_may_go_on_behind_the_block_that_leaves_rows():
