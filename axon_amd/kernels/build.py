@@ -57,6 +57,10 @@ class BuildError(RuntimeError):
     pass
 
 
+class MissingError(BuildError):
+    """Nothing that failed to build: a compiler or a header is not there."""
+
+
 def _say(msg: str) -> None:
     print(f"[axon_amd build] {msg}", file=sys.stderr, flush=True)
 
@@ -145,7 +149,7 @@ def _find(tool: str, extra: List[str]) -> str:
     for cand in [shutil.which(tool)] + extra:
         if cand and os.path.exists(cand):
             return cand
-    raise BuildError(f"{tool} was not found: the native library cannot be built")
+    raise MissingError(f"{tool} was not found: the native library cannot be built")
 
 
 def _run(cmd: List[str], what: str) -> None:
@@ -218,7 +222,7 @@ def build_calls(force: bool = False) -> str:
     if not force and _fresh(name, CALLS_SOURCES, flags):
         return os.path.join(built_dir(), name)
     if not os.path.exists(os.path.join(include, "Python.h")):
-        raise BuildError(f"no Python.h in {include}")
+        raise MissingError(f"no Python.h in {include}")
     return _build(name, CALLS_SOURCES, _find("g++", ["/usr/bin/g++", "/usr/bin/c++"]), flags, ["-fPIC"], force)
 
 
@@ -236,6 +240,6 @@ def build_all(force: bool = True) -> List[str]:
     built = [build_host(force), build_kernels("float32", force), build_kernels("bfloat16", force)]
     try:
         built.append(build_calls(force))
-    except BuildError as e:                      # the calls go through ctypes then
+    except MissingError as e:                    # the calls go through ctypes then; what does not compile is an error here
         _say(str(e))
     return built

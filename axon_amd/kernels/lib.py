@@ -184,15 +184,17 @@ _PLAIN = ["axk_argmax_workspace", "axk_attention_decode_chunk", "axk_attention_d
 
 
 def _calls_module():
-    """The native callables of this interpreter (see csrc/host/calls.cpp), or None where they cannot be built."""
+    """The native callables of this interpreter (see csrc/host/calls.cpp), or None, and a line that says why, where there are none:
+    without Python's headers or a compiler, in a folder that cannot be written, or if they do not build."""
     global _calls
     if _calls is False:
         try:
             loader = importlib.machinery.ExtensionFileLoader("axon_calls", build.build_calls())
             _calls = importlib.util.module_from_spec(importlib.util.spec_from_loader("axon_calls", loader))
             loader.exec_module(_calls)
-        except (build.BuildError, ImportError):
+        except (build.BuildError, ImportError, OSError) as e:
             _calls = None
+            build._say(f"kernels are called through ctypes, at some 2 us more a launch: {e}")
     return _calls
 
 
