@@ -302,7 +302,6 @@ int axk_gather_rows(const void* x, long x_stride, const int32_t* rows, void* out
 // r = sigmoid(gates r), i = sigmoid(gates i), a = exp(-decay r softplus(lam)),
 // S = a S + sqrt(1 - a^2) (i u), out = S gelu(y); then the state row is brought up to date
 // (S, and the convolution's inputs from x).  gates [T, channels / block_width, 2 block_width].
-// terms and n_tokens are not used (they were room for an earlier form of the stretches' kernel).
 // axk_gated_scan_stretches: the same with spans, for requests of many tokens: what does not depend on the state is worked out
 // by other waves than the one that is left with a multiply-add a step (the same bits).
 int axk_causal_conv(const void* x, long x_stride, const void* w, const void* bias, int bias_is_f32, const float* state,
@@ -311,7 +310,7 @@ int axk_causal_conv(const void* x, long x_stride, const void* w, const void* bia
 int axk_gated_scan(const float* gates, const float* u, const void* y, long y_stride, const void* x, long x_stride,
                    const void* lam, int lam_is_f32, float decay, float* state, long state_stride, const int32_t* spans,
                    int n_spans, const int32_t* positions, const int32_t* seq_rows, void* out, int channels, int block_width,
-                   int taps, float* terms, int n_tokens, void* stream);
+                   int taps, void* stream);
 int axk_gated_scan_stretches(const float* gates, const float* u, const void* y, long y_stride, const void* x, long x_stride,
                              const void* lam, int lam_is_f32, float decay, float* state, long state_stride, const int32_t* spans,
                              int n_spans, const int32_t* positions, void* out, int channels, int block_width, int taps, void* stream);

@@ -349,7 +349,7 @@ extern "C" int axk_causal_conv(const void* x, long x_stride, const void* w, cons
 extern "C" int axk_gated_scan(const float* gates, const float* u, const void* y, long y_stride, const void* x, long x_stride,
                               const void* lam, int lam_is_f32, float decay, float* state, long state_stride,
                               const int32_t* spans, int n_spans, const int32_t* positions, const int32_t* seq_rows, void* out,
-                              int channels, int block_width, int taps, float* terms, int n_tokens, void* stream) {
+                              int channels, int block_width, int taps, void* stream) {
   AXK_REQUIRE(n_spans >= 0 && channels > 0 && block_width > 0 && channels % block_width == 0 && taps >= 1,
               "gated_scan: bad sizes spans=%d channels=%d block width=%d taps=%d", n_spans, channels, block_width, taps);
   AXK_REQUIRE(state_stride >= 2L * taps * channels, "gated_scan: a state row of %ld floats does not hold 2 x %d x %d",

@@ -119,7 +119,7 @@ _SIGNATURES = {
     "axk_causal_conv": [c_void_p, c_long, c_void_p, c_void_p, c_int, c_void_p, c_long, c_void_p, c_void_p, c_void_p, c_int, c_int,
                         c_int, c_void_p],
     "axk_gated_scan": [c_void_p, c_void_p, c_void_p, c_long, c_void_p, c_long, c_void_p, c_int, c_float, c_void_p, c_long,
-                       c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_int, c_void_p],
+                       c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p],
     "axk_gated_scan_stretches": [c_void_p, c_void_p, c_void_p, c_long, c_void_p, c_long, c_void_p, c_int, c_float, c_void_p, c_long,
                                  c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p],
     "axk_state_conv": [c_void_p, c_long, c_void_p, c_void_p, c_int, c_int, c_void_p, c_long, c_long, c_long, c_void_p, c_void_p,
@@ -1111,7 +1111,7 @@ class Kernels:
         self._check(self.run.axk_gated_scan(_ptr(gates), _ptr(u), _ptr(y), y.stride(0), _ptr(x), x.stride(0), _ptr(lam),
                                             self._vec_flag(lam, "scan lam"), float(decay), _ptr(state), state.stride(0),
                                             _ptr(spans), n, _ptr(positions), _ptr(seq_rows), _ptr(out), C, int(block_width),
-                                            int(taps), None, T, _queue()))
+                                            int(taps), _queue()))
         return out
 
     # ------------------------------------------------------------------ a state-space mixer with per-request state

@@ -63,9 +63,9 @@ def test_long_walk(dtype, lengths):
     got, want = (torch.empty(T, C, dtype=elem, device=dev) for _ in range(2))
     assert T > 4 * len(lengths)
     k.gated_scan(gates, u, y, x, lam, 8.0, state, spans, pos, seq, got, width, taps)
-    # without room for the terms a thread takes its channel's tokens one after another
+    # the other entry point: a thread takes its channel's tokens one after another
     assert k.lib.axk_gated_scan(_ptr(gates), _ptr(u), _ptr(y), C, _ptr(x), C, _ptr(lam), 1, 8.0, _ptr(kept), kept.stride(0),
-                                _ptr(spans), len(lengths), _ptr(pos), _ptr(seq), _ptr(want), C, width, taps, None, T, _stream()) == 0
+                                _ptr(spans), len(lengths), _ptr(pos), _ptr(seq), _ptr(want), C, width, taps, _stream()) == 0
     assert torch.equal(got, want) and torch.equal(state, kept)
 
 
@@ -89,5 +89,5 @@ def test_long_walk_by_width(dtype, lengths, channels):
     got, want = (torch.full((T, C), float("nan"), dtype=elem, device=dev) for _ in range(2))
     k.gated_scan(gates, u, yx[:, :C], yx[:, C:], lam, 8.0, state, spans, pos, seq, got, width, taps)
     assert k.lib.axk_gated_scan(_ptr(gates), _ptr(u), _ptr(yx), 2 * C, _ptr(yx[:, C:]), 2 * C, _ptr(lam), 1, 8.0, _ptr(kept), kept.stride(0),
-                                _ptr(spans), len(lengths), _ptr(pos), _ptr(seq), _ptr(want), C, width, taps, None, T, _stream()) == 0
+                                _ptr(spans), len(lengths), _ptr(pos), _ptr(seq), _ptr(want), C, width, taps, _stream()) == 0
     assert torch.equal(got, want) and torch.equal(state, kept)
