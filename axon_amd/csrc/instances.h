@@ -35,6 +35,7 @@ enum {
   INST_ATTENTION_F32_DECODE,     // float32 build, head_dim, waves a block
   INST_GEMM_FMA_BY_CHAIN,    // beside gemm_fma: rows of X a block, gated, numbers loaded four at a time
   INST_GEMM_FMA_FLOW,        // beside gemm_fma<128>: rows to LDS by direct loads; gated
+  INST_HEADS_PREPARE,        // 1: a block a token, 0: several
   INST_KINDS
 };
 

@@ -19,6 +19,7 @@
 #include <math.h>
 
 #include "api.h"
+#include "instances.h"
 #include "recurrence.h"
 
 namespace {
@@ -992,8 +993,12 @@ extern "C" int axk_heads_prepare(const float* proj, long stride, int q_at, int n
                 "heads_prepare: a convolution wants q, k and v side by side, all stored, normed head by head or not at all");
   }
   if (n_tokens == 0) return 0;
-  // a token's units side by side in several blocks (2,126 tokens of 16 + 2 heads, us, in one block / five: 23.8 / 22.3)
-  const int per_token = min((n_q + n_k + 3) / 4, 16);
+  // Few tokens: a token's units side by side in several blocks.  From 1,024 tokens on there are blocks enough, and what all blocks of a
+  // token do again (with norm_rows the sums over its whole rows) counts.  us, one block a token / up to 16: 32 + 8 heads of 128 normed
+  // over whole rows, 2,048 tokens 35 / 104, 16 + 2 17.2 / 25.7, of 8,192 tokens 52 / 124; with a convolution 16 + 2, 4,096 tokens 39.7 /
+  // 52.1; no norm 19.7 / 25.8; normed head by head 31.8 / 34.5, 2,048 tokens 19.4 / 19.5, and of 1,024 32 + 8 27.9 / 21.5.
+  const int per_token = n_tokens >= 1024 ? 1 : min((n_q + n_k + 3) / 4, 16);
+  if (n_tokens >= 1024) { AXK_INSTANCE(INST_HEADS_PREPARE, 1); } else { AXK_INSTANCE(INST_HEADS_PREPARE, 0); }
 #define HEADS_ARGS proj, stride, q_at, n_q, k_at, n_k, v_at, v_width, dim, q_gain, q_gain_is_f32, k_gain, k_gain_is_f32, eps, rot, neighbours, \
                    magnitude, table, positions, seq_rows, block_table, table_stride, (elem_t*)cache, page_size, (elem_t*)q_out, write_kv,      \
                    q_temp_coef, q_temp_every, norm_rows, cv

@@ -246,6 +246,40 @@ def check_rmsnorm(dtype, dim):
 
 
 # --------------------------------------------------------------------------- the cases
+def check_heads_prepare(dtype, T, form):
+    """Queries, keys and values of T tokens in one call: the bits of calls of 200 of them.  form: normed head by head, over whole rows,
+    not at all, or behind a convolution (single tokens, whose state the calls leave as they find it for the others)."""
+    k = kernels(dtype)
+    td, nq, nk, dim, page, conv = getattr(torch, dtype), 5, 2, 24, 16, form == "conv"
+    W = (nq + 2 * nk) * dim
+    proj = rnd(T, W, seed=T, device="cuda")
+    freqs, table = P.rope_freqs(dim // 2, 100.0).cuda(), torch.empty(T, dim // 4, 2, device="cuda")
+    pos = (torch.arange(T, dtype=torch.int32) % page).cuda()
+    seq = (torch.arange(T, dtype=torch.int32) if conv else torch.arange(T, dtype=torch.int32) // page).cuda()
+    k.rope_table(pos, freqs, table)
+    pages = int(seq.max()) + 1
+    block_table = torch.randperm(pages, generator=torch.Generator().manual_seed(1)).int().view(pages, 1).cuda()
+    gains = [None, None] if form == "none" else [rnd(n * dim if form == "rows" else dim, seed=n, device="cuda") for n in (nq, nk)]
+    w = rnd(W, 3, seed=9, device="cuda").to(td)
+
+    def run(step):
+        q = torch.full((T, nq * dim), 3.0, dtype=td, device="cuda")
+        cache = torch.full((pages, 1, page, 2 * nk * dim), 3.0, dtype=td, device="cuda")
+        state = rnd(pages, 4 * W, seed=8, device="cuda") if conv else None
+        for a in range(0, T, step):
+            b = min(T, a + step)
+            k.heads_prepare(proj[a:b], 0, nq, nq * dim, nk, (nq + nk) * dim, nk * dim, dim, *gains, 1e-6, dim // 2, False, 1.25, table[a:b],
+                            pos[a:b], seq[a:b], block_table, cache, page, q[a:b], norm_rows=form == "rows",
+                            conv=(w, state, 2 * W, None) if conv else None)
+        return q, cache, state
+    got = {}
+    hit = launched(k, dtype, lambda: got.setdefault("all", run(T)))
+    for a, b in zip(got["all"], run(200)):
+        assert a is None or torch.equal(a, b)
+    assert not bool((got["all"][0] == 3.0).all(1).any())
+    return hit
+
+
 # (names of the instances the case is meant to select, the check, its arguments)
 BF, F32 = "bfloat16", "float32"
 def check_grouped(dtype, M, G, N, K, glu):
@@ -503,6 +537,9 @@ CASES = [
     (F32, ["attention_f32_prefill<128>", "attention_f32_decode<128,1>"], check_attention_f32, (7, 1, 128, 64, 600, 0, 7)),
     (F32, ["attention_f32_decode<64,4>"], check_attention_f32, (8, 4, 64, 16, 140, 0, 40)),
     (F32, ["attention_f32_decode<128,4>"], check_attention_f32, (8, 4, 128, 32, 150, 60, 33)),
+    # heads laid out for attention: several blocks a token in steps of up to 1,023 tokens, one beyond
+    *[(dtype, [f"heads_prepare<{int(T > 1023)}>"], check_heads_prepare, (dtype, T, form))
+      for dtype in (BF, F32) for T, form in ((1023, "rows"), (1024, "rows"), (1024, "heads"), (1025, "none"), (1030, "conv"))],
     # attention on the matrix cores: (head size, query heads a block, pages of 64 positions or more)
     # and (head size, waves a block) (one wave a block in the decoding kernel up to 2,560 blocks of
     # positions, four beyond; two heads a block in the prompt kernel where tiles x heads are more
