@@ -36,6 +36,7 @@ enum {
   INST_GEMM_FMA_BY_CHAIN,    // beside gemm_fma: rows of X a block, gated, numbers loaded four at a time
   INST_GEMM_FMA_FLOW,        // beside gemm_fma<128>: rows to LDS by direct loads; gated
   INST_HEADS_PREPARE,        // 1: a block a token, 0: several
+  INST_STATE_CONV,           // 1: runs of tokens, 0: a thread a (token, channel)
   INST_KINDS
 };
 

@@ -17,7 +17,8 @@ const char* const KIND_NAMES[INST_KINDS] = {"gemm_fma", "gemm_tile", "gemm_strea
                                             "gemm_split_reduce", "attention_rows", "attention_prefill",
                                             "attention_decode", "rmsnorm", "grouped_gemm", "causal_conv",
                                             "latent_prompt", "latent_tokens", "gemm_kept", "attention_f32_prefill",
-                                            "attention_f32_decode", "gemm_fma_by_chain", "gemm_fma_flow", "heads_prepare"};
+                                            "attention_f32_decode", "gemm_fma_by_chain", "gemm_fma_flow", "heads_prepare",
+                                            "state_conv"};
 
 struct Registry {
   std::mutex lock;

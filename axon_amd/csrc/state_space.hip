@@ -18,6 +18,7 @@
 
 #include "api.h"
 #include "common.h"
+#include "instances.h"
 
 namespace {
 
@@ -703,9 +704,14 @@ extern "C" int axk_state_conv(const float* x, long x_stride, const void* w, cons
               "state_conv: step sizes of %d heads need their inputs", heads);
   AXK_REQUIRE(n_tokens <= 65535, "state_conv: %d tokens in one step (at most 65535)", n_tokens);
   if (n_tokens == 0) return 0;
-  // (from 256 tokens on, where it is the faster; terms of a token's head are stored as a pair)
-  if (n_tokens >= 256 && taps >= 2 && taps <= 4 && channels % 4 == 0 && x_stride % 4 == 0 && (((uintptr_t)x | (uintptr_t)u) & 15) == 0 &&
+  // Runs want enough of them to fill the chip: 6.2 million products (tokens x channels x taps).  us, a thread a (token, channel) / runs, one request:
+  // four taps 256 tokens of 2,560 channels 5.9 / 6.6, 512 9.4 / 7.8, but 512 single tokens 8.1 / 10.0; 256 of 6,144 11.4 / 8.0, single ones
+  // 10.9 / 10.2; 2,048 of 512 8.4 / 8.0, single ones 7.8 / 10.5; two taps 2,048 of 512 6.5 / 7.6, 512 of 6,144 13.9 / 9.0; four taps 1,024 of 64
+  // 2.9 / 12.6.  (Terms of a token's head are stored as a pair.)
+  if (n_tokens >= 256 && (long)n_tokens * channels * taps >= 6200000 && taps >= 2 && taps <= 4 && channels % 4 == 0 && x_stride % 4 == 0 &&
+      (((uintptr_t)x | (uintptr_t)u) & 15) == 0 &&
       ((uintptr_t)terms & 7) == 0) {
+    AXK_INSTANCE(INST_STATE_CONV, 1);
     auto kernel = taps == 2 ? state_conv_runs_kernel<2> : taps == 3 ? state_conv_runs_kernel<3> : state_conv_runs_kernel<4>;
     kernel<<<dim3(ceil_div(channels / 4 + heads, 128), ceil_div(n_tokens, SS_CONV_RUN)), 128, 0, (hipStream_t)stream>>>(
         x, x_stride, (const elem_t*)w, bias, bias_is_f32, silu, state, state_stride, copy_elems, tail_at, positions, seq_rows, u, n_tokens,
@@ -713,6 +719,7 @@ extern "C" int axk_state_conv(const float* x, long x_stride, const void* w, cons
     AXK_LAUNCH_CHECK("state_conv");
     return 0;
   }
+  AXK_INSTANCE(INST_STATE_CONV, 0);
   dim3 grid(ceil_div(channels + heads, 256), n_tokens);
   state_conv_kernel<<<grid, 256, 0, (hipStream_t)stream>>>(x, x_stride, (const elem_t*)w, bias, bias_is_f32, silu, state,
                                                           state_stride, copy_elems, tail_at, positions, seq_rows, u, channels,

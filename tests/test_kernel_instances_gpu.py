@@ -280,6 +280,21 @@ def check_heads_prepare(dtype, T, form):
     return hit
 
 
+def check_state_conv(dtype, T, C, taps):
+    """The convolution of one request's tokens against the same sums of float64."""
+    k = kernels(dtype)
+    td, copy = getattr(torch, dtype), (taps - 1) * C
+    x, w = rnd(T, C, seed=1, device="cuda"), rnd(C, taps, seed=2, device="cuda").to(td)
+    bias, state = rnd(C, seed=3, device="cuda"), rnd(1, 2 * copy, seed=4, device="cuda")
+    u, pos = torch.empty(T, C, device="cuda"), torch.arange(6, 6 + T, dtype=torch.int32, device="cuda")
+    hit = launched(k, dtype, lambda: k.state_conv(x, w, bias, state, copy, 0, pos, torch.zeros_like(pos), u, False))
+    rows = torch.cat([state[0, copy:].view(taps - 1, C), x]).double()         # the copy behind position 5
+    want = bias.double() + sum(rows[i:i + T] * w[:, i].double() for i in range(taps))
+    size = bias.double().abs() + sum((rows[i:i + T] * w[:, i].double()).abs() for i in range(taps))
+    assert bool(((u.double() - want).abs() <= (taps + 1) * 2.0 ** -24 * size).all())
+    return hit
+
+
 # (names of the instances the case is meant to select, the check, its arguments)
 BF, F32 = "bfloat16", "float32"
 def check_grouped(dtype, M, G, N, K, glu):
@@ -537,6 +552,9 @@ CASES = [
     (F32, ["attention_f32_prefill<128>", "attention_f32_decode<128,1>"], check_attention_f32, (7, 1, 128, 64, 600, 0, 7)),
     (F32, ["attention_f32_decode<64,4>"], check_attention_f32, (8, 4, 64, 16, 140, 0, 40)),
     (F32, ["attention_f32_decode<128,4>"], check_attention_f32, (8, 4, 128, 32, 150, 60, 33)),
+    # the convolution before a state-space scan: a thread a (token, channel), or runs of tokens
+    *[(dtype, [f"state_conv<{runs}>"], check_state_conv, (dtype, T, C, taps))
+      for dtype in (BF, F32) for T, C, taps, runs in ((300, 70, 3, 0), (260, 6000, 4, 1), (700, 4436, 2, 1), (2051, 1036, 3, 1))],
     # heads laid out for attention: several blocks a token in steps of up to 1,023 tokens, one beyond
     *[(dtype, [f"heads_prepare<{int(T > 1023)}>"], check_heads_prepare, (dtype, T, form))
       for dtype in (BF, F32) for T, form in ((1023, "rows"), (1024, "rows"), (1024, "heads"), (1025, "none"), (1030, "conv"))],

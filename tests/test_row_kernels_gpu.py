@@ -73,7 +73,8 @@ def test_scaled_sums(dim, outputs, normed, shifted, dtype):
 def test_state_convolution_of_many_tokens(lengths, taps, heads, pad, dtype):
     """Runs of eight tokens a thread: the bits of the requests one after the other, a thread a (token, channel), whatever runs
     their first tokens fall into."""
-    k, C, T, R = kernels(dtype), 268, sum(lengths), len(lengths)
+    k, T, R = kernels(dtype), sum(lengths), len(lengths)
+    C = 6200000 // (T * taps) // 4 * 4 + 12              # as few channels as the runs are taken for, and a block's last threads idle
     g = torch.Generator(device="cuda").manual_seed(T + taps)
     rows = torch.randn(T, C + pad, generator=g, device="cuda")
     w = torch.randn(C, taps, generator=g, device="cuda").to(k.dtype)
@@ -92,7 +93,9 @@ def test_state_convolution_of_many_tokens(lengths, taps, heads, pad, dtype):
         more = dict(raw=raw[a:b], dt_bias=dt_bias, a_log=a_log, terms=terms) if heads else {}
         k.state_conv(rows[a:b, :C], w, bias, state, copy, tail_at, positions[a:b].contiguous(), seq_rows[a:b].contiguous(), u, True, **more)
         return u, terms
+    k.reset_instances()
     whole, whole_terms = conv(0, T)
+    assert k.instances(launched=True) == ["state_conv<1>"]
     at = 0
     for n in lengths:
         for a in range(at, at + n, 255):                 # fewer tokens: the other kernel
@@ -102,6 +105,18 @@ def test_state_convolution_of_many_tokens(lengths, taps, heads, pad, dtype):
             assert torch.equal(u[first:], whole[a + first:b])
             assert not heads or torch.equal(terms, whole_terms[a:b])
         at += n
+    assert "state_conv<0>" in k.instances(launched=True)
+
+
+@pytest.mark.parametrize("T,C,taps,runs", [(256, 6056, 4, True), (256, 6052, 4, False), (255, 8000, 4, False), (1024, 64, 4, False), (512, 2560, 4, False),
+                                           (512, 6056, 2, True), (512, 6060, 5, False), (512, 6062, 2, False)])
+def test_the_convolution_by_runs_wants_enough_of_them(T, C, taps, runs):
+    k = kernels("bfloat16")
+    x, w = torch.zeros(T, C, device="cuda"), torch.zeros(C, taps, dtype=torch.bfloat16, device="cuda")
+    i, u = torch.zeros(T, dtype=torch.int32, device="cuda"), torch.empty(T, C, device="cuda")
+    k.reset_instances()
+    k.state_conv(x, w, None, torch.zeros(1, 2 * (taps - 1) * C, device="cuda"), (taps - 1) * C, 0, i, i, u)
+    assert k.instances(launched=True) == [f"state_conv<{int(runs)}>"]
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
