@@ -82,21 +82,34 @@ __device__ inline float4 load_vec4(const void* p, int is_f32, int i) {
   return make_float4(a.f, b.f, c.f, d.f);
 }
 
-// GROUPS groups of COUNT neighbouring numbers of such a vector, `stride` apart from number `first` on; for those from `end` on the last
-// one again.  All are asked for before the first is widened: where load_vec's choice of type stands between two loads, each is
-// waited for.
-template <int GROUPS, int COUNT>
-__device__ inline void load_vec_apart(const void* p, int is_f32, int first, int stride, int end, float (&out)[GROUPS][COUNT]) {
+// GROUPS groups of COUNT neighbouring numbers of such a vector, `stride` apart from `base` on, this thread's `mine` behind
+// that; of a group that goes past `end` the last COUNT before it, and with SKIP none of groups that begin there for every thread
+// (nothing then goes to `out`).  All are asked for before the first is widened: where load_vec's choice of type stands between two loads,
+// each is waited for.
+template <int GROUPS, int COUNT, bool SKIP>
+__device__ inline void load_vec_apart(const void* p, int is_f32, int base, int mine, int stride, int end, float (&out)[GROUPS][COUNT]) {
+  auto first = [&](int c) { return min(base + c * stride + mine, end - COUNT); };
   if (is_f32) {
 #pragma unroll
-    for (int c = 0; c < GROUPS * COUNT; ++c)
-      out[c / COUNT][c % COUNT] = ((const float*)p)[min(first + c / COUNT * stride + c % COUNT, end - 1)];
+    for (int c = 0; c < GROUPS; ++c) {
+      if (SKIP && base + c * stride >= end) continue;
+#pragma unroll
+      for (int e = 0; e < COUNT; ++e) out[c][e] = ((const float*)p)[first(c) + e];
+    }
   } else {
-    bf16_t raw[GROUPS * COUNT];
+    bf16_t raw[GROUPS][COUNT];
 #pragma unroll
-    for (int c = 0; c < GROUPS * COUNT; ++c) raw[c] = ((const bf16_t*)p)[min(first + c / COUNT * stride + c % COUNT, end - 1)];
+    for (int c = 0; c < GROUPS; ++c) {
+      if (SKIP && base + c * stride >= end) continue;
 #pragma unroll
-    for (int c = 0; c < GROUPS * COUNT; ++c) out[c / COUNT][c % COUNT] = bf16_to_float(raw[c]);
+      for (int e = 0; e < COUNT; ++e) raw[c][e] = ((const bf16_t*)p)[first(c) + e];
+    }
+#pragma unroll
+    for (int c = 0; c < GROUPS; ++c) {
+      if (SKIP && base + c * stride >= end) continue;
+#pragma unroll
+      for (int e = 0; e < COUNT; ++e) out[c][e] = bf16_to_float(raw[c][e]);
+    }
   }
 }
 

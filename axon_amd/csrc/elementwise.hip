@@ -74,7 +74,9 @@ __device__ inline void store4(elem_t* dst, float a, float b, float c, float d) {
 
 // Rows whose width is a multiple of 4: thread t takes the float4 t, t + 256, ...; the first
 // NORM_CACHED of them stay in registers between the sum and the scaling.  The order of the
-// sum depends on the width alone.
+// sum depends on the width alone.  BESIDE: the gain is asked for beside the row, not behind its sum, which many narrow rows, whose blocks
+// cover each other's waits, would rather have (8,192 rows of 512 with a bfloat16 gain 8.8 us so, 8.2 behind; of 4,096 32.7 / 37.8).
+template <bool BESIDE>
 __global__ void __launch_bounds__(NORM_THREADS)
 rmsnorm_vec_kernel(const float* __restrict__ x, const int32_t* __restrict__ rows, const void* __restrict__ gain,
                    int gain_is_f32, elem_t* __restrict__ out, int dim, float eps) {
@@ -82,13 +84,13 @@ rmsnorm_vec_kernel(const float* __restrict__ x, const int32_t* __restrict__ rows
   const int r = blockIdx.x, n4 = dim >> 2;
   const float4* src = reinterpret_cast<const float4*>(x + (size_t)(rows ? rows[r] : r) * dim);
   float4 kept[NORM_CACHED];
-  float g[NORM_CACHED][4];                           // the gain is asked for beside the row, not behind its sum
+  float g[NORM_CACHED][4];
 #pragma unroll
   for (int c = 0; c < NORM_CACHED; ++c) {
     const int i = threadIdx.x + c * NORM_THREADS;
     kept[c] = i < n4 ? src[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   }
-  load_vec_apart<NORM_CACHED, 4>(gain, gain_is_f32, 4 * threadIdx.x, 4 * NORM_THREADS, dim, g);
+  if constexpr (BESIDE) load_vec_apart<NORM_CACHED, 4, true>(gain, gain_is_f32, 0, 4 * threadIdx.x, 4 * NORM_THREADS, dim, g);
   float ss = 0.0f;
 #pragma unroll
   for (int c = 0; c < NORM_CACHED; ++c) {
@@ -112,6 +114,10 @@ rmsnorm_vec_kernel(const float* __restrict__ x, const int32_t* __restrict__ rows
     const int i = threadIdx.x + c * NORM_THREADS;
     if (i < n4) {
       const int e = i * 4;
+      if constexpr (!BESIDE) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) g[c][k] = load_vec(gain, gain_is_f32, e + k);
+      }
       store4(dst + e, (kept[c].x * inv) * g[c][0], (kept[c].y * inv) * g[c][1], (kept[c].z * inv) * g[c][2], (kept[c].w * inv) * g[c][3]);
     }
   }
@@ -152,8 +158,8 @@ extern "C" int axk_rmsnorm(const float* x, const int32_t* rows, const void* gain
   const bool vec = dim % 4 == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)out & 15) == 0;
   if (vec) {
     AXK_INSTANCE(INST_RMSNORM, 1);
-    rmsnorm_vec_kernel<<<n_rows, NORM_THREADS, 0, (hipStream_t)stream>>>(x, rows, gain, gain_is_f32, (elem_t*)out, dim,
-                                                                        eps);
+    auto kernel = dim <= 512 && n_rows >= 4096 ? rmsnorm_vec_kernel<false> : rmsnorm_vec_kernel<true>;
+    kernel<<<n_rows, NORM_THREADS, 0, (hipStream_t)stream>>>(x, rows, gain, gain_is_f32, (elem_t*)out, dim, eps);
   } else {
     AXK_INSTANCE(INST_RMSNORM, 0);
     rmsnorm_kernel<<<n_rows, NORM_THREADS, 0, (hipStream_t)stream>>>(x, rows, gain, gain_is_f32, (elem_t*)out, dim, eps);
@@ -277,7 +283,8 @@ extern "C" int axk_swiglu(const void* gate_up, void* out, int n_tokens, int n_ff
 // dtype if asked for (what the next sublayer's products read).  The sum of squares as in rmsnorm_kernel.
 // A row of few others is bound by how often it waits for memory: all that a thread needs of rows of up to
 // KEPT x 256 values (y, x, gain) is asked for at once, where y was read twice and x and the gain only behind
-// the sum.  Rows of 2,048 values, us, so / here: 8 rows 7.1 / 4.4, 2,048 rows 13.8 / 11.4.
+// the sum.  Rows of 2,048 values, us, so / here: 8 rows 7.1 / 4.4, 2,048 rows 13.8 / 11.4.  No more than the row has, or what is asked for
+// in vain costs more: 8,192 rows of 64 5.0 / 7.4 with four a thread, 5.0 with one.
 template <int KEPT>
 __global__ void __launch_bounds__(NORM_THREADS)
 norm_add_kernel(const float* __restrict__ y, const void* __restrict__ gain, int gain_is_f32, float eps, float mult,
@@ -295,7 +302,7 @@ norm_add_kernel(const float* __restrict__ y, const void* __restrict__ gain, int 
       v[c] = src[i];
       was[c] = dst[i];
     }
-    load_vec_apart<KEPT, 1>(gain, gain_is_f32, threadIdx.x, NORM_THREADS, dim, g);
+    load_vec_apart<KEPT, 1, false>(gain, gain_is_f32, 0, threadIdx.x, NORM_THREADS, dim, g);
 #pragma unroll
     for (int c = 0; c < KEPT; ++c) {
       v[c] = (int)threadIdx.x + c * NORM_THREADS < dim ? v[c] : 0.0f;
@@ -326,7 +333,7 @@ extern "C" int axk_norm_add(const float* y, const void* gain, int gain_is_f32, f
                             int n_rows, int dim, void* stream) {
   AXK_REQUIRE(n_rows >= 0 && dim > 0, "norm_add: bad sizes rows=%d dim=%d", n_rows, dim);
   if (n_rows == 0) return 0;
-  auto kernel = dim <= 4 * NORM_THREADS ? norm_add_kernel<4> : dim <= 8 * NORM_THREADS ? norm_add_kernel<8>
+  auto kernel = dim <= NORM_THREADS ? norm_add_kernel<1> : dim <= 2 * NORM_THREADS ? norm_add_kernel<2> : dim <= 4 * NORM_THREADS ? norm_add_kernel<4> : dim <= 8 * NORM_THREADS ? norm_add_kernel<8>
               : dim <= 16 * NORM_THREADS ? norm_add_kernel<16> : norm_add_kernel<0>;
   kernel<<<n_rows, NORM_THREADS, 0, (hipStream_t)stream>>>(y, gain, gain_is_f32, eps, mult, x, (elem_t*)rounded, dim);
   AXK_LAUNCH_CHECK("norm_add");

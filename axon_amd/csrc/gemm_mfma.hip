@@ -921,7 +921,7 @@ gemm_split_reduce_norm_kernel(const float* __restrict__ partial, int M, int N, c
     const int n = i * 4;
     float4* dst = reinterpret_cast<float4*>(out + (size_t)m * out_stride + n);
     float4 r = *dst;
-    load_vec_apart<1, 4>(norm.gain, norm.gain_is_f32, n, 0, N, gain);
+    load_vec_apart<1, 4, false>(norm.gain, norm.gain_is_f32, 0, n, 0, N, gain);
     float4 g = summed_segments<SPLITS>(partial + (size_t)m * N + n, plane);
     if (bias) {
       g.x += load_vec(bias, bias_is_f32, n);

@@ -650,6 +650,9 @@ state_space_carry_kernel(const float* __restrict__ u, const float* __restrict__ 
 // out[t, part] = ((v / sqrt(mean(v^2) + eps)) gain) with v = y[t, part] silu(z[t, part]): the gate first,
 // then the norm of each of `parts` equal parts of a row by its own root mean square.  A block a (token, part):
 // a strided chain a thread, a butterfly a wave, the four waves in order.
+// KEPT x 256 values of a part are read once, and their gain beside them, not behind the sum; no more than the part has (us, gain behind / four a
+// thread / here: 8,192 tokens of four parts of 16 26.4 / 30.0 / 26.4, of 640 53 / 43 / 43, 8 of one part of 1,024 3.2 / 2.6 / 2.6).
+template <int KEPT>
 __global__ void __launch_bounds__(256)
 gated_group_norm_kernel(const float* __restrict__ y, const float* __restrict__ z, long z_stride, const void* __restrict__ gain,
                         int gain_is_f32, float eps, elem_t* __restrict__ out, int width, int parts) {
@@ -657,32 +660,33 @@ gated_group_norm_kernel(const float* __restrict__ y, const float* __restrict__ z
   const int t = blockIdx.x / parts, part = blockIdx.x % parts, size = width / parts;
   const float* ys = y + (long)t * width + (long)part * size;
   const float* zs = z + (long)t * z_stride + (long)part * size;
-  float kept[4], gate[4], g[4][1];    // parts of up to 1,024 values are read once, and their gain beside them, not behind the sum
+  float kept[KEPT], gate[KEPT], g[KEPT][1];
   float ss = 0.0f;
 #pragma unroll
-  for (int c = 0; c < 4; ++c) {
+  for (int c = 0; c < KEPT; ++c) {
     const int i = min((int)threadIdx.x + 256 * c, size - 1);
     kept[c] = ys[i];
     gate[c] = zs[i];
   }
-  load_vec_apart<4, 1>(gain, gain_is_f32, part * size + threadIdx.x, 256, (part + 1) * size, g);
+  load_vec_apart<KEPT, 1, false>(gain, gain_is_f32, part * size, threadIdx.x, 256, (part + 1) * size, g);
 #pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    kept[c] = (int)threadIdx.x + 256 * c < size ? kept[c] * ss_silu(gate[c]) : 0.0f;
+  for (int c = 0; c < KEPT; ++c) {
+    if ((int)threadIdx.x + 256 * c < size) kept[c] *= ss_silu(gate[c]);
+    else kept[c] = 0.0f;
     ss = fmaf(kept[c], kept[c], ss);
   }
-  for (int i = threadIdx.x + 1024; i < size; i += 256) {
+  for (int i = threadIdx.x + 256 * KEPT; i < size; i += 256) {
     const float v = ys[i] * ss_silu(zs[i]);
     ss = fmaf(v, v, ss);
   }
   const float inv = 1.0f / sqrtf(block_sum_256(ss, partial) / (float)size + eps);
   elem_t* dst = out + (long)t * width + (long)part * size;
 #pragma unroll
-  for (int c = 0; c < 4; ++c) {
+  for (int c = 0; c < KEPT; ++c) {
     const int i = threadIdx.x + 256 * c;
     if (i < size) dst[i] = from_float((kept[c] * inv) * g[c][0]);
   }
-  for (int i = threadIdx.x + 1024; i < size; i += 256) {
+  for (int i = threadIdx.x + 256 * KEPT; i < size; i += 256) {
     const float v = ys[i] * ss_silu(zs[i]);
     dst[i] = from_float((v * inv) * load_vec(gain, gain_is_f32, part * size + i));
   }
@@ -793,8 +797,9 @@ extern "C" int axk_gated_group_norm(const float* y, const float* z, long z_strid
               "gated_group_norm: bad sizes T=%d width=%d parts=%d", n_tokens, width, parts);
   if (n_tokens == 0) return 0;
   AXK_REQUIRE((long)n_tokens * parts <= 2147483647L, "gated_group_norm: %d tokens in %d parts", n_tokens, parts);
-  gated_group_norm_kernel<<<(unsigned)((long)n_tokens * parts), 256, 0, (hipStream_t)stream>>>(y, z, z_stride, gain, gain_is_f32, eps,
-                                                                                               (elem_t*)out, width, parts);
+  const int size = width / parts;
+  auto kernel = size <= 256 ? gated_group_norm_kernel<1> : size <= 512 ? gated_group_norm_kernel<2> : gated_group_norm_kernel<4>;
+  kernel<<<(unsigned)((long)n_tokens * parts), 256, 0, (hipStream_t)stream>>>(y, z, z_stride, gain, gain_is_f32, eps, (elem_t*)out, width, parts);
   AXK_LAUNCH_CHECK("gated_group_norm");
   return 0;
 }

@@ -1,4 +1,4 @@
-"""The norm on a sublayer's output at the edges of what a thread keeps of a row (4, 8 and 16 times 256 values, and wider rows),
+"""The norm on a sublayer's output at the edges of what a thread keeps of a row (1, 2, 4, 8 and 16 times 256 values, and wider rows),
 and whose rounded rows a block takes for the stream's."""
 import pytest
 import torch
@@ -11,7 +11,7 @@ from axon_amd.parts.block import SublayerNormBlock
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
-@pytest.mark.parametrize("dim", [1, 255, 1023, 1024, 1025, 2048, 2049, 4095, 4096, 4097, 5000])
+@pytest.mark.parametrize("dim", [1, 255, 256, 257, 512, 513, 1023, 1024, 1025, 2048, 2049, 4095, 4096, 4097, 5000])
 def test_rows_of_any_width(dim, dtype):
     k = kernels(dtype)
     g = torch.Generator(device="cuda").manual_seed(dim)

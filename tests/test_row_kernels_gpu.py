@@ -205,3 +205,37 @@ def test_outputs_of_stretches_that_end_anywhere_in_a_chunk(n_state, dtype):
         k.state_space_scan(u[rows], terms[rows], skip, stepped, copy, tail_at, None, positions[rows], slots[rows], conv_in[rows], y, heads,
                            groups, vdim, n_state, taps)
         assert torch.equal(y, whole[rows]), at
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("dim", [4, 64, 508, 512, 516, 1024])
+def test_norms_of_many_rows_are_those_of_few(dim, dtype):
+    """Many narrow rows ask for the gain behind the sum, others beside the row: the same bits."""
+    k, T = kernels(dtype), 4096
+    g = torch.Generator(device="cuda").manual_seed(dim)
+    x, gain = torch.randn(T, dim, generator=g, device="cuda"), torch.randn(dim, generator=g, device="cuda")
+    for vector in (gain, gain.to(k.dtype)):
+        many, few = (torch.empty(n, dim, dtype=k.dtype, device="cuda") for n in (T, 7))
+        k.rmsnorm(x, vector, 1e-5, many)
+        rows = torch.tensor([0, 1, 63, 64, 2047, 4094, 4095], dtype=torch.int32, device="cuda")
+        k.rmsnorm(x, vector, 1e-5, few, rows)
+        assert torch.equal(many[rows.long()], few)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("size", [1, 64, 255, 256, 257, 512, 513, 1024, 1025, 1300])
+def test_gated_norms_of_parts(size, dtype):
+    """At the edges of what a thread keeps of a part (one, two and four values) and beyond."""
+    k, T, parts, eps = kernels(dtype), 3, 2, 1e-5
+    g = torch.Generator(device="cuda").manual_seed(size)
+    y, z = torch.randn(T, size * parts, generator=g, device="cuda"), torch.randn(T, size * parts + 4, generator=g, device="cuda")[:, :size * parts]
+    gain = torch.randn(size * parts, generator=g, device="cuda")
+    for vector in (gain, gain.to(k.dtype)):
+        out = torch.empty(T, size * parts, dtype=k.dtype, device="cuda")
+        k.gated_group_norm(y, z, vector, eps, out, parts)
+        v = (y.double() * z.double() * torch.sigmoid(z.double())).view(T, parts, size)
+        want = (v / torch.sqrt(v.square().mean(2, keepdim=True) + eps)).view(T, -1) * vector.double()
+        # the gate's exponential, sum, quotient and product in what is summed and scaled; the mean's chain and folds, a root, two quotients, two products;
+        # and a bfloat16 output is rounded to eight bits, by up to 2^-8 of itself
+        bound = (size / 256 + 32) * 2.0 ** -24 * want.abs() + (2.0 ** -8 if dtype == "bfloat16" else 0.0) * want.abs()
+        assert bool(((out.double() - want).abs() <= bound).all())
