@@ -135,8 +135,9 @@ __device__ inline float inverse_rms(const float* __restrict__ row, int dim, floa
 // A block a row.  y1 may be null; scales are float32 [dim]; norm_eps < 0: that output is taken as it is.  h null: no
 // norm behind the sum; share null: no shift.  With a shift every row is a request of its own.
 // Few rows wait for memory and do little else, so rows of up to KEPT x 256 G numbers are asked for at once, with everything that the
-// sums and the shift want of them, and are not read again behind them (KEPT 0: any width, read as often as used).
-// 16 rows of 2,048, us, read again / here: 5.6 / 4.5.
+// sums and the shift want of them, and are not read again behind them (KEPT 0: any width, read as often as used, and what is used once).
+// 16 rows of 2,048, us, read again / here: 5.6 / 4.5; one output without a norm, 64 rows of 4,096, 2.6 / 3.0; two with one, 2,048 rows of 2,560
+// 14.6, with four groups 16.1, with the three it has 14.4.
 template <int G, int KEPT>
 __global__ void __launch_bounds__(ST_THREADS)
 scaled_sum_kernel(const float* __restrict__ y0, const float* __restrict__ s0, float norm_eps0, const float* __restrict__ y1,
@@ -223,15 +224,21 @@ scaled_sum_kernel(const float* __restrict__ y0, const float* __restrict__ s0, fl
     const float inv0 = norm_eps0 >= 0.0f ? inverse_rms<G>(y0 + at, dim, norm_eps0, partial[0]) : 1.0f;
     const float inv1 = y1 != nullptr && norm_eps1 >= 0.0f ? inverse_rms<G>(y1 + at, dim, norm_eps1, partial[1]) : 1.0f;
     for (int i = G * threadIdx.x; i < dim; i += G * ST_THREADS) {
-      float v[G], y[G], z[G] = {}, sc0[G], sc1[G] = {};
+      float v[G], y[G], s[G];
       st_load<G>(x + at + i, v);
       st_load<G>(y0 + at + i, y);
-      st_load<G>(s0 + i, sc0);
+      st_load<G>(s0 + i, s);
+#pragma unroll
+      for (int e = 0; e < G; ++e) y[e] = (y[e] * inv0) * s[e];
       if (y1 != nullptr) {
+        float z[G];
         st_load<G>(y1 + at + i, z);
-        st_load<G>(s1 + i, sc1);
+        st_load<G>(s1 + i, s);
+#pragma unroll
+        for (int e = 0; e < G; ++e) y[e] = fmaf(z[e] * inv1, s[e], y[e]);
       }
-      add(v, y, z, sc0, sc1, inv0, inv1, ss);
+#pragma unroll
+      for (int e = 0; e < G; ++e) { v[e] += y[e]; ss = fmaf(v[e], v[e], ss); }
       st_store<G>(x + at + i, v);
     }
     if (h == nullptr) return;
@@ -330,9 +337,10 @@ extern "C" int axk_scaled_sum(const float* y0, const float* s0, float norm_eps0,
   const bool vec = dim % 4 == 0 && state_stride % 4 == 0 &&
                    (((uintptr_t)y0 | (uintptr_t)s0 | (uintptr_t)y1 | (uintptr_t)s1 | (uintptr_t)x | (uintptr_t)gain | (uintptr_t)h |
                      (uintptr_t)share | (uintptr_t)state) & 15) == 0;
-  const int kept = dim <= 4 * ST_THREADS ? 1 : dim <= 8 * ST_THREADS ? 2 : dim <= 16 * ST_THREADS ? 4 : 0;
+  const bool again = h != nullptr || norm_eps0 >= 0.0f || (y1 != nullptr && norm_eps1 >= 0.0f);       // a row is used behind its sum
+  const int kept = !again || dim > 16 * ST_THREADS ? 0 : (dim + 4 * ST_THREADS - 1) / (4 * ST_THREADS);
   auto kernel = !vec ? scaled_sum_kernel<1, 0> : kept == 1 ? scaled_sum_kernel<4, 1> : kept == 2 ? scaled_sum_kernel<4, 2>
-              : kept == 4 ? scaled_sum_kernel<4, 4> : scaled_sum_kernel<4, 0>;
+              : kept == 3 ? scaled_sum_kernel<4, 3> : kept == 4 ? scaled_sum_kernel<4, 4> : scaled_sum_kernel<4, 0>;
   kernel<<<n_tokens, ST_THREADS, 0, (hipStream_t)stream>>>(y0, s0, norm_eps0, y1, s1, norm_eps1, x, gain, eps, (elem_t*)h, share, state,
                                                            state_stride, positions, seq_rows, dim);
   AXK_LAUNCH_CHECK("scaled_sum");

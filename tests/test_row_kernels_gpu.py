@@ -1,5 +1,5 @@
 """Row kernels at the edges of what a thread keeps or takes at once: the embedding's eights, the scaled sum's rows of up to 1,024,
-2,048 and 4,096 numbers and wider ones, the convolution by runs of tokens."""
+2,048, 3,072 and 4,096 numbers and wider ones, the convolution by runs of tokens."""
 import pytest
 import torch
 
@@ -29,7 +29,7 @@ def test_embedding_rows(dim, dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
-@pytest.mark.parametrize("dim", [4, 1000, 1023, 1024, 1028, 2048, 2052, 4096, 4100])
+@pytest.mark.parametrize("dim", [4, 1000, 1023, 1024, 1028, 2048, 2052, 3072, 3076, 4096, 4100])
 @pytest.mark.parametrize("outputs,normed,shifted", [(1, False, False), (2, False, False), (1, True, True), (2, True, False), (2, True, True)])
 def test_scaled_sums(dim, outputs, normed, shifted, dtype):
     k, T, eps = kernels(dtype), 3, 1e-5
