@@ -39,10 +39,16 @@ extern "C" int axk_embed_scaled(const int32_t* tokens, const void* table, int pa
   AXK_REQUIRE(n_tokens >= 0 && dim > 0 && vocab > 0, "embed: bad sizes T=%d dim=%d vocab=%d", n_tokens, dim, vocab);
   AXK_REQUIRE(!packed || dim % 32 == 0, "embed: a packed table has rows of whole blocks of 32, not %d", dim);
   if (n_tokens == 0) return 0;
-  if (dim % 8 == 0 && (((uintptr_t)table | (uintptr_t)x) & 15) == 0)
+  // (A packed table's eights are 256 bytes apart, a line each a lane: steps of many tokens, whose rows come from HBM side by side, are the
+  // faster with eight lanes on one.  us, singles / eights: 152,064 packed rows of 3,584, 512 tokens 11.8 / 8.7, 1,024 15.9 / 16.4, 8,192 100 /
+  // 107; not packed 8,192 57.8 / 39.3.)
+  if (dim % 8 == 0 && (((uintptr_t)table | (uintptr_t)x) & 15) == 0 && !(packed && n_tokens >= 1024)) {
+    AXK_INSTANCE(INST_EMBED, 1);
     embed_kernel<true><<<dim3(n_tokens, ceil_div(dim, 8 * 256)), 256, 0, (hipStream_t)stream>>>(tokens, (const elem_t*)table, packed, x, dim, scale);
-  else
+  } else {
+    AXK_INSTANCE(INST_EMBED, 0);
     embed_kernel<false><<<n_tokens, 256, 0, (hipStream_t)stream>>>(tokens, (const elem_t*)table, packed, x, dim, scale);
+  }
   AXK_LAUNCH_CHECK("embed");
   return 0;
 }

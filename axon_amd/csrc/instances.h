@@ -37,6 +37,7 @@ enum {
   INST_GEMM_FMA_FLOW,        // beside gemm_fma<128>: rows to LDS by direct loads; gated
   INST_HEADS_PREPARE,        // 1: a block a token, 0: several
   INST_STATE_CONV,           // 1: runs of tokens, 0: a thread a (token, channel)
+  INST_EMBED,                // 1: eight numbers a thread, 0: one
   INST_KINDS
 };
 

@@ -295,6 +295,18 @@ def check_state_conv(dtype, T, C, taps):
     return hit
 
 
+def check_embed(dtype, T, dim, packed):
+    """Rows of a table, widened and scaled."""
+    k = kernels(dtype)
+    table = rnd(50, dim, seed=dim, device="cuda").to(getattr(torch, dtype))
+    tokens = torch.randint(0, 50, (T,), generator=torch.Generator().manual_seed(T), dtype=torch.int32).cuda()
+    out = torch.full((T + 1, dim), 7.0, device="cuda")
+    held = k.pack_matrix(table) if packed else table
+    hit = launched(k, dtype, lambda: k.embed(tokens, held, out[:T], 0.3))
+    assert torch.equal(out[:T], table[tokens.long()].float() * torch.tensor(0.3, device="cuda")) and bool((out[T] == 7.0).all())
+    return hit
+
+
 # (names of the instances the case is meant to select, the check, its arguments)
 BF, F32 = "bfloat16", "float32"
 def check_grouped(dtype, M, G, N, K, glu):
@@ -552,6 +564,9 @@ CASES = [
     (F32, ["attention_f32_prefill<128>", "attention_f32_decode<128,1>"], check_attention_f32, (7, 1, 128, 64, 600, 0, 7)),
     (F32, ["attention_f32_decode<64,4>"], check_attention_f32, (8, 4, 64, 16, 140, 0, 40)),
     (F32, ["attention_f32_decode<128,4>"], check_attention_f32, (8, 4, 128, 32, 150, 60, 33)),
+    # the embedding: eight numbers a thread, or one (unaligned rows, and many tokens of a packed table)
+    *[(dtype, [f"embed<{eights}>"], check_embed, (dtype, T, dim, False)) for dtype in (BF, F32) for T, dim, eights in ((5, 40, 1), (3, 35, 0), (1030, 64, 1))],
+    *[(BF, [f"embed<{int(T < 1024)}>"], check_embed, (BF, T, dim, True)) for T, dim in ((1023, 64), (1024, 64), (1100, 192), (7, 2112))],
     # the convolution before a state-space scan: a thread a (token, channel), or runs of tokens
     *[(dtype, [f"state_conv<{runs}>"], check_state_conv, (dtype, T, C, taps))
       for dtype in (BF, F32) for T, C, taps, runs in ((300, 70, 3, 0), (260, 6000, 4, 1), (700, 4436, 2, 1), (2051, 1036, 3, 1))],
