@@ -152,12 +152,15 @@ __global__ void route_scored_wave_kernel(const float* __restrict__ logits, long 
 // Which place a pair gets inside its expert's stretch is not fixed (atomic counters); no result
 // depends on it: every row of a product is a chain of its own.  Pairs whose expert is n_experts or more (an
 // identity, which has no matrices) are not listed.
-// Bound by its waits: the first SORT_KEPT pairs a thread are read at once and keep the place that counting them gave, so that they
-// are neither read nor counted again; the experts' stretches and tiles are summed up by all threads; and the lists are put in order in
-// LDS where they fit (`staged`), since two scattered words a pair are as many lines.  us, two counts a pair, one thread for the stretches
-// and scattered words / here: 2,048 tokens, 4 of 32 13.2 / 8.2, 6 of 64 21.9 / 8.3, 8 of 64 (too many to be staged) 26.8 / 16.5.
+// Bound by its waits: the first KEPT pairs a thread are read at once and keep the place that counting them gave, so that they
+// are neither read nor counted again; the experts' stretches and tiles are summed up by all threads, in as many steps as there are experts
+// for; and the lists are put in order in LDS where they fit (`staged`), since two scattered words a pair are as many lines.  us, two counts a
+// pair, one thread for the stretches and scattered words / here: 2,048 tokens, 4 of 32 13.2 / 8.2, 6 of 64 21.9 / 8.3, 8 of 64 (too many to be
+// staged) 26.8 / 16.5.  Few pairs want no more places than they are (8 tokens, 2 of 8, 2.4 / 3.8 with sixteen of them and six steps each of three
+// sums / 2.3 here; 4 of 32 4.3 / 3.8 / 2.5): one, four or sixteen a thread.
 #define SORT_THREADS 1024
 #define SORT_KEPT 16
+template <int KEPT>
 __global__ void __launch_bounds__(SORT_THREADS)
 route_sort_kernel(const int32_t* __restrict__ experts, int n_pairs, int n_experts, int top, int32_t* __restrict__ sorted,
                   int32_t* __restrict__ sorted_tokens, int32_t* __restrict__ tiles, int32_t* __restrict__ n_tiles,
@@ -167,20 +170,20 @@ route_sort_kernel(const int32_t* __restrict__ experts, int n_pairs, int n_expert
   __shared__ int waves[3][SORT_THREADS / AXON_WAVE], all;
   int *first = counts + n_experts, *next = first + n_experts;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  int expert[SORT_KEPT], rank[SORT_KEPT];
+  int expert[KEPT], rank[KEPT];
 #pragma unroll
-  for (int i = 0; i < SORT_KEPT; ++i) expert[i] = tid + SORT_THREADS * i < n_pairs ? experts[tid + SORT_THREADS * i] : n_experts;
+  for (int i = 0; i < KEPT; ++i) expert[i] = tid + SORT_THREADS * i < n_pairs ? experts[tid + SORT_THREADS * i] : n_experts;
   for (int e = tid; e < n_experts; e += SORT_THREADS) counts[e] = 0;
   __syncthreads();
 #pragma unroll
-  for (int i = 0; i < SORT_KEPT; ++i)
+  for (int i = 0; i < KEPT; ++i)
     if (expert[i] < n_experts) rank[i] = atomicAdd(&counts[expert[i]], 1);
   __syncthreads();
-  const bool more = n_pairs > SORT_THREADS * SORT_KEPT;
+  const bool more = n_pairs > SORT_THREADS * KEPT;
   if (more) {
     for (int e = tid; e < n_experts; e += SORT_THREADS) next[e] = counts[e];
     __syncthreads();
-    for (int p = tid + SORT_THREADS * SORT_KEPT; p < n_pairs; p += SORT_THREADS)
+    for (int p = tid + SORT_THREADS * KEPT; p < n_pairs; p += SORT_THREADS)
       if (experts[p] < n_experts) atomicAdd(&counts[experts[p]], 1);
     __syncthreads();
   }
@@ -192,18 +195,20 @@ route_sort_kernel(const int32_t* __restrict__ experts, int n_pairs, int n_expert
     sums[1] += (counts[e] + tile_rows - 1) / tile_rows;
     sums[2] += (counts[e] + wide_rows - 1) / wide_rows;
   }
+  int upto[3] = {sums[0], sums[1], sums[2]};
+  for (int off = 1; off < 64 && off < n_experts; off <<= 1) {      // (of fewer experts the lanes behind them are not asked)
 #pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    int upto = sums[k];
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const int other = __shfl_up(upto, off, 64);
-      upto += lane >= off ? other : 0;
+    for (int k = 0; k < 3; ++k) {
+      const int other = __shfl_up(upto[k], off, 64);
+      upto[k] += lane >= off ? other : 0;
     }
-    before[k] = upto - sums[k];
-    if (lane == 63) waves[k][wave] = upto;
   }
+#pragma unroll
+  for (int k = 0; k < 3; ++k) before[k] = upto[k] - sums[k];
   if (n_experts > 64) {                        // (else the first wave has them all)
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      if (lane == 63) waves[k][wave] = upto[k];
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < 3; ++k)
@@ -223,7 +228,7 @@ route_sort_kernel(const int32_t* __restrict__ experts, int n_pairs, int n_expert
       }
     before[0] += n;
   }
-  if (tid == (n_experts > 64 ? SORT_THREADS - 1 : 63)) {       // (its experts are the last, or it has none)
+  if (tid == (n_experts > 64 ? SORT_THREADS : n_experts) - 1) {       // (its experts are the last, or it has none)
     *n_tiles = before[1];
     if (wide_tiles) *n_wide = before[2];
     if (first_of) first_of[n_experts] = before[0];
@@ -242,9 +247,9 @@ route_sort_kernel(const int32_t* __restrict__ experts, int n_pairs, int n_expert
     if (place_of) place_of[p] = place;
   };
 #pragma unroll
-  for (int i = 0; i < SORT_KEPT; ++i)
+  for (int i = 0; i < KEPT; ++i)
     if (expert[i] < n_experts) put(tid + SORT_THREADS * i, first[expert[i]] + rank[i]);
-  for (int p = tid + SORT_THREADS * SORT_KEPT; p < n_pairs; p += SORT_THREADS)
+  for (int p = tid + SORT_THREADS * KEPT; p < n_pairs; p += SORT_THREADS)
     if (experts[p] < n_experts) put(p, atomicAdd(&next[experts[p]], 1));
   if (!staged) return;
   __syncthreads();
@@ -394,7 +399,8 @@ extern "C" int axk_route_sort(const int32_t* experts, int n_pairs, int n_experts
               "route_sort: a second list of tiles (of %d) comes with its length", wide_rows);
   const long lists = 3l * n_experts * (long)sizeof(int), order = (long)n_pairs * (long)sizeof(int);
   const bool staged = n_pairs > SORT_THREADS && lists + order <= 60 * 1024;       // (a launch gets 64 KB unasked)
-  route_sort_kernel<<<1, SORT_THREADS, lists + (staged ? order : 0), (hipStream_t)stream>>>(
+  auto kernel = n_pairs <= SORT_THREADS ? route_sort_kernel<1> : n_pairs <= 4 * SORT_THREADS ? route_sort_kernel<4> : route_sort_kernel<SORT_KEPT>;
+  kernel<<<1, SORT_THREADS, lists + (staged ? order : 0), (hipStream_t)stream>>>(
       experts, n_pairs, n_experts, top, sorted, sorted_tokens, tiles, n_tiles, place_of, first_of, tile_rows, wide_tiles, n_wide,
       wide_tiles ? wide_rows : tile_rows, staged);
   AXK_LAUNCH_CHECK("route_sort");

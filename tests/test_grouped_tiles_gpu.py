@@ -108,7 +108,8 @@ def test_lists_of_128_rows(T, H, F):
     assert torch.equal(got[0], got[1]) and not bool(got[0].isnan().any())
 
 
-@pytest.mark.parametrize("T,E,top,identities", [(1, 1, 1, 0), (300, 7, 3, 2), (2050, 1500, 8, 0), (9000, 40, 2, 8), (5000, 4096, 4, 0), (2048, 32, 4, 0), (1024, 64, 8, 1)])
+@pytest.mark.parametrize("T,E,top,identities", [(1, 1, 1, 0), (300, 7, 3, 2), (2050, 1500, 8, 0), (9000, 40, 2, 8), (5000, 4096, 4, 0), (2048, 32, 4, 0), (1024, 64, 8, 1),
+                                                (1024, 5, 1, 0), (1025, 64, 1, 2), (2048, 65, 2, 0), (2049, 63, 2, 1), (8192, 2, 2, 0)])
 def test_sorting_pairs(T, E, top, identities):
     """More pairs than the block keeps, more experts than it has threads, experts without a pair, and pairs that are not listed."""
     k, P = kernels("bfloat16"), T * top
