@@ -64,36 +64,37 @@ __device__ __forceinline__ int page_index(int p, int page_size) { return p >> (3
 __device__ __forceinline__ int page_offset(int p, int page_size) { return p & (page_size - 1); }
 
 // ============================================================================ prompt portions
-// A block takes 32 tokens of a tile and one query head and walks their blocks of
+// A block takes 64 or 32 tokens of a tile and one query head and walks their blocks of
 // positions; a block's K [64][HD] and V^T [HD][64] go through LDS, rows in the order [16 k][q][i] so that
 // a 16-byte read is a lane's operand of four products, rows a multiple of 16 bytes and an odd number
 // of them apart (16 rows fall into 16 slots of the 64 banks).  The next block's numbers are asked for
-// while this one is multiplied.  Sixteen tokens have two waves: each scores half of the positions, the scores meet in LDS, both
-// work out the weights and each sums half of the dims, so that the tokens that see most, which a prompt waits for, take half as
-// long.  grid (pairs of tiles, heads, 8): which tile of the pair and which quarter of it.
-// Bound by the tokens that see most: a wave's 128 products of 32 cycles a block of positions (head size 128) are a third of its
-// time, behind them stand the stage's writes, the exponentials and three barriers.  16 heads, us, 64 tokens a block and a wave
-// for sixteen of them / here: 777 tokens 105 / 70, three requests of 100 to 341 53 / 37, 200 tokens 36 / 23, 2,048 tokens 260 / 257
-// (67 TFLOP/s; twice the stages, no more blocks than the chip holds).
-template <int HD>
+// while this one is multiplied.  A wave has sixteen tokens, or with SHARED two waves have: each scores half of the positions, the
+// scores meet in LDS, both work out the weights and each sums half of the dims, so that the tokens that see most, which a prompt waits
+// for, take half as long.  grid (pairs of tiles, heads, 4 or 8): which tile of the pair and which part of it.
+// Bound by the tokens that see most where all blocks have a place on the chip: a wave's 128 products of 32 cycles a block of positions (head
+// size 128) are a third of its time, behind them stand the stage's writes, the exponentials and three barriers; and where blocks
+// wait for places by what they stage, which with SHARED is twice as much (launch_attention_f32_prefill).
+template <int HD, bool SHARED>
 __global__ void __launch_bounds__(256, 2)
 attention_f32_prefill_kernel(const float* __restrict__ q, int q_stride, const float* __restrict__ k_cache,
                              const float* __restrict__ v_cache, const int32_t* __restrict__ block_table, int table_stride,
                              const int32_t* __restrict__ positions, const int32_t* __restrict__ seq_rows,
                              float* __restrict__ out, const int32_t* __restrict__ tiles, int n_heads, int n_kv_heads,
                              int page_size, int window, float scale) {
-  constexpr int KG = HD / 16, DT = HD / 16, K_LD = HD + 4, V_LD = ATT_BLOCK + 4, DH = DT / 2, LOADS = ATT_BLOCK * HD / 4 / 256;
-  extern __shared__ __align__(16) float smem[];      // K [64][K_LD], V^T [HD][V_LD], the scores of the waves' tiles [4][2][64][4]
+  constexpr int KG = HD / 16, DT = HD / 16, K_LD = HD + 4, V_LD = ATT_BLOCK + 4, LOADS = ATT_BLOCK * HD / 4 / 256;
+  constexpr int WAVES = SHARED ? 2 : 1, TOKENS = 64 / WAVES, PT = 4 / WAVES, DH = DT / WAVES;      // of sixteen tokens; a block's; a wave's tiles of positions, of dims
+  constexpr int DS = DH < 4 ? DH : 4;                // tiles of dims whose numbers are read together
+  extern __shared__ __align__(16) float smem[];      // K [64][K_LD], V^T [HD][V_LD], SHARED: the scores of the waves' tiles [4][2][64][4]
   float* ks = smem;
   float* vs = smem + ATT_BLOCK * K_LD;
   f32x4* scores = reinterpret_cast<f32x4*>(vs + HD * V_LD);
-  const int32_t* mine = tiles + 4 * blockIdx.x + 2 * (blockIdx.z >> 2);
-  const int skip = 32 * (blockIdx.z & 3), count = mine[1] - skip, t0 = mine[0] + skip;
+  const int32_t* mine = tiles + 4 * blockIdx.x + 2 * (blockIdx.z / (2 * WAVES));
+  const int skip = TOKENS * (blockIdx.z % (2 * WAVES)), count = mine[1] - skip, t0 = mine[0] + skip;
   if (count <= 0) return;                            // the same for the whole block
   const int head = blockIdx.y, kvh = head / (n_heads / n_kv_heads);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r16 = lane & 15, g4 = lane >> 4;
-  const int group = wave >> 1, half = __builtin_amdgcn_readfirstlane(wave & 1), d0 = half * DH;
-  const int n = min(count, 32), first_pos = positions[t0], last_pos = positions[t0 + n - 1];
+  const int group = wave / WAVES, half = SHARED ? __builtin_amdgcn_readfirstlane(wave & 1) : 0, d0 = half * DH;
+  const int n = min(count, TOKENS), first_pos = positions[t0], last_pos = positions[t0 + n - 1];
   const bool wave_live = 16 * group < n;
   const int row = t0 + min(16 * group + r16, n - 1), pos = positions[row];
   const int lo = window > 0 ? max(0, pos + 1 - window) : 0;
@@ -156,28 +157,35 @@ attention_f32_prefill_kernel(const float* __restrict__ q, int q_stride, const fl
     const bool spoiled = whole ? (__syncthreads(), false) : __syncthreads_or(odd);
     if (b < b_end) fetch(p0 + ATT_BLOCK);
     const bool seen = p0 <= pos && p0 + ATT_BLOCK - 1 >= lo;               // by this lane's token
-    const bool works = wave_live && __any(seen);                           // the same for both waves of sixteen tokens
+    const bool works = wave_live && __any(seen);                           // the same for all waves of sixteen tokens
 
-    f32x4 s[4] = {F32_ZERO, F32_ZERO, F32_ZERO, F32_ZERO};
+    f32x4 s[4];
     if (works) {
-      f32x4 part[2] = {F32_ZERO, F32_ZERO};
+      f32x4 part[PT];
+#pragma unroll
+      for (int t = 0; t < PT; ++t) part[t] = F32_ZERO;
 #pragma unroll
       for (int g = 0; g < KG; ++g) {
-        f32x4 a[2];
+        f32x4 a[PT];
 #pragma unroll
-        for (int t = 0; t < 2; ++t) a[t] = *reinterpret_cast<const f32x4*>(&ks[(32 * half + 16 * t + r16) * K_LD + 16 * g + 4 * g4]);
+        for (int t = 0; t < PT; ++t) a[t] = *reinterpret_cast<const f32x4*>(&ks[(16 * PT * half + 16 * t + r16) * K_LD + 16 * g + 4 * g4]);
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
-          for (int t = 0; t < 2; ++t) F32_STEP(part[t], a[t], qf[g], i);
+          for (int t = 0; t < PT; ++t) F32_STEP(part[t], a[t], qf[g], i);
       }
 #pragma unroll
-      for (int t = 0; t < 2; ++t) scores[(2 * wave + t) * 64 + lane] = part[t];
+      for (int t = 0; t < PT; ++t) {
+        if (SHARED) scores[(2 * wave + t) * 64 + lane] = part[t];
+        else s[t] = part[t];
+      }
     }
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");        // the next block's loads stay under way
+    if (SHARED) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");        // the next block's loads stay under way
     if (!works) continue;
+    if (SHARED) {
 #pragma unroll
-    for (int t = 0; t < 4; ++t) s[t] = scores[(4 * group + t) * 64 + lane];
+      for (int t = 0; t < 4; ++t) s[t] = scores[(4 * group + t) * 64 + lane];
+    }
     float m_b, l_b;
     f32_weights(s, p0, lo, pos, scale, g4, m_b, l_b);
     f32x4 o[DH];
@@ -188,15 +196,17 @@ attention_f32_prefill_kernel(const float* __restrict__ q, int q_stride, const fl
 #pragma unroll
       for (int d = 0; d < DH; ++d) o[d] = F32_ZERO;
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        f32x4 a[DH];
+      for (int t = 0; t < 4; ++t)
 #pragma unroll
-        for (int d = 0; d < DH; ++d) a[d] = *reinterpret_cast<const f32x4*>(&vs[(16 * (d0 + d) + r16) * V_LD + 16 * t + 4 * g4]);
+        for (int dh = 0; dh < DH; dh += DS) {
+          f32x4 a[DS];
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+          for (int d = 0; d < DS; ++d) a[d] = *reinterpret_cast<const f32x4*>(&vs[(16 * (d0 + dh + d) + r16) * V_LD + 16 * t + 4 * g4]);
 #pragma unroll
-          for (int d = 0; d < DH; ++d) F32_STEP(o[d], a[d], pf[t], i);
-      }
+          for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int d = 0; d < DS; ++d) F32_STEP(o[dh + d], a[d], pf[t], i);
+        }
     } else {
 #pragma unroll
       for (int d = 0; d < DH; ++d) o[d] = F32_ZERO;
@@ -496,12 +506,20 @@ int launch_attention_f32_prefill(const float* q, int q_stride, const float* k_ca
                                  const int32_t* block_table, int table_stride, const int32_t* positions,
                                  const int32_t* seq_rows, float* out, const int32_t* tiles, int n_tiles, int n_heads,
                                  int n_kv_heads, int head_dim, int page_size, int window, float scale, hipStream_t stream) {
-#define LAUNCH(HD)                                                                                                   \
+  // Two waves for sixteen tokens while the chip has a place for each of their blocks, or nearly: by the most blocks of 64 tokens there can be, a
+  // CU's worth and a half at head size 128, where prompts' blocks are unequally long and the long ones go first; one at head size 64, where a block
+  // has half the products for the same stages; one and a half of them where a window makes them equally long.  us, 64 tokens a block / 32, of so
+  // many blocks of 64: head size 128, 900 tokens of 16 heads (240) 108 / 77, 1,500 (384) 208 / 172, of 28 (672) 265 / 282, 3,000 of 16 (752) 538 / 610,
+  // 8,192 of 16 3,786 / 4,732; window 300, 3,000 of 4 (192) 54 / 51, 1,300 of 16 (384) 78 / 89; head size 64, 900 of 16 heads (240) 61 / 50, 500 of
+  // 40 (320) 36 / 41, 2,048 of 16 133 / 153, window 300, 1,900 of 4 (120) 29 / 23, 2,300 (144) 29 / 32.
+  const long blocks = 4L * n_tiles * n_heads;
+  const bool shared = blocks <= (window > 0 ? (head_dim == 128 ? 256 : 128) : (head_dim == 128 ? 384 : 256));
+#define LAUNCH(HD, SHARED)                                                                                           \
   {                                                                                                                  \
-    constexpr int lds = (ATT_BLOCK * (HD + 4) + HD * (ATT_BLOCK + 4) + 4 * 2 * 64 * 4) * (int)sizeof(float);                          \
+    constexpr int lds = (ATT_BLOCK * (HD + 4) + HD * (ATT_BLOCK + 4) + (SHARED ? 4 * 2 * 64 * 4 : 0)) * (int)sizeof(float); \
     static bool configured = lds <= 48 * 1024;                                                                       \
     if (!configured) {                                                                                               \
-      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attention_f32_prefill_kernel<HD>),           \
+      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attention_f32_prefill_kernel<HD, SHARED>),   \
                                          hipFuncAttributeMaxDynamicSharedMemorySize, lds);                           \
       if (e != hipSuccess) {                                                                                         \
         axk_set_error("attention_prefill: cannot reserve %d bytes of LDS: %s", lds, hipGetErrorString(e));           \
@@ -510,11 +528,13 @@ int launch_attention_f32_prefill(const float* q, int q_stride, const float* k_ca
       configured = true;                                                                                             \
     }                                                                                                                \
     AXK_INSTANCE(INST_ATTENTION_F32_PREFILL, HD);                                                                    \
-    attention_f32_prefill_kernel<HD><<<dim3(n_tiles, n_heads, 8), 256, lds, stream>>>(                               \
+    AXK_INSTANCE(INST_ATTENTION_F32_WAVES, HD, SHARED ? 2 : 1);                                                      \
+    attention_f32_prefill_kernel<HD, SHARED><<<dim3(n_tiles, n_heads, SHARED ? 8 : 4), 256, lds, stream>>>(          \
         q, q_stride, k_cache, v_cache, block_table, table_stride, positions, seq_rows, out, tiles, n_heads,          \
         n_kv_heads, page_size, window, scale);                                                                       \
   }
-  if (head_dim == 64) LAUNCH(64) else LAUNCH(128)
+  if (head_dim == 64) { if (shared) LAUNCH(64, true) else LAUNCH(64, false) }
+  else { if (shared) LAUNCH(128, true) else LAUNCH(128, false) }
 #undef LAUNCH
   AXK_LAUNCH_CHECK("attention_prefill");
   return 0;

@@ -38,6 +38,7 @@ enum {
   INST_HEADS_PREPARE,        // 1: a block a token, 0: several
   INST_STATE_CONV,           // 1: runs of tokens, 0: a thread a (token, channel)
   INST_EMBED,                // 1: eight numbers a thread, 0: one
+  INST_ATTENTION_F32_WAVES,      // beside attention_f32_prefill: head_dim, waves for sixteen tokens
   INST_KINDS
 };
 

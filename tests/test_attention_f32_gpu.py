@@ -30,7 +30,7 @@ def _same(a, b):
 
 @pytest.mark.parametrize("nh,nkv,hd,page,T,window", [(2, 2, 64, 4, 1, 0), (4, 1, 64, 8, 65, 0), (7, 1, 128, 16, 130, 0),
                                                      (16, 1, 64, 64, 63, 40), (8, 4, 128, 128, 300, 70), (6, 2, 128, 64, 257, 64),
-                                                     (2, 1, 64, 32, 400, 0)])
+                                                     (2, 1, 64, 32, 400, 0), (64, 4, 128, 16, 330, 0), (48, 3, 64, 32, 300, 100)])
 @pytest.mark.parametrize("spoiled", [False, True])
 def test_prompts_and_decoding_have_the_bits_of_the_rows_kernel(nh, nkv, hd, page, T, window, spoiled):
     k, q, cache, sizes, want = _case(nh, nkv, hd, page, T, window, T * 2 // 3 if spoiled else None)
@@ -39,8 +39,11 @@ def test_prompts_and_decoding_have_the_bits_of_the_rows_kernel(nh, nkv, hd, page
         tiles = [(a, min(cut, T - a)) for a in range(0, T, cut)]
         pairs = [tiles[i] + (tiles[i + 1] if i + 1 < len(tiles) else (0, 0)) for i in range(0, len(tiles), 2)]
         out = torch.full_like(q, 5.0)
+        k.reset_instances()
         k.attention_prefill(q, nh * hd, *cache, out, torch.tensor(pairs, dtype=torch.int32).cuda(), *sizes)
         assert _same(out, want), cut
+        # two waves for sixteen tokens where there are few blocks
+        assert f"attention_f32_waves<{hd},{1 if nh >= 48 else 2}>" in k.instances(launched=True)
     chunks = -(-T // k.attention_decode_chunk) + 1
     partial = torch.full((k.attention_decode_workspace(T, nh, hd, chunks),), float("nan"), device="cuda")
     out = torch.full_like(q, 5.0)

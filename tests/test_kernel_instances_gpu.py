@@ -560,8 +560,12 @@ CASES = [
     *[(BF, [f"latent_prompt<{rt},{qc},0,{sink}>", f"latent_tokens<{rt},{qc},{sink}>"], check_latent, (rank, rot, sink))
       for rt, qc, rank, rot in ((4, 4, 48, 16), (8, 8, 112, 48), (32, 20, 192, 64)) for sink in (0, 1)],
     # the float32 build's attention on the matrix cores: (head size) and (head size, waves a block)
-    (F32, ["attention_f32_prefill<64>", "attention_f32_decode<64,1>"], check_attention_f32, (4, 2, 64, 16, 333, 90, 5)),
-    (F32, ["attention_f32_prefill<128>", "attention_f32_decode<128,1>"], check_attention_f32, (7, 1, 128, 64, 600, 0, 7)),
+    (F32, ["attention_f32_prefill<64>", "attention_f32_waves<64,2>", "attention_f32_decode<64,1>"], check_attention_f32, (4, 2, 64, 16, 333, 90, 5)),
+    (F32, ["attention_f32_prefill<128>", "attention_f32_waves<128,2>", "attention_f32_decode<128,1>"], check_attention_f32, (7, 1, 128, 64, 600, 0, 7)),
+    (F32, ["attention_f32_waves<64,1>"], check_attention_f32, (16, 2, 64, 16, 600, 0, 3)),             # more blocks than CUs
+    (F32, ["attention_f32_waves<64,1>"], check_attention_f32, (12, 4, 64, 16, 330, 100, 3)),
+    (F32, ["attention_f32_waves<128,1>"], check_attention_f32, (16, 1, 128, 16, 800, 0, 3)),
+    (F32, ["attention_f32_waves<128,1>"], check_attention_f32, (16, 1, 128, 16, 600, 300, 3)),
     (F32, ["attention_f32_decode<64,4>"], check_attention_f32, (8, 4, 64, 16, 140, 0, 40)),
     (F32, ["attention_f32_decode<128,4>"], check_attention_f32, (8, 4, 128, 32, 150, 60, 33)),
     # the embedding: eight numbers a thread, or one (unaligned rows, and many tokens of a packed table)
