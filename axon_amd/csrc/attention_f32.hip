@@ -400,7 +400,7 @@ __device__ __forceinline__ void f32_decode_shared(const float* __restrict__ qrow
 // once, and (o_b, m_b, l_b) of every head are left in `partial` for the fold (work list and layout as in
 // attention_mfma.hip).  BW blocks of positions a block of threads: four of a wave each, or one, which at head size 128 four waves
 // share (us with the fold, a wave alone / so: 5 tokens of 16 heads over 2 at 800 positions 15.0 / 12.4, 8 at 2,048 18.3 / 14.5, 9 of 28 over 4
-// at 4,000 44.6 / 38.2, 64 at 1,000 58 / 53; of 64, half as much to wait for: 32 over 32 at 1,500 156 / 181, 16 over 16 at 500 18.7 / 21.3).
+// at 4,000 44.6 / 38.2, 64 at 1,000 58 / 53; 16 of 16 over 16 at 500 37.8 / 33.9, at 5,000 260 / 244; of 64, half as much to wait for: 32 over 32 at 1,500 156 / 181, 16 over 16 at 500 18.7 / 21.3).
 // Bound by the wait for the pages: 8 tokens of 16 heads over
 // 2 at 777 positions 64 -> 19 us with the fold, at 2,048 144 -> 17.
 template <int HD, int BW>
@@ -430,6 +430,11 @@ attention_f32_decode_kernel(const float* __restrict__ q, int q_stride, const flo
                           chunk * (DC_CHUNK / ATT_BLOCK) + sub) * (HD + 2);
   const float* qrow = q + (size_t)t * q_stride + (size_t)(kvh * group + min(r16, group - 1)) * HD;
   if constexpr (BW == 1 && HD == 128) {
+    if (pos - p0 < 16) {                               // one tile: nothing to share (1 token of 16 heads over 2 at 12 positions, us, shared / so: 7.7 / 7.0)
+      if (wave == 0)
+        f32_decode_block<HD, 1>(qrow, k_head, v_head, table_row, page_stride, page_size, p0, lo, pos, scale, r16, g4, r16 < group, dst);
+      return;
+    }
     f32_decode_shared<HD>(qrow, k_head, v_head, table_row, page_stride, page_size, p0, lo, pos, scale, r16, g4, wave, r16 < group, dst);
   } else {
     // A context's last block often holds a few positions: 32 heads over 32, 200 tokens at 10 positions 103 us with all four
