@@ -354,7 +354,9 @@ latent_attention_mfma_kernel(const float* __restrict__ q_full, const bf16_t* __r
 // latent dims; (o, m, l) are left unscaled for the kernel that folds a token's blocks.  All that a wave reads of the page is asked
 // for before its first product: such a step is 136 blocks of eight tokens over a window of 1,024, and a wave that had the block to
 // itself waited for memory sixteen times one after the other.  The chains, their order and so the bits are those of the kernel
-// above.  16 heads, latents of 512 + 64, eight tokens at 200 to 2,500 positions over a window of 1,024: 32.3 -> 12.5 us.
+// above.  16 heads, latents of 512 + 64, eight tokens at 200 to 2,500 positions over a window of 1,024: 32.3 -> 12.5 us.  Of a smaller
+// latent only what it has is asked for, and by all four waves: 32 heads of 256 + 64, 60 tokens over a window of 1,024, us, the walk / all that the
+// instance has room for / here 54 / 70 / 49.5, 16 heads of 208 + 16 28 / 37 / 25.
 template <int RT, int QC>
 __global__ void __launch_bounds__(256)
 latent_attention_blocks_kernel(const float* __restrict__ q_full, const bf16_t* __restrict__ cache,
@@ -386,13 +388,15 @@ latent_attention_blocks_kernel(const float* __restrict__ q_full, const bf16_t* _
     qv[i][1] = *reinterpret_cast<const float4*>(src + 4);
   }
   __builtin_amdgcn_sched_barrier(0);
-  uint4 kf[QC];                                         // (chunks and tiles that the sizes lack: the last again, not used)
+  uint4 kf[QC];                                         // (chunks and tiles that the sizes lack are not asked for: the same for the wave)
 #pragma unroll
-  for (int c = 0; c < QC; ++c) kf[c] = *reinterpret_cast<const uint4*>(krow + 32 * min(c, qc - 1));
+  for (int c = 0; c < QC; ++c)
+    if (c < qc) kf[c] = *reinterpret_cast<const uint4*>(krow + 32 * c);
   uint2 v[OWN][4];
 #pragma unroll
   for (int e = 0; e < OWN; ++e) {
-    const bf16_t* vrow = vbase + (long)(16 * min(wave * OWN + e, rt - 1) + j) * page_size;
+    if (4 * e + wave >= rt) continue;                   // a wave has every fourth tile: of a small latent as many as the others
+    const bf16_t* vrow = vbase + (long)(16 * (4 * e + wave) + j) * page_size;
 #pragma unroll
     for (int c = 0; c < 4; ++c) v[e][c] = *reinterpret_cast<const uint2*>(vrow + 16 * c);
   }
@@ -451,7 +455,7 @@ latent_attention_blocks_kernel(const float* __restrict__ q_full, const bf16_t* _
     for (int c = 0; c < 2; ++c)
       acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(la_frag(make_uint4(v[e][2 * c].x, v[e][2 * c].y, v[e][2 * c + 1].x, v[e][2 * c + 1].y)),
                                                     la_frag(pf[c]), acc, 0, 0, 0);
-    const int dt = wave * OWN + e;
+    const int dt = 4 * e + wave;
     if (dt < rt) *reinterpret_cast<float2*>(dst + 16 * dt + 4 * g) = make_float2(acc[0], acc[1]),
                  *reinterpret_cast<float2*>(dst + 16 * dt + 4 * g + 2) = make_float2(acc[2], acc[3]);
   }
@@ -785,9 +789,9 @@ static void launch_latent_mfma(const float* q_full, const void* cache, const int
                                const int32_t* positions, const int32_t* seq_rows, float* o_lat, int n_tokens, int heads, int rank,
                                int rot, int page_size, int window, float scale, const float* sink, float* partial, int n_chunks,
                                bool mixed_only, hipStream_t stream) {
-  if (sink) { AXK_INSTANCE(INST_LATENT_TOKENS, RT, QC, 1); } else { AXK_INSTANCE(INST_LATENT_TOKENS, RT, QC, 0); }
   const long items = (long)n_tokens * (heads / 16);
   if (partial) {
+    AXK_INSTANCE(INST_LATENT_BLOCKS, RT, QC);
     latent_attention_blocks_kernel<RT, QC><<<dim3((unsigned)items, n_chunks), 256, 0, stream>>>(
         q_full, (const bf16_t*)cache, block_table, table_stride, positions, seq_rows, heads, rank, rot, page_size, window, scale, partial,
         n_chunks);
@@ -795,6 +799,7 @@ static void launch_latent_mfma(const float* q_full, const void* cache, const int
         partial, o_lat, rank, n_chunks, sink, heads);
     return;
   }
+  if (sink) { AXK_INSTANCE(INST_LATENT_TOKENS, RT, QC, 1); } else { AXK_INSTANCE(INST_LATENT_TOKENS, RT, QC, 0); }
   const unsigned grid = (unsigned)((items + LAM_WAVES - 1) / LAM_WAVES);
   if (sink)
     latent_attention_mfma_kernel<RT, QC, true><<<grid, LAM_WAVES * 64, 0, stream>>>(

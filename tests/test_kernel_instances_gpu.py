@@ -355,7 +355,13 @@ def check_latent(rank, rot, sink):
     w = torch.exp(s - m)
     want = torch.matmul(w, val) / (w.sum(-1, keepdim=True) + (0 if sinks is None else torch.exp(sinks.double()[:, None, None] - m)))
     # the weights are rounded to 8 bits: each off by at most 2^-9 of itself
-    assert float((got["out"].view(T, heads, rank).transpose(0, 1).double() - want).abs().max()) <= 2.0 ** -8 * float(val.abs().max())
+    bound = 2.0 ** -8 * float(val.abs().max())
+    assert float((got["out"].view(T, heads, rank).transpose(0, 1).double() - want).abs().max()) <= bound
+    few = torch.full((3, heads * rank), float("nan"), device="cuda")              # the last tokens' blocks of positions side by side
+    rows = torch.zeros(3, dtype=torch.int32, device="cuda")
+    hit |= launched(k, "bfloat16", lambda: k.latent_attention(q[T - 3:], cache, table, pos[T - 3:], rows, few, heads, rank, rot, page, 0, scale,
+                                                              sink=sinks, span=T))
+    assert float((few.view(3, heads, rank).transpose(0, 1).double() - want[:, T - 3:]).abs().max()) <= bound
     return hit
 
 
@@ -554,11 +560,11 @@ CASES = [
     (F32, ["causal_conv<0>"], check_conv, (F32, 1023, 260)),
     (F32, ["causal_conv<1>"], check_conv, (F32, 2049, 640)),
     # latent attention: many tokens by (tiles of 16 latent dims, chunks of 32 key dims, bounds known when compiled, sink), and
-    # the kernel of a wave a token
+    # the kernels of a wave a token and of its blocks side by side
     *[(BF, [f"latent_prompt<{rt},{qc},1,{sink}>"], check_latent, (16 * rt, 32 * qc - 16 * rt, sink))
       for rt, qcs in ((32, (17, 18, 20)), (16, (9, 10, 12)), (8, (5, 6, 8)), (4, (3, 4, 6))) for qc in qcs for sink in (0, 1)],
-    *[(BF, [f"latent_prompt<{rt},{qc},0,{sink}>", f"latent_tokens<{rt},{qc},{sink}>"], check_latent, (rank, rot, sink))
-      for rt, qc, rank, rot in ((4, 4, 48, 16), (8, 8, 112, 48), (32, 20, 192, 64)) for sink in (0, 1)],
+    *[(BF, [f"latent_prompt<{rt},{qc},0,{sink}>", f"latent_tokens<{rt},{qc},{sink}>", f"latent_blocks<{rt},{qc}>"], check_latent,
+       (rank, rot, sink)) for rt, qc, rank, rot in ((4, 4, 48, 16), (8, 8, 112, 48), (32, 20, 192, 64)) for sink in (0, 1)],
     # the float32 build's attention on the matrix cores: (head size) and (head size, waves a block)
     (F32, ["attention_f32_prefill<64>", "attention_f32_waves<64,2>", "attention_f32_decode<64,1>"], check_attention_f32, (4, 2, 64, 16, 333, 90, 5)),
     (F32, ["attention_f32_prefill<128>", "attention_f32_waves<128,2>", "attention_f32_decode<128,1>"], check_attention_f32, (7, 1, 128, 64, 600, 0, 7)),
