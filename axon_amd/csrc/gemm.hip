@@ -735,12 +735,17 @@ static void launch_fma_few(const elem_t* x, int x_stride, const elem_t* w, const
 // columns and gated 5,632 at 129 to 2,048 rows, all within 5 % of it; of 32 rows the first three blocks take 5 more).  64 rows of all / so, K 2,048: 2,048
 // columns, 129 and 200 rows 47 / 30, 300 48 / 40, 626 76 / 56, 1,500 118 / 105; 2,560 columns, 430 rows 76 / 56, 777 117 / 84, 1,024
 // 117 / 101; gated 5,632, 129 rows 117 / 86, 900 405 / 367, 1,500 620 / 570.  Blocks of 112 and of 128 rows, one a CU, are the best of none.
-static int flow_rows(int columns, int m, bool glu) {
+// With K the other heights' times grow faster than those of 64 rows, gated 96 excepted, by one in 80,000 k (each height at 14 shapes and K 256
+// to 14,336: so chosen 0.916 of the time with 64 rows for all, 1.005 of the best height's, none over 2 % longer than with 64; without that up to 22 %:
+// 900 rows of 4,096 of K 11,008 759 / 865 with 80, gated 512 of 5,632 1,158 / 1,305 with 32).
+static int flow_rows(int columns, int m, int k, bool glu) {
   int best = 0;
   double least = 0.0;
+  const double dear = 1.0 + (k > 1024 ? (k - 1024) / 80000.0 : 0.0);
   auto is = [&](int rows, double alone, double each, double odd) {
     const long blocks = ((long)columns * ceil_div(m, rows) + 255) / 256;
-    const double cost = blocks == 1 ? alone : blocks * each + (blocks % 2 ? odd : 0.0) + (rows == 32 && blocks <= 3 ? 5.0 : 0.0);
+    double cost = blocks == 1 ? alone : blocks * each + (blocks % 2 ? odd : 0.0) + (rows == 32 && blocks <= 3 ? 5.0 : 0.0);
+    if (rows != 64 && !(glu && rows == 96)) cost *= dear;
     if (best == 0 || cost < least) {
       best = rows;
       least = cost;
@@ -770,6 +775,7 @@ static int launch_flow(unsigned columns, const float* x, int x_stride, const flo
     }
     configured = true;
   }
+  AXK_INSTANCE(INST_GEMM_FMA_FLOW_ROWS, rows, GLU);
   kernel<<<dim3(columns, ceil_div(m, rows)), 256, lds, stream>>>(x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode);
   return 0;
 }
@@ -787,7 +793,7 @@ static int launch_fma_tiles(dim3 tiles, const elem_t* x, int x_stride, const ele
     if (k >= ((long)tiles.x * tiles.y <= 512 ? FLOW_LEAST_K : 640)) {
       AXK_INSTANCE(INST_GEMM_FMA_FLOW, GLU);
 #define FLOW(WAVES_M, TM, TN) return launch_flow<GLU, WAVES_M, TM, TN>(tiles.x, x, x_stride, w, bias, bias_is_f32, out, out_stride, m, n, k, mode, stream)
-      const int rows = flow_rows(tiles.x, m, GLU);
+      const int rows = flow_rows(tiles.x, m, k, GLU);
       if (rows == 32) FLOW(2, 1, 2);
       if (rows == 96) FLOW(2, 3, 2);
       if constexpr (!GLU) {

@@ -40,6 +40,7 @@ enum {
   INST_EMBED,                // 1: eight numbers a thread, 0: one
   INST_ATTENTION_F32_WAVES,      // beside attention_f32_prefill: head_dim, waves for sixteen tokens
   INST_LATENT_BLOCKS,        // tiles of 16 latent dims, chunks of 32 key dims: blocks of positions side by side
+  INST_GEMM_FMA_FLOW_ROWS,   // beside gemm_fma_flow: rows a block; gated
   INST_KINDS
 };
 

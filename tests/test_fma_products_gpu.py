@@ -166,9 +166,10 @@ def test_direct_loads_at_every_end_of_k(K):
     assert {"gemm_fma_flow<0>", "gemm_fma_flow<1>"} <= set(k.instances(launched=True))
 
 
-@pytest.mark.parametrize("M,N,K", [(129, 2048, 644), (97, 2560, 512), (300, 2050, 192), (626, 2048, 228), (777, 2560, 644), (1500, 2048, 640),
-                                   (64, 8200, 516), (65, 4100, 512), (1025, 1000, 196)])
-def test_rows_a_block_by_what_the_cus_get(M, N, K):
+@pytest.mark.parametrize("M,N,K,rows,gated", [(129, 2048, 644, 32, 32), (97, 2560, 512, 32, None), (300, 2050, 192, 48, 32), (626, 2048, 228, 80, 96),
+                                              (777, 2560, 644, 32, 32), (1500, 2048, 640, 96, 96), (64, 8200, 516, 32, 32), (65, 4100, 512, 32, 32),
+                                              (1025, 1000, 196, 80, 96), (896, 2048, 644, 64, 64), (777, 11264, 644, 80, 64)])
+def test_rows_a_block_by_what_the_cus_get(M, N, K, rows, gated):
     """Tiles of 32, 48, 64, 80 and 96 rows, the last ones of a product among them: the bits of chains of fmaf."""
     k = kernels("float32")
     g = torch.Generator(device="cuda").manual_seed(M + N)
@@ -176,11 +177,30 @@ def test_rows_a_block_by_what_the_cus_get(M, N, K):
     out = torch.full((M + 1, N), float("nan"), device="cuda")
     k.reset_instances()
     k.gemm(x, w, out[:M], None, MODE_STORE_F32)
-    assert "gemm_fma_flow<0>" in k.instances(launched=True)
+    assert {"gemm_fma_flow<0>", f"gemm_fma_flow_rows<{rows},0>"} <= set(k.instances(launched=True))
     want = _by_chains(k, x, w)
     assert torch.equal(out[:M], want) and bool(out[M:].isnan().all())
     half = N // 2
     got, act = (torch.full((M, half), float("nan"), device="cuda") for _ in range(2))
     k.gemm(x, w[:2 * half], got, None, MODE_SWIGLU)
+    assert gated is None or f"gemm_fma_flow_rows<{gated},1>" in k.instances(launched=True)         # (None: too few outputs for tiles)
     k.swiglu(want[:, :2 * half].contiguous(), act)
     assert torch.equal(got, act)
+
+
+@pytest.mark.parametrize("M,N,least,rows,gated", [(129, 2048, 192, 32, 32), (300, 2050, 192, 48, 32), (896, 2048, 192, 64, 64), (626, 2048, 192, 80, 96),
+                                                  (1500, 2048, 640, 96, 96)])
+def test_every_height_at_every_end_of_k(M, N, least, rows, gated):
+    """Whole and broken last steps, an odd and an even number of them."""
+    k = kernels("float32")
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    for K in range(least, least + 68, 4):
+        x, w = torch.randn(M, K, generator=g, device="cuda"), torch.randn(N, K, generator=g, device="cuda")
+        out, act, got = (torch.full((M, n), float("nan"), device="cuda") for n in (N, N // 2, N // 2))
+        k.reset_instances()
+        k.gemm(x, w, out, None, MODE_STORE_F32)
+        k.gemm(x, w[:N // 2 * 2], got, None, MODE_SWIGLU)
+        assert {f"gemm_fma_flow_rows<{rows},0>", f"gemm_fma_flow_rows<{gated},1>"} <= set(k.instances(launched=True))
+        want = _by_chains(k, x, w)
+        k.swiglu(want[:, :N // 2 * 2].contiguous(), act)
+        assert torch.equal(out, want) and torch.equal(got, act), K

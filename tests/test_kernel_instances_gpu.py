@@ -400,6 +400,10 @@ CASES = [
                                   (32, 31, 48, 100, MODE_SWIGLU), (128, 129, 48, 100, MODE_SWIGLU), (64, 128, 96, 290, MODE_SWIGLU))],
     (F32, ["gemm_fma_flow<0>"], check_gemm, (F32, 200, 259, 260, MODE_STORE_F32)),
     (F32, ["gemm_fma_flow<1>"], check_gemm, (F32, 129, 48, 292, MODE_SWIGLU)),
+    *[(F32, [f"gemm_fma_flow_rows<{rows},0>"], check_gemm, (F32, M, N, K, MODE_STORE_F32))
+      for rows, M, N, K in ((32, 129, 2048, 260), (48, 300, 2050, 228), (64, 896, 2048, 292), (80, 626, 2048, 228), (96, 1500, 2048, 644))],
+    *[(F32, [f"gemm_fma_flow_rows<{rows},1>"], check_gemm, (F32, M, 1024, K, MODE_SWIGLU))
+      for rows, M, K in ((32, 129, 260), (64, 896, 292), (96, 626, 228))],
     # chain by chain: fewer chains than waves, and numbers loaded singly but for one tile of rows and W
     *[(d, [f"gemm_fma_by_chain<{rows},{int(mode == MODE_SWIGLU)},{int(K % 4 == 0)}>"], check_gemm, (d, M, N, K, mode)) for d in (F32, BF)
       for rows, M in ((16, 5), (32, 20), (64, 70)) for N, K, mode in ((259, 100, MODE_STORE_F32), (259, 70, MODE_STORE_F32), (48, 96, MODE_SWIGLU),
