@@ -41,6 +41,7 @@ enum {
   INST_ATTENTION_F32_WAVES,      // beside attention_f32_prefill: head_dim, waves for sixteen tokens
   INST_LATENT_BLOCKS,        // tiles of 16 latent dims, chunks of 32 key dims: blocks of positions side by side
   INST_GEMM_FMA_FLOW_ROWS,   // beside gemm_fma_flow: rows a block; gated
+  INST_GATED_SCAN,           // 1: waves that feed the walk, 0: a thread a channel
   INST_KINDS
 };
 

@@ -18,7 +18,7 @@ const char* const KIND_NAMES[INST_KINDS] = {"gemm_fma", "gemm_tile", "gemm_strea
                                             "attention_decode", "rmsnorm", "grouped_gemm", "causal_conv",
                                             "latent_prompt", "latent_tokens", "gemm_kept", "attention_f32_prefill",
                                             "attention_f32_decode", "gemm_fma_by_chain", "gemm_fma_flow", "heads_prepare",
-                                            "state_conv", "embed", "attention_f32_waves", "latent_blocks", "gemm_fma_flow_rows"};
+                                            "state_conv", "embed", "attention_f32_waves", "latent_blocks", "gemm_fma_flow_rows", "gated_scan"};
 
 struct Registry {
   std::mutex lock;

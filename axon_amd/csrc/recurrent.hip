@@ -191,7 +191,8 @@ __global__ void gated_scan_kernel(const float* __restrict__ gates, const float* 
 // Tokens that the feeding threads have side by side: four at a time, since the walk reads four.
 __host__ __device__ inline int scan_rows(int width) { return SCAN_FEEDERS / width / 4 * 4; }
 // Channels a block has: of a lone request as many as give every CU a block, 16 of each of several, 64 of those that are short
-// (the blocks that are too many then leave at once).  us by width, 2,560 channels: 2,048 tokens of a request 53.5 with 8, 46.8 with
+// (the blocks that are too many then leave at once, or are not launched where `longest` says so; requests take their first channels to the
+// XCDs in turn: 100 requests of 64 tokens of 64 channels, all on one XCD, 25.8 us, so 13.4).  us by width, 2,560 channels: 2,048 tokens of a request 53.5 with 8, 46.8 with
 // 10, 50.0 with 16, 91.9 with 32 (5,120 channels 64.1 with 10, 67.1 with 20, 79.1 with 16); requests of 1,000, 700 and 400 38.9 with 10, 35.7 with
 // 16, 48.5 with 32; five of 300 39.8, 33.8, 28.7, and 31.7 with 64; 64 of 32 tokens 93.0 with 16, 39.7 with 64.
 #define SCAN_SHORT 128
@@ -213,8 +214,8 @@ gated_scan_stretch_kernel(const float* __restrict__ gates, const float* __restri
   __shared__ __align__(16) float as[2][SCAN_FLOATS], bs[2][SCAN_FLOATS], ss[2][SCAN_FLOATS];
   const int slot = spans[3 * blockIdx.y], first = spans[3 * blockIdx.y + 1], count = spans[3 * blockIdx.y + 2];
   if (gridDim.y > 1 && count <= SCAN_SHORT) width = SCAN_WIDEST;
-  // neighbouring channels on one XCD: their rows share cache lines
-  const int per_xcd = ((channels + width - 1) / width + 7) / 8, c0 = ((blockIdx.x % 8) * per_xcd + blockIdx.x / 8) * width;
+  // neighbouring channels on one XCD: their rows share cache lines; the requests' first ones on all in turn
+  const int per_xcd = ((channels + width - 1) / width + 7) / 8, c0 = ((blockIdx.x + blockIdx.y) % 8 * per_xcd + blockIdx.x / 8) * width;
   if ((int)blockIdx.x / 8 >= per_xcd || c0 >= channels || count <= 0) return;
   const int rows = scan_rows(width), chunk = SCAN_EACH * rows, pitch = chunk + 4, chunks = (count + chunk - 1) / chunk;
   if (threadIdx.x >= SCAN_FEEDERS) {
@@ -357,6 +358,7 @@ extern "C" int axk_gated_scan(const float* gates, const float* u, const void* y,
   AXK_REQUIRE((spans != nullptr || seq_rows != nullptr) && positions != nullptr, "gated_scan: neither spans nor slots, or no positions");
   AXK_REQUIRE(n_spans <= 65535, "gated_scan: %d requests in one step (at most 65535)", n_spans);
   if (n_spans == 0) return 0;
+  AXK_INSTANCE(INST_GATED_SCAN, 0);
   dim3 grid(ceil_div(channels, 64), n_spans);
   gated_scan_kernel<<<grid, 64, 0, (hipStream_t)stream>>>(gates, u, (const elem_t*)y, y_stride, (const elem_t*)x, x_stride, lam,
                                                          lam_is_f32, decay, state, state_stride, spans, positions,
@@ -368,7 +370,7 @@ extern "C" int axk_gated_scan(const float* gates, const float* u, const void* y,
 extern "C" int axk_gated_scan_stretches(const float* gates, const float* u, const void* y, long y_stride, const void* x, long x_stride,
                                         const void* lam, int lam_is_f32, float decay, float* state, long state_stride,
                                         const int32_t* spans, int n_spans, const int32_t* positions, void* out, int channels,
-                                        int block_width, int taps, void* stream) {
+                                        int block_width, int taps, int longest, void* stream) {
   AXK_REQUIRE(n_spans >= 0 && channels > 0 && block_width > 0 && channels % block_width == 0 && taps >= 1,
               "gated_scan: bad sizes spans=%d channels=%d block width=%d taps=%d", n_spans, channels, block_width, taps);
   AXK_REQUIRE(state_stride >= 2L * taps * channels, "gated_scan: a state row of %ld floats does not hold 2 x %d x %d",
@@ -376,7 +378,9 @@ extern "C" int axk_gated_scan_stretches(const float* gates, const float* u, cons
   AXK_REQUIRE(spans != nullptr && positions != nullptr, "gated_scan: no spans or no positions");
   AXK_REQUIRE(n_spans <= 65535, "gated_scan: %d requests in one step (at most 65535)", n_spans);
   if (n_spans == 0) return 0;
-  const int width = scan_width(channels, n_spans);
+  // several requests that are known to be short: no more blocks than have work
+  const int width = n_spans > 1 && longest > 0 && longest <= SCAN_SHORT ? SCAN_WIDEST : scan_width(channels, n_spans);
+  AXK_INSTANCE(INST_GATED_SCAN, 1);
   const dim3 grid(8 * ceil_div(ceil_div(channels, width), 8), n_spans);
   gated_scan_stretch_kernel<<<grid, SCAN_FEEDERS + AXON_WAVE, 0, (hipStream_t)stream>>>(
       gates, u, (const elem_t*)y, y_stride, (const elem_t*)x, x_stride, lam, lam_is_f32, decay, state, state_stride, spans, positions,

@@ -121,7 +121,7 @@ _SIGNATURES = {
     "axk_gated_scan": [c_void_p, c_void_p, c_void_p, c_long, c_void_p, c_long, c_void_p, c_int, c_float, c_void_p, c_long,
                        c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p],
     "axk_gated_scan_stretches": [c_void_p, c_void_p, c_void_p, c_long, c_void_p, c_long, c_void_p, c_int, c_float, c_void_p, c_long,
-                                 c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p],
+                                 c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p],
     "axk_state_conv": [c_void_p, c_long, c_void_p, c_void_p, c_int, c_int, c_void_p, c_long, c_long, c_long, c_void_p, c_void_p,
                        c_void_p, c_int, c_int, c_int, c_void_p, c_long, c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p],
     "axk_state_space_scan": [c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_long, c_long, c_long, c_void_p, c_int, c_void_p,
@@ -1087,31 +1087,53 @@ class Kernels:
                                              w.shape[1], _queue()))
         return u
 
-    def gated_scan(self, gates, u, y, x, lam, decay: float, state, spans, positions, seq_rows, out, block_width: int, taps: int):
+    @staticmethod
+    def scan_groups(lengths: Sequence[int], channels: int) -> List[tuple]:
+        """Which of a step's requests, longest first, have which kernel of the gated scan: (first, end, the longest's tokens, or 0: a
+        thread a channel).  Requests of more than 128 tokens have a kernel whose blocks hold few channels; shorter ones, which would
+        leave most of its blocks without work, 64 a block; and the shortest a thread a channel, which takes 0.45 us a token and no
+        more the more channels there are: up to 8 tokens, 16 if they are a quarter of a wave a SIMD, all if they are one.  us, fed / a
+        thread a channel: 64 requests of 32 tokens of 2,560 channels 61 / 32, 16 of 16 14.7 / 10.5, 16 of 8 13.8 / 6.6, 4 of 16 of 1,024
+        5.2 / 9.6, 300 of 5 of 512 81 / 7.9, 100 of 64 72 / 45."""
+        limit = 128 if sum(16 < n <= 128 for n in lengths) * channels >= 65536 else 16 if sum(8 < n <= 16 for n in lengths) * channels >= 16384 else 8
+        long = next((i for i, n in enumerate(lengths) if n <= 128), len(lengths))
+        fed = next((i for i, n in enumerate(lengths) if n <= limit), len(lengths))
+        cuts = [(0, long, lengths[0]), (long, fed, lengths[long] if long < fed else 0), (fed, len(lengths), 0)]
+        return [g for g in cuts if g[0] < g[1]]
+
+    def gated_scan(self, gates, u, y, x, lam, decay: float, state, spans, positions, seq_rows, out, block_width: int, taps: int,
+                   lengths: Optional[Sequence[int]] = None):
         """The gated linear recurrence over each request's tokens (see csrc/recurrent.hip): gates
         [T, C / block_width, 2 block_width] and u [T, C] float32; y, x [T, C] compute dtype (rows may be
         strided); state float32 [slots, >= 2 taps C]; spans int32 [n, 3] = (slot, first token, tokens) or
-        None (each token a request of its own in slot seq_rows[t]); out [T, C] compute dtype."""
+        None (each token a request of its own in slot seq_rows[t]); out [T, C] compute dtype.  `lengths`: the spans' tokens on the
+        host, where the spans are given longest first; each then has the kernel for its length."""
         self._f32(gates, "scan gates"); self._f32(u, "scan u"); self._elem(y, "scan y"); self._elem(x, "scan x")
         self._f32(state, "scan state"); self._elem(out, "scan out"); self._i32(seq_rows, "seq_rows"); self._i32(positions, "positions")
         T, C = u.shape
         if (gates.shape != (T, 2 * C) and gates.numel() != T * 2 * C) or y.shape != (T, C) or x.shape != (T, C) or out.shape != (T, C) \
                 or y.stride(1) != 1 or x.stride(1) != 1 or not out.is_contiguous() or lam.numel() != C or seq_rows.numel() != T:
             raise KernelError(f"gated_scan: gates {tuple(gates.shape)}, u {tuple(u.shape)}, y {tuple(y.shape)}, out {tuple(out.shape)}")
+        shared = (_ptr(gates), _ptr(u), _ptr(y), y.stride(0), _ptr(x), x.stride(0), _ptr(lam), self._vec_flag(lam, "scan lam"), float(decay),
+                  _ptr(state), state.stride(0))
         n = T
         if spans is not None:
             self._i32(spans, "scan spans")
             n = spans.shape[0]
-            if T > 4 * n:            # stretches of tokens
-                self._check(self.run.axk_gated_scan_stretches(
-                    _ptr(gates), _ptr(u), _ptr(y), y.stride(0), _ptr(x), x.stride(0), _ptr(lam), self._vec_flag(lam, "scan lam"),
-                    float(decay), _ptr(state), state.stride(0), _ptr(spans), n, _ptr(positions), _ptr(out), C, int(block_width),
-                    int(taps), _queue()))
-                return out
-        self._check(self.run.axk_gated_scan(_ptr(gates), _ptr(u), _ptr(y), y.stride(0), _ptr(x), x.stride(0), _ptr(lam),
-                                            self._vec_flag(lam, "scan lam"), float(decay), _ptr(state), state.stride(0),
-                                            _ptr(spans), n, _ptr(positions), _ptr(seq_rows), _ptr(out), C, int(block_width),
-                                            int(taps), _queue()))
+        if spans is None or lengths is None:
+            groups = [(0, n, 1 if spans is not None and T > 4 * n else 0)] if n else []
+        elif len(lengths) != n or any(a < b for a, b in zip(lengths, lengths[1:])):
+            raise KernelError(f"gated_scan: {len(lengths)} lengths for {n} spans, or not the longest first")
+        else:
+            groups = self.scan_groups(lengths, C)
+        for first, end, longest in groups:
+            at = None if spans is None else _ptr(spans) + 12 * first
+            if longest:              # stretches of tokens
+                self._check(self.run.axk_gated_scan_stretches(*shared, at, end - first, _ptr(positions), _ptr(out), C, int(block_width), int(taps),
+                                                              0 if lengths is None else int(longest), _queue()))
+            else:
+                self._check(self.run.axk_gated_scan(*shared, at, end - first, _ptr(positions), _ptr(seq_rows), _ptr(out), C, int(block_width),
+                                                    int(taps), _queue()))
         return out
 
     # ------------------------------------------------------------------ a state-space mixer with per-request state

@@ -38,6 +38,17 @@ def step_spans(ctx) -> Optional[torch.Tensor]:
     return spans
 
 
+def longest_first(ctx):
+    """The same spans, longest first, and their tokens on the host; (None, None) in a step of single tokens."""
+    if ctx.decode_only:
+        return None, None
+    made = ctx.shared.get("longest_spans")
+    if made is None:
+        rows = sorted(([s.slot, s.q_start, s.q_len] for s in ctx.spans), key=lambda r: -r[2])
+        made = ctx.shared["longest_spans"] = (upload(rows, ctx.rt.device), [r[2] for r in rows])
+    return made
+
+
 class GatedRecurrence(Mixer):
     graph_safe = True
     stores_output = True
@@ -98,8 +109,8 @@ class GatedRecurrence(Mixer):
         gates = ctx.ws.take((T, 2 * C), torch.float32)
         k.grouped_gemm(u, self.w_gates, gates, x_group_stride=self.bw, out_group_stride=2 * self.bw, bias=self.b_gates)
         mixed = ctx.ws.take((T, C), ctx.rt.dtype)
-        k.gated_scan(gates, u, y, x, self.lam, self.decay, state, step_spans(ctx), ctx.positions, ctx.seq_rows, mixed, self.bw,
-                     self.taps)
+        spans, lengths = longest_first(ctx)
+        k.gated_scan(gates, u, y, x, self.lam, self.decay, state, spans, ctx.positions, ctx.seq_rows, mixed, self.bw, self.taps, lengths)
         k.gemm(mixed, self.w_o, out, None, MODE_ADD_F32 if accumulate else MODE_STORE_F32)
 
 

@@ -307,6 +307,28 @@ def check_embed(dtype, T, dim, packed):
     return hit
 
 
+def check_gated_scan(dtype, T):
+    """The gated recurrence of one request against a loop of float64."""
+    k, C, taps = kernels(dtype), 24, 3
+    td = getattr(torch, dtype)
+    gates, u = rnd(T, 2 * C, seed=1, device="cuda"), rnd(T, C, seed=2, device="cuda")
+    y, x = (rnd(T, C, seed=n, device="cuda").to(td) for n in (3, 4))
+    lam, state = rnd(C, seed=5, device="cuda"), rnd(1, 2 * taps * C, seed=6, device="cuda")
+    pos, out = torch.arange(T, dtype=torch.int32, device="cuda"), torch.empty(T, C, dtype=td, device="cuda")
+    spans, before = torch.tensor([[0, 0, T]], dtype=torch.int32, device="cuda"), state[0, taps * C:].double().cpu()      # behind position -1
+    hit = launched(k, dtype, lambda: k.gated_scan(gates, u, y, x, lam, 8.0, state, spans, pos, torch.zeros_like(pos), out, C, taps))
+    g, U, Y, L = gates.double().cpu(), u.double().cpu(), y.double().cpu(), lam.double().cpu()
+    S, want = before[:C].clone(), []
+    for t in range(T):
+        log_a = -8.0 * torch.sigmoid(g[t, :C]) * torch.nn.functional.softplus(L)
+        S = torch.exp(log_a) * S + torch.sqrt(-torch.expm1(2 * log_a)) * torch.sigmoid(g[t, C:]) * U[t]
+        want.append(S * torch.nn.functional.gelu(Y[t], approximate="tanh"))
+    want = torch.stack(want)
+    limit = 1e-2 if dtype == "bfloat16" else 2e-5
+    assert float((out.double().cpu() - want).abs().max()) <= limit * max(1.0, float(want.abs().max()))
+    return hit
+
+
 # (names of the instances the case is meant to select, the check, its arguments)
 BF, F32 = "bfloat16", "float32"
 def check_grouped(dtype, M, G, N, K, glu):
@@ -578,6 +600,8 @@ CASES = [
     (F32, ["attention_f32_waves<128,1>"], check_attention_f32, (16, 1, 128, 16, 600, 300, 3)),
     (F32, ["attention_f32_decode<64,4>"], check_attention_f32, (8, 4, 64, 16, 140, 0, 40)),
     (F32, ["attention_f32_decode<128,4>"], check_attention_f32, (8, 4, 128, 32, 150, 60, 33)),
+    # the gated recurrence: a thread a channel, or waves that feed the walk
+    *[(dtype, [f"gated_scan<{int(T > 4)}>"], check_gated_scan, (dtype, T)) for dtype in (BF, F32) for T in (4, 77)],
     # the embedding: eight numbers a thread, or one (unaligned rows, and many tokens of a packed table)
     *[(dtype, [f"embed<{eights}>"], check_embed, (dtype, T, dim, False)) for dtype in (BF, F32) for T, dim, eights in ((5, 40, 1), (3, 35, 0), (1030, 64, 1))],
     *[(BF, [f"embed<{int(T < 1024)}>"], check_embed, (BF, T, dim, True)) for T, dim in ((1023, 64), (1024, 64), (1100, 192), (7, 2112))],

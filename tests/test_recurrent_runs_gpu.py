@@ -91,3 +91,33 @@ def test_long_walk_by_width(dtype, lengths, channels):
     assert k.lib.axk_gated_scan(_ptr(gates), _ptr(u), _ptr(yx), 2 * C, _ptr(yx[:, C:]), 2 * C, _ptr(lam), 1, 8.0, _ptr(kept), kept.stride(0),
                                 _ptr(spans), len(lengths), _ptr(pos), _ptr(seq), _ptr(want), C, width, taps, _stream()) == 0
     assert torch.equal(got, want) and torch.equal(state, kept)
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
+@pytest.mark.parametrize("lengths, channels, kernels_run", [([300, 129, 128, 40, 17, 16, 9, 8, 1], 512, {0, 1}), ([64] * 3 + [1] * 30, 64, {0, 1}),
+                                                            ([8, 5, 5], 192, {0}), ([128] * 40, 2048, {0}), ([200, 150], 2560, {1}),
+                                                            ([16] * 20 + [9] * 5, 2560, {0}), ([100, 17], 960, {1})])
+def test_requests_of_every_length_have_their_kernel(dtype, lengths, channels, kernels_run):
+    """Longest first, with their lengths on the host: the bits of a thread a channel, whichever kernels ran."""
+    from axon_amd.kernels import kernels
+    from axon_amd.kernels.lib import KernelError, _ptr, _stream
+    k, dev, C, width, taps = kernels(dtype), "cuda:0", channels, channels // 2, 4
+    elem = getattr(torch, dtype)
+    torch.manual_seed(7)
+    seq, pos, spans = _rows(lengths, dev)
+    T = sum(lengths)
+    gates, u = torch.randn(T, 2 * C, device=dev), torch.randn(T, C, device=dev)
+    y, x = (torch.randn(T, C, device=dev).to(elem) for _ in range(2))
+    lam = torch.rand(C, device=dev)
+    state = torch.randn(len(lengths), 2 * taps * C, device=dev)
+    kept = state.clone()
+    got, want = (torch.full((T, C), float("nan"), dtype=elem, device=dev) for _ in range(2))
+    k.reset_instances()
+    k.gated_scan(gates, u, y, x, lam, 8.0, state, spans, pos, seq, got, width, taps, lengths)
+    assert {f"gated_scan<{i}>" for i in kernels_run} == set(k.instances(launched=True))
+    assert k.lib.axk_gated_scan(_ptr(gates), _ptr(u), _ptr(y), C, _ptr(x), C, _ptr(lam), 1, 8.0, _ptr(kept), kept.stride(0),
+                                _ptr(spans), len(lengths), _ptr(pos), _ptr(seq), _ptr(want), C, width, taps, _stream()) == 0
+    assert torch.equal(got, want) and torch.equal(state, kept)
+    for wrong in (lengths[:-1], lengths[::-1] if lengths[0] != lengths[-1] else lengths + [1]):
+        with pytest.raises(KernelError, match="lengths"):
+            k.gated_scan(gates, u, y, x, lam, 8.0, state, spans, pos, seq, got, width, taps, wrong)
