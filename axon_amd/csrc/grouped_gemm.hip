@@ -518,7 +518,7 @@ int launch_wide(const GroupedArgs& a, dim3 grid, hipStream_t s) {
     }
     configured = true;
   }
-  AXK_INSTANCE(INST_GROUPED_GEMM, 2, 1);
+  AXK_INSTANCE(INST_GROUPED_GEMM, 5, 1);
   grouped_gemm_wide_kernel<<<grid, 512, lds, s>>>(a);
   return 0;
 }

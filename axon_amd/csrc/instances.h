@@ -26,7 +26,7 @@ enum {
   INST_ATTENTION_PREFILL,    // head_dim, query heads a block, pages of 64 positions or more
   INST_ATTENTION_DECODE,     // head_dim, waves a block
   INST_RMSNORM,              // 1: rows read as float4
-  INST_GROUPED_GEMM,         // 2, 3: matrix cores through LDS, 256 (tiles of 64 or 128 rows) and 128 rows of W a block, 1, 4: from memory, a long and a short K, 0: 32-bit FMA; gated epilogue
+  INST_GROUPED_GEMM,         // 2, 3: matrix cores through LDS, 256 and 128 rows of W a block, 5: 256 by tiles of 128 rows, 1, 4: from memory, a long and a short K, 0: 32-bit FMA; gated epilogue
   INST_CAUSAL_CONV,          // 1: runs of tokens, 0: a thread a (token, channel)
   INST_LATENT_PROMPT,        // tiles of 16 latent dims, chunks of 32 key dims, bounds known when compiled, sink
   INST_LATENT_TOKENS,        // tiles of 16 latent dims, chunks of 32 key dims, sink
@@ -42,6 +42,8 @@ enum {
   INST_LATENT_BLOCKS,        // tiles of 16 latent dims, chunks of 32 key dims: blocks of positions side by side
   INST_GEMM_FMA_FLOW_ROWS,   // beside gemm_fma_flow: rows a block; gated
   INST_GATED_SCAN,           // 1: waves that feed the walk, 0: a thread a channel
+  INST_MASKED_BLOCKS,        // maps, tiles of 16 value dims, chunks of 32 key dims: blocks of positions side by side
+  INST_MASKED_FOLD,          // maps, value dims a lane
   INST_KINDS
 };
 

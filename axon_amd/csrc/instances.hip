@@ -18,7 +18,8 @@ const char* const KIND_NAMES[INST_KINDS] = {"gemm_fma", "gemm_tile", "gemm_strea
                                             "attention_decode", "rmsnorm", "grouped_gemm", "causal_conv",
                                             "latent_prompt", "latent_tokens", "gemm_kept", "attention_f32_prefill",
                                             "attention_f32_decode", "gemm_fma_by_chain", "gemm_fma_flow", "heads_prepare",
-                                            "state_conv", "embed", "attention_f32_waves", "latent_blocks", "gemm_fma_flow_rows", "gated_scan"};
+                                            "state_conv", "embed", "attention_f32_waves", "latent_blocks", "gemm_fma_flow_rows", "gated_scan",
+                                            "masked_blocks", "masked_fold"};
 
 struct Registry {
   std::mutex lock;

@@ -941,6 +941,7 @@ static int launch_masked_mfma(const void* q, const void* cache, const int32_t* b
   const int n_chunks = partial ? masked_chunks(mask_kind, mask_size, keep, span) : 1;
   if (tiles == nullptr && partial != nullptr) {
     const int hc = grp < 16 ? grp : 16;
+    AXK_INSTANCE(INST_MASKED_BLOCKS, MAPS, DT, KC);
     masked_attention_blocks_kernel<MAPS, DT, KC><<<dim3(n_tiles, kv_heads * ((grp + hc - 1) / hc), n_chunks), 64, 0, stream>>>(
         (const bf16_t*)q, (const bf16_t*)cache, block_table, table_stride, positions, seq_rows, heads, kv_heads, dim, vdim, page_size,
         mask_kind, mask_size, scale, softcap, partial, n_chunks, keep);
@@ -952,12 +953,11 @@ static int launch_masked_mfma(const void* q, const void* cache, const int32_t* b
   }
   if (partial) {
 #define MA_FOLD(OWN)                                                                                                            \
+  AXK_INSTANCE(INST_MASKED_FOLD, MAPS, OWN);                                                                                    \
   masked_attention_fold_kernel<MAPS, OWN><<<dim3(n_tiles, heads), 64, 0, stream>>>(partial, n_chunks, tiles, gate, gate_stride, \
                                                                                    (bf16_t*)out, heads, vdim, lambda, out_scale, eps, \
                                                                                    sink_log2, gate_per_head, sinks)
-    if (vdim <= 64) MA_FOLD(1);
-    else if (vdim <= 128) MA_FOLD(2);
-    else MA_FOLD(4);
+    if (vdim <= 64) { MA_FOLD(1); } else if (vdim <= 128) { MA_FOLD(2); } else { MA_FOLD(4); }
 #undef MA_FOLD
   }
   return 0;

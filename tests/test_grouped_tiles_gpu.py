@@ -129,3 +129,29 @@ def test_sorting_pairs(T, E, top, identities):
     for listed, made, rows in ((tiles, n, 64), (wide, n_wide, 128)):
         want = [[e, first[e] + i, min(rows, int(count[e]) - i)] for e in range(E) for i in range(0, int(count[e]), rows)]
         assert int(made) == len(want) and listed.view(-1, 3)[:len(want)].tolist() == want
+
+
+@pytest.mark.parametrize("weight_on", ["output", "input"])
+def test_routed_experts_of_many_rows_take_lists_of_128(weight_on, monkeypatch):
+    """The part on the 128-row side of its rule: the bits of lists of 64 rows."""
+    from axon_amd.config.base import PartSpec
+    from axon_amd.parts.base import CacheSpec, build_part
+    from axon_amd.weights import WeightStore
+    from gpu_helpers import DictSource, PartHarness
+    T, H, E, ff = 1000, 64, 4, 2048
+    part = build_part("feed_forward", PartSpec("routed_experts", {"hidden_size": H, "experts": E, "top": 2, "ff": ff, "limit": 3.0, "weight_on": weight_on}), "l0.")
+    g = torch.Generator().manual_seed(3)
+    hs = PartHarness("bfloat16", CacheSpec(entries=1, heads=1, head_dim=8), page_size=64, n_pages=32, max_seq_len=1024)
+    part.load(WeightStore(DictSource({d.name: torch.randn(*d.shape, generator=g) * 0.2 for d in part.tensors()}), hs.rt.device, hs.rt.dtype), hs.rt)
+    h, ctx, k = torch.randn(T, H, generator=g).bfloat16().cuda(), hs.ctx([0] * T), hs.rt.k
+    assert k.grouped_gemm_wide(2 * T, E, ff, H) and not k.grouped_gemm_wide(T, E, ff, H)
+    got = []
+    for wide in (True, False):
+        if not wide:
+            monkeypatch.setattr(k, "grouped_gemm_wide", lambda *a: False)
+        out = torch.full((T, H), float("nan"), device="cuda")
+        k.reset_instances()
+        part.forward(ctx, h, out, accumulate=False)
+        assert ("grouped_gemm<5,1>" in k.instances(launched=True)) == wide
+        got.append(out)
+    assert torch.equal(got[0], got[1]) and not bool(got[0].isnan().any())

@@ -245,7 +245,6 @@ def check_rmsnorm(dtype, dim):
     return hit
 
 
-# --------------------------------------------------------------------------- the cases
 def check_heads_prepare(dtype, T, form):
     """Queries, keys and values of T tokens in one call: the bits of calls of 200 of them.  form: normed head by head, over whole rows,
     not at all, or behind a convolution (single tokens, whose state the calls leave as they find it for the others)."""
@@ -329,6 +328,54 @@ def check_gated_scan(dtype, T):
     return hit
 
 
+def check_wide_lists(T, H, F):
+    """The gated routed product by tiles of 128 rows: the bits of tiles of 16."""
+    k, E, top = kernels("bfloat16"), 5, 2
+    P = T * top
+    h, wu = rnd(T, H, seed=1, device="cuda").bfloat16(), rnd(E, 2 * F, H, seed=2, scale=0.2, device="cuda").bfloat16()
+    chosen = rnd(T, E, seed=3).topk(top, 1).indices.int().contiguous().cuda()
+
+    def run(rows):
+        most = k.route_max_tiles(P, E, rows)
+        pairs, tokens, tiles, n = (torch.zeros(size, dtype=torch.int32, device="cuda") for size in (P, P, 3 * most, 1))
+        k.route_sort(chosen, E, pairs, tokens, tiles, n, tile_rows=rows)
+        out = torch.full((P, F), float("nan"), dtype=torch.bfloat16, device="cuda")
+        k.grouped_gemm(h, wu, out, x_group_stride=0, out_group_stride=0, glu=(float("inf"), 1.0, 0.0), routed=(tiles, n, most, tokens, pairs, rows), rows=P)
+        return out
+    got = {}
+    hit = launched(k, "bfloat16", lambda: got.setdefault("out", run(128)))
+    assert torch.equal(got["out"], run(16)) and not bool(got["out"].isnan().any())
+    return hit
+
+
+def check_masked_blocks(maps, dim, vdim, page, softcap, gated):
+    """Single tokens whose blocks of positions run side by side, against the walk of a wave a token (up to the order of the sums), with
+    a bend, with gates by head and by dim, in pages of several blocks."""
+    k, heads, kv, contexts = kernels("bfloat16"), 6, 2, [0, 63, 64, 200, 413]
+    T, need = len(contexts), [c // page + 1 for c in contexts]
+    order = torch.randperm(sum(need), generator=torch.Generator().manual_seed(2)).int().cuda()
+    table = torch.zeros(T, max(need), dtype=torch.int32, device="cuda")
+    for i, n in enumerate(need):
+        table[i, :n] = order[sum(need[:i]):sum(need[:i + 1])]
+    cache = rnd(sum(need), 1, page, kv * (maps * dim + vdim), seed=3, device="cuda").bfloat16()
+    q = rnd(T, heads * maps * dim, seed=4, device="cuda").bfloat16()
+    gate = None if not gated else rnd(T, heads * (vdim if gated == "dims" else 1) + 5, seed=5, device="cuda")[:, :heads * (vdim if gated == "dims" else 1)]
+    pos, rows = torch.tensor(contexts, dtype=torch.int32, device="cuda"), torch.arange(T, dtype=torch.int32, device="cuda")
+
+    def attend(span):
+        out = torch.full((T, heads * vdim), float("nan"), dtype=torch.bfloat16, device="cuda")
+        k.masked_attention(q, cache, table, pos, rows, out, heads, kv, maps, dim, vdim, page, "causal", 0, dim ** -0.5, softcap=softcap, lam=0.3,
+                           out_scale=0.7, eps=1e-6, gate=gate, gate_per_head=gated == "heads", span=span)
+        return out.double()
+    got = {}
+    hit = launched(k, "bfloat16", lambda: got.setdefault("out", attend(max(contexts) + 1)))
+    walk = attend(0)
+    # one rounding of weights to 8 bits and one of the output on either side, over values of a few units
+    assert float((got["out"] - walk).abs().max()) <= 2.0 ** -7 * float(walk.abs().max()) * (4 if maps == 2 else 1)
+    return hit
+
+
+# --------------------------------------------------------------------------- the cases
 # (names of the instances the case is meant to select, the check, its arguments)
 BF, F32 = "bfloat16", "float32"
 def check_grouped(dtype, M, G, N, K, glu):
@@ -578,6 +625,7 @@ CASES = [
     (BF, ["grouped_gemm<3,0>"], check_grouped, (BF, 300, 3, 40, 64, False)),       # many rows: tiles of 64 through LDS
     (BF, ["grouped_gemm<3,1>"], check_grouped, (BF, 270, 2, 72, 160, True)),
     (BF, ["grouped_gemm<2,1>"], check_grouped, (BF, 1030, 16, 200, 96, True)),     # gated, two rounds of large blocks
+    (BF, ["grouped_gemm<5,1>"], check_wide_lists, (260, 704, 300)),                # lists of tiles of 128 rows
     (F32, ["grouped_gemm<0,0>"], check_grouped, (F32, 50, 3, 40, 64, False)),
     (F32, ["grouped_gemm<0,1>"], check_grouped, (F32, 19, 2, 72, 160, True)),
     # the short convolution: a thread a (token, channel), and runs of tokens in long steps
@@ -600,6 +648,10 @@ CASES = [
     (F32, ["attention_f32_waves<128,1>"], check_attention_f32, (16, 1, 128, 16, 600, 300, 3)),
     (F32, ["attention_f32_decode<64,4>"], check_attention_f32, (8, 4, 64, 16, 140, 0, 40)),
     (F32, ["attention_f32_decode<128,4>"], check_attention_f32, (8, 4, 128, 32, 150, 60, 33)),
+    # decoding attention by blocks of positions (maps, tiles of 16 value dims, chunks of 32 key dims), and what adds them up (value dims a lane)
+    *[(BF, [f"masked_blocks<{maps},{dt},{kc}>", f"masked_fold<{maps},{own}>"], check_masked_blocks, (maps, dim, vdim, page, softcap, gated))
+      for maps in (1, 2) for dt, own, vdim in ((4, 1, 48), (8, 2, 128), (16, 4, 208))
+      for kc, dim, page, softcap, gated in ((2, 40, 64, 0.0, "dims"), (4, 128, 192, 20.0, None), (8, 256, 128, 0.0, "heads"))],
     # the gated recurrence: a thread a channel, or waves that feed the walk
     *[(dtype, [f"gated_scan<{int(T > 4)}>"], check_gated_scan, (dtype, T)) for dtype in (BF, F32) for T in (4, 77)],
     # the embedding: eight numbers a thread, or one (unaligned rows, and many tokens of a packed table)
