@@ -1098,7 +1098,7 @@ class Kernels:
         limit = 128 if sum(16 < n <= 128 for n in lengths) * channels >= 65536 else 16 if sum(8 < n <= 16 for n in lengths) * channels >= 16384 else 8
         long = next((i for i, n in enumerate(lengths) if n <= 128), len(lengths))
         fed = next((i for i, n in enumerate(lengths) if n <= limit), len(lengths))
-        cuts = [(0, long, lengths[0]), (long, fed, lengths[long] if long < fed else 0), (fed, len(lengths), 0)]
+        cuts = [(0, long, lengths[0] if long else 0), (long, fed, lengths[long] if long < fed else 0), (fed, len(lengths), 0)]
         return [g for g in cuts if g[0] < g[1]]
 
     def gated_scan(self, gates, u, y, x, lam, decay: float, state, spans, positions, seq_rows, out, block_width: int, taps: int,

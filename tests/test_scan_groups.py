@@ -5,7 +5,7 @@ from axon_amd.kernels.lib import Kernels
 
 
 @pytest.mark.parametrize("channels", [1, 64, 512, 2560, 8192])
-@pytest.mark.parametrize("lengths", [[1], [8], [9], [128], [129], [2000] + [1] * 20, [300, 300, 64, 64, 20, 9, 3, 1], [100] * 100, [5] * 300,
+@pytest.mark.parametrize("lengths", [[], [1], [8], [9], [128], [129], [2000] + [1] * 20, [300, 300, 64, 64, 20, 9, 3, 1], [100] * 100, [5] * 300,
                                      [64] * 4 + [1] * 30, [16] * 16, [17] * 300 + [16] * 3, [129, 128, 17, 16, 9, 8]])
 def test_groups_cover_the_requests(lengths, channels):
     groups = Kernels.scan_groups(lengths, channels)
