@@ -35,7 +35,7 @@ enum {
   INST_ATTENTION_F32_DECODE,     // float32 build, head_dim, waves a block
   INST_GEMM_FMA_BY_CHAIN,    // beside gemm_fma: rows of X a block, gated, numbers loaded four at a time
   INST_GEMM_FMA_FLOW,        // beside gemm_fma<128>: rows to LDS by direct loads; gated
-  INST_HEADS_PREPARE,        // 1: a block a token, 0: several
+  INST_HEADS_PREPARE,        // blocks a token: 1: one, 2: of up to eight or sixteen units, 0: of four
   INST_STATE_CONV,           // 1: runs of tokens, 0: a thread a (token, channel)
   INST_EMBED,                // 1: eight numbers a thread, 0: one
   INST_ATTENTION_F32_WAVES,      // beside attention_f32_prefill: head_dim, waves for sixteen tokens

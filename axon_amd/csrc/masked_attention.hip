@@ -993,12 +993,17 @@ extern "C" int axk_heads_prepare(const float* proj, long stride, int q_at, int n
                 "heads_prepare: a convolution wants q, k and v side by side, all stored, normed head by head or not at all");
   }
   if (n_tokens == 0) return 0;
-  // Few tokens: a token's units side by side in several blocks.  From 1,024 tokens on there are blocks enough, and what all blocks of a
-  // token do again (with norm_rows the sums over its whole rows) counts.  us, one block a token / up to 16: 32 + 8 heads of 128 normed
-  // over whole rows, 2,048 tokens 35 / 104, 16 + 2 17.2 / 25.7, of 8,192 tokens 52 / 124; with a convolution 16 + 2, 4,096 tokens 39.7 /
-  // 52.1; no norm 19.7 / 25.8; normed head by head 31.8 / 34.5, 2,048 tokens 19.4 / 19.5, and of 1,024 32 + 8 27.9 / 21.5.
-  const int per_token = n_tokens >= 1024 ? 1 : min((n_q + n_k + 3) / 4, 16);
-  if (n_tokens >= 1024) { AXK_INSTANCE(INST_HEADS_PREPARE, 1); } else { AXK_INSTANCE(INST_HEADS_PREPARE, 0); }
+  // Few tokens: a token's units side by side in several blocks, a unit a wave.  From 1,024 tokens on there are blocks enough, and what all
+  // blocks of a token do again counts: one block with norm_rows (the sums over its whole rows) and with a convolution, else two at least, of up
+  // to eight units normed head by head and sixteen not normed.  us at 1,024 / 2,048 / 8,192 tokens, one block, so, a unit a wave: 16 + 2 heads of
+  // 128 normed head by head 10.9 / 17.5 / 53, 9.8 / 16.8 / 55, 10.4 / 18.5 / 61; 32 + 8 25.5 / 35 / 175, 18.8 / 32 / 174, 19.9 / 35 / 192; not normed 16 + 2
+  // 6.9 / 11.2 / 30.4, 6.2 / 10.8 / 31.2, 8.2 / 14.1 / 46; one block and a unit a wave: with a convolution 16 + 2 16.6 / 25.9 / 70, 18.0 / 28.8 / 96,
+  // normed over whole rows 9.4 / 15.5 / 47, 13.9 / 24.5 / 119, 32 + 8 22.5 / 32 / 161, 36 / 101 / 403.
+  const int units = n_q + n_k;
+  int per_token = min((units + 3) / 4, 16);
+  if (n_tokens < 1024) { AXK_INSTANCE(INST_HEADS_PREPARE, 0); }
+  else if (norm_rows || conv_w != nullptr) { per_token = 1; AXK_INSTANCE(INST_HEADS_PREPARE, 1); }
+  else { per_token = min(per_token, max(2, q_gain != nullptr ? (units + 7) / 8 : (units + 15) / 16)); AXK_INSTANCE(INST_HEADS_PREPARE, 2); }
 #define HEADS_ARGS proj, stride, q_at, n_q, k_at, n_k, v_at, v_width, dim, q_gain, q_gain_is_f32, k_gain, k_gain_is_f32, eps, rot, neighbours, \
                    magnitude, table, positions, seq_rows, block_table, table_stride, (elem_t*)cache, page_size, (elem_t*)q_out, write_kv,      \
                    q_temp_coef, q_temp_every, norm_rows, cv

@@ -245,11 +245,11 @@ def check_rmsnorm(dtype, dim):
     return hit
 
 
-def check_heads_prepare(dtype, T, form):
+def check_heads_prepare(dtype, T, form, nq):
     """Queries, keys and values of T tokens in one call: the bits of calls of 200 of them.  form: normed head by head, over whole rows,
     not at all, or behind a convolution (single tokens, whose state the calls leave as they find it for the others)."""
     k = kernels(dtype)
-    td, nq, nk, dim, page, conv = getattr(torch, dtype), 5, 2, 24, 16, form == "conv"
+    td, nk, dim, page, conv = getattr(torch, dtype), 2, 24, 16, form == "conv"
     W = (nq + 2 * nk) * dim
     proj = rnd(T, W, seed=T, device="cuda")
     freqs, table = P.rope_freqs(dim // 2, 100.0).cuda(), torch.empty(T, dim // 4, 2, device="cuda")
@@ -660,9 +660,11 @@ CASES = [
     # the convolution before a state-space scan: a thread a (token, channel), or runs of tokens
     *[(dtype, [f"state_conv<{runs}>"], check_state_conv, (dtype, T, C, taps))
       for dtype in (BF, F32) for T, C, taps, runs in ((300, 70, 3, 0), (260, 6000, 4, 1), (700, 4436, 2, 1), (2051, 1036, 3, 1))],
-    # heads laid out for attention: several blocks a token in steps of up to 1,023 tokens, one beyond
-    *[(dtype, [f"heads_prepare<{int(T > 1023)}>"], check_heads_prepare, (dtype, T, form))
-      for dtype in (BF, F32) for T, form in ((1023, "rows"), (1024, "rows"), (1024, "heads"), (1025, "none"), (1030, "conv"))],
+    # heads laid out for attention: blocks of four units in steps of up to 1,023 tokens; beyond, one block a token where all would do something
+    # again, else of up to eight or sixteen units
+    *[(dtype, [f"heads_prepare<{blocks}>"], check_heads_prepare, (dtype, T, form, nq))
+      for dtype in (BF, F32) for T, form, nq, blocks in ((1023, "rows", 5, 0), (1024, "rows", 5, 1), (1024, "heads", 5, 2), (1025, "none", 5, 2),
+                                                         (1030, "conv", 5, 1), (1024, "heads", 23, 2), (1024, "none", 31, 2), (1100, "heads", 1, 2))],
     # attention on the matrix cores: (head size, query heads a block, pages of 64 positions or more)
     # and (head size, waves a block) (one wave a block in the decoding kernel up to 2,560 blocks of
     # positions, four beyond; two heads a block in the prompt kernel where tiles x heads are more
