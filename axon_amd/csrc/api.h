@@ -321,7 +321,8 @@ int axk_gated_scan_stretches(const float* gates, const float* u, const void* y, 
 // [taps - 1][channels] of the convolution's last inputs, oldest first; the state behind position p is in copy p & 1.
 // axk_state_conv: u[t, c] = act(bias[c] + sum_k w[c, k] in(t - (taps - 1 - k))) over float32 rows x (silu: act is
 // silu, else none), inputs before the step from the state; with heads > 0 also terms[t, h] = (dt, a) with
-// dt = softplus(raw[t, h] + dt_bias[h]), a = exp(-exp(a_log[h]) dt).  Reads the state only.
+// dt = softplus(raw[t, h] + dt_bias[h]), a = exp(-exp(a_log[h]) dt).  Reads the state only.  single: each token is a request of its
+// own (it changes no bit, only which kernel is taken).
 // axk_state_space_scan: per request of the step (spans [n][3] = (slot, first token, tokens); null: each token a
 // request of its own in slot seq_rows[t]) and head, over its tokens in order, S = a S + dt B x^T, y = S^T C + D x
 // with u [T, channels] = [x: heads P | B: groups N | C: groups N]; y float32 [T, heads P]; then the state row is
@@ -334,7 +335,7 @@ int axk_gated_scan_stretches(const float* gates, const float* u, const void* y, 
 int axk_state_conv(const float* x, long x_stride, const void* w, const void* bias, int bias_is_f32, int silu, const float* state,
                    long state_stride, long copy_elems, long tail_at, const int32_t* positions, const int32_t* seq_rows, float* u,
                    int n_tokens, int channels, int taps, const float* raw, long raw_stride, const void* dt_bias,
-                   int dt_bias_is_f32, const void* a_log, int a_log_is_f32, float* terms, int heads, void* stream);
+                   int dt_bias_is_f32, const void* a_log, int a_log_is_f32, float* terms, int heads, int single, void* stream);
 int axk_state_space_scan(const float* u, const float* terms, const void* d_skip, int d_is_f32, float* state, long state_stride,
                          long copy_elems, long tail_at, const int32_t* spans, int n_spans, const int32_t* positions,
                          const int32_t* seq_rows, const float* conv_in, long conv_in_stride, float* y, int heads, int groups,

@@ -698,7 +698,7 @@ extern "C" int axk_state_conv(const float* x, long x_stride, const void* w, cons
                               const float* state, long state_stride, long copy_elems, long tail_at, const int32_t* positions,
                               const int32_t* seq_rows, float* u, int n_tokens, int channels, int taps, const float* raw,
                               long raw_stride, const void* dt_bias, int dt_bias_is_f32, const void* a_log, int a_log_is_f32,
-                              float* terms, int heads, void* stream) {
+                              float* terms, int heads, int single, void* stream) {
   AXK_REQUIRE(n_tokens >= 0 && channels > 0 && taps >= 1 && x_stride >= channels && heads >= 0,
               "state_conv: bad sizes T=%d channels=%d taps=%d heads=%d row stride %ld", n_tokens, channels, taps, heads, x_stride);
   AXK_REQUIRE(tail_at >= 0 && copy_elems >= tail_at + (long)(taps - 1) * channels && state_stride >= 2 * copy_elems,
@@ -708,11 +708,12 @@ extern "C" int axk_state_conv(const float* x, long x_stride, const void* w, cons
               "state_conv: step sizes of %d heads need their inputs", heads);
   AXK_REQUIRE(n_tokens <= 65535, "state_conv: %d tokens in one step (at most 65535)", n_tokens);
   if (n_tokens == 0) return 0;
-  // Runs want enough of them to fill the chip: 6.2 million products (tokens x channels x taps).  us, a thread a (token, channel) / runs, one request:
-  // four taps 256 tokens of 2,560 channels 5.9 / 6.6, 512 9.4 / 7.8, but 512 single tokens 8.1 / 10.0; 256 of 6,144 11.4 / 8.0, single ones
-  // 10.9 / 10.2; 2,048 of 512 8.4 / 8.0, single ones 7.8 / 10.5; two taps 2,048 of 512 6.5 / 7.6, 512 of 6,144 13.9 / 9.0; four taps 1,024 of 64
-  // 2.9 / 12.6.  (Terms of a token's head are stored as a pair.)
-  if (n_tokens >= 256 && (long)n_tokens * channels * taps >= 6200000 && taps >= 2 && taps <= 4 && channels % 4 == 0 && x_stride % 4 == 0 &&
+  // Runs want enough of them to fill the chip: 4 million products (tokens x channels x taps), 6.2 where every token asks the state for its
+  // earlier inputs.  us, a thread a (token, channel) / runs: four taps of 2,560 channels, 256 tokens of one request, or in twenties, 6.7 / 7.5, 384 8.3 / 8.3,
+  // 448 9.3 / 8.4, 600 11.8 / 8.7, single ones 448 8.0 / 10.5, 600 10.7 / 11.0, 700 12.5 / 11.3; 600 of 1,280 7.7 / 7.4, 1,024 11.3 / 8.5, single 10.2 / 10.6; two
+  // taps, 600 of 2,560 8.3 / 8.3, 1,024 12.7 / 9.2, single 12.2 / 10.6; four taps 1,024 of 64 2.9 / 12.6.  (Terms of a token's head are stored as a pair.)
+  if (n_tokens >= 256 && (long)n_tokens * channels * taps >= (single ? 6200000 : 4000000) && taps >= 2 && taps <= 4 && channels % 4 == 0 &&
+      x_stride % 4 == 0 &&
       (((uintptr_t)x | (uintptr_t)u) & 15) == 0 &&
       ((uintptr_t)terms & 7) == 0) {
     AXK_INSTANCE(INST_STATE_CONV, 1);

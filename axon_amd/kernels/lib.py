@@ -123,7 +123,7 @@ _SIGNATURES = {
     "axk_gated_scan_stretches": [c_void_p, c_void_p, c_void_p, c_long, c_void_p, c_long, c_void_p, c_int, c_float, c_void_p, c_long,
                                  c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p],
     "axk_state_conv": [c_void_p, c_long, c_void_p, c_void_p, c_int, c_int, c_void_p, c_long, c_long, c_long, c_void_p, c_void_p,
-                       c_void_p, c_int, c_int, c_int, c_void_p, c_long, c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_void_p],
+                       c_void_p, c_int, c_int, c_int, c_void_p, c_long, c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_int, c_void_p],
     "axk_state_space_scan": [c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_long, c_long, c_long, c_void_p, c_int, c_void_p,
                              c_void_p, c_void_p, c_long, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_int, c_int, c_void_p,
                              c_void_p, c_void_p, c_void_p],
@@ -1138,11 +1138,12 @@ class Kernels:
 
     # ------------------------------------------------------------------ a state-space mixer with per-request state
     def state_conv(self, x, w, bias, state, copy_elems: int, tail_at: int, positions, seq_rows, u, silu: bool = True,
-                   raw=None, dt_bias=None, a_log=None, terms=None) -> torch.Tensor:
+                   raw=None, dt_bias=None, a_log=None, terms=None, single: bool = False) -> torch.Tensor:
         """u[t, c] = act(bias[c] + sum_k w[c, k] x(t - (taps - 1 - k))) over float32 rows x [T, C] (a view whose
         rows may be strided), inputs before the step from the float32 state rows (two copies of `copy_elems`
         floats, the kept inputs from `tail_at`: see csrc/state_space.hip).  With `raw` [T, heads] (float32, a
-        view), `dt_bias`, `a_log` and `terms` [T, heads, 2]: the heads' (dt, a) as well."""
+        view), `dt_bias`, `a_log` and `terms` [T, heads, 2]: the heads' (dt, a) as well.  `single`: each token is a request of
+        its own (it changes no bit)."""
         self._f32_rows(x, "conv x"); self._elem(w, "conv w"); self._f32(state, "conv state"); self._f32(u, "conv u")
         self._i32(seq_rows, "seq_rows"); self._i32(positions, "positions")
         T, C = u.shape
@@ -1161,7 +1162,7 @@ class Kernels:
             _ptr(x), x.stride(0), _ptr(w), _ptr(bias), self._vec_flag(bias, "conv bias"), 1 if silu else 0, _ptr(state),
             state.stride(0), int(copy_elems), int(tail_at), _ptr(positions), _ptr(seq_rows), _ptr(u), T, C, w.shape[1],
             _ptr(raw), 0 if raw is None else raw.stride(0), _ptr(dt_bias), self._vec_flag(dt_bias, "dt bias"), _ptr(a_log),
-            self._vec_flag(a_log, "A_log"), _ptr(terms), heads, _queue()))
+            self._vec_flag(a_log, "A_log"), _ptr(terms), heads, 1 if single else 0, _queue()))
         return u
 
     def state_space_scan(self, u, terms, d_skip, state, copy_elems: int, tail_at: int, spans, positions, seq_rows, conv_in, y,

@@ -127,7 +127,7 @@ class SelectiveStateSpace(Mixer):
         z, xbc, raw = proj[:, :self.inner], proj[:, self.inner:self.inner + self.channels], proj[:, self.inner + self.channels:]
         u, terms = ctx.ws.take((T, self.channels), f32), ctx.ws.take((T, self.heads, 2), f32)
         k.state_conv(xbc, self.conv_w, self.conv_b, state, self.copy_elems, self.tail_at, ctx.positions, ctx.seq_rows, u,
-                     silu=True, raw=raw, dt_bias=self.dt_bias, a_log=self.a_log, terms=terms)
+                     silu=True, raw=raw, dt_bias=self.dt_bias, a_log=self.a_log, terms=terms, single=ctx.decode_only)
         y = ctx.ws.take((T, self.inner), f32)
         k.state_space_scan(u, terms, self.d_skip, state, self.copy_elems, self.tail_at, step_spans(ctx), ctx.positions,
                            ctx.seq_rows, xbc, y, self.heads, self.groups, self.vdim, self.n_state, self.taps,

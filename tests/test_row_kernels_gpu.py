@@ -74,7 +74,7 @@ def test_state_convolution_of_many_tokens(lengths, taps, heads, pad, dtype):
     """Runs of eight tokens a thread: the bits of the requests one after the other, a thread a (token, channel), whatever runs
     their first tokens fall into."""
     k, T, R = kernels(dtype), sum(lengths), len(lengths)
-    C = 6200000 // (T * taps) // 4 * 4 + 12              # as few channels as the runs are taken for, and a block's last threads idle
+    C = 4000000 // (T * taps) // 4 * 4 + 12              # as few channels as the runs are taken for, and a block's last threads idle
     g = torch.Generator(device="cuda").manual_seed(T + taps)
     rows = torch.randn(T, C + pad, generator=g, device="cuda")
     w = torch.randn(C, taps, generator=g, device="cuda").to(k.dtype)
@@ -108,14 +108,15 @@ def test_state_convolution_of_many_tokens(lengths, taps, heads, pad, dtype):
     assert "state_conv<0>" in k.instances(launched=True)
 
 
-@pytest.mark.parametrize("T,C,taps,runs", [(256, 6056, 4, True), (256, 6052, 4, False), (255, 8000, 4, False), (1024, 64, 4, False), (512, 2560, 4, False),
-                                           (512, 6056, 2, True), (512, 6060, 5, False), (512, 6062, 2, False)])
-def test_the_convolution_by_runs_wants_enough_of_them(T, C, taps, runs):
+@pytest.mark.parametrize("T,C,taps,single,runs", [(256, 3908, 4, False, True), (256, 3904, 4, False, False), (256, 6056, 4, True, True), (256, 6052, 4, True, False),
+                                                  (255, 8000, 4, False, False), (1024, 64, 4, False, False), (512, 2560, 4, False, True), (512, 2560, 4, True, False),
+                                                  (512, 6056, 2, True, True), (512, 6060, 5, False, False), (512, 6062, 2, False, False)])
+def test_the_convolution_by_runs_wants_enough_of_them(T, C, taps, single, runs):
     k = kernels("bfloat16")
     x, w = torch.zeros(T, C, device="cuda"), torch.zeros(C, taps, dtype=torch.bfloat16, device="cuda")
     i, u = torch.zeros(T, dtype=torch.int32, device="cuda"), torch.empty(T, C, device="cuda")
     k.reset_instances()
-    k.state_conv(x, w, None, torch.zeros(1, 2 * (taps - 1) * C, device="cuda"), (taps - 1) * C, 0, i, i, u)
+    k.state_conv(x, w, None, torch.zeros(1, 2 * (taps - 1) * C, device="cuda"), (taps - 1) * C, 0, i, i, u, single=single)
     assert k.instances(launched=True) == [f"state_conv<{int(runs)}>"]
 
 
