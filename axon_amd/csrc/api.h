@@ -303,7 +303,8 @@ int axk_gather_rows(const void* x, long x_stride, const int32_t* rows, void* out
 // S = a S + sqrt(1 - a^2) (i u), out = S gelu(y); then the state row is brought up to date
 // (S, and the convolution's inputs from x).  gates [T, channels / block_width, 2 block_width].
 // axk_gated_scan_stretches: the same with spans, for requests of many tokens: what does not depend on the state is worked out
-// by other waves than the one that is left with a multiply-add a step (the same bits).  longest: no request has more tokens (0: not known).
+// by other waves than the one that is left with a multiply-add a step (the same bits).  n_long: the spans of more than 128 tokens
+// come first and are so many (-1: not known); alone: if they are one, it has as many blocks as it can use, whatever comes with it.
 int axk_causal_conv(const void* x, long x_stride, const void* w, const void* bias, int bias_is_f32, const float* state,
                     long state_stride, const int32_t* positions, const int32_t* seq_rows, float* u, int n_tokens,
                     int channels, int taps, void* stream);
@@ -313,8 +314,8 @@ int axk_gated_scan(const float* gates, const float* u, const void* y, long y_str
                    int taps, void* stream);
 int axk_gated_scan_stretches(const float* gates, const float* u, const void* y, long y_stride, const void* x, long x_stride,
                              const void* lam, int lam_is_f32, float decay, float* state, long state_stride, const int32_t* spans,
-                             int n_spans, const int32_t* positions, void* out, int channels, int block_width, int taps, int longest,
-                             void* stream);
+                             int n_spans, const int32_t* positions, void* out, int channels, int block_width, int taps, int n_long,
+                             int alone, void* stream);
 
 // A selective state-space mixer in its recurrent form (csrc/state_space.hip).  A request's state row (float32, rows
 // state_stride apart) holds two copies of copy_elems floats: the heads' states [heads][N][P] first, and from tail_at

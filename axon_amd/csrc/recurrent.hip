@@ -190,16 +190,20 @@ __global__ void gated_scan_kernel(const float* __restrict__ gates, const float* 
 #define SCAN_WIDEST 64
 // Tokens that the feeding threads have side by side: four at a time, since the walk reads four.
 __host__ __device__ inline int scan_rows(int width) { return SCAN_FEEDERS / width / 4 * 4; }
-// Channels a block has: of a lone request as many as give every CU a block, 16 of each of several, 64 of those that are short
-// (the blocks that are too many then leave at once, or are not launched where `longest` says so; requests take their first channels to the
-// XCDs in turn: 100 requests of 64 tokens of 64 channels, all on one XCD, 25.8 us, so 13.4).  us by width, 2,560 channels: 2,048 tokens of a request 53.5 with 8, 46.8 with
-// 10, 50.0 with 16, 91.9 with 32 (5,120 channels 64.1 with 10, 67.1 with 20, 79.1 with 16); requests of 1,000, 700 and 400 38.9 with 10, 35.7 with
-// 16, 48.5 with 32; five of 300 39.8, 33.8, 28.7, and 31.7 with 64; 64 of 32 tokens 93.0 with 16, 39.7 with 64.
+// Channels a block has: of a lone request, or one that outlasts those beside it, as many as give every CU a block, 16 of each of several, 64 of those that are short, 16 of these too while
+// all blocks have a place (512).  The short ones have blocks of their own behind the long ones' (where it is not known which they are, as many as if
+// they were long, and those that are too many leave at once: a block launched in vain costs some 10 ns); requests take their first channels to the
+// XCDs in turn (100 requests of 64 tokens of 64 channels, all on one XCD, 25.8 us, so 13.4).  us by width, 2,560 channels: 2,048 tokens of a request 53.5
+// with 8, 46.8 with 10, 50.0 with 16, 91.9 with 32 (5,120 channels 64.1 with 10, 67.1 with 20, 79.1 with 16); requests of 1,000, 700 and 400 38.9 with 10,
+// 35.7 with 16, 48.5 with 32; five of 300 39.8, 33.8, 28.7, and 31.7 with 64; 64 of 32 tokens 93.0 with 16, 39.7 with 64; one of 300 and 60 of 64, 1,024
+// channels, in vain / not 54 / 35.
 #define SCAN_SHORT 128
 __host__ inline int scan_width(int channels, int requests) {
   const int width = requests > 1 ? 16 : (channels + 255) / 256;
   return width < 8 ? 8 : width <= 16 ? (width + 1) / 2 * 2 : width <= 20 ? 20 : 32;
 }
+// Blocks of a request, as many on each XCD.
+__host__ __device__ inline int scan_blocks(int channels, int width) { return ((channels + width - 1) / width + 7) / 8 * 8; }
 // Floats a channel has in LDS: four more than its tokens, so that lanes side by side meet different banks.
 #define SCAN_FLOATS (SCAN_FEEDERS * SCAN_EACH + 4 * SCAN_WIDEST)
 
@@ -210,13 +214,18 @@ gated_scan_stretch_kernel(const float* __restrict__ gates, const float* __restri
                           const elem_t* __restrict__ x, long x_stride, const void* __restrict__ lam, int lam_is_f32, float decay,
                           float* __restrict__ state, long state_stride, const int32_t* __restrict__ spans,
                           const int32_t* __restrict__ positions, elem_t* __restrict__ out, int channels, int block_width, int taps,
-                          int width) {
+                          int n_long, int width_long, int width_short) {
   __shared__ __align__(16) float as[2][SCAN_FLOATS], bs[2][SCAN_FLOATS], ss[2][SCAN_FLOATS];
-  const int slot = spans[3 * blockIdx.y], first = spans[3 * blockIdx.y + 1], count = spans[3 * blockIdx.y + 2];
-  if (gridDim.y > 1 && count <= SCAN_SHORT) width = SCAN_WIDEST;
+  // the blocks of the long requests, request by request, then those of the short ones
+  const int per_long = scan_blocks(channels, width_long), per_short = scan_blocks(channels, width_short);
+  const bool is_long = (int)blockIdx.x < n_long * per_long;
+  const int b = blockIdx.x - (is_long ? 0 : n_long * per_long), per = is_long ? per_long : per_short;
+  const int request = b / per + (is_long ? 0 : n_long), place = b % per;
+  const int slot = spans[3 * request], first = spans[3 * request + 1], count = spans[3 * request + 2];
+  const int width = !is_long || (width_short > width_long && count <= SCAN_SHORT) ? width_short : width_long;
   // neighbouring channels on one XCD: their rows share cache lines; the requests' first ones on all in turn
-  const int per_xcd = ((channels + width - 1) / width + 7) / 8, c0 = ((blockIdx.x + blockIdx.y) % 8 * per_xcd + blockIdx.x / 8) * width;
-  if ((int)blockIdx.x / 8 >= per_xcd || c0 >= channels || count <= 0) return;
+  const int per_xcd = scan_blocks(channels, width) / 8, c0 = ((place + request) % 8 * per_xcd + place / 8) * width;
+  if (place / 8 >= per_xcd || c0 >= channels || count <= 0) return;
   const int rows = scan_rows(width), chunk = SCAN_EACH * rows, pitch = chunk + 4, chunks = (count + chunk - 1) / chunk;
   if (threadIdx.x >= SCAN_FEEDERS) {
     const int lane = threadIdx.x - SCAN_FEEDERS, c = c0 + lane;
@@ -370,21 +379,25 @@ extern "C" int axk_gated_scan(const float* gates, const float* u, const void* y,
 extern "C" int axk_gated_scan_stretches(const float* gates, const float* u, const void* y, long y_stride, const void* x, long x_stride,
                                         const void* lam, int lam_is_f32, float decay, float* state, long state_stride,
                                         const int32_t* spans, int n_spans, const int32_t* positions, void* out, int channels,
-                                        int block_width, int taps, int longest, void* stream) {
+                                        int block_width, int taps, int n_long, int alone, void* stream) {
   AXK_REQUIRE(n_spans >= 0 && channels > 0 && block_width > 0 && channels % block_width == 0 && taps >= 1,
               "gated_scan: bad sizes spans=%d channels=%d block width=%d taps=%d", n_spans, channels, block_width, taps);
   AXK_REQUIRE(state_stride >= 2L * taps * channels, "gated_scan: a state row of %ld floats does not hold 2 x %d x %d",
               state_stride, taps, channels);
   AXK_REQUIRE(spans != nullptr && positions != nullptr, "gated_scan: no spans or no positions");
   AXK_REQUIRE(n_spans <= 65535, "gated_scan: %d requests in one step (at most 65535)", n_spans);
+  AXK_REQUIRE(n_long <= n_spans, "gated_scan: %d long ones of %d requests", n_long, n_spans);
   if (n_spans == 0) return 0;
-  // several requests that are known to be short: no more blocks than have work
-  const int width = n_spans > 1 && longest > 0 && longest <= SCAN_SHORT ? SCAN_WIDEST : scan_width(channels, n_spans);
+  const int most = n_long < 0 ? n_spans : n_long;       // (not known: as many blocks as if all were long)
+  const int width = scan_width(channels, n_spans == 1 || (most == 1 && alone) ? 1 : 2);
+  const bool few = (long)most * scan_blocks(channels, width) + (long)(n_spans - most) * scan_blocks(channels, 16) <= 512;
+  const int width_short = n_spans == 1 ? width : n_long >= 0 && few ? 16 : SCAN_WIDEST;
+  const long blocks = (long)most * scan_blocks(channels, width) + (long)(n_spans - most) * scan_blocks(channels, width_short);
+  AXK_REQUIRE(blocks <= 2147483647L, "gated_scan: %ld blocks are more than one launch takes", blocks);
   AXK_INSTANCE(INST_GATED_SCAN, 1);
-  const dim3 grid(8 * ceil_div(ceil_div(channels, width), 8), n_spans);
-  gated_scan_stretch_kernel<<<grid, SCAN_FEEDERS + AXON_WAVE, 0, (hipStream_t)stream>>>(
+  gated_scan_stretch_kernel<<<(unsigned)blocks, SCAN_FEEDERS + AXON_WAVE, 0, (hipStream_t)stream>>>(
       gates, u, (const elem_t*)y, y_stride, (const elem_t*)x, x_stride, lam, lam_is_f32, decay, state, state_stride, spans, positions,
-      (elem_t*)out, channels, block_width, taps, width);
+      (elem_t*)out, channels, block_width, taps, most, width, width_short);
   AXK_LAUNCH_CHECK("gated_scan_stretches");
   return 0;
 }

@@ -8,6 +8,8 @@ other implementation behind these calls: without the library they fail.
 from __future__ import annotations
 
 import ctypes
+import functools
+import itertools
 import importlib.machinery
 import importlib.util
 import types
@@ -121,7 +123,7 @@ _SIGNATURES = {
     "axk_gated_scan": [c_void_p, c_void_p, c_void_p, c_long, c_void_p, c_long, c_void_p, c_int, c_float, c_void_p, c_long,
                        c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p],
     "axk_gated_scan_stretches": [c_void_p, c_void_p, c_void_p, c_long, c_void_p, c_long, c_void_p, c_int, c_float, c_void_p, c_long,
-                                 c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p],
+                                 c_void_p, c_int, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p],
     "axk_state_conv": [c_void_p, c_long, c_void_p, c_void_p, c_int, c_int, c_void_p, c_long, c_long, c_long, c_void_p, c_void_p,
                        c_void_p, c_int, c_int, c_int, c_void_p, c_long, c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_int, c_void_p],
     "axk_state_space_scan": [c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_long, c_long, c_long, c_void_p, c_int, c_void_p,
@@ -1088,18 +1090,42 @@ class Kernels:
         return u
 
     @staticmethod
-    def scan_groups(lengths: Sequence[int], channels: int) -> List[tuple]:
-        """Which of a step's requests, longest first, have which kernel of the gated scan: (first, end, the longest's tokens, or 0: a
-        thread a channel).  Requests of more than 128 tokens have a kernel whose blocks hold few channels; shorter ones, which would
-        leave most of its blocks without work, 64 a block; and the shortest a thread a channel, which takes 0.45 us a token and no
-        more the more channels there are: up to 8 tokens, 16 if they are a quarter of a wave a SIMD, all if they are one.  us, fed / a
-        thread a channel: 64 requests of 32 tokens of 2,560 channels 61 / 32, 16 of 16 14.7 / 10.5, 16 of 8 13.8 / 6.6, 4 of 16 of 1,024
-        5.2 / 9.6, 300 of 5 of 512 81 / 7.9, 100 of 64 72 / 45."""
-        limit = 128 if sum(16 < n <= 128 for n in lengths) * channels >= 65536 else 16 if sum(8 < n <= 16 for n in lengths) * channels >= 16384 else 8
-        long = next((i for i, n in enumerate(lengths) if n <= 128), len(lengths))
-        fed = next((i for i, n in enumerate(lengths) if n <= limit), len(lengths))
-        cuts = [(0, long, lengths[0] if long else 0), (long, fed, lengths[long] if long < fed else 0), (fed, len(lengths), 0)]
-        return [g for g in cuts if g[0] < g[1]]
+    @functools.lru_cache(maxsize=64)
+    def scan_groups(lengths: tuple, channels: int) -> tuple:
+        """Which of a step's requests, longest first, have which kernel of the gated scan: (first, end, whether its walk is fed by other waves;
+        else a thread a channel).  One launch that feeds takes all of them but where a thread a channel for those of up to 8, 16, 32, 64 or 128
+        tokens takes a seventh off by an estimate (us, fitted to 108 measured steps of 512 to 5,120 channels): a turn of a fed block
+        is 1.7 and the chip has 512 blocks at a time; a thread a channel has 3, 0.46 a token of the longest and 0.0002 a wave and token.  One
+        launch / with single tokens a thread a channel: 512 tokens beside 100 single ones of 2,560 channels 53 / 22, 2,000 beside 20 47 / 49; 64
+        requests of 32 47 / 34; requests of 300, 100, 50, 20, 8, 4 and 1 tokens 15 / 23, and 27 if those of up to 128 are a launch of their own."""
+        n, wide, narrow = len(lengths), -(-channels // 64), -(-channels // 16)
+        runs = [(t, len(list(same))) for t, same in itertools.groupby(lengths)]
+        alone = max(8, -(-channels // 256))           # channels of a block of a lone request, as the kernel's rule has it
+        alone = (alone + 1) // 2 * 2 if alone <= 16 else 20 if alone <= 20 else 32
+
+        def fed(least):                               # the requests of `least` tokens or more
+            mine = [r for r in runs if r[0] >= least]
+            long, count = sum(c for t, c in mine if t > 128), sum(c for _, c in mine)
+            width = alone if count == 1 or (long == 1 and lengths[0] > 512) else 16
+            each = -(-channels // width)
+            few = long * each + (count - long) * narrow <= 512
+            short = narrow if few else wide
+            wait = work = 0.0
+            for t, c in mine:
+                of_long = t > 128 or count == 1
+                turns = -(-t // (512 // width // 4 * 8 if of_long else 64 if few else 16)) + 2
+                wait = max(wait, 1.7 * turns)
+                work += c * turns * (0.0058 * each if t > 128 else 0.0045 * short)
+            return max(wait, work) + (4.8 if long * each + (count - long) * short > 512 else 0.0)
+        best, cut = 0.85 * fed(0), n
+        for limit in (8, 16, 32, 64, 128):
+            rest = [r for r in runs if r[0] <= limit]
+            if not rest:
+                continue
+            cost = fed(limit + 1) + 3.0 + 0.46 * rest[0][0] + 0.0002 * sum(t * c for t, c in rest) * channels / 64
+            if cost < best:
+                best, cut = cost, n - sum(c for _, c in rest)
+        return tuple(g for g in ((0, cut, True), (cut, n, False)) if g[0] < g[1])
 
     def gated_scan(self, gates, u, y, x, lam, decay: float, state, spans, positions, seq_rows, out, block_width: int, taps: int,
                    lengths: Optional[Sequence[int]] = None):
@@ -1121,16 +1147,17 @@ class Kernels:
             self._i32(spans, "scan spans")
             n = spans.shape[0]
         if spans is None or lengths is None:
-            groups = [(0, n, 1 if spans is not None and T > 4 * n else 0)] if n else []
+            groups = [(0, n, spans is not None and T > 4 * n)] if n else []
         elif len(lengths) != n or any(a < b for a, b in zip(lengths, lengths[1:])):
             raise KernelError(f"gated_scan: {len(lengths)} lengths for {n} spans, or not the longest first")
         else:
-            groups = self.scan_groups(lengths, C)
-        for first, end, longest in groups:
+            groups = self.scan_groups(tuple(lengths), C)
+        for first, end, fed in groups:
             at = None if spans is None else _ptr(spans) + 12 * first
-            if longest:              # stretches of tokens
+            if fed:                  # stretches of tokens
                 self._check(self.run.axk_gated_scan_stretches(*shared, at, end - first, _ptr(positions), _ptr(out), C, int(block_width), int(taps),
-                                                              0 if lengths is None else int(longest), _queue()))
+                                                              -1 if lengths is None else sum(t > 128 for t in lengths[first:end]),
+                                                              int(lengths is not None and lengths[0] > 512), _queue()))
             else:
                 self._check(self.run.axk_gated_scan(*shared, at, end - first, _ptr(positions), _ptr(seq_rows), _ptr(out), C, int(block_width),
                                                     int(taps), _queue()))

@@ -45,7 +45,7 @@ def longest_first(ctx):
     made = ctx.shared.get("longest_spans")
     if made is None:
         rows = sorted(([s.slot, s.q_start, s.q_len] for s in ctx.spans), key=lambda r: -r[2])
-        made = ctx.shared["longest_spans"] = (upload(rows, ctx.rt.device), [r[2] for r in rows])
+        made = ctx.shared["longest_spans"] = (upload(rows, ctx.rt.device), tuple(r[2] for r in rows))
     return made
 
 

@@ -94,9 +94,10 @@ def test_long_walk_by_width(dtype, lengths, channels):
 
 
 @pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
-@pytest.mark.parametrize("lengths, channels, kernels_run", [([300, 129, 128, 40, 17, 16, 9, 8, 1], 512, {0, 1}), ([64] * 3 + [1] * 30, 64, {0, 1}),
-                                                            ([8, 5, 5], 192, {0}), ([128] * 40, 2048, {0}), ([200, 150], 2560, {1}),
-                                                            ([16] * 20 + [9] * 5, 2560, {0}), ([100, 17], 960, {1})])
+@pytest.mark.parametrize("lengths, channels, kernels_run", [([300, 129, 128, 40, 17, 16, 9, 8, 1], 512, {1}), ([64] * 3 + [1] * 30, 64, {1}),
+                                                            ([8, 5, 5], 192, {1}), ([128] * 4, 2048, {1}), ([200, 150], 2560, {1}), ([300, 40], 5120, {1}),
+                                                            ([16] * 20 + [9] * 5, 2560, {0}), ([100, 17], 960, {1}), ([60] * 2 + [2] * 5, 512, {1}), ([256], 5120, {1}),
+                                                            ([300, 129] + [100] * 3 + [5] * 90, 2560, {0, 1}), ([700] + [1] * 60, 2560, {0, 1})])
 def test_requests_of_every_length_have_their_kernel(dtype, lengths, channels, kernels_run):
     """Longest first, with their lengths on the host: the bits of a thread a channel, whichever kernels ran."""
     from axon_amd.kernels import kernels
